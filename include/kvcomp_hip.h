@@ -354,6 +354,11 @@ typedef struct kvc_compressed_desc {
     const void *d_tail_f16;
     int64_t tail_tokens;
 } kvc_compressed_desc;
+/* The dense fp16 history of one tensor (KVCompCtx.get, models/cache/kvcomp_encode.py:138-151): the compressed tokens
+ * decoded and dequantized, the fp16 tail behind them, both straight into d_out_f16 [tokens + tail_tokens, batch, heads,
+ * head_dim] (16-byte aligned, like the tail).  elapsed_ms (may be NULL) makes the call wait. */
+int kvc_restore(int is_k, const kvc_compressed_desc *c, int64_t block_size, void *d_out_f16, int64_t batch,
+                int64_t heads, int64_t head_dim, float *elapsed_ms, void *stream);
 int64_t kvc_attention_workspace_bytes(int64_t total_tokens, int64_t v_compressed_tokens, int64_t batch,
                                       int64_t q_heads, int64_t head_dim);
 int kvc_attention_decode(const kvc_compressed_desc *k, const kvc_compressed_desc *v, const void *d_q_f16,

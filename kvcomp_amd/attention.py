@@ -17,8 +17,9 @@ import torch
 
 from . import _lib, kvcomp_cuda
 from ._lib import check
-from .compute import dims_to_mask, expected_groups
+from .compute import dims_to_mask
 from .ctx import KVCompCtx
+from .kvcomp_cuda import build_lut  # noqa: F401
 
 
 def _ptr(t):
@@ -27,16 +28,6 @@ def _ptr(t):
 
 def _stream(dev):
     return C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-
-
-def build_lut(decode_codebook: torch.Tensor, tree_format: int = kvcomp_cuda.TREE_I8) -> torch.Tensor:
-    """Decode table of one codebook (device uint8 tensor of kvc_lut_bytes() bytes)."""
-    L = _lib.lib()
-    lut = torch.empty(int(L.kvc_lut_bytes()), dtype=torch.uint8, device=decode_codebook.device)
-    with torch.cuda.device(decode_codebook.device):
-        check(L.kvc_build_lut(_ptr(decode_codebook), decode_codebook.numel(), tree_format, 1, 0, _ptr(lut),
-                              _stream(decode_codebook.device)))
-    return lut
 
 
 def k_scores(ctx: KVCompCtx, lut: torch.Tensor, q: torch.Tensor, out: Optional[torch.Tensor] = None,
@@ -79,19 +70,10 @@ class CompressedAttention:
     def __init__(self, k_ctx: KVCompCtx, v_ctx: KVCompCtx):
         assert k_ctx.is_k and not v_ctx.is_k
         self.k, self.v = k_ctx, v_ctx
-        self._k_lut = self._v_lut = None
-        self._k_lut_src = self._v_lut_src = None
         self._workspace = None
-        self._keep = []
 
     def _luts(self):
-        # decode tables follow the contexts' codebooks (built once, rebuilt if a codebook is replaced)
-        # (a context has no codebook until its first block is compressed)
-        if self.k.decode_codebook is not None and self._k_lut_src is not self.k.decode_codebook:
-            self._k_lut, self._k_lut_src = build_lut(self.k.decode_codebook, self.k.tree_format), self.k.decode_codebook
-        if self.v.decode_codebook is not None and self._v_lut_src is not self.v.decode_codebook:
-            self._v_lut, self._v_lut_src = build_lut(self.v.decode_codebook, self.v.tree_format), self.v.decode_codebook
-        return self._k_lut, self._v_lut
+        return self.k.decode_lut(), self.v.decode_lut()
 
     @staticmethod
     def _bracket(prof, key):
@@ -108,32 +90,7 @@ class CompressedAttention:
             ev.record()
 
     def _desc(self, ctx: KVCompCtx, lut) -> "_lib.CompressedDesc":
-        d = _lib.CompressedDesc()
-        if ctx._probe is not None:
-            ctx.poll_stores()                              # what queued stores have left, if it has arrived: no wait
-        if ctx.compressed_ctx_len:
-            d.d_luts = lut.data_ptr()
-            # (addresses and sizes straight from the contexts' growing arrays: a tensor view per field and call costs more
-            # host time than a short-context step takes on the device)
-            d.d_block_infos, d.block_infos_bytes = ctx._block_infos.address_and_numel()
-            d.d_thread_infos, d.thread_infos_bytes = ctx._thread_infos.address_and_numel()
-            enc, enc_bytes = ctx.encoded_nosync()          # an address and a bound: no wait for queued encodes
-            d.d_encoded, d.encoded_bytes = enc.data_ptr(), enc_bytes
-            # the kernels take the quantization parameters by pointer: they must cover every group of the stream
-            groups = expected_groups(ctx.compressed_ctx_len, ctx.block_size, ctx.batch_size, ctx.head_num, ctx.head_dim, ctx.quant_dims)
-            (d.d_quant_min_ints, n_min), (d.d_quant_scales_f16, n_scale) = ctx._min_ints.address_and_numel(), ctx._scales.address_and_numel()
-            assert n_min == groups and n_scale == groups, \
-                "the context holds %d minima and %d scales for %d quantization groups" % (n_min, n_scale, groups)
-        d.rows_per_codebook = 0
-        d.quant_mask = dims_to_mask(ctx.quant_dims)
-        d.max_tile_bytes, d.max_stream_bytes, d.max_code_bits = ctx.max_tile_bytes, ctx.max_stream_bytes, ctx.max_code_bits
-        d.tokens = ctx.compressed_ctx_len
-        tail = ctx.buffer
-        d.tail_tokens = 0 if tail is None else tail.shape[0]
-        if d.tail_tokens:
-            self._keep.append(tail.contiguous())
-            d.d_tail_f16 = self._keep[-1].data_ptr()
-        return d
+        return ctx.descriptor()
 
     def attend(self, q: torch.Tensor, scale: Optional[float] = None, out: Optional[torch.Tensor] = None,
                kernel_ms: Optional[list] = None) -> torch.Tensor:
@@ -150,7 +107,6 @@ class CompressedAttention:
             self._workspace = torch.empty(need + need // 4, dtype=torch.uint8, device=q.device)
         if out is None:
             out = torch.empty(B, Hq, D, dtype=torch.float32, device=q.device)
-        self._keep = []
         kd, vd = self._desc(self.k, k_lut), self._desc(self.v, v_lut)
         q = q.contiguous()
         ms = (C.c_float * 2)()

@@ -67,11 +67,18 @@ constexpr size_t KVC_WS_SLOT_BYTES = 16384;
 int kvc_workspace_slot(void **slot, void *stream);   // stream: the one the call launches on (a recorded call gets a slot of its own)
 int kvc_quant_params(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                      float eb, int8_t *d_min_i8, void *d_scale_f16, void *stream);
+// What a caller that keeps its decode tables knows beyond the stream itself (all zero: nothing).
+struct KvcDecodeHints {
+    const uint32_t *luts;          // tables from kvc_build_lut; NULL: derived from the decode tree per call
+    int64_t rows_per_codebook;
+    int64_t max_tile_bytes, max_stream_bytes;
+    int max_code_bits;
+};
 int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_tree_bytes, int tree_format,
                const uint8_t *d_block_infos, int64_t block_infos_bytes, const uint8_t *d_thread_infos,
                int64_t thread_infos_bytes, const uint8_t *d_encoded, int64_t encoded_bytes, const int8_t *d_min,
                const void *d_scale, int quant_mask, void *d_out, int64_t tokens, int64_t batch, int64_t heads,
-               int64_t head_dim, float *elapsed_ms, void *stream);
+               int64_t head_dim, float *elapsed_ms, void *stream, const KvcDecodeHints &hints);
 int kvc_launch_build_lut(const uint8_t *d_tree, int64_t tree_bytes, int tree_format, uint32_t *d_lut,
                          int n_codebooks, int64_t tree_stride_bytes, hipStream_t stream);
 
@@ -86,25 +93,31 @@ int kvc_launch_build_lut(const uint8_t *d_tree, int64_t tree_bytes, int tree_for
     } while (0)
 
 // Optional event bracket implementing the reference's "returns elapsed milliseconds" contract
-// (kvcomp_cuda_extension/src/kernels.cu:1026-1048).
-struct KvcTimer {
+// (kvcomp_cuda_extension/src/kernels.cu:1026-1048).  The two events come from a small pool per device (kvc_host.hip):
+// creating and destroying a pair costs a timed call more host time than recording it.
+struct KvcEventPair {
     hipEvent_t a = nullptr, b = nullptr;
+    int dev = -1;
+};
+KvcEventPair kvc_take_events();
+void kvc_give_events(const KvcEventPair &p);
+struct KvcTimer {
+    KvcEventPair ev;
     hipStream_t s;
     float *out;
     KvcTimer(float *out_, hipStream_t s_) : s(s_), out(out_) {
         if (out) {
-            (void)hipEventCreate(&a);
-            (void)hipEventCreate(&b);
-            (void)hipEventRecord(a, s);
+            ev = kvc_take_events();
+            (void)hipEventRecord(ev.a, s);
         }
     }
+    KvcTimer(const KvcTimer &) = delete;
+    ~KvcTimer() { if (ev.a) kvc_give_events(ev); }
     int finish() {
         if (!out) return 0;
-        hipError_t e = hipEventRecord(b, s);
-        if (e == hipSuccess) e = hipEventSynchronize(b);
-        if (e == hipSuccess) e = hipEventElapsedTime(out, a, b);
-        (void)hipEventDestroy(a);
-        (void)hipEventDestroy(b);
+        hipError_t e = hipEventRecord(ev.b, s);
+        if (e == hipSuccess) e = hipEventSynchronize(ev.b);
+        if (e == hipSuccess) e = hipEventElapsedTime(out, ev.a, ev.b);
         return kvc_check_hip(e, "event timing");
     }
 };

@@ -164,7 +164,7 @@ static int kvc_entropy_decode(int is_k, const uint8_t *d_encoded, int64_t encode
                               int64_t block_infos_bytes, const uint8_t *d_thread_infos, int64_t thread_infos_bytes,
                               const uint8_t *d_decode_tree, int64_t decode_tree_bytes, int tree_format, void *d_out,
                               int64_t tokens, int64_t stride, int64_t head_dim, float *elapsed_ms, void *stream_,
-                              const KvcDequantArgs *deq = nullptr)
+                              const KvcDequantArgs *deq = nullptr, const KvcDecodeHints &hints = {})
 {
     hipStream_t stream = (hipStream_t)stream_;
     if (tokens == 0) {
@@ -178,21 +178,27 @@ static int kvc_entropy_decode(int is_k, const uint8_t *d_encoded, int64_t encode
         const int64_t heads_x_batch = stride / head_dim;
         const int rc = deq ? kvc_expand(is_k, 1, d_decode_tree, decode_tree_bytes, tree_format, d_block_infos, block_infos_bytes,
                                         d_thread_infos, thread_infos_bytes, d_encoded, encoded_bytes, deq->min_i8, deq->scale,
-                                        deq->mask, d_out, tokens, deq->B, deq->H, head_dim, elapsed_ms, stream_)
+                                        deq->mask, d_out, tokens, deq->B, deq->H, head_dim, elapsed_ms, stream_, hints)
                            : kvc_expand(is_k, 0, d_decode_tree, decode_tree_bytes, tree_format, d_block_infos, block_infos_bytes,
                                         d_thread_infos, thread_infos_bytes, d_encoded, encoded_bytes, nullptr, nullptr, 0, d_out,
-                                        tokens, 1, heads_x_batch, head_dim, elapsed_ms, stream_);
+                                        tokens, 1, heads_x_batch, head_dim, elapsed_ms, stream_, hints);
         if (rc != 1) return rc;
     }
-    void *slot;
-    if (int rc = kvc_workspace_slot(&slot, (void *)stream_)) return rc;
+    void *slot = nullptr;
+    if (!hints.luts) {
+        if (int rc = kvc_workspace_slot(&slot, (void *)stream_)) return rc;
+    }
     KvcStreamArgs s;
     int64_t rows;
     if (int rc = kvc_fill_stream_args(s, d_encoded, encoded_bytes, d_block_infos, block_infos_bytes, d_thread_infos,
-                                      thread_infos_bytes, (const uint32_t *)slot, is_k, tokens, stride, head_dim, &rows))
+                                      thread_infos_bytes, hints.luts ? hints.luts : (const uint32_t *)slot, is_k, tokens, stride, head_dim,
+                                      &rows))
         return rc;
+    s.rows_per_codebook = hints.luts ? (int)hints.rows_per_codebook : 0;
     KvcTimer timer(elapsed_ms, stream);
-    if (int rc = kvc_launch_build_lut(d_decode_tree, decode_tree_bytes, tree_format, (uint32_t *)slot, 1, 0, stream)) return rc;
+    if (!hints.luts) {
+        if (int rc = kvc_launch_build_lut(d_decode_tree, decode_tree_bytes, tree_format, (uint32_t *)slot, 1, 0, stream)) return rc;
+    }
     const KvcDequantArgs q = deq ? *deq : KvcDequantArgs{nullptr, nullptr, 0, 1, 1, 1, 1};
     if (is_k && deq) hipLaunchKernelGGL(kvc_decode_k_kernel<true>, kvc_grid(s, rows), dim3(KVC_WG), 0, stream, s, d_out, q);
     else if (is_k) hipLaunchKernelGGL(kvc_decode_k_kernel<false>, kvc_grid(s, rows), dim3(KVC_WG), 0, stream, s, d_out, q);
@@ -247,4 +253,51 @@ extern "C" int kvc_decode_dequant(int is_k, const uint8_t *d_encoded, int64_t en
     return kvc_entropy_decode(is_k, d_encoded, encoded_bytes, d_block_infos, block_infos_bytes, d_thread_infos,
                               thread_infos_bytes, d_decode_tree, decode_tree_bytes, tree_format, d_out_f16, tokens,
                               batch * heads * head_dim, head_dim, elapsed_ms, stream, &q);
+}
+
+// ---------------------------------------------------------------------------------------------------
+// the whole dense history of one tensor: KVCompCtx.get (models/cache/kvcomp_encode.py:138-151), compressed part
+// and fp16 tail into one output
+// ---------------------------------------------------------------------------------------------------
+// Bound by HBM (2 bytes read and written per element).  The tail used to be joined by concatenating it with the decoded
+// part, which copied the decoded part once more: 232 us of the 330 us that a 256-head x 128 x 4177-token history took.
+__global__ void __launch_bounds__(KVC_WG) kvc_tail_copy_kernel(const uint4 *__restrict__ src, uint4 *__restrict__ dst, int64_t n16)
+{
+    for (int64_t i = (int64_t)blockIdx.x * KVC_WG + threadIdx.x; i < n16; i += (int64_t)gridDim.x * KVC_WG) dst[i] = src[i];
+}
+
+extern "C" int kvc_restore(int is_k, const kvc_compressed_desc *c, int64_t block_size, void *d_out_f16, int64_t batch,
+                           int64_t heads, int64_t head_dim, float *elapsed_ms, void *stream_)
+{
+    hipStream_t stream = (hipStream_t)stream_;
+    KVC_REQUIRE(c != nullptr && d_out_f16 != nullptr, "NULL argument");
+    KVC_REQUIRE(batch > 0 && heads > 0 && head_dim > 0 && head_dim % 8 == 0, "head_dim must be a positive multiple of 8");
+    KVC_REQUIRE((c->quant_mask & ~(int64_t)0xF) == 0, "bad quantization group mask");
+    KVC_REQUIRE(c->tokens >= 0 && c->tail_tokens >= 0, "negative token count");
+    KVC_REQUIRE(block_size > 0 && c->tokens % block_size == 0, "token count must be whole quantization blocks");
+    KVC_REQUIRE(c->tokens == 0 || (c->d_luts && c->d_quant_min_ints && c->d_quant_scales_f16), "NULL argument");
+    KVC_REQUIRE(c->tail_tokens == 0 || c->d_tail_f16, "tail pointer is NULL");
+    KVC_REQUIRE((((uintptr_t)d_out_f16 | (uintptr_t)(c->tail_tokens ? c->d_tail_f16 : nullptr)) & 15) == 0,
+                "the output and the tail must be 16-byte aligned");
+    const int64_t stride = batch * heads * head_dim;
+    KvcTimer timer(elapsed_ms, stream);
+    if (c->tokens) {
+        const KvcDequantArgs q = {c->d_quant_min_ints, reinterpret_cast<const __half *>(c->d_quant_scales_f16), (int)c->quant_mask,
+                                  (int)block_size, (int)batch, (int)heads, (int)head_dim};
+        const KvcDecodeHints hints = {(const uint32_t *)c->d_luts, c->rows_per_codebook, c->max_tile_bytes, c->max_stream_bytes,
+                                      (int)c->max_code_bits};
+        if (int rc = kvc_entropy_decode(is_k, c->d_encoded, c->encoded_bytes, c->d_block_infos, c->block_infos_bytes, c->d_thread_infos,
+                                        c->thread_infos_bytes, nullptr, 0, KVC_TREE_I8, d_out_f16, c->tokens, stride, head_dim, nullptr,
+                                        stream_, &q, hints))
+            return rc;
+    }
+    if (c->tail_tokens) {
+        const int64_t n16 = c->tail_tokens * stride / 8;
+        int64_t wgs = (n16 + KVC_WG - 1) / KVC_WG;
+        if (wgs > 8192) wgs = 8192;
+        hipLaunchKernelGGL(kvc_tail_copy_kernel, dim3((unsigned)wgs), dim3(KVC_WG), 0, stream, reinterpret_cast<const uint4 *>(c->d_tail_f16),
+                           reinterpret_cast<uint4 *>(d_out_f16) + c->tokens * stride / 8, n16);
+        KVC_HIP(hipGetLastError());
+    }
+    return timer.finish();
 }

@@ -1104,7 +1104,7 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
                const uint8_t *d_block_infos, int64_t block_infos_bytes, const uint8_t *d_thread_infos,
                int64_t thread_infos_bytes, const uint8_t *d_encoded, int64_t encoded_bytes, const int8_t *d_min,
                const void *d_scale, int quant_mask, void *d_out, int64_t tokens, int64_t batch, int64_t heads,
-               int64_t head_dim, float *elapsed_ms, void *stream_)
+               int64_t head_dim, float *elapsed_ms, void *stream_, const KvcDecodeHints &hints)
 {
     hipStream_t stream = (hipStream_t)stream_;
     if (head_dim <= 0 || head_dim > KVC_K_VEC_LEN || head_dim % 8 != 0) return 1;
@@ -1115,14 +1115,18 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
     KVC_REQUIRE(!deq || (((uintptr_t)d_scale & 3) == 0 && ((uintptr_t)d_min & 1) == 0),
                 "quant_scales must be 4-byte aligned and quant_min_ints 2-byte aligned");
     void *slot = nullptr;
-    if (int rc = kvc_workspace_slot(&slot, stream_)) return rc;
+    if (!hints.luts) {
+        if (int rc = kvc_workspace_slot(&slot, stream_)) return rc;
+    }
     KvcFusedArgs a;
     a.sched_nseg = 0;
     int64_t rows;
     const int64_t stride = batch * heads * head_dim;
     if (int rc = kvc_fill_stream_args(a.s, d_encoded, encoded_bytes, d_block_infos, block_infos_bytes, d_thread_infos,
-                                      thread_infos_bytes, (const uint32_t *)slot, is_k, tokens, stride, head_dim, &rows))
+                                      thread_infos_bytes, hints.luts ? hints.luts : (const uint32_t *)slot, is_k, tokens, stride,
+                                      head_dim, &rows))
         return rc;
+    a.s.rows_per_codebook = hints.luts ? (int)hints.rows_per_codebook : 0;
     KVC_REQUIRE(((uintptr_t)d_out & 15) == 0, "output pointer must be 16-byte aligned");
     a.min_i8 = d_min;
     a.scale = reinterpret_cast<const __half *>(d_scale);
@@ -1143,7 +1147,8 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
     const int slots = (!is_k && head_dim % KVC_WAVE != 0) ? 2 : 1;
     const int out_words = is_k ? (deq ? KvcSlab<true, true>::WORDS : KvcSlab<true, false>::WORDS)
                                : (deq ? KvcSlab<false, true>::WORDS : KvcSlab<false, false>::WORDS);
-    const size_t lds = kvc_plan_lds(a, slots, deq ? 1 : 0, encoded_bytes, rows * a.s.cols, 0, 0, 0, out_words);
+    const size_t lds = kvc_plan_lds(a, slots, deq ? 1 : 0, encoded_bytes, rows * a.s.cols, hints.max_tile_bytes,
+                                    hints.max_stream_bytes, hints.max_code_bits, out_words);
     a.expand = deq ? 2 : 1;
     a.out_words = out_words;
     // One tile per wave: measured on MI355X at 65 536 K / 49 152 V tiles, plain decode runs 1.2 to 1.4 times faster
@@ -1152,7 +1157,9 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
     const int forced_tpw = kvc_option(KVC_OPT_FUSED_TILES_PER_WAVE);
     a.s.tiles_per_wave = forced_tpw > 0 ? (forced_tpw > 64 ? 64 : forced_tpw) : 1;
     KvcTimer timer(elapsed_ms, stream);
-    if (int rc = kvc_launch_build_lut(d_decode_tree, decode_tree_bytes, tree_format, (uint32_t *)slot, 1, 0, stream)) return rc;
+    if (!hints.luts) {
+        if (int rc = kvc_launch_build_lut(d_decode_tree, decode_tree_bytes, tree_format, (uint32_t *)slot, 1, 0, stream)) return rc;
+    }
     const dim3 grid = kvc_grid(a.s, rows);
     const int kind = is_k ? 0 : slots;
 #define KVC_EXPAND_LAUNCH(K, Q) hipLaunchKernelGGL((kvc_expand_kernel<K, Q>), grid, dim3(KVC_WG), lds, stream, a)

@@ -149,6 +149,41 @@ int kvc_workspace_slot(void **slot, void *stream)
 }
 
 // ---------------------------------------------------------------------------------------------------
+// event pairs for timed calls: at most KVC_EVENT_PAIRS unused ones are kept per device, what is given back beyond
+// that is destroyed
+// ---------------------------------------------------------------------------------------------------
+constexpr int KVC_EVENT_PAIRS = 8;
+static std::mutex g_event_mutex;
+static KvcEventPair g_events[KVC_MAX_DEVICES][KVC_EVENT_PAIRS];
+static int g_events_held[KVC_MAX_DEVICES] = {};
+
+KvcEventPair kvc_take_events()
+{
+    KvcEventPair p;
+    (void)hipGetDevice(&p.dev);
+    if (p.dev >= 0 && p.dev < KVC_MAX_DEVICES) {
+        std::lock_guard<std::mutex> lock(g_event_mutex);
+        if (g_events_held[p.dev] > 0) return g_events[p.dev][--g_events_held[p.dev]];
+    }
+    (void)hipEventCreate(&p.a);
+    (void)hipEventCreate(&p.b);
+    return p;
+}
+
+void kvc_give_events(const KvcEventPair &p)
+{
+    if (p.dev >= 0 && p.dev < KVC_MAX_DEVICES) {
+        std::lock_guard<std::mutex> lock(g_event_mutex);
+        if (g_events_held[p.dev] < KVC_EVENT_PAIRS) {
+            g_events[p.dev][g_events_held[p.dev]++] = p;
+            return;
+        }
+    }
+    (void)hipEventDestroy(p.a);
+    (void)hipEventDestroy(p.b);
+}
+
+// ---------------------------------------------------------------------------------------------------
 // calculate_buffer_size (kvcomp_cuda_extension/src/kernels.cu:893-917)
 // ---------------------------------------------------------------------------------------------------
 extern "C" int kvc_calculate_buffer_size(int64_t tokens, int64_t stride, int is_k, int64_t head_num,

@@ -12,15 +12,17 @@ get_only_compressed, get_decode_quant_ints, mat_vec_mul, build_codebook, get_cr)
   * batch > 1 and per-channel K (QuantMode.ChannelQuant) are accepted.
 """
 import ast
+import ctypes as C
 import math
+import struct
 from typing import Dict, List, Optional, Tuple
 
 import torch
 
-from . import kvcomp_cuda
+from . import _lib, kvcomp_cuda
 from ._lib import KvcompError
 from .compute import (QUANT_MODE_MAP, QuantMode, blocks_to_compress, cut_tensor_ctx_len_0, dequant, dims_to_mask,  # noqa: F401
-                      mask_keepdim_shape, quant, safe_cat)
+                      expected_groups, mask_keepdim_shape, quant, safe_cat)
 
 
 class ExtractCacheConfig:
@@ -107,6 +109,11 @@ class _Growable:
     def __init__(self):
         self.data: Optional[torch.Tensor] = None
         self.used = 0
+        self.address = 0          # of `data`, and elements per row of it: kept beside it for callers on the per-token path
+        self.row = 1
+
+    def _hold(self, data: torch.Tensor):
+        self.data, self.address, self.row = data, data.data_ptr(), math.prod(data.shape[1:])
 
     def append(self, t: torch.Tensor):
         n = t.shape[0]
@@ -114,24 +121,24 @@ class _Growable:
         # context never holds much more than its stream
         if self.data is None:
             cap = n + max(n // 4, 16)
-            self.data = torch.empty((cap,) + tuple(t.shape[1:]), dtype=t.dtype, device=t.device)
+            self._hold(torch.empty((cap,) + tuple(t.shape[1:]), dtype=t.dtype, device=t.device))
         elif self.used + n > self.data.shape[0]:
             cap = self.used + n + max((self.used + n) // 4, 16)
             grown = torch.empty((cap,) + tuple(self.data.shape[1:]), dtype=self.data.dtype, device=self.data.device)
             grown[:self.used] = self.data[:self.used]
-            self.data = grown
+            self._hold(grown)
         self.data[self.used:self.used + n] = t
         self.used += n
 
     def reserve(self, n: int, tail_shape, dtype, device):
         """Make room for n more rows behind the filled part (which is kept); returns the view of those rows."""
         if self.data is None:
-            self.data = torch.empty((n + max(n // 4, 16),) + tuple(tail_shape), dtype=dtype, device=device)
+            self._hold(torch.empty((n + max(n // 4, 16),) + tuple(tail_shape), dtype=dtype, device=device))
         elif self.used + n > self.data.shape[0]:
             cap = self.used + n + max((self.used + n) // 4, 16)
             grown = torch.empty((cap,) + tuple(self.data.shape[1:]), dtype=self.data.dtype, device=self.data.device)
             grown[:self.used] = self.data[:self.used]
-            self.data = grown
+            self._hold(grown)
         return self.data[self.used:self.used + n]
 
     def trim(self):
@@ -140,20 +147,15 @@ class _Growable:
         if self.data is not None and self.data.shape[0] > cap:
             kept = torch.empty((cap,) + tuple(self.data.shape[1:]), dtype=self.data.dtype, device=self.data.device)
             kept[:self.used] = self.data[:self.used]
-            self.data = kept
+            self._hold(kept)
 
     @property
     def view(self) -> Optional[torch.Tensor]:
         return None if self.data is None else self.data[:self.used]
 
-    def address_and_numel(self):
-        """(device address, elements) of the filled part without making a tensor for it (0, 0 while empty)."""
-        if self.data is None:
-            return 0, 0
-        row = 1
-        for n in self.data.shape[1:]:
-            row *= n
-        return self.data.data_ptr(), self.used * row
+
+# the seventeen 8-byte fields of kvc_compressed_desc, in order
+_DESC = struct.Struct("=17q")
 
 
 class KVCompCtx:
@@ -192,6 +194,11 @@ class KVCompCtx:
         else:
             assert (batch_size * head_num * head_dim) % kvcomp_cuda.V_VEC_PER_BLK == 0, "hidden size must be divisible by VEC_PER_BLK"
             assert self.block_size % kvcomp_cuda.V_VEC_LEN == 0, "block size must be divisible by VEC_LEN"
+        self._mask = dims_to_mask(self.quant_dims)
+        self._groups_per_block = expected_groups(self.block_size, self.block_size, batch_size, head_num, head_dim, self.quant_dims)
+        self._descriptor = _lib.CompressedDesc()
+        self._lut: Optional[torch.Tensor] = None       # decode tables of _lut_source, see decode_lut
+        self._lut_source: Optional[torch.Tensor] = None
         self._encoded = _Growable()
         self._block_infos = _Growable()
         self._thread_infos = _Growable()
@@ -309,13 +316,6 @@ class KVCompCtx:
         self._probe = None
         self._accept(p[1], int(w[8]), int(w[2]), int(w[3]))
         self._issue_probe()
-
-    def encoded_nosync(self):
-        """(payload buffer, upper bound of the bytes in use) without waiting for queued encodes: for callers that
-        only need an address and a bound, like the fused kernels."""
-        if self._encoded.data is None:
-            return None, 0
-        return self._encoded.data, min(self._encoded.used + self._enc_pending, self._encoded.data.numel())
 
     def _append_encoded(self, encoded_: torch.Tensor):
         self._sync_sizes()
@@ -609,6 +609,38 @@ class KVCompCtx:
                   self.head_num, self.head_dim, self.tree_format)
         return decoded, t_ms
 
+    def decode_lut(self) -> Optional[torch.Tensor]:
+        """The decode tables of this context's codebook (kvc_build_lut), built once per codebook; None before the first
+        block has been compressed."""
+        if self._lut_source is not self.decode_codebook:
+            self._lut = kvcomp_cuda.build_lut(self.decode_codebook, self.tree_format)
+            self._lut_source = self.decode_codebook
+        return self._lut
+
+    def descriptor(self) -> "_lib.CompressedDesc":
+        """kvc_compressed_desc of everything held, refilled in place.  Does not wait for queued stores: addresses and a
+        bound of the payload are enough for the kernels.  Addresses and sizes come straight from the growing arrays, in
+        one go: a tensor view or a ctypes assignment per field costs more host time than a short-context step takes on
+        the device."""
+        if self._probe is not None:
+            self.poll_stores()                             # what queued stores have left, if it has arrived: no wait
+        tokens, tail = self.compressed_ctx_len, self._tail_len
+        tail_address = self._tail.data_ptr() if tail else 0
+        if tokens == 0:
+            _DESC.pack_into(self._descriptor, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, self._mask, 0, 0, 0, 0, tail_address, tail)
+            return self._descriptor
+        lut = self.decode_lut()
+        mins, scales, encoded = self._min_ints, self._scales, self._encoded
+        # the kernels take the quantization parameters by pointer: they must cover every group of the stream
+        groups = tokens // self.block_size * self._groups_per_block
+        assert mins.used * mins.row == groups and scales.used * scales.row == groups, \
+            "the context holds %d minima and %d scales for %d quantization groups" % (mins.used * mins.row, scales.used * scales.row, groups)
+        _DESC.pack_into(self._descriptor, 0, lut.data_ptr(), 0, self._block_infos.address, self._block_infos.used,
+                        self._thread_infos.address, self._thread_infos.used, encoded.address,
+                        min(encoded.used + self._enc_pending, encoded.data.shape[0]), mins.address, scales.address, self._mask,
+                        self.max_tile_bytes, self.max_stream_bytes, self.max_code_bits, tokens, tail_address, tail)
+        return self._descriptor
+
     # decode and dequantize in one kernel (no uint8 tensor in between); False = the reference's two steps
     fused_get = True
 
@@ -616,12 +648,7 @@ class KVCompCtx:
         """kvcomp_encode.py:153-166: decode + dequantize the compressed part -> ([ctx_c, B, H, D] fp16, ms)."""
         if KVCompCtx.fused_get:
             self._assert_ready()
-            out = torch.empty(self.compressed_ctx_len, self.batch_size, self.head_num, self.head_dim, dtype=torch.float16,
-                              device=self.device)
-            t_ms = kvcomp_cuda.decode_dequant(self.is_k, self.encoded_data, self.block_infos, self.thread_infos,
-                                              self.decode_codebook, self.quant_min_ints, self.quant_scales,
-                                              dims_to_mask(self.quant_dims), self.block_size, out, self.tree_format)
-            return out, t_ms
+            return self._restore(with_tail=False)
         decoded, t_ms = self.get_decode_quant_ints()
         start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         start.record()
@@ -630,11 +657,23 @@ class KVCompCtx:
         end.synchronize()
         return out.flatten(0, 1), t_ms + start.elapsed_time(end)
 
+    def _restore(self, with_tail: bool) -> Tuple[torch.Tensor, float]:
+        """The compressed part and (with_tail) the tail behind it, decoded straight into one tensor, and the milliseconds
+        that took on the device."""
+        desc = self.descriptor()
+        tail = desc.tail_tokens if with_tail else 0
+        out = torch.empty(desc.tokens + tail, self.batch_size, self.head_num, self.head_dim, dtype=torch.float16, device=self.device)
+        t_ms = kvcomp_cuda.restore(self.is_k, desc, self.block_size, out, with_tail)
+        return out, t_ms
+
     def get(self) -> Tuple[torch.Tensor, float]:
         """kvcomp_encode.py:138-151: compressed part followed by the uncompressed tail.  (While nothing has
         been compressed yet the tail is everything; the reference asserts in that state.)"""
         if self.compressed_ctx_len == 0:
             return self.buffer.clone(), 0.0
+        if KVCompCtx.fused_get:
+            self._assert_ready()
+            return self._restore(with_tail=True)
         out, t_ms = self.get_only_compressed()
         if self.buffer is not None and self.buffer.shape[0] > 0:
             out = torch.cat([out, self.buffer], dim=0)

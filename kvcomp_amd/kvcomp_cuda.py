@@ -337,6 +337,32 @@ def decode_dequant(is_k: bool, in_tensor, block_infos, thread_infos, decode_code
     return ms.value
 
 
+def build_lut(decode_codebook: torch.Tensor, tree_format: int = TREE_I8) -> torch.Tensor:
+    """Decode table of one codebook (device uint8 tensor of kvc_lut_bytes() bytes)."""
+    L = _lib.lib()
+    lut = torch.empty(int(L.kvc_lut_bytes()), dtype=torch.uint8, device=decode_codebook.device)
+    with torch.cuda.device(decode_codebook.device):
+        check(L.kvc_build_lut(_ptr(decode_codebook), decode_codebook.numel(), tree_format, 1, 0, _ptr(lut), _stream(decode_codebook)))
+    return lut
+
+
+def restore(is_k: bool, desc, block_size: int, out: torch.Tensor, with_tail: bool = True) -> float:
+    """kvc_restore: the tokens that `desc` (a _lib.CompressedDesc) describes, decoded and dequantized into `out` (device fp16
+    [tokens (+ tail), B, H, D]) with the fp16 tail behind them; returns elapsed milliseconds."""
+    _require(out.is_cuda and out.dtype == torch.float16 and out.dim() == 4 and out.is_contiguous(),
+             "out must be a contiguous device float16 tensor [T, B, H, D]")
+    T, B, H, D = out.shape
+    if not with_tail:
+        whole, desc = desc, _lib.CompressedDesc()
+        C.memmove(C.byref(desc), C.byref(whole), C.sizeof(desc))
+        desc.tail_tokens = 0
+    _require(T == desc.tokens + desc.tail_tokens, "out holds %d tokens, %d are to be restored" % (T, desc.tokens + desc.tail_tokens))
+    ms = C.c_float(0.0)
+    with torch.cuda.device(out.device):
+        check(_lib.lib().kvc_restore(int(is_k), C.byref(desc), block_size, _ptr(out), B, H, D, C.byref(ms), _stream(out)))
+    return ms.value
+
+
 def _fused(is_k, decode_code_book, block_infos, thread_infos, encoded_data, quant_min_ints, quant_scales, B, Cout,
            head_num, head_dim, tree_format):
     for t, n in ((decode_code_book, "decode_code_book"), (block_infos, "block_infos"), (thread_infos, "thread_infos"),
