@@ -400,6 +400,24 @@ int kvc_quant(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H,
               float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, void *d_min_f16,
               int64_t *d_counts, void *stream);
 
+/* ---- the first store of a stream: quant, then build_codebook over its symbols (models/cache/kvcomp_encode.py:86-103) --
+ * kvc_quant_codebook: kvc_quant, and the code of the symbols it wrote, built on the host.  smoothed_symbols: symbols
+ *   0 .. smoothed_symbols - 1 count once more than they occur.  *out receives the tables as kvc_build_codebook_host
+ *   returns them (the int8 tree where the code fits it, else the int16 tree), the longest code and the code bits of all
+ *   symbols written (without the padding of each lane stream to whole bytes).  Waits for the symbol counts, not for the
+ *   stream; cannot be recorded into a graph.
+ * kvc_put_bytes: copies host bytes to device memory in stream order without waiting; h_src may be reused at once. */
+typedef struct kvc_codebook {
+    int32_t tree_format, max_code_bits;
+    int64_t encode_bytes, decode_bytes, payload_bits;
+    uint8_t encode_table[256 * 8];
+    uint8_t decode_tree[512 * 5];
+} kvc_codebook;
+int kvc_quant_codebook(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
+                       float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, int smoothed_symbols,
+                       kvc_codebook *out, void *stream);
+int kvc_put_bytes(void *d_dst, const void *h_src, int64_t bytes, void *stream);
+
 /* ---- simulated quantization: quant_error (utils/compute.py:108-133), the value the reference's model caches
  * keep (models/cache/kvcomp_quant.py:51-69): quant_ints followed by (quant_int + min_quant) * quant_scale,
  * every step an fp16 tensor op on un-cast fp16 symbols and minima (so minima outside int8 do not wrap).

@@ -36,6 +36,12 @@ class EncodeJob(C.Structure):
                 ("d_stream_bytes", C.c_void_p), ("d_result", C.c_void_p)]
 
 
+class Codebook(C.Structure):
+    """kvc_codebook of include/kvcomp_hip.h."""
+    _fields_ = [("tree_format", C.c_int32), ("max_code_bits", C.c_int32), ("encode_bytes", C.c_int64), ("decode_bytes", C.c_int64),
+                ("payload_bits", C.c_int64), ("encode_table", C.c_uint8 * (256 * 8)), ("decode_tree", C.c_uint8 * (512 * 5))]
+
+
 # name -> argtypes (every function returns int unless listed in _RESTYPES)
 _SIGNATURES = {
     "kvc_abi_version": [],
@@ -71,6 +77,8 @@ _SIGNATURES = {
     "kvc_k_mat_vec_mul": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32p, _vp],
     "kvc_quant_groups": [_i64, _i64, _i64, _i64, _i64, _int],
     "kvc_quant": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp, _vp, _vp, _vp, _vp],
+    "kvc_quant_codebook": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp, _vp, _int, C.POINTER(Codebook), _vp],
+    "kvc_put_bytes": [_vp, _vp, _i64, _vp],
     "kvc_quant_error": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp],
     "kvc_calibration_copy": [_vp, _vp, _i64, _vp],
     "kvc_h2_codes": [_i64p, _vp, _vp],

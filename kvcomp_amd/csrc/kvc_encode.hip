@@ -72,14 +72,14 @@ __device__ __forceinline__ const uint8_t *kvc_table_of_row(const KvcEncodeArgs &
 // First launch of an encode call: clears the status words (a kernel, not a memset, so that the call can be recorded
 // in a HIP graph), fixes the block_info.offset of the first tile (from the device counter when there is one) and
 // checks that every codebook was built.
-__global__ void __launch_bounds__(KVC_WAVE) kvc_encode_init_kernel(KvcEncodeArgs a)
+__device__ __forceinline__ void kvc_encode_init(const KvcEncodeArgs &a)
 {
     __shared__ uint32_t s_bad;
     const int tid = threadIdx.x;
     if (tid == 0) s_bad = 0;
     __syncthreads();
     if (a.codebook_meta)
-        for (int i = tid; i < a.n_codebooks; i += KVC_WAVE)
+        for (int i = tid; i < a.n_codebooks; i += (int)blockDim.x)
             if (a.codebook_meta[4 * i + 3] != 0) atomicOr(&s_bad, KVC_ENC_ERR_CODEBOOK);
     __syncthreads();
     if (tid < KVC_ENC_STATUS_WORDS) {
@@ -88,10 +88,12 @@ __global__ void __launch_bounds__(KVC_WAVE) kvc_encode_init_kernel(KvcEncodeArgs
         if (tid == KVC_ENC_ST_BASE) v = a.base_global_offset + (a.stream_bytes ? *a.stream_bytes : 0u);
         a.status[tid] = v;
     }
+    __syncthreads();
 }
+__global__ void __launch_bounds__(KVC_WAVE) kvc_encode_init_kernel(KvcEncodeArgs a) { kvc_encode_init(a); }
 
-// Last launch: hands the call's outcome to the caller's device words (see kvc_encode_job).
-__global__ void kvc_encode_publish_kernel(KvcEncodeArgs a)
+// Hands the call's outcome to the caller's device words (see kvc_encode_job): one thread, behind everything else.
+__device__ __forceinline__ void kvc_encode_publish(const KvcEncodeArgs &a)
 {
     const uint32_t total = a.status[0], err = a.status[1];
     if (a.result) {
@@ -105,6 +107,8 @@ __global__ void kvc_encode_publish_kernel(KvcEncodeArgs a)
     }
     if (a.stream_bytes && !err) *a.stream_bytes = a.status[KVC_ENC_ST_BASE] - a.base_global_offset + total;
 }
+
+__global__ void kvc_encode_publish_kernel(KvcEncodeArgs a) { kvc_encode_publish(a); }
 
 // The 128 (or fewer) symbols of this lane's vector, 4 per register in stream order.
 //   K: token 64*row + lane, channels vec_len*col ..          (kernels.cu:439-444: one contiguous run)
@@ -888,12 +892,14 @@ __device__ __forceinline__ uint32_t kvc_wave_sum_u32(uint32_t v)
     return v;
 }
 
+// First launch of a one-pass call: what kvc_encode_init_kernel does, by the first workgroup, and the marks.
 __global__ void __launch_bounds__(KVC_WG) kvc_encode_mark_kernel(KvcEncodeArgs a)
 {
     const int64_t tile = (int64_t)blockIdx.x * KVC_WG + threadIdx.x;
     if (tile < a.tiles) reinterpret_cast<uint64_t *>(a.block_infos)[tile] = kvc_bi_word(0u, 0u, KVC_BI_NOT_READY);
     if (tile < (a.tiles + KVC_ONCE_GROUP_TILES - 1) / KVC_ONCE_GROUP_TILES) kvc_group_words(a)[tile] = kvc_group_word(0u, KVC_BI_NOT_READY);
     if (blockIdx.x == 0) {
+        kvc_encode_init(a);
         for (int i = threadIdx.x; i < KVC_ONCE_PART_LINES * KVC_ONCE_PART_STRIDE; i += KVC_WG) a.status[KVC_ONCE_PART_WORD + i] = 0u;
         if (threadIdx.x == 0) {
             a.status[KVC_ONCE_BASE_WORD] = a.status[KVC_ENC_ST_BASE];
@@ -1305,7 +1311,10 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
         }
     }
     __syncthreads();
-    if (!s_again) return;
+    if (!s_again) {                                       // the rule
+        if (tid == 0) kvc_encode_publish(a.e);
+        return;
+    }
     // ---- the whole call again, two passes inside this workgroup ----
     const int64_t tiles = a.e.tiles;
     for (int64_t tile = wave; tile < tiles; tile += KVC_WAVES_PER_WG) {      // count: thread_infos, byte_nums, group parameters
@@ -1388,6 +1397,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
     if (tid == 0) {
         a.e.status[1] = (a.e.status[1] & KVC_ENC_ERR_CODEBOOK) | s_err;
         a.e.status[3] = s_longest;
+        kvc_encode_publish(a.e);
     }
 }
 
@@ -1491,15 +1501,12 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         sa.min_i8 = src->min_i8;
         sa.scale_f16 = reinterpret_cast<__half *>(src->scale_f16);
     }
-    hipLaunchKernelGGL(kvc_encode_init_kernel, dim3(1), dim3(KVC_WAVE), 0, stream, a);
     // one pass (each wave counts, places and emits its tile) where the block_infos can serve as 64-bit status words.
-    // From uint8 symbols there is no quantizing to save and the one-pass kernel runs at three waves per SIMD: measured on
-    // MI355X at 65 536 / 49 152 tiles, K symbols encode 1.5 times and V symbols 1.6 times faster in one pass (which
-    // fetches them through its LDS tile, whole token rows per load instruction) than in two.  So by default large
-    // calls take the one pass (the option's values 2 and 3 send every call through it).
+    // Measured on MI355X at 65 536 / 49 152 tiles, K symbols encode 1.5 times and V symbols 1.6 times faster in one pass
+    // (which fetches them through its LDS tile, whole token rows per load instruction) than in two; at 96 tiles the one
+    // pass is three launches instead of six.
     const int one_pass = kvc_option(KVC_OPT_ENCODE_ONE_PASS);
-    const bool symbols_in_one_pass = one_pass > 1 || (one_pass == 1 && a.tiles >= 8192);
-    if ((src ? one_pass != 0 : symbols_in_one_pass) && ((uintptr_t)c.d_block_infos & 7) == 0 &&
+    if (one_pass != 0 && ((uintptr_t)c.d_block_infos & 7) == 0 &&
         (a.tiles + KVC_ONCE_GROUP_TILES - 1) / KVC_ONCE_GROUP_TILES <= KVC_ONCE_MAX_GROUPS) {
         // how often a wave may find a word of its look-back not ready; -1 makes the call take the give-up path
         // (every wave still ends normally) so that tests can reach it from the host
@@ -1528,11 +1535,11 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
             hipLaunchKernelGGL(kvc_encode_once_kernel<2>, dim3(wgs1), dim3(KVC_WG), lds, stream, sa, run);
             hipLaunchKernelGGL(kvc_encode_finish_kernel<2>, dim3(1), dim3(KVC_WG), 0, stream, sa);
         }
-        if (a.result || a.stream_bytes) hipLaunchKernelGGL(kvc_encode_publish_kernel, dim3(1), dim3(1), 0, stream, a);
         KVC_HIP(hipGetLastError());
         *slot_out = slot;
         return 0;
     }
+    hipLaunchKernelGGL(kvc_encode_init_kernel, dim3(1), dim3(KVC_WAVE), 0, stream, a);
     if (!src) hipLaunchKernelGGL(kvc_encode_count_kernel, dim3(wgs), dim3(KVC_WG), 0, stream, a);
     else if (is_k) hipLaunchKernelGGL(kvc_store_count_kernel<true>, dim3(wgs), dim3(KVC_WG), 0, stream, sa);
     else hipLaunchKernelGGL(kvc_store_count_kernel<false>, dim3(wgs), dim3(KVC_WG), 0, stream, sa);

@@ -1,0 +1,185 @@
+// kvc_first.hip -- the first store of a context: quantize, learn the codebook, hand it to the device.
+//
+//   kvc_quant_codebook  <- quant + build_codebook of the first stored chunk (models/cache/kvcomp_encode.py:86-103,
+//                          src/huffman.cpp:99-157)
+//   kvc_put_bytes          host bytes to device memory without a copy engine or a pinned buffer
+//
+// What a first store waits for is the histogram of its symbols: 256 numbers.  The quantizers count while they write
+// (kvc_quant.hip), a one-workgroup kernel stores the counters to pinned host memory behind them, and the calling thread
+// looks at that memory until they are there.  The host then builds the code in some microseconds; the tie-exact
+// construction is one serial chain, which a lane of the GPU needed 65 us for (13 symbols).
+#include "kvc_common.h"
+
+#include <atomic>
+#include <chrono>
+#include <cstring>
+#include <mutex>
+
+namespace {
+// Counters on the device (zero between calls: the kernel that hands them over clears them) and where the host reads
+// them.  A call holds one block and returns it before it returns; at most KVC_COUNT_BLOCKS unused ones are kept per device.
+struct CountBlock {
+    unsigned long long *d_counts = nullptr;    // [256]
+    unsigned long long *h_counts = nullptr;    // [256] counters, [256] number of the call that stored them
+    unsigned long long calls = 0;
+    int dev = -1;
+};
+constexpr int KVC_COUNT_BLOCKS = 4, KVC_COUNT_DEVICES = 16;
+std::mutex g_count_mutex;
+CountBlock g_count_blocks[KVC_COUNT_DEVICES][KVC_COUNT_BLOCKS];
+int g_count_held[KVC_COUNT_DEVICES] = {};
+
+void free_block(CountBlock &b)
+{
+    if (b.d_counts) (void)hipFree(b.d_counts);
+    if (b.h_counts) (void)hipHostFree(b.h_counts);
+    b = CountBlock();
+}
+
+int take_block(CountBlock &b)
+{
+    int dev = 0;
+    KVC_HIP(hipGetDevice(&dev));
+    KVC_REQUIRE(dev >= 0 && dev < KVC_COUNT_DEVICES, "device index %d out of range", dev);
+    {
+        std::lock_guard<std::mutex> lock(g_count_mutex);
+        if (g_count_held[dev] > 0) {
+            b = g_count_blocks[dev][--g_count_held[dev]];
+            return 0;
+        }
+    }
+    b.dev = dev;
+    int rc = kvc_check_hip(hipMalloc((void **)&b.d_counts, 256 * 8), "hipMalloc");
+    if (!rc) rc = kvc_check_hip(hipHostMalloc((void **)&b.h_counts, 257 * 8, hipHostMallocDefault), "hipHostMalloc");
+    if (!rc) rc = kvc_check_hip(hipMemset(b.d_counts, 0, 256 * 8), "hipMemset");
+    if (!rc) rc = kvc_check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");       // once per block: the call may be on any stream
+    if (rc) {
+        free_block(b);
+        return rc;
+    }
+    b.h_counts[256] = 0;
+    return 0;
+}
+
+void give_block(CountBlock &b)
+{
+    {
+        std::lock_guard<std::mutex> lock(g_count_mutex);
+        if (g_count_held[b.dev] < KVC_COUNT_BLOCKS) {
+            g_count_blocks[b.dev][g_count_held[b.dev]++] = b;
+            return;
+        }
+    }
+    free_block(b);
+}
+}  // namespace
+
+// 2 KB over the bus.  System-scope stores, then the call's number with release order: a reader that sees the number sees
+// the counters.
+__global__ void __launch_bounds__(256) kvc_counts_to_host_kernel(unsigned long long *__restrict__ counts, unsigned long long *host,
+                                                                 unsigned long long call)
+{
+    const int t = threadIdx.x;
+    __hip_atomic_store(&host[t], counts[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    counts[t] = 0;
+    __threadfence_system();
+    __syncthreads();
+    if (t == 0) __hip_atomic_store(&host[256], call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Looks for the call's number for at most 5 ms (a first store's quantizer takes 0.01 to 0.3 ms), then lets the runtime wait
+// for the stream.
+static int wait_for_counts(const CountBlock &b, hipStream_t stream)
+{
+    const auto began = std::chrono::steady_clock::now();
+    for (;;) {
+        for (int i = 0; i < 256; i++) {
+            if (__atomic_load_n(&b.h_counts[256], __ATOMIC_ACQUIRE) == b.calls) return 0;
+            __builtin_ia32_pause();
+        }
+        if (std::chrono::steady_clock::now() - began > std::chrono::milliseconds(5)) break;
+    }
+    KVC_HIP(hipStreamSynchronize(stream));
+    KVC_REQUIRE(__atomic_load_n(&b.h_counts[256], __ATOMIC_ACQUIRE) == b.calls, "the symbol counts did not arrive");
+    return 0;
+}
+
+extern "C" int kvc_quant_codebook(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
+                                  float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, int smoothed_symbols,
+                                  kvc_codebook *out, void *stream_)
+{
+    hipStream_t stream = (hipStream_t)stream_;
+    KVC_REQUIRE(out != nullptr, "NULL argument");
+    KVC_REQUIRE(NB > 0, "nothing to quantize");
+    KVC_REQUIRE(smoothed_symbols >= 0 && smoothed_symbols <= 256, "smoothed_symbols must be 0 .. 256");
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (stream) KVC_HIP(hipStreamIsCapturing(stream, &capturing));
+    KVC_REQUIRE(capturing == hipStreamCaptureStatusNone, "the first store of a context waits for its codebook and cannot be recorded into a graph");
+    CountBlock block;
+    if (int rc = take_block(block)) return rc;
+    block.calls++;
+    int rc = kvc_quant(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, d_min_i8, d_scale_f16, nullptr, (int64_t *)block.d_counts, stream_);
+    if (!rc) {
+        hipLaunchKernelGGL(kvc_counts_to_host_kernel, dim3(1), dim3(256), 0, stream, block.d_counts, block.h_counts, block.calls);
+        rc = kvc_check_hip(hipGetLastError(), "kvc_counts_to_host_kernel launch");
+    }
+    if (!rc) rc = wait_for_counts(block, stream);
+    if (rc) {
+        (void)hipStreamSynchronize(stream);                // whatever was queued may still write the block
+        free_block(block);
+        return rc;
+    }
+    int64_t counts[256];
+    for (int s = 0; s < 256; s++) counts[s] = (int64_t)block.h_counts[s];
+    give_block(block);
+    int64_t smoothed[256];
+    for (int s = 0; s < 256; s++) smoothed[s] = counts[s] + (s < smoothed_symbols ? 1 : 0);
+    // the reference's int8 tree where the code fits it, the int16 tree where it does not
+    int shift = 0;
+    out->tree_format = KVC_TREE_I8;
+    rc = kvc_build_codebook_host(smoothed, KVC_TREE_I8, &shift, out->encode_table, sizeof(out->encode_table), &out->encode_bytes,
+                                 out->decode_tree, sizeof(out->decode_tree), &out->decode_bytes);
+    if (rc) {
+        out->tree_format = KVC_TREE_I16;
+        if (int rc16 = kvc_build_codebook_host(smoothed, KVC_TREE_I16, &shift, out->encode_table, sizeof(out->encode_table), &out->encode_bytes,
+                                               out->decode_tree, sizeof(out->decode_tree), &out->decode_bytes))
+            return rc16;
+    }
+    KVC_REQUIRE(shift == 0, "shift must be 0");
+    out->max_code_bits = 0;
+    out->payload_bits = 0;
+    const uint32_t *entry = reinterpret_cast<const uint32_t *>(out->encode_table);
+    for (int64_t s = 0; s < out->encode_bytes / 8; s++) {
+        const uint32_t length = entry[2 * s + 1];
+        if ((int)length > out->max_code_bits) out->max_code_bits = (int)length;
+        out->payload_bits += counts[s] * (int64_t)length;
+    }
+    return 0;
+}
+
+// The bytes travel in the kernel's argument block (written by the host when it queues the launch).  A codebook's tables
+// are some hundred bytes: one launch, where a copy from pageable memory makes the host wait for the stream.
+struct KvcPutArgs {
+    uint32_t words[960];
+    uint8_t *dst;
+    int bytes;
+};
+__global__ void __launch_bounds__(256) kvc_put_bytes_kernel(KvcPutArgs a)
+{
+    const uint8_t *src = reinterpret_cast<const uint8_t *>(a.words);
+    for (int i = threadIdx.x; i < a.bytes; i += 256) a.dst[i] = src[i];
+}
+
+extern "C" int kvc_put_bytes(void *d_dst, const void *h_src, int64_t bytes, void *stream_)
+{
+    KVC_REQUIRE(bytes >= 0 && (bytes == 0 || (d_dst && h_src)), "NULL argument");
+    KvcPutArgs a;
+    for (int64_t at = 0; at < bytes; at += (int64_t)sizeof(a.words)) {
+        const int64_t n = bytes - at < (int64_t)sizeof(a.words) ? bytes - at : (int64_t)sizeof(a.words);
+        std::memcpy(a.words, (const uint8_t *)h_src + at, (size_t)n);
+        a.dst = (uint8_t *)d_dst + at;
+        a.bytes = (int)n;
+        hipLaunchKernelGGL(kvc_put_bytes_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream_, a);
+    }
+    return kvc_check_hip(hipGetLastError(), "kvc_put_bytes_kernel launch");
+}

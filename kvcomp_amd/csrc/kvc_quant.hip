@@ -49,7 +49,56 @@ struct KvcQuantArgs {
     __half *min_f16;       // optional
     __half *xhat;          // optional: simulated-quantization values, same shape as x
     uint32_t *minmax;      // block modes: {ord(min), ord(max)} per group
+    unsigned long long *counts;    // HIST kernels: 256 counters that the symbols written are added to
 };
+
+// ---------------------------------------------------------------------------------------------------
+// symbol counts on the way out (HIST kernels)
+// ---------------------------------------------------------------------------------------------------
+// A first store needs the histogram of the symbols it has just written.  Counting them while they are in registers
+// costs the quantizers, which wait for HBM, little (402 M symbols: per-token rows of 12 288 222 us without, 239 us with;
+// per-channel groups 214 and 235 us), where kvc_histogram_kernel reads every symbol back (111 us).  One counter per (bin, lane & 31), as there:
+// counter (bin, c) lies in LDS bank c, so the lanes of a half wave never collide.  64 bins (8 KB, so that the counters do
+// not cost occupancy) hold every symbol that an error bound of 1/62 or more gives; the rare others go to the global
+// counters one by one.
+constexpr int KVC_HIST_BINS = 64;
+constexpr int KVC_HIST_WGS = 1536;          // at most this many workgroups: each clears and adds up its counters once
+
+__device__ __forceinline__ void kvc_hist_clear(uint32_t *s_bins)
+{
+    for (int i = threadIdx.x; i < KVC_HIST_BINS * 32; i += KVC_WG) s_bins[i] = 0;
+    __syncthreads();
+}
+// four symbols, one per byte
+__device__ __forceinline__ void kvc_hist_add4(const KvcQuantArgs &a, uint32_t *s_bins, uint32_t w)
+{
+    const uint32_t col = threadIdx.x & 31;
+    if ((w & 0xc0c0c0c0u) == 0u) {
+        atomicAdd(&s_bins[((w << 5) & 0x7e0u) | col], 1u);
+        atomicAdd(&s_bins[((w >> 3) & 0x7e0u) | col], 1u);
+        atomicAdd(&s_bins[((w >> 11) & 0x7e0u) | col], 1u);
+        atomicAdd(&s_bins[((w >> 19) & 0x7e0u) | col], 1u);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t s = (w >> (8 * k)) & 0xffu;
+            if (s < (uint32_t)KVC_HIST_BINS) atomicAdd(&s_bins[(s << 5) | col], 1u);
+            else atomicAdd(&a.counts[s], 1ull);
+        }
+    }
+}
+// every thread of the workgroup, once, after its last symbol
+__device__ __forceinline__ void kvc_hist_flush(const KvcQuantArgs &a, uint32_t *s_bins)
+{
+    __syncthreads();
+    const int tid = threadIdx.x;
+    if (tid < KVC_HIST_BINS) {
+        uint32_t c = 0;
+#pragma unroll
+        for (int k = 0; k < 32; k++) c += s_bins[(tid << 5) | ((k + tid) & 31)];
+        if (c) atomicAdd(&a.counts[tid], (unsigned long long)c);
+    }
+}
 
 // Writes the symbols and/or the simulated-quantization values of two adjacent elements.
 __device__ __forceinline__ void kvc_quant_store2(const KvcQuantArgs &a, int64_t i, float v0, float v1,
@@ -66,8 +115,9 @@ __device__ __forceinline__ void kvc_quant_store2(const KvcQuantArgs &a, int64_t 
 
 // ... of eight adjacent elements of one group (i a multiple of 8; 8- and 16-byte stores)
 template <int GSTEP>   // element k belongs to group g[k * GSTEP]: 0 = one group for all eight, 1 = a group each
-__device__ __forceinline__ void kvc_quant_store8(const KvcQuantArgs &a, int64_t i, const uint4 &raw, const KvcGroupParams *g)
+__device__ __forceinline__ uint2 kvc_quant_store8(const KvcQuantArgs &a, int64_t i, const uint4 &raw, const KvcGroupParams *g)
 {
+    uint2 sym = make_uint2(0u, 0u);
     const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
     float v[8];
 #pragma unroll
@@ -82,7 +132,8 @@ __device__ __forceinline__ void kvc_quant_store8(const KvcQuantArgs &a, int64_t 
             lo |= (uint32_t)kvc_quant_one(v[k], g[k * GSTEP]) << (8 * k);
             hi |= (uint32_t)kvc_quant_one(v[4 + k], g[(4 + k) * GSTEP]) << (8 * k);
         }
-        *reinterpret_cast<uint2 *>(a.sym + i) = make_uint2(lo, hi);
+        sym = make_uint2(lo, hi);
+        *reinterpret_cast<uint2 *>(a.sym + i) = sym;
     }
     if (a.xhat) {
         uint32_t o[4];
@@ -92,6 +143,7 @@ __device__ __forceinline__ void kvc_quant_store8(const KvcQuantArgs &a, int64_t 
                    ((uint32_t)__half_as_ushort(kvc_quant_error_one(v[2 * k + 1], g[(2 * k + 1) * GSTEP])) << 16);
         *reinterpret_cast<uint4 *>(a.xhat + i) = make_uint4(o[0], o[1], o[2], o[3]);
     }
+    return sym;
 }
 
 __device__ __forceinline__ void kvc_quant_minmax8(const uint4 &raw, float &mn, float &mx)
@@ -207,44 +259,63 @@ __device__ __forceinline__ uint32_t kvc_half_pair_bits(__half lo, __half hi)
 // 64 tokens in registers, so the block is read once (64 loads in flight), finds minima and maxima with packed fp16
 // min / max and quantizes two channels per instruction (kvc_quant_pair_biased: the same symbols as the fp32 chain for
 // every fp16 input, see kvc_quant_math.h).
+template <bool HIST>
 __global__ void __launch_bounds__(KVC_WG) kvc_quant_channel_once_kernel(KvcQuantArgs a)
 {
+    __shared__ uint32_t s_bins[HIST ? KVC_HIST_BINS * 32 : 1];
+    if constexpr (HIST) kvc_hist_clear(s_bins);
     const int64_t stride = a.B * a.H * a.D;
     const int64_t pairs = stride >> 1;
-    const int64_t gid = (int64_t)blockIdx.x * KVC_WG + threadIdx.x;
-    if (gid >= a.NB * pairs) return;
-    const int64_t nb = gid / pairs, c = (gid - nb * pairs) * 2;
-    const int64_t base = nb * KVC_WAVE * stride + c;
-    const __half *p = a.x + base;
-    uint32_t raw[KVC_WAVE];
+    for (int64_t gid = (int64_t)blockIdx.x * KVC_WG + threadIdx.x; gid < a.NB * pairs; gid += (int64_t)gridDim.x * KVC_WG) {
+        const int64_t nb = gid / pairs, c = (gid - nb * pairs) * 2;
+        const int64_t base = nb * KVC_WAVE * stride + c;
+        const __half *p = a.x + base;
+        uint32_t raw[KVC_WAVE];
 #pragma unroll
-    for (int t = 0; t < KVC_WAVE; t++) raw[t] = *reinterpret_cast<const uint32_t *>(p + t * stride);
-    kvc_half2 mn = __builtin_bit_cast(kvc_half2, raw[0]), mx = mn;
+        for (int t = 0; t < KVC_WAVE; t++) raw[t] = *reinterpret_cast<const uint32_t *>(p + t * stride);
+        kvc_half2 mn = __builtin_bit_cast(kvc_half2, raw[0]), mx = mn;
 #pragma unroll
-    for (int t = 1; t < KVC_WAVE; t++) {
-        const kvc_half2 x = __builtin_bit_cast(kvc_half2, raw[t]);
-        mn = __builtin_elementwise_min(mn, x);
-        mx = __builtin_elementwise_max(mx, x);
-    }
-    const uint32_t mnw = __builtin_bit_cast(uint32_t, mn), mxw = __builtin_bit_cast(uint32_t, mx);
-    const KvcGroupParams g0 = kvc_group_params(kvc_half_lo(mnw), kvc_half_lo(mxw), a.eb);
-    const KvcGroupParams g1 = kvc_group_params(kvc_half_hi(mnw), kvc_half_hi(mxw), a.eb);
-    const int64_t g = nb * stride + c;
-    kvc_quant_publish(a, g, g0);
-    kvc_quant_publish(a, g + 1, g1);
-    if (kvc_packed_quantizer_applies(g0, kvc_half_lo(mxw)) && kvc_packed_quantizer_applies(g1, kvc_half_hi(mxw))) {
-        const KvcPackedParams pp = kvc_packed_params(g0, g1);
-        const uint32_t min2 = kvc_half_pair_bits(g0.min_h, g1.min_h), scale2 = kvc_half_pair_bits(g0.scale_h, g1.scale_h);
-#pragma unroll
-        for (int t = 0; t < KVC_WAVE; t++) {
-            const uint32_t u = kvc_quant_pair_biased(raw[t], pp);
-            if (a.sym) *reinterpret_cast<uint16_t *>(a.sym + base + t * stride) = (uint16_t)kvc_low_bytes4(u, u);
-            if (a.xhat) *reinterpret_cast<uint32_t *>(a.xhat + base + t * stride) = kvc_quant_error_pair(u, min2, scale2);
+        for (int t = 1; t < KVC_WAVE; t++) {
+            const kvc_half2 x = __builtin_bit_cast(kvc_half2, raw[t]);
+            mn = __builtin_elementwise_min(mn, x);
+            mx = __builtin_elementwise_max(mx, x);
         }
-    } else {                                               // quotients beyond the packed arithmetic's range, or a zero scale
-#pragma unroll                                             // (fully: a run-time index would move the block out of the registers)
-        for (int t = 0; t < KVC_WAVE; t++) kvc_quant_store2(a, base + t * stride, kvc_half_lo(raw[t]), kvc_half_hi(raw[t]), g0, g1);
+        const uint32_t mnw = __builtin_bit_cast(uint32_t, mn), mxw = __builtin_bit_cast(uint32_t, mx);
+        const KvcGroupParams g0 = kvc_group_params(kvc_half_lo(mnw), kvc_half_lo(mxw), a.eb);
+        const KvcGroupParams g1 = kvc_group_params(kvc_half_hi(mnw), kvc_half_hi(mxw), a.eb);
+        const int64_t g = nb * stride + c;
+        kvc_quant_publish(a, g, g0);
+        kvc_quant_publish(a, g + 1, g1);
+        if (kvc_packed_quantizer_applies(g0, kvc_half_lo(mxw)) && kvc_packed_quantizer_applies(g1, kvc_half_hi(mxw))) {
+            const KvcPackedParams pp = kvc_packed_params(g0, g1);
+            const uint32_t min2 = kvc_half_pair_bits(g0.min_h, g1.min_h), scale2 = kvc_half_pair_bits(g0.scale_h, g1.scale_h);
+#pragma unroll
+            for (int t = 0; t < KVC_WAVE; t += 2) {
+                const uint32_t u0 = kvc_quant_pair_biased(raw[t], pp), u1 = kvc_quant_pair_biased(raw[t + 1], pp);
+                const uint32_t w = kvc_low_bytes4(u0, u1);             // two channels of token t, of token t + 1
+                if (a.sym) {
+                    *reinterpret_cast<uint16_t *>(a.sym + base + t * stride) = (uint16_t)w;
+                    *reinterpret_cast<uint16_t *>(a.sym + base + (t + 1) * stride) = (uint16_t)(w >> 16);
+                }
+                if constexpr (HIST) kvc_hist_add4(a, s_bins, w);
+                if (a.xhat) {
+                    *reinterpret_cast<uint32_t *>(a.xhat + base + t * stride) = kvc_quant_error_pair(u0, min2, scale2);
+                    *reinterpret_cast<uint32_t *>(a.xhat + base + (t + 1) * stride) = kvc_quant_error_pair(u1, min2, scale2);
+                }
+            }
+        } else {                                               // quotients beyond the packed arithmetic's range, or a zero scale
+#pragma unroll                                                 // (fully: a run-time index would move the block out of the registers)
+            for (int t = 0; t < KVC_WAVE; t++) {
+                const float v0 = kvc_half_lo(raw[t]), v1 = kvc_half_hi(raw[t]);
+                kvc_quant_store2(a, base + t * stride, v0, v1, g0, g1);
+                if constexpr (HIST) {
+                    atomicAdd(&a.counts[kvc_quant_one(v0, g0)], 1ull);
+                    atomicAdd(&a.counts[kvc_quant_one(v1, g1)], 1ull);
+                }
+            }
+        }
     }
+    if constexpr (HIST) kvc_hist_flush(a, s_bins);
 }
 
 // ---- row groups (masks 0xE, 0xC, 0x8): a group is one contiguous run of R elements; one wave per
@@ -281,74 +352,125 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_kernel(KvcQuantArgs a, i
     }
 }
 
-// Row groups of 512 to 512 NIT elements (a multiple of 8, 16-byte aligned buffers), symbols and / or simulated-quantization
-// values out: the
-// wave keeps the row in registers (NIT 16-byte loads per lane in flight), so it is read once, and quantizes two
-// elements per instruction (kvc_quant_pair_biased, as the per-channel kernel above).
-template <int NIT>
+// Row groups of at least 512 elements and at most 512 NIT WPR (a multiple of 8, 16-byte aligned buffers), symbols and / or
+// simulated-quantization values out: WPR waves keep the row in registers (NIT 16-byte loads per lane in flight), so it is
+// read once, and quantize two elements per instruction (kvc_quant_pair_biased, as the per-channel kernel above).
+// Bound by HBM (2 bytes in, 1 out per element).  One wave per row up to 16 384 elements; longer rows do not fit a wave's
+// registers and are spread over the workgroup's four waves, whose minima and maxima meet in LDS: rows of 32 768 (4096 of
+// them, with counts) 82 us against 138 us (without) for kvc_quant_row_kernel, which reads every row twice.
+template <int NIT, int WPR, bool HIST>
 __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_once_kernel(KvcQuantArgs a, int64_t R, int64_t groups)
 {
-    const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * KVC_WAVES_PER_WG + (threadIdx.x >> 6);
-    if (g >= groups) return;
-    const __half *p = a.x + g * R;
-    uint4 raw[NIT];
+    static_assert(WPR == 1 || WPR == KVC_WAVES_PER_WG, "a wave or a workgroup per row");
+    __shared__ uint32_t s_bins[HIST ? KVC_HIST_BINS * 32 : 1];
+    __shared__ float s_lo[KVC_WAVES_PER_WG], s_hi[KVC_WAVES_PER_WG];
+    if constexpr (HIST) kvc_hist_clear(s_bins);
+    constexpr int ROWS = KVC_WAVES_PER_WG / WPR;           // rows of a workgroup
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int at = WPR == 1 ? lane : (int)threadIdx.x;     // this thread's place among those of the row
+    constexpr int STEP = 512 * WPR;
+    for (int64_t g = (int64_t)blockIdx.x * ROWS + (WPR == 1 ? wave : 0); g < groups; g += (int64_t)gridDim.x * ROWS) {
+        const __half *p = a.x + g * R;
+        uint4 raw[NIT];
 #pragma unroll
-    for (int j = 0; j < NIT; j++) {
-        const int64_t i = 8 * lane + 512 * j;
-        if (i < R) raw[j] = *reinterpret_cast<const uint4 *>(p + i);
-    }
-    // R >= 512 (the launcher's condition): every lane holds the row's first chunk
-    kvc_half2 mn = __builtin_bit_cast(kvc_half2, raw[0].x), mx = mn;
-    {
-        const uint32_t w[3] = {raw[0].y, raw[0].z, raw[0].w};
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const kvc_half2 x = __builtin_bit_cast(kvc_half2, w[k]);
-            mn = __builtin_elementwise_min(mn, x);
-            mx = __builtin_elementwise_max(mx, x);
+        for (int j = 0; j < NIT; j++) {
+            const int64_t i = 8 * at + STEP * j;
+            if (i < R) raw[j] = *reinterpret_cast<const uint4 *>(p + i);
         }
-    }
+        // R >= 512 WPR (the launcher's condition): every thread holds a chunk of the row's first ones
+        kvc_half2 mn = __builtin_bit_cast(kvc_half2, raw[0].x), mx = mn;
+        {
+            const uint32_t w[3] = {raw[0].y, raw[0].z, raw[0].w};
 #pragma unroll
-    for (int j = 1; j < NIT; j++) {
-        if (8 * lane + 512 * j < R) {
-            const uint32_t w[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
+            for (int k = 0; k < 3; k++) {
                 const kvc_half2 x = __builtin_bit_cast(kvc_half2, w[k]);
                 mn = __builtin_elementwise_min(mn, x);
                 mx = __builtin_elementwise_max(mx, x);
             }
         }
-    }
-    const uint32_t mnw = __builtin_bit_cast(uint32_t, mn), mxw = __builtin_bit_cast(uint32_t, mx);
-    const float lo = kvc_wave_min(fminf(kvc_half_lo(mnw), kvc_half_hi(mnw)));
-    const float hi = kvc_wave_max(fmaxf(kvc_half_lo(mxw), kvc_half_hi(mxw)));
-    const KvcGroupParams gp = kvc_group_params(lo, hi, a.eb);
-    if (lane == 0) kvc_quant_publish(a, g, gp);
-    if (!kvc_packed_quantizer_applies(gp, hi)) {           // (wave-uniform) quotients beyond the packed arithmetic's range, or a zero scale
+#pragma unroll
+        for (int j = 1; j < NIT; j++) {
+            if (8 * at + STEP * j < R) {
+                const uint32_t w[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const kvc_half2 x = __builtin_bit_cast(kvc_half2, w[k]);
+                    mn = __builtin_elementwise_min(mn, x);
+                    mx = __builtin_elementwise_max(mx, x);
+                }
+            }
+        }
+        const uint32_t mnw = __builtin_bit_cast(uint32_t, mn), mxw = __builtin_bit_cast(uint32_t, mx);
+        float lo = kvc_wave_min(fminf(kvc_half_lo(mnw), kvc_half_hi(mnw)));
+        float hi = kvc_wave_max(fmaxf(kvc_half_lo(mxw), kvc_half_hi(mxw)));
+        if constexpr (WPR > 1) {
+            if (lane == 0) {
+                s_lo[wave] = lo;
+                s_hi[wave] = hi;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < WPR; w++) {
+                lo = fminf(lo, s_lo[w]);
+                hi = fmaxf(hi, s_hi[w]);
+            }
+            __syncthreads();                               // read: the next row may overwrite them
+        }
+        const KvcGroupParams gp = kvc_group_params(lo, hi, a.eb);
+        if (at == 0) kvc_quant_publish(a, g, gp);
+        if (!kvc_packed_quantizer_applies(gp, hi)) {       // (uniform) quotients beyond the packed arithmetic's range, or a zero scale
+#pragma unroll
+            for (int j = 0; j < NIT; j++) {
+                const int64_t i = 8 * at + STEP * j;
+                if (i < R) {
+                    const uint2 w = kvc_quant_store8<0>(a, g * R + i, raw[j], &gp);
+                    if constexpr (HIST) {
+                        kvc_hist_add4(a, s_bins, w.x);
+                        kvc_hist_add4(a, s_bins, w.y);
+                    }
+                }
+            }
+            continue;
+        }
+        const KvcPackedParams pp = kvc_packed_params(gp, gp);
+        const uint32_t min2 = kvc_half_pair_bits(gp.min_h, gp.min_h), scale2 = kvc_half_pair_bits(gp.scale_h, gp.scale_h);
 #pragma unroll
         for (int j = 0; j < NIT; j++) {
-            const int64_t i = 8 * lane + 512 * j;
-            if (i < R) kvc_quant_store8<0>(a, g * R + i, raw[j], &gp);
-        }
-        return;
-    }
-    const KvcPackedParams pp = kvc_packed_params(gp, gp);
-    const uint32_t min2 = kvc_half_pair_bits(gp.min_h, gp.min_h), scale2 = kvc_half_pair_bits(gp.scale_h, gp.scale_h);
-#pragma unroll
-    for (int j = 0; j < NIT; j++) {
-        const int64_t i = 8 * lane + 512 * j;
-        if (i < R) {
-            const uint32_t u0 = kvc_quant_pair_biased(raw[j].x, pp), u1 = kvc_quant_pair_biased(raw[j].y, pp);
-            const uint32_t u2 = kvc_quant_pair_biased(raw[j].z, pp), u3 = kvc_quant_pair_biased(raw[j].w, pp);
-            if (a.sym) *reinterpret_cast<uint2 *>(a.sym + g * R + i) = make_uint2(kvc_low_bytes4(u0, u1), kvc_low_bytes4(u2, u3));
-            if (a.xhat)
-                *reinterpret_cast<uint4 *>(a.xhat + g * R + i) = make_uint4(kvc_quant_error_pair(u0, min2, scale2), kvc_quant_error_pair(u1, min2, scale2),
-                                                                           kvc_quant_error_pair(u2, min2, scale2), kvc_quant_error_pair(u3, min2, scale2));
+            const int64_t i = 8 * at + STEP * j;
+            if (i < R) {
+                const uint32_t u0 = kvc_quant_pair_biased(raw[j].x, pp), u1 = kvc_quant_pair_biased(raw[j].y, pp);
+                const uint32_t u2 = kvc_quant_pair_biased(raw[j].z, pp), u3 = kvc_quant_pair_biased(raw[j].w, pp);
+                const uint2 w = make_uint2(kvc_low_bytes4(u0, u1), kvc_low_bytes4(u2, u3));
+                if (a.sym) *reinterpret_cast<uint2 *>(a.sym + g * R + i) = w;
+                if constexpr (HIST) {
+                    kvc_hist_add4(a, s_bins, w.x);
+                    kvc_hist_add4(a, s_bins, w.y);
+                }
+                if (a.xhat)
+                    *reinterpret_cast<uint4 *>(a.xhat + g * R + i) = make_uint4(kvc_quant_error_pair(u0, min2, scale2), kvc_quant_error_pair(u1, min2, scale2),
+                                                                               kvc_quant_error_pair(u2, min2, scale2), kvc_quant_error_pair(u3, min2, scale2));
+            }
         }
     }
+    if constexpr (HIST) kvc_hist_flush(a, s_bins);
 }
+
+template <bool HIST>
+static void kvc_launch_row_once(const KvcQuantArgs &a, int64_t R, int64_t groups, hipStream_t stream)
+{
+    auto grid = [&](int waves_per_row) {
+        const int64_t rows = KVC_WAVES_PER_WG / waves_per_row, wgs = (groups + rows - 1) / rows;
+        return dim3((unsigned)(HIST && wgs > KVC_HIST_WGS ? KVC_HIST_WGS : wgs));
+    };
+    constexpr int W = KVC_WAVES_PER_WG;
+    if (R <= 512 * 8) hipLaunchKernelGGL((kvc_quant_row_once_kernel<8, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * 24) hipLaunchKernelGGL((kvc_quant_row_once_kernel<24, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * 32) hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * W * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, W, HIST>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
+    else hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, W, HIST>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
+}
+constexpr int64_t KVC_ROW_ONCE_MAX = 512 * KVC_WAVES_PER_WG * 32;
 
 // ---- block groups (masks 0xF, 0xD): rows of R contiguous elements map many-to-one onto groups;
 // wave-reduce each row, then merge rows with atomics on an order-preserving integer image. -----------
@@ -405,6 +527,85 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_block_apply_kernel(KvcQuantA
     }
 }
 
+// The same two passes with 16-byte loads and packed fp16 arithmetic (rows a multiple of 8 elements, aligned buffers), in
+// one launch each; the second also counts the symbols (HIST).  Bound by HBM: 2 bytes per element in each pass, 1 out.  One
+// wave per row.  (Half2 loads and the fp32 chain, above, took 39 + 20 us for 8192 rows of 4096.)
+__global__ void __launch_bounds__(KVC_WG) kvc_quant_block_minmax8_kernel(KvcQuantArgs a, int64_t R, int64_t rows)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * KVC_WAVES_PER_WG + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const uint4 *p = reinterpret_cast<const uint4 *>(a.x + row * R);
+    const int64_t n = R >> 3;
+    kvc_half2 mn = {(_Float16)INFINITY, (_Float16)INFINITY}, mx = -mn;
+    auto take = [&](const uint4 &v) {
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const kvc_half2 x = __builtin_bit_cast(kvc_half2, w[k]);
+            mn = __builtin_elementwise_min(mn, x);
+            mx = __builtin_elementwise_max(mx, x);
+        }
+    };
+    int64_t i = lane;
+    for (; i + 3 * KVC_WAVE < n; i += 4 * KVC_WAVE) {      // four loads in flight
+        const uint4 v0 = p[i], v1 = p[i + KVC_WAVE], v2 = p[i + 2 * KVC_WAVE], v3 = p[i + 3 * KVC_WAVE];
+        take(v0);
+        take(v1);
+        take(v2);
+        take(v3);
+    }
+    for (; i < n; i += KVC_WAVE) take(p[i]);
+    const uint32_t mnw = __builtin_bit_cast(uint32_t, mn), mxw = __builtin_bit_cast(uint32_t, mx);
+    const float lo = kvc_wave_min(fminf(kvc_half_lo(mnw), kvc_half_hi(mnw)));
+    const float hi = kvc_wave_max(fmaxf(kvc_half_lo(mxw), kvc_half_hi(mxw)));
+    if (lane == 0) {
+        const int64_t g = kvc_block_group_of_row(a, row);
+        atomicMin(&a.minmax[2 * g], kvc_f2ord(lo));
+        atomicMax(&a.minmax[2 * g + 1], kvc_f2ord(hi));
+    }
+}
+
+template <bool HIST>
+__global__ void __launch_bounds__(KVC_WG) kvc_quant_block_apply8_kernel(KvcQuantArgs a, int64_t R, int64_t rows)
+{
+    __shared__ uint32_t s_bins[HIST ? KVC_HIST_BINS * 32 : 1];
+    if constexpr (HIST) kvc_hist_clear(s_bins);
+    const int lane = threadIdx.x & 63;
+    for (int64_t row = (int64_t)blockIdx.x * KVC_WAVES_PER_WG + (threadIdx.x >> 6); row < rows; row += (int64_t)gridDim.x * KVC_WAVES_PER_WG) {
+        const int64_t g = kvc_block_group_of_row(a, row);
+        const float hi = kvc_ord2f(a.minmax[2 * g + 1]);
+        const KvcGroupParams gp = kvc_group_params(kvc_ord2f(a.minmax[2 * g]), hi, a.eb);
+        const bool packed = kvc_packed_quantizer_applies(gp, hi);
+        const KvcPackedParams pp = kvc_packed_params(gp, gp);
+        const uint32_t min2 = kvc_half_pair_bits(gp.min_h, gp.min_h), scale2 = kvc_half_pair_bits(gp.scale_h, gp.scale_h);
+        const bool first = a.mask == KVC_MASK_K_BLOCK ? (row % a.BS == 0) : ((row / a.B) % a.BS == 0);
+        if (first && lane == 0) kvc_quant_publish(a, g, gp);
+        const int64_t base = row * R;
+#pragma unroll 4
+        for (int64_t i = 8 * lane; i < R; i += 8 * KVC_WAVE) {
+            const uint4 v = *reinterpret_cast<const uint4 *>(a.x + base + i);
+            uint2 w;
+            if (packed) {                                  // wave-uniform
+                const uint32_t u0 = kvc_quant_pair_biased(v.x, pp), u1 = kvc_quant_pair_biased(v.y, pp);
+                const uint32_t u2 = kvc_quant_pair_biased(v.z, pp), u3 = kvc_quant_pair_biased(v.w, pp);
+                w = make_uint2(kvc_low_bytes4(u0, u1), kvc_low_bytes4(u2, u3));
+                if (a.sym) *reinterpret_cast<uint2 *>(a.sym + base + i) = w;
+                if (a.xhat)
+                    *reinterpret_cast<uint4 *>(a.xhat + base + i) = make_uint4(kvc_quant_error_pair(u0, min2, scale2), kvc_quant_error_pair(u1, min2, scale2),
+                                                                              kvc_quant_error_pair(u2, min2, scale2), kvc_quant_error_pair(u3, min2, scale2));
+            } else {
+                w = kvc_quant_store8<0>(a, base + i, v, &gp);
+            }
+            if constexpr (HIST) {
+                kvc_hist_add4(a, s_bins, w.x);
+                kvc_hist_add4(a, s_bins, w.y);
+            }
+        }
+    }
+    if constexpr (HIST) kvc_hist_flush(a, s_bins);
+}
+
 extern "C" int64_t kvc_quant_groups(int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int mask)
 {
     return NB * ((mask & 1) ? 1 : BS) * ((mask & 2) ? 1 : B) * ((mask & 4) ? 1 : H) * ((mask & 8) ? 1 : D);
@@ -434,13 +635,19 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
     a.min_f16 = reinterpret_cast<__half *>(d_min_f16);
     a.xhat = reinterpret_cast<__half *>(d_xhat_f16);
     a.minmax = nullptr;
+    a.counts = reinterpret_cast<unsigned long long *>(d_counts);
+    const bool want_counts = d_counts != nullptr;
+    bool counted = false;                                  // by the kernel that wrote the symbols
     const int64_t stride = B * H * D;
     if (quant_mask == KVC_MASK_CHANNEL) {
         const bool wide = stride % 8 == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.sym & 7) == 0 && ((uintptr_t)a.xhat & 15) == 0;
         const bool once = BS == KVC_WAVE && (a.sym != nullptr || a.xhat != nullptr);   // the block fits a thread's registers
         const int64_t threads = NB * (once || !wide ? stride / 2 : stride / 8);
         const dim3 grid((unsigned)((threads + KVC_WG - 1) / KVC_WG));
-        if (once) hipLaunchKernelGGL(kvc_quant_channel_once_kernel, grid, dim3(KVC_WG), 0, stream, a);
+        if (once && want_counts) {
+            hipLaunchKernelGGL(kvc_quant_channel_once_kernel<true>, dim3(grid.x > KVC_HIST_WGS ? KVC_HIST_WGS : grid.x), dim3(KVC_WG), 0, stream, a);
+            counted = true;
+        } else if (once) hipLaunchKernelGGL(kvc_quant_channel_once_kernel<false>, grid, dim3(KVC_WG), 0, stream, a);
         else if (wide) hipLaunchKernelGGL(kvc_quant_channel8_kernel, grid, dim3(KVC_WG), 0, stream, a);
         else hipLaunchKernelGGL(kvc_quant_channel_kernel, grid, dim3(KVC_WG), 0, stream, a);
     } else if (quant_mask == KVC_MASK_V_TOKEN || quant_mask == KVC_MASK_SIM_TOKEN || quant_mask == KVC_MASK_VECTOR) {
@@ -448,12 +655,12 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
         const int64_t groups = NB * BS * stride / R;
         const int wide = R % 8 == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.sym & 7) == 0 && ((uintptr_t)a.xhat & 15) == 0;
         const dim3 grid((unsigned)((groups + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG));
-        const bool once = wide && (a.sym != nullptr || a.xhat != nullptr) && R >= 512;  // the row fits a wave's registers
-        if (once && R <= 512 * 8) hipLaunchKernelGGL(kvc_quant_row_once_kernel<8>, grid, dim3(KVC_WG), 0, stream, a, R, groups);
-        else if (once && R <= 512 * 16) hipLaunchKernelGGL(kvc_quant_row_once_kernel<16>, grid, dim3(KVC_WG), 0, stream, a, R, groups);
-        else if (once && R <= 512 * 24) hipLaunchKernelGGL(kvc_quant_row_once_kernel<24>, grid, dim3(KVC_WG), 0, stream, a, R, groups);
-        else if (once && R <= 512 * 32) hipLaunchKernelGGL(kvc_quant_row_once_kernel<32>, grid, dim3(KVC_WG), 0, stream, a, R, groups);
+        // the row fits the registers of a wave or a workgroup
+        const bool once = wide && (a.sym != nullptr || a.xhat != nullptr) && R >= 512 && R <= KVC_ROW_ONCE_MAX;
+        if (once && want_counts) kvc_launch_row_once<true>(a, R, groups, stream);
+        else if (once) kvc_launch_row_once<false>(a, R, groups, stream);
         else hipLaunchKernelGGL(kvc_quant_row_kernel, grid, dim3(KVC_WG), 0, stream, a, R, groups, wide);
+        counted = once && want_counts;
     } else if (quant_mask == KVC_MASK_K_BLOCK || quant_mask == KVC_MASK_SIM_BLOCK) {
         const int64_t R = quant_mask == KVC_MASK_K_BLOCK ? stride : H * D;
         const int64_t rows = NB * BS * stride / R;
@@ -464,13 +671,23 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
         a.minmax = reinterpret_cast<uint32_t *>(slot);
         const unsigned row_wgs = (unsigned)((rows + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG);
         hipLaunchKernelGGL(kvc_quant_block_init_kernel, dim3((unsigned)((groups + KVC_WG - 1) / KVC_WG)), dim3(KVC_WG), 0, stream, a.minmax, groups);
-        hipLaunchKernelGGL(kvc_quant_block_minmax_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
-        hipLaunchKernelGGL(kvc_quant_block_apply_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
+        const bool wide = R % 8 == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.sym & 7) == 0 && ((uintptr_t)a.xhat & 15) == 0;
+        if (wide) hipLaunchKernelGGL(kvc_quant_block_minmax8_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
+        else hipLaunchKernelGGL(kvc_quant_block_minmax_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
+        if (wide && want_counts) {
+            hipLaunchKernelGGL(kvc_quant_block_apply8_kernel<true>, dim3(row_wgs > KVC_HIST_WGS ? KVC_HIST_WGS : row_wgs), dim3(KVC_WG), 0, stream,
+                               a, R, rows);
+            counted = true;
+        } else if (wide && (a.sym || a.xhat)) {
+            hipLaunchKernelGGL(kvc_quant_block_apply8_kernel<false>, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
+        } else {
+            hipLaunchKernelGGL(kvc_quant_block_apply_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
+        }
     } else {
         return kvc_fail(-1, "unsupported quantization group mask 0x%x", quant_mask);
     }
     KVC_HIP(hipGetLastError());
-    if (d_counts) return kvc_histogram(d_sym, NB * BS * stride, d_counts, stream_);
+    if (want_counts && !counted) return kvc_histogram(d_sym, NB * BS * stride, d_counts, stream_);
     return 0;
 }
 

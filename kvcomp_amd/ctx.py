@@ -233,7 +233,8 @@ class KVCompCtx:
     def _device_state(self) -> torch.Tensor:
         if self._state is None:
             self._state = torch.zeros(16, dtype=torch.int32, device=self.device)
-            self._state[8] = self._encoded.used
+            if self._encoded.used:
+                self._state[8] = self._encoded.used
         return self._state
 
     def _bookkeeping(self):
@@ -245,6 +246,13 @@ class KVCompCtx:
         to the front of the tail) and the error is raised."""
         if self._enc_pending == 0:
             return
+        p = self._probe
+        if p is not None and p[1] == len(self._unverified):     # a copy of the device words behind the last store is on its way
+            p[0].synchronize()
+            if int(self._host_words[1]) == 0:
+                self.waits += 1
+                self.poll_stores()
+                return
         self.waits += 1
         try:
             _, max_tile, max_stream, _ = kvcomp_cuda.encode_result(self._state[:8], self._encoded.data.numel())
@@ -292,15 +300,19 @@ class KVCompCtx:
 
     def _issue_probe(self):
         """Ask for a copy of the device words without waiting for it (nothing is asked for while the stream is being
-        recorded into a graph, or while an earlier copy is on its way)."""
-        if self._probe is not None or not self._unverified or torch.cuda.is_current_stream_capturing():
+        recorded into a graph, or while an earlier copy is on its way on another stream; one on this stream is replaced
+        by the newer one, which arrives after it in the same place and covers more stores)."""
+        if not self._unverified or torch.cuda.is_current_stream_capturing():
+            return
+        stream = torch.cuda.current_stream(self.device)
+        if self._probe is not None and self._probe[2] != stream:
             return
         if self._host_words is None:
             self._host_words = torch.empty(16, dtype=torch.int32, pin_memory=True)
         self._host_words.copy_(self._state, non_blocking=True)
         ev = torch.cuda.Event()
-        ev.record()
-        self._probe = (ev, len(self._unverified))
+        ev.record(stream)
+        self._probe = (ev, len(self._unverified), stream)
 
     def poll_stores(self):
         """Look, without waiting, at what the stores queued by async_store have left: sizes and size hints are brought
@@ -309,12 +321,12 @@ class KVCompCtx:
         p = self._probe
         if p is None or not p[0].query():
             return
-        w = self._host_words
-        if int(w[1]) != 0:
+        w = self._host_words.tolist()
+        self._probe = None
+        if w[1] != 0:
             self._sync_sizes()                                 # takes the stores back and raises, with the library's message
             return
-        self._probe = None
-        self._accept(p[1], int(w[8]), int(w[2]), int(w[3]))
+        self._accept(p[1], w[8], w[2], w[3])
         self._issue_probe()
 
     def _append_encoded(self, encoded_: torch.Tensor):
@@ -444,10 +456,9 @@ class KVCompCtx:
             self._store_fused(to_compress, mask)
             return None
         blocked = to_compress.reshape(-1, self.block_size, self.batch_size, self.head_num, self.head_dim)
-        quant_ints, min_ints, quant_scale = quant(blocked, self.quant_dims, self.quant_scale_rel)
         if self.encode_codebook is None and self.device_codebook:
-            self._first_chunk_on_device(quant_ints, min_ints, quant_scale)
-            return quant_ints
+            return self._first_chunk(blocked)
+        quant_ints, min_ints, quant_scale = quant(blocked, self.quant_dims, self.quant_scale_rel)
         sizes = kvcomp_cuda.calculate_buffer_size(quant_ints, self.is_k, self.head_num, self.head_dim)
         KVCompCtx.buffer_ctx_len[self.device] = to_compress.shape[0]
         bi_buf, ti_buf, idx_buf, payload_buf = self._scratch(sizes)
@@ -473,8 +484,8 @@ class KVCompCtx:
         self.compressed_ctx_len += quant_ints.shape[0] * quant_ints.shape[1]
         return quant_ints
 
-    # The first chunk's codebook is built on the device (histogram, Huffman code, tables: no 256 reads of single counts
-    # by the host and no wait before the encode is queued); False: by the host builder, as in the reference.
+    # The first chunk's codebook comes from counts that the quantizer takes while it writes the symbols; False: from a
+    # histogram pass over them, as in the reference.
     device_codebook = True
     # With a codebook in place, store(want_symbols=False) queues the fused quantize + encode and returns without
     # waiting for it: sizes and errors are learnt the next time something asks for them (encoded_data, get_cr, ...),
@@ -486,10 +497,11 @@ class KVCompCtx:
     # stores of up to this many blocks are queued without a wait; longer ones (a second chunk of a prompt) are waited for
     ASYNC_KEEP_BLOCKS = 8
 
-    def _encode_direct(self, T: int, *, tables, table_bytes, symbols=None, cache=None, mask=0, meta=None,
-                       min_ints=None, quant_scale=None, keep=None, lost_if_dropped=False):
+    def _encode_direct(self, T: int, *, tables, table_bytes, symbols=None, cache=None, mask=0, most_bytes=None, keep=None,
+                       lost_if_dropped=False):
         """Queue one encode whose outputs go straight to their final places in this context's buffers; nothing waits.
-        Quantizes `cache` on the fly (fused store) or takes `symbols` with their min_ints / quant_scale."""
+        Quantizes `cache` on the fly (fused store) or takes `symbols` whose parameters are in place already.  most_bytes:
+        what the payload is known not to exceed."""
         nb = T // self.block_size
         B, H, D = self.batch_size, self.head_num, self.head_dim
         sizes = kvcomp_cuda.buffer_sizes(T, B * H * D, self.is_k, H, D)
@@ -502,18 +514,15 @@ class KVCompCtx:
         ti = self._thread_infos.reserve(sizes[1], (), torch.uint8, self.device)
         mn = self._min_ints.reserve(nb, gshape[1:], torch.int8, self.device)
         sc = self._scales.reserve(nb, gshape[1:], torch.float16, self.device)
-        worst = T * B * H * D                                  # the reference's pre-allocation: a byte per symbol
+        worst = T * B * H * D if most_bytes is None else most_bytes       # the reference's pre-allocation: a byte per symbol
         if (self._encoded.data is None or
                 self._encoded.used + self._enc_pending + worst > self._encoded.data.numel()):
             self._sync_sizes()                                 # growing copies the filled part: it has to be known
             self._encoded.reserve(worst, (), torch.uint8, self.device)
-        if cache is None:
-            mn.copy_(min_ints)
-            sc.copy_(quant_scale)
         kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
                                  table_bytes=table_bytes, block_infos=bi, thread_infos=ti, encoded=self._encoded.data,
                                  symbols=symbols, cache=cache, quant_mask=mask, eb=self.quant_scale_rel, min_ints=mn, scales=sc,
-                                 codebook_meta=meta, stream_bytes=state[8:9], result=state[:8])
+                                 stream_bytes=state[8:9], result=state[:8])
         self._block_infos.used += sizes[0]
         self._thread_infos.used += sizes[1]
         self._min_ints.used += nb
@@ -522,30 +531,33 @@ class KVCompCtx:
         self.compressed_ctx_len += T
         self._unverified.append((T, keep, self._bookkeeping(), worst, lost_if_dropped))
 
-    def _first_chunk_on_device(self, quant_ints, min_ints, quant_scale):
-        """Codebook of the first stored chunk (kvcomp_encode.py:99-103) and its encode, queued back to back on the
-        device: histogram -> Huffman code and tables (kvc_build_codebook_device) -> encode with the table where it lies.
-        The host then reads the sizes (one wait) and keeps the codebook in the reference's form."""
-        counts = kvcomp_cuda.symbol_counts_chunks(quant_ints.reshape(-1), 1)
-        if self.codebook_smoothing:
-            counts[0, :self._smoothed_symbols()] += 1
-        T = quant_ints.shape[0] * quant_ints.shape[1]
-        for fmt in (kvcomp_cuda.TREE_I8, kvcomp_cuda.TREE_I16):
-            enc, trees, meta = kvcomp_cuda.build_codebook_device(counts, fmt)
-            self._encode_direct(T, tables=enc, table_bytes=enc.shape[1], symbols=quant_ints, meta=meta, min_ints=min_ints,
-                                quant_scale=quant_scale)
-            self._trim_after_sync = True                       # a byte per symbol was reserved
-            try:
-                self._sync_sizes()                             # (a failure leaves the context as it was before the encode)
-                break
-            except KvcompError:
-                # status 4: the code does not fit the int8 tree (kvc_build_codebook_device) -- once more with the wide one
-                if fmt == kvcomp_cuda.TREE_I8 and int(meta[0, 3]) == 4:
-                    continue
-                raise
-        shift, enc_bytes, dec_bytes, status = (int(v) for v in meta[0].cpu())
-        assert status == 0 and shift == 0, "shift must be 0"
-        self._set_codebook(enc[0, :enc_bytes].cpu(), trees[0, :dec_bytes].cpu(), tree_format=fmt)
+    def _first_chunk(self, blocked: torch.Tensor) -> torch.Tensor:
+        """The first stored chunk: quantized, its codebook built from the symbols just written (kvcomp_encode.py:86-103; the
+        one thing that is waited for) and encoded with it.  The counts and the code lengths bound the payload to within a
+        byte per lane stream, so the buffer is as large as the stream needs, and with them at hand neither a symbol without
+        a code nor too small a buffer is possible; with codes of at most seven bits nor is a tile beyond 8191 bytes, so
+        the encode need not be waited for either."""
+        nb, T, device = blocked.shape[0], blocked.shape[0] * self.block_size, self.device
+        gshape = mask_keepdim_shape(blocked.shape, self._mask)
+        min_ints = self._min_ints.reserve(nb, gshape[1:], torch.int8, device)
+        quant_scale = self._scales.reserve(nb, gshape[1:], torch.float16, device)
+        sym, book = kvcomp_cuda.quant_codebook(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale,
+                                               self._smoothed_symbols() if self.codebook_smoothing else 0)
+        self.waits += 1
+        enc, dec = kvcomp_cuda.put_codebook(book, device)
+        vectors = T * self.batch_size * self.head_num * self.head_dim // (self.head_dim if self.is_k else kvcomp_cuda.V_VEC_LEN)
+        cannot_fail = book.max_code_bits <= 7
+        small = T <= self.ASYNC_KEEP_BLOCKS * self.block_size
+        queued = self.async_store and (cannot_fail or small)
+        self._encode_direct(T, symbols=sym, tables=enc, table_bytes=enc.numel(), most_bytes=book.payload_bits // 8 + vectors + 1,
+                            keep=blocked.flatten(0, 1).clone() if queued and not cannot_fail else None)
+        if queued:
+            self._issue_probe()
+        else:
+            self._sync_sizes()                                 # (a failure leaves the context as it was before the encode)
+        self.tree_format, self.max_code_bits = book.tree_format, book.max_code_bits
+        self.encode_codebook, self.decode_codebook = enc, dec
+        return sym
 
     def _smoothed_symbols(self) -> int:
         return min(256, int(math.ceil(1.0 / self.quant_scale_rel)) + 3)      # symbols 0 .. ceil(1 / eb) + 2

@@ -138,6 +138,35 @@ def build_codebook_device(counts: torch.Tensor, tree_format: int = TREE_I8):
     return enc, trees, meta
 
 
+def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: float, min_ints: torch.Tensor, scales: torch.Tensor,
+                   smoothed_symbols: int):
+    """kvc_quant_codebook on a device fp16 [NB, BS, B, H, D] tensor: (symbols uint8 of the same shape, _lib.Codebook).
+    min_ints (int8) and scales (fp16) receive the group parameters.  Waits for the symbol counts only."""
+    _require(blocked.is_cuda and blocked.dtype == torch.float16 and blocked.dim() == 5 and blocked.is_contiguous(),
+             "a contiguous device float16 tensor of shape [NB, BS, B, H, D] is expected")
+    L = _lib.lib()
+    groups = L.kvc_quant_groups(*blocked.shape, quant_mask)
+    _require(min_ints.is_cuda and min_ints.dtype == torch.int8 and min_ints.numel() >= groups, "min_ints: int8 device tensor of the group count")
+    _require(scales.is_cuda and scales.dtype == torch.float16 and scales.numel() >= groups, "scales: fp16 device tensor of the group count")
+    sym = torch.empty(blocked.shape, dtype=torch.uint8, device=blocked.device)
+    book = _lib.Codebook()
+    with torch.cuda.device(blocked.device):
+        check(L.kvc_quant_codebook(_ptr(blocked), *blocked.shape, quant_mask, float(quant_scale_rel), _ptr(sym), _ptr(min_ints),
+                                   _ptr(scales), smoothed_symbols, C.byref(book), _stream(blocked)))
+    return sym, book
+
+
+def put_codebook(book: "_lib.Codebook", device):
+    """(encode table, decode tree) of a _lib.Codebook as device uint8 tensors, copied in stream order; nothing waits."""
+    enc_bytes, dec_bytes = book.encode_bytes, book.decode_bytes
+    at = (enc_bytes + 15) // 16 * 16                     # one allocation, the tree on a 16-byte boundary
+    both = torch.empty(at + dec_bytes, dtype=torch.uint8, device=device)
+    packed = C.string_at(C.addressof(book.encode_table), enc_bytes).ljust(at, b"\0") + C.string_at(C.addressof(book.decode_tree), dec_bytes)
+    with torch.cuda.device(device):
+        check(_lib.lib().kvc_put_bytes(_ptr(both), packed, len(packed), _stream(both)))
+    return both[:enc_bytes], both[at:]
+
+
 def _entropy_encode(is_k, input, encode_code_book, block_infos, thread_infos, idx_offset, encoded_data,
                     base_global_offset, head_num, head_dim):
     for t, n in ((input, "input"), (encode_code_book, "encode_code_book"), (block_infos, "block_infos"),
