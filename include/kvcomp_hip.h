@@ -425,6 +425,26 @@ int kvc_put_bytes(void *d_dst, const void *h_src, int64_t bytes, void *stream);
 int kvc_quant_error(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                     float eb, void *d_xhat_f16, void *stream);
 
+/* ---- the dense caches of the simulated-quantization backend (models/cache/kvcomp_quant.py:14-124) -------------
+ * fp16 [batch, heads, capacity, head_dim] each.
+ * kvc_append_dense: `tokens` new tokens to positions `at` .. of both caches: values as they are, keys rotated
+ *   (apply_rotary_pos_emb_single, utils/compute.py:25-33: t * cos + rotate_half(t) * sin, every product and the sum
+ *   rounded to fp16) unless d_cos and d_sin are NULL.  Strides in elements; the head_dim elements of a row are adjacent.
+ * kvc_quant_in_place: quant_error (utils/compute.py:108-133) on `tokens` tokens (whole blocks) where they lie: element
+ *   (b, h, t, d) at d_x_f16[b * stride_b + h * stride_h + t * head_dim + d]; KVC_MASK_CHANNEL, _VECTOR, _SIM_TOKEN or
+ *   _SIM_BLOCK groups, results bit for bit kvc_quant_error's.  Returns 1, having done nothing, for a layout it does not
+ *   take (head_dim not a multiple of 8 or above 128, rows off 16-byte boundaries, groups beyond a workgroup's registers). */
+typedef struct kvc_append_job {
+    const void *d_k, *d_v, *d_cos, *d_sin;
+    void *d_k_cache, *d_v_cache;
+    int64_t batch, heads, tokens, head_dim, capacity, at;
+    int64_t k_stride_b, k_stride_h, k_stride_t, v_stride_b, v_stride_h, v_stride_t;
+    int64_t cos_stride_b, cos_stride_t, sin_stride_b, sin_stride_t;
+} kvc_append_job;
+int kvc_append_dense(const kvc_append_job *job, void *stream);
+int kvc_quant_in_place(void *d_x_f16, int64_t batch, int64_t heads, int64_t tokens, int64_t head_dim, int64_t stride_b,
+                       int64_t stride_h, int64_t block_size, int quant_mask, float eb, void *stream);
+
 /* ---- dequantizer: (sym + min_i) * scale (models/cache/kvcomp_encode.py:146,161) --------------------
  * d_out fp16 = RN16(f32(sym + min_i) * f32(scale)), same shape as d_sym. */
 int kvc_dequant(const uint8_t *d_sym, const int8_t *d_min_i8, const void *d_scale_f16,

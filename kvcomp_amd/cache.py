@@ -26,7 +26,7 @@ from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
-from .compute import apply_rotary_pos_emb_single, blocks_to_compress, quant_dequant_sim, safe_cat
+from .compute import append_dense, apply_rotary_pos_emb_single, blocks_to_compress, quant_in_place, safe_cat
 from .ctx import KVCompCacheConfigStatic, KVCompCtx
 
 
@@ -48,7 +48,7 @@ class _DenseHistory:
         self.length = 0
         self.quantized = 0        # leading tokens already replaced by their simulated-quantization values
 
-    def append(self, t: torch.Tensor):
+    def make_room(self, t: torch.Tensor):
         n = t.shape[2]
         if self.data is None or self.length + n > self.data.shape[2]:
             cap = max(2 * (self.length + n), 256)
@@ -56,14 +56,17 @@ class _DenseHistory:
             if self.data is not None:
                 grown[:, :, :self.length].copy_(self.data[:, :, :self.length])
             self.data = grown
+
+    def append(self, t: torch.Tensor):
+        self.make_room(t)
+        n = t.shape[2]
         self.data[:, :, self.length:self.length + n].copy_(t)
         self.length += n
 
     def quantize_blocks(self, block_size, recent_size, eb, mode):
         n = blocks_to_compress(self.length - self.quantized, block_size, recent_size)
         if n > 0:
-            region = self.data[:, :, self.quantized:self.quantized + n * block_size]
-            region.copy_(quant_dequant_sim(region, block_size, eb, mode))
+            quant_in_place(self.data[:, :, self.quantized:self.quantized + n * block_size], block_size, eb, mode)
             self.quantized += n * block_size
 
     def view(self, lo=0, hi=None, empty_is_none=False):
@@ -71,6 +74,29 @@ class _DenseHistory:
         if self.data is None or (empty_is_none and hi <= lo):
             return None
         return self.data[:, :, lo:hi]
+
+
+class _LayerViews(list):
+    """A per-layer list of views into the dense caches, made when they are looked at: an update then costs no tensor views
+    that its caller does not use."""
+
+    def __init__(self, histories, make):
+        super().__init__([None] * len(histories))
+        self._histories, self._make = histories, make
+
+    def __getitem__(self, i):
+        if isinstance(i, slice):
+            return [self[j] for j in range(*i.indices(len(self)))]
+        return self._make(self._histories[i])
+
+    def __iter__(self):
+        return (self._make(h) for h in self._histories)
+
+    def __reversed__(self):
+        return (self._make(h) for h in reversed(self._histories))
+
+    def __repr__(self):
+        return repr(list(self))
 
 
 class KVCompCachePytorchQuant:
@@ -82,35 +108,43 @@ class KVCompCachePytorchQuant:
         self.batch_size = batch_size
         self.head_num = head_num
         self.head_dim = head_dim
-        self.compressed_k_cache: List[Optional[torch.Tensor]] = [None] * layer_num
-        self.compressed_v_cache: List[Optional[torch.Tensor]] = [None] * layer_num
-        self.k_cache_buffer: List[Optional[torch.Tensor]] = [None] * layer_num
-        self.v_cache_buffer: List[Optional[torch.Tensor]] = [None] * layer_num
-        self.coss: List[Optional[torch.Tensor]] = [None] * layer_num
-        self.sins: List[Optional[torch.Tensor]] = [None] * layer_num
         self._k = [_DenseHistory() for _ in range(layer_num)]
         self._v = [_DenseHistory() for _ in range(layer_num)]
+        # (the reference's compressed caches stay None until a block has been quantized; its tails can be empty)
+        quantized, tail = (lambda h: h.view(0, h.quantized, empty_is_none=True)), (lambda h: h.view(h.quantized))
+        self.compressed_k_cache: List[Optional[torch.Tensor]] = _LayerViews(self._k, quantized)
+        self.compressed_v_cache: List[Optional[torch.Tensor]] = _LayerViews(self._v, quantized)
+        self.k_cache_buffer: List[Optional[torch.Tensor]] = _LayerViews(self._k, tail)
+        self.v_cache_buffer: List[Optional[torch.Tensor]] = _LayerViews(self._v, tail)
+        self.coss: List[Optional[torch.Tensor]] = [None] * layer_num
+        self.sins: List[Optional[torch.Tensor]] = [None] * layer_num
 
     # -- helpers ---------------------------------------------------------------------------------------
-    def _rope_in(self, key_states, layer_idx, cache_kwargs):
+    def _append(self, key_states, value_states, layer_idx, cache_kwargs):
+        """The new tokens behind both histories of the layer, in one launch where the tensors allow it; keys rotated,
+        unless they are stored un-rotated with the angles beside them.  """
         cos, sin = cache_kwargs['cos'], cache_kwargs['sin']
-        if _config().enable_pre_rope:                  # keys are stored un-rotated, the angles beside them
+        k, v = self._k[layer_idx], self._v[layer_idx]
+        if _config().enable_pre_rope:
             self.coss[layer_idx] = safe_cat(self.coss[layer_idx], cos, dim=1)
             self.sins[layer_idx] = safe_cat(self.sins[layer_idx], sin, dim=1)
-            return key_states
-        return apply_rotary_pos_emb_single(key_states, cos, sin)
+            cos = sin = None
+        k.make_room(key_states)
+        v.make_room(value_states)
+        if k.length == v.length and append_dense(key_states, value_states, cos, sin, k.data, v.data, k.length):
+            k.length += key_states.shape[2]
+            v.length += value_states.shape[2]
+            return
+        if cos is not None:
+            key_states = apply_rotary_pos_emb_single(key_states, cos, sin)
+        k.append(key_states)
+        v.append(value_states)
 
     def _publish(self, layer_idx):
-        k, v = self._k[layer_idx], self._v[layer_idx]
-        # (the reference's compressed caches stay None until a block has been quantized; its tails can be empty)
-        self.compressed_k_cache[layer_idx] = k.view(0, k.quantized, empty_is_none=True)
-        self.compressed_v_cache[layer_idx] = v.view(0, v.quantized, empty_is_none=True)
-        self.k_cache_buffer[layer_idx] = k.view(k.quantized)
-        self.v_cache_buffer[layer_idx] = v.view(v.quantized)
-        keys = k.view()
+        keys = self._k[layer_idx].view()
         if _config().enable_pre_rope:
             keys = apply_rotary_pos_emb_single(keys, self.coss[layer_idx], self.sins[layer_idx])
-        return keys, v.view()
+        return keys, self._v[layer_idx].view()
 
     # -- the Cache contract ------------------------------------------------------------------------------
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
@@ -120,19 +154,15 @@ class KVCompCachePytorchQuant:
             assert not cfg.enable_quant, "Disable quant to enable cache collect."
         if cfg.enable_quant is False:
             return self.update_disable(key_states, value_states, layer_idx, cache_kwargs)
-        key_states = self._rope_in(key_states, layer_idx, cache_kwargs)
+        self._append(key_states, value_states, layer_idx, cache_kwargs)
         k, v = self._k[layer_idx], self._v[layer_idx]
-        k.append(key_states)
-        v.append(value_states)
         k.quantize_blocks(cfg.k_block_size, cfg.k_recent_size, cfg.k_quant_scale_rel, cfg.k_quant_mode)
         v.quantize_blocks(cfg.v_block_size, cfg.v_recent_size, cfg.v_quant_scale_rel, cfg.v_quant_mode)
         return self._publish(layer_idx)
 
     def update_disable(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
                        cache_kwargs: Optional[Dict[str, Any]] = None) -> Tuple[torch.Tensor, torch.Tensor]:
-        key_states = self._rope_in(key_states, layer_idx, cache_kwargs)
-        self._k[layer_idx].append(key_states)
-        self._v[layer_idx].append(value_states)
+        self._append(key_states, value_states, layer_idx, cache_kwargs)
         keys, values = self._publish(layer_idx)
         ex = KVCompCacheConfigStatic.extract_cache
         if ex is not None:                              # kvcomp_quant.py:92-100

@@ -4,6 +4,7 @@ Same names and argument meaning as the reference (utils/compute.py:5-143); the q
 as HIP kernels through the C ABI, the tail bookkeeping (`cut_tensor*`, `safe_cat`) is plain tensor slicing.
 """
 import ctypes as C
+import struct
 from enum import Enum
 from typing import List, Optional, Tuple
 
@@ -130,6 +131,59 @@ def quant_dequant_sim(tensor: torch.Tensor, block_size: int, quant_scale_rel: fl
     with torch.cuda.device(x.device):
         check(_lib.lib().kvc_quant_error(_ptr(x), *shape5, mask, float(quant_scale_rel), _ptr(out), _stream(x)))
     return out.permute(0, 2, 1, 3) if heads_inside else out
+
+
+def quant_in_place(region: torch.Tensor, block_size: int, quant_scale_rel: float, quant_mode: QuantMode) -> None:
+    """quant_dequant_sim over a [B, H, T, D] stretch of a dense cache (T a multiple of block_size), where it lies."""
+    B, H, T, D = region.shape
+    if T == 0:
+        return
+    if region.stride(3) == 1 and region.stride(2) == D:
+        with torch.cuda.device(region.device):
+            rc = _lib.lib().kvc_quant_in_place(_ptr(region), B, H, T, D, region.stride(0), region.stride(1), block_size,
+                                               _SIM_PLAN[quant_mode][1], float(quant_scale_rel), _stream(region))
+        if rc == 0:
+            return
+        if rc != 1:
+            check(rc)
+    region.copy_(quant_dequant_sim(region, block_size, quant_scale_rel, quant_mode))
+
+
+# the twenty-two 8-byte fields of kvc_append_job, in order
+_APPEND = struct.Struct("=22q")
+
+
+def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], k_cache: torch.Tensor,
+                 v_cache: torch.Tensor, at: int) -> bool:
+    """kvc_append_dense: k (rotated by cos / sin [1 or B, T, D], unless they are None) and v, [B, H, T, D] fp16, to
+    positions at .. of the [B, H, capacity, D] caches.  False, having done nothing, for tensors it does not take."""
+    B, H, T, D = k.shape
+    f16 = torch.float16
+    if not (k.dtype is f16 and v.dtype is f16 and k.is_cuda and v.is_cuda and D % 2 == 0 and v.shape == k.shape and
+            k.device == v.device == k_cache.device == v_cache.device and k_cache.dtype is f16 and v_cache.dtype is f16 and
+            k_cache.shape == v_cache.shape == (B, H, k_cache.shape[2], D)):
+        return False
+    kb, kh, kt, kd = k.stride()
+    vb, vh, vt, vd = v.stride()
+    if kd != 1 or vd != 1:
+        return False
+    cos_p = sin_p = cb = ct = sb = st = 0
+    if cos is not None:
+        if not (cos.dtype is f16 and sin.dtype is f16 and cos.is_cuda and sin.is_cuda and cos.shape == sin.shape and
+                cos.dim() == 3 and cos.shape[0] in (1, B) and cos.shape[1] == T and cos.shape[2] == D):
+            return False
+        (cb, ct, cd), (sb, st, sd) = cos.stride(), sin.stride()
+        if cd != 1 or sd != 1:
+            return False
+        if cos.shape[0] == 1:
+            cb = sb = 0
+        cos_p, sin_p = cos.data_ptr(), sin.data_ptr()
+    device = k.device
+    job = _APPEND.pack(k.data_ptr(), v.data_ptr(), cos_p, sin_p, k_cache.data_ptr(), v_cache.data_ptr(), B, H, T, D, k_cache.shape[2], at,
+                       kb, kh, kt, vb, vh, vt, cb, ct, sb, st)
+    with torch.cuda.device(device):
+        check(_lib.lib().kvc_append_dense(job, _stream(k)))
+    return True
 
 
 def quant_error(error_cache, buffer, new_tensor, block_size: int, recent_size: int, quant_scale_rel: float,

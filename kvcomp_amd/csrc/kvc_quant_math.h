@@ -133,3 +133,49 @@ __device__ __forceinline__ uint32_t kvc_low_bytes4(uint32_t a, uint32_t b) { ret
 
 __device__ __forceinline__ float kvc_half_lo(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w & 0xffffu))); }
 __device__ __forceinline__ float kvc_half_hi(uint32_t w) { return __half2float(__ushort_as_half((unsigned short)(w >> 16))); }
+
+// The simulated-quantization values of two elements from kvc_quant_pair_biased's result: u - 1024 is the fp16 symbol the
+// reference keeps un-cast (rint(x / scale) - min, exact), then its two fp16 tensor ops (utils/compute.py:130):
+// (symbol + min) -- the sum of two integers, exact -- times scale, one rounding.
+__device__ __forceinline__ uint32_t kvc_quant_error_pair(uint32_t u, uint32_t min2, uint32_t scale2)
+{
+#pragma clang fp contract(off)
+    const kvc_half2 bias = {(_Float16)1024.f, (_Float16)1024.f};
+    const kvc_half2 sym = __builtin_bit_cast(kvc_half2, u) - bias;
+    const kvc_half2 v = (sym + __builtin_bit_cast(kvc_half2, min2)) * __builtin_bit_cast(kvc_half2, scale2);
+    return __builtin_bit_cast(uint32_t, v);
+}
+// kvc_quant_pair_biased gives the reference's integers where every quotient x / scale of the group stays within +-512
+// (kvc_quant_math.h); the group's smallest and largest quotients say whether it does (false for a zero scale too).
+__device__ __forceinline__ bool kvc_packed_quantizer_applies(const KvcGroupParams &g, float mx)
+{
+    return fabsf(g.min_i) <= 500.f && fabsf(mx * g.rcp) <= 500.f;
+}
+__device__ __forceinline__ uint32_t kvc_half_pair_bits(__half lo, __half hi)
+{
+    return (uint32_t)__half_as_ushort(lo) | ((uint32_t)__half_as_ushort(hi) << 16);
+}
+
+__device__ __forceinline__ float kvc_wave_min(float v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = fminf(v, __shfl_xor(v, off, 64));
+    return v;
+}
+__device__ __forceinline__ float kvc_wave_max(float v)
+{
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
+    return v;
+}
+
+// order-preserving float <-> uint map for atomicMin / atomicMax
+__device__ __forceinline__ uint32_t kvc_f2ord(float f)
+{
+    const uint32_t u = __float_as_uint(f);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float kvc_ord2f(uint32_t o)
+{
+    return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
+}
