@@ -359,6 +359,8 @@ typedef struct kvc_compressed_desc {
  * head_dim] (16-byte aligned, like the tail).  elapsed_ms (may be NULL) makes the call wait. */
 int kvc_restore(int is_k, const kvc_compressed_desc *c, int64_t block_size, void *d_out_f16, int64_t batch,
                 int64_t heads, int64_t head_dim, float *elapsed_ms, void *stream);
+/* Copy whole 16-byte units between device buffers in stream order (a token's rows to the end of a tail). */
+int kvc_copy_rows(void *d_dst, const void *d_src, int64_t bytes, void *stream);
 int64_t kvc_attention_workspace_bytes(int64_t total_tokens, int64_t v_compressed_tokens, int64_t batch,
                                       int64_t q_heads, int64_t head_dim);
 int kvc_attention_decode(const kvc_compressed_desc *k, const kvc_compressed_desc *v, const void *d_q_f16,

@@ -26,8 +26,8 @@ def _ptr(t):
     return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
 
 
-def _stream(dev):
-    return C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+def _stream(t):
+    return C.c_void_p(_lib.stream_of(t))
 
 
 def k_scores(ctx: KVCompCtx, lut: torch.Tensor, q: torch.Tensor, out: Optional[torch.Tensor] = None,
@@ -37,13 +37,13 @@ def k_scores(ctx: KVCompCtx, lut: torch.Tensor, q: torch.Tensor, out: Optional[t
     if out is None:
         out = torch.empty(B, Hq, ctx.compressed_ctx_len, dtype=torch.float32, device=q.device)
     ms = C.c_float(0.0)
-    with torch.cuda.device(q.device):
+    with _lib.device_guard(q):
         check(_lib.lib().kvc_k_scores_lut(
             _ptr(lut), 0, _ptr(ctx.block_infos), ctx.block_infos.numel(), _ptr(ctx.thread_infos), ctx.thread_infos.numel(),
             _ptr(ctx.encoded_data), ctx.encoded_data.numel(), _ptr(ctx.quant_min_ints), _ptr(ctx.quant_scales),
             dims_to_mask(ctx.quant_dims), _ptr(q), _ptr(out), 1 if out.dtype == torch.float32 else 0, ctx.max_tile_bytes,
             ctx.max_stream_bytes, ctx.max_code_bits,
-            ctx.compressed_ctx_len, B, ctx.head_num, Hq, D, C.byref(ms) if timed else None, _stream(q.device)))
+            ctx.compressed_ctx_len, B, ctx.head_num, Hq, D, C.byref(ms) if timed else None, _stream(q)))
     return out, float(ms.value)
 
 
@@ -54,13 +54,13 @@ def v_partials(ctx: KVCompCtx, lut: torch.Tensor, p: torch.Tensor, out: Optional
     if out is None:
         out = torch.empty(T // kvcomp_cuda.V_VEC_LEN, B, Hq, ctx.head_dim, dtype=torch.float32, device=p.device)
     ms = C.c_float(0.0)
-    with torch.cuda.device(p.device):
+    with _lib.device_guard(p):
         check(_lib.lib().kvc_v_partials_lut(
             _ptr(lut), 0, _ptr(ctx.block_infos), ctx.block_infos.numel(), _ptr(ctx.thread_infos), ctx.thread_infos.numel(),
             _ptr(ctx.encoded_data), ctx.encoded_data.numel(), _ptr(ctx.quant_min_ints), _ptr(ctx.quant_scales),
             dims_to_mask(ctx.quant_dims), _ptr(p), _ptr(out), 1 if out.dtype == torch.float32 else 0, ctx.max_tile_bytes,
             ctx.max_stream_bytes, ctx.max_code_bits,
-            T, B, ctx.head_num, Hq, ctx.head_dim, C.byref(ms) if timed else None, _stream(p.device)))
+            T, B, ctx.head_num, Hq, ctx.head_dim, C.byref(ms) if timed else None, _stream(p)))
     return out, float(ms.value)
 
 
@@ -71,6 +71,7 @@ class CompressedAttention:
         assert k_ctx.is_k and not v_ctx.is_k
         self.k, self.v = k_ctx, v_ctx
         self._workspace = None
+        self._workspace_key = None
 
     def _luts(self):
         return self.k.decode_lut(), self.v.decode_lut()
@@ -98,22 +99,28 @@ class CompressedAttention:
         (kvc_attention_decode): scores, softmax and the weighted sum of values never pass through PyTorch.
         `kernel_ms`, if a list, receives (fused K kernel ms, fused V kernel ms) -- which makes the call wait."""
         B, Hq, D = q.shape
-        assert q.dtype == torch.float16 and self.v.ctx_len == self.k.ctx_len
-        scale = scale if scale is not None else 1.0 / math.sqrt(D)
-        k_lut, v_lut = self._luts()
+        k, v = self.k, self.v
+        assert q.dtype is torch.float16 and v.ctx_len == k.ctx_len
+        if scale is None:
+            scale = 1.0 / math.sqrt(D)
         L = _lib.lib()
-        need = int(L.kvc_attention_workspace_bytes(self.k.ctx_len, self.v.compressed_ctx_len, B, Hq, D))
-        if self._workspace is None or self._workspace.numel() < need or self._workspace.device != q.device:
-            self._workspace = torch.empty(need + need // 4, dtype=torch.uint8, device=q.device)
+        # (what the workspace has to hold grows with the tokens: asked for in steps of 1024)
+        key = ((k.ctx_len + 1023) // 1024, B, Hq, D, q.get_device())
+        if key != self._workspace_key:
+            need = int(L.kvc_attention_workspace_bytes(key[0] * 1024, key[0] * 1024, B, Hq, D))
+            if self._workspace is None or self._workspace.numel() < need or self._workspace.device != q.device:
+                self._workspace = torch.empty(need + need // 4, dtype=torch.uint8, device=q.device)
+            self._workspace_key = key
         if out is None:
             out = torch.empty(B, Hq, D, dtype=torch.float32, device=q.device)
-        kd, vd = self._desc(self.k, k_lut), self._desc(self.v, v_lut)
+        kd, vd = k.descriptor(), v.descriptor()
         q = q.contiguous()
-        ms = (C.c_float * 2)()
-        with torch.cuda.device(q.device):
-            check(L.kvc_attention_decode(C.byref(kd), C.byref(vd), _ptr(q), float(scale), _ptr(self._workspace),
-                                         self._workspace.numel(), _ptr(out), B, self.k.head_num, Hq, D, None,
-                                         ms if kernel_ms is not None else None, _stream(q.device)))
+        ms = (C.c_float * 2)() if kernel_ms is not None else None
+        with _lib.device_guard(q):
+            rc = L.kvc_attention_decode(kd, vd, q.data_ptr(), scale, self._workspace.data_ptr(), self._workspace.numel(), out.data_ptr(),
+                                        B, k.head_num, Hq, D, None, ms, _lib.stream_of(q))
+        if rc:
+            check(rc)
         if kernel_ms is not None:
             kernel_ms[:] = [float(ms[0]), float(ms[1])]
         return out

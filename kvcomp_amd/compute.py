@@ -60,7 +60,7 @@ def _ptr(t):
 
 
 def _stream(t):
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return C.c_void_p(_lib.stream_of(t))
 
 
 def quant(tensor: torch.Tensor, quant_dims: List[int], quant_scale_rel: float,
@@ -80,7 +80,7 @@ def quant(tensor: torch.Tensor, quant_dims: List[int], quant_scale_rel: float,
     min_i8 = torch.empty(gshape, dtype=torch.int8, device=tensor.device)
     scale = torch.empty(gshape, dtype=torch.float16, device=tensor.device)
     NB, BS, B, H, D = tensor.shape
-    with torch.cuda.device(tensor.device):
+    with _lib.device_guard(tensor):
         check(_lib.lib().kvc_quant(_ptr(tensor), NB, BS, B, H, D, mask, float(quant_scale_rel), _ptr(sym), _ptr(min_i8),
                                    _ptr(scale), None, _ptr(counts), _stream(tensor)))
     return sym, min_i8, scale
@@ -94,7 +94,7 @@ def dequant(quant_ints: torch.Tensor, min_ints: torch.Tensor, quant_scale: torch
     mask = dims_to_mask(quant_dims)
     NB, BS, B, H, D = quant_ints.shape
     out = torch.empty(quant_ints.shape, dtype=torch.float16, device=quant_ints.device)
-    with torch.cuda.device(quant_ints.device):
+    with _lib.device_guard(quant_ints):
         check(_lib.lib().kvc_dequant(_ptr(quant_ints), _ptr(min_ints.contiguous()), _ptr(quant_scale.contiguous()),
                                      NB, BS, B, H, D, mask, _ptr(out), _stream(quant_ints)))
     return out
@@ -128,7 +128,7 @@ def quant_dequant_sim(tensor: torch.Tensor, block_size: int, quant_scale_rel: fl
         x = tensor.contiguous()
         shape5 = (B * H * NB, block_size, 1, 1, D)
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _lib.device_guard(x):
         check(_lib.lib().kvc_quant_error(_ptr(x), *shape5, mask, float(quant_scale_rel), _ptr(out), _stream(x)))
     return out.permute(0, 2, 1, 3) if heads_inside else out
 
@@ -139,7 +139,7 @@ def quant_in_place(region: torch.Tensor, block_size: int, quant_scale_rel: float
     if T == 0:
         return
     if region.stride(3) == 1 and region.stride(2) == D:
-        with torch.cuda.device(region.device):
+        with _lib.device_guard(region):
             rc = _lib.lib().kvc_quant_in_place(_ptr(region), B, H, T, D, region.stride(0), region.stride(1), block_size,
                                                _SIM_PLAN[quant_mode][1], float(quant_scale_rel), _stream(region))
         if rc == 0:
@@ -178,10 +178,9 @@ def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], 
         if cos.shape[0] == 1:
             cb = sb = 0
         cos_p, sin_p = cos.data_ptr(), sin.data_ptr()
-    device = k.device
     job = _APPEND.pack(k.data_ptr(), v.data_ptr(), cos_p, sin_p, k_cache.data_ptr(), v_cache.data_ptr(), B, H, T, D, k_cache.shape[2], at,
                        kb, kh, kt, vb, vh, vt, cb, ct, sb, st)
-    with torch.cuda.device(device):
+    with _lib.device_guard(k):
         check(_lib.lib().kvc_append_dense(job, _stream(k)))
     return True
 

@@ -266,6 +266,19 @@ __global__ void __launch_bounds__(KVC_WG) kvc_tail_copy_kernel(const uint4 *__re
     for (int64_t i = (int64_t)blockIdx.x * KVC_WG + threadIdx.x; i < n16; i += (int64_t)gridDim.x * KVC_WG) dst[i] = src[i];
 }
 
+// d_dst and d_src 16-byte aligned, bytes a multiple of 16; in stream order, nothing waits
+extern "C" int kvc_copy_rows(void *d_dst, const void *d_src, int64_t bytes, void *stream)
+{
+    KVC_REQUIRE(bytes >= 0 && bytes % 16 == 0 && (((uintptr_t)d_dst | (uintptr_t)d_src) & 15) == 0, "rows off 16-byte boundaries");
+    if (bytes == 0) return 0;
+    KVC_REQUIRE(d_dst != nullptr && d_src != nullptr, "NULL argument");
+    int64_t wgs = (bytes / 16 + KVC_WG - 1) / KVC_WG;
+    if (wgs > 8192) wgs = 8192;
+    hipLaunchKernelGGL(kvc_tail_copy_kernel, dim3((unsigned)wgs), dim3(KVC_WG), 0, (hipStream_t)stream, reinterpret_cast<const uint4 *>(d_src),
+                       reinterpret_cast<uint4 *>(d_dst), bytes / 16);
+    return kvc_check_hip(hipGetLastError(), "kvc_tail_copy_kernel launch");
+}
+
 extern "C" int kvc_restore(int is_k, const kvc_compressed_desc *c, int64_t block_size, void *d_out_f16, int64_t batch,
                            int64_t heads, int64_t head_dim, float *elapsed_ms, void *stream_)
 {
@@ -292,12 +305,8 @@ extern "C" int kvc_restore(int is_k, const kvc_compressed_desc *c, int64_t block
             return rc;
     }
     if (c->tail_tokens) {
-        const int64_t n16 = c->tail_tokens * stride / 8;
-        int64_t wgs = (n16 + KVC_WG - 1) / KVC_WG;
-        if (wgs > 8192) wgs = 8192;
-        hipLaunchKernelGGL(kvc_tail_copy_kernel, dim3((unsigned)wgs), dim3(KVC_WG), 0, stream, reinterpret_cast<const uint4 *>(c->d_tail_f16),
-                           reinterpret_cast<uint4 *>(d_out_f16) + c->tokens * stride / 8, n16);
-        KVC_HIP(hipGetLastError());
+        if (int rc = kvc_copy_rows(reinterpret_cast<__half *>(d_out_f16) + c->tokens * stride, c->d_tail_f16, c->tail_tokens * stride * 2, stream_))
+            return rc;
     }
     return timer.finish();
 }

@@ -194,6 +194,7 @@ class KVCompCtx:
         else:
             assert (batch_size * head_num * head_dim) % kvcomp_cuda.V_VEC_PER_BLK == 0, "hidden size must be divisible by VEC_PER_BLK"
             assert self.block_size % kvcomp_cuda.V_VEC_LEN == 0, "block size must be divisible by VEC_LEN"
+        self._row_bytes = 2 * batch_size * head_num * head_dim
         self._mask = dims_to_mask(self.quant_dims)
         self._groups_per_block = expected_groups(self.block_size, self.block_size, batch_size, head_num, head_dim, self.quant_dims)
         self._descriptor = _lib.CompressedDesc()
@@ -356,7 +357,12 @@ class KVCompCtx:
             if self._tail_len:
                 grown[:self._tail_len] = self._tail[:self._tail_len]
             self._tail = grown
-        self._tail[self._tail_len:self._tail_len + n] = cache
+        row = self._row_bytes
+        to, src = self._tail.data_ptr() + self._tail_len * row, cache.data_ptr()
+        if n and (to | src | row) & 15 == 0 and cache.is_contiguous():
+            kvcomp_cuda.copy_rows(self._tail, to, src, n * row)      # (half the host time of an assignment to a slice)
+        elif n:
+            self._tail[self._tail_len:self._tail_len + n] = cache
         self._tail_len += n
 
     def _tail_drop_front(self, n: int):
@@ -373,10 +379,11 @@ class KVCompCtx:
     quant_scales = property(lambda self: self._scales.view)
 
     def _check(self, cache: torch.Tensor):
-        assert cache.dtype == torch.float16, "cache must be float16"
-        assert cache.shape[1] == self.batch_size, "batch size mismatch"
-        assert cache.shape[2] == self.head_num, "head num mismatch"
-        assert cache.shape[3] == self.head_dim, "head dim mismatch"
+        assert cache.dtype is torch.float16, "cache must be float16"
+        shape = cache.shape
+        assert shape[1] == self.batch_size, "batch size mismatch"
+        assert shape[2] == self.head_num, "head num mismatch"
+        assert shape[3] == self.head_dim, "head dim mismatch"
 
     def _scratch(self, sizes):
         dev = self.device

@@ -43,7 +43,7 @@ def _ptr(t: torch.Tensor):
 
 
 def _stream(t: torch.Tensor):
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return C.c_void_p(_lib.stream_of(t))
 
 
 def _require(cond, msg):
@@ -113,7 +113,7 @@ def symbol_counts_chunks(symbols: torch.Tensor, n_chunks: int) -> torch.Tensor:
     device int64 tensor [n_chunks, 256]; nothing waits for the host."""
     _dev_u8(symbols, "symbols")
     _require(symbols.is_contiguous() and n_chunks > 0 and symbols.numel() % n_chunks == 0, "symbols must split into equal chunks")
-    with torch.cuda.device(symbols.device):
+    with _lib.device_guard(symbols):
         counts = torch.zeros(n_chunks, 256, dtype=torch.int64, device=symbols.device)
         check(_lib.lib().kvc_histogram_chunks(_ptr(symbols), symbols.numel() // n_chunks, n_chunks, _ptr(counts), _stream(symbols)))
     return counts
@@ -130,7 +130,7 @@ def build_codebook_device(counts: torch.Tensor, tree_format: int = TREE_I8):
     n = counts.shape[0]
     cap = int(_lib.lib().kvc_codebook_tree_capacity(tree_format))
     _require(cap > 0, "unknown tree format")
-    with torch.cuda.device(counts.device):
+    with _lib.device_guard(counts):
         enc = torch.empty(n, 2048, dtype=torch.uint8, device=counts.device)
         trees = torch.empty(n, cap, dtype=torch.uint8, device=counts.device)
         meta = torch.empty(n, 4, dtype=torch.int32, device=counts.device)
@@ -150,7 +150,7 @@ def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: floa
     _require(scales.is_cuda and scales.dtype == torch.float16 and scales.numel() >= groups, "scales: fp16 device tensor of the group count")
     sym = torch.empty(blocked.shape, dtype=torch.uint8, device=blocked.device)
     book = _lib.Codebook()
-    with torch.cuda.device(blocked.device):
+    with _lib.device_guard(blocked):
         check(L.kvc_quant_codebook(_ptr(blocked), *blocked.shape, quant_mask, float(quant_scale_rel), _ptr(sym), _ptr(min_ints),
                                    _ptr(scales), smoothed_symbols, C.byref(book), _stream(blocked)))
     return sym, book
@@ -162,7 +162,7 @@ def put_codebook(book: "_lib.Codebook", device):
     at = (enc_bytes + 15) // 16 * 16                     # one allocation, the tree on a 16-byte boundary
     both = torch.empty(at + dec_bytes, dtype=torch.uint8, device=device)
     packed = C.string_at(C.addressof(book.encode_table), enc_bytes).ljust(at, b"\0") + C.string_at(C.addressof(book.decode_tree), dec_bytes)
-    with torch.cuda.device(device):
+    with _lib.device_guard(both):
         check(_lib.lib().kvc_put_bytes(_ptr(both), packed, len(packed), _stream(both)))
     return both[:enc_bytes], both[at:]
 
@@ -179,7 +179,7 @@ def _entropy_encode(is_k, input, encode_code_book, block_infos, thread_infos, id
     _require(idx_offset.numel() >= sizes[2], "idx_offset buffer too small")
     total, max_tile, max_stream = C.c_int64(0), C.c_int64(0), C.c_int64(0)
     fn = _lib.lib().kvc_k_entropy_encode if is_k else _lib.lib().kvc_v_entropy_encode
-    with torch.cuda.device(input.device):
+    with _lib.device_guard(input):
         check(fn(_ptr(input), tokens, stride, _ptr(encode_code_book), encode_code_book.numel(), _ptr(block_infos),
                  _ptr(thread_infos), _ptr(idx_offset), _ptr(encoded_data), encoded_data.numel(),
                  int(base_global_offset) & 0xFFFFFFFF, head_num, head_dim, C.byref(total), C.byref(max_tile), C.byref(max_stream),
@@ -220,7 +220,7 @@ def store_fused(is_k: bool, cache: torch.Tensor, quant_mask: int, quant_scale_re
     _require(min_ints.dtype == torch.int8 and min_ints.numel() >= groups and min_ints.is_cuda, "min_ints: int8 device tensor of the group count")
     _require(scales.dtype == torch.float16 and scales.numel() >= groups and scales.is_cuda, "scales: fp16 device tensor of the group count")
     total, max_tile, max_stream = C.c_int64(0), C.c_int64(0), C.c_int64(0)
-    with torch.cuda.device(cache.device):
+    with _lib.device_guard(cache):
         check(_lib.lib().kvc_store_fused(int(is_k), _ptr(cache), T, B, H, D, quant_mask, float(quant_scale_rel),
                                          _ptr(encode_code_book), encode_code_book.numel(), _ptr(min_ints), _ptr(scales),
                                          _ptr(block_infos), _ptr(thread_infos), _ptr(idx_offset), _ptr(encoded_data),
@@ -245,7 +245,6 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
     job = _lib.EncodeJob()
     job.is_k, job.quant_mask, job.eb = int(is_k), int(quant_mask), float(eb)
     _require((symbols is None) != (cache is None), "give either symbols or cache")
-    dev = (symbols if symbols is not None else cache).device
     if symbols is not None:
         _dev_u8(symbols, "symbols")
         _require(symbols.is_contiguous() and symbols.numel() == tokens * batch * head_num * head_dim, "symbols: wrong size")
@@ -287,15 +286,15 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
         job.d_stream_bytes = stream_bytes.data_ptr()
     if result is not None:
         job.d_result = result.data_ptr()
-    with torch.cuda.device(dev):
-        check(_lib.lib().kvc_encode_async(C.byref(job), C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)))
+    with _lib.device_guard(encoded):
+        check(_lib.lib().kvc_encode_async(C.byref(job), _stream(encoded)))
 
 
 def encode_result(result: torch.Tensor, encoded_cap: int):
     """kvc_encode_result: wait for the stream, raise if any call sharing `result` failed, and return
     (payload bytes of the latest call, largest tile payload, longest lane stream, tiles encoded so far)."""
     total, max_tile, max_stream, tiles = C.c_int64(0), C.c_int64(0), C.c_int64(0), C.c_int64(0)
-    with torch.cuda.device(result.device):
+    with _lib.device_guard(result):
         check(_lib.lib().kvc_encode_result(_ptr(result), encoded_cap, C.byref(total), C.byref(max_tile), C.byref(max_stream),
                                            C.byref(tiles), _stream(result)))
     return total.value, max_tile.value, max_stream.value, tiles.value
@@ -322,7 +321,7 @@ def _entropy_decode(is_k, in_tensor, block_infos, thread_infos, decode_code_book
     tokens, stride = _geometry(out)
     ms = C.c_float(0.0)
     fn = _lib.lib().kvc_k_entropy_decode if is_k else _lib.lib().kvc_v_entropy_decode
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out):
         check(fn(_ptr(in_tensor), in_tensor.numel(), _ptr(block_infos), block_infos.numel(), _ptr(thread_infos),
                  thread_infos.numel(), _ptr(decode_code_book), decode_code_book.numel(), tree_format, _ptr(out),
                  tokens, stride, head_num, head_dim, C.byref(ms), _stream(out)))
@@ -357,7 +356,7 @@ def decode_dequant(is_k: bool, in_tensor, block_infos, thread_infos, decode_code
     _require(quant_min_ints.numel() == groups and quant_scales.numel() == groups,
              "%d minima and %d scales for %d quantization groups" % (quant_min_ints.numel(), quant_scales.numel(), groups))
     ms = C.c_float(0.0)
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out):
         check(_lib.lib().kvc_decode_dequant(int(is_k), _ptr(in_tensor), in_tensor.numel(), _ptr(block_infos), block_infos.numel(),
                                             _ptr(thread_infos), thread_infos.numel(), _ptr(decode_code_book),
                                             decode_code_book.numel(), tree_format, _ptr(quant_min_ints.contiguous()),
@@ -370,9 +369,15 @@ def build_lut(decode_codebook: torch.Tensor, tree_format: int = TREE_I8) -> torc
     """Decode table of one codebook (device uint8 tensor of kvc_lut_bytes() bytes)."""
     L = _lib.lib()
     lut = torch.empty(int(L.kvc_lut_bytes()), dtype=torch.uint8, device=decode_codebook.device)
-    with torch.cuda.device(decode_codebook.device):
+    with _lib.device_guard(decode_codebook):
         check(L.kvc_build_lut(_ptr(decode_codebook), decode_codebook.numel(), tree_format, 1, 0, _ptr(lut), _stream(decode_codebook)))
     return lut
+
+
+def copy_rows(on: torch.Tensor, dst: int, src: int, nbytes: int) -> None:
+    """kvc_copy_rows between two addresses on the device of `on`, on its current stream."""
+    with _lib.device_guard(on):
+        check(_lib.lib().kvc_copy_rows(dst, src, nbytes, _lib.stream_of(on)))
 
 
 def restore(is_k: bool, desc, block_size: int, out: torch.Tensor, with_tail: bool = True) -> float:
@@ -387,7 +392,7 @@ def restore(is_k: bool, desc, block_size: int, out: torch.Tensor, with_tail: boo
         desc.tail_tokens = 0
     _require(T == desc.tokens + desc.tail_tokens, "out holds %d tokens, %d are to be restored" % (T, desc.tokens + desc.tail_tokens))
     ms = C.c_float(0.0)
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out):
         check(_lib.lib().kvc_restore(int(is_k), C.byref(desc), block_size, _ptr(out), B, H, D, C.byref(ms), _stream(out)))
     return ms.value
 
@@ -432,7 +437,7 @@ def _fused(is_k, decode_code_book, block_infos, thread_infos, encoded_data, quan
     _require(quant_min_ints.numel() == n, "quant_min_ints and quant_scales must have the same number of elements")
     ms = C.c_float(0.0)
     fn = _lib.lib().kvc_k_decode_and_mat_vec_mul if is_k else _lib.lib().kvc_v_decode_and_mat_vec_mul
-    with torch.cuda.device(B.device):
+    with _lib.device_guard(B):
         check(fn(_ptr(decode_code_book), decode_code_book.numel(), tree_format, _ptr(block_infos), block_infos.numel(),
                  _ptr(thread_infos), thread_infos.numel(), _ptr(encoded_data), encoded_data.numel(),
                  _ptr(quant_min_ints), _ptr(quant_scales), mask, _ptr(B), _ptr(Cout), tokens, batch, head_num, q_heads,
@@ -468,6 +473,6 @@ def k_mat_vec_mul_cuda_export(k: torch.Tensor, q: torch.Tensor, out: torch.Tenso
         _require(t.dtype == torch.float16, "%s must be of type half" % n)
         _require(t.is_contiguous(), "%s must be contiguous" % n)
     ms = C.c_float(0.0)
-    with torch.cuda.device(k.device):
+    with _lib.device_guard(k):
         check(_lib.lib().kvc_k_mat_vec_mul(_ptr(k), _ptr(q), _ptr(out), ctx, batch, heads, dim, C.byref(ms), _stream(k)))
     return float(ms.value)
