@@ -735,9 +735,9 @@ def main():
     # template arguments: query heads per KV head, then 0 = K tile, 3 / 4 = V tile with the softmax on the fly
     # (4: head_dim is not a multiple of 64, tiles may straddle two heads), then rounded mode
     v_kind = 3 if D % 64 == 0 else 4
-    mfma = kctx.max_code_bits <= 7, vctx.max_code_bits <= 7
-    name = lambda kind, m: ("kvc_fused_mfma_kernel<%d, %d, true>" % (rep, kind)) if m else ("kvc_fused_kernel<%d, %d>" % (rep, kind))
-    dom, dom_ms, dom_bytes = ((name(0, mfma[0]), k_ms, kb) if k_ms >= v_ms else (name(v_kind, mfma[1]), v_ms, vb))
+    # (codes of more than 7 bits: the last template argument)
+    name = lambda kind, ctx: "kvc_fused_mfma_kernel<%d, %d, true, %s>" % (rep, kind, "true" if ctx.max_code_bits > 7 else "false")
+    dom, dom_ms, dom_bytes = ((name(0, kctx), k_ms, kb) if k_ms >= v_ms else (name(v_kind, vctx), v_ms, vb))
     achieved = dom_bytes / dom_ms / 1e6
     value = (kb + vb) / (ms_per_step * 1e-3) / 1e9
     result = {

@@ -302,7 +302,8 @@ int kvc_v_decode_and_mat_vec_mul(const uint8_t *d_decode_tree, int64_t decode_tr
  *                        largest tile payload / longest lane stream in the payload (from the encoder),
  *                        0 = unknown.  They only size the LDS staging; tiles that exceed them are decoded
  *                        from global memory.
- *     max_code_bits:     longest code of the codebook(s), 0 = unknown.  It only sizes the table kept in LDS
+ *     max_code_bits:     longest code of the codebook(s), 0 = unknown; + 256 where every symbol lies below 64 (codes
+ *                        longer than 7 bits then take the matrix-core kernels too).  It only sizes the table kept in LDS
  *                        (fewer bytes, more waves per CU); a codebook with longer codes than stated still
  *                        decodes correctly, on the slow path. */
 int64_t kvc_lut_bytes(void);

@@ -27,7 +27,7 @@ constexpr int KVC_STAGE_WORDS = KVC_STAGE_BYTES / 4;
 // ---------------------------------------------------------------------------------------------------
 // decode look-up table (built on the device from the decode tree, see kvc_lut.hip)
 //
-//   header   {lbits, lmax, n_long, group, fused_group, fused_check, OR of the symbols' fp16 bit patterns, 0}
+//   header   {lbits, lmax, n_long, group, fused_group, fused_check, OR of the symbols' fp16 bit patterns, n_esc}
 //   long[ ]  codes longer than lbits: {code left-aligned in 32 bits, len | sym << 8}
 //   entry[ ] 1 << lbits words indexed by the next lbits stream bits: len | sym << 8, or 0 when the
 //            code is longer than lbits (search long[]) or the bits match no code.
@@ -36,6 +36,8 @@ constexpr int KVC_STAGE_WORDS = KVC_STAGE_BYTES / 4;
 //            length in its lowest mantissa byte (zero for any integer <= 255, so read as a float the entry
 //            is the symbol to within 4e-6 relative, read as a shift count it is the length).  Indices
 //            whose code is longer than lbits or that match no code hold "symbol 0, length 1".
+//   esc[ ]   the n_esc codes longer than 7 bits (at most 64 are listed): {code, first stream bit in bit 0; len | sym << 8},
+//            for the loops whose table index has 7 bits
 //   group    how many symbols may be decoded from one 32-bit window: floor(32 / lmax), one of 8,4,2,1.
 //   fused_group / fused_check
 //            the same for the fused kernels, whose window has 30 usable bits: 8 if lmax <= 3, 4 if
@@ -49,8 +51,10 @@ constexpr int KVC_LUT_HEADER_WORDS = 8;
 constexpr int KVC_LUT_LONG_WORDS = 2 * KVC_LUT_MAX_LONG;
 constexpr int KVC_LUT_ENTRY_WORDS = 1 << KVC_LUT_MAX_BITS;
 constexpr int KVC_LUT_FENTRY_OFFSET = KVC_LUT_HEADER_WORDS + KVC_LUT_LONG_WORDS + KVC_LUT_ENTRY_WORDS;
-constexpr int KVC_LUT_WORDS = KVC_LUT_FENTRY_OFFSET + KVC_LUT_ENTRY_WORDS;
-constexpr int KVC_LUT_BYTES = KVC_LUT_WORDS * 4;          // 10272
+constexpr int KVC_LUT_ESC_OFFSET = KVC_LUT_FENTRY_OFFSET + KVC_LUT_ENTRY_WORDS;
+constexpr int KVC_LUT_ESC_BITS = 7, KVC_LUT_ESC_MAX = 64;
+constexpr int KVC_LUT_WORDS = KVC_LUT_ESC_OFFSET + 2 * KVC_LUT_ESC_MAX;
+constexpr int KVC_LUT_BYTES = KVC_LUT_WORDS * 4;          // 10784
 constexpr int KVC_TREE_MAX_NODES = 512;                   // 2 * 256 symbols - 2, rounded up
 
 // ---------------------------------------------------------------------------------------------------
@@ -72,8 +76,11 @@ struct KvcDecodeHints {
     const uint32_t *luts;          // tables from kvc_build_lut; NULL: derived from the decode tree per call
     int64_t rows_per_codebook;
     int64_t max_tile_bytes, max_stream_bytes;
-    int max_code_bits;
+    int code_hint;                 // as kvc_compressed_desc::max_code_bits
 };
+// kvc_compressed_desc::max_code_bits: the longest code, and whether every symbol is known to lie below 64
+static inline int kvc_hint_bits(int64_t hint) { return (int)(hint & 0xff); }
+static inline bool kvc_hint_small_alphabet(int64_t hint) { return (hint & 0x100) != 0; }
 int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_tree_bytes, int tree_format,
                const uint8_t *d_block_infos, int64_t block_infos_bytes, const uint8_t *d_thread_infos,
                int64_t thread_infos_bytes, const uint8_t *d_encoded, int64_t encoded_bytes, const int8_t *d_min,

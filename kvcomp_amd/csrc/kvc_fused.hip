@@ -618,6 +618,64 @@ __device__ __forceinline__ void kvc_fast_emit2(const uint32_t *stage, uint32_t &
     }
 }
 
+// The same for codebooks with codes of more than 7 bits (see kvc_mfma_dot_long): 8 symbols per refill through a table of 7
+// index bits with four-byte entries, in which the prefixes of longer codes hold zero; those are looked for in the list at
+// esc_addr.  entry_of(symbol) makes the upper part of a table entry.
+template <bool SKEW, class Put, class Entry>
+__device__ __forceinline__ void kvc_fast_emit_long(const uint32_t *stage, uint32_t &u, uint32_t fentry_base, uint32_t mask4, uint32_t esc_addr,
+                                                   uint32_t nesc, int i0, int n, Put &&put, Entry &&entry_of)
+{
+    const uint32_t sbase = (uint32_t)(uintptr_t)(const kvc_lds_word *)stage;
+#pragma unroll 1
+    for (int i = i0; i < i0 + n; i += 8) {
+        uint32_t lo, hi;
+        auto refill = [&]() {
+            const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
+            const uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2];
+            lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
+        };
+        refill();
+        uint32_t R = lo, es = 0;
+        kvc_static_for<8>([&](auto g_) {
+            constexpr int g = decltype(g_)::value;
+            if (g == 4) {
+                es &= 0xffu;
+                R = __builtin_amdgcn_alignbit(hi, lo, es);
+                u += es;
+                es = 0;
+            }
+            uint32_t e = *(const kvc_lds_u32 *)(uintptr_t)((R & mask4) | fentry_base);
+            if (__builtin_expect(__any(e == 0u), 0)) {           // wave-uniform
+                u += es & 0xffu;
+                refill();
+                const uint32_t win = __builtin_amdgcn_alignbit(hi, lo, 2u);
+                uint32_t len = e & 0xffu;
+                if (e == 0u) {
+                    len = 1u;                                    // (bits that match no code: symbol 0)
+                    e = entry_of(0u);
+                    for (uint32_t j = 0; j < nesc; j++) {
+                        const kvc_lds_u32 *c = (const kvc_lds_u32 *)(uintptr_t)(esc_addr + 8u * j);
+                        const uint32_t l = c[1] & 0xffu;
+                        if (((win ^ c[0]) << (32u - l)) == 0u) {
+                            len = l;
+                            e = entry_of((c[1] >> 8) & 0xffu);
+                        }
+                    }
+                }
+                u += len;
+                es = 0;
+                refill();
+                R = lo;
+            } else {
+                if (g != 3 && g != 7) R = __builtin_amdgcn_alignbit(R, R, e);
+                es += e;
+            }
+            put(i, g_, e);
+        });
+        u += es & 0xffu;
+    }
+}
+
 // One symbol per refill, table and long-code list in global memory (codes beyond the table index, tiles
 // that do not fit the staging area, windows that may overflow); put1(i, symbol as an fp32 pattern).
 template <bool GSRC, class Put>
@@ -666,11 +724,13 @@ struct KvcSlab {
     static constexpr int WORDS = IS_K ? 64 * K_ROW_WORDS : SLAB * 64 * ESZ / 4;
 };
 
+constexpr int KVC_EXPAND_LONG_WORDS = (1 << KVC_LUT_ESC_BITS) + 2 * KVC_LUT_ESC_MAX;
 #ifndef KVC_EXPAND_OCC
 #define KVC_EXPAND_OCC 1
 #endif
-template <int KIND, bool DEQ>
-__global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_kernel(KvcFusedArgs a)
+// LONG: for codebooks with codes of more than 7 bits and symbols below 64
+template <int KIND, bool DEQ, bool LONG>
+__device__ __forceinline__ void kvc_expand_body(const KvcFusedArgs &a)
 {
     constexpr bool IS_K = KIND == 0;
     constexpr int SLOTS = KvcGeom<KIND>::SLOTS;
@@ -691,7 +751,21 @@ __global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_kernel(KvcF
     const int64_t cb = a.s.rows_per_codebook ? row / a.s.rows_per_codebook : 0;
     const uint32_t *__restrict__ lut_g = a.s.luts + cb * KVC_LUT_WORDS;
     const uint32_t lbits = lut_g[0], nlong = lut_g[2];
-    const bool fast_book = nlong == 0 && lbits <= (uint32_t)KVC_LUT_MAX_BITS && (1u << lbits) <= (uint32_t)a.table_words;
+    const uint32_t nesc = LONG ? lut_g[7] : 0u;
+    const bool long_book = LONG && lut_g[1] > (uint32_t)KVC_LUT_ESC_BITS && nesc <= (uint32_t)KVC_LUT_ESC_MAX && a.table_words >= KVC_EXPAND_LONG_WORDS;
+    const bool fast_book = !LONG && nlong == 0 && lbits <= (uint32_t)KVC_LUT_MAX_BITS && (1u << lbits) <= (uint32_t)a.table_words;
+    // the upper part of a table entry: the symbol as fp16 (dequantizing) or as an fp32 pattern
+    auto entry_of = [](uint32_t sym) {
+        return DEQ ? (uint32_t)__half_as_ushort(__float2half_rn((float)sym)) << 16 : __float_as_uint((float)sym);
+    };
+    if (long_book) {
+        const uint32_t *entries = lut_g + KVC_LUT_HEADER_WORDS + KVC_LUT_LONG_WORDS;         // first stream bit in the index's top bit
+        for (uint32_t i = tid; i < (1u << KVC_LUT_ESC_BITS); i += KVC_WG) {
+            const uint32_t e = entries[(__brev(i) >> (32 - KVC_LUT_ESC_BITS)) << (lbits - KVC_LUT_ESC_BITS)], len = e & 0xffu;
+            s_fentry[i] = len == 0u || len > (uint32_t)KVC_LUT_ESC_BITS ? 0u : entry_of((e >> 8) & 0xffu) | len;
+        }
+        for (uint32_t i = tid; i < 2 * nesc; i += KVC_WG) s_fentry[(1 << KVC_LUT_ESC_BITS) + i] = lut_g[KVC_LUT_ESC_OFFSET + i];
+    }
     if (fast_book)
         for (uint32_t i = tid; i < (1u << lbits); i += KVC_WG) {
             uint32_t e = lut_g[KVC_LUT_FENTRY_OFFSET + i];
@@ -703,10 +777,10 @@ __global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_kernel(KvcF
     if (lane < KVC_PACK_LEAD) pack[lane] = 0;
     if (a.row_words) rows[lane * a.row_words] = 0;
     __syncthreads();
-    const uint32_t mask4 = ((1u << lbits) - 1u) << 2;
+    const uint32_t mask4 = ((1u << (LONG ? (uint32_t)KVC_LUT_ESC_BITS : lbits)) - 1u) << 2;
     const int n = IS_K ? D : KVC_V_TOKENS;
     const uint32_t fe = (uint32_t)(uintptr_t)(kvc_lds_u32 *)s_fentry;
-    const bool fast_loop = fast_book && lut_g[1] <= 7u && n % 8 == 0;     // four codes of <= 7 bits fit a half window
+    const bool fast_loop = LONG ? long_book : fast_book && lut_g[1] <= 7u && n % 8 == 0;     // four codes of <= 7 bits fit a half window
     const bool wide16 = DEQ || (D & 15) == 0;                 // K rows start on 16-byte boundaries
     const uint32_t lb = 2u;
 
@@ -774,7 +848,11 @@ __global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_kernel(KvcF
         };
         for (int i0 = 0; i0 < n; i0 += S::SLAB) {
             const int len = n - i0 < S::SLAB ? n - i0 : S::SLAB;
-            if (fast) {
+            if (LONG && fast) {
+                const uint32_t esc = fe + (4u << KVC_LUT_ESC_BITS);
+                if (skew) kvc_fast_emit_long<true>(words, u, fe, mask4, esc, nesc, i0, len, put, entry_of);
+                else kvc_fast_emit_long<false>(words, u, fe, mask4, esc, nesc, i0, len, put, entry_of);
+            } else if (fast) {
                 if (skew) kvc_fast_emit2<4, true>(words, u, fe, mask4, i0, len, put);
                 else kvc_fast_emit2<4, false>(words, u, fe, mask4, i0, len, put);
             } else if (st.fits) {
@@ -825,6 +903,18 @@ __global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_kernel(KvcF
     }
 }
 
+template <int KIND, bool DEQ>
+__global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_kernel(KvcFusedArgs a)
+{
+    kvc_expand_body<KIND, DEQ, false>(a);
+}
+// (K: V's groups are so large that few of its codebooks have such codes)
+template <bool DEQ>
+__global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_long_kernel(KvcFusedArgs a)
+{
+    kvc_expand_body<0, DEQ, true>(a);
+}
+
 // ---------------------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------------------
@@ -844,10 +934,12 @@ static void kvc_launch_fused(int kind, const KvcFusedArgs &a, dim3 grid, size_t 
 // from global memory, so the sizes only affect speed.  Everything stays within 64 KiB per workgroup.
 static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_bytes, int64_t tiles,
                            int64_t max_tile_bytes, int64_t max_stream_bytes, int max_code_bits, int64_t extra_words = 0,
-                           bool allow_pairs = true, int64_t mfma_ops_words = 0)
+                           bool allow_pairs = true, int64_t mfma_ops_words = 0, int long_table_words = 0)
 {
+    const int64_t slack = KVC_LDS_SLACK_WORDS + (long_table_words ? KVC_LDS_LONG_SLACK_WORDS : 0);
     const int force_rows = kvc_option(KVC_OPT_FUSED_ROWS);   // 0 / 1 overrides the choice below
     a.table_words = 1 << ((max_code_bits >= 1 && max_code_bits <= KVC_LUT_MAX_BITS) ? max_code_bits : KVC_LUT_MAX_BITS);
+    if (long_table_words) a.table_words = long_table_words;
     if (a.table_words < 4) a.table_words = 4;   // keeps the per-wave areas 16-byte aligned
     // room for the two-symbol table (8 bytes per index of 2 * longest-code bits) when the codes are short
     const int pair_limit = kvc_option(KVC_OPT_FUSED_PAIR_BITS);
@@ -866,7 +958,7 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
     }
     // per wave, besides the payload
     const int64_t ops_words = mfma_ops_words ? mfma_ops_words : (int64_t)slots * 128 * rep + extra_words;
-    const int64_t budget = (65536 / 4 - a.table_words - KVC_LDS_SLACK_WORDS) / KVC_WAVES_PER_WG - ops_words;   // words per wave
+    const int64_t budget = (65536 / 4 - a.table_words - slack) / KVC_WAVES_PER_WG - ops_words;   // words per wave
     const int64_t mean_tile = encoded_bytes / (tiles > 0 ? tiles : 1);
     // without the encoder's figure: tiles hold thousands of symbols, so their sizes stay close to the mean
     int64_t tile_bytes = max_tile_bytes > 0 ? max_tile_bytes : mean_tile + mean_tile / 4 + 256;
@@ -903,7 +995,7 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
     if (use_skew) a.skew = 2;
     a.pack_logical = (int)pack;
     a.pack_words = (int)physical(pack);
-    return 4 * ((size_t)a.table_words + KVC_LDS_SLACK_WORDS +
+    return 4 * ((size_t)a.table_words + (size_t)slack +
                 (size_t)KVC_WAVES_PER_WG * (size_t)(ops_words + a.pack_words + KVC_WAVE * a.row_words));
 }
 
@@ -993,7 +1085,7 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
                      const int8_t *d_min, const void *d_scale, int quant_mask, const void *d_x, void *d_out,
                      int64_t tokens, int64_t batch, int64_t kv_heads, int64_t q_heads, int64_t head_dim,
                      float *elapsed_ms, void *stream_, const uint32_t *d_luts = nullptr, int rows_per_codebook = 0,
-                     int out_f32 = 0, int64_t max_tile_bytes = 0, int64_t max_stream_bytes = 0, int max_code_bits = 0,
+                     int out_f32 = 0, int64_t max_tile_bytes = 0, int64_t max_stream_bytes = 0, int code_hint = 0,
                      const KvcFusedExtra *extra = nullptr)
 {
     hipStream_t stream = (hipStream_t)stream_;
@@ -1044,15 +1136,19 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     const int slots = (!is_k && head_dim % KVC_WAVE != 0) ? 2 : 1;
     const int kind = is_k ? 0 : (a.scores ? 2 : 0) + slots;
     const int rounded = kvc_option(KVC_OPT_FUSED_ROUNDED) != 0;
-    // The matrix-core kernels take the common case: a codebook known to have codes of at most 7 bits, the plain or
+    // The matrix-core kernels take the common case: a codebook whose longest code is known, the plain or
     // skewed packed payload, results that can be stored four at a time.
     const int64_t out_stride = (extra && extra->out_stride) ? extra->out_stride : tokens;
     const int want_mfma = kvc_option(KVC_OPT_FUSED_MFMA);
-    const bool mfma = want_mfma != 0 && max_code_bits >= 1 && max_code_bits <= 7 &&
+    const int max_code_bits = kvc_hint_bits(code_hint);
+    // longer codes: kernels of their own, where a list of at most 64 codes and the entries' format are sure to do
+    const bool long_codes = max_code_bits > KVC_LUT_ESC_BITS;
+    const bool mfma = want_mfma != 0 && max_code_bits >= 1 && (!long_codes || (rounded && kvc_hint_small_alphabet(code_hint) && kind != 1 && kind != 2)) &&
                       kvc_option(KVC_OPT_FUSED_ROWS) != 1 && ((uintptr_t)d_out & 15) == 0 &&
                       (is_k ? out_stride % 4 == 0 : head_dim % 4 == 0);
     const size_t lds = mfma ? kvc_plan_lds(a, slots, (int)rep, encoded_bytes, rows * a.s.cols, max_tile_bytes, max_stream_bytes,
-                                           max_code_bits, 0, true, kvc_mfma_ops_words(slots, (int)rep, rounded))
+                                           max_code_bits, 0, !long_codes, kvc_mfma_ops_words(slots, (int)rep, rounded),
+                                         long_codes ? KVC_LONG_TABLE_WORDS : 0)
                             : kvc_plan_lds(a, slots, rounded ? (int)rep + 1 : (int)rep, encoded_bytes, rows * a.s.cols,
                                            max_tile_bytes, max_stream_bytes, max_code_bits, 0, !rounded);
     a.rounded = rounded;
@@ -1084,7 +1180,8 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
                 a.table_words, a.pack_words, a.pack_logical, a.skew, a.row_words, a.pair_bits, a.s.tiles_per_wave, a.rounded);
     if (mfma) {
         if (trace_plan) fprintf(stderr, "[kvcomp]   matrix-core kernel\n");
-        kvc_launch_fused_mfma((int)rep, kind, rounded != 0, a, grid, lds, stream);
+        if (long_codes) kvc_launch_fused_long((int)rep, kind, a, grid, lds, stream);
+        else kvc_launch_fused_mfma((int)rep, kind, rounded != 0, a, grid, lds, stream);
         KVC_HIP(hipGetLastError());
         return timer.finish();
     }
@@ -1147,8 +1244,10 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
     const int slots = (!is_k && head_dim % KVC_WAVE != 0) ? 2 : 1;
     const int out_words = is_k ? (deq ? KvcSlab<true, true>::WORDS : KvcSlab<true, false>::WORDS)
                                : (deq ? KvcSlab<false, true>::WORDS : KvcSlab<false, false>::WORDS);
+    const int code_bits = kvc_hint_bits(hints.code_hint);
+    const bool long_codes = is_k && code_bits > KVC_LUT_ESC_BITS && kvc_hint_small_alphabet(hints.code_hint) && kvc_option(KVC_OPT_FUSED_ROWS) != 1;
     const size_t lds = kvc_plan_lds(a, slots, deq ? 1 : 0, encoded_bytes, rows * a.s.cols, hints.max_tile_bytes,
-                                    hints.max_stream_bytes, hints.max_code_bits, out_words);
+                                    hints.max_stream_bytes, code_bits, out_words, true, 0, long_codes ? KVC_EXPAND_LONG_WORDS : 0);
     a.expand = deq ? 2 : 1;
     a.out_words = out_words;
     // One tile per wave: measured on MI355X at 65 536 K / 49 152 V tiles, plain decode runs 1.2 to 1.4 times faster
@@ -1163,7 +1262,10 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
     const dim3 grid = kvc_grid(a.s, rows);
     const int kind = is_k ? 0 : slots;
 #define KVC_EXPAND_LAUNCH(K, Q) hipLaunchKernelGGL((kvc_expand_kernel<K, Q>), grid, dim3(KVC_WG), lds, stream, a)
-    if (deq) {
+    if (long_codes) {
+        if (deq) hipLaunchKernelGGL(kvc_expand_long_kernel<true>, grid, dim3(KVC_WG), lds, stream, a);
+        else hipLaunchKernelGGL(kvc_expand_long_kernel<false>, grid, dim3(KVC_WG), lds, stream, a);
+    } else if (deq) {
         if (kind == 0) KVC_EXPAND_LAUNCH(0, true);
         else if (kind == 1) KVC_EXPAND_LAUNCH(1, true);
         else KVC_EXPAND_LAUNCH(2, true);

@@ -80,6 +80,8 @@ constexpr int kvc_fused_mfma_occupancy(int rep, int kind)
     return rep == 1 ? (kind == 0 ? KVC_MFMA_OCC_K1 : (kind == 1 || kind == 3 || kind == 4) ? KVC_MFMA_OCC_V1 + 1 : KVC_MFMA_OCC_V1)
                     : (rep == 4 && kind == 0) ? 6 : kvc_fused_occupancy(rep, kind);
 }
+// the same for codebooks with codes of more than 7 bits (kvc_fused_mfma_long.hip)
+constexpr int kvc_fused_long_occupancy(int rep, int kind) { return rep == 1 ? (kind == 0 ? 7 : 6) : rep == 2 ? 5 : rep == 4 ? 4 : 1; }
 constexpr int KVC_PRE_CHUNKS = 4;     // 16-byte chunks per lane fetched one tile ahead (4 KiB of payload)
 constexpr int KVC_PACK_LEAD = 4;      // zero words in front of the packed payload: bit positions never drop below 2
 
@@ -145,6 +147,8 @@ __device__ __forceinline__ uint32_t kvc_refill_address(uint32_t stage_base, uint
     return (a << 2) + stage_base;
 }
 constexpr int KVC_LDS_SLACK_WORDS = 48;
+// what a lane can run further where codes of up to 32 bits are taken in the same loops
+constexpr int KVC_LDS_LONG_SLACK_WORDS = 96;
 
 // Rounded mode: RN16((sym + min) * scale) as the reference's dequantizer computes it (sym + min exactly, one
 // rounding of the product).  Both steps are fp16 instructions: the sum of two small integers is exact in fp16
@@ -484,4 +488,8 @@ constexpr int kvc_mfma_ops_words(int slots, int rep, bool rounded)
 {
     return slots * (KVC_MFMA_GROUPS * kvc_mfma_sets(rep) * 8 + (rounded ? KVC_MFMA_GROUPS * 4 : 0));
 }
+// codes of more than 7 bits: 128 two-byte entries, then the list of those codes
+constexpr int KVC_LONG_TABLE_WORDS = (1 << KVC_LUT_ESC_BITS) / 2 + 2 * KVC_LUT_ESC_MAX;
+// kinds 0, 3 and 4, rounded arithmetic only
+void kvc_launch_fused_long(int rep, int kind, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);
 void kvc_launch_fused_mfma(int rep, int kind, bool rounded, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);

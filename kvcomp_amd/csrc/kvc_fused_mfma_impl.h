@@ -437,6 +437,82 @@ __device__ __forceinline__ void kvc_mfma_pair_dot(uint32_t sbase, uint32_t &u, u
     }
 }
 
+// Codes of any length, for alphabets of at most 64 symbols: 8 symbols per refill through the two-byte table of 7 index bits
+// (see HALF above), in which the prefixes of longer codes hold zero.  Codes beyond 7 bits are those of symbols that occur
+// next to never (with 23 symbols at error bound 0.05 and per-channel groups one in a million, with one scale per block one
+// in 300): a wave in which a lane meets one leaves the loop's course for it, compares the lane's window with the codes of
+// the list in LDS (esc_addr: {code, length | symbol << 8} each), and starts a new window behind it.  The fp32-FMA kernels,
+// which served these codebooks, look symbols up one per refill in global memory once a code has more than 10 bits:
+// K products of 1 x 32 heads x 128 x 8192 tokens, one scale per block, 68 us.
+template <bool SKEW, int NM, bool ROUNDED, bool BCAST>
+__device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, uint32_t fe, uint32_t mask, uint32_t esc_addr, uint32_t nesc,
+                                                  int n, uint32_t &bptr, uint32_t &msptr, kvc_f4 (&acc)[NM], bool holder)
+{
+    asm volatile("" : "+v"(msptr));
+#pragma unroll 1
+    for (int i = 0; i < n; i += 8) {
+        const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
+        uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2];
+        uint32_t lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
+        uint32_t R = lo, es = 0;
+        uint32_t e[4];
+        kvc_static_for<8>([&](auto g_) {
+            constexpr int g = decltype(g_)::value;
+            if (g == 4) {
+                es &= 31u;                                       // at most 4 x 7 bits since u
+                R = __builtin_amdgcn_alignbit(hi, lo, es);
+                u += es;
+                es = 0;
+            }
+            uint32_t f = *(const kvc_lds_u16 *)(uintptr_t)((R & mask) | fe);
+            if (__builtin_expect(__any(f == 0u), 0)) {           // wave-uniform
+                u += es & 31u;
+                wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
+                w0 = wp[0], w1 = wp[1], w2 = wp[2];
+                // the 32 bits from the code on (the window starts a bit before it)
+                const uint32_t win = __builtin_amdgcn_alignbit(__builtin_amdgcn_alignbit(w2, w1, u), __builtin_amdgcn_alignbit(w1, w0, u), 1u);
+                uint32_t len = f & 31u;
+                if (f == 0u) {
+                    len = 1u;                                    // (bits that match no code: symbol 0)
+                    for (uint32_t j = 0; j < nesc; j++) {
+                        const kvc_w2 c = *(const kvc_lds_w2 *)(uintptr_t)(esc_addr + 8u * j);
+                        const uint32_t l = c.y & 0xffu;
+                        if (((win ^ c.x) << (32u - l)) == 0u) {
+                            len = l;
+                            f = (uint32_t)__half_as_ushort(__float2half_rn((float)((c.y >> 8) & 0xffu)));
+                        }
+                    }
+                }
+                u += len;
+                es = 0;
+                wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
+                w0 = wp[0], w1 = wp[1], w2 = wp[2];
+                lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
+                R = lo;
+            } else {
+                if (g != 3 && g != 7) R = __builtin_amdgcn_alignbit(R, R, f);
+                es += f;
+            }
+            e[g % 4] = f;
+            if constexpr (g % 4 == 3) {
+                constexpr int q = g / 4;
+                uint32_t a01 = ((e[1] << 16) | e[0]) & 0xffe0ffe0u, a23 = ((e[3] << 16) | e[2]) & 0xffe0ffe0u;
+                if (ROUNDED) {
+                    const kvc_w4 ms = *(const kvc_lds_w4 *)(uintptr_t)(msptr + q * 16);
+                    a01 = kvc_dequant_pair(a01, ms.x, ms.z);
+                    a23 = kvc_dequant_pair(a23, ms.y, ms.w);
+                }
+#pragma unroll
+                for (int s = 0; s < NM; s++)
+                    acc[s] = kvc_mfma4<BCAST>(a01, a23, kvc_read_columns<BCAST>(bptr + (q * NM + s) * 32, holder), acc[s]);
+            }
+        });
+        u += es & 31u;
+        bptr += 2 * NM * 32;
+        msptr += 32;
+    }
+}
+
 // One symbol per refill, generic table and long-code list in global memory; words from LDS (staged, bit-reversed)
 // or from global memory (raw, bounds-checked word by word).  Returns this lane's sums, one per query head.
 template <int REP, bool GSRC, bool ROUNDED>
@@ -498,8 +574,11 @@ __device__ __forceinline__ float kvc_quad_next(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xF5 /* quad_perm:[1,1,3,3] */, 0xf, 0xf, false));
 }
 
-template <int REP, int KIND, bool ROUNDED>
-__global__ void __launch_bounds__(KVC_WG, kvc_fused_mfma_occupancy(REP, KIND)) kvc_fused_mfma_kernel(KvcFusedArgs a_in)
+// LONG: for codebooks with codes of more than 7 bits (kvc_mfma_dot_long), kernels of their own
+// (kvc_fused_mfma_long.hip): beside the other loops it would cost them registers.
+template <int REP, int KIND, bool ROUNDED, bool LONG = false>
+__global__ void __launch_bounds__(KVC_WG, LONG ? kvc_fused_long_occupancy(REP, KIND) : kvc_fused_mfma_occupancy(REP, KIND))
+kvc_fused_mfma_kernel(KvcFusedArgs a_in)
 {
     const KvcFusedArgs &a = a_in;
     constexpr bool IS_K = KIND == 0;
@@ -552,7 +631,10 @@ __global__ void __launch_bounds__(KVC_WG, kvc_fused_mfma_occupancy(REP, KIND)) k
     const int64_t cb = a.s.rows_per_codebook ? (a.sched_nseg ? 0 : (int)blockIdx.y) / a.s.rows_per_codebook : 0;
     const uint32_t *__restrict__ lut_g = a.s.luts + cb * KVC_LUT_WORDS;
     const uint32_t lbits = lut_g[0], lmax = lut_g[1], nlong = lut_g[2];
-    const bool fast_book = nlong == 0 && lmax >= 1u && lmax <= 7u && (1u << lbits) <= (uint32_t)a.table_words;
+    const uint32_t nesc = LONG ? lut_g[7] : 0u;
+    const bool fast_book = LONG ? lmax > (uint32_t)KVC_LUT_ESC_BITS && nesc <= (uint32_t)KVC_LUT_ESC_MAX &&
+                                      (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u && a.table_words >= KVC_LONG_TABLE_WORDS
+                                : nlong == 0 && lmax >= 1u && lmax <= 7u && (1u << lbits) <= (uint32_t)a.table_words;
     // one-symbol entries: the symbol as fp16 in the upper half, the code length (never beyond the index width, which
     // bounds how far a corrupt stream can run) in the lowest byte
     auto fentry = [&](uint32_t i) {
@@ -563,15 +645,26 @@ __global__ void __launch_bounds__(KVC_WG, kvc_fused_mfma_occupancy(REP, KIND)) k
     const uint32_t pbits = 2u * lmax;
     // two symbols per look-up: twice the longest code fits the index, and no symbol's fp16 pattern needs the five
     // bits the lengths of a two-symbol entry go to (header word 6: OR of all the patterns)
-    const bool pairs = fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
+    const bool pairs = !LONG && fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
                        (1u << pbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
     // codes of 6 or 7 bits: two-byte entries (see kvc_mfma_dot), where no symbol's fp16 pattern needs its five lowest bits.
     // Not for V tiles that may straddle two heads: with that loop beside the others the kernel needs one register more
     // than six waves per SIMD leave it, and the compiler then spills in the per-tile path of every variant.
-    constexpr bool HALF_OK = SLOTS == 1;
+    constexpr bool HALF_OK = SLOTS == 1 && !LONG;
     const bool half_table = HALF_OK && fast_book && !pairs && lbits >= 6u && a.half_table != 0 && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
-    const uint32_t lead_bits = half_table ? 1u : 2u;                   // bits of the window below the table index
-    if (pairs) {
+    const uint32_t lead_bits = LONG || half_table ? 1u : 2u;                   // bits of the window below the table index
+    if constexpr (LONG) {
+        if (fast_book) {
+            uint16_t *t16 = reinterpret_cast<uint16_t *>(smem);
+            const uint32_t *entries = lut_g + KVC_LUT_HEADER_WORDS + KVC_LUT_LONG_WORDS;     // first stream bit in the index's top bit
+            for (uint32_t i = tid; i < (1u << KVC_LUT_ESC_BITS); i += KVC_WG) {
+                const uint32_t e = entries[(__brev(i) >> (32 - KVC_LUT_ESC_BITS)) << (lbits - KVC_LUT_ESC_BITS)], len = e & 0xffu;
+                t16[i] = len == 0u || len > (uint32_t)KVC_LUT_ESC_BITS
+                             ? (uint16_t)0 : (uint16_t)(__half_as_ushort(__float2half_rn((float)((e >> 8) & 0xffu))) | len);
+            }
+            for (uint32_t i = tid; i < 2 * nesc; i += KVC_WG) smem[(1 << KVC_LUT_ESC_BITS) / 2 + i] = lut_g[KVC_LUT_ESC_OFFSET + i];
+        }
+    } else if (pairs) {
         // the one-symbol table goes to the (not yet used) per-wave areas; the two-symbol table is derived from it
         uint32_t *tmp = smem + a.table_words;
         for (uint32_t i = tid; i < (1u << lbits); i += KVC_WG) tmp[i] = fentry(i);
@@ -596,7 +689,7 @@ __global__ void __launch_bounds__(KVC_WG, kvc_fused_mfma_occupancy(REP, KIND)) k
     for (int i = lane; i < SLOTS * T::BTAB_SLOT_WORDS; i += KVC_WAVE) btab[i] = 0;
     if (lane < KVC_PACK_LEAD) pack[lane] = 0;
     __syncthreads();
-    const uint32_t mask4 = ((1u << lbits) - 1u) << lead_bits, maskp = ((1u << pbits) - 1u) << 2;
+    const uint32_t mask4 = ((1u << (LONG ? (uint32_t)KVC_LUT_ESC_BITS : lbits)) - 1u) << lead_bits, maskp = ((1u << pbits) - 1u) << 2;
     const int n = IS_K ? D : KVC_V_TOKENS;                             // symbols per lane stream
     // symbols per refill in the main part (a multiple of four); what is left goes eight per refill
     const int per = pairs ? (pbits <= 7u ? 16 : 12) : (lmax <= 3u ? 16 : lmax <= 5u ? 12 : 8);
@@ -678,7 +771,9 @@ __global__ void __launch_bounds__(KVC_WG, kvc_fused_mfma_occupancy(REP, KIND)) k
             const bool holder = lane < 16;
             auto run = [&](auto skew_) {
                 constexpr bool SK = decltype(skew_)::value;
-                if (pairs) {
+                if constexpr (LONG) {
+                    kvc_mfma_dot_long<SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, fe + (2u << KVC_LUT_ESC_BITS), nesc, n, bptr, msptr, acc, holder);
+                } else if (pairs) {
                     if (per == 16) kvc_mfma_pair_dot<4, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
                     else kvc_mfma_pair_dot<3, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
                     if (n - n_main) kvc_mfma_pair_dot<2, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n - n_main, bptr, msptr, acc, holder);
@@ -759,4 +854,3 @@ __global__ void __launch_bounds__(KVC_WG, kvc_fused_mfma_occupancy(REP, KIND)) k
         plan = plan_next;
     }
 }
-

@@ -18,7 +18,7 @@ kvc_build_lut_kernel(const uint8_t *__restrict__ trees, int64_t tree_stride, int
     __shared__ int16_t s_parent[KVC_TREE_MAX_NODES];
     __shared__ uint8_t s_leaf[KVC_TREE_MAX_NODES];
     __shared__ uint8_t s_bit[KVC_TREE_MAX_NODES];
-    __shared__ uint32_t s_lmax, s_nlong;
+    __shared__ uint32_t s_lmax, s_nlong, s_nesc;
     __shared__ float s_avg;   // sum over leaves of len * 2^-len: the mean code length if the code is well matched
     __shared__ uint32_t s_symbits;   // OR over the symbols' fp16 patterns
 
@@ -28,7 +28,7 @@ kvc_build_lut_kernel(const uint8_t *__restrict__ trees, int64_t tree_stride, int
     int n_nodes = tree_bytes / node_bytes;
     if (n_nodes > KVC_TREE_MAX_NODES) n_nodes = KVC_TREE_MAX_NODES;
 
-    if (tid == 0) { s_lmax = 0; s_nlong = 0; s_avg = 0.f; s_symbits = 0; }
+    if (tid == 0) { s_lmax = 0; s_nlong = 0; s_nesc = 0; s_avg = 0.f; s_symbits = 0; }
     for (int n = tid; n < KVC_TREE_MAX_NODES; n += KVC_WG) {
         int leaf = 0, a = -1, b = -1;
         if (n < n_nodes) {
@@ -90,6 +90,13 @@ kvc_build_lut_kernel(const uint8_t *__restrict__ trees, int64_t tree_stride, int
     const uint32_t lbits = lmax == 0 ? 1u : (lmax < (uint32_t)KVC_LUT_MAX_BITS ? lmax : (uint32_t)KVC_LUT_MAX_BITS);
 #pragma unroll
     for (int k = 0; k < KVC_TREE_MAX_NODES / KVC_WG; k++) {
+        if (my_len[k] > (uint32_t)KVC_LUT_ESC_BITS) {
+            const uint32_t slot = atomicAdd(&s_nesc, 1u);
+            if (slot < (uint32_t)KVC_LUT_ESC_MAX) {
+                lut[KVC_LUT_ESC_OFFSET + 2 * slot] = __brev(my_code[k] << (32 - my_len[k]));
+                lut[KVC_LUT_ESC_OFFSET + 2 * slot + 1] = my_len[k] | ((uint32_t)(s_child[0][tid + k * KVC_WG] & 0xff) << 8);
+            }
+        }
         if (my_len[k] > lbits) {
             uint32_t slot = atomicAdd(&s_nlong, 1u);
             if (slot < (uint32_t)KVC_LUT_MAX_LONG) {
@@ -140,7 +147,7 @@ kvc_build_lut_kernel(const uint8_t *__restrict__ trees, int64_t tree_stride, int
         lut[4] = (lmax <= 3 || roomy8) ? 8u : lmax <= 7 ? 30u / lmax : roomy ? 4u : 2u;
         lut[5] = (roomy8 || (lmax > 7 && roomy)) ? 1u : 0u;
         lut[6] = s_symbits;       // low bits clear in every symbol's fp16 pattern: room for lengths in a packed entry
-        lut[7] = 0;
+        lut[7] = s_nesc;
     }
 }
 

@@ -628,6 +628,12 @@ class KVCompCtx:
                   self.head_num, self.head_dim, self.tree_format)
         return decoded, t_ms
 
+    @property
+    def code_hint(self) -> int:
+        """kvc_compressed_desc::max_code_bits of this context's codebook."""
+        table = self.encode_codebook
+        return self.max_code_bits | (0x100 if table is not None and table.shape[0] <= 64 * 8 else 0)
+
     def decode_lut(self) -> Optional[torch.Tensor]:
         """The decode tables of this context's codebook (kvc_build_lut), built once per codebook; None before the first
         block has been compressed."""
@@ -657,7 +663,7 @@ class KVCompCtx:
         _DESC.pack_into(self._descriptor, 0, lut.data_ptr(), 0, self._block_infos.address, self._block_infos.used,
                         self._thread_infos.address, self._thread_infos.used, encoded.address,
                         min(encoded.used + self._enc_pending, encoded.data.shape[0]), mins.address, scales.address, self._mask,
-                        self.max_tile_bytes, self.max_stream_bytes, self.max_code_bits, tokens, tail_address, tail)
+                        self.max_tile_bytes, self.max_stream_bytes, self.code_hint, tokens, tail_address, tail)
         return self._descriptor
 
     # decode and dequantize in one kernel (no uint8 tensor in between); False = the reference's two steps
