@@ -355,6 +355,13 @@ typedef struct kvc_compressed_desc {
     const void *d_tail_f16;
     int64_t tail_tokens;
 } kvc_compressed_desc;
+/* KVCompCtx.mat_vec_mul (models/cache/kvcomp_encode.py:209-280) over the compressed tokens of one tensor.  K: d_x fp16 q
+ * [batch, q_heads, head_dim] -> d_out fp16 scores [batch, q_heads, tokens] (d_partial_f16 unused).  V: d_x fp16 p
+ * [batch, q_heads, tokens] -> d_out fp16 [batch, q_heads, head_dim], the sums of the per-128-token products that
+ * kvc_v_partials_lut writes, which go to d_partial_f16 [tokens / 128, batch, q_heads, head_dim].  elapsed_ms (may be NULL)
+ * makes the call wait. */
+int kvc_mat_vec_mul(int is_k, const kvc_compressed_desc *c, const void *d_x_f16, void *d_partial_f16, void *d_out_f16,
+                    int64_t batch, int64_t kv_heads, int64_t q_heads, int64_t head_dim, float *elapsed_ms, void *stream);
 /* The dense fp16 history of one tensor (KVCompCtx.get, models/cache/kvcomp_encode.py:138-151): the compressed tokens
  * decoded and dequantized, the fp16 tail behind them, both straight into d_out_f16 [tokens + tail_tokens, batch, heads,
  * head_dim] (16-byte aligned, like the tail).  elapsed_ms (may be NULL) makes the call wait. */

@@ -89,6 +89,7 @@ _SIGNATURES = {
     "kvc_h2_scratch_bytes": [_i64],
     "kvc_h2_encode": [_vp, _i64, _vp, _vp, _vp, _i64, _vp, _i64, _i64p, _vp],
     "kvc_copy_rows": [_vp, _vp, _i64, _vp],
+    "kvc_mat_vec_mul": [_int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _f32p, _vp],
     "kvc_restore": [_int, _vp, _i64, _vp, _i64, _i64, _i64, _f32p, _vp],
     "kvc_attention_workspace_bytes": [_i64, _i64, _i64, _i64, _i64],
     "kvc_attention_decode": [C.POINTER(CompressedDesc), C.POINTER(CompressedDesc), _vp, C.c_float, _vp, _i64, _vp,

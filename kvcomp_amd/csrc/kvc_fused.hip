@@ -1350,6 +1350,61 @@ extern "C" int kvc_v_partials_lut(const void *d_luts, int64_t rows_per_codebook,
 }
 
 // ---------------------------------------------------------------------------------------------------
+// the two matrix-vector products of KVCompCtx.mat_vec_mul (models/cache/kvcomp_encode.py:209-280) from a descriptor
+// ---------------------------------------------------------------------------------------------------
+// out[i] = RN16(sum over groups of part[g][i]), fp32 sums; n even.  Reads 2 bytes per group and element: bound by the round
+// trips to memory at this size (64 groups x 4096 elements: 0.5 MB), so a wave has eight rows in flight and the workgroup's
+// four waves share the groups.
+__global__ void __launch_bounds__(KVC_WG) kvc_sum_partials_kernel(const uint32_t *__restrict__ part, int64_t groups, int64_t pairs, uint32_t *__restrict__ out)
+{
+    __shared__ float2 s_sum[KVC_WAVES_PER_WG][KVC_WAVE];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t i = (int64_t)blockIdx.x * KVC_WAVE + lane;
+    float2 sum = make_float2(0.f, 0.f);
+    if (i < pairs) {
+#pragma unroll 8
+        for (int64_t g = wave; g < groups; g += KVC_WAVES_PER_WG) {
+            const uint32_t w = part[g * pairs + i];
+            sum.x += kvc_half_bits_to_float(w & 0xffffu);
+            sum.y += kvc_half_bits_to_float(w >> 16);
+        }
+    }
+    s_sum[wave][lane] = sum;
+    __syncthreads();
+    if (wave == 0 && i < pairs) {
+#pragma unroll
+        for (int w = 1; w < KVC_WAVES_PER_WG; w++) {
+            sum.x += s_sum[w][lane].x;
+            sum.y += s_sum[w][lane].y;
+        }
+        out[i] = (uint32_t)__half_as_ushort(__float2half_rn(sum.x)) | ((uint32_t)__half_as_ushort(__float2half_rn(sum.y)) << 16);
+    }
+}
+
+extern "C" int kvc_mat_vec_mul(int is_k, const kvc_compressed_desc *c, const void *d_x_f16, void *d_partial_f16, void *d_out_f16,
+                               int64_t batch, int64_t kv_heads, int64_t q_heads, int64_t head_dim, float *elapsed_ms, void *stream_)
+{
+    hipStream_t stream = (hipStream_t)stream_;
+    KVC_REQUIRE(c != nullptr && d_x_f16 != nullptr && d_out_f16 != nullptr && (is_k || d_partial_f16 != nullptr), "NULL argument");
+    KVC_REQUIRE(c->tokens > 0 && c->d_luts != nullptr, "nothing is compressed");
+    KVC_REQUIRE((((uintptr_t)d_out_f16 | (uintptr_t)d_partial_f16) & 3) == 0, "results must be 4-byte aligned");
+    KvcTimer timer(elapsed_ms, stream);
+    if (int rc = kvc_fused(is_k, nullptr, 0, KVC_TREE_I8, c->d_block_infos, c->block_infos_bytes, c->d_thread_infos, c->thread_infos_bytes,
+                           c->d_encoded, c->encoded_bytes, c->d_quant_min_ints, c->d_quant_scales_f16, (int)c->quant_mask, d_x_f16,
+                           is_k ? d_out_f16 : d_partial_f16, c->tokens, batch, kv_heads, q_heads, head_dim, nullptr, stream_,
+                           (const uint32_t *)c->d_luts, (int)c->rows_per_codebook, 0, c->max_tile_bytes, c->max_stream_bytes,
+                           (int)c->max_code_bits))
+        return rc;
+    if (!is_k) {
+        const int64_t pairs = batch * q_heads * head_dim / 2;
+        hipLaunchKernelGGL(kvc_sum_partials_kernel, dim3((unsigned)((pairs + KVC_WAVE - 1) / KVC_WAVE)), dim3(KVC_WG), 0, stream,
+                           reinterpret_cast<const uint32_t *>(d_partial_f16), c->tokens / KVC_V_TOKENS, pairs, reinterpret_cast<uint32_t *>(d_out_f16));
+        KVC_HIP(hipGetLastError());
+    }
+    return timer.finish();
+}
+
+// ---------------------------------------------------------------------------------------------------
 // one-call decode attention over a compressed cache (no counterpart in the reference, whose models
 // decompress everything and run dense attention; models/cache/kvcomp_quant.py:74-75)
 //

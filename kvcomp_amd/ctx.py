@@ -711,29 +711,17 @@ class KVCompCtx:
         assert B.dtype == torch.float16, "B must be float16"
         assert len(B.shape) == 3, "B must be 3D tensor"
         assert B.shape[0] == self.batch_size, "batch size mismatch"
-        assert B.shape[1] % self.head_num == 0, "head num mismatch"
-        q_heads = B.shape[1]
+        q_heads, tokens, part = B.shape[1], self.compressed_ctx_len, None
+        assert q_heads % self.head_num == 0, "head num mismatch"
         if self.is_k:
             assert B.shape[2] == self.head_dim, "head dim mismatch"
-            C = torch.empty(self.batch_size, q_heads, self.compressed_ctx_len, dtype=torch.float16, device=self.device)
-            t_ms = kvcomp_cuda.k_decode_and_mat_vec_mul_cuda_export(
-                self.decode_codebook, self.block_infos, self.thread_infos, self.encoded_data,
-                self.quant_min_ints.reshape(-1), self.quant_scales.reshape(-1), B.contiguous(), C, self.head_num, self.head_dim,
-                self.tree_format)
-            return C, t_ms
-        assert B.shape[2] == self.compressed_ctx_len, "ctx len mismatch"
-        C = torch.empty(self.compressed_ctx_len // kvcomp_cuda.V_VEC_LEN, self.batch_size, q_heads, self.head_dim,
-                        dtype=torch.float16, device=self.device)
-        t_ms = kvcomp_cuda.v_decode_and_mat_vec_mul_cuda_export(
-            self.decode_codebook, self.block_infos, self.thread_infos, self.encoded_data,
-            self.quant_min_ints.reshape(-1), self.quant_scales.reshape(-1), B.contiguous(), C, self.head_num, self.head_dim,
-            self.tree_format)
-        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        start.record()
-        C = C.sum(dim=0, keepdim=True, dtype=torch.float32).to(torch.float16)
-        end.record()
-        end.synchronize()
-        return C, t_ms + start.elapsed_time(end)
+            out = torch.empty(self.batch_size, q_heads, tokens, dtype=torch.float16, device=self.device)
+        else:
+            assert B.shape[2] == tokens, "ctx len mismatch"
+            part = torch.empty(tokens // kvcomp_cuda.V_VEC_LEN, self.batch_size, q_heads, self.head_dim, dtype=torch.float16, device=self.device)
+            out = torch.empty(1, self.batch_size, q_heads, self.head_dim, dtype=torch.float16, device=self.device)
+        t_ms = kvcomp_cuda.mat_vec_mul(self.is_k, self.descriptor(), B.contiguous(), part, out, self.head_num, self.head_dim)
+        return out, t_ms
 
     def build_codebook(self, tensors: List[torch.Tensor]):
         """kvcomp_encode.py:282-306: one codebook from the quantized whole blocks of sample tensors."""

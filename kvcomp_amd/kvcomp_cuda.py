@@ -380,6 +380,15 @@ def copy_rows(on: torch.Tensor, dst: int, src: int, nbytes: int) -> None:
         check(_lib.lib().kvc_copy_rows(dst, src, nbytes, _lib.stream_of(on)))
 
 
+def mat_vec_mul(is_k: bool, desc, x: torch.Tensor, part, out: torch.Tensor, head_num: int, head_dim: int) -> float:
+    """kvc_mat_vec_mul over what `desc` (a _lib.CompressedDesc) describes; returns elapsed milliseconds."""
+    ms = C.c_float(0.0)
+    with _lib.device_guard(x):
+        check(_lib.lib().kvc_mat_vec_mul(int(is_k), C.byref(desc), x.data_ptr(), 0 if part is None else part.data_ptr(), out.data_ptr(),
+                                         x.shape[0], head_num, x.shape[1], head_dim, C.byref(ms), _stream(x)))
+    return float(ms.value)
+
+
 def restore(is_k: bool, desc, block_size: int, out: torch.Tensor, with_tail: bool = True) -> float:
     """kvc_restore: the tokens that `desc` (a _lib.CompressedDesc) describes, decoded and dequantized into `out` (device fp16
     [tokens (+ tail), B, H, D]) with the fp16 tail behind them; returns elapsed milliseconds."""
