@@ -106,6 +106,9 @@ int kvc_abi_version(void);
  *                           share their heads' operand tables).
  *   "attention_tail_in_merge": 1 (default): kvc_attention_decode handles V's fp16 tail (up to 1024 tokens, K compressed
  *                           at least as far as V) inside its merge kernel; 0: with two kernels of its own.
+ *   "attention_joint":       -1 (default): kvc_attention_decode takes K and V of small caches in one launch, a 128-token group
+ *                           of a head per workgroup, where head_dim is a multiple of 64 and codes have at most 7 bits;
+ *                           0: never; 1: whatever the cache's size.
  *   "decode_pipelined":      1 (default): plain decode and decode + dequantize run on the fused kernels' tile
  *                           pipeline; 0: on the simpler stand-alone kernels. */
 int kvc_set_option(const char *name, int value);

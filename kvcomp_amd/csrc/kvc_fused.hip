@@ -37,6 +37,7 @@
 // Slow path (codebooks with codes longer than the table index, tiles larger than the staging area, or
 // the rare overflow above): one symbol per refill, generic table read from global memory, payload read
 // from LDS or -- for an oversized tile -- from global memory.
+#include "kvc_attend.h"
 #include "kvc_fused_common.h"
 
 // -- slow path ----------------------------------------------------------------------------------------
@@ -1710,16 +1711,6 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
     float *ml = reinterpret_cast<float *>((char *)d_workspace + p.ml_off);
     const int rep = (int)(q_heads / kv_heads);
     KvcTimer timer(elapsed_ms, stream);
-    // ---- scores
-    if (k->tokens) {
-        KvcFusedExtra ex = {p.scores_stride, nullptr, 0, 1.f, nullptr};
-        if (int rc = kvc_fused(1, nullptr, 0, KVC_TREE_I8, k->d_block_infos, k->block_infos_bytes, k->d_thread_infos,
-                               k->thread_infos_bytes, k->d_encoded, k->encoded_bytes, k->d_quant_min_ints,
-                               k->d_quant_scales_f16, k->quant_mask, d_q_f16, scores, k->tokens, batch, kv_heads, q_heads,
-                               head_dim, fused_kernel_ms, stream_, (const uint32_t *)k->d_luts, (int)k->rows_per_codebook, 1,
-                               k->max_tile_bytes, k->max_stream_bytes, k->max_code_bits, &ex))
-            return rc;
-    }
     // V's fp16 tail is handled by the merge kernel itself when it is short enough and K's compressed part reaches at
     // least as far as V's (the V kernel then needs no score of K's tail); otherwise by two kernels of its own
     KvcTailArgs tail = {};
@@ -1740,6 +1731,23 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
         tail.kv_heads = (int)kv_heads;
         tail.rep = rep;
     }
+    // small caches: K and V in one launch (unless the caller asked for the two kernels' times)
+    bool joint = false;
+    if (!fused_kernel_ms && (tail_in_merge || v->tail_tokens == 0)) {
+        if (int rc = kvc_attend_groups(k, v, d_q_f16, softmax_scale, scores, p.scores_stride, part, ml, batch, kv_heads, q_heads, head_dim,
+                                       stream, &joint))
+            return rc;
+    }
+    // ---- scores
+    if (k->tokens && !joint) {
+        KvcFusedExtra ex = {p.scores_stride, nullptr, 0, 1.f, nullptr};
+        if (int rc = kvc_fused(1, nullptr, 0, KVC_TREE_I8, k->d_block_infos, k->block_infos_bytes, k->d_thread_infos,
+                               k->thread_infos_bytes, k->d_encoded, k->encoded_bytes, k->d_quant_min_ints,
+                               k->d_quant_scales_f16, k->quant_mask, d_q_f16, scores, k->tokens, batch, kv_heads, q_heads,
+                               head_dim, fused_kernel_ms, stream_, (const uint32_t *)k->d_luts, (int)k->rows_per_codebook, 1,
+                               k->max_tile_bytes, k->max_stream_bytes, k->max_code_bits, &ex))
+            return rc;
+    }
     if (k->tail_tokens && !tail_in_merge) {
         const int64_t items = k->tail_tokens * batch * kv_heads;
         hipLaunchKernelGGL(kvc_tail_scores_kernel, dim3((unsigned)((items + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG)), dim3(KVC_WG),
@@ -1747,7 +1755,7 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
                            scores, p.scores_stride, k->tokens, k->tail_tokens, (int)batch, (int)kv_heads, rep, (int)head_dim);
     }
     // ---- weighted values per group
-    if (v->tokens) {
+    if (v->tokens && !joint) {
         KvcFusedExtra ex = {0, scores, p.scores_stride, softmax_scale, ml};
         if (int rc = kvc_fused(0, nullptr, 0, KVC_TREE_I8, v->d_block_infos, v->block_infos_bytes, v->d_thread_infos,
                                v->thread_infos_bytes, v->d_encoded, v->encoded_bytes, v->d_quant_min_ints,

@@ -61,6 +61,7 @@ const OptionDef g_option_defs[KVC_OPT_COUNT] = {
     {"encode_lookback_polls", "KVCOMP_ENCODE_LOOKBACK_POLLS", 1 << 18},   // one-pass encoder: looks that may find a word not ready before a wave gives up (some tenths of a second); -1: treat every call as given up
     {"fused_schedule_v", "KVCOMP_FUSED_SCHEDULE_V", -1},         // the same for V launches: -1 follow fused_schedule (default schedule: runs that cover whole heads)
     {"fused_tiles_per_wave_v", "KVCOMP_FUSED_TILES_PER_WAVE_V", -1},   // plain grid, V launches: -1 follow fused_tiles_per_wave (default: the tiles of one head or head pair)
+    {"attention_joint", "KVCOMP_ATTENTION_JOINT", -1},             // kvc_attention_decode: K and V of a 128-token group in one workgroup; -1 choose per call, 0 never, 1 wherever it applies
 };
 std::atomic<int> g_options[KVC_OPT_COUNT];
 std::once_flag g_options_once;
