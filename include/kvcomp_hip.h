@@ -306,7 +306,8 @@ int kvc_v_decode_and_mat_vec_mul(const uint8_t *d_decode_tree, int64_t decode_tr
  *                        0 = unknown.  They only size the LDS staging; tiles that exceed them are decoded
  *                        from global memory.
  *     max_code_bits:     longest code of the codebook(s), 0 = unknown; + 256 where every symbol lies below 64 (codes
- *                        longer than 7 bits then take the matrix-core kernels too).  It only sizes the table kept in LDS
+ *                        longer than 7 bits then take the matrix-core kernels too); + 4096 * kvc_codebook::pair_bits
+ *                        where it is known (V is then decoded two symbols at a time).  It only sizes the table kept in LDS
  *                        (fewer bytes, more waves per CU); a codebook with longer codes than stated still
  *                        decodes correctly, on the slow path. */
 int64_t kvc_lut_bytes(void);
@@ -419,12 +420,14 @@ int kvc_quant(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H,
  *   returns them (the int8 tree where the code fits it, else the int16 tree), the longest code and the code bits of all
  *   symbols written (without the padding of each lane stream to whole bytes).  Waits for the symbol counts, not for the
  *   stream; cannot be recorded into a graph.
+ *   pair_bits: index bits of a decode table that next to all pairs of these symbols fit, 2 .. 7, or 0.
  * kvc_put_bytes: copies host bytes to device memory in stream order without waiting; h_src may be reused at once. */
 typedef struct kvc_codebook {
     int32_t tree_format, max_code_bits;
     int64_t encode_bytes, decode_bytes, payload_bits;
     uint8_t encode_table[256 * 8];
     uint8_t decode_tree[512 * 5];
+    int32_t pair_bits;
 } kvc_codebook;
 int kvc_quant_codebook(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                        float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, int smoothed_symbols,

@@ -41,7 +41,8 @@ class EncodeJob(C.Structure):
 class Codebook(C.Structure):
     """kvc_codebook of include/kvcomp_hip.h."""
     _fields_ = [("tree_format", C.c_int32), ("max_code_bits", C.c_int32), ("encode_bytes", C.c_int64), ("decode_bytes", C.c_int64),
-                ("payload_bits", C.c_int64), ("encode_table", C.c_uint8 * (256 * 8)), ("decode_tree", C.c_uint8 * (512 * 5))]
+                ("payload_bits", C.c_int64), ("encode_table", C.c_uint8 * (256 * 8)), ("decode_tree", C.c_uint8 * (512 * 5)),
+                ("pair_bits", C.c_int32)]
 
 
 # name -> argtypes (every function returns int unless listed in _RESTYPES)

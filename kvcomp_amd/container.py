@@ -62,7 +62,8 @@ def dumps(ctx: KVCompCtx) -> bytes:
         "quant_scale_rel": float(ctx.quant_scale_rel), "quant_dims": [int(d) for d in ctx.quant_dims],
         "block_size": ctx.block_size, "recent_size": ctx.recent_size,
         "ctx_len": ctx.ctx_len, "compressed_ctx_len": ctx.compressed_ctx_len,
-        "tree_format": ctx.tree_format, "max_code_bits": ctx.max_code_bits, "max_tile_bytes": ctx.max_tile_bytes, "max_stream_bytes": ctx.max_stream_bytes,
+        "tree_format": ctx.tree_format, "max_code_bits": ctx.max_code_bits,
+        "pair_bits": getattr(ctx, "pair_bits", 0), "max_tile_bytes": ctx.max_tile_bytes, "max_stream_bytes": ctx.max_stream_bytes,
         "config": str(cfg) if cfg is not None else None,
         "sections": [],
     }
@@ -211,6 +212,7 @@ def loads(data: bytes, device: Optional[torch.device] = None) -> KVCompCtx:
     ctx.ctx_len = header["ctx_len"]
     ctx.compressed_ctx_len = header["compressed_ctx_len"]
     ctx.max_code_bits = header["max_code_bits"]
+    ctx.pair_bits = header.get("pair_bits", 0)
     ctx.max_tile_bytes = header["max_tile_bytes"]
     ctx.max_stream_bytes = header["max_stream_bytes"]
     KVCompCtx.buffer_ctx_len.setdefault(device, 0)

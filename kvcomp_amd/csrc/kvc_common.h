@@ -78,8 +78,10 @@ struct KvcDecodeHints {
     int64_t max_tile_bytes, max_stream_bytes;
     int code_hint;                 // as kvc_compressed_desc::max_code_bits
 };
-// kvc_compressed_desc::max_code_bits: the longest code, and whether every symbol is known to lie below 64
+// kvc_compressed_desc::max_code_bits: the longest code, whether every symbol is known to lie below 64, and
+// kvc_codebook::pair_bits
 static inline int kvc_hint_bits(int64_t hint) { return (int)(hint & 0xff); }
+static inline int kvc_hint_pair_bits(int64_t hint) { return (int)(hint >> 12 & 7); }
 static inline bool kvc_hint_small_alphabet(int64_t hint) { return (hint & 0x100) != 0; }
 int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_tree_bytes, int tree_format,
                const uint8_t *d_block_infos, int64_t block_infos_bytes, const uint8_t *d_thread_infos,

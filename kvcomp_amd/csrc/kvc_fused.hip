@@ -935,7 +935,7 @@ static void kvc_launch_fused(int kind, const KvcFusedArgs &a, dim3 grid, size_t 
 // from global memory, so the sizes only affect speed.  Everything stays within 64 KiB per workgroup.
 static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_bytes, int64_t tiles,
                            int64_t max_tile_bytes, int64_t max_stream_bytes, int max_code_bits, int64_t extra_words = 0,
-                           bool allow_pairs = true, int64_t mfma_ops_words = 0, int long_table_words = 0)
+                           bool allow_pairs = true, int64_t mfma_ops_words = 0, int long_table_words = 0, int narrow_pair_bits = 0)
 {
     const int64_t slack = KVC_LDS_SLACK_WORDS + (long_table_words ? KVC_LDS_LONG_SLACK_WORDS : 0);
     const int force_rows = kvc_option(KVC_OPT_FUSED_ROWS);   // 0 / 1 overrides the choice below
@@ -956,6 +956,12 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
         // eight bytes per entry (fp32 symbols), four in the matrix-core kernels (fp16 symbols)
         const int words = (mfma_ops_words ? 1 : 2) << a.pair_bits;
         if (a.table_words < words) a.table_words = words;
+    }
+    a.narrow_pair_bits = 0;
+    if (narrow_pair_bits && a.pair_bits == 0 && max_code_bits >= 1 && max_code_bits <= KVC_LUT_ESC_BITS && narrow_pair_bits <= pair_limit) {
+        a.narrow_pair_bits = narrow_pair_bits;
+        a.table_words = (1 << (narrow_pair_bits > max_code_bits ? narrow_pair_bits : max_code_bits)) + (1 << max_code_bits);
+        if (a.table_words < 8) a.table_words = 8;
     }
     // per wave, besides the payload
     const int64_t ops_words = mfma_ops_words ? mfma_ops_words : (int64_t)slots * 128 * rep + extra_words;
@@ -1149,7 +1155,7 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
                       (is_k ? out_stride % 4 == 0 : head_dim % 4 == 0);
     const size_t lds = mfma ? kvc_plan_lds(a, slots, (int)rep, encoded_bytes, rows * a.s.cols, max_tile_bytes, max_stream_bytes,
                                            max_code_bits, 0, !long_codes, kvc_mfma_ops_words(slots, (int)rep, rounded),
-                                         long_codes ? KVC_LONG_TABLE_WORDS : 0)
+                                         long_codes ? KVC_LONG_TABLE_WORDS : 0, is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint))
                             : kvc_plan_lds(a, slots, rounded ? (int)rep + 1 : (int)rep, encoded_bytes, rows * a.s.cols,
                                            max_tile_bytes, max_stream_bytes, max_code_bits, 0, !rounded);
     a.rounded = rounded;

@@ -32,6 +32,7 @@ struct KvcFusedArgs {
     int skew;            // 0, or 2: every 32 payload words are followed by a copy of the next two (see kvc_skewed)
     int row_words;       // LDS words per lane stream (odd); 0 = decode from the packed payload
     int pair_bits;       // index width of the two-symbol table the host made room for; 0 = none
+    int narrow_pair_bits; // matrix-core V kernels: index bits of a two-symbol table that next to all pairs that occur fit; 0 = none
     int double_window;   // refill 64 stream bits at a time where the vector length allows
     int builtin_dpp;     // fp32-FMA kernels: lane permutes through the compiler's intrinsic instead of inline assembly
     int half_table;      // matrix-core kernels: two-byte table entries for codes of 6 or 7 bits

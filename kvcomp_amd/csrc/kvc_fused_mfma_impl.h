@@ -43,6 +43,7 @@ typedef __attribute__((address_space(3))) kvc_w2 kvc_lds_w2;
 typedef __attribute__((address_space(3))) kvc_w4 kvc_lds_w4;
 
 constexpr float KVC_LO_SCALE = 4096.f;
+constexpr uint32_t KVC_NARROW_MISS = 0x7e007e00u;    // fp16 NaN in the place of both symbols
 constexpr uint32_t KVC_PAIR_LEN_MASK = 0x1fu;      // both code lengths of a two-symbol entry (at most 30)
 
 __device__ __forceinline__ uint32_t kvc_lds_addr(const void *p)
@@ -642,11 +643,23 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
         const uint32_t len = (e & 0xffu) > lbits ? lbits : (e & 0xffu);
         return ((uint32_t)__half_as_ushort(__float2half_rn(__uint_as_float(e & 0xffffff00u))) << 16) | len;
     };
-    const uint32_t pbits = 2u * lmax;
+    // V: a two-symbol table with fewer index bits than the longest pair of codes needs, where pairs that do not fit next to
+    // never occur (KvcFusedArgs::narrow_pair_bits).  A code with smoothing gives every symbol the error bound allows a code, so
+    // its longest ones are mostly unused and would keep V from looking up pairs at all.  What does not fit is a pair of NaN in
+    // the table; a tile that meets one ends with NaN sums and is decoded again, one symbol per look-up, through the whole
+    // table behind the narrow one (at a multiple of its size, so that "window bits | offset" is an entry's address).
+    // Batch 4 x 32 heads x 96 x 32 768 tokens, heavy-tailed data, 7 index bits for codes of up to 6: V 88 -> 74 us.  With 8
+    // bits (three pairs per half window, 256 words) it measured no better than one symbol per look-up (38.6 / 39.8 us at
+    // batch 8 x 32 x 128 x 4096), and K, which has no such codebooks, 8 % slower for the scalars spilled.
+    constexpr bool NARROW_OK = !IS_K && !LONG;
+    const uint32_t one_at = (uint32_t)a.narrow_pair_bits > lbits ? (uint32_t)a.narrow_pair_bits : lbits;
+    const bool narrow = NARROW_OK && fast_book && a.narrow_pair_bits != 0 && (uint32_t)a.narrow_pair_bits < 2u * lmax &&
+                        (1u << one_at) + (1u << lbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
+    const uint32_t pbits = narrow ? (uint32_t)a.narrow_pair_bits : 2u * lmax;
     // two symbols per look-up: twice the longest code fits the index, and no symbol's fp16 pattern needs the five
     // bits the lengths of a two-symbol entry go to (header word 6: OR of all the patterns)
-    const bool pairs = !LONG && fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
-                       (1u << pbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
+    const bool pairs = narrow || (!LONG && fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
+                                 (1u << pbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u);
     // codes of 6 or 7 bits: two-byte entries (see kvc_mfma_dot), where no symbol's fp16 pattern needs its five lowest bits.
     // Not for V tiles that may straddle two heads: with that loop beside the others the kernel needs one register more
     // than six waves per SIMD leave it, and the compiler then spills in the per-tile path of every variant.
@@ -663,6 +676,16 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
                              ? (uint16_t)0 : (uint16_t)(__half_as_ushort(__float2half_rn((float)((e >> 8) & 0xffu))) | len);
             }
             for (uint32_t i = tid; i < 2 * nesc; i += KVC_WG) smem[(1 << KVC_LUT_ESC_BITS) / 2 + i] = lut_g[KVC_LUT_ESC_OFFSET + i];
+        }
+    } else if (NARROW_OK && narrow) {
+        uint32_t *one = smem + (1u << one_at);
+        for (uint32_t i = tid; i < (1u << lbits); i += KVC_WG) one[i] = fentry(i);
+        __syncthreads();
+        const uint32_t m1 = (1u << lbits) - 1u;
+        for (uint32_t idx = tid; idx < (1u << pbits); idx += KVC_WG) {
+            const uint32_t e0 = one[idx & m1], l0 = e0 & 0xffu;
+            const uint32_t e1 = one[(idx >> l0) & m1], l = l0 + (e1 & 0xffu);
+            smem[idx] = l <= pbits ? (e1 & 0xffff0000u) | (e0 >> 16) | l : KVC_NARROW_MISS | pbits;
         }
     } else if (pairs) {
         // the one-symbol table goes to the (not yet used) per-wave areas; the two-symbol table is derived from it
@@ -761,32 +784,38 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
         }
         if (fast_book && st.fits) {
             kvc_f4 acc[NM];
-#pragma unroll
-            for (int s = 0; s < NM; s++) acc[s] = kvc_f4{0.f, 0.f, 0.f, 0.f};
-            uint32_t u = st.u0;
-            uint32_t bptr = kvc_lds_addr(my_btab) + (lane & 3) * 8, msptr = kvc_lds_addr(my_mstab);
             const uint32_t sbase = kvc_lds_addr(pack);
             // one head per tile: all sixteen blocks share their operand columns, which lanes 0 - 15 then hold for all
             constexpr bool BCAST = SLOTS == 1;
             const bool holder = lane < 16;
-            auto run = [&](auto skew_) {
+            auto run = [&](auto skew_, bool whole) {
                 constexpr bool SK = decltype(skew_)::value;
+#pragma unroll
+                for (int s = 0; s < NM; s++) acc[s] = kvc_f4{0.f, 0.f, 0.f, 0.f};
+                uint32_t u = st.u0;
+                uint32_t bptr = kvc_lds_addr(my_btab) + (lane & 3) * 8, msptr = kvc_lds_addr(my_mstab);
                 if constexpr (LONG) {
                     kvc_mfma_dot_long<SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, fe + (2u << KVC_LUT_ESC_BITS), nesc, n, bptr, msptr, acc, holder);
-                } else if (pairs) {
+                } else if (pairs && !whole) {
                     if (per == 16) kvc_mfma_pair_dot<4, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
                     else kvc_mfma_pair_dot<3, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
                     if (n - n_main) kvc_mfma_pair_dot<2, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n - n_main, bptr, msptr, acc, holder);
                 } else {
-                    if (per == 16) kvc_mfma_dot<8, SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
-                    else if (per == 12) kvc_mfma_dot<6, SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
-                    const int rest = per == 8 ? n : n - n_main;
+                    if (!whole && per == 16) kvc_mfma_dot<8, SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
+                    else if (!whole && per == 12) kvc_mfma_dot<6, SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
+                    const int rest = whole || per == 8 ? n : n - n_main;
+                    const uint32_t tab = whole ? fe + (4u << one_at) : fe;
                     if (HALF_OK && rest && half_table) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, HALF_OK>(sbase, u, fe, mask4, rest, bptr, msptr, acc, holder);
-                    else if (rest) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, rest, bptr, msptr, acc, holder);
+                    else if (rest) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST>(sbase, u, tab, mask4, rest, bptr, msptr, acc, holder);
                 }
             };
-            if (a.skew) run(std::true_type{});
-            else run(std::false_type{});
+            for (bool whole = false;; whole = true) {
+                if (a.skew) run(std::true_type{}, whole);
+                else run(std::false_type{}, whole);
+                if (!NARROW_OK || !narrow || whole) break;
+                const bool missed = __builtin_isnan(acc[0][0]) || __builtin_isnan(acc[0][1]) || __builtin_isnan(acc[0][2]) || __builtin_isnan(acc[0][3]);
+                if (!__any(missed)) break;                     // (NaN of q or of the weights: the same again)
+            }
             // register i of lane 4 b + j: row 4 b + i, column 4 set + j; the even columns take their low parts from
             // the lane to their right and carry the results of query head 2 set + j / 2
             int lane_e = lane;

@@ -208,6 +208,7 @@ class KVCompCtx:
         self._tail: Optional[torch.Tensor] = None      # [capacity, B, H, D]; the first _tail_len tokens are the tail
         self._tail_len = 0
         self.max_code_bits = 0           # longest code of the codebook (0 = unknown)
+        self.pair_bits = 0             # index width that next to all pairs of symbols fit (kvc_codebook::pair_bits, 0 = none known)
         self.max_tile_bytes = 0            # largest tile payload seen so far (sizes the fused decoders' LDS staging)
         self.max_stream_bytes = 0          # longest lane stream seen so far (sizes the fused decoders' LDS rows)
         self.encode_codebook: Optional[torch.Tensor] = None
@@ -562,7 +563,7 @@ class KVCompCtx:
             self._issue_probe()
         else:
             self._sync_sizes()                                 # (a failure leaves the context as it was before the encode)
-        self.tree_format, self.max_code_bits = book.tree_format, book.max_code_bits
+        self.tree_format, self.max_code_bits, self.pair_bits = book.tree_format, book.max_code_bits, book.pair_bits
         self.encode_codebook, self.decode_codebook = enc, dec
         return sym
 
@@ -632,7 +633,7 @@ class KVCompCtx:
     def code_hint(self) -> int:
         """kvc_compressed_desc::max_code_bits of this context's codebook."""
         table = self.encode_codebook
-        return self.max_code_bits | (0x100 if table is not None and table.shape[0] <= 64 * 8 else 0)
+        return self.max_code_bits | self.pair_bits << 12 | (0x100 if table is not None and table.shape[0] <= 64 * 8 else 0)
 
     def decode_lut(self) -> Optional[torch.Tensor]:
         """The decode tables of this context's codebook (kvc_build_lut), built once per codebook; None before the first
@@ -742,7 +743,7 @@ class KVCompCtx:
 
     def _set_codebook(self, enc: torch.Tensor, dec: torch.Tensor, tree_format: int = kvcomp_cuda.TREE_I8):
         """enc / dec: CPU byte tensors from kvcomp_cuda.build_codebook."""
-        self.tree_format = tree_format
+        self.tree_format, self.pair_bits = tree_format, 0
         lengths = enc.view(torch.int32)[1::2]
         self.max_code_bits = int(lengths.max())      # sizes the fused decoders' table in LDS
         self.encode_codebook = enc.to(self.device)
