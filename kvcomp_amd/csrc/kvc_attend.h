@@ -2,11 +2,13 @@
 #pragma once
 #include "kvc_common.h"
 
-// Workgroups (128-token groups x KV heads x batch entries) up to which the joint kernel is taken.  Beyond, the chip is full of
-// waves either way, and the two kernels, whose waves hold fewer registers and no tables of both streams, are as fast or
-// faster.  Two kernels against this one, head_dim 128: 1024 workgroups 26.9 / 20.9 us, 1536 29.6 / 26.4, 2048 33.6 / 34.4,
-// 3072 43.6 / 45.0 (one query head per KV head; two and four alike); eight query heads: 1024 41.2 / 30.6, 1536 48.3 / 50.0.
-constexpr int64_t KVC_ATTEND_MAX_WGS = 1536, KVC_ATTEND_MAX_WGS_8 = 1024;
+// Workgroups (128-token groups x KV heads x batch entries) up to which the joint kernel is taken, by query heads per KV head.
+// Beyond, the chip is full of waves either way, and the two kernels, whose waves hold fewer registers and no tables of both
+// streams, are as fast or faster.  Two kernels against this one in us, head_dim 128 / 64:
+//   1 query head    1024 workgroups 27.2 : 20.7 / 23.5 : 17.2    1536 29.8 : 30.0 / 24.8 : 24.0    2048 34.1 : 34.1 / 25.8 : 25.9
+//   4 query heads   1536            36.8 : 34.8 / 30.4 : 28.6    2048 41.3 : 40.5 / 32.4 : 31.9    3072 58.5 : 58.0 / 41.2 : 45.4
+//   8 query heads   2048            70.5 : 48.6 / 47.0 : 37.7    3072 81.8 : 72.0 / 54.8 : 53.8
+constexpr int64_t kvc_attend_max_wgs(int64_t rep) { return rep <= 2 ? 1536 : rep == 4 ? 2048 : 3072; }
 constexpr int KVC_ATTEND_K_PAIR_BITS = 6;         // longest code for which K's table of two symbols per look-up is built
 
 // Partials [groups, B * Hq, D] and their (maximum, sum of weights) of all whole groups of 128 tokens that V holds compressed,

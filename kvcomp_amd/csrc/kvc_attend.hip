@@ -8,8 +8,15 @@
 // wave each; the V waves keep their symbols as bytes in 32 registers until the K waves have left the scores in LDS, the four
 // waves turn those into softmax weights, and the V waves then multiply: 32 groups of four tokens, one matrix instruction
 // each.  Scores of these groups never go to memory.  Calls of (batch x KV heads x query heads per KV head x head_dim, tokens),
-// two kernels -> this one, the merge of the groups included: 1 x 8 x 4 x 128, 1000: 28.0 -> 19.1 us; 1 x 32 x 1 x 128, 4096:
-// 24.6 -> 18.9; 1 x 32 x 1 x 64, 4096: 20.7 -> 15.5; 1 x 8 x 8 x 128, 3000: 35.8 -> 24.5.
+// two kernels -> this one, the merge of the groups included: 1 x 8 x 4 x 128, 1000: 28.0 -> 16.5 us; 1 x 32 x 1 x 128, 4096:
+// 24.8 -> 18.2; 1 x 32 x 1 x 64, 4096: 21.0 -> 14.6; 1 x 8 x 8 x 128, 3000: 35.3 -> 19.4.
+//
+// Where a wave's 23 500 cycles go (clock stamps, 1 x 32 heads x 128 x 1024 tokens, one workgroup per CU): loads 5200, tables
+// and staging 2700, 128 look-ups in a row 12 000 (V; K alike), scores to weights and two barriers 1400, the products 2150.
+// The operands of K's products and of V's are read by all lanes, without a branch, and V's some groups ahead: with the read
+// under the branch that the larger launches use (it saves LDS time) each group of four waited for its own round trip:
+// K 13 900 cycles, V's products 4200.  Registers are given away for that: five waves per SIMD (four with four and eight query
+// heads), which is what the LDS leaves room for.
 //
 // The chain itself is halved by looking up two K symbols at a time with codes of 5 and 6 bits, too.  The larger launches do
 // not: there the bank conflicts of the table of 1024 or 4096 words cost more than the look-ups saved, because waves of
@@ -37,6 +44,7 @@ struct KvcAttendArgs {
 template <bool PAIRS>
 __device__ __forceinline__ void kvc_decode_bytes(uint32_t sbase, uint32_t u, uint32_t fe, uint32_t mask, kvc_w32 &vd)
 {
+    asm volatile("" : "+v"(mask));                               // in a vector register: mask and offset in one instruction
     constexpr int N = PAIRS ? 4 : 8;                             // look-ups per refill: 8 symbols, half from each half window
 #pragma unroll 1
     for (int i = 0; i < KVC_V_TOKENS / 8; i++) {
@@ -102,7 +110,7 @@ __device__ __forceinline__ void kvc_decode_bytes_slow(const uint32_t *words, uin
 }
 
 template <int REP>
-__global__ void __launch_bounds__(KVC_WG, 4) kvc_attend_group_kernel(KvcAttendArgs j)
+__global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP <= 2 ? 5 : 4, REP <= 2 ? 5 : 4))) kvc_attend_group_kernel(KvcAttendArgs j)
 {
     constexpr int NM = kvc_mfma_sets(REP);
     using T = KvcMfmaTables<REP>;
@@ -219,8 +227,7 @@ __global__ void __launch_bounds__(KVC_WG, 4) kvc_attend_group_kernel(KvcAttendAr
     __syncthreads();
     // ---- decode: K tiles to scores, V tiles to bytes
     kvc_w32 vd;
-    const uint32_t sbase = kvc_lds_addr(pack), fe = kvc_lds_addr(is_k ? ktab : vtab);
-    const bool holder = lane < 16;
+    const uint32_t sbase = kvc_lds_addr(pack), fe_k = kvc_lds_addr(smem), fe_v = kvc_lds_addr(vtab);
     const int rows4 = (lane >> 2) * 4, cj = lane & 3;
     if (active && is_k) {
         float *dst = s_scores + wave * KVC_WAVE;
@@ -239,10 +246,10 @@ __global__ void __launch_bounds__(KVC_WG, 4) kvc_attend_group_kernel(KvcAttendAr
                 // 30 bits of a half window hold three pairs of codes of up to 5 bits, two of 6
                 int n_main = kb <= 5u ? D / 12 * 12 : 0;
                 while ((D - n_main) % 8 != 0) n_main -= 12;
-                if (n_main) kvc_mfma_pair_dot<3, false, NM, true, true>(sbase, u, fe, mask, n_main, bptr, msptr, acc, holder);
-                kvc_mfma_pair_dot<2, false, NM, true, true>(sbase, u, fe, mask, D - n_main, bptr, msptr, acc, holder);
+                if (n_main) kvc_mfma_pair_dot<3, false, NM, true, true, true>(sbase, u, fe_k, mask, n_main, bptr, msptr, acc, true);
+                kvc_mfma_pair_dot<2, false, NM, true, true, true>(sbase, u, fe_k, mask, D - n_main, bptr, msptr, acc, true);
             } else {
-                kvc_mfma_dot<4, false, NM, true, true>(sbase, u, fe, mask, D, bptr, msptr, acc, holder);
+                kvc_mfma_dot<4, false, NM, true, true, false, true>(sbase, u, fe_k, mask, D, bptr, msptr, acc, true);
             }
 #pragma unroll
             for (int q = 0; q < NM; q++) {
@@ -268,8 +275,8 @@ __global__ void __launch_bounds__(KVC_WG, 4) kvc_attend_group_kernel(KvcAttendAr
         if (!v_fast || !st.fits)
             kvc_decode_bytes_slow(st.fits ? pack : st.gwords, st.fits ? (uint32_t)j.v.pack_logical : st.gnwords, st.fits,
                                   st.fits ? st.u0 + 2u : st.gpos, lut_v, vd);
-        else if (v_pairs) kvc_decode_bytes<true>(sbase, st.u0, fe, mask, vd);
-        else kvc_decode_bytes<false>(sbase, st.u0, fe, mask, vd);
+        else if (v_pairs) kvc_decode_bytes<true>(sbase, st.u0, fe_v, mask, vd);
+        else kvc_decode_bytes<false>(sbase, st.u0, fe_v, mask, vd);
     }
     if (!whole) return;                                                                   // uniform over the workgroup
     __syncthreads();
@@ -298,14 +305,35 @@ __global__ void __launch_bounds__(KVC_WG, 4) kvc_attend_group_kernel(KvcAttendAr
 #pragma unroll
     for (int q = 0; q < NM; q++) acc[q] = kvc_f4{0.f, 0.f, 0.f, 0.f};
     const uint32_t bptr = kvc_lds_addr(btab_v) + cj * 8, msptr = kvc_lds_addr(mstab);
+    // the operands of a few groups are asked for while the groups before them are multiplied (left to itself the compiler asks for
+    // them right before their use: 32 groups, 48 LDS round trips, 3400 cycles)
+    constexpr int AHEAD = NM <= 2 ? 4 : 2;
+    kvc_w4 ms[2][AHEAD];
+    kvc_w2 cols[2][AHEAD][NM];
+    auto ask = [&](auto buf_, int i0) {
+        constexpr int buf = decltype(buf_)::value;
 #pragma unroll
-    for (int i = 0; i < KVC_MFMA_GROUPS; i++) {
-        const kvc_w4 ms = *(const kvc_lds_w4 *)(uintptr_t)(msptr + i * 16);
-        const uint32_t a01 = kvc_dequant_pair(__builtin_amdgcn_perm(0x64u, vd[i], 0x04010400u), ms.x, ms.z);
-        const uint32_t a23 = kvc_dequant_pair(__builtin_amdgcn_perm(0x64u, vd[i], 0x04030402u), ms.y, ms.w);
+        for (int k = 0; k < AHEAD; k++) {
+            ms[buf][k] = *(const kvc_lds_w4 *)(uintptr_t)(msptr + (i0 + k) * 16);
 #pragma unroll
-        for (int q = 0; q < NM; q++) acc[q] = kvc_mfma4<true>(a01, a23, kvc_read_columns<true>(bptr + (i * NM + q) * 32, holder), acc[q]);
-    }
+            for (int q = 0; q < NM; q++) cols[buf][k][q] = kvc_read_columns<true, true>(bptr + ((i0 + k) * NM + q) * 32, true);
+        }
+    };
+    ask(std::integral_constant<int, 0>{}, 0);
+    kvc_static_for<KVC_MFMA_GROUPS / AHEAD>([&](auto s_) {
+        constexpr int s = decltype(s_)::value, buf = s & 1;
+        if constexpr ((s + 1) * AHEAD < KVC_MFMA_GROUPS) ask(std::integral_constant<int, buf ^ 1>{}, (s + 1) * AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < AHEAD; k++) {
+            const uint32_t four = vd[s * AHEAD + k];
+            const uint32_t a01 = kvc_dequant_pair(__builtin_amdgcn_perm(0x64u, four, 0x04010400u), ms[buf][k].x, ms[buf][k].z);
+            const uint32_t a23 = kvc_dequant_pair(__builtin_amdgcn_perm(0x64u, four, 0x04030402u), ms[buf][k].y, ms[buf][k].w);
+#pragma unroll
+            for (int q = 0; q < NM; q++) acc[q] = kvc_mfma4<true>(a01, a23, cols[buf][k][q], acc[q]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
     float *out = reinterpret_cast<float *>(j.v.out) + (((int64_t)pos.row * j.v.batch + pos.b) * j.v.q_heads + pos.h * REP) * D + pos.d0;
 #pragma unroll
     for (int q = 0; q < NM; q++) {
@@ -370,7 +398,7 @@ int kvc_attend_groups(const kvc_compressed_desc *k, const kvc_compressed_desc *v
     const int64_t groups = v->tokens / KVC_V_TOKENS, wgs = groups * bh;
     const int64_t k_tiles = k->tokens / KVC_WAVE * bh, k_rest = k_tiles - wgs * KVC_ATTEND_K_TILES;
     if (k_tiles > (int64_t)1 << 30) return 0;
-    if (want < 0 && wgs > (rep == 8 ? KVC_ATTEND_MAX_WGS_8 : KVC_ATTEND_MAX_WGS)) return 0;
+    if (want < 0 && wgs > kvc_attend_max_wgs(rep)) return 0;
     KvcAttendArgs j = {};
     if (int rc = kvc_attend_fill(j.k, k, 1, batch, kv_heads, q_heads, head_dim)) return rc;
     if (int rc = kvc_attend_fill(j.v, v, 0, batch, kv_heads, q_heads, head_dim)) return rc;

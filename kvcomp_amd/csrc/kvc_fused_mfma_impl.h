@@ -62,9 +62,12 @@ __device__ __forceinline__ kvc_f4 kvc_mfma4(uint32_t a01, uint32_t a23, kvc_w2 b
 }
 
 // This lane's operand columns of one group: an 8-byte LDS read, by the first sixteen lanes only where they serve all.
-template <bool BCAST>
+// EVERY: by all lanes all the same.  That takes more of the LDS's time, but no branch: the read can be issued far ahead of its
+// use, which is what counts in a launch of a few waves per SIMD (kvc_attend.hip).
+template <bool BCAST, bool EVERY = false>
 __device__ __forceinline__ kvc_w2 kvc_read_columns(uint32_t addr, bool holder)
 {
+    if constexpr (EVERY) return *(const kvc_lds_w2 *)(uintptr_t)addr;
     kvc_w2 b;
     // whatever the registers hold: with the broadcast the matrix core reads the operand from the first sixteen lanes
     // and from no other, so the rest need no defined value (and no instruction to give them one)
@@ -348,7 +351,7 @@ __device__ __forceinline__ void kvc_mfma_stage_ops(const KvcFusedArgs &a, const 
 // word, which the LDS serves in one cycle (with four-byte entries a 64-entry table has two words per bank and 42 % of
 // its LDS cycles are bank conflicts).  Costs an instruction per two symbols (join and mask instead of a byte permute);
 // the lengths of a half window (at most 4 x 7 bits) are summed in five bits, above which symbol bits pile up.
-template <int G, bool SKEW, int NM, bool ROUNDED, bool BCAST, bool HALF = false>
+template <int G, bool SKEW, int NM, bool ROUNDED, bool BCAST, bool HALF = false, bool EVERY = false>
 __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32_t fe, uint32_t mask4, int n,
                                              uint32_t &bptr, uint32_t &msptr, kvc_f4 (&acc)[NM], bool holder)
 {
@@ -388,7 +391,7 @@ __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32
                 }
 #pragma unroll
                 for (int s = 0; s < NM; s++)
-                    acc[s] = kvc_mfma4<BCAST>(a01, a23, kvc_read_columns<BCAST>(bptr + (q * NM + s) * 32, holder), acc[s]);
+                    acc[s] = kvc_mfma4<BCAST>(a01, a23, kvc_read_columns<BCAST, EVERY>(bptr + (q * NM + s) * 32, holder), acc[s]);
             }
         });
         u += HALF ? used1 + (es & 31u) : es & 0xffu;
@@ -398,7 +401,7 @@ __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32
 }
 
 // Two symbols per look-up: PG pairs from each half window, 4 PG symbols per refill; n a multiple of 4 PG.
-template <int PG, bool SKEW, int NM, bool ROUNDED, bool BCAST>
+template <int PG, bool SKEW, int NM, bool ROUNDED, bool BCAST, bool EVERY = false>
 __device__ __forceinline__ void kvc_mfma_pair_dot(uint32_t sbase, uint32_t &u, uint32_t fe, uint32_t maskp, int n,
                                                   uint32_t &bptr, uint32_t &msptr, kvc_f4 (&acc)[NM], bool holder)
 {
@@ -429,7 +432,7 @@ __device__ __forceinline__ void kvc_mfma_pair_dot(uint32_t sbase, uint32_t &u, u
                 }
 #pragma unroll
                 for (int s = 0; s < NM; s++)
-                    acc[s] = kvc_mfma4<BCAST>(a01, a23, kvc_read_columns<BCAST>(bptr + (q * NM + s) * 32, holder), acc[s]);
+                    acc[s] = kvc_mfma4<BCAST>(a01, a23, kvc_read_columns<BCAST, EVERY>(bptr + (q * NM + s) * 32, holder), acc[s]);
             }
         });
         u += used1 + (es & KVC_PAIR_LEN_MASK);
