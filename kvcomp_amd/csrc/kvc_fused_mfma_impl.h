@@ -791,6 +791,11 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
             // one head per tile: all sixteen blocks share their operand columns, which lanes 0 - 15 then hold for all
             constexpr bool BCAST = SLOTS == 1;
             const bool holder = lane < 16;
+            // ... except with two and with eight query heads, where all lanes read them (no branch around the reads, see
+            // kvc_read_columns): 8 x 8 x 8 x 128 x 4096 tokens K 32.1 -> 30.2, V 35.5 -> 33.5 us, two heads 27.6 -> 27.1 each.  With
+            // four heads the LDS has no time for it (16 x 8 x 4 x 128 x 8192: K 47.1 -> 49.2, V 51.9 -> 54.0); with one it is
+            // as long as it is broad (8 x 32 x 128 x 4177: 84.4 -> 84.7, 4 x 32 x 96 x 32 768: 164.5 -> 161.8 altogether).
+            constexpr bool EV = BCAST && (REP == 2 || REP == 8);
             auto run = [&](auto skew_, bool whole) {
                 constexpr bool SK = decltype(skew_)::value;
 #pragma unroll
@@ -800,16 +805,16 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
                 if constexpr (LONG) {
                     kvc_mfma_dot_long<SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, fe + (2u << KVC_LUT_ESC_BITS), nesc, n, bptr, msptr, acc, holder);
                 } else if (pairs && !whole) {
-                    if (per == 16) kvc_mfma_pair_dot<4, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
-                    else kvc_mfma_pair_dot<3, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
-                    if (n - n_main) kvc_mfma_pair_dot<2, SK, NM, ROUNDED, BCAST>(sbase, u, fe, maskp, n - n_main, bptr, msptr, acc, holder);
+                    if (per == 16) kvc_mfma_pair_dot<4, SK, NM, ROUNDED, BCAST, EV>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
+                    else kvc_mfma_pair_dot<3, SK, NM, ROUNDED, BCAST, EV>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
+                    if (n - n_main) kvc_mfma_pair_dot<2, SK, NM, ROUNDED, BCAST, EV>(sbase, u, fe, maskp, n - n_main, bptr, msptr, acc, holder);
                 } else {
-                    if (!whole && per == 16) kvc_mfma_dot<8, SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
-                    else if (!whole && per == 12) kvc_mfma_dot<6, SK, NM, ROUNDED, BCAST>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
+                    if (!whole && per == 16) kvc_mfma_dot<8, SK, NM, ROUNDED, BCAST, false, EV>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
+                    else if (!whole && per == 12) kvc_mfma_dot<6, SK, NM, ROUNDED, BCAST, false, EV>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
                     const int rest = whole || per == 8 ? n : n - n_main;
                     const uint32_t tab = whole ? fe + (4u << one_at) : fe;
-                    if (HALF_OK && rest && half_table) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, HALF_OK>(sbase, u, fe, mask4, rest, bptr, msptr, acc, holder);
-                    else if (rest) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST>(sbase, u, tab, mask4, rest, bptr, msptr, acc, holder);
+                    if (HALF_OK && rest && half_table) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, HALF_OK, EV>(sbase, u, fe, mask4, rest, bptr, msptr, acc, holder);
+                    else if (rest) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, false, EV>(sbase, u, tab, mask4, rest, bptr, msptr, acc, holder);
                 }
             };
             for (bool whole = false;; whole = true) {
