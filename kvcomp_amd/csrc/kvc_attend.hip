@@ -18,9 +18,11 @@
 // K 13 900 cycles, V's products 4200.  Registers are given away for that: five waves per SIMD (four with four and eight query
 // heads), which is what the LDS leaves room for.
 //
-// The chain itself is halved by looking up two K symbols at a time with codes of 5 and 6 bits, too.  The larger launches do
-// not: there the bank conflicts of the table of 1024 or 4096 words cost more than the look-ups saved, because waves of
-// other tiles fill the wait anyway.
+// Two symbols per look-up where every pair of codes fits the table (K up to 6 bits, V up to 4): as many look-ups in a row again
+// saved.  Tables that hold nearly all pairs of 7-bit codes, with a second look-up for the rest, gain nothing: waiting for
+// every look-up's outcome and building 2048 entries cost what the look-ups saved (18.9 -> 19.0 us at 1024 workgroups).
+// One symbol at a time, V's entries have two bytes, so that 128 of them are two words per LDS bank: 1024 workgroups 19.1 ->
+// 18.2 us.  For K, whose two-byte entries take more instructions to join, it gains 0.3 us there and costs 0.3 to 0.5 below.
 #include "kvc_attend.h"
 #include "kvc_fused_mfma_impl.h"
 
@@ -40,7 +42,7 @@ struct KvcAttendArgs {
 };
 
 // -- V tiles as bytes ------------------------------------------------------------------------------------
-// Table entries: {code length(s) | symbol << 8 [| second symbol << 16]}; register i of `vd` holds tokens 4 i .. 4 i + 3.
+// Table entries: {code length(s) | symbol << 8 [| second symbol << 16]}, two bytes each without the second symbol; register i of `vd` holds tokens 4 i .. 4 i + 3.
 template <bool PAIRS>
 __device__ __forceinline__ void kvc_decode_bytes(uint32_t sbase, uint32_t u, uint32_t fe, uint32_t mask, kvc_w32 &vd)
 {
@@ -56,7 +58,8 @@ __device__ __forceinline__ void kvc_decode_bytes(uint32_t sbase, uint32_t u, uin
         kvc_static_for<N>([&](auto p_) {
             constexpr int p = decltype(p_)::value;
             if constexpr (p == N / 2) R = __builtin_amdgcn_alignbit(hi, lo, es);        // at most 28 bits so far
-            e[p] = *(const kvc_lds_u32 *)(uintptr_t)((R & mask) | fe);
+            if constexpr (PAIRS) e[p] = *(const kvc_lds_u32 *)(uintptr_t)((R & mask) | fe);
+            else e[p] = *(const kvc_lds_u16 *)(uintptr_t)((R & mask) | fe);
             if constexpr (p != N / 2 - 1 && p != N - 1) R = __builtin_amdgcn_alignbit(R, R, e[p]);
             es += e[p];
         });
@@ -200,15 +203,16 @@ __global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP
             vtab[tid] = ((e1 & 0xff00u) << 8) | (e0 & 0xff00u) | ((e0 & 0xffu) + (e1 & 0xffu));
         }
     } else if (tid < (1 << vb)) {
-        vtab[tid] = tmp[128 + tid];
+        reinterpret_cast<uint16_t *>(vtab)[tid] = (uint16_t)tmp[128 + tid];
     }
+    const uint32_t lead_bits = is_k || v_pairs ? 2u : 1u;                                 // bits of the window below the table index
     KvcStaged st = {};
     KvcTableState tabs = {-1, -1, -1, 0, 0};
     if (active) {
         const KvcFusedArgs &a = is_k ? j.k : j.v;
         uint32_t first, longest;
         st = kvc_stage_payload(a, lane, raw, pack, first, longest);
-        if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - 2u;                      // two bits before the lane's first code
+        if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;               // one or two bits before the lane's first code
         if (is_k) {
             const KvcTablePlan plan = {0, 1, 0};
             float bias[REP], unscale;
@@ -241,7 +245,7 @@ __global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP
 #pragma unroll
             for (int q = 0; q < NM; q++) acc[q] = kvc_f4{0.f, 0.f, 0.f, 0.f};
             uint32_t u = st.u0, bptr = kvc_lds_addr(btab) + cj * 8, msptr = kvc_lds_addr(mstab);
-            const uint32_t mask = ((1u << (k_pairs ? 2 * kb : kb)) - 1u) << 2;
+            const uint32_t mask = ((1u << (k_pairs ? 2 * kb : kb)) - 1u) << lead_bits;
             if (k_pairs) {
                 // 30 bits of a half window hold three pairs of codes of up to 5 bits, two of 6
                 int n_main = kb <= 5u ? D / 12 * 12 : 0;
@@ -265,16 +269,16 @@ __global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP
             }
         } else {
             KvcVec<REP> res;
-            if (st.fits) res = kvc_mfma_slow_tile<REP, false, true>(pack, (uint32_t)j.k.pack_logical, st.u0 + 2u, lut_k, D, btab, mstab, 0u);
+            if (st.fits) res = kvc_mfma_slow_tile<REP, false, true>(pack, (uint32_t)j.k.pack_logical, st.u0 + lead_bits, lut_k, D, btab, mstab, 0u);
             else res = kvc_mfma_slow_tile<REP, true, true>(st.gwords, st.gnwords, st.gpos, lut_k, D, btab, mstab, 0u);
 #pragma unroll
             for (int r = 0; r < REP; r++) dst[r * dst_step + lane] = res.v[r];
         }
     } else if (active) {
-        const uint32_t mask = ((1u << (v_pairs ? 2 * vb : vb)) - 1u) << 2;
+        const uint32_t mask = ((1u << (v_pairs ? 2 * vb : vb)) - 1u) << lead_bits;
         if (!v_fast || !st.fits)
             kvc_decode_bytes_slow(st.fits ? pack : st.gwords, st.fits ? (uint32_t)j.v.pack_logical : st.gnwords, st.fits,
-                                  st.fits ? st.u0 + 2u : st.gpos, lut_v, vd);
+                                  st.fits ? st.u0 + lead_bits : st.gpos, lut_v, vd);
         else if (v_pairs) kvc_decode_bytes<true>(sbase, st.u0, fe_v, mask, vd);
         else kvc_decode_bytes<false>(sbase, st.u0, fe_v, mask, vd);
     }
