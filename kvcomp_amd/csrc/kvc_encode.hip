@@ -54,6 +54,7 @@ struct KvcEncodeArgs {
     // one pass only: how often a wave may find a word of its look-back not ready before it gives up, and whether the
     // call is to be treated as if a wave had given up (both from the option "encode_lookback_polls")
     int max_polls, force_order;
+    int wave_bytes;                // one-pass kernel from symbols: LDS of a wave
 };
 
 constexpr int KVC_ENC_STATUS_WORDS = 16;            // status words in front of the per-1024-tile payload totals
@@ -1003,9 +1004,11 @@ __device__ __forceinline__ void kvc_load_code_table_marked(const KvcEncodeArgs &
 // staging area, which is free by then), and otherwise the first tile is placed and written out before the second is
 // packed -- with both sizes published long before, so that nobody waits for this wave in the meantime.
 constexpr int KVC_ONCE_WAVE_BYTES = 12560;               // three workgroups of four waves per compute unit (160 KB)
+constexpr int KVC_ONCE_SMALL_WAVE_BYTES = 9696;          // four; symbols in, tiles known to be small on average (see the launcher)
 constexpr int kvc_once_par_bytes(int front) { return front == 2 ? 4 * KVC_V_TOKENS * 4 : 0; }
 constexpr int kvc_once_stage_bytes(int front) { return front == 1 ? KVC_STAGE_K_BYTES : front == 2 ? KVC_STAGE_VF16_BYTES : KVC_STAGE_VSYM_BYTES; }
 constexpr int kvc_once_area_bytes(int front) { return KVC_ONCE_WAVE_BYTES - kvc_once_par_bytes(front); }
+static_assert(KVC_ONCE_SMALL_WAVE_BYTES >= KVC_IMAGE_WORDS * 4 && KVC_ONCE_SMALL_WAVE_BYTES % 16 == 0, "an area holds any one image");
 static_assert(KVC_STAGE_VSYM_BYTES >= KVC_STAGE_K_BYTES, "symbols in: the staging area serves K and V tiles");
 static_assert(kvc_once_area_bytes(0) - kvc_once_stage_bytes(0) >= KVC_IMAGE_WORDS * 4 &&
               kvc_once_area_bytes(1) - kvc_once_stage_bytes(1) >= KVC_IMAGE_WORDS * 4 &&
@@ -1082,8 +1085,9 @@ __global__ void __launch_bounds__(KVC_WG, 3) kvc_encode_once_kernel(KvcStoreArgs
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bool own_table = a.e.rows_per_codebook != 0;
     uint2 *s_table = reinterpret_cast<uint2 *>(s_dyn) + (own_table ? wave * 256 : 0);
-    uint8_t *s_wave = s_dyn + (own_table ? KVC_WAVES_PER_WG : 1) * 256 * sizeof(uint2) + wave * KVC_ONCE_WAVE_BYTES;
-    constexpr int PAR_BYTES = kvc_once_par_bytes(FRONT), AREA_BYTES = kvc_once_area_bytes(FRONT);
+    uint8_t *s_wave = s_dyn + (own_table ? KVC_WAVES_PER_WG : 1) * 256 * sizeof(uint2) + wave * (FRONT == 0 ? a.e.wave_bytes : KVC_ONCE_WAVE_BYTES);
+    constexpr int PAR_BYTES = kvc_once_par_bytes(FRONT);
+    const int AREA_BYTES = (FRONT == 0 ? a.e.wave_bytes : KVC_ONCE_WAVE_BYTES) - PAR_BYTES;
     uint32_t *s_par = reinterpret_cast<uint32_t *>(s_wave);
     uint32_t *area = reinterpret_cast<uint32_t *>(s_wave + PAR_BYTES);
     uint8_t *s_stage = s_wave + PAR_BYTES + AREA_BYTES - kvc_once_stage_bytes(FRONT);
@@ -1234,6 +1238,15 @@ __global__ void __launch_bounds__(KVC_WG, 3) kvc_encode_once_kernel(KvcStoreArgs
             kvc_wave_lds_sync();
         }
         if (it + 1 < run && tile + 1 < a.e.tiles) {
+            if (FRONT == 0 && cur.packs && my_words * 4u > (uint32_t)(a.e.wave_bytes - kvc_once_stage_bytes(0))) {
+                // (a wave with little LDS: the next tile's symbols need the place of this image)
+                uint32_t off = 0;
+                err |= kvc_once_place(a.e, cur, image, base, lane, &polls, &off);
+                next_off = off + cur.bn;
+                first_placed = true;
+                kvc_wave_lds_sync();
+                continue;
+            }
             pd = cur;                                      // placed together with the next tile
             continue;
         }
@@ -1515,7 +1528,15 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         a.force_order = polls_opt < 0;
         sa.e = a;
         const int front = !src ? 0 : is_k ? 1 : 2;
-        const size_t lds = (size_t)(a.rows_per_codebook ? KVC_WAVES_PER_WG : 1) * 256 * sizeof(uint2) + (size_t)KVC_WAVES_PER_WG * KVC_ONCE_WAVE_BYTES;
+        // From symbols the kernel has registers for five waves per SIMD, and LDS for three where a wave must hold any tile's
+        // image beside its staging area.  The room in `encoded` bounds the mean tile (a first store reserves what its code
+        // needs): where that leaves a fifth of margin, waves get less LDS and four of them fit; the odd run whose first image
+        // is larger is placed before its second tile is counted, as a wave's only tile would be.  402 M symbols: 316 -> 288 us,
+        // 134 M: 110 -> 101 us.
+        const bool small = front == 0 && a.rows_per_codebook == 0 &&
+                           a.encoded_cap / a.tiles <= (KVC_ONCE_SMALL_WAVE_BYTES - kvc_once_stage_bytes(0)) * 4 / 5;
+        sa.e.wave_bytes = small ? KVC_ONCE_SMALL_WAVE_BYTES : KVC_ONCE_WAVE_BYTES;
+        const size_t lds = (size_t)(a.rows_per_codebook ? KVC_WAVES_PER_WG : 1) * 256 * sizeof(uint2) + (size_t)KVC_WAVES_PER_WG * sa.e.wave_bytes;
         hipLaunchKernelGGL(kvc_encode_mark_kernel, dim3((unsigned)((a.tiles + KVC_WG - 1) / KVC_WG)), dim3(KVC_WG), 0, stream, a);
         // two tiles per wave (the look-back of the first hides behind the count of the second) where all tiles share
         // the codebook and there are enough of them to keep the chip full.  Longer runs would need the payloads of

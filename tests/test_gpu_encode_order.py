@@ -161,3 +161,38 @@ def test_forced_give_up_on_the_queued_path_leaves_no_error():
     for a, b in zip(want[:3], got[:3]):
         assert np.array_equal(a, b)
     assert int(got[3][1]) == 0 and int(got[3][0]) == want[0].size and tuple(got[3][2:5]) == tuple(want[3][2:5])
+
+
+@pytest.mark.parametrize("is_k,D", [(True, 128), (False, 128), (True, 72), (False, 96)])
+@pytest.mark.parametrize("spare", [0, 1 << 20])
+def test_small_tiles_on_average_with_large_ones_among_them(is_k, D, spare):
+    """Symbols in, with room for little more than the payload: waves then have less LDS, and a run whose first image leaves
+    no room for the second tile's symbols is placed at once.  Three tiles in ten hold some 7 KB, the others 1 KB; every order
+    of the two within a run occurs.  `spare`: room enough for the larger areas."""
+    from kvcomp_amd import _lib
+    from kvcomp_amd import kvcomp_cuda as m
+    T, B, H = 2560, 1, 3 if D == 128 else 8
+    g = torch.Generator().manual_seed(11)
+    rows, cols = (T // 64, H) if is_k else (T // 128, H * D // 64)
+    wide = torch.rand(rows, cols, generator=g) < 0.3
+    wide = wide.repeat_interleave(T // rows, 0).repeat_interleave(H * D // cols, 1)
+    sym = torch.where(wide, torch.randint(0, 40, (T, H * D), generator=g), torch.zeros((), dtype=torch.int64)).to(torch.uint8)
+    counts = torch.bincount(sym.flatten().int(), minlength=256)
+    table = m.build_codebook_from_counts(counts)[1]
+    pay, bi, ti = O.encode_tiles(sym.numpy().reshape(T // 64, 64, B, H, D), is_k, table.numpy(), 0, vec_len=D if is_k else 128)
+    sizes = bi.view(np.uint32).reshape(-1, 2)[:, 1]
+    per_tile = 64 * D if is_k else 8192
+    assert sizes.max() <= 8191 and (per_tile < 8192 or sizes.max() > 9696 - 4352) and pay.size / sizes.size < 4275
+    block, thread = (torch.zeros(n, dtype=torch.uint8, device=DEV) for n in (bi.size, ti.size))
+    payload = torch.zeros(pay.size + spare, dtype=torch.uint8, device=DEV)
+    result = torch.zeros(8, dtype=torch.int32, device=DEV)
+    tables = table.to(DEV)
+    was = _lib.set_option("encode_one_pass", 3)                 # two tiles per wave
+    try:
+        m.encode_async(is_k, batch=B, head_num=H, head_dim=D, tokens=T, symbols=sym.to(DEV), encode_tables=tables, table_bytes=tables.numel(),
+                       block_infos=block, thread_infos=thread, encoded=payload, result=result)
+        total = m.encode_result(result, payload.numel())[0]
+    finally:
+        _lib.set_option("encode_one_pass", was)
+    assert total == pay.size and np.array_equal(payload[:total].cpu().numpy(), pay)
+    assert np.array_equal(block.cpu().numpy(), bi) and np.array_equal(thread.cpu().numpy(), ti)
