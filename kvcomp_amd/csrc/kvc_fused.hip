@@ -297,13 +297,15 @@ __device__ __forceinline__ KvcStaged kvc_stage_tile(const KvcFusedArgs &a, int r
         if (s == 1 && !straddles) continue;                    // no lane of this tile belongs to a second head
         const bool live = KIND != 0 || 2 * lane < D;
         if (EXPAND == 1) continue;
-        if (EXPAND == 2) {                           // element i of slot s -> {min, scale} as two fp16 at ops[s * 128 + i]
+        if (EXPAND == 2) {   // elements 2 p and 2 p + 1 of slot s -> their minima, their scales as fp16 pairs at ops[s * 128 + 2 p], + 1
+            uint32_t mn_h[2], sc_h[2];
 #pragma unroll
             for (int half = 0; half < 2; half++) {
-                const int i = 2 * lane + half;
-                const uint32_t mn_h = __half_as_ushort(__float2half_rn((float)raw.min_int(s, half, pmode)));   // exact
-                ops[s * 128 + i] = __uint_as_float(mn_h | ((live ? raw.scale_bits(s, half, pmode) : 0u) << 16));
+                mn_h[half] = __half_as_ushort(__float2half_rn((float)raw.min_int(s, half, pmode)));            // exact
+                sc_h[half] = live ? raw.scale_bits(s, half, pmode) : 0u;
             }
+            ops[s * 128 + 2 * lane] = __uint_as_float(mn_h[0] | (mn_h[1] << 16));
+            ops[s * 128 + 2 * lane + 1] = __uint_as_float(sc_h[0] | (sc_h[1] << 16));
             continue;
         }
         float wgt[REP][2];                           // the two elements' weights: q, p, or exp(score - max)
@@ -716,12 +718,19 @@ __device__ __forceinline__ void kvc_slow_emit(const uint32_t *words, uint32_t nw
 //   K: [64 tokens][SLAB channels], rows one 32-bit word longer than the 64 bytes they carry (so that the lanes'
 //      rows start in all banks); a lane packs the elements of its own row in a register, one word at a time
 //   V: [SLAB tokens][64 channels], dense; consecutive elements of a lane lie a row apart, so they are written singly
-template <bool IS_K, bool DEQ>
+//
+// Dequantizing, the kernels are bound by latency at three to five waves per SIMD (vector ALUs 30 % busy, LDS 56 %) and by how
+// the rows are written, so the slab is as small as it can be where its size does not matter to the writes -- V, whose rows
+// are a tile's 64 channels whatever their number: 8 tokens, 32 -> 8: 76.6 -> 71.8 us at batch 8 x 32 heads x 128 x 4096
+// tokens --, and for K full cache lines are worth more than the fourth workgroup per CU: rows of 64 channels (128 bytes)
+// 84.6 us, 32 channels 90.5, 16 channels 122.8.  With codes of more than 7 bits K stays at 32 (114.5 against 139.7).
+template <bool IS_K, bool DEQ, bool HALF_ROWS>
 struct KvcSlab {
     using elem = std::conditional_t<DEQ, uint16_t, uint8_t>;
     static constexpr int ESZ = (int)sizeof(elem);
-    static constexpr int SLAB = IS_K ? 64 / ESZ : 32;          // elements per lane between two copies
-    static constexpr int K_ROW_WORDS = 64 / 4 + 1;
+    static constexpr int SLAB = IS_K ? (DEQ && HALF_ROWS ? 32 : 64) : (DEQ ? 8 : 32);   // elements per lane between two copies
+    static constexpr int K_PIECES = SLAB * ESZ / 16;           // 16-byte pieces of a K row
+    static constexpr int K_ROW_WORDS = 4 * K_PIECES + 1;
     static constexpr int WORDS = IS_K ? 64 * K_ROW_WORDS : SLAB * 64 * ESZ / 4;
 };
 
@@ -730,12 +739,12 @@ constexpr int KVC_EXPAND_LONG_WORDS = (1 << KVC_LUT_ESC_BITS) + 2 * KVC_LUT_ESC_
 #define KVC_EXPAND_OCC 1
 #endif
 // LONG: for codebooks with codes of more than 7 bits and symbols below 64
-template <int KIND, bool DEQ, bool LONG>
+template <int KIND, bool DEQ, bool LONG, bool HALF_ROWS = LONG>
 __device__ __forceinline__ void kvc_expand_body(const KvcFusedArgs &a)
 {
     constexpr bool IS_K = KIND == 0;
     constexpr int SLOTS = KvcGeom<KIND>::SLOTS;
-    using S = KvcSlab<IS_K, DEQ>;
+    using S = KvcSlab<IS_K, DEQ, HALF_ROWS>;
     using elem = typename S::elem;
     extern __shared__ __align__(16) uint32_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -816,24 +825,44 @@ __device__ __forceinline__ void kvc_expand_body(const KvcFusedArgs &a)
         const bool skew = st.fits && !a.row_words && a.skew;
         uint32_t u = st.fits ? st.u0 : st.gpos;                 // fast: lb bits before the code; slow: at the code
         if (st.fits && !fast) u += lb;
-        // the value of element i: the symbol itself, or RN16((symbol + min_i) * scale_i) (an exact fp16 sum and one
-        // fp16 multiplication).  FAST: e is a table entry of this kernel; otherwise the symbol as an fp32 pattern.
-        auto value = [&](int i, uint32_t e, bool from_table) -> uint32_t {
+        // the value of element i, symbol as an fp32 pattern: itself, or RN16((symbol + min_i) * scale_i) (an exact fp16 sum and
+        // one fp16 multiplication)
+        auto value = [&](int i, uint32_t e) -> uint32_t {
             if (DEQ) {
-                const __half sym = from_table ? __ushort_as_half((unsigned short)(e >> 16)) : __float2half_rn(__uint_as_float(e));
-                const uint32_t ms = __float_as_uint(my_ops[i]);
-                const __half mn = __ushort_as_half((unsigned short)(ms & 0xffffu)), sc = __ushort_as_half((unsigned short)(ms >> 16));
-                return (uint32_t)__half_as_ushort(__hmul(__hadd(sym, mn), sc));
+                const int shift = 16 * (i & 1);
+                const uint32_t mn = __float_as_uint(my_ops[i & ~1]) >> shift, sc = __float_as_uint(my_ops[i | 1]) >> shift;
+                const __half m = __ushort_as_half((unsigned short)mn), c = __ushort_as_half((unsigned short)sc);
+                return (uint32_t)__half_as_ushort(__hmul(__hadd(__float2half_rn(__uint_as_float(e)), m), c));
             }
             return (uint32_t)__uint_as_float(e);                           // the low mantissa bits add less than one
         };
         uint32_t *slab_w = reinterpret_cast<uint32_t *>(slab);
-        uint32_t cur = 0;
-        // fast loop: element i + g of the lane, g known at compile time
+        uint32_t cur = 0, e4[4];
+        // fast loop: element i + g of the lane, g known at compile time.  Dequantizing: four elements at a time, their
+        // parameters in one 16-byte read, two elements per fp16 instruction.
         auto put = [&](int i, auto g_, uint32_t e) {
             constexpr int g = decltype(g_)::value;
             constexpr int PER = 4 / S::ESZ;                                // elements per word
-            const uint32_t v = value(i + g, e, true);
+            if constexpr (DEQ) {
+                e4[g % 4] = e;
+                if constexpr (g % 4 == 3) {
+                    const uint4 ms = *reinterpret_cast<const uint4 *>(my_ops + i + g - 3);
+                    const uint32_t v01 = kvc_dequant_pair(kvc_pack_hi16(e4[0], e4[1]), ms.x, ms.y);
+                    const uint32_t v23 = kvc_dequant_pair(kvc_pack_hi16(e4[2], e4[3]), ms.z, ms.w);
+                    const int j = (i & (S::SLAB - 1)) + g - 3;
+                    if (IS_K) {
+                        slab_w[lane * S::K_ROW_WORDS + j / 2] = v01;
+                        slab_w[lane * S::K_ROW_WORDS + j / 2 + 1] = v23;
+                    } else {
+                        slab[j * KVC_WAVE + lane] = (elem)v01;
+                        slab[(j + 1) * KVC_WAVE + lane] = (elem)(v01 >> 16);
+                        slab[(j + 2) * KVC_WAVE + lane] = (elem)v23;
+                        slab[(j + 3) * KVC_WAVE + lane] = (elem)(v23 >> 16);
+                    }
+                }
+                return;
+            }
+            const uint32_t v = value(i + g, e);
             if (IS_K) {
                 cur = (g % PER == 0) ? v : cur | (v << (8 * S::ESZ * (g % PER)));
                 if (g % PER == PER - 1)
@@ -845,7 +874,7 @@ __device__ __forceinline__ void kvc_expand_body(const KvcFusedArgs &a)
         // slow loop: one element at a time
         auto put1 = [&](int i, uint32_t e) {
             const int j = i & (S::SLAB - 1);
-            slab[IS_K ? lane * (S::K_ROW_WORDS * 4 / S::ESZ) + j : j * KVC_WAVE + lane] = (elem)value(i, e, false);
+            slab[IS_K ? lane * (S::K_ROW_WORDS * 4 / S::ESZ) + j : j * KVC_WAVE + lane] = (elem)value(i, e);
         };
         for (int i0 = 0; i0 < n; i0 += S::SLAB) {
             const int len = n - i0 < S::SLAB ? n - i0 : S::SLAB;
@@ -865,11 +894,11 @@ __device__ __forceinline__ void kvc_expand_body(const KvcFusedArgs &a)
             // ---- copy the slab out, 16 bytes per lane and store
             constexpr int PER16 = 16 / S::ESZ;                             // elements per piece
             if (IS_K) {
-                // rows of `len` elements (64 bytes when full): four lanes per row
+                // rows of `len` elements, K_PIECES lanes per row
                 elem *out = reinterpret_cast<elem *>(a.out) + (int64_t)row * KVC_WAVE * a.s.stride + (int64_t)col * D + i0;
 #pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    const int f = lane + KVC_WAVE * t, r = f >> 2, c = f & 3;
+                for (int t = 0; t < S::K_PIECES; t++) {
+                    const int f = lane + KVC_WAVE * t, r = f / S::K_PIECES, c = f % S::K_PIECES;
                     if (c * PER16 < len) {
                         const uint32_t *src = slab_w + r * S::K_ROW_WORDS + 4 * c;
                         uint4 v = make_uint4(src[0], src[1], src[2], src[3]);
@@ -908,6 +937,12 @@ template <int KIND, bool DEQ>
 __global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_kernel(KvcFusedArgs a)
 {
     kvc_expand_body<KIND, DEQ, false>(a);
+}
+// K tiles of more than KVC_EXPAND_WIDE_TILE_BYTES, which do not fit beside a slab of whole cache lines
+constexpr int64_t KVC_EXPAND_WIDE_TILE_BYTES = 5120;
+__global__ void __launch_bounds__(KVC_WG, KVC_EXPAND_OCC) kvc_expand_big_tiles_kernel(KvcFusedArgs a)
+{
+    kvc_expand_body<0, true, false, true>(a);
 }
 // (K: V's groups are so large that few of its codebooks have such codes)
 template <bool DEQ>
@@ -1249,10 +1284,14 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
     a.q_heads = (int)heads;
     a.head_dim = (int)head_dim;
     const int slots = (!is_k && head_dim % KVC_WAVE != 0) ? 2 : 1;
-    const int out_words = is_k ? (deq ? KvcSlab<true, true>::WORDS : KvcSlab<true, false>::WORDS)
-                               : (deq ? KvcSlab<false, true>::WORDS : KvcSlab<false, false>::WORDS);
     const int code_bits = kvc_hint_bits(hints.code_hint);
     const bool long_codes = is_k && code_bits > KVC_LUT_ESC_BITS && kvc_hint_small_alphabet(hints.code_hint) && kvc_option(KVC_OPT_FUSED_ROWS) != 1;
+    const int64_t mean_tile = encoded_bytes / (rows * a.s.cols);
+    const bool big_tiles = (hints.max_tile_bytes > 0 ? hints.max_tile_bytes : mean_tile + mean_tile / 4 + 256) > KVC_EXPAND_WIDE_TILE_BYTES ||
+                           kvc_option(KVC_OPT_FUSED_ROWS) == 1;
+    const int out_words = !is_k ? (deq ? KvcSlab<false, true, false>::WORDS : KvcSlab<false, false, false>::WORDS)
+                          : !deq ? KvcSlab<true, false, false>::WORDS
+                          : long_codes || big_tiles ? KvcSlab<true, true, true>::WORDS : KvcSlab<true, true, false>::WORDS;
     const size_t lds = kvc_plan_lds(a, slots, deq ? 1 : 0, encoded_bytes, rows * a.s.cols, hints.max_tile_bytes,
                                     hints.max_stream_bytes, code_bits, out_words, true, 0, long_codes ? KVC_EXPAND_LONG_WORDS : 0);
     a.expand = deq ? 2 : 1;
@@ -1273,7 +1312,8 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
         if (deq) hipLaunchKernelGGL(kvc_expand_long_kernel<true>, grid, dim3(KVC_WG), lds, stream, a);
         else hipLaunchKernelGGL(kvc_expand_long_kernel<false>, grid, dim3(KVC_WG), lds, stream, a);
     } else if (deq) {
-        if (kind == 0) KVC_EXPAND_LAUNCH(0, true);
+        if (kind == 0 && big_tiles) hipLaunchKernelGGL(kvc_expand_big_tiles_kernel, grid, dim3(KVC_WG), lds, stream, a);
+        else if (kind == 0) KVC_EXPAND_LAUNCH(0, true);
         else if (kind == 1) KVC_EXPAND_LAUNCH(1, true);
         else KVC_EXPAND_LAUNCH(2, true);
     } else {

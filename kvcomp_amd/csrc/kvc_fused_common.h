@@ -160,6 +160,18 @@ __device__ __forceinline__ float kvc_rounded_value(__half sym, uint32_t ms)
     return __half2float(__hmul(__hadd(sym, mn), sc));
 }
 
+typedef _Float16 kvc_h2 __attribute__((ext_vector_type(2)));
+// {x.lo, x.hi} -> RN16((x + mn) * sc) per half: the sum of two small integers is exact in fp16, the product is
+// rounded once
+__device__ __forceinline__ uint32_t kvc_dequant_pair(uint32_t x, uint32_t mn, uint32_t sc)
+{
+    const kvc_h2 v = (__builtin_bit_cast(kvc_h2, x) + __builtin_bit_cast(kvc_h2, mn)) * __builtin_bit_cast(kvc_h2, sc);
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+// upper halves of two table entries side by side: {a >> 16, b >> 16 << 16}
+__device__ __forceinline__ uint32_t kvc_pack_hi16(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+
 template <int REP>
 struct KvcVec {
     float v[REP];

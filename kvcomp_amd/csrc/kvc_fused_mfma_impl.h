@@ -34,7 +34,6 @@
 #pragma once
 #include "kvc_fused_common.h"
 
-typedef _Float16 kvc_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 kvc_h4 __attribute__((ext_vector_type(4)));
 typedef float kvc_f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t kvc_w2 __attribute__((ext_vector_type(2)));
@@ -75,17 +74,6 @@ __device__ __forceinline__ kvc_w2 kvc_read_columns(uint32_t addr, bool holder)
     if (!BCAST || holder) b = *(const kvc_lds_w2 *)(uintptr_t)addr;
     return b;
 }
-
-// {x.lo, x.hi} -> RN16((x + mn) * sc) per half: the sum of two small integers is exact in fp16, the product is
-// rounded once
-__device__ __forceinline__ uint32_t kvc_dequant_pair(uint32_t x, uint32_t mn, uint32_t sc)
-{
-    const kvc_h2 v = (__builtin_bit_cast(kvc_h2, x) + __builtin_bit_cast(kvc_h2, mn)) * __builtin_bit_cast(kvc_h2, sc);
-    return __builtin_bit_cast(uint32_t, v);
-}
-
-// upper halves of two table entries side by side: {a >> 16, b >> 16 << 16}
-__device__ __forceinline__ uint32_t kvc_pack_hi16(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 
 // -- operand tables -----------------------------------------------------------------------------------
 // btab  [slot][group g][set][column j][element k]  fp16: weight part of element 4 g + k for column 4 set + j;
