@@ -109,11 +109,15 @@ class _Growable:
     def __init__(self):
         self.data: Optional[torch.Tensor] = None
         self.used = 0
-        self.address = 0          # of `data`, and elements per row of it: kept beside it for callers on the per-token path
-        self.row = 1
+        self.row = 1              # elements per row of `data`
 
     def _hold(self, data: torch.Tensor):
-        self.data, self.address, self.row = data, data.data_ptr(), math.prod(data.shape[1:])
+        self.data, self.row = data, math.prod(data.shape[1:])
+
+    @property
+    def address(self) -> int:
+        """Of `data`; asked for every time, since a copy of this object holds memory of its own."""
+        return self.data.data_ptr()
 
     def append(self, t: torch.Tensor):
         n = t.shape[0]
@@ -231,6 +235,14 @@ class KVCompCtx:
         self._host_words: Optional[torch.Tensor] = None
         self._trim_after_sync = False
         self.waits = 0                     # how often this context has waited for the device to learn sizes
+
+    def __getstate__(self):
+        # (copies and pickles: the descriptor holds addresses and is refilled on every use)
+        return {name: value for name, value in self.__dict__.items() if name != "_descriptor"}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._descriptor = _lib.CompressedDesc()
 
     def _device_state(self) -> torch.Tensor:
         if self._state is None:

@@ -1,0 +1,60 @@
+"""Contexts can be copied like any object that holds tensors: a copy has memory of its own, and nothing in it refers to the
+original's."""
+import copy
+import pickle
+
+import pytest
+import torch
+
+from kvcomp_amd.cache import KVCompCache
+from kvcomp_amd.ctx import KVCompCacheConfig, KVCompCacheConfigStatic, KVCompCtx, QuantMode
+
+
+def _config():
+    KVCompCacheConfigStatic.config = KVCompCacheConfig("t", QuantMode.ChannelQuant, QuantMode.TokenQuant, 64, 128, 64, 128, 0.1, 0.2)
+
+
+@pytest.mark.parametrize("how", [copy.deepcopy, lambda x: pickle.loads(pickle.dumps(x))])
+def test_a_copy_refers_to_its_own_memory(how):
+    _config()
+    ctx = KVCompCtx(True, 1, 2, 64, 0.1)
+    for g in (ctx._encoded, ctx._block_infos, ctx._thread_infos, ctx._min_ints, ctx._scales):
+        g.append(torch.arange(40, dtype=torch.uint8))
+    ctx.decode_codebook = ctx._lut_source = torch.zeros(6, dtype=torch.uint8)
+    ctx._lut = torch.zeros(4)
+    got = how(ctx)
+    for name in ("_encoded", "_block_infos", "_thread_infos", "_min_ints", "_scales"):
+        mine, theirs = getattr(got, name), getattr(ctx, name)
+        assert torch.equal(mine.view, theirs.view) and mine.address == mine.data.data_ptr() != theirs.address
+    assert got._descriptor is not ctx._descriptor
+    assert got._lut_source is got.decode_codebook            # the copy's tables still belong to its codebook
+
+
+def test_moved_data_is_seen():
+    _config()
+    g = KVCompCtx(False, 1, 2, 64, 0.2)._encoded
+    g.append(torch.zeros(8, dtype=torch.uint8))
+    g.data = g.data.clone()
+    assert g.address == g.data.data_ptr()
+
+
+def test_dense_caches_can_be_copied():
+    _config()
+    copy.deepcopy(KVCompCache(1, 2, 64, 2))
+
+
+@pytest.mark.gpu
+def test_attention_over_a_copy_outlives_the_original():
+    from kvcomp_amd.attention import CompressedAttention
+    from tests import _synth as S
+    _config()
+    pair = KVCompCtx(True, 1, 4, 128, 0.1), KVCompCtx(False, 1, 4, 128, 0.2)
+    for c, x in zip(pair, (S.synth_k(300, 1, 4, 128), S.synth_v(300, 1, 4, 128))):
+        c.store(x.to("cuda:0"))
+    q = S.synth_q(1, 4, 128).to("cuda:0")
+    want = CompressedAttention(*pair).attend(q)
+    twin = copy.deepcopy(pair)
+    for c in pair:
+        for g in (c._encoded, c._block_infos, c._thread_infos, c._min_ints, c._scales):
+            g.data.zero_()
+    assert torch.equal(CompressedAttention(*twin).attend(q), want)
