@@ -118,16 +118,25 @@ class _Here:
 _HERE_GUARD = _Here()
 
 
+def _not_on_a_gpu(t):
+    return ValueError("Expected a cuda device, but got: %s" % t.device)
+
+
 def device_guard(t):
     """`with` this around a library call on the tensor's device: torch.cuda.device, where that is not current already (the
-    guard costs a microsecond, a fifth of a launch)."""
+    guard costs a microsecond, a fifth of a launch).  A tensor in host memory is refused: its address is none for a kernel."""
     index = t.get_device()
+    if index < 0:
+        raise _not_on_a_gpu(t)
     return _HERE_GUARD if torch._C._cuda_getDevice() == index else torch.cuda.device(index)
 
 
 def stream_of(t) -> int:
     """Address of the current stream of the tensor's device, without an object for it."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    index = t.get_device()
+    if index < 0:
+        raise _not_on_a_gpu(t)
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 class KvcompError(RuntimeError):

@@ -16,7 +16,7 @@ from typing import Optional
 import torch
 
 from . import _lib, kvcomp_cuda
-from ._lib import check
+from ._lib import KvcompError, check
 from .compute import dims_to_mask
 from .ctx import KVCompCtx
 from .kvcomp_cuda import build_lut  # noqa: F401
@@ -101,6 +101,8 @@ class CompressedAttention:
         B, Hq, D = q.shape
         k, v = self.k, self.v
         assert q.dtype is torch.float16 and v.ctx_len == k.ctx_len
+        if not q.device == k.device == v.device:
+            raise KvcompError("queries on %s, keys on %s, values on %s" % (q.device, k.device, v.device))
         if scale is None:
             scale = 1.0 / math.sqrt(D)
         L = _lib.lib()

@@ -138,7 +138,7 @@ def quant_in_place(region: torch.Tensor, block_size: int, quant_scale_rel: float
     B, H, T, D = region.shape
     if T == 0:
         return
-    if region.stride(3) == 1 and region.stride(2) == D:
+    if region.is_cuda and region.dtype is torch.float16 and region.stride(3) == 1 and region.stride(2) == D:
         with _lib.device_guard(region):
             rc = _lib.lib().kvc_quant_in_place(_ptr(region), B, H, T, D, region.stride(0), region.stride(1), block_size,
                                                _SIM_PLAN[quant_mode][1], float(quant_scale_rel), _stream(region))
@@ -169,7 +169,7 @@ def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], 
         return False
     cos_p = sin_p = cb = ct = sb = st = 0
     if cos is not None:
-        if not (cos.dtype is f16 and sin.dtype is f16 and cos.is_cuda and sin.is_cuda and cos.shape == sin.shape and
+        if not (cos.dtype is f16 and sin.dtype is f16 and cos.device == sin.device == k.device and cos.shape == sin.shape and
                 cos.dim() == 3 and cos.shape[0] in (1, B) and cos.shape[1] == T and cos.shape[2] == D):
             return False
         (cb, ct, cd), (sb, st, sd) = cos.stride(), sin.stride()

@@ -186,7 +186,9 @@ def loads(data: bytes, device: Optional[torch.device] = None) -> KVCompCtx:
     cfg = KVCompCacheConfigStatic.config
     if cfg is None:
         raise ContainerError("KVCompCacheConfigStatic.config must be set before loading (written with: %s)" % header["config"])
-    device = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
+    device = torch.device(device if device is not None else "cuda")
+    if device.type == "cuda" and device.index is None:           # as tensors name it
+        device = torch.device("cuda", torch.cuda.current_device())
     ctx = KVCompCtx(header["is_k"], header["batch_size"], header["head_num"], header["head_dim"], header["quant_scale_rel"])
     if (ctx.block_size, ctx.recent_size, [int(d) for d in ctx.quant_dims]) != (header["block_size"], header["recent_size"], header["quant_dims"]):
         raise ContainerError("the active cache configuration (block %d, recent %d, dims %s) differs from the one the stream was "

@@ -372,7 +372,7 @@ class KVCompCtx:
             self._tail = grown
         row = self._row_bytes
         to, src = self._tail.data_ptr() + self._tail_len * row, cache.data_ptr()
-        if n and (to | src | row) & 15 == 0 and cache.is_contiguous():
+        if n and (to | src | row) & 15 == 0 and cache.is_cuda and cache.is_contiguous():
             kvcomp_cuda.copy_rows(self._tail, to, src, n * row)      # (half the host time of an assignment to a slice)
         elif n:
             self._tail[self._tail_len:self._tail_len + n] = cache
