@@ -217,6 +217,8 @@ def loads(data: bytes, device: Optional[torch.device] = None) -> KVCompCtx:
     ctx.pair_bits = header.get("pair_bits", 0)
     ctx.max_tile_bytes = header["max_tile_bytes"]
     ctx.max_stream_bytes = header["max_stream_bytes"]
+    if ctx.decode_codebook is not None:
+        ctx._build_lut()
     KVCompCtx.buffer_ctx_len.setdefault(device, 0)
     return ctx
 

@@ -577,6 +577,7 @@ class KVCompCtx:
             self._sync_sizes()                                 # (a failure leaves the context as it was before the encode)
         self.tree_format, self.max_code_bits, self.pair_bits = book.tree_format, book.max_code_bits, book.pair_bits
         self.encode_codebook, self.decode_codebook = enc, dec
+        self._build_lut()
         return sym
 
     def _smoothed_symbols(self) -> int:
@@ -647,12 +648,23 @@ class KVCompCtx:
         table = self.encode_codebook
         return self.max_code_bits | self.pair_bits << 12 | (0x100 if table is not None and table.shape[0] <= 64 * 8 else 0)
 
-    def decode_lut(self) -> Optional[torch.Tensor]:
-        """The decode tables of this context's codebook (kvc_build_lut), built once per codebook; None before the first
-        block has been compressed."""
-        if self._lut_source is not self.decode_codebook:
+    def _build_lut(self):
+        """The decode tables of the codebook that has just been put in place, on the stream that put it there: whoever is
+        ordered behind that, on whatever stream, finds them built."""
+        if self.decode_codebook.is_cuda:
             self._lut = kvcomp_cuda.build_lut(self.decode_codebook, self.tree_format)
             self._lut_source = self.decode_codebook
+
+    def decode_lut(self) -> Optional[torch.Tensor]:
+        """The decode tables of this context's codebook (kvc_build_lut); None before the first block has been compressed."""
+        if self._lut_source is not self.decode_codebook:
+            # a codebook assigned from outside, on a stream that nobody can name: the tables are waited for once, so that
+            # other streams may read them.  While the stream is being recorded nothing is built yet: the graph builds tables
+            # of its own, and they are not taken for ones that anyone else can use.
+            self._lut = kvcomp_cuda.build_lut(self.decode_codebook, self.tree_format)
+            if not torch.cuda.is_current_stream_capturing():
+                torch.cuda.current_stream(self._lut.device).synchronize()
+                self._lut_source = self.decode_codebook
         return self._lut
 
     def descriptor(self) -> "_lib.CompressedDesc":
@@ -760,6 +772,7 @@ class KVCompCtx:
         self.max_code_bits = int(lengths.max())      # sizes the fused decoders' table in LDS
         self.encode_codebook = enc.to(self.device)
         self.decode_codebook = dec.to(self.device)
+        self._build_lut()
 
     @property
     def shape(self):
