@@ -15,7 +15,7 @@ import ast
 import ctypes as C
 import math
 import struct
-from typing import Dict, List, Optional, Tuple
+from typing import Dict, List, NamedTuple, Optional, Tuple
 
 import torch
 
@@ -158,6 +158,17 @@ class _Growable:
         return None if self.data is None else self.data[:self.used]
 
 
+class _QueuedStore(NamedTuple):
+    """An encode that was queued and has not been seen to succeed."""
+    tokens: int
+    rows: Optional[torch.Tensor]     # its tokens' fp16 rows, if they were kept
+    books: tuple                     # the bookkeeping as it stood right after the store
+    worst: int                       # the store's share of _enc_pending
+    lost: bool                       # its tokens are gone if it has to be taken back: counted in ctx_len, rows not kept
+    certain: bool                    # nothing about it can fail, whatever a later store does
+    codebook: bool                   # it brought the codebook, which goes with it
+
+
 # the seventeen 8-byte fields of kvc_compressed_desc, in order
 _DESC = struct.Struct("=17q")
 
@@ -224,12 +235,10 @@ class KVCompCtx:
         # word 8 counts the payload bytes in _encoded; _enc_pending bounds the bytes the host has not learnt of yet
         self._state: Optional[torch.Tensor] = None
         self._enc_pending = 0
-        # Stores that were queued and not yet seen to succeed, oldest first: (tokens, their fp16 rows or None, the
-        # bookkeeping as it stood right after the store, the store's share of _enc_pending, whether the tokens are gone
-        # if the store has to be taken back: counted in ctx_len, rows not kept); _verified is the
-        # bookkeeping behind the last store that is known to be good.  _probe = (event, stores covered) while a copy of
-        # the device words to _host_words (pinned) is on its way: reading it later costs no wait.
-        self._unverified: list = []
+        # Stores that were queued and not yet seen to succeed, oldest first; _verified is the bookkeeping behind the last
+        # store that is known to be good.  _probe = (event, stores covered) while a copy of the device words to
+        # _host_words (pinned) is on its way: reading it later costs no wait.
+        self._unverified: List[_QueuedStore] = []
         self._verified = None
         self._probe = None
         self._host_words: Optional[torch.Tensor] = None
@@ -280,11 +289,11 @@ class KVCompCtx:
         """The first n_stores queued stores are done and good; `used` payload bytes lie in _encoded behind them."""
         done, self._unverified = self._unverified[:n_stores], self._unverified[n_stores:]
         self._encoded.used = used
-        self._enc_pending = sum(u[3] for u in self._unverified)
+        self._enc_pending = sum(u.worst for u in self._unverified)
         self.max_tile_bytes = max(self.max_tile_bytes, max_tile)
         self.max_stream_bytes = max(self.max_stream_bytes, max_stream)
         if done:
-            self._verified = done[-1][2] + (used,)
+            self._verified = done[-1].books + (used,)
         if self._trim_after_sync and not self._unverified:
             self._trim_after_sync = False
             self._encoded.trim()                               # a byte per symbol was reserved; the stream is a fraction of it
@@ -292,9 +301,19 @@ class KVCompCtx:
     def _roll_back(self):
         """Back to the last store that is known to be good: the stores queued since then are dropped from the
         bookkeeping, the device's words say so too, and the tokens of those stores return to the front of the tail
-        (rows that were not kept -- stores recorded into a graph -- are lost and leave ctx_len)."""
+        (rows that were not kept -- stores recorded into a graph -- are lost and leave ctx_len).  A store that cannot fail
+        is good even if nobody has looked at it yet; where its payload ends is what its last tile says."""
         if self._verified is None:
             return
+        good = 0
+        while good < len(self._unverified) and self._unverified[good].certain:
+            good += 1
+        dropped = self._unverified[good:]
+        if good:
+            books = self._unverified[good - 1].books
+            infos = self._block_infos.data[:books[0]].cpu().view(torch.int32)            # {offset, byte_num} per tile
+            self.max_tile_bytes = max(self.max_tile_bytes, int((infos[1::2] & 0xffff).max()))
+            self._verified = books + ((int(infos[-2]) & 0xffffffff) + (int(infos[-1]) & 0xffff),)
         (self._block_infos.used, self._thread_infos.used, self._min_ints.used, self._scales.used, self.compressed_ctx_len,
          self._encoded.used) = self._verified
         st = self._state
@@ -302,13 +321,16 @@ class KVCompCtx:
         st[4] = self._block_infos.used // 8
         st[8] = self._encoded.used
         self._enc_pending = 0
-        rows = [u[1] for u in self._unverified if u[1] is not None]
-        self.ctx_len -= sum(u[0] for u in self._unverified if u[4])
+        rows = [u.rows for u in dropped if u.rows is not None]
+        self.ctx_len -= sum(u.tokens for u in dropped if u.lost)
         if rows:
             if self._tail_len:
                 rows.append(self._tail[:self._tail_len])
             self._tail = torch.cat(rows, dim=0)
             self._tail_len = self._tail.shape[0]
+        if any(u.codebook for u in dropped):
+            self.encode_codebook = self.decode_codebook = self._lut = self._lut_source = None
+            self.tree_format, self.max_code_bits, self.pair_bits = kvcomp_cuda.TREE_I8, 0, 0
         self._unverified = []
         self._probe = None
 
@@ -518,7 +540,7 @@ class KVCompCtx:
     ASYNC_KEEP_BLOCKS = 8
 
     def _encode_direct(self, T: int, *, tables, table_bytes, symbols=None, cache=None, mask=0, most_bytes=None, keep=None,
-                       lost_if_dropped=False):
+                       lost_if_dropped=False, certain=False, codebook=False):
         """Queue one encode whose outputs go straight to their final places in this context's buffers; nothing waits.
         Quantizes `cache` on the fly (fused store) or takes `symbols` whose parameters are in place already.  most_bytes:
         what the payload is known not to exceed."""
@@ -549,7 +571,7 @@ class KVCompCtx:
         self._scales.used += nb
         self._enc_pending += worst
         self.compressed_ctx_len += T
-        self._unverified.append((T, keep, self._bookkeeping(), worst, lost_if_dropped))
+        self._unverified.append(_QueuedStore(T, keep, self._bookkeeping(), worst, lost_if_dropped, certain, codebook))
 
     def _first_chunk(self, blocked: torch.Tensor) -> torch.Tensor:
         """The first stored chunk: quantized, its codebook built from the symbols just written (kvcomp_encode.py:86-103; the
@@ -570,7 +592,7 @@ class KVCompCtx:
         small = T <= self.ASYNC_KEEP_BLOCKS * self.block_size
         queued = self.async_store and (cannot_fail or small)
         self._encode_direct(T, symbols=sym, tables=enc, table_bytes=enc.numel(), most_bytes=book.payload_bits // 8 + vectors + 1,
-                            keep=blocked.flatten(0, 1).clone() if queued and not cannot_fail else None)
+                            keep=blocked.flatten(0, 1).clone() if queued and not cannot_fail else None, certain=cannot_fail, codebook=True)
         if queued:
             self._issue_probe()
         else:
