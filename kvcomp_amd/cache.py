@@ -26,7 +26,7 @@ from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
-from .compute import append_dense, apply_rotary_pos_emb_single, blocks_to_compress, quant_in_place, safe_cat
+from .compute import append_dense, apply_rotary_pos_emb_single, blocks_to_compress, quant_in_place, safe_cat, takes_append
 from .ctx import KVCompCacheConfigStatic, KVCompCtx
 
 
@@ -48,9 +48,12 @@ class _DenseHistory:
         self.length = 0
         self.quantized = 0        # leading tokens already replaced by their simulated-quantization values
 
+    def has_room(self, n: int) -> bool:
+        return self.data is not None and self.length + n <= self.data.shape[2]
+
     def make_room(self, t: torch.Tensor):
         n = t.shape[2]
-        if self.data is None or self.length + n > self.data.shape[2]:
+        if not self.has_room(n):
             cap = max(2 * (self.length + n), 256)
             grown = torch.empty(t.shape[0], t.shape[1], cap, t.shape[3], dtype=t.dtype, device=t.device)
             if self.data is not None:
@@ -122,19 +125,23 @@ class KVCompCachePytorchQuant:
     # -- helpers ---------------------------------------------------------------------------------------
     def _append(self, key_states, value_states, layer_idx, cache_kwargs):
         """The new tokens behind both histories of the layer, in one launch where the tensors allow it; keys rotated,
-        unless they are stored un-rotated with the angles beside them.  """
+        unless they are stored un-rotated with the angles beside them."""
         cos, sin = cache_kwargs['cos'], cache_kwargs['sin']
         k, v = self._k[layer_idx], self._v[layer_idx]
         if _config().enable_pre_rope:
             self.coss[layer_idx] = safe_cat(self.coss[layer_idx], cos, dim=1)
             self.sins[layer_idx] = safe_cat(self.sins[layer_idx], sin, dim=1)
             cos = sin = None
-        k.make_room(key_states)
-        v.make_room(value_states)
-        if k.length == v.length and append_dense(key_states, value_states, cos, sin, k.data, v.data, k.length):
-            k.length += key_states.shape[2]
-            v.length += value_states.shape[2]
-            return
+        # (the histories take the type and shape of what is appended first: of the rotated keys, which differ from the keys'
+        # own where the angles are wider)
+        n = key_states.shape[2]
+        if k.length == v.length and (k.has_room(n) and v.has_room(n) or takes_append(key_states, value_states, cos, sin)):
+            k.make_room(key_states)
+            v.make_room(value_states)
+            if append_dense(key_states, value_states, cos, sin, k.data, v.data, k.length):
+                k.length += n
+                v.length += n
+                return
         if cos is not None:
             key_states = apply_rotary_pos_emb_single(key_states, cos, sin)
         k.append(key_states)

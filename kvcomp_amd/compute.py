@@ -153,28 +153,34 @@ def quant_in_place(region: torch.Tensor, block_size: int, quant_scale_rel: float
 _APPEND = struct.Struct("=22q")
 
 
+def takes_append(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor]) -> bool:
+    """Whether append_dense takes these rows and angles: fp16 on one GPU, elements of a row adjacent, angles for every
+    token, shared by the batch or not.  The rotated keys are then what the keys are: fp16 of the same shape."""
+    f16 = torch.float16
+    if not (k.dtype is f16 and v.dtype is f16 and k.is_cuda and k.device == v.device and v.shape == k.shape and k.dim() == 4 and
+            k.shape[3] % 2 == 0 and k.stride(3) == 1 and v.stride(3) == 1):
+        return False
+    return cos is None or (cos.dtype is f16 and sin.dtype is f16 and cos.device == sin.device == k.device and
+                           cos.shape == sin.shape and cos.dim() == 3 and cos.shape[0] in (1, k.shape[0]) and
+                           cos.shape[1:] == k.shape[2:] and cos.stride(2) == 1 and sin.stride(2) == 1)
+
+
 def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], k_cache: torch.Tensor,
                  v_cache: torch.Tensor, at: int) -> bool:
     """kvc_append_dense: k (rotated by cos / sin [1 or B, T, D], unless they are None) and v, [B, H, T, D] fp16, to
     positions at .. of the [B, H, capacity, D] caches.  False, having done nothing, for tensors it does not take."""
+    if not takes_append(k, v, cos, sin):
+        return False
     B, H, T, D = k.shape
     f16 = torch.float16
-    if not (k.dtype is f16 and v.dtype is f16 and k.is_cuda and v.is_cuda and D % 2 == 0 and v.shape == k.shape and
-            k.device == v.device == k_cache.device == v_cache.device and k_cache.dtype is f16 and v_cache.dtype is f16 and
-            k_cache.shape == v_cache.shape == (B, H, k_cache.shape[2], D)):
+    if not (k_cache.dtype is f16 and v_cache.dtype is f16 and k.device == k_cache.device == v_cache.device and
+            k_cache.shape == v_cache.shape == (B, H, k_cache.shape[2], D) and k_cache.is_contiguous() and v_cache.is_contiguous()):
         return False
-    kb, kh, kt, kd = k.stride()
-    vb, vh, vt, vd = v.stride()
-    if kd != 1 or vd != 1:
-        return False
+    kb, kh, kt, _ = k.stride()
+    vb, vh, vt, _ = v.stride()
     cos_p = sin_p = cb = ct = sb = st = 0
     if cos is not None:
-        if not (cos.dtype is f16 and sin.dtype is f16 and cos.device == sin.device == k.device and cos.shape == sin.shape and
-                cos.dim() == 3 and cos.shape[0] in (1, B) and cos.shape[1] == T and cos.shape[2] == D):
-            return False
-        (cb, ct, cd), (sb, st, sd) = cos.stride(), sin.stride()
-        if cd != 1 or sd != 1:
-            return False
+        (cb, ct, _), (sb, st, _) = cos.stride(), sin.stride()
         if cos.shape[0] == 1:
             cb = sb = 0
         cos_p, sin_p = cos.data_ptr(), sin.data_ptr()

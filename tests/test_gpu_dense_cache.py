@@ -10,6 +10,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
+def _no_quant():
+    from kvcomp_amd.ctx import KVCompCacheConfig, KVCompCacheConfigStatic
+    KVCompCacheConfigStatic.extract_cache = None
+    KVCompCacheConfigStatic.config = KVCompCacheConfig("t", None, None, None, None, None, None, None, None, enable_quant=False)
+
+
 # groups of every layout: head_dim off 16 elements, blocks that do not fit a thread's registers, tokens that take a
 # wave's registers (up to 8192 elements), a workgroup's (two sizes) and more than those
 @pytest.mark.parametrize("mode,B,H,T,D,bs", [
@@ -60,3 +66,28 @@ def test_appended_rows_equal_the_rotation_in_pytorch(B, H, T, D, at, angles):
         assert torch.equal(cache[:, :, at:at + T].contiguous().view(torch.int16), rows.contiguous().view(torch.int16))
         assert (cache[:, :, :at] == 7).all() and (cache[:, :, at + T:] == 7).all()
     assert not append_dense(k, v, cos, sin, kc[:, :, :, :D - 2], vc[:, :, :, :D - 2], at)    # a cache of another shape
+
+
+@pytest.mark.parametrize("wide", ["cos", "sin", "both"])
+def test_angles_in_fp32_keep_the_keys_in_fp32(wide):
+    """The rotation of fp16 keys by fp32 angles is fp32 in PyTorch, and the history holds it as it is."""
+    from kvcomp_amd.cache import KVCompCachePytorchQuant
+    from kvcomp_amd.compute import apply_rotary_pos_emb_single
+    _no_quant()
+    k = S.synth_k(12, 2, 3, 64).permute(1, 2, 0, 3).contiguous().to(DEV)
+    cos, sin = (t.to(DEV).float() if wide in (n, "both") else t.to(DEV) for t, n in zip(_rope(12, 64), ("cos", "sin")))
+    cache = KVCompCachePytorchQuant(2, 3, 64, 1)
+    for lo, hi in ((0, 10), (10, 11), (11, 12)):
+        keys, values = cache.update(k[:, :, lo:hi], k[:, :, lo:hi], 0, {"cos": cos[:, lo:hi], "sin": sin[:, lo:hi]})
+    want = apply_rotary_pos_emb_single(k, cos, sin)
+    assert want.dtype is torch.float32 and torch.equal(keys, want) and keys.dtype is torch.float32 and torch.equal(values, k)
+
+
+def test_angles_of_several_sequences_spread_the_keys_of_one():
+    from kvcomp_amd.cache import KVCompCachePytorchQuant
+    from kvcomp_amd.compute import apply_rotary_pos_emb_single
+    _no_quant()
+    k = S.synth_k(5, 1, 3, 64).permute(1, 2, 0, 3).contiguous().to(DEV)
+    cos, sin = (torch.cat([t[:, :5], t[:, 5:10]]).to(DEV) for t in _rope(10, 64))
+    keys, _ = KVCompCachePytorchQuant(1, 3, 64, 1).update(k, k, 0, {"cos": cos, "sin": sin})
+    assert torch.equal(keys, apply_rotary_pos_emb_single(k, cos, sin))

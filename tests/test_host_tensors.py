@@ -101,3 +101,11 @@ def test_the_dense_cache_works_on_host_tensors_until_a_block_is_quantized():
     one, zero = torch.ones(1, 20, 64, dtype=torch.float16), torch.zeros(1, 20, 64, dtype=torch.float16)
     k, v = cache.update(x, x, 0, {"cos": one, "sin": zero})
     assert torch.equal(k, x) and torch.equal(v, x)
+
+
+def test_angles_in_fp32_keep_the_keys_in_fp32():
+    cache = KVCompCachePytorchQuant(1, 2, 64, 1)
+    k = torch.randn(1, 2, 3, 64, generator=torch.Generator().manual_seed(1)).to(torch.float16)
+    cos, sin = (torch.rand(1, 3, 64, generator=torch.Generator().manual_seed(s)) for s in (2, 3))
+    keys, values = cache.update(k, k, 0, {"cos": cos, "sin": sin})
+    assert keys.dtype is torch.float32 and torch.equal(keys, compute.apply_rotary_pos_emb_single(k, cos, sin)) and values.dtype is torch.float16
