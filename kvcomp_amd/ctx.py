@@ -246,8 +246,10 @@ class KVCompCtx:
         self.waits = 0                     # how often this context has waited for the device to learn sizes
 
     def __getstate__(self):
-        # (copies and pickles: the descriptor holds addresses and is refilled on every use)
-        return {name: value for name, value in self.__dict__.items() if name != "_descriptor"}
+        # (copies and pickles: the descriptor holds addresses and is refilled on every use.  Queued stores are waited for: a
+        # copy cannot share the event and the pinned words that will say what became of them.)
+        self._sync_sizes()
+        return {**{name: value for name, value in self.__dict__.items() if name != "_descriptor"}, "_probe": None, "_host_words": None}
 
     def __setstate__(self, state):
         self.__dict__.update(state)

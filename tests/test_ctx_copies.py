@@ -30,6 +30,32 @@ def test_a_copy_refers_to_its_own_memory(how):
     assert got._lut_source is got.decode_codebook            # the copy's tables still belong to its codebook
 
 
+@pytest.mark.parametrize("how", [copy.deepcopy, lambda x: pickle.loads(pickle.dumps(x))])
+def test_a_queued_store_is_waited_for(how, monkeypatch):
+    """A context whose store has not been looked at yet holds an event and pinned words, which no copy can have."""
+    from kvcomp_amd import kvcomp_cuda
+    from kvcomp_amd.ctx import _QueuedStore
+
+    class Event:                                              # like torch.cuda.Event: cannot be pickled
+        def __reduce__(self):
+            raise TypeError("cannot pickle 'Event' object")
+    _config()
+    ctx = KVCompCtx(True, 1, 2, 64, 0.1)
+    for g in (ctx._encoded, ctx._block_infos, ctx._thread_infos, ctx._min_ints, ctx._scales):
+        g.append(torch.arange(40, dtype=torch.uint8))
+    ctx._state = torch.zeros(16, dtype=torch.int32)
+    ctx._state[8] = 33
+    ctx._verified = ctx._bookkeeping() + (0,)
+    ctx._unverified = [_QueuedStore(64, None, ctx._bookkeeping(), 40, False, True, True)]
+    ctx._enc_pending, ctx._encoded.used = 40, 0
+    ctx._host_words, ctx._probe = torch.zeros(16, dtype=torch.int32), (Event(), 0, None)
+    monkeypatch.setattr(kvcomp_cuda, "encode_result", lambda *a: (33, 20, 9, 1))
+    got = how(ctx)
+    for c in (got, ctx):
+        assert c._encoded.used == 33 and c._enc_pending == 0 and not c._unverified and c.max_tile_bytes == 20
+    assert got._probe is None and got._host_words is None
+
+
 def test_moved_data_is_seen():
     _config()
     g = KVCompCtx(False, 1, 2, 64, 0.2)._encoded
@@ -58,3 +84,24 @@ def test_attention_over_a_copy_outlives_the_original():
         for g in (c._encoded, c._block_infos, c._thread_infos, c._min_ints, c._scales):
             g.data.zero_()
     assert torch.equal(CompressedAttention(*twin).attend(q), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", [copy.deepcopy, lambda x: pickle.loads(pickle.dumps(x))])
+def test_contexts_as_the_model_caches_hold_them_can_be_copied_right_after_a_store(how):
+    from kvcomp_amd.attention import CompressedAttention
+    from tests import _synth as S
+    _config()
+    pair = KVCompCtx(True, 1, 4, 128, 0.1), KVCompCtx(False, 1, 4, 128, 0.2)
+    for c, x in zip(pair, (S.synth_k(300, 1, 4, 128), S.synth_v(300, 1, 4, 128))):
+        c.codebook_smoothing = c.async_store = True
+        c.store(x.to("cuda:0"), want_symbols=False)
+        assert c._probe is not None
+    twin = how(pair)
+    q = S.synth_q(1, 4, 128).to("cuda:0")
+    want = CompressedAttention(*pair).attend(q)
+    for c, x in zip(twin, (S.synth_k(1, 1, 4, 128, 5), S.synth_v(1, 1, 4, 128, 5))):
+        assert torch.equal(c.encoded_data, pair[0 if c.is_k else 1].encoded_data)
+        c.store(x.to("cuda:0"), want_symbols=False)               # the copy goes on by itself
+    assert pair[0].ctx_len == 300 and twin[0].ctx_len == 301
+    assert torch.equal(CompressedAttention(*pair).attend(q), want)
