@@ -47,6 +47,7 @@ class _DenseHistory:
         self.data: Optional[torch.Tensor] = None
         self.length = 0
         self.quantized = 0        # leading tokens already replaced by their simulated-quantization values
+        self.updates = 0          # how often the cache has been updated: views made before the last one are out of date
 
     def has_room(self, n: int) -> bool:
         return self.data is not None and self.length + n <= self.data.shape[2]
@@ -80,26 +81,61 @@ class _DenseHistory:
 
 
 class _LayerViews(list):
-    """A per-layer list of views into the dense caches, made when they are looked at: an update then costs no tensor views
-    that its caller does not use."""
+    """A per-layer list of views into the dense caches.  It is a list like any other, except that the views of a layer that
+    has been updated are made when the list is looked at: an update then costs no tensor views that its caller does not use
+    (two to five microseconds each, and there would be four of them; an update of one token takes about fifteen)."""
 
     def __init__(self, histories, make):
         super().__init__([None] * len(histories))
-        self._histories, self._make = histories, make
+        self._histories, self._make, self._seen = histories, make, [0] * len(histories)
 
-    def __getitem__(self, i):
-        if isinstance(i, slice):
-            return [self[j] for j in range(*i.indices(len(self)))]
-        return self._make(self._histories[i])
+    def _fill(self):
+        for i, h in enumerate(self._histories):
+            if self._seen[i] != h.updates:
+                self._seen[i] = h.updates
+                list.__setitem__(self, i, self._make(h))
 
-    def __iter__(self):
-        return (self._make(h) for h in self._histories)
+    def __radd__(self, other):
+        return other + self.copy()
 
-    def __reversed__(self):
-        return (self._make(h) for h in reversed(self._histories))
 
-    def __repr__(self):
-        return repr(list(self))
+def _looks(name):
+    method = getattr(list, name)
+
+    def looks(self, *args, **kwargs):
+        for views in (self, *args):
+            if isinstance(views, _LayerViews):
+                views._fill()
+        return method(self, *args, **kwargs)
+    return looks
+
+
+for _name in ("__getitem__", "__setitem__", "__delitem__", "__iter__", "__reversed__", "__contains__", "__eq__", "__ne__", "__lt__",
+              "__le__", "__gt__", "__ge__", "__add__", "__iadd__", "__mul__", "__rmul__", "__repr__", "__reduce_ex__", "copy", "count",
+              "index", "pop", "remove", "reverse", "sort"):
+    setattr(_LayerViews, _name, _looks(_name))
+
+
+# (the reference's compressed caches stay None until a block has been quantized; its tails can be empty)
+def _quantized_part(h: _DenseHistory):
+    return h.view(0, h.quantized, empty_is_none=True)
+
+
+def _tail_part(h: _DenseHistory):
+    return h.view(h.quantized)
+
+
+def _per_layer(name):
+    """An attribute that is a _LayerViews, filled before anybody gets it (what reads a list's memory directly, like
+    torch.cat, sees the views too)."""
+    def get(self) -> List[Optional[torch.Tensor]]:
+        views = self.__dict__[name]
+        views._fill()
+        return views
+
+    def put(self, values):
+        get(self)[:] = values
+    return property(get, put)
 
 
 class KVCompCachePytorchQuant:
@@ -113,14 +149,13 @@ class KVCompCachePytorchQuant:
         self.head_dim = head_dim
         self._k = [_DenseHistory() for _ in range(layer_num)]
         self._v = [_DenseHistory() for _ in range(layer_num)]
-        # (the reference's compressed caches stay None until a block has been quantized; its tails can be empty)
-        quantized, tail = (lambda h: h.view(0, h.quantized, empty_is_none=True)), (lambda h: h.view(h.quantized))
-        self.compressed_k_cache: List[Optional[torch.Tensor]] = _LayerViews(self._k, quantized)
-        self.compressed_v_cache: List[Optional[torch.Tensor]] = _LayerViews(self._v, quantized)
-        self.k_cache_buffer: List[Optional[torch.Tensor]] = _LayerViews(self._k, tail)
-        self.v_cache_buffer: List[Optional[torch.Tensor]] = _LayerViews(self._v, tail)
+        self._compressed_k, self._compressed_v = _LayerViews(self._k, _quantized_part), _LayerViews(self._v, _quantized_part)
+        self._k_tail, self._v_tail = _LayerViews(self._k, _tail_part), _LayerViews(self._v, _tail_part)
         self.coss: List[Optional[torch.Tensor]] = [None] * layer_num
         self.sins: List[Optional[torch.Tensor]] = [None] * layer_num
+
+    compressed_k_cache, compressed_v_cache = _per_layer("_compressed_k"), _per_layer("_compressed_v")
+    k_cache_buffer, v_cache_buffer = _per_layer("_k_tail"), _per_layer("_v_tail")
 
     # -- helpers ---------------------------------------------------------------------------------------
     def _append(self, key_states, value_states, layer_idx, cache_kwargs):
@@ -148,10 +183,13 @@ class KVCompCachePytorchQuant:
         v.append(value_states)
 
     def _publish(self, layer_idx):
-        keys = self._k[layer_idx].view()
+        k, v = self._k[layer_idx], self._v[layer_idx]
+        k.updates += 1
+        v.updates += 1
+        keys = k.view()
         if _config().enable_pre_rope:
             keys = apply_rotary_pos_emb_single(keys, self.coss[layer_idx], self.sins[layer_idx])
-        return keys, self._v[layer_idx].view()
+        return keys, v.view()
 
     # -- the Cache contract ------------------------------------------------------------------------------
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor, layer_idx: int,
