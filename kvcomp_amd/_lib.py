@@ -131,6 +131,18 @@ def device_guard(t):
     return _HERE_GUARD if torch._C._cuda_getDevice() == index else torch.cuda.device(index)
 
 
+_grad_enabled, _trace, _forward = torch.is_grad_enabled, torch._C._get_tracing_state, torch.autograd.forward_ad
+
+
+def recorded(*tensors) -> bool:
+    """Whether PyTorch would record an operation on these tensors (for a gradient, a tangent or a trace): a kernel that
+    takes their addresses would leave no trace of itself then."""
+    for t in tensors:
+        if t is not None and t.requires_grad and _grad_enabled():
+            return True
+    return _forward._current_level >= 0 or _trace() is not None
+
+
 def stream_of(t) -> int:
     """Address of the current stream of the tensor's device, without an object for it."""
     index = t.get_device()

@@ -138,11 +138,12 @@ def quant_in_place(region: torch.Tensor, block_size: int, quant_scale_rel: float
     B, H, T, D = region.shape
     if T == 0:
         return
-    if region.is_cuda and region.dtype is torch.float16 and region.stride(3) == 1 and region.stride(2) == D:
+    if region.is_cuda and region.dtype is torch.float16 and region.stride(3) == 1 and region.stride(2) == D and not _lib.recorded(region):
         with _lib.device_guard(region):
             rc = _lib.lib().kvc_quant_in_place(_ptr(region), B, H, T, D, region.stride(0), region.stride(1), block_size,
                                                _SIM_PLAN[quant_mode][1], float(quant_scale_rel), _stream(region))
         if rc == 0:
+            torch.autograd.graph.increment_version((region,))
             return
         if rc != 1:
             check(rc)
@@ -158,7 +159,7 @@ def takes_append(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], 
     token, shared by the batch or not.  The rotated keys are then what the keys are: fp16 of the same shape."""
     f16 = torch.float16
     if not (k.dtype is f16 and v.dtype is f16 and k.is_cuda and k.device == v.device and v.shape == k.shape and k.dim() == 4 and
-            k.shape[3] % 2 == 0 and k.stride(3) == 1 and v.stride(3) == 1):
+            k.shape[3] % 2 == 0 and k.stride(3) == 1 and v.stride(3) == 1) or _lib.recorded(k, v, cos, sin):
         return False
     return cos is None or (cos.dtype is f16 and sin.dtype is f16 and cos.device == sin.device == k.device and
                            cos.shape == sin.shape and cos.dim() == 3 and cos.shape[0] in (1, k.shape[0]) and
@@ -174,7 +175,8 @@ def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], 
     B, H, T, D = k.shape
     f16 = torch.float16
     if not (k_cache.dtype is f16 and v_cache.dtype is f16 and k.device == k_cache.device == v_cache.device and
-            k_cache.shape == v_cache.shape == (B, H, k_cache.shape[2], D) and k_cache.is_contiguous() and v_cache.is_contiguous()):
+            k_cache.shape == v_cache.shape == (B, H, k_cache.shape[2], D) and k_cache.is_contiguous() and v_cache.is_contiguous()) or \
+            _lib.recorded(k_cache, v_cache):
         return False
     kb, kh, kt, _ = k.stride()
     vb, vh, vt, _ = v.stride()
@@ -188,6 +190,7 @@ def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], 
                        kb, kh, kt, vb, vh, vt, cb, ct, sb, st)
     with _lib.device_guard(k):
         check(_lib.lib().kvc_append_dense(job, _stream(k)))
+    torch.autograd.graph.increment_version((k_cache, v_cache))
     return True
 
 

@@ -396,7 +396,7 @@ class KVCompCtx:
             self._tail = grown
         row = self._row_bytes
         to, src = self._tail.data_ptr() + self._tail_len * row, cache.data_ptr()
-        if n and (to | src | row) & 15 == 0 and cache.is_cuda and cache.is_contiguous():
+        if n and (to | src | row) & 15 == 0 and cache.is_cuda and cache.is_contiguous() and not _lib.recorded(cache, self._tail):
             kvcomp_cuda.copy_rows(self._tail, to, src, n * row)      # (half the host time of an assignment to a slice)
         elif n:
             self._tail[self._tail_len:self._tail_len + n] = cache
@@ -745,7 +745,7 @@ class KVCompCtx:
         been compressed yet the tail is everything; the reference asserts in that state.)"""
         if self.compressed_ctx_len == 0:
             return self.buffer.clone(), 0.0
-        if KVCompCtx.fused_get:
+        if KVCompCtx.fused_get and not (self._tail_len and _lib.recorded(self._tail)):
             self._assert_ready()
             return self._restore(with_tail=True)
         out, t_ms = self.get_only_compressed()

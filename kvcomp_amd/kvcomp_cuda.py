@@ -374,10 +374,11 @@ def build_lut(decode_codebook: torch.Tensor, tree_format: int = TREE_I8) -> torc
     return lut
 
 
-def copy_rows(on: torch.Tensor, dst: int, src: int, nbytes: int) -> None:
-    """kvc_copy_rows between two addresses on the device of `on`, on its current stream."""
-    with _lib.device_guard(on):
-        check(_lib.lib().kvc_copy_rows(dst, src, nbytes, _lib.stream_of(on)))
+def copy_rows(into: torch.Tensor, dst: int, src: int, nbytes: int) -> None:
+    """kvc_copy_rows to an address inside `into`, on its device's current stream."""
+    with _lib.device_guard(into):
+        check(_lib.lib().kvc_copy_rows(dst, src, nbytes, _lib.stream_of(into)))
+    torch.autograd.graph.increment_version((into,))
 
 
 def mat_vec_mul(is_k: bool, desc, x: torch.Tensor, part, out: torch.Tensor, head_num: int, head_dim: int) -> float:
