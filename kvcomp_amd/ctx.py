@@ -212,7 +212,6 @@ class KVCompCtx:
         self._row_bytes = 2 * batch_size * head_num * head_dim
         self._mask = dims_to_mask(self.quant_dims)
         self._groups_per_block = expected_groups(self.block_size, self.block_size, batch_size, head_num, head_dim, self.quant_dims)
-        self._descriptor = _lib.CompressedDesc()
         self._lut: Optional[torch.Tensor] = None       # decode tables of _lut_source, see decode_lut
         self._lut_source: Optional[torch.Tensor] = None
         self._encoded = _Growable()
@@ -246,14 +245,10 @@ class KVCompCtx:
         self.waits = 0                     # how often this context has waited for the device to learn sizes
 
     def __getstate__(self):
-        # (copies and pickles: the descriptor holds addresses and is refilled on every use.  Queued stores are waited for: a
-        # copy cannot share the event and the pinned words that will say what became of them.)
+        # (copies and pickles: queued stores are waited for, since a copy cannot share the event and the pinned words that
+        # will say what became of them)
         self._sync_sizes()
-        return {**{name: value for name, value in self.__dict__.items() if name != "_descriptor"}, "_probe": None, "_host_words": None}
-
-    def __setstate__(self, state):
-        self.__dict__.update(state)
-        self._descriptor = _lib.CompressedDesc()
+        return {**self.__dict__, "_probe": None, "_host_words": None}
 
     def _device_state(self) -> torch.Tensor:
         if self._state is None:
@@ -692,28 +687,31 @@ class KVCompCtx:
         return self._lut
 
     def descriptor(self) -> "_lib.CompressedDesc":
-        """kvc_compressed_desc of everything held, refilled in place.  Does not wait for queued stores: addresses and a
-        bound of the payload are enough for the kernels.  Addresses and sizes come straight from the growing arrays, in
-        one go: a tensor view or a ctypes assignment per field costs more host time than a short-context step takes on
-        the device."""
+        """kvc_compressed_desc of everything held; every call has its own, since the library reads it without the GIL.  Does
+        not wait for queued stores: addresses and a bound of the payload are enough for the kernels.  Addresses and sizes
+        come straight from the growing arrays, in one go: a tensor view or a ctypes assignment per field costs more host
+        time than a short-context step takes on the device."""
         if self._probe is not None:
             self.poll_stores()                             # what queued stores have left, if it has arrived: no wait
         tokens, tail = self.compressed_ctx_len, self._tail_len
         tail_address = self._tail.data_ptr() if tail else 0
+        desc = _lib.CompressedDesc()
         if tokens == 0:
-            _DESC.pack_into(self._descriptor, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, self._mask, 0, 0, 0, 0, tail_address, tail)
-            return self._descriptor
+            _DESC.pack_into(desc, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, self._mask, 0, 0, 0, 0, tail_address, tail)
+            return desc
         lut = self.decode_lut()
         mins, scales, encoded = self._min_ints, self._scales, self._encoded
         # the kernels take the quantization parameters by pointer: they must cover every group of the stream
         groups = tokens // self.block_size * self._groups_per_block
         assert mins.used * mins.row == groups and scales.used * scales.row == groups, \
             "the context holds %d minima and %d scales for %d quantization groups" % (mins.used * mins.row, scales.used * scales.row, groups)
-        _DESC.pack_into(self._descriptor, 0, lut.data_ptr(), 0, self._block_infos.address, self._block_infos.used,
+        _DESC.pack_into(desc, 0, lut.data_ptr(), 0, self._block_infos.address, self._block_infos.used,
                         self._thread_infos.address, self._thread_infos.used, encoded.address,
                         min(encoded.used + self._enc_pending, encoded.data.shape[0]), mins.address, scales.address, self._mask,
                         self.max_tile_bytes, self.max_stream_bytes, self.code_hint, tokens, tail_address, tail)
-        return self._descriptor
+        return desc
+
+    _descriptor = property(descriptor)                     # (as an attribute: another one every time)
 
     # decode and dequantize in one kernel (no uint8 tensor in between); False = the reference's two steps
     fused_get = True

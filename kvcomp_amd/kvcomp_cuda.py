@@ -397,8 +397,7 @@ def restore(is_k: bool, desc, block_size: int, out: torch.Tensor, with_tail: boo
              "out must be a contiguous device float16 tensor [T, B, H, D]")
     T, B, H, D = out.shape
     if not with_tail:
-        whole, desc = desc, _lib.CompressedDesc()
-        C.memmove(C.byref(desc), C.byref(whole), C.sizeof(desc))
+        desc = _lib.CompressedDesc.from_buffer_copy(desc)
         desc.tail_tokens = 0
     _require(T == desc.tokens + desc.tail_tokens, "out holds %d tokens, %d are to be restored" % (T, desc.tokens + desc.tail_tokens))
     ms = C.c_float(0.0)

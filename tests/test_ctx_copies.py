@@ -56,6 +56,17 @@ def test_a_queued_store_is_waited_for(how, monkeypatch):
     assert got._probe is None and got._host_words is None
 
 
+def test_every_call_has_a_descriptor_of_its_own():
+    """Two threads may attend over one context: the library reads what a call was given without the GIL."""
+    _config()
+    ctx = KVCompCtx(True, 1, 2, 64, 0.1)
+    ctx.store(torch.zeros(20, 1, 2, 64, dtype=torch.float16))
+    first = ctx.descriptor()
+    ctx.store(torch.zeros(5, 1, 2, 64, dtype=torch.float16))
+    second = ctx.descriptor()
+    assert (first.tail_tokens, second.tail_tokens) == (20, 25) and first.d_tail_f16 == second.d_tail_f16 == ctx._tail.data_ptr()
+
+
 def test_moved_data_is_seen():
     _config()
     g = KVCompCtx(False, 1, 2, 64, 0.2)._encoded
