@@ -134,13 +134,18 @@ def device_guard(t):
 _grad_enabled, _trace, _forward = torch.is_grad_enabled, torch._C._get_tracing_state, torch.autograd.forward_ad
 
 
+def hooked() -> bool:
+    """Whether tangents are carried along or a trace is being taken."""
+    return _forward._current_level >= 0 or _trace() is not None
+
+
 def recorded(*tensors) -> bool:
     """Whether PyTorch would record an operation on these tensors (for a gradient, a tangent or a trace): a kernel that
     takes their addresses would leave no trace of itself then."""
     for t in tensors:
         if t is not None and t.requires_grad and _grad_enabled():
             return True
-    return _forward._current_level >= 0 or _trace() is not None
+    return hooked()
 
 
 def stream_of(t) -> int:

@@ -77,7 +77,7 @@ class _DenseHistory:
         hi = self.length if hi is None else hi
         if self.data is None or (empty_is_none and hi <= lo):
             return None
-        return self.data[:, :, lo:hi]
+        return self.data.narrow(2, lo, hi - lo)
 
 
 class _LayerViews(list):

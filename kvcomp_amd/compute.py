@@ -154,43 +154,59 @@ def quant_in_place(region: torch.Tensor, block_size: int, quant_scale_rel: float
 _APPEND = struct.Struct("=22q")
 
 
+def _append_job(k, v, cos, sin):
+    """The fields of kvc_append_job that come from the rows and the angles, or None for ones that kvc_append_dense does not
+    take: fp16 on one GPU, elements of a row adjacent, angles for every token, shared by the batch or not.  (Devices by their
+    index, shapes and strides asked for once: the checks are a good part of the host time of a one-token append.)"""
+    f16, gpu = torch.float16, k.get_device()
+    if not (gpu >= 0 and k.dtype is f16 and v.dtype is f16 and v.get_device() == gpu and k.dim() == 4):
+        return None
+    shape = k.shape
+    B, H, T, D = shape
+    kb, kh, kt, kd = k.stride()
+    if v.shape != shape or D % 2 or kd != 1:
+        return None
+    vb, vh, vt, vd = v.stride()
+    if vd != 1:
+        return None
+    if cos is None:
+        return k.data_ptr(), v.data_ptr(), 0, 0, B, H, T, D, kb, kh, kt, vb, vh, vt, 0, 0, 0, 0
+    if not (cos.dtype is f16 and sin.dtype is f16 and cos.get_device() == gpu and sin.get_device() == gpu and cos.dim() == 3):
+        return None
+    angles = cos.shape
+    if sin.shape != angles or angles[1] != T or angles[2] != D or angles[0] not in (1, B):
+        return None
+    (cb, ct, cd), (sb, st, sd) = cos.stride(), sin.stride()
+    if cd != 1 or sd != 1:
+        return None
+    if angles[0] == 1:
+        cb = sb = 0
+    return k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(), B, H, T, D, kb, kh, kt, vb, vh, vt, cb, ct, sb, st
+
+
 def takes_append(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor]) -> bool:
-    """Whether append_dense takes these rows and angles: fp16 on one GPU, elements of a row adjacent, angles for every
-    token, shared by the batch or not.  The rotated keys are then what the keys are: fp16 of the same shape."""
-    f16 = torch.float16
-    if not (k.dtype is f16 and v.dtype is f16 and k.is_cuda and k.device == v.device and v.shape == k.shape and k.dim() == 4 and
-            k.shape[3] % 2 == 0 and k.stride(3) == 1 and v.stride(3) == 1) or _lib.recorded(k, v, cos, sin):
-        return False
-    return cos is None or (cos.dtype is f16 and sin.dtype is f16 and cos.device == sin.device == k.device and
-                           cos.shape == sin.shape and cos.dim() == 3 and cos.shape[0] in (1, k.shape[0]) and
-                           cos.shape[1:] == k.shape[2:] and cos.stride(2) == 1 and sin.stride(2) == 1)
+    """Whether append_dense takes these rows and angles, as far as their types and layouts go.  The rotated keys are then
+    what the keys are: fp16 of the same shape."""
+    return _append_job(k, v, cos, sin) is not None
 
 
 def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], k_cache: torch.Tensor,
                  v_cache: torch.Tensor, at: int) -> bool:
     """kvc_append_dense: k (rotated by cos / sin [1 or B, T, D], unless they are None) and v, [B, H, T, D] fp16, to
-    positions at .. of the [B, H, capacity, D] caches.  False, having done nothing, for tensors it does not take."""
-    if not takes_append(k, v, cos, sin):
+    positions at .. of the [B, H, capacity, D] caches.  False, having done nothing, for tensors it does not take or that
+    PyTorch would record.  (No view handed out before holds the positions written: their version need not move.)"""
+    job = _append_job(k, v, cos, sin)
+    if job is None or _lib.recorded(k, v, cos, sin, k_cache, v_cache):
         return False
-    B, H, T, D = k.shape
-    f16 = torch.float16
-    if not (k_cache.dtype is f16 and v_cache.dtype is f16 and k.device == k_cache.device == v_cache.device and
-            k_cache.shape == v_cache.shape == (B, H, k_cache.shape[2], D) and k_cache.is_contiguous() and v_cache.is_contiguous()) or \
-            _lib.recorded(k_cache, v_cache):
+    k_p, v_p, cos_p, sin_p, B, H, T, D, *strides = job
+    f16, gpu, held = torch.float16, k.get_device(), k_cache.shape
+    if not (k_cache.dtype is f16 and v_cache.dtype is f16 and k_cache.get_device() == gpu and v_cache.get_device() == gpu and
+            len(held) == 4 and held[0] == B and held[1] == H and held[3] == D and v_cache.shape == held and
+            k_cache.is_contiguous() and v_cache.is_contiguous()):
         return False
-    kb, kh, kt, _ = k.stride()
-    vb, vh, vt, _ = v.stride()
-    cos_p = sin_p = cb = ct = sb = st = 0
-    if cos is not None:
-        (cb, ct, _), (sb, st, _) = cos.stride(), sin.stride()
-        if cos.shape[0] == 1:
-            cb = sb = 0
-        cos_p, sin_p = cos.data_ptr(), sin.data_ptr()
-    job = _APPEND.pack(k.data_ptr(), v.data_ptr(), cos_p, sin_p, k_cache.data_ptr(), v_cache.data_ptr(), B, H, T, D, k_cache.shape[2], at,
-                       kb, kh, kt, vb, vh, vt, cb, ct, sb, st)
+    packed = _APPEND.pack(k_p, v_p, cos_p, sin_p, k_cache.data_ptr(), v_cache.data_ptr(), B, H, T, D, held[2], at, *strides)
     with _lib.device_guard(k):
-        check(_lib.lib().kvc_append_dense(job, _stream(k)))
-    torch.autograd.graph.increment_version((k_cache, v_cache))
+        check(_lib.lib().kvc_append_dense(packed, _lib.stream_of(k)))
     return True
 
 

@@ -391,7 +391,10 @@ class KVCompCtx:
             self._tail = grown
         row = self._row_bytes
         to, src = self._tail.data_ptr() + self._tail_len * row, cache.data_ptr()
-        if n and (to | src | row) & 15 == 0 and cache.is_cuda and cache.is_contiguous() and not _lib.recorded(cache, self._tail):
+        if (n and (to | src | row) & 15 == 0 and cache.is_cuda and cache.is_contiguous() and
+                not (cache.requires_grad or self._tail.requires_grad or _lib.hooked())):
+            if self._tail_len == 0:                                  # where views of an earlier tail may lie
+                torch.autograd.graph.increment_version((self._tail,))
             kvcomp_cuda.copy_rows(self._tail, to, src, n * row)      # (half the host time of an assignment to a slice)
         elif n:
             self._tail[self._tail_len:self._tail_len + n] = cache

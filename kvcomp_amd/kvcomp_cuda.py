@@ -375,10 +375,9 @@ def build_lut(decode_codebook: torch.Tensor, tree_format: int = TREE_I8) -> torc
 
 
 def copy_rows(into: torch.Tensor, dst: int, src: int, nbytes: int) -> None:
-    """kvc_copy_rows to an address inside `into`, on its device's current stream."""
+    """kvc_copy_rows to an address inside `into`, on its device's current stream; `into` keeps its version."""
     with _lib.device_guard(into):
         check(_lib.lib().kvc_copy_rows(dst, src, nbytes, _lib.stream_of(into)))
-    torch.autograd.graph.increment_version((into,))
 
 
 def mat_vec_mul(is_k: bool, desc, x: torch.Tensor, part, out: torch.Tensor, head_num: int, head_dim: int) -> float:

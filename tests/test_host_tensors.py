@@ -84,7 +84,10 @@ def test_blocks_in_host_memory_are_refused_by_the_simulated_quantizer():
 def test_rows_and_angles_elsewhere_than_the_caches_are_left_to_pytorch(which):
     class Elsewhere(torch.Tensor):                               # claims to lie on a GPU
         is_cuda = property(lambda self: True)
-        device = property(lambda self: torch.device("cuda", 1 if which in self.at else 0))
+        device = property(lambda self: torch.device("cuda", self.get_device()))
+
+        def get_device(self):
+            return 1 if which in self.at else 0
 
     def at(name, *shape):
         t = torch.zeros(*shape, dtype=torch.float16).as_subclass(Elsewhere)

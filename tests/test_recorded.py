@@ -14,6 +14,9 @@ DEV = "cuda:0"
 class _OnGpu(torch.Tensor):
     is_cuda = property(lambda self: True)
 
+    def get_device(self):
+        return 0
+
 
 @pytest.fixture
 def calls(monkeypatch):
@@ -53,17 +56,26 @@ def test_tangents_and_traces_are_left_to_pytorch():
     assert seen == [True] and not _lib.recorded(x)
 
 
-def test_writes_of_kernels_move_the_version(calls):
-    kc, vc = _tensor(1, 2, 8, 64), _tensor(1, 2, 8, 64)
-    before = kc._version, vc._version
-    assert compute.append_dense(_tensor(1, 2, 3, 64), _tensor(1, 2, 3, 64), None, None, kc, vc, 0)
-    assert (kc._version, vc._version) > before and vc._version > before[1]
-    at, view = kc._version, kc[:, :, 2:4]
-    compute.quant_in_place(view, 2, 0.1, QuantMode.ChannelQuant)
-    assert calls[-1] == "kvc_quant_in_place" and kc._version > at
-    at = vc._version
-    kvcomp_cuda.copy_rows(vc, 0, 0, 0)
-    assert vc._version > at
+def test_writes_over_what_views_hold_move_the_version(calls):
+    cache = _tensor(1, 2, 8, 64)
+    at = cache._version
+    compute.quant_in_place(cache[:, :, 2:4], 2, 0.1, QuantMode.ChannelQuant)
+    assert calls == ["kvc_quant_in_place"] and cache._version > at
+
+
+@pytest.mark.gpu
+def test_a_tail_that_was_written_over_since_is_refused_by_backward():
+    _quantized()
+    x = S.synth_k(400, 1, 2, 64).to(DEV)
+    ctx = KVCompCtx(True, 1, 2, 64, 0.1)
+    ctx.store(x[:70])                                              # 6 tokens stay behind the first block
+    q = torch.ones(ctx.buffer.shape, dtype=torch.float16, device=DEV, requires_grad=True)
+    loss = (ctx.buffer * q).float().sum()                          # saves the view
+    tail = ctx._tail
+    ctx.store(x[70:170])                                           # one more block leaves, and the tail starts again
+    assert ctx._tail is tail and ctx.buffer.shape[0] == 42
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        loss.backward()
 
 
 def _quantized():
