@@ -421,6 +421,8 @@ int kvc_quant(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H,
  *   symbols written (without the padding of each lane stream to whole bytes).  Waits for the symbol counts, not for the
  *   stream; cannot be recorded into a graph.
  *   pair_bits: index bits of a decode table that next to all pairs of these symbols fit, 2 .. 7, or 0.
+ * kvc_put_codebook: the encode table to d_tables, the decode tree behind it on the next 16-byte boundary, and the decode
+ *   tables of kvc_build_lut (one codebook) to d_lut, in stream order without waiting; book may be reused at once.
  * kvc_put_bytes: copies host bytes to device memory in stream order without waiting; h_src may be reused at once. */
 typedef struct kvc_codebook {
     int32_t tree_format, max_code_bits;
@@ -432,6 +434,7 @@ typedef struct kvc_codebook {
 int kvc_quant_codebook(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                        float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, int smoothed_symbols,
                        kvc_codebook *out, void *stream);
+int kvc_put_codebook(const kvc_codebook *book, void *d_tables, void *d_lut, void *stream);
 int kvc_put_bytes(void *d_dst, const void *h_src, int64_t bytes, void *stream);
 
 /* ---- simulated quantization: quant_error (utils/compute.py:108-133), the value the reference's model caches

@@ -586,7 +586,7 @@ class KVCompCtx:
         sym, book = kvcomp_cuda.quant_codebook(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale,
                                                self._smoothed_symbols() if self.codebook_smoothing else 0)
         self.waits += 1
-        enc, dec = kvcomp_cuda.put_codebook(book, device)
+        enc, dec, lut = kvcomp_cuda.put_codebook(book, device)
         vectors = T * self.batch_size * self.head_num * self.head_dim // (self.head_dim if self.is_k else kvcomp_cuda.V_VEC_LEN)
         cannot_fail = book.max_code_bits <= 7
         small = T <= self.ASYNC_KEEP_BLOCKS * self.block_size
@@ -599,7 +599,7 @@ class KVCompCtx:
             self._sync_sizes()                                 # (a failure leaves the context as it was before the encode)
         self.tree_format, self.max_code_bits, self.pair_bits = book.tree_format, book.max_code_bits, book.pair_bits
         self.encode_codebook, self.decode_codebook = enc, dec
-        self._build_lut()
+        self._lut, self._lut_source = lut, dec
         return sym
 
     def _smoothed_symbols(self) -> int:

@@ -157,14 +157,14 @@ def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: floa
 
 
 def put_codebook(book: "_lib.Codebook", device):
-    """(encode table, decode tree) of a _lib.Codebook as device uint8 tensors, copied in stream order; nothing waits."""
-    enc_bytes, dec_bytes = book.encode_bytes, book.decode_bytes
-    at = (enc_bytes + 15) // 16 * 16                     # one allocation, the tree on a 16-byte boundary
-    both = torch.empty(at + dec_bytes, dtype=torch.uint8, device=device)
-    packed = C.string_at(C.addressof(book.encode_table), enc_bytes).ljust(at, b"\0") + C.string_at(C.addressof(book.decode_tree), dec_bytes)
-    with _lib.device_guard(both):
-        check(_lib.lib().kvc_put_bytes(_ptr(both), packed, len(packed), _stream(both)))
-    return both[:enc_bytes], both[at:]
+    """(encode table, decode tree, decode tables) of a _lib.Codebook as device uint8 tensors, in stream order; nothing waits."""
+    L = _lib.lib()
+    enc_bytes, lut_bytes = book.encode_bytes, L.kvc_lut_bytes()
+    at = lut_bytes + (enc_bytes + 15) // 16 * 16         # one allocation, each part on a 16-byte boundary
+    held = torch.empty(at + book.decode_bytes, dtype=torch.uint8, device=device)
+    with _lib.device_guard(held):
+        check(L.kvc_put_codebook(C.addressof(book), held.data_ptr() + lut_bytes, held.data_ptr(), _lib.stream_of(held)))
+    return held[lut_bytes:lut_bytes + enc_bytes], held[at:], held[:lut_bytes]
 
 
 def _entropy_encode(is_k, input, encode_code_book, block_infos, thread_infos, idx_offset, encoded_data,

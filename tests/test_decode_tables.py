@@ -12,10 +12,6 @@ def _config():
     KVCompCacheConfigStatic.config = KVCompCacheConfig("t", QuantMode.ChannelQuant, QuantMode.TokenQuant, 64, 128, 64, 128, 0.1, 0.2)
 
 
-class _OnGpu(torch.Tensor):
-    is_cuda = property(lambda self: True)
-
-
 @pytest.fixture
 def built(monkeypatch):
     """Tables built so far, as (codebook, table)."""
@@ -28,18 +24,52 @@ def built(monkeypatch):
     return made
 
 
-def test_the_first_store_builds_the_tables(monkeypatch, built):
+def test_the_first_store_brings_the_tables(monkeypatch, built):
     _config()
     ctx = KVCompCtx(True, 1, 2, 64, 0.1)
     ctx.device = torch.device("cpu")
     book = _lib.Codebook(tree_format=3, max_code_bits=3)
-    enc, dec = (torch.zeros(24, dtype=torch.uint8).as_subclass(_OnGpu) for _ in range(2))
+    enc, dec, lut = (torch.zeros(24, dtype=torch.uint8) for _ in range(3))
     monkeypatch.setattr(kvcomp_cuda, "quant_codebook", lambda *a: (a[0].to(torch.uint8), book))
-    monkeypatch.setattr(kvcomp_cuda, "put_codebook", lambda *a: (enc, dec))
+    monkeypatch.setattr(kvcomp_cuda, "put_codebook", lambda *a: (enc, dec, lut))
     monkeypatch.setattr(KVCompCtx, "_encode_direct", lambda self, T, **kw: None)
     ctx._first_chunk(torch.zeros(1, 64, 1, 2, 64, dtype=torch.float16))
-    assert [c is dec for c, _ in built] == [True]
-    assert ctx.decode_lut() is built[0][1] and len(built) == 1
+    assert ctx.decode_lut() is lut and ctx.decode_codebook is dec and not built
+
+
+def test_a_codebook_put_in_place_later_brings_them_too(monkeypatch, built):
+    _config()
+    ctx = KVCompCtx(True, 1, 2, 64, 0.1)
+
+    class Codebook(torch.Tensor):
+        is_cuda = property(lambda self: True)
+
+        def to(self, device):
+            return self
+    ctx._set_codebook(torch.zeros(24, dtype=torch.uint8), torch.zeros(24, dtype=torch.uint8).as_subclass(Codebook))
+    assert len(built) == 1 and built[0][0] is ctx.decode_codebook and ctx.decode_lut() is built[0][1] and len(built) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("symbols", [2, 23, 100, 250])             # 250: the tables do not fit one launch's arguments
+def test_the_launch_that_brings_a_codebook_builds_its_tables(symbols):
+    _config()
+    book = _lib.Codebook()
+    g = torch.Generator().manual_seed(symbols)
+    x = torch.randint(0, symbols, (4, 64, 1, 2, 64), generator=g).to(torch.float16)
+    x[:, 0], x[:, 1] = 0.0, float(symbols - 1)                      # the step of every block is (symbols - 1) * eb = 1
+    x = x.to("cuda:0")
+    mins, scales = torch.empty(4, dtype=torch.int8, device="cuda:0"), torch.empty(4, dtype=torch.float16, device="cuda:0")
+    sym, book = kvcomp_cuda.quant_codebook(x, kvcomp_cuda.MASK_K_BLOCK, 1.0 / (symbols - 1), mins, scales, 0)
+    enc, dec, lut = kvcomp_cuda.put_codebook(book, torch.device("cuda:0"))
+    assert bytes(enc.cpu().tolist()) == bytes(book.encode_table)[:book.encode_bytes]
+    assert bytes(dec.cpu().tolist()) == bytes(book.decode_tree)[:book.decode_bytes]
+    want = kvcomp_cuda.build_lut(dec, book.tree_format)
+    # (entries beyond 1 << index bits, and list places beyond their counts, are never written or read)
+    words, ref = lut.view(torch.int32).cpu(), want.view(torch.int32).cpu()
+    bits, fast = int(ref[0]), 8 + 512 + 1024
+    assert torch.equal(words[:8], ref[:8]) and torch.equal(words[520:520 + (1 << bits)], ref[520:520 + (1 << bits)])
+    assert torch.equal(words[fast:fast + (1 << bits)], ref[fast:fast + (1 << bits)])
 
 
 def test_tables_of_an_assigned_codebook_are_waited_for_and_never_shared_out_of_a_recording(monkeypatch, built):

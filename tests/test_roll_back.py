@@ -32,7 +32,7 @@ def test_a_failed_second_store_leaves_a_prompt_that_nobody_has_looked_at(monkeyp
                 block_infos[8 * i:8 * i + 8] = torch.frombuffer(bytearray(struct.pack("<IHH", at + 700 * i, 700, 0)), dtype=torch.uint8)
         sizes.append(700 * n)
     monkeypatch.setattr(kvcomp_cuda, "quant_codebook", lambda x, *a: (x.to(torch.uint8), book))
-    monkeypatch.setattr(kvcomp_cuda, "put_codebook", lambda *a: (torch.zeros(24, dtype=torch.uint8), torch.zeros(24, dtype=torch.uint8)))
+    monkeypatch.setattr(kvcomp_cuda, "put_codebook", lambda *a: tuple(torch.zeros(24, dtype=torch.uint8) for _ in range(3)))
     monkeypatch.setattr(kvcomp_cuda, "encode_async", encode)
     monkeypatch.setattr(KVCompCtx, "_issue_probe", lambda self: None)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
