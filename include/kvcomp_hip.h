@@ -298,6 +298,9 @@ int kvc_v_decode_and_mat_vec_mul(const uint8_t *d_decode_tree, int64_t decode_tr
  * points above derive it on every call; these take tables prepared once per codebook:
  *   kvc_build_lut: n_codebooks trees, tree_stride_bytes apart, each tree_bytes long -> d_luts
  *                  (n_codebooks * kvc_lut_bytes() bytes, 16-byte aligned).
+ *                  Behind the tables, V's kernels count on the device how often a table that kvc_codebook::pair_bits
+ *                  asked for was too narrow; calls that take a kvc_compressed_desc stop using it where that happens to more
+ *                  than one tile in sixteen.  Results do not depend on it.
  *   kvc_k_scores_lut / kvc_v_partials_lut: as kvc_k_/v_decode_and_mat_vec_mul, plus
  *     rows_per_codebook: tile rows (64 tokens for K, 128 for V) that share one table; 0 = one table for all
  *     out_f32:           1 writes fp32 results instead of fp16

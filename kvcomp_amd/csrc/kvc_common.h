@@ -53,8 +53,15 @@ constexpr int KVC_LUT_ENTRY_WORDS = 1 << KVC_LUT_MAX_BITS;
 constexpr int KVC_LUT_FENTRY_OFFSET = KVC_LUT_HEADER_WORDS + KVC_LUT_LONG_WORDS + KVC_LUT_ENTRY_WORDS;
 constexpr int KVC_LUT_ESC_OFFSET = KVC_LUT_FENTRY_OFFSET + KVC_LUT_ENTRY_WORDS;
 constexpr int KVC_LUT_ESC_BITS = 7, KVC_LUT_ESC_MAX = 64;
-constexpr int KVC_LUT_WORDS = KVC_LUT_ESC_OFFSET + 2 * KVC_LUT_ESC_MAX;
-constexpr int KVC_LUT_BYTES = KVC_LUT_WORDS * 4;          // 10784
+// What V's kernels learn about the narrow two-symbol table (kvc_narrow_miss): counters behind the tables, each in a 64-byte
+// line of its own, and a bit of the header word that holds the symbols' fp16 patterns, which turns the table off.
+constexpr int KVC_LUT_NARROW_OFFSET = KVC_LUT_ESC_OFFSET + 2 * KVC_LUT_ESC_MAX;
+constexpr int KVC_NARROW_LINE_WORDS = 16, KVC_NARROW_COUNTERS = 64;
+constexpr int KVC_LUT_NARROW_WORD = 6;
+constexpr uint32_t KVC_LUT_NARROW_OFF = 0x80000000u;
+constexpr int KVC_LUT_WORDS = KVC_LUT_NARROW_OFFSET + KVC_NARROW_LINE_WORDS * KVC_NARROW_COUNTERS;
+constexpr int KVC_LUT_BYTES = KVC_LUT_WORDS * 4;          // 14880
+static_assert(KVC_LUT_BYTES % 16 == 0, "decode tables of several codebooks lie one behind the other");
 constexpr int KVC_TREE_MAX_NODES = 512;                   // 2 * 256 symbols - 2, rounded up
 
 // ---------------------------------------------------------------------------------------------------

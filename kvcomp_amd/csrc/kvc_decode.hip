@@ -65,7 +65,7 @@ __device__ __forceinline__ void kvc_decode_wave_sync()
 template <bool DEQ>
 __global__ void __launch_bounds__(KVC_WG) kvc_decode_k_kernel(KvcStreamArgs a, void *__restrict__ out_, KvcDequantArgs q)
 {
-    __shared__ uint32_t s_lut[KVC_LUT_WORDS];
+    __shared__ uint32_t s_lut[KVC_LUT_NARROW_OFFSET];
     __shared__ __align__(16) uint32_t s_stage[KVC_WAVES_PER_WG][KVC_STAGE_WORDS];
     __shared__ uint32_t s_out[KVC_WAVES_PER_WG][KVC_WAVE * KVC_KOUT_ROW_WORDS];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -116,7 +116,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_decode_k_kernel(KvcStreamArgs a, v
 template <bool DEQ>
 __global__ void __launch_bounds__(KVC_WG) kvc_decode_v_kernel(KvcStreamArgs a, void *__restrict__ out_, KvcDequantArgs q)
 {
-    __shared__ uint32_t s_lut[KVC_LUT_WORDS];
+    __shared__ uint32_t s_lut[KVC_LUT_NARROW_OFFSET];
     __shared__ __align__(16) uint32_t s_stage[KVC_WAVES_PER_WG][KVC_STAGE_WORDS];
     __shared__ __align__(16) uint8_t s_out[KVC_WAVES_PER_WG][KVC_V_TOKENS * KVC_WAVE];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

@@ -1402,8 +1402,10 @@ extern "C" int kvc_v_partials_lut(const void *d_luts, int64_t rows_per_codebook,
 // out[i] = RN16(sum over groups of part[g][i]), fp32 sums; n even.  Reads 2 bytes per group and element: bound by the round
 // trips to memory at this size (64 groups x 4096 elements: 0.5 MB), so a wave has eight rows in flight and the workgroup's
 // four waves share the groups.
-__global__ void __launch_bounds__(KVC_WG) kvc_sum_partials_kernel(const uint32_t *__restrict__ part, int64_t groups, int64_t pairs, uint32_t *__restrict__ out)
+__global__ void __launch_bounds__(KVC_WG) kvc_sum_partials_kernel(const uint32_t *__restrict__ part, int64_t groups, int64_t pairs,
+                                                                  uint32_t *__restrict__ out, uint32_t *lut, int64_t tiles)
 {
+    if (lut && blockIdx.x == 0 && threadIdx.x >= KVC_WG - KVC_WAVE) kvc_narrow_decide(lut, tiles, threadIdx.x & 63, kvc_narrow_missed(lut, threadIdx.x & 63));
     __shared__ float2 s_sum[KVC_WAVES_PER_WG][KVC_WAVE];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t i = (int64_t)blockIdx.x * KVC_WAVE + lane;
@@ -1428,6 +1430,17 @@ __global__ void __launch_bounds__(KVC_WG) kvc_sum_partials_kernel(const uint32_t
     }
 }
 
+// the decode tables whose narrow two-symbol table the call's V kernel may have used, for kvc_narrow_decide
+static uint32_t *kvc_narrow_words(const kvc_compressed_desc *v)
+{
+    if (kvc_hint_pair_bits(v->max_code_bits) == 0 || v->rows_per_codebook != 0) return nullptr;
+    return reinterpret_cast<uint32_t *>(const_cast<void *>(v->d_luts));
+}
+static int64_t kvc_v_tiles(const kvc_compressed_desc *v, int64_t batch, int64_t kv_heads, int64_t head_dim)
+{
+    return v->tokens / KVC_V_TOKENS * (batch * kv_heads * head_dim / KVC_WAVE);
+}
+
 extern "C" int kvc_mat_vec_mul(int is_k, const kvc_compressed_desc *c, const void *d_x_f16, void *d_partial_f16, void *d_out_f16,
                                int64_t batch, int64_t kv_heads, int64_t q_heads, int64_t head_dim, float *elapsed_ms, void *stream_)
 {
@@ -1445,7 +1458,8 @@ extern "C" int kvc_mat_vec_mul(int is_k, const kvc_compressed_desc *c, const voi
     if (!is_k) {
         const int64_t pairs = batch * q_heads * head_dim / 2;
         hipLaunchKernelGGL(kvc_sum_partials_kernel, dim3((unsigned)((pairs + KVC_WAVE - 1) / KVC_WAVE)), dim3(KVC_WG), 0, stream,
-                           reinterpret_cast<const uint32_t *>(d_partial_f16), c->tokens / KVC_V_TOKENS, pairs, reinterpret_cast<uint32_t *>(d_out_f16));
+                           reinterpret_cast<const uint32_t *>(d_partial_f16), c->tokens / KVC_V_TOKENS, pairs, reinterpret_cast<uint32_t *>(d_out_f16),
+                           kvc_narrow_words(c), kvc_v_tiles(c, batch, kv_heads, head_dim));
         KVC_HIP(hipGetLastError());
     }
     return timer.finish();
@@ -1581,10 +1595,11 @@ struct KvcTailArgs {
     int batch, kv_heads, rep;
 };
 
-template <int U>
+// DECIDES: a wave of the first workgroup also looks at what the V kernel's narrow table missed (kvc_narrow_decide).
+template <int U, bool DECIDES>
 __global__ void __launch_bounds__(KVC_COMBINE_WAVES * KVC_WAVE)
 kvc_attention_combine_kernel(const float *__restrict__ part, const float *__restrict__ ml, int64_t groups,
-                             int64_t bhq_count, int D, float *__restrict__ out, KvcTailArgs tail)
+                             int64_t bhq_count, int D, float *__restrict__ out, KvcTailArgs tail, uint32_t *lut, int64_t tiles)
 {
     __shared__ float s_max[KVC_COMBINE_WAVES];
     __shared__ float s_num[KVC_COMBINE_WAVES][128];
@@ -1593,6 +1608,8 @@ kvc_attention_combine_kernel(const float *__restrict__ part, const float *__rest
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t bhq = blockIdx.x;
     const int d0 = lane < D ? lane : 0, d1 = lane + 64 < D ? lane + 64 : 0;
+    uint32_t missed = 0;                                  // (asked for now, looked at when the wave has nothing else to do)
+    if (DECIDES && blockIdx.x == 0 && wave == KVC_COMBINE_WAVES - 1) missed = kvc_narrow_missed(lut, lane);
     float M = -INFINITY, n0 = 0.f, n1 = 0.f, den = 0.f;   // this wave's running maximum and its sums relative to it
     for (int64_t g0 = wave; g0 < groups; g0 += U * KVC_COMBINE_WAVES) {
         float mg[U], lg[U], p0[U], p1[U];
@@ -1701,7 +1718,9 @@ kvc_attention_combine_kernel(const float *__restrict__ part, const float *__rest
             dn += s_den[w];
         }
         out[bhq * D + d] = num / dn;
+        return;
     }
+    if (DECIDES && blockIdx.x == 0 && wave == KVC_COMBINE_WAVES - 1) kvc_narrow_decide(lut, tiles, lane, missed);
 }
 
 static int64_t kvc_round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
@@ -1821,12 +1840,21 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
     const int64_t groups = tail_in_merge ? v->tokens / KVC_V_TOKENS : p.groups;
     const dim3 cgrid((unsigned)(batch * q_heads)), cblock(KVC_COMBINE_WAVES * KVC_WAVE);
     const int64_t per_wave = (groups + KVC_COMBINE_WAVES - 1) / KVC_COMBINE_WAVES;
-    if (per_wave <= 4)
-        hipLaunchKernelGGL(kvc_attention_combine_kernel<4>, cgrid, cblock, 0, stream, part, ml, groups, batch * q_heads, (int)head_dim, d_out_f32, tail);
-    else if (per_wave <= 8)
-        hipLaunchKernelGGL(kvc_attention_combine_kernel<8>, cgrid, cblock, 0, stream, part, ml, groups, batch * q_heads, (int)head_dim, d_out_f32, tail);
-    else
-        hipLaunchKernelGGL(kvc_attention_combine_kernel<16>, cgrid, cblock, 0, stream, part, ml, groups, batch * q_heads, (int)head_dim, d_out_f32, tail);
+    uint32_t *lut = v->tokens && !joint ? kvc_narrow_words(v) : nullptr;
+    const int64_t tiles = kvc_v_tiles(v, batch, kv_heads, head_dim);
+#define KVC_COMBINE(U, DECIDES) \
+    hipLaunchKernelGGL((kvc_attention_combine_kernel<U, DECIDES>), cgrid, cblock, 0, stream, part, ml, groups, batch * q_heads, (int)head_dim, d_out_f32, tail, lut, tiles)
+    if (per_wave <= 4) {
+        if (lut) KVC_COMBINE(4, true);
+        else KVC_COMBINE(4, false);
+    } else if (per_wave <= 8) {
+        if (lut) KVC_COMBINE(8, true);
+        else KVC_COMBINE(8, false);
+    } else {
+        if (lut) KVC_COMBINE(16, true);
+        else KVC_COMBINE(16, false);
+    }
+#undef KVC_COMBINE
     KVC_HIP(hipGetLastError());
     return timer.finish();
 }

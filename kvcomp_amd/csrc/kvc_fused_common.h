@@ -192,6 +192,52 @@ __device__ __forceinline__ void kvc_static_for(Body &&body)
     }
 }
 
+// -- the narrow two-symbol table of V's kernels --------------------------------------------------------
+// The table is as wide as the first store's symbols asked for.  Where later data are not like them, tiles meet pairs that do
+// not fit and are decoded twice.  A tile that did is counted, and the kernel that closes the call (one wave of it) adds the
+// counters up and turns the table off for this codebook where it costs more than it gives.  Everything here decides about
+// speed alone: both loops give the same bits, whoever reads or writes these words in between.
+// One tile in sixteen: V kernel in us with the table / one symbol per look-up, by the share of tiles decoded twice,
+//   4 x 32 heads x 96 x 32 768 tokens   1 %: 72.7 / 90.1   6 %: 79.4 / 90.3   11 %: 84.8 / 89.9   24 %: 95.2 / 90.5
+//   8 x 32 heads x 128 x 8192           1 %: 52.2 / 61.8   6 %: 57.0 / 61.8   11 %: 60.0 / 61.6   24 %: 68.4 / 61.7
+//   4 x 32 heads x 128 x 8192           1 %: 35.5 / 37.5   6 %: 37.8 / 37.7   11 %: 39.8 / 37.6   24 %: 43.0 / 37.4
+// (Counters in lines of their own: into one word, every atomic waits for the one before it, and the wave's next loads for
+// it: 244 us instead of 95 in the first row.  The off bit lies in a word that is read anyway.)
+constexpr int KVC_NARROW_TOO_MANY = 16;
+__device__ __forceinline__ void kvc_narrow_miss(const uint32_t *lut, uint32_t block)
+{
+    // (lane number and constants are made here, where they are used: kept in registers across the decode loops they cost some
+    // of the kernels a wave per SIMD)
+    uint32_t id, one, at = block % KVC_NARROW_COUNTERS * (KVC_NARROW_LINE_WORDS * 4u) + KVC_LUT_NARROW_OFFSET * 4u;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(id));
+    if (id != 0) return;
+    asm volatile("v_mov_b32 %0, 1" : "=v"(one));
+    asm volatile("" : "+v"(at));
+    __hip_atomic_fetch_add(reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(const_cast<uint32_t *>(lut)) + at), one,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// One wave, all its lanes: a counter each.
+__device__ __forceinline__ uint32_t *kvc_narrow_counter(uint32_t *lut, int lane)
+{
+    static_assert(KVC_NARROW_COUNTERS == KVC_WAVE, "a counter per lane");
+    return lut + KVC_LUT_NARROW_OFFSET + KVC_NARROW_LINE_WORDS * lane;
+}
+__device__ __forceinline__ uint32_t kvc_narrow_missed(uint32_t *lut, int lane)
+{
+    return __hip_atomic_load(kvc_narrow_counter(lut, lane), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// `tiles`: how many the launch before this one decoded (with this table, if it was on); `missed`: kvc_narrow_missed
+__device__ __forceinline__ void kvc_narrow_decide(uint32_t *lut, uint64_t tiles, int lane, uint32_t missed)
+{
+    if (!__any(missed != 0u)) return;
+    uint32_t *mine = kvc_narrow_counter(lut, lane);
+    __hip_atomic_store(mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) missed += __shfl_xor(missed, s);
+    if (lane == 0 && missed * (uint64_t)KVC_NARROW_TOO_MANY > tiles)
+        __hip_atomic_store(lut + KVC_LUT_NARROW_WORD, lut[KVC_LUT_NARROW_WORD] | KVC_LUT_NARROW_OFF, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // -- tile geometry ------------------------------------------------------------------------------------
 // KIND 0: K tile (64 tokens x head_dim channels of one (batch, head); lane = token)
 // KIND 1: V tile (128 tokens x 64 flat channels; lane = channel), head_dim a multiple of 64: one head per tile

@@ -638,7 +638,8 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     // never occur (KvcFusedArgs::narrow_pair_bits).  A code with smoothing gives every symbol the error bound allows a code, so
     // its longest ones are mostly unused and would keep V from looking up pairs at all.  What does not fit is a pair of NaN in
     // the table; a tile that meets one ends with NaN sums and is decoded again, one symbol per look-up, through the whole
-    // table behind the narrow one (at a multiple of its size, so that "window bits | offset" is an entry's address).
+    // table behind the narrow one (at a multiple of its size, so that "window bits | offset" is an entry's address); where that
+    // happens to many tiles, later launches decode all of theirs like that (kvc_narrow_miss).
     // Batch 4 x 32 heads x 96 x 32 768 tokens, heavy-tailed data, 7 index bits for codes of up to 6: V 88 -> 74 us.  With 8
     // bits (three pairs per half window, 256 words) it measured no better than one symbol per look-up (38.6 / 39.8 us at
     // batch 8 x 32 x 128 x 4096), and K, which has no such codebooks, 8 % slower for the scalars spilled.
@@ -712,6 +713,8 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     const uint32_t fe = kvc_lds_addr(smem);                            // 0: the table opens the workgroup's LDS
 
     if (ntiles <= 0) return;
+    // bit 0: tiles are decoded through the whole table; bit 1: whatever comes of it
+    const int mode = !NARROW_OK || !narrow ? 2 : (lut_g[KVC_LUT_NARROW_WORD] & KVC_LUT_NARROW_OFF) ? 3 : 0;
     KvcRaw<REP, SLOTS, KvcGeom<KIND>::XW> raw;
     // (the one place where the tile's batch entry, head and channel offset are worked out by division)
     KvcTilePos pos = kvc_tile_pos<IS_K>(a, row, col);
@@ -805,12 +808,16 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
                     else if (rest) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, false, EV>(sbase, u, tab, mask4, rest, bptr, msptr, acc, holder);
                 }
             };
-            for (bool whole = false;; whole = true) {
-                if (a.skew) run(std::true_type{}, whole);
-                else run(std::false_type{}, whole);
-                if (!NARROW_OK || !narrow || whole) break;
-                const bool missed = __builtin_isnan(acc[0][0]) || __builtin_isnan(acc[0][1]) || __builtin_isnan(acc[0][2]) || __builtin_isnan(acc[0][3]);
-                if (!__any(missed)) break;                     // (NaN of q or of the weights: the same again)
+            for (int m = mode;; m = 1) {
+                if (a.skew) run(std::true_type{}, (m & 1) != 0);
+                else run(std::false_type{}, (m & 1) != 0);
+                if (!NARROW_OK || (m & 2)) break;
+                const bool nan = __any(__builtin_isnan(acc[0][0]) || __builtin_isnan(acc[0][1]) || __builtin_isnan(acc[0][2]) || __builtin_isnan(acc[0][3]));
+                if (m & 1) {                                   // (NaN of q or of the weights: no miss, and the same again)
+                    if (!nan) kvc_narrow_miss(a.s.luts, blockIdx.x + blockIdx.y);
+                    break;
+                }
+                if (!nan) break;
             }
             // register i of lane 4 b + j: row 4 b + i, column 4 set + j; the even columns take their low parts from
             // the lane to their right and carry the results of query head 2 set + j / 2

@@ -130,6 +130,7 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
         }
         lut[KVC_LUT_FENTRY_OFFSET + idx] = e;
     }
+    for (int i = KVC_LUT_NARROW_OFFSET + tid; i < KVC_LUT_WORDS; i += KVC_WG) lut[i] = 0u;
     __syncthreads();
     if (tid == 0) {
         uint32_t nlong = s_nlong < (uint32_t)KVC_LUT_MAX_LONG ? s_nlong : (uint32_t)KVC_LUT_MAX_LONG;
