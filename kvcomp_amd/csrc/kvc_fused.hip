@@ -1178,6 +1178,15 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     const int slots = (!is_k && head_dim % KVC_WAVE != 0) ? 2 : 1;
     const int kind = is_k ? 0 : (a.scores ? 2 : 0) + slots;
     const int rounded = kvc_option(KVC_OPT_FUSED_ROUNDED) != 0;
+    if (!is_k && kvc_tile_spans_many_heads(head_dim)) {
+        a.rounded = rounded;
+        KvcTimer timer(elapsed_ms, stream);
+        if (!d_luts) {
+            if (int rc = kvc_launch_build_lut(d_decode_tree, decode_tree_bytes, tree_format, (uint32_t *)slot, 1, 0, stream)) return rc;
+        }
+        if (int rc = kvc_launch_v_small_heads((int)rep, a, rows, stream)) return rc;
+        return timer.finish();
+    }
     // The matrix-core kernels take the common case: a codebook whose longest code is known, the plain or
     // skewed packed payload, results that can be stored four at a time.
     const int64_t out_stride = (extra && extra->out_stride) ? extra->out_stride : tokens;
@@ -1250,6 +1259,8 @@ int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_t
     if (deq) {
         if (is_k && quant_mask != KVC_MASK_K_BLOCK && quant_mask != KVC_MASK_CHANNEL) return 1;
         if (!is_k && quant_mask != KVC_MASK_V_TOKEN && quant_mask != KVC_MASK_SIM_TOKEN && quant_mask != KVC_MASK_VECTOR) return 1;
+        // (parameters of a head's or batch entry's own: kept for two of the heads that a tile may touch)
+        if (!is_k && kvc_tile_spans_many_heads(head_dim) && quant_mask != KVC_MASK_V_TOKEN) return 1;
     }
     KVC_REQUIRE(!deq || (((uintptr_t)d_scale & 3) == 0 && ((uintptr_t)d_min & 1) == 0),
                 "quant_scales must be 4-byte aligned and quant_min_ints 2-byte aligned");

@@ -241,8 +241,22 @@ __device__ __forceinline__ void kvc_narrow_decide(uint32_t *lut, uint64_t tiles,
 // -- tile geometry ------------------------------------------------------------------------------------
 // KIND 0: K tile (64 tokens x head_dim channels of one (batch, head); lane = token)
 // KIND 1: V tile (128 tokens x 64 flat channels; lane = channel), head_dim a multiple of 64: one head per tile
-// KIND 2: V tile with any other head_dim: the 64 channels may straddle two heads (two operand tables)
+// KIND 2: V tile with any other head_dim: the 64 channels may straddle two heads (two operand tables); the small ones of
+//         which they may touch more go to kvc_v_small_heads.hip
 // KIND 3, 4: as 1, 2 but with the softmax over the group's scores computed on the fly
+// Whether a tile of 64 flat channels can touch more than two heads: tiles start at every multiple of gcd(head_dim, 64) inside
+// a head, and behind the latest start the head has only that many channels left.
+constexpr bool kvc_tile_spans_many_heads(int64_t head_dim)
+{
+    int64_t g = KVC_WAVE;
+    while (head_dim % g != 0) g /= 2;
+    return KVC_WAVE - g > head_dim;
+}
+static_assert(kvc_tile_spans_many_heads(40) && kvc_tile_spans_many_heads(24) && kvc_tile_spans_many_heads(16) && kvc_tile_spans_many_heads(8) &&
+              !kvc_tile_spans_many_heads(32) && !kvc_tile_spans_many_heads(48) && !kvc_tile_spans_many_heads(56) && !kvc_tile_spans_many_heads(72),
+              "the head sizes that take the kernel of their own");
+int kvc_launch_v_small_heads(int rep, const KvcFusedArgs &a, int64_t rows, hipStream_t stream);
+
 template <int KIND>
 struct KvcGeom {
     static constexpr bool IS_K = KIND == 0;
