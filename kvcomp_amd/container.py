@@ -175,6 +175,11 @@ def check_consistency(header: dict):
     fmt = header.get("tree_format", 3)                     # absent in files written before the field existed: int8 nodes
     if fmt not in (3, 5) or numel("decode_codebook") % fmt:
         fail("decode tree of %d bytes in node format %r" % (numel("decode_codebook"), fmt))
+    # hints of the decoders: sizes of their tables and staging areas
+    for name, most in (("max_code_bits", 32), ("pair_bits", 7), ("max_tile_bytes", 8191), ("max_stream_bytes", 8191)):
+        value = header.get(name, 0)                        # (pair_bits: absent in files written before the field existed)
+        if type(value) is not int or not 0 <= value <= most:
+            fail("%s is %r, expected 0 .. %d" % (name, value, most))
     tail_shape = list(secs["tail"]["shape"]) if secs["tail"]["nbytes"] else [0, B, H, D]
     if tail_shape != [total - comp, B, H, D]:
         fail("the tail has shape %s, expected %s" % (tail_shape, [total - comp, B, H, D]))

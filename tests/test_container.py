@@ -94,6 +94,17 @@ def test_inconsistent_sections_are_refused():
             pytest.fail("accepted: " + what)
 
 
+@pytest.mark.parametrize("name", ["pair_bits", "max_code_bits", "max_tile_bytes", "max_stream_bytes"])
+@pytest.mark.parametrize("value", [-1, 1 << 40, 3.5, "7", None, True])
+def test_hints_that_no_encoder_leaves_are_refused(name, value):
+    from kvcomp_amd import container as Cn
+    blob = Cn.dumps(_Stub())
+    with pytest.raises(Cn.ContainerError, match=name):
+        Cn.parse_header(_rewrite_header(blob, lambda h: h.update({name: value})))
+    Cn.parse_header(_rewrite_header(blob, lambda h: h.update({name: 7})))
+    Cn.parse_header(_rewrite_header(blob, lambda h: h.pop("pair_bits")))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("D", [128, 96])
 def test_save_load_round_trip_on_gpu(tmp_path, D):
