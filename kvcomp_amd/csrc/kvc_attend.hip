@@ -11,12 +11,14 @@
 // two kernels -> this one, the merge of the groups included: 1 x 8 x 4 x 128, 1000: 28.0 -> 16.5 us; 1 x 32 x 1 x 128, 4096:
 // 24.8 -> 18.2; 1 x 32 x 1 x 64, 4096: 21.0 -> 14.6; 1 x 8 x 8 x 128, 3000: 35.3 -> 19.4.
 //
-// Where a wave's 23 500 cycles go (clock stamps, 1 x 32 heads x 128 x 1024 tokens, one workgroup per CU): loads 5200, tables
-// and staging 2700, 128 look-ups in a row 12 000 (V; K alike), scores to weights and two barriers 1400, the products 2150.
+// Where a V wave's 21 600 cycles go (clock stamps, 1 x 32 heads x 128 x 1024 tokens, one workgroup per CU): arguments,
+// one-symbol tables and the tile's loads 5000, tables, staging and operands 2000, 128 look-ups in a row 11 600 (K alike),
+// scores to weights and two barriers 1300, the products 1700.  With four workgroups per CU (4096 tokens) the look-ups take
+// 16 600: the waves then share the LDS.
 // The operands of K's products and of V's are read by all lanes, without a branch, and V's some groups ahead: with the read
-// under the branch that the larger launches use (it saves LDS time) each group of four waited for its own round trip:
-// K 13 900 cycles, V's products 4200.  Registers are given away for that: five waves per SIMD (four with four and eight query
-// heads), which is what the LDS leaves room for.
+// under the branch that the larger launches use (it saves LDS time) each group of four waited for its own round trip: 1 x 8 x
+// 4 x 128, 1000 tokens 19.2 -> 16.5 us.  Registers are given away for that: five waves per SIMD (four with four and eight
+// query heads), which is what the LDS leaves room for.
 //
 // Two symbols per look-up where every pair of codes fits the table (K up to 6 bits, V up to 4): as many look-ups in a row again
 // saved.  Tables that hold nearly all pairs of 7-bit codes, with a second look-up for the rest, gain nothing: waiting for
@@ -310,7 +312,7 @@ __global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP
     for (int q = 0; q < NM; q++) acc[q] = kvc_f4{0.f, 0.f, 0.f, 0.f};
     const uint32_t bptr = kvc_lds_addr(btab_v) + cj * 8, msptr = kvc_lds_addr(mstab);
     // the operands of a few groups are asked for while the groups before them are multiplied (left to itself the compiler asks for
-    // them right before their use: 32 groups, 48 LDS round trips, 3400 cycles)
+    // them right before their use: 32 groups, 48 LDS round trips)
     constexpr int AHEAD = NM <= 2 ? 4 : 2;
     kvc_w4 ms[2][AHEAD];
     kvc_w2 cols[2][AHEAD][NM];

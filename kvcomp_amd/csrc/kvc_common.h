@@ -36,6 +36,7 @@ constexpr int KVC_STAGE_WORDS = KVC_STAGE_BYTES / 4;
 //            length in its lowest mantissa byte (zero for any integer <= 255, so read as a float the entry
 //            is the symbol to within 4e-6 relative, read as a shift count it is the length).  Indices
 //            whose code is longer than lbits or that match no code hold "symbol 0, length 1".
+//   narrow[] 64 counters behind esc[] and bit 31 of the header's word 6, see KVC_LUT_NARROW_OFFSET
 //   esc[ ]   the n_esc codes longer than 7 bits (at most 64 are listed): {code, first stream bit in bit 0; len | sym << 8},
 //            for the loops whose table index has 7 bits
 //   group    how many symbols may be decoded from one 32-bit window: floor(32 / lmax), one of 8,4,2,1.
