@@ -1441,10 +1441,13 @@ __global__ void __launch_bounds__(KVC_WG) kvc_sum_partials_kernel(const uint32_t
     }
 }
 
-// the decode tables whose narrow two-symbol table the call's V kernel may have used, for kvc_narrow_decide
+// the decode tables whose narrow two-symbol table the call's V kernel may have used (kvc_plan_lds: where a table of all pairs
+// would be too wide), for kvc_narrow_decide
 static uint32_t *kvc_narrow_words(const kvc_compressed_desc *v)
 {
-    if (kvc_hint_pair_bits(v->max_code_bits) == 0 || v->rows_per_codebook != 0) return nullptr;
+    const int bits = kvc_hint_bits(v->max_code_bits);
+    if (kvc_hint_pair_bits(v->max_code_bits) == 0 || 2 * bits <= kvc_option(KVC_OPT_FUSED_PAIR_BITS) || bits > KVC_LUT_ESC_BITS) return nullptr;
+    if (v->rows_per_codebook != 0) return nullptr;
     return reinterpret_cast<uint32_t *>(const_cast<void *>(v->d_luts));
 }
 static int64_t kvc_v_tiles(const kvc_compressed_desc *v, int64_t batch, int64_t kv_heads, int64_t head_dim)
