@@ -719,8 +719,8 @@ __device__ __forceinline__ void kvc_slow_emit(const uint32_t *words, uint32_t nw
 //      rows start in all banks); a lane packs the elements of its own row in a register, one word at a time
 //   V: [SLAB tokens][64 channels], dense; consecutive elements of a lane lie a row apart, so they are written singly
 //
-// Dequantizing, the kernels are bound by latency at three to five waves per SIMD (vector ALUs 30 % busy, LDS 56 %) and by how
-// the rows are written, so the slab is as small as it can be where its size does not matter to the writes -- V, whose rows
+// Dequantizing, the kernels are bound by latency at two (K) to four (V) waves per SIMD (vector ALUs 28 - 32 % busy, LDS 46 - 59 %)
+// and by how the rows are written, so the slab is as small as it can be where its size does not matter to the writes -- V, whose rows
 // are a tile's 64 channels whatever their number: 8 tokens, 32 -> 8: 76.6 -> 71.8 us at batch 8 x 32 heads x 128 x 4096
 // tokens --, and for K full cache lines are worth more than the fourth workgroup per CU: rows of 64 channels (128 bytes)
 // 84.6 us, 32 channels 90.5, 16 channels 122.8.  With codes of more than 7 bits K stays at 32 (114.5 against 139.7).
