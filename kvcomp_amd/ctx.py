@@ -352,7 +352,7 @@ class KVCompCtx:
         up to date, and a store that failed on the device is reported here (KvcompError) with the context rolled back to
         the last good store.  Called by store() and by the attention operator; cheap when nothing is outstanding."""
         p = self._probe
-        if p is None or not p[0].query():
+        if p is None or torch.cuda.is_current_stream_capturing() or not p[0].query():      # (an event must not be asked for then)
             return
         w = self._host_words.tolist()
         self._probe = None

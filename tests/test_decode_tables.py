@@ -84,6 +84,26 @@ def test_tables_of_an_assigned_codebook_are_waited_for_and_never_shared_out_of_a
     assert ctx.decode_lut() is built[1][1] and len(waits) == 1
 
 
+def test_nothing_is_asked_of_an_event_while_a_stream_is_recorded(monkeypatch):
+    _config()
+
+    class Event:
+        asked = 0
+
+        def query(self):
+            self.asked += 1
+            return False
+    ctx, event = KVCompCtx(True, 1, 2, 64, 0.1), Event()
+    ctx._probe = event, 1, None
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    ctx.poll_stores()
+    ctx.descriptor()
+    assert event.asked == 0
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    ctx.poll_stores()
+    assert event.asked == 1
+
+
 def _stored(T=700):
     _config()
     pair = KVCompCtx(True, 1, 4, 128, 0.1), KVCompCtx(False, 1, 4, 128, 0.2)
@@ -117,8 +137,7 @@ def test_eager_calls_before_the_replay_of_a_first_call_that_was_recorded():
     k, v = _stored()
     q = S.synth_q(1, 4, 128).to("cuda:0")
     att, out = CompressedAttention(k, v), torch.empty(1, 4, 128, device="cuda:0")
-    torch.cuda.synchronize()
-    k.poll_stores(), v.poll_stores()        # (nothing is asked of the device while it is recorded)
+    assert k._probe is not None and v._probe is not None      # nobody has looked at the stores yet, and the recording must not
     graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
     with torch.cuda.graph(graph, stream=side):
         att.attend(q, out=out)
