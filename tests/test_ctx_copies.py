@@ -116,3 +116,31 @@ def test_contexts_as_the_model_caches_hold_them_can_be_copied_right_after_a_stor
         c.store(x.to("cuda:0"), want_symbols=False)               # the copy goes on by itself
     assert pair[0].ctx_len == 300 and twin[0].ctx_len == 301
     assert torch.equal(CompressedAttention(*pair).attend(q), want)
+
+
+@pytest.mark.gpu
+def test_two_threads_attend_over_one_pair_of_contexts():
+    import threading
+    from kvcomp_amd.attention import CompressedAttention
+    from tests import _synth as S
+    _config()
+    pair = KVCompCtx(True, 2, 4, 128, 0.1), KVCompCtx(False, 2, 4, 128, 0.2)
+    for c, x in zip(pair, (S.synth_k(900, 2, 4, 128), S.synth_v(900, 2, 4, 128))):
+        c.store(x.to("cuda:0"))
+    queries = [S.synth_q(2, 4 * rep, 128, seed).to("cuda:0") for seed, rep in ((1, 1), (2, 4))]
+    want = [CompressedAttention(*pair).attend(q) for q in queries]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def run(q, w):
+        att = CompressedAttention(*pair)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(60):
+                if not torch.equal(att.attend(q), w):
+                    wrong.append(q.shape)
+    threads = [threading.Thread(target=run, args=a) for a in zip(queries, want)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
