@@ -20,11 +20,13 @@ def _words(ctx):
 
 
 @pytest.fixture(autouse=True)
-def two_launches():
+def the_kernels_that_have_the_table():
+    """... whatever the environment presets."""
     from kvcomp_amd import _lib
-    was = _lib.set_option("attention_joint", 0)
+    was = {name: _lib.set_option(name, value) for name, value in (("attention_joint", 0), ("fused_mfma", -1), ("fused_pair_bits", 8), ("fused_rows", -1))}
     yield
-    _lib.set_option("attention_joint", was)
+    for name, value in was.items():
+        _lib.set_option(name, value)
 
 
 @pytest.mark.parametrize("by", ["attend", "mat_vec_mul"])
