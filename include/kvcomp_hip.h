@@ -232,6 +232,21 @@ typedef struct kvc_encode_job {
     uint32_t *d_result;               /* may be NULL if d_stream_bytes is not */
 } kvc_encode_job;
 int kvc_encode_async(const kvc_encode_job *job, void *stream);
+
+/* The same for callers that would rather not wait for what the host has to do in between.
+ * kvc_encode_prepare: the first launch of an encode from symbols whose table and payload buffer are not known yet
+ *   (d_encode_tables, encode_table_bytes, d_encoded and encoded_cap are not looked at).  d_result's eight words and
+ *   *d_stream_bytes are cleared.  d_scratch: kvc_encode_scratch_bytes() of device memory on a 16-byte boundary, in use until
+ *   the encode has run.  *prepared receives what to pass on.
+ * kvc_encode_queue: kvc_encode_async, continuing what was prepared on the same stream for the same tokens and outputs
+ *   (prepared = 0: nothing was; d_scratch is not used then).  h_outcome, if not NULL: 16 words of pinned host memory that
+ *   receive d_result's eight words, *d_stream_bytes and, last, outcome_number (word 9), as the call ends on the device.
+ * kvc_wait_outcome: waits until outcome_number has arrived in such words. */
+int64_t kvc_encode_scratch_bytes(void);
+int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream);
+int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, uint32_t *h_outcome, uint32_t outcome_number,
+                     void *stream);
+int kvc_wait_outcome(const uint32_t *h_outcome, uint32_t outcome_number);
 int kvc_encode_result(const uint32_t *d_result, int64_t encoded_cap, int64_t *h_total_bytes, int64_t *h_max_tile_bytes,
                       int64_t *h_max_stream_bytes, int64_t *h_tiles, void *stream);
 
@@ -424,6 +439,8 @@ int kvc_quant(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H,
  *   symbols written (without the padding of each lane stream to whole bytes).  Waits for the symbol counts, not for the
  *   stream; cannot be recorded into a graph.
  *   pair_bits: index bits of a decode table that next to all pairs of these symbols fit, 2 .. 7, or 0.
+ * kvc_quant_counted, kvc_counted_codebook: the two halves of kvc_quant_codebook.  The first queues the quantizer and hands out
+ *   what the second, called exactly once, waits with; the host is free in between.
  * kvc_put_codebook: the encode table to d_tables, the decode tree behind it on the next 16-byte boundary, and the decode
  *   tables of kvc_build_lut (one codebook) to d_lut, in stream order without waiting; book may be reused at once.
  * kvc_put_bytes: copies host bytes to device memory in stream order without waiting; h_src may be reused at once. */
@@ -434,6 +451,9 @@ typedef struct kvc_codebook {
     uint8_t decode_tree[512 * 5];
     int32_t pair_bits;
 } kvc_codebook;
+int kvc_quant_counted(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
+                      float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, void **counted, void *stream);
+int kvc_counted_codebook(void *counted, int smoothed_symbols, kvc_codebook *out, void *stream);
 int kvc_quant_codebook(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                        float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, int smoothed_symbols,
                        kvc_codebook *out, void *stream);

@@ -62,6 +62,9 @@ _SIGNATURES = {
     "kvc_store_fused": [_int, _vp, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64,
                         _u32, _i64p, _i64p, _i64p, _vp],
     "kvc_encode_async": [C.POINTER(EncodeJob), _vp],
+    "kvc_encode_scratch_bytes": [],
+    "kvc_encode_prepare": [C.POINTER(EncodeJob), _vp, _i64, _intp, _vp],
+    "kvc_encode_queue": [C.POINTER(EncodeJob), _vp, _int, _vp, _u32, _vp],
     "kvc_encode_result": [_vp, _i64, _i64p, _i64p, _i64p, _i64p, _vp],
     "kvc_k_entropy_decode": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _int, _vp, _i64, _i64, _i64, _i64, _f32p, _vp],
     "kvc_v_entropy_decode": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _int, _vp, _i64, _i64, _i64, _i64, _f32p, _vp],
@@ -81,6 +84,9 @@ _SIGNATURES = {
     "kvc_quant_groups": [_i64, _i64, _i64, _i64, _i64, _int],
     "kvc_quant": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp, _vp, _vp, _vp, _vp],
     "kvc_quant_codebook": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp, _vp, _int, C.POINTER(Codebook), _vp],
+    "kvc_wait_outcome": [_vp, _u32],
+    "kvc_quant_counted": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp, _vp, C.POINTER(_vp), _vp],
+    "kvc_counted_codebook": [_vp, _int, C.POINTER(Codebook), _vp],
     "kvc_append_dense": [_vp, _vp],
     "kvc_quant_in_place": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp],
     "kvc_put_codebook": [_vp, _vp, _vp, _vp],
@@ -101,7 +107,7 @@ _SIGNATURES = {
     "kvc_dequant": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _int, _vp, _vp],
 }
 _RESTYPES = {"kvc_quant_groups": _i64, "kvc_lut_bytes": _i64, "kvc_codebook_tree_capacity": _i64, "kvc_attention_workspace_bytes": _i64,
-             "kvc_h2_scratch_bytes": _i64}
+             "kvc_h2_scratch_bytes": _i64, "kvc_encode_scratch_bytes": _i64}
 
 EXPORTED_SYMBOLS = sorted(list(_SIGNATURES) + ["kvc_last_error"])
 

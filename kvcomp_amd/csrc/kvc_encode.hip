@@ -51,6 +51,9 @@ struct KvcEncodeArgs {
     // results left on the device (kvc_encode_async): see kvc_encode_job in include/kvcomp_hip.h
     uint32_t *stream_bytes;    // NULL, or in / out: payload bytes already in `encoded`; this call appends behind them
     uint32_t *result;          // NULL, or uint32[8]
+    uint32_t *outcome;         // NULL, or 16 words of pinned host memory that receive the results too (kvc_encode_queue)
+    uint32_t outcome_number;
+    int clear;                 // the result words are new: cleared by the call's first launch
     // one pass only: how often a wave may find a word of its look-back not ready before it gives up, and whether the
     // call is to be treated as if a wave had given up (both from the option "encode_lookback_polls")
     int max_polls, force_order;
@@ -78,6 +81,10 @@ __device__ __forceinline__ void kvc_encode_init(const KvcEncodeArgs &a)
     __shared__ uint32_t s_bad;
     const int tid = threadIdx.x;
     if (tid == 0) s_bad = 0;
+    if (a.clear) {
+        if (tid < 8) a.result[tid] = 0u;
+        if (tid == 8) *a.stream_bytes = 0u;
+    }
     __syncthreads();
     if (a.codebook_meta)
         for (int i = tid; i < a.n_codebooks; i += (int)blockDim.x)
@@ -86,7 +93,7 @@ __device__ __forceinline__ void kvc_encode_init(const KvcEncodeArgs &a)
     if (tid < KVC_ENC_STATUS_WORDS) {
         uint32_t v = 0;
         if (tid == 1) v = s_bad;
-        if (tid == KVC_ENC_ST_BASE) v = a.base_global_offset + (a.stream_bytes ? *a.stream_bytes : 0u);
+        if (tid == KVC_ENC_ST_BASE) v = a.base_global_offset + (a.stream_bytes && !a.clear ? *a.stream_bytes : 0u);
         a.status[tid] = v;
     }
     __syncthreads();
@@ -107,6 +114,13 @@ __device__ __forceinline__ void kvc_encode_publish(const KvcEncodeArgs &a)
         if (a.status[6] > a.result[6]) a.result[6] = a.status[6];
     }
     if (a.stream_bytes && !err) *a.stream_bytes = a.status[KVC_ENC_ST_BASE] - a.base_global_offset + total;
+    if (a.outcome) {
+        // the host looks at these words without asking the runtime: system-scope stores, then the call's number with release
+        // order (as kvc_counts_to_host_kernel); a copy and an event behind the call cost 8 us of host time and a launch
+        for (int i = 0; i < 8; i++) __hip_atomic_store(&a.outcome[i], a.result[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&a.outcome[8], *a.stream_bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&a.outcome[9], a.outcome_number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 __global__ void kvc_encode_publish_kernel(KvcEncodeArgs a) { kvc_encode_publish(a); }
@@ -1424,6 +1438,10 @@ struct KvcStoreSource {
     void *scale_f16;
 };
 
+// How far an encode call has come before kvc_encode_launch: nothing, the status words set, the block_infos marked as well
+// (then it takes one pass, else two).
+enum { KVC_ENC_FRESH = 0, KVC_ENC_CLEARED = 1, KVC_ENC_MARKED = 2 };
+
 // Everything an encode call is made of; the classic entry points fill in what they have and leave the rest zero.
 struct KvcEncodeCall {
     int is_k;
@@ -1437,6 +1455,13 @@ struct KvcEncodeCall {
     uint32_t base_global_offset;
     uint32_t *d_stream_bytes, *d_result;
     const KvcStoreSource *src;
+    // kvc_encode_prepare / kvc_encode_queue: scratch of the caller's instead of a slot of the ring; the first launch only, or
+    // everything but the first launch
+    void *scratch;
+    int clear;
+    bool first_launch_only;
+    int first_launch;                                      // what is done already: KVC_ENC_FRESH, KVC_ENC_CLEARED or KVC_ENC_MARKED
+    uint32_t *h_outcome, outcome_number;
 };
 
 static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
@@ -1452,7 +1477,8 @@ static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
 }
 
 // Queue the launches of one encode call (init, count, per-1024-tile sums, offsets, emit, publish); waits for nothing.
-// *slot receives the call's status words on the device.
+// *slot receives the call's status words on the device.  With first_launch_only: only the first of them; returns what that
+// was (positive), or an error.
 static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_t stream)
 {
     int64_t sizes[4];
@@ -1469,8 +1495,9 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     KVC_REQUIRE(c.stride % 4 == 0, "stride must be a multiple of 4");
     KVC_REQUIRE(c.rows_per_codebook >= 0 && (c.rows_per_codebook == 0 || (c.table_stride >= c.table_bytes && c.table_stride % 8 == 0)),
                 "tables of several codebooks must be a multiple of 8 bytes apart and not overlap");
-    void *slot;
-    if (int rc = kvc_workspace_slot(&slot, (void *)stream)) return rc;
+    void *slot = c.scratch;
+    if (!slot)
+        if (int rc = kvc_workspace_slot(&slot, (void *)stream)) return rc;
     KvcEncodeArgs a;
     a.sym = c.d_sym;
     a.stride = c.stride;
@@ -1494,6 +1521,9 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     a.idx_offset = reinterpret_cast<uint32_t *>(c.d_idx_offset);
     a.stream_bytes = c.d_stream_bytes;
     a.result = c.d_result;
+    a.outcome = c.h_outcome;
+    a.outcome_number = c.outcome_number;
+    a.clear = c.clear;
     a.max_polls = 0;
     a.force_order = 0;
     const int64_t chunks = (a.tiles + 1023) / 1024;
@@ -1519,8 +1549,19 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     // (which fetches them through its LDS tile, whole token rows per load instruction) than in two; at 96 tiles the one
     // pass is three launches instead of six.
     const int one_pass = kvc_option(KVC_OPT_ENCODE_ONE_PASS);
-    if (one_pass != 0 && ((uintptr_t)c.d_block_infos & 7) == 0 &&
-        (a.tiles + KVC_ONCE_GROUP_TILES - 1) / KVC_ONCE_GROUP_TILES <= KVC_ONCE_MAX_GROUPS) {
+    const bool fits = ((uintptr_t)c.d_block_infos & 7) == 0 && (a.tiles + KVC_ONCE_GROUP_TILES - 1) / KVC_ONCE_GROUP_TILES <= KVC_ONCE_MAX_GROUPS;
+    const bool once = c.first_launch == KVC_ENC_FRESH ? one_pass != 0 && fits : c.first_launch == KVC_ENC_MARKED && fits;
+    *slot_out = slot;
+    if (c.first_launch == KVC_ENC_FRESH) {
+        if (once) hipLaunchKernelGGL(kvc_encode_mark_kernel, dim3((unsigned)((a.tiles + KVC_WG - 1) / KVC_WG)), dim3(KVC_WG), 0, stream, a);
+        else hipLaunchKernelGGL(kvc_encode_init_kernel, dim3(1), dim3(KVC_WAVE), 0, stream, a);
+    }
+    a.clear = 0;                                           // (once per call)
+    if (c.first_launch_only) {
+        if (int rc = kvc_check_hip(hipGetLastError(), "encode init launch")) return rc;
+        return once ? KVC_ENC_MARKED : KVC_ENC_CLEARED;
+    }
+    if (once) {
         // how often a wave may find a word of its look-back not ready; -1 makes the call take the give-up path
         // (every wave still ends normally) so that tests can reach it from the host
         const int polls_opt = kvc_option(KVC_OPT_ENCODE_LOOKBACK_POLLS);
@@ -1537,11 +1578,10 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
                            a.encoded_cap / a.tiles <= (KVC_ONCE_SMALL_WAVE_BYTES - kvc_once_stage_bytes(0)) * 4 / 5;
         sa.e.wave_bytes = small ? KVC_ONCE_SMALL_WAVE_BYTES : KVC_ONCE_WAVE_BYTES;
         const size_t lds = (size_t)(a.rows_per_codebook ? KVC_WAVES_PER_WG : 1) * 256 * sizeof(uint2) + (size_t)KVC_WAVES_PER_WG * sa.e.wave_bytes;
-        hipLaunchKernelGGL(kvc_encode_mark_kernel, dim3((unsigned)((a.tiles + KVC_WG - 1) / KVC_WG)), dim3(KVC_WG), 0, stream, a);
         // two tiles per wave (the look-back of the first hides behind the count of the second) where all tiles share
         // the codebook and there are enough of them to keep the chip full.  Longer runs would need the payloads of
         // more than one waiting tile in LDS.
-        const int want = one_pass;
+        const int want = one_pass != 0 ? one_pass : 1;
         int run = want == 1 ? (a.tiles >= 8192 ? 2 : 1) : want - 1;       // 2, 3: always one, two tiles per wave
         run = run < 1 ? 1 : run > 2 ? 2 : run;
         if (a.rows_per_codebook != 0) run = 1;
@@ -1557,10 +1597,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
             hipLaunchKernelGGL(kvc_encode_finish_kernel<2>, dim3(1), dim3(KVC_WG), 0, stream, sa);
         }
         KVC_HIP(hipGetLastError());
-        *slot_out = slot;
         return 0;
     }
-    hipLaunchKernelGGL(kvc_encode_init_kernel, dim3(1), dim3(KVC_WAVE), 0, stream, a);
     if (!src) hipLaunchKernelGGL(kvc_encode_count_kernel, dim3(wgs), dim3(KVC_WG), 0, stream, a);
     else if (is_k) hipLaunchKernelGGL(kvc_store_count_kernel<true>, dim3(wgs), dim3(KVC_WG), 0, stream, sa);
     else hipLaunchKernelGGL(kvc_store_count_kernel<false>, dim3(wgs), dim3(KVC_WG), 0, stream, sa);
@@ -1571,7 +1609,6 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     else hipLaunchKernelGGL(kvc_store_emit_kernel<false>, dim3(wgs), dim3(KVC_WG), 0, stream, sa);
     if (a.result || a.stream_bytes) hipLaunchKernelGGL(kvc_encode_publish_kernel, dim3(1), dim3(1), 0, stream, a);
     KVC_HIP(hipGetLastError());
-    *slot_out = slot;
     return 0;
 }
 
@@ -1686,14 +1723,13 @@ extern "C" int kvc_store_fused(int is_k, const void *d_x_f16, int64_t tokens, in
 // reference, whose encoder copies its counters to the host and waits for the device on every call,
 // kvcomp_cuda_extension/src/kernels.cu:950-965)
 // ---------------------------------------------------------------------------------------------------
-extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream)
+static int kvc_encode_job_check(const kvc_encode_job *job, KvcEncodeCall &c)
 {
     KVC_REQUIRE(job != nullptr, "NULL argument");
     KVC_REQUIRE(job->batch > 0 && job->heads > 0 && job->head_dim > 0 && job->tokens > 0, "empty geometry");
     KVC_REQUIRE(job->d_result != nullptr || job->d_stream_bytes != nullptr, "the call would leave no result anywhere");
     const int64_t stride = job->batch * job->heads * job->head_dim;
     KVC_REQUIRE(job->tokens % (job->is_k ? KVC_K_VEC_PER_BLK : KVC_V_VEC_LEN) == 0, "token count must be whole tiles");
-    KvcEncodeCall c = {};
     c.is_k = job->is_k;
     c.d_sym = job->d_sym;
     c.tokens = job->tokens;
@@ -1712,6 +1748,47 @@ extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream)
     c.base_global_offset = job->base_global_offset;
     c.d_stream_bytes = job->d_stream_bytes;
     c.d_result = job->d_result;
+    return 0;
+}
+
+extern "C" int64_t kvc_encode_scratch_bytes(void) { return KVC_WS_SLOT_BYTES; }
+
+// The launches in front of an encode whose table is not known yet (a first store: they run while the host builds the code).
+extern "C" int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream)
+{
+    KVC_REQUIRE(prepared != nullptr, "NULL argument");
+    *prepared = KVC_ENC_FRESH;
+    KvcEncodeCall c = {};
+    if (int rc = kvc_encode_job_check(job, c)) return rc;
+    KVC_REQUIRE(job->d_result != nullptr && job->d_stream_bytes != nullptr, "NULL argument");
+    KVC_REQUIRE(d_scratch != nullptr && ((uintptr_t)d_scratch & 15) == 0 && scratch_bytes >= (int64_t)KVC_WS_SLOT_BYTES, "scratch memory: %lld bytes, on a 16-byte boundary",
+                (long long)KVC_WS_SLOT_BYTES);
+    KVC_REQUIRE(job->d_sym != nullptr && job->rows_per_codebook == 0 && job->d_codebook_meta == nullptr, "only an encode from symbols with one codebook can be prepared");
+    static const uint8_t no_table[8] = {};
+    c.d_tables = no_table;                                 // (not read by the launch; the call has its own)
+    c.table_bytes = 8;
+    c.scratch = d_scratch;
+    c.clear = 1;
+    c.first_launch_only = true;
+    void *slot;
+    const int rc = kvc_encode_launch(c, &slot, (hipStream_t)stream);
+    if (rc < 0) return rc;
+    *prepared = rc;
+    return 0;
+}
+
+extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, uint32_t *h_outcome, uint32_t outcome_number, void *stream)
+{
+    KvcEncodeCall c = {};
+    if (int rc = kvc_encode_job_check(job, c)) return rc;
+    KVC_REQUIRE(prepared == KVC_ENC_FRESH || ((prepared == KVC_ENC_CLEARED || prepared == KVC_ENC_MARKED) && d_scratch && job->d_sym &&
+                                              job->rows_per_codebook == 0 && job->d_result && job->d_stream_bytes),
+                "the call does not continue what was prepared");
+    KVC_REQUIRE(h_outcome == nullptr || (job->d_result && job->d_stream_bytes && ((uintptr_t)h_outcome & 3) == 0), "an outcome needs d_result and d_stream_bytes");
+    c.scratch = prepared ? d_scratch : nullptr;
+    c.first_launch = prepared;
+    c.h_outcome = h_outcome;
+    c.outcome_number = outcome_number;
     KvcStoreSource src = {job->d_x_f16, job->batch, job->heads, job->quant_mask, job->eb, job->d_min_i8, job->d_scale_f16};
     if (!job->d_sym) {
         KVC_REQUIRE(kvc_store_fused_supported(job->is_k, job->quant_mask, job->batch, job->heads, job->head_dim),
@@ -1731,6 +1808,8 @@ extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream)
     void *slot;
     return kvc_encode_launch(c, &slot, (hipStream_t)stream);
 }
+
+extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream) { return kvc_encode_queue(job, nullptr, KVC_ENC_FRESH, nullptr, 0u, stream); }
 
 extern "C" int kvc_encode_result(const uint32_t *d_result, int64_t encoded_cap, int64_t *h_total_bytes, int64_t *h_max_tile_bytes,
                                  int64_t *h_max_stream_bytes, int64_t *h_tiles, void *stream)

@@ -8,7 +8,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <vector>
 
 // ---------------------------------------------------------------------------------------------------
 // errors
@@ -225,49 +224,47 @@ extern "C" int kvc_calculate_buffer_size(int64_t tokens, int64_t stride, int is_
 // arrives at the same codes.)
 // ---------------------------------------------------------------------------------------------------
 namespace {
-struct HNode {
-    int64_t f;
-    int left, right, sym;
-};
+// Everything of one construction, without an allocation: at most 256 leaves and 255 inner nodes.
+struct HuffmanBuild {
+    int64_t f[511];
+    int16_t left[511], right[511], sym[511];
+    int nodes = 0;
+    int16_t h[256];
+    int n = 0;
 
-struct FreqHeap {
-    std::vector<int> h;
-    const std::vector<HNode> &nodes;
-    explicit FreqHeap(const std::vector<HNode> &n) : nodes(n) {}
-    bool less(int a, int b) const { return nodes[a].f < nodes[b].f; }
-    void push(int x)
+    int add(int64_t freq, int l, int r, int s)
     {
-        h.push_back(x);
-        size_t pos = h.size() - 1;
+        f[nodes] = freq;
+        left[nodes] = (int16_t)l;
+        right[nodes] = (int16_t)r;
+        sym[nodes] = (int16_t)s;
+        return nodes++;
+    }
+    void sift_up(int pos, int x)
+    {
         while (pos > 0) {
-            size_t par = (pos - 1) >> 1;
-            if (!less(x, h[par])) break;
+            const int par = (pos - 1) >> 1;
+            if (!(f[x] < f[h[par]])) break;
             h[pos] = h[par];
             pos = par;
         }
-        h[pos] = x;
+        h[pos] = (int16_t)x;
     }
+    void push(int x) { sift_up(n++, x); }
     int pop()
     {
-        int last = h.back();
-        h.pop_back();
-        if (h.empty()) return last;
-        int top = h[0];
-        size_t pos = 0, child = 1, n = h.size();
+        const int last = h[--n];
+        if (n == 0) return last;
+        const int top = h[0];
+        int pos = 0, child = 1;
         while (child < n) {
-            size_t right = child + 1;
-            if (right < n && !less(h[child], h[right])) child = right;
+            const int right_child = child + 1;
+            if (right_child < n && !(f[h[child]] < f[h[right_child]])) child = right_child;
             h[pos] = h[child];
             pos = child;
             child = 2 * pos + 1;
         }
-        while (pos > 0) {
-            size_t par = (pos - 1) >> 1;
-            if (!less(last, h[par])) break;
-            h[pos] = h[par];
-            pos = par;
-        }
-        h[pos] = last;
+        sift_up(pos, last);
         return top;
     }
 };
@@ -276,39 +273,35 @@ struct FreqHeap {
 // code/length per symbol; returns number of distinct symbols or -1 when a code exceeds 32 bits.
 static int kvc_huffman_codes(const int64_t *counts, uint32_t code[256], uint32_t length[256])
 {
-    std::vector<HNode> nodes;
-    nodes.reserve(512);
-    FreqHeap heap(nodes);
+    HuffmanBuild t;
     for (int s = 0; s < 256; s++) {
         code[s] = 0;
         length[s] = 0;
-        if (counts[s] > 0) {
-            nodes.push_back({counts[s], -1, -1, s});
-            heap.push((int)nodes.size() - 1);
-        }
+        if (counts[s] > 0) t.push(t.add(counts[s], -1, -1, s));
     }
-    int distinct = (int)nodes.size();
+    const int distinct = t.nodes;
     if (distinct < 2) return distinct;   // 0 symbols: nothing; 1 symbol: empty code (huffman.cpp:60-71)
-    while (heap.h.size() > 1) {
-        int a = heap.pop();
-        int b = heap.pop();
-        nodes.push_back({nodes[a].f + nodes[b].f, a, b, -1});
-        heap.push((int)nodes.size() - 1);
+    while (t.n > 1) {
+        const int a = t.pop();
+        const int b = t.pop();
+        t.push(t.add(t.f[a] + t.f[b], a, b, -1));
     }
-    struct Item { int node; uint64_t code; int len; };
-    std::vector<Item> stack{{heap.h[0], 0, 0}};
-    while (!stack.empty()) {
-        Item it = stack.back();
-        stack.pop_back();
-        const HNode &nd = nodes[it.node];
-        if (nd.left < 0) {
-            if (it.len > 32) return -1;
-            code[nd.sym] = (uint32_t)it.code;
-            length[nd.sym] = (uint32_t)it.len;
+    // a node's children come before it: from the root (the last one) down, every node hands its code to them
+    uint64_t node_code[511];
+    int node_len[511];
+    node_code[t.nodes - 1] = 0;
+    node_len[t.nodes - 1] = 0;
+    for (int i = t.nodes - 1; i >= 0; i--) {
+        const int len = node_len[i];
+        if (t.left[i] < 0) {
+            if (len > 32) return -1;
+            code[t.sym[i]] = (uint32_t)node_code[i];
+            length[t.sym[i]] = (uint32_t)len;
         } else {
-            if (it.len >= 63) return -1;
-            stack.push_back({nd.right, (it.code << 1) | 1u, it.len + 1});
-            stack.push_back({nd.left, it.code << 1, it.len + 1});
+            if (len >= 63) return -1;
+            node_code[t.left[i]] = node_code[i] << 1;
+            node_code[t.right[i]] = (node_code[i] << 1) | 1u;
+            node_len[t.left[i]] = node_len[t.right[i]] = len + 1;
         }
     }
     return distinct;
@@ -353,7 +346,9 @@ extern "C" int kvc_build_codebook_host(const int64_t *h_counts256, int tree_form
     *encode_bytes = eb;
     // decode tree: insert symbols in ascending order, appending nodes on demand (huffman.cpp:229-252)
     struct TNode { bool leaf; int child[2]; };
-    std::vector<TNode> tree(2, TNode{false, {-1, -1}});
+    TNode tree[512];                                       // (a full binary tree of at most 256 leaves, without its root)
+    int nodes = 2;
+    tree[0] = tree[1] = TNode{false, {-1, -1}};
     for (int s = 0; s < 256; s++) {
         if (h_counts256[s] <= 0) continue;
         int idx = -1, last = -1;
@@ -361,8 +356,8 @@ extern "C" int kvc_build_codebook_host(const int64_t *h_counts256, int tree_form
             int bit = (int)((code[s] >> (length[s] - 1 - i)) & 1u);
             idx = (idx == -1) ? bit : tree[idx].child[bit];
             if (idx == -1) {
-                tree.push_back(TNode{false, {-1, -1}});
-                idx = (int)tree.size() - 1;
+                idx = nodes++;
+                tree[idx] = TNode{false, {-1, -1}};
                 tree[last].child[bit] = idx;
             }
             last = idx;
@@ -370,19 +365,19 @@ extern "C" int kvc_build_codebook_host(const int64_t *h_counts256, int tree_form
         tree[idx].leaf = true;
         tree[idx].child[0] = tree[idx].child[1] = s;
     }
-    int64_t db = (int64_t)tree.size() * tree_format;
+    int64_t db = (int64_t)nodes * tree_format;
     KVC_REQUIRE(db <= decode_cap, "decode tree needs %lld bytes", (long long)db);
     if (tree_format == KVC_TREE_I8) {
-        KVC_REQUIRE(tree.size() <= 128 && mx <= 127,
-                    "code not representable in the reference's int8 tree (%zu nodes, max symbol %d): "
-                    "use KVC_TREE_I16", tree.size(), mx);
-        for (size_t n = 0; n < tree.size(); n++) {
+        KVC_REQUIRE(nodes <= 128 && mx <= 127,
+                    "code not representable in the reference's int8 tree (%d nodes, max symbol %d): "
+                    "use KVC_TREE_I16", nodes, mx);
+        for (int n = 0; n < nodes; n++) {
             h_decode_tree[3 * n] = tree[n].leaf ? 1 : 0;
             h_decode_tree[3 * n + 1] = (uint8_t)(int8_t)tree[n].child[0];
             h_decode_tree[3 * n + 2] = (uint8_t)(int8_t)tree[n].child[1];
         }
     } else {
-        for (size_t n = 0; n < tree.size(); n++) {
+        for (int n = 0; n < nodes; n++) {
             int16_t a = (int16_t)tree[n].child[0], b = (int16_t)tree[n].child[1];
             h_decode_tree[5 * n] = tree[n].leaf ? 1 : 0;
             std::memcpy(h_decode_tree + 5 * n + 1, &a, 2);

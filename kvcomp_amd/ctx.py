@@ -12,7 +12,9 @@ get_only_compressed, get_decode_quant_ints, mat_vec_mul, build_codebook, get_cr)
   * batch > 1 and per-channel K (QuantMode.ChannelQuant) are accepted.
 """
 import ast
+import collections
 import ctypes as C
+import itertools
 import math
 import struct
 from typing import Dict, List, NamedTuple, Optional, Tuple
@@ -134,14 +136,16 @@ class _Growable:
         self.data[self.used:self.used + n] = t
         self.used += n
 
-    def reserve(self, n: int, tail_shape, dtype, device):
-        """Make room for n more rows behind the filled part (which is kept); returns the view of those rows."""
+    def reserve(self, n: int, tail_shape, dtype, device, pending: int = 0):
+        """Make room for n more rows behind the filled part (which is kept, with `pending` rows behind it); returns the view
+        of the rows behind the filled part."""
+        kept = self.used + pending
         if self.data is None:
             self._hold(torch.empty((n + max(n // 4, 16),) + tuple(tail_shape), dtype=dtype, device=device))
-        elif self.used + n > self.data.shape[0]:
-            cap = self.used + n + max((self.used + n) // 4, 16)
+        elif kept + n > self.data.shape[0]:
+            cap = kept + n + max((kept + n) // 4, 16)
             grown = torch.empty((cap,) + tuple(self.data.shape[1:]), dtype=self.data.dtype, device=self.data.device)
-            grown[:self.used] = self.data[:self.used]
+            grown[:kept] = self.data[:kept]
             self._hold(grown)
         return self.data[self.used:self.used + n]
 
@@ -156,6 +160,43 @@ class _Growable:
     @property
     def view(self) -> Optional[torch.Tensor]:
         return None if self.data is None else self.data[:self.used]
+
+
+class _Outcome:
+    """Pinned host words that a context's queued encodes leave their result in: written by an encode's last kernel and closed
+    with the number of the call (word 9).  Used like an event; looking costs no call into the runtime, where a copy and an
+    event behind every encode cost ten microseconds of host time and a launch."""
+    _numbers = itertools.count(1)
+    _late: collections.deque = collections.deque()       # words whose context is gone while a kernel may still write to them
+    __slots__ = ("words", "_seen", "number", "stream")
+
+    def __init__(self):
+        for _ in range(len(_Outcome._late)):
+            try:
+                late = _Outcome._late.popleft()
+            except IndexError:
+                break
+            if int(late[0][9]) != late[1]:
+                _Outcome._late.append(late)
+        self.number = self.stream = 0
+        self.words = torch.empty(16, dtype=torch.int32, pin_memory=True)
+        self._seen = self.words.numpy()
+        self._seen[9] = 0
+
+    def ask(self, stream: int) -> Tuple[int, int]:
+        """What the next encode on `stream` is to be told."""
+        self.number, self.stream = (next(_Outcome._numbers) & 0x7fffffff) or 1, stream
+        return self.words.data_ptr(), self.number
+
+    def query(self) -> bool:
+        return int(self._seen[9]) == self.number
+
+    def synchronize(self):
+        _lib.check(_lib.lib().kvc_wait_outcome(self.words.data_ptr(), self.number))
+
+    def __del__(self):
+        if getattr(self, "_seen", None) is not None and not self.query():
+            self._late.append((self._seen, self.number))
 
 
 class _QueuedStore(NamedTuple):
@@ -235,12 +276,13 @@ class KVCompCtx:
         self._state: Optional[torch.Tensor] = None
         self._enc_pending = 0
         # Stores that were queued and not yet seen to succeed, oldest first; _verified is the bookkeeping behind the last
-        # store that is known to be good.  _probe = (event, stores covered) while a copy of the device words to
-        # _host_words (pinned) is on its way: reading it later costs no wait.
+        # store that is known to be good.  _probe = (event, stores covered, stream) while the device words are on their way to
+        # the host: an encode's own _outcome, or a copy to _host_words (pinned).  Reading them later costs no wait.
         self._unverified: List[_QueuedStore] = []
         self._verified = None
         self._probe = None
         self._host_words: Optional[torch.Tensor] = None
+        self._outcome: Optional[_Outcome] = None
         self._trim_after_sync = False
         self.waits = 0                     # how often this context has waited for the device to learn sizes
 
@@ -248,7 +290,7 @@ class KVCompCtx:
         # (copies and pickles: queued stores are waited for, since a copy cannot share the event and the pinned words that
         # will say what became of them)
         self._sync_sizes()
-        return {**self.__dict__, "_probe": None, "_host_words": None}
+        return {**self.__dict__, "_probe": None, "_host_words": None, "_outcome": None}
 
     def _device_state(self) -> torch.Tensor:
         if self._state is None:
@@ -269,7 +311,7 @@ class KVCompCtx:
         p = self._probe
         if p is not None and p[1] == len(self._unverified):     # a copy of the device words behind the last store is on its way
             p[0].synchronize()
-            if int(self._host_words[1]) == 0:
+            if p[0].query() and int(self._arrived_words(p)[1]) == 0:
                 self.waits += 1
                 self.poll_stores()
                 return
@@ -335,17 +377,33 @@ class KVCompCtx:
         """Ask for a copy of the device words without waiting for it (nothing is asked for while the stream is being
         recorded into a graph, or while an earlier copy is on its way on another stream; one on this stream is replaced
         by the newer one, which arrives after it in the same place and covers more stores)."""
-        if not self._unverified or torch.cuda.is_current_stream_capturing():
+        p = self._probe
+        if not self._unverified or (p is not None and p[1] == len(self._unverified)) or torch.cuda.is_current_stream_capturing():
             return
-        stream = torch.cuda.current_stream(self.device)
-        if self._probe is not None and self._probe[2] != stream:
+        stream = _lib.stream_of(self._state)
+        if p is not None and p[2] != stream:
             return
         if self._host_words is None:
             self._host_words = torch.empty(16, dtype=torch.int32, pin_memory=True)
         self._host_words.copy_(self._state, non_blocking=True)
         ev = torch.cuda.Event()
-        ev.record(stream)
+        ev.record(torch.cuda.current_stream(self.device))
         self._probe = (ev, len(self._unverified), stream)
+
+    def _ask_outcome(self):
+        """The _Outcome that the encode about to be queued is to write, or None (as for _issue_probe, which then asks for a
+        copy behind it where that is possible)."""
+        if self.device.type != "cuda" or torch.cuda.is_current_stream_capturing():
+            return None
+        stream = _lib.stream_of(self._state)
+        if self._probe is not None and self._probe[2] != stream:
+            return None
+        if self._outcome is None or (self._outcome.stream != stream and not self._outcome.query()):
+            self._outcome = _Outcome()                         # (words that another stream may still write to are left to it)
+        return self._outcome
+
+    def _arrived_words(self, probe):
+        return probe[0].words if isinstance(probe[0], _Outcome) else self._host_words
 
     def poll_stores(self):
         """Look, without waiting, at what the stores queued by async_store have left: sizes and size hints are brought
@@ -354,7 +412,7 @@ class KVCompCtx:
         p = self._probe
         if p is None or torch.cuda.is_current_stream_capturing() or not p[0].query():      # (an event must not be asked for then)
             return
-        w = self._host_words.tolist()
+        w = self._arrived_words(p).tolist()
         self._probe = None
         if w[1] != 0:
             self._sync_sizes()                                 # takes the stores back and raises, with the library's message
@@ -538,33 +596,48 @@ class KVCompCtx:
     async_store = False
     # stores of up to this many blocks are queued without a wait; longer ones (a second chunk of a prompt) are waited for
     ASYNC_KEEP_BLOCKS = 8
+    # a growing payload buffer takes up to this many bytes along of which it is not known yet whether they are payload (a copy
+    # of this much takes about as long as a wait)
+    COPY_PENDING = 8 << 20
 
     def _encode_direct(self, T: int, *, tables, table_bytes, symbols=None, cache=None, mask=0, most_bytes=None, keep=None,
-                       lost_if_dropped=False, certain=False, codebook=False):
+                       lost_if_dropped=False, certain=False, codebook=False, prepared=None):
         """Queue one encode whose outputs go straight to their final places in this context's buffers; nothing waits.
         Quantizes `cache` on the fly (fused store) or takes `symbols` whose parameters are in place already.  most_bytes:
-        what the payload is known not to exceed."""
+        what the payload is known not to exceed; prepared: what _prepare_encode returned."""
         nb = T // self.block_size
         B, H, D = self.batch_size, self.head_num, self.head_dim
-        sizes = kvcomp_cuda.buffer_sizes(T, B * H * D, self.is_k, H, D)
-        gshape = mask_keepdim_shape((nb, self.block_size, B, H, D), dims_to_mask(self.quant_dims))
+        sizes = kvcomp_cuda.buffer_sizes(T, B * H * D, self.is_k, H, D) if prepared is None else prepared.sizes
         state = self._device_state()
         if not self._unverified:
             self._sync_sizes()                                 # (a no-op unless sizes are outstanding for another reason)
             self._verified = self._bookkeeping() + (self._encoded.used,)
-        bi = self._block_infos.reserve(sizes[0], (), torch.uint8, self.device)
-        ti = self._thread_infos.reserve(sizes[1], (), torch.uint8, self.device)
-        mn = self._min_ints.reserve(nb, gshape[1:], torch.int8, self.device)
-        sc = self._scales.reserve(nb, gshape[1:], torch.float16, self.device)
+        if prepared is None:
+            bi = self._block_infos.reserve(sizes[0], (), torch.uint8, self.device)
+            ti = self._thread_infos.reserve(sizes[1], (), torch.uint8, self.device)
+            mn = sc = None                                     # (symbols: their parameters are in place)
+            if cache is not None:
+                gshape = mask_keepdim_shape((nb, self.block_size, B, H, D), self._mask)
+                mn = self._min_ints.reserve(nb, gshape[1:], torch.int8, self.device)
+                sc = self._scales.reserve(nb, gshape[1:], torch.float16, self.device)
         worst = T * B * H * D if most_bytes is None else most_bytes       # the reference's pre-allocation: a byte per symbol
         if (self._encoded.data is None or
                 self._encoded.used + self._enc_pending + worst > self._encoded.data.numel()):
-            self._sync_sizes()                                 # growing copies the filled part: it has to be known
-            self._encoded.reserve(worst, (), torch.uint8, self.device)
-        kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
-                                 table_bytes=table_bytes, block_infos=bi, thread_infos=ti, encoded=self._encoded.data,
-                                 symbols=symbols, cache=cache, quant_mask=mask, eb=self.quant_scale_rel, min_ints=mn, scales=sc,
-                                 stream_bytes=state[8:9], result=state[:8])
+            # growing copies the filled part, or -- while queued stores have yet to say how much that is -- what it can be at most
+            if self._probe is not None:
+                self.poll_stores()
+            if self._enc_pending > self.COPY_PENDING or (self._enc_pending and torch.cuda.is_current_stream_capturing()):
+                self._sync_sizes()
+            self._encoded.reserve(worst, (), torch.uint8, self.device, self._enc_pending)
+        outcome = self._ask_outcome()
+        told = None if outcome is None else outcome.ask(_lib.stream_of(state))
+        if prepared is not None:
+            kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told)
+        else:
+            kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
+                                     table_bytes=table_bytes, block_infos=bi, thread_infos=ti, encoded=self._encoded.data,
+                                     symbols=symbols, cache=cache, quant_mask=mask, eb=self.quant_scale_rel, min_ints=mn, scales=sc,
+                                     stream_bytes=state[8:9], result=state[:8], outcome=told)
         self._block_infos.used += sizes[0]
         self._thread_infos.used += sizes[1]
         self._min_ints.used += nb
@@ -572,6 +645,21 @@ class KVCompCtx:
         self._enc_pending += worst
         self.compressed_ctx_len += T
         self._unverified.append(_QueuedStore(T, keep, self._bookkeeping(), worst, lost_if_dropped, certain, codebook))
+        if outcome is not None:
+            self._probe = (outcome, len(self._unverified), outcome.stream)
+
+    def _prepare_encode(self, T: int, symbols: torch.Tensor):
+        """For a first store, while the quantizer runs: the buffers of the encode and the launch that needs no codebook."""
+        B, H, D = self.batch_size, self.head_num, self.head_dim
+        sizes = kvcomp_cuda.buffer_sizes(T, B * H * D, self.is_k, H, D)
+        bi = self._block_infos.reserve(sizes[0], (), torch.uint8, self.device)
+        ti = self._thread_infos.reserve(sizes[1], (), torch.uint8, self.device)
+        state = torch.empty(16, dtype=torch.int32, device=self.device)
+        prepared = kvcomp_cuda.encode_prepare(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, symbols=symbols,
+                                              block_infos=bi, thread_infos=ti, state=state)
+        self._state = state                                    # (cleared, on this stream)
+        self._ask_outcome()
+        return prepared
 
     def _first_chunk(self, blocked: torch.Tensor) -> torch.Tensor:
         """The first stored chunk: quantized, its codebook built from the symbols just written (kvcomp_encode.py:86-103; the
@@ -583,16 +671,22 @@ class KVCompCtx:
         gshape = mask_keepdim_shape(blocked.shape, self._mask)
         min_ints = self._min_ints.reserve(nb, gshape[1:], torch.int8, device)
         quant_scale = self._scales.reserve(nb, gshape[1:], torch.float16, device)
+        prepared = []
+
+        def meanwhile(symbols):
+            if self._state is None and self._encoded.used == 0:
+                prepared.extend((self._prepare_encode(T, symbols), kvcomp_cuda.codebook_room(device)))
         sym, book = kvcomp_cuda.quant_codebook(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale,
-                                               self._smoothed_symbols() if self.codebook_smoothing else 0)
+                                               self._smoothed_symbols() if self.codebook_smoothing else 0, meanwhile)
         self.waits += 1
-        enc, dec, lut = kvcomp_cuda.put_codebook(book, device)
+        enc, dec, lut = kvcomp_cuda.put_codebook(book, device, *prepared[1:])
         vectors = T * self.batch_size * self.head_num * self.head_dim // (self.head_dim if self.is_k else kvcomp_cuda.V_VEC_LEN)
         cannot_fail = book.max_code_bits <= 7
         small = T <= self.ASYNC_KEEP_BLOCKS * self.block_size
         queued = self.async_store and (cannot_fail or small)
         self._encode_direct(T, symbols=sym, tables=enc, table_bytes=enc.numel(), most_bytes=book.payload_bits // 8 + vectors + 1,
-                            keep=blocked.flatten(0, 1).clone() if queued and not cannot_fail else None, certain=cannot_fail, codebook=True)
+                            keep=blocked.flatten(0, 1).clone() if queued and not cannot_fail else None, certain=cannot_fail, codebook=True,
+                            prepared=prepared[0] if prepared else None)
         if queued:
             self._issue_probe()
         else:

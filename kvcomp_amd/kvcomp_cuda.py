@@ -17,7 +17,7 @@ Differences from the reference, all deliberate:
   * kernels run on torch's current stream rather than the legacy default stream.
 """
 import ctypes as C
-from typing import List, Tuple
+from typing import List, NamedTuple, Tuple
 
 import torch
 
@@ -139,9 +139,10 @@ def build_codebook_device(counts: torch.Tensor, tree_format: int = TREE_I8):
 
 
 def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: float, min_ints: torch.Tensor, scales: torch.Tensor,
-                   smoothed_symbols: int):
+                   smoothed_symbols: int, meanwhile=None):
     """kvc_quant_codebook on a device fp16 [NB, BS, B, H, D] tensor: (symbols uint8 of the same shape, _lib.Codebook).
-    min_ints (int8) and scales (fp16) receive the group parameters.  Waits for the symbol counts only."""
+    min_ints (int8) and scales (fp16) receive the group parameters.  Waits for the symbol counts only; `meanwhile`, if given, is
+    called with the symbol tensor once the quantizer is queued."""
     _require(blocked.is_cuda and blocked.dtype == torch.float16 and blocked.dim() == 5 and blocked.is_contiguous(),
              "a contiguous device float16 tensor of shape [NB, BS, B, H, D] is expected")
     L = _lib.lib()
@@ -150,21 +151,37 @@ def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: floa
     _require(scales.is_cuda and scales.dtype == torch.float16 and scales.numel() >= groups, "scales: fp16 device tensor of the group count")
     sym = torch.empty(blocked.shape, dtype=torch.uint8, device=blocked.device)
     book = _lib.Codebook()
+    stream = _lib.stream_of(blocked)
     with _lib.device_guard(blocked):
-        check(L.kvc_quant_codebook(_ptr(blocked), *blocked.shape, quant_mask, float(quant_scale_rel), _ptr(sym), _ptr(min_ints),
-                                   _ptr(scales), smoothed_symbols, C.byref(book), _stream(blocked)))
+        counted = C.c_void_p(0)
+        check(L.kvc_quant_counted(blocked.data_ptr(), *blocked.shape, quant_mask, float(quant_scale_rel), sym.data_ptr(), min_ints.data_ptr(),
+                                  scales.data_ptr(), C.byref(counted), stream))
+        try:
+            if meanwhile is not None:
+                meanwhile(sym)
+        finally:
+            rc = L.kvc_counted_codebook(counted, smoothed_symbols, C.byref(book), stream)
+        check(rc)
     return sym, book
 
 
-def put_codebook(book: "_lib.Codebook", device):
-    """(encode table, decode tree, decode tables) of a _lib.Codebook as device uint8 tensors, in stream order; nothing waits."""
+def codebook_room(device) -> torch.Tensor:
+    """Device memory for what put_codebook puts in place, whatever the codebook."""
+    return torch.empty(_lib.lib().kvc_lut_bytes() + 256 * 8 + 512 * 5, dtype=torch.uint8, device=device)
+
+
+def put_codebook(book: "_lib.Codebook", device, room: torch.Tensor = None):
+    """(encode table, decode tree, decode tables) of a _lib.Codebook as device uint8 tensors, in stream order; nothing waits.
+    They share one piece of memory: `room`, if codebook_room has been asked for it already."""
     L = _lib.lib()
-    enc_bytes, lut_bytes = book.encode_bytes, L.kvc_lut_bytes()
-    at = lut_bytes + (enc_bytes + 15) // 16 * 16         # one allocation, each part on a 16-byte boundary
-    held = torch.empty(at + book.decode_bytes, dtype=torch.uint8, device=device)
-    with _lib.device_guard(held):
-        check(L.kvc_put_codebook(C.addressof(book), held.data_ptr() + lut_bytes, held.data_ptr(), _lib.stream_of(held)))
-    return held[lut_bytes:lut_bytes + enc_bytes], held[at:], held[:lut_bytes]
+    if room is None:
+        room = codebook_room(device)
+    enc_bytes, lut_bytes, address = book.encode_bytes, L.kvc_lut_bytes(), room.data_ptr()
+    at = lut_bytes + (enc_bytes + 15) // 16 * 16         # each part on a 16-byte boundary
+    _require(room.numel() >= at + book.decode_bytes, "not enough room for the codebook")
+    with _lib.device_guard(room):
+        check(L.kvc_put_codebook(C.addressof(book), address + lut_bytes, address, _lib.stream_of(room)))
+    return room[lut_bytes:lut_bytes + enc_bytes], room[at:at + book.decode_bytes], room[:lut_bytes]
 
 
 def _entropy_encode(is_k, input, encode_code_book, block_infos, thread_infos, idx_offset, encoded_data,
@@ -237,11 +254,12 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
                  symbols: torch.Tensor = None, cache: torch.Tensor = None, quant_mask: int = 0, eb: float = 0.0,
                  min_ints: torch.Tensor = None, scales: torch.Tensor = None, table_stride: int = 0, rows_per_codebook: int = 0,
                  codebook_meta: torch.Tensor = None, base_global_offset: int = 0, stream_bytes: torch.Tensor = None,
-                 result: torch.Tensor = None):
+                 result: torch.Tensor = None, outcome=None):
     """kvc_encode_async: queue one encode (from `symbols`, or quantizing `cache` on the fly into min_ints / scales) with
     one table per `rows_per_codebook` tile rows, and return without waiting.  `result` (device int32[8], zeroed once)
     and `stream_bytes` (device int32[1]: payload bytes already in `encoded`, moved on by the call) stay on the device;
-    encode_result() reads them.  The output tensors are written from their first element on."""
+    encode_result() reads them.  The output tensors are written from their first element on.
+    outcome: (address of 16 words of pinned host memory, number), see kvc_encode_queue."""
     job = _lib.EncodeJob()
     job.is_k, job.quant_mask, job.eb = int(is_k), int(quant_mask), float(eb)
     _require((symbols is None) != (cache is None), "give either symbols or cache")
@@ -286,8 +304,51 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
         job.d_stream_bytes = stream_bytes.data_ptr()
     if result is not None:
         job.d_result = result.data_ptr()
+    address, number = (0, 0) if outcome is None else outcome
     with _lib.device_guard(encoded):
-        check(_lib.lib().kvc_encode_async(C.byref(job), _stream(encoded)))
+        check(_lib.lib().kvc_encode_queue(C.byref(job), 0, 0, address, number, _lib.stream_of(encoded)))
+
+
+class PreparedEncode(NamedTuple):
+    job: "_lib.EncodeJob"
+    scratch: torch.Tensor
+    done: int
+    sizes: tuple
+
+
+def encode_prepare(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens: int, symbols: torch.Tensor,
+                   block_infos: torch.Tensor, thread_infos: torch.Tensor, state: torch.Tensor):
+    """kvc_encode_prepare: what an encode from `symbols` can have done before its table is known.  `state` (device int32[16]):
+    its first eight words are the encode's `result`, word 8 its `stream_bytes`; they are cleared.  encode_prepared does the
+    rest, on the same stream."""
+    L = _lib.lib()
+    _dev_u8(symbols, "symbols")
+    sizes = buffer_sizes(tokens, batch * head_num * head_dim, is_k, head_num, head_dim)
+    _require(symbols.is_contiguous() and symbols.numel() == tokens * batch * head_num * head_dim, "symbols: wrong size")
+    for t, n, need in ((block_infos, "block_infos", sizes[0]), (thread_infos, "thread_infos", sizes[1])):
+        _dev_u8(t, n)
+        _require(t.numel() >= need, n + " buffer too small")
+    _require(state.is_cuda and state.dtype == torch.int32 and state.is_contiguous() and state.numel() >= 16, "state: device int32 [16]")
+    at = state.data_ptr()
+    job = _lib.EncodeJob(is_k=int(is_k), d_sym=symbols.data_ptr(), tokens=tokens, batch=batch, heads=head_num, head_dim=head_dim,
+                         d_block_infos=block_infos.data_ptr(), d_thread_infos=thread_infos.data_ptr(), d_result=at, d_stream_bytes=at + 32)
+    scratch = torch.empty(L.kvc_encode_scratch_bytes(), dtype=torch.uint8, device=symbols.device)
+    done = C.c_int(0)
+    with _lib.device_guard(symbols):
+        check(L.kvc_encode_prepare(C.byref(job), scratch.data_ptr(), scratch.numel(), C.byref(done), _lib.stream_of(symbols)))
+    return PreparedEncode(job, scratch, done.value, sizes)
+
+
+def encode_prepared(prepared: PreparedEncode, encode_table: torch.Tensor, encoded: torch.Tensor, outcome=None):
+    """What encode_prepare left to be done, now that the table and the payload buffer are there (once per preparation)."""
+    job, at = prepared.job, prepared.scratch.data_ptr()
+    for t, n in ((encode_table, "encode_table"), (encoded, "encoded")):
+        _dev_u8(t, n)
+    job.d_encode_tables, job.encode_table_bytes = encode_table.data_ptr(), encode_table.numel()
+    job.d_encoded, job.encoded_cap = encoded.data_ptr(), encoded.numel()
+    address, number = (0, 0) if outcome is None else outcome
+    with _lib.device_guard(encoded):
+        check(_lib.lib().kvc_encode_queue(C.byref(job), at, prepared.done, address, number, _lib.stream_of(encoded)))
 
 
 def encode_result(result: torch.Tensor, encoded_cap: int):
