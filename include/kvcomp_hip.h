@@ -239,13 +239,14 @@ int kvc_encode_async(const kvc_encode_job *job, void *stream);
  *   *d_stream_bytes are cleared.  d_scratch: kvc_encode_scratch_bytes() of device memory on a 16-byte boundary, in use until
  *   the encode has run.  *prepared receives what to pass on.
  * kvc_encode_queue: kvc_encode_async, continuing what was prepared on the same stream for the same tokens and outputs
- *   (prepared = 0: nothing was; d_scratch is not used then).  h_outcome, if not NULL: 16 words of pinned host memory that
+ *   (prepared = 0: nothing was; d_scratch is not used then).  longest_code: bits of the longest code in the (one) encode
+ *   table, 0 if not known; symbols with longer codes are errors.  h_outcome, if not NULL: 16 words of pinned host memory that
  *   receive d_result's eight words, *d_stream_bytes and, last, outcome_number (word 9), as the call ends on the device.
  * kvc_wait_outcome: waits until outcome_number has arrived in such words. */
 int64_t kvc_encode_scratch_bytes(void);
 int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream);
-int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, uint32_t *h_outcome, uint32_t outcome_number,
-                     void *stream);
+int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,
+                     uint32_t outcome_number, void *stream);
 int kvc_wait_outcome(const uint32_t *h_outcome, uint32_t outcome_number);
 int kvc_encode_result(const uint32_t *d_result, int64_t encoded_cap, int64_t *h_total_bytes, int64_t *h_max_tile_bytes,
                       int64_t *h_max_stream_bytes, int64_t *h_tiles, void *stream);

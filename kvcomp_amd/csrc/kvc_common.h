@@ -205,14 +205,22 @@ __device__ __forceinline__ const T &kvc_kernarg_again()
     return *(const T *)p;
 }
 
-// inclusive prefix sum over the 64 lanes of a wave
-__device__ __forceinline__ uint32_t kvc_wave_inclusive_scan(uint32_t v, int lane)
+// Sum over the 64 lanes, and inclusive prefix sum, the same way (every lane active).  The prefix sum adds lanes 1, 2, 4 and 8 to
+// the left within rows of 16, then the rows' totals; as six shuffles through the LDS it took ten times as long.
+__device__ __forceinline__ uint32_t kvc_wave_sum_dpp_u32(uint32_t v)
 {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        uint32_t t = __shfl_up(v, off, 64);
-        if (lane >= off) v += t;
-    }
+    KVC_DPP_REDUCE("v_add_u32_dpp", v);
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+__device__ __forceinline__ uint32_t kvc_wave_inclusive_scan(uint32_t v)
+{
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);      // row_shr:1
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);     // row_bcast:15 into rows 1 and 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);     // row_bcast:31 into rows 2 and 3
     return v;
 }
 #endif

@@ -25,6 +25,8 @@
 #include "kvc_common.h"
 #include "kvc_quant_math.h"
 
+#include <type_traits>
+
 struct KvcEncodeArgs {
     const uint8_t *sym;        // [tokens, stride]
     int64_t stride;
@@ -100,37 +102,40 @@ __device__ __forceinline__ void kvc_encode_init(const KvcEncodeArgs &a)
 }
 __global__ void __launch_bounds__(KVC_WAVE) kvc_encode_init_kernel(KvcEncodeArgs a) { kvc_encode_init(a); }
 
-// Hands the call's outcome to the caller's device words (see kvc_encode_job): one thread, behind everything else.
-__device__ __forceinline__ void kvc_encode_publish(const KvcEncodeArgs &a)
+// Hands the call's outcome to the caller's words (see kvc_encode_job), behind everything else: by the first ten threads of a
+// workgroup, a word each -- one after the other, the round trips to the host's memory took 4 us.
+__device__ __forceinline__ void kvc_encode_publish(const KvcEncodeArgs &a, int tid)
 {
-    const uint32_t total = a.status[0], err = a.status[1];
-    if (a.result) {
-        a.result[0] = total;
-        a.result[1] |= err;
-        if (a.status[2] > a.result[2]) a.result[2] = a.status[2];
-        if (a.status[3] > a.result[3]) a.result[3] = a.status[3];
-        a.result[4] += (uint32_t)a.tiles;
-        a.result[5] = a.status[KVC_ENC_ST_BASE];
-        if (a.status[6] > a.result[6]) a.result[6] = a.status[6];
+    if (tid >= 10) return;                                     // (word 9 of the outcome is the call's number)
+    const uint32_t total = a.status[0], err = a.status[1], first = a.status[KVC_ENC_ST_BASE];
+    uint32_t word = 0;
+    if (a.result && tid < 8) {
+        const uint32_t old = a.result[tid], mine = tid == 2 || tid == 3 || tid == 6 ? a.status[tid] : 0u;
+        word = tid == 0 ? total : tid == 1 ? old | err : tid == 4 ? old + (uint32_t)a.tiles : tid == 5 ? first : old > mine ? old : mine;
+        a.result[tid] = word;
     }
-    if (a.stream_bytes && !err) *a.stream_bytes = a.status[KVC_ENC_ST_BASE] - a.base_global_offset + total;
+    if (a.stream_bytes && tid == 8) {
+        word = err ? *a.stream_bytes : first - a.base_global_offset + total;
+        *a.stream_bytes = word;
+    }
     if (a.outcome) {
         // the host looks at these words without asking the runtime: system-scope stores, then the call's number with release
         // order (as kvc_counts_to_host_kernel); a copy and an event behind the call cost 8 us of host time and a launch
-        for (int i = 0; i < 8; i++) __hip_atomic_store(&a.outcome[i], a.result[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(&a.outcome[8], *a.stream_bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(&a.outcome[9], a.outcome_number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (tid < 9) __hip_atomic_store(&a.outcome[tid], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __threadfence_system();
+        __builtin_amdgcn_wave_barrier();
+        if (tid == 9) __hip_atomic_store(&a.outcome[9], a.outcome_number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
-__global__ void kvc_encode_publish_kernel(KvcEncodeArgs a) { kvc_encode_publish(a); }
+__global__ void __launch_bounds__(KVC_WAVE) kvc_encode_publish_kernel(KvcEncodeArgs a) { kvc_encode_publish(a, threadIdx.x); }
 
 // The 128 (or fewer) symbols of this lane's vector, 4 per register in stream order.
 //   K: token 64*row + lane, channels vec_len*col ..          (kernels.cu:439-444: one contiguous run)
 //   V: channel 64*col + lane, tokens 128*row ..              (kernels.cu:514-519: one byte per token row)
 __device__ __forceinline__ void kvc_load_vector(const KvcEncodeArgs &a, int64_t tile, int lane, uint32_t v[32])
 {
-    const int64_t row = tile / a.cols, col = tile - row * a.cols;
+    const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
     if (a.is_k) {
         const uint8_t *p = a.sym + (row * KVC_WAVE + lane) * a.stride + col * a.vec_len;
         const int nd = a.vec_len >> 2;
@@ -166,6 +171,17 @@ constexpr int KVC_STAGE_K_BYTES = 32 * (128 + 4);       // 32 tokens of up to 12
 constexpr int KVC_STAGE_VSYM_BYTES = 64 * (64 + 4);     // 64 channels of 64 tokens
 constexpr int KVC_STAGE_VF16_BYTES = 64 * (32 + 4);     // 64 channels of 32 tokens
 
+__device__ __forceinline__ void kvc_transpose_4x4(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3, uint32_t (&c)[4])
+{
+    // {w0.b0 w1.b0 w0.b1 w1.b1}, {w0.b2 w1.b2 w0.b3 w1.b3}, the same of w2 and w3; then a channel's four tokens
+    const uint32_t a_lo = __builtin_amdgcn_perm(w1, w0, 0x05010400u), a_hi = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
+    const uint32_t b_lo = __builtin_amdgcn_perm(w3, w2, 0x05010400u), b_hi = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
+    c[0] = __builtin_amdgcn_perm(b_lo, a_lo, 0x05040100u);
+    c[1] = __builtin_amdgcn_perm(b_lo, a_lo, 0x07060302u);
+    c[2] = __builtin_amdgcn_perm(b_hi, a_hi, 0x05040100u);
+    c[3] = __builtin_amdgcn_perm(b_hi, a_hi, 0x07060302u);
+}
+
 // The same vectors of a V tile fetched four channels per lane: 16 lanes cover a token's 64 symbols, a load instruction
 // four tokens (the byte-per-token-row loads above move 64 bytes per instruction, 128 instructions per tile; these move
 // 256 bytes, 32 instructions), four tokens of four channels are transposed in registers and go to the staging area
@@ -174,7 +190,7 @@ constexpr int KVC_STAGE_VF16_BYTES = 64 * (32 + 4);     // 64 channels of 32 tok
 __device__ __forceinline__ void kvc_load_vector_v_tile(const KvcEncodeArgs &a, int64_t tile, int lane, uint8_t *s_stage, uint32_t v[32])
 {
     constexpr int RS = 64 + 4;
-    const int64_t row = tile / a.cols, col = tile - row * a.cols;
+    const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
     const int pr = lane & 15, sub = lane >> 4;
     const uint8_t *p = a.sym + (row * KVC_V_TOKENS + 4 * sub) * a.stride + col * KVC_WAVE + 4 * pr;
     uint32_t w[32];
@@ -186,17 +202,11 @@ __device__ __forceinline__ void kvc_load_vector_v_tile(const KvcEncodeArgs &a, i
     for (int h = 0; h < 2; h++) {
 #pragma unroll
         for (int jj = 4 * h; jj < 4 * h + 4; jj++) {
-            const uint32_t w0 = w[4 * jj], w1 = w[4 * jj + 1], w2 = w[4 * jj + 2], w3 = w[4 * jj + 3];
-            // {w0.b0 w1.b0 w0.b1 w1.b1}, {w0.b2 w1.b2 w0.b3 w1.b3}, the same of w2 and w3; then a channel's four tokens
-            const uint32_t a_lo = __builtin_amdgcn_perm(w1, w0, 0x05010400u), a_hi = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
-            const uint32_t b_lo = __builtin_amdgcn_perm(w3, w2, 0x05010400u), b_hi = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
-            const uint32_t c0 = __builtin_amdgcn_perm(b_lo, a_lo, 0x05040100u), c1 = __builtin_amdgcn_perm(b_lo, a_lo, 0x07060302u);
-            const uint32_t c2 = __builtin_amdgcn_perm(b_hi, a_hi, 0x05040100u), c3 = __builtin_amdgcn_perm(b_hi, a_hi, 0x07060302u);
+            uint32_t c[4];
+            kvc_transpose_4x4(w[4 * jj], w[4 * jj + 1], w[4 * jj + 2], w[4 * jj + 3], c);
             uint8_t *dst = s_stage + (4 * pr) * RS + 16 * (jj - 4 * h) + 4 * sub;
-            *reinterpret_cast<uint32_t *>(dst) = c0;
-            *reinterpret_cast<uint32_t *>(dst + RS) = c1;
-            *reinterpret_cast<uint32_t *>(dst + 2 * RS) = c2;
-            *reinterpret_cast<uint32_t *>(dst + 3 * RS) = c3;
+#pragma unroll
+            for (int k = 0; k < 4; k++) *reinterpret_cast<uint32_t *>(dst + k * RS) = c[k];
         }
         kvc_wave_lds_sync();
 #pragma unroll
@@ -222,7 +232,7 @@ __device__ __forceinline__ void kvc_read_k_rows(const uint8_t *s_stage, int RS, 
 // vec_len <= 128.
 __device__ __forceinline__ void kvc_load_vector_k_tile(const KvcEncodeArgs &a, int64_t tile, int lane, uint8_t *s_stage, uint32_t (&v)[32])
 {
-    const int64_t row = tile / a.cols, col = tile - row * a.cols;
+    const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
     const int nd = a.vec_len >> 2, RS = a.vec_len + 4;
     const int per = KVC_WAVE / nd;                                     // tokens per load instruction (at least 2)
     const int r = lane / nd, cw = lane - r * nd;
@@ -257,6 +267,98 @@ __device__ __forceinline__ void kvc_load_vector_k_tile(const KvcEncodeArgs &a, i
     }
 }
 
+// The same two hand-overs with sixteen symbols per load, for 16-byte aligned symbols and rows: eight loads per lane and tile,
+// few enough that a run's second tile can be on its way while the first is counted and packed.
+// K: vectors of 4 ND symbols; PIECES lanes cover a token's run, PER tokens a load instruction.
+typedef uint32_t kvc_u32x4 __attribute__((ext_vector_type(4)));
+template <int ND>
+__device__ __forceinline__ void kvc_load_k_wide(const KvcEncodeArgs &a, int64_t tile, int lane, kvc_u32x4 (&q)[8])
+{
+    constexpr int PIECES = ND / 4, PER = KVC_WAVE / PIECES, LOADS = (KVC_WAVE + PER - 1) / PER;
+    const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
+    const int r = lane / PIECES, piece = lane - r * PIECES;
+    const uint8_t *p = a.sym + (row * KVC_WAVE + r) * a.stride + col * (4 * ND) + 16 * piece;
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) {
+        // (lanes without a piece of a row load what another lane loads)
+        const bool mine = PER * PIECES == KVC_WAVE || (r < PER && r + PER * i < KVC_WAVE);
+        q[i] = *reinterpret_cast<const kvc_u32x4 *>(p + (mine ? (int64_t)(PER * i) * a.stride : -(int64_t)r * a.stride));
+    }
+}
+
+// Rows lie one behind the other in the area (at most four load instructions' worth, 4 KB), so that rows of an even number of
+// pieces start on the same few banks: their pieces are permuted by the row's number, which leaves the reads (sixteen lanes
+// take a piece of a row each at a time) and the writes without conflicts.
+template <int ND>
+__device__ __forceinline__ void kvc_stage_k_wide(int lane, uint8_t *s_stage, const kvc_u32x4 (&q)[8], uint32_t (&v)[32])
+{
+    constexpr int PIECES = ND / 4, PER = KVC_WAVE / PIECES, EVEN = PIECES & -PIECES, MASK = EVEN - 1, SHIFT = EVEN == 8 ? 1 : EVEN == 4 ? 2 : 3;
+    static_assert(4 * PER * ND * 4 <= KVC_STAGE_VSYM_BYTES, "four load instructions fit the area");
+    const int r = lane / PIECES, piece = lane - r * PIECES;
+    kvc_u32x4 *area = reinterpret_cast<kvc_u32x4 *>(s_stage);
+#pragma unroll
+    for (int h = 0; h < (4 * PER < KVC_WAVE ? 2 : 1); h++) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int at = r + PER * i;                    // row of the area
+            if (PER * PIECES == KVC_WAVE || (r < PER && at + 4 * PER * h < KVC_WAVE)) area[at * PIECES + (piece ^ ((at >> SHIFT) & MASK))] = q[4 * h + i];
+        }
+        kvc_wave_lds_sync();
+        const int mine = lane - 4 * PER * h;               // this lane's row of the area, if it is in this part
+        if (mine >= 0 && mine < 4 * PER) {
+            const kvc_u32x4 *rowp = area + mine * PIECES;
+            const int x = (mine >> SHIFT) & MASK;
+#pragma unroll
+            for (int j = 0; j < PIECES; j++) {
+                const kvc_u32x4 w = rowp[j ^ x];
+                v[4 * j] = w.x;
+                v[4 * j + 1] = w.y;
+                v[4 * j + 2] = w.z;
+                v[4 * j + 3] = w.w;
+            }
+        }
+        kvc_wave_lds_sync();
+    }
+}
+
+// V: four lanes cover a token's 64 symbols, a lane has eight consecutive tokens of sixteen channels; four tokens of four
+// channels are transposed in registers.  The area holds a quarter of the tile at a time (tokens 0 .. 3 of every eight of the
+// first 64, then of the others, then 4 .. 7), as [channel][8 words]: the less it takes, the more images can wait beside it.
+__device__ __forceinline__ void kvc_load_v_wide(const KvcEncodeArgs &a, int64_t tile, int lane, kvc_u32x4 (&q)[8])
+{
+    const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
+    const uint8_t *p = a.sym + (row * KVC_V_TOKENS + 8 * (lane >> 2)) * a.stride + col * KVC_WAVE + 16 * (lane & 3);
+#pragma unroll
+    for (int i = 0; i < 8; i++) q[i] = *reinterpret_cast<const kvc_u32x4 *>(p + (int64_t)i * a.stride);
+}
+
+__device__ __forceinline__ void kvc_stage_v_wide(int lane, uint8_t *s_stage, const kvc_u32x4 (&q)[8], uint32_t (&v)[32])
+{
+    constexpr int RS = 32 + 4;                             // bytes per channel: reads and writes touch every bank once
+    static_assert(64 * RS <= KVC_STAGE_VF16_BYTES, "a quarter of the tile fits the area");
+    uint8_t *dst = s_stage + 16 * (lane & 3) * RS + 4 * ((lane >> 2) & 7);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const kvc_u32x4 t0 = q[4 * h], t1 = q[4 * h + 1], t2 = q[4 * h + 2], t3 = q[4 * h + 3];
+        uint32_t c[4][4];
+        kvc_transpose_4x4(t0.x, t1.x, t2.x, t3.x, c[0]);
+        kvc_transpose_4x4(t0.y, t1.y, t2.y, t3.y, c[1]);
+        kvc_transpose_4x4(t0.z, t1.z, t2.z, t3.z, c[2]);
+        kvc_transpose_4x4(t0.w, t1.w, t2.w, t3.w, c[3]);
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            if (lane >> 5 == g) {
+#pragma unroll
+                for (int k = 0; k < 16; k++) *reinterpret_cast<uint32_t *>(dst + k * RS) = c[k >> 2][k & 3];
+            }
+            kvc_wave_lds_sync();
+#pragma unroll
+            for (int j = 0; j < 8; j++) v[16 * g + 2 * j + h] = *reinterpret_cast<const uint32_t *>(s_stage + lane * RS + 4 * j);
+            kvc_wave_lds_sync();
+        }
+    }
+}
+
 // What the count step of one tile finds out (every field wave-uniform except `start`).
 struct KvcTileCount {
     uint32_t start;      // first byte of this lane's stream inside the tile payload
@@ -283,7 +385,7 @@ __device__ __forceinline__ KvcTileCount kvc_count_vectors(const KvcEncodeArgs &a
         }
     }
     const uint32_t bytes = (bits + 7u) >> 3;
-    const uint32_t end = kvc_wave_inclusive_scan(bytes, lane);
+    const uint32_t end = kvc_wave_inclusive_scan(bytes);
     a.thread_infos[tile * KVC_WAVE + lane] = (uint16_t)((end << 3) + (bytes << 3) - bits);
     KvcTileCount c;
     c.start = end - bytes;
@@ -353,7 +455,7 @@ __global__ void __launch_bounds__(1024) kvc_encode_chunk_sum_kernel(KvcEncodeArg
     const int64_t tile = (int64_t)blockIdx.x * 1024 + tid;
     uint32_t bn = 0;
     if (tile < a.tiles) bn = reinterpret_cast<const uint32_t *>(a.block_infos + 8 * tile)[1] & 0xffffu;
-    const uint32_t incl = kvc_wave_inclusive_scan(bn, lane);
+    const uint32_t incl = kvc_wave_inclusive_scan(bn);
     if (lane == KVC_WAVE - 1) s_wave[wave] = incl;
     __syncthreads();
     if (tid == 0) {
@@ -379,8 +481,8 @@ __global__ void __launch_bounds__(1024) kvc_encode_scan_kernel(KvcEncodeArgs a)
     const int64_t tile = (int64_t)blockIdx.x * 1024 + tid;
     uint32_t bn = 0;
     if (tile < a.tiles) bn = reinterpret_cast<const uint32_t *>(a.block_infos + 8 * tile)[1] & 0xffffu;
-    const uint32_t incl = kvc_wave_inclusive_scan(bn, lane);
-    const uint32_t part_w = kvc_wave_inclusive_scan(part, lane);
+    const uint32_t incl = kvc_wave_inclusive_scan(bn);
+    const uint32_t part_w = kvc_wave_inclusive_scan(part);
     uint32_t mx = bn;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -401,7 +503,7 @@ __global__ void __launch_bounds__(1024) kvc_encode_scan_kernel(KvcEncodeArgs a)
     if (tile < a.tiles) reinterpret_cast<uint32_t *>(a.block_infos + 8 * tile)[0] = before + incl - bn;
     if (blockIdx.x == 0) {
         // the grand total, by the first workgroup
-        const uint32_t all_w = kvc_wave_inclusive_scan(all, lane);
+        const uint32_t all_w = kvc_wave_inclusive_scan(all);
         __syncthreads();
         if (lane == KVC_WAVE - 1) s_before[wave] = all_w;
         __syncthreads();
@@ -529,22 +631,34 @@ __device__ __forceinline__ void kvc_write_image(const KvcEncodeArgs &a, const Kv
 }
 
 // The same for an image that was packed from its first word on, while the payload starts p.head bytes into an
-// aligned word of the destination: every output word is put together from two image words.
+// aligned word of the destination: every output word is put together from two image words, four words of a lane at a time.
 __device__ __forceinline__ void kvc_write_image_shifted(const KvcEncodeArgs &a, const KvcEmitPlace &p, int lane, const uint32_t *image)
 {
-    uint8_t *dst = a.encoded + p.off - p.head;                 // 4-byte aligned
+    uint32_t *dst = reinterpret_cast<uint32_t *>(a.encoded + p.off - p.head);
     const uint32_t lo = p.head, hi = p.head + p.bn;            // valid byte range of the output words
-    const uint32_t nwords = (hi + 3u) >> 2;
     const uint32_t shift = 8u * (4u - p.head);                 // 32, 24, 16, 8
-    for (uint32_t f = lane; f < nwords; f += KVC_WAVE) {
-        const uint32_t cur = f < (uint32_t)KVC_IMAGE_WORDS ? image[f] : 0u, prev = f ? image[f - 1] : 0u;
-        const uint32_t b0 = 4u * f, word = (uint32_t)((((uint64_t)cur << 32) | prev) >> shift);
-        if (b0 >= lo && b0 + 4u <= hi) {
-            reinterpret_cast<uint32_t *>(dst)[f] = word;
-        } else {
+    const uint32_t first = lo ? 1u : 0u, end = hi >> 2;        // whole words
+    for (uint32_t f0 = lane; f0 < end; f0 += 4 * KVC_WAVE) {
+        uint32_t word[4];
 #pragma unroll
-            for (uint32_t k = 0; k < 4; k++)
-                if (b0 + k >= lo && b0 + k < hi) dst[b0 + k] = (uint8_t)(word >> (8u * k));
+        for (uint32_t k = 0; k < 4; k++) {
+            const uint32_t f = f0 + k * KVC_WAVE < end ? f0 + k * KVC_WAVE : f0;
+            const uint32_t cur = image[f], prev = image[f ? f - 1 : 0];
+            word[k] = lo ? (uint32_t)((((uint64_t)cur << 32) | prev) >> shift) : cur;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++) {
+            const uint32_t f = f0 + k * KVC_WAVE;
+            if (f >= first && f < end) dst[f] = word[k];
+        }
+    }
+    // the bytes at the ragged ends: of word 0 by lanes 0 .. 3, of the last word by lanes 4 .. 7
+    if (lane < 8) {
+        const uint32_t f = lane < 4 ? 0u : end, b = 4u * f + (lane & 3);
+        const bool ragged = lane < 4 ? lo != 0u : (end != 0u || lo == 0u) && (hi & 3u) != 0u;
+        if (ragged && b >= lo && b < hi) {
+            const uint32_t at = b - lo;                        // byte of the payload: image word at / 4
+            reinterpret_cast<uint8_t *>(dst)[b] = (uint8_t)(image[at >> 2] >> (8u * (at & 3u)));
         }
     }
 }
@@ -900,13 +1014,6 @@ __device__ __forceinline__ uint64_t *kvc_group_words(const KvcEncodeArgs &a)
 __device__ __forceinline__ uint64_t kvc_status_load(const uint64_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void kvc_status_store(uint64_t *p, uint64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-__device__ __forceinline__ uint32_t kvc_wave_sum_u32(uint32_t v)
-{
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, 64);
-    return v;
-}
-
 // First launch of a one-pass call: what kvc_encode_init_kernel does, by the first workgroup, and the marks.
 __global__ void __launch_bounds__(KVC_WG) kvc_encode_mark_kernel(KvcEncodeArgs a)
 {
@@ -953,7 +1060,7 @@ __device__ __forceinline__ uint32_t kvc_look_back_in_group(const KvcEncodeArgs &
     uint64_t w = first_look;
     while (r > 0) {
         if (!__any((uint32_t)(w >> 48) == KVC_BI_NOT_READY)) {
-            in_group = kvc_wave_sum_u32(lane < r ? (uint32_t)(w >> 32) & 0xffffu : 0u);
+            in_group = kvc_wave_sum_dpp_u32(lane < r ? (uint32_t)(w >> 32) & 0xffffu : 0u);
             break;
         }
         if (++*polls > a.max_polls) break;
@@ -980,7 +1087,7 @@ __device__ __forceinline__ uint32_t kvc_look_back_groups(const KvcEncodeArgs &a,
         const uint64_t not_ready = __ballot(state == KVC_BI_NOT_READY), known = __ballot(state == 0u);
         const int first_nr = not_ready ? __builtin_ctzll(not_ready) : 64, first_kn = known ? __builtin_ctzll(known) : 64;
         const int stop = first_kn < first_nr ? first_kn + 1 : first_nr;     // lanes below it count: sizes, then maybe an end
-        before += kvc_wave_sum_u32(lane < stop ? bytes : 0u);
+        before += kvc_wave_sum_dpp_u32(lane < stop ? bytes : 0u);
         if (first_kn < first_nr) break;                    // a group whose end is known closes the sum
         j -= stop;
         if (first_nr < 64) {
@@ -1017,17 +1124,19 @@ __device__ __forceinline__ void kvc_load_code_table_marked(const KvcEncodeArgs &
 // is staged and counted; the second tile's image goes behind the first one's when both fit (it may then run into the
 // staging area, which is free by then), and otherwise the first tile is placed and written out before the second is
 // packed -- with both sizes published long before, so that nobody waits for this wave in the meantime.
+constexpr int KVC_ONCE_IMAGE_BYTES = (KVC_MAX_TILE_BYTES + 3 + 16) / 16 * 16;   // the largest image, see kvc_once_image_words
 constexpr int KVC_ONCE_WAVE_BYTES = 12560;               // three workgroups of four waves per compute unit (160 KB)
 constexpr int KVC_ONCE_SMALL_WAVE_BYTES = 9696;          // four; symbols in, tiles known to be small on average (see the launcher)
 constexpr int kvc_once_par_bytes(int front) { return front == 2 ? 4 * KVC_V_TOKENS * 4 : 0; }
 constexpr int kvc_once_stage_bytes(int front) { return front == 1 ? KVC_STAGE_K_BYTES : front == 2 ? KVC_STAGE_VF16_BYTES : KVC_STAGE_VSYM_BYTES; }
 constexpr int kvc_once_area_bytes(int front) { return KVC_ONCE_WAVE_BYTES - kvc_once_par_bytes(front); }
-static_assert(KVC_ONCE_SMALL_WAVE_BYTES >= KVC_IMAGE_WORDS * 4 && KVC_ONCE_SMALL_WAVE_BYTES % 16 == 0, "an area holds any one image");
+static_assert(KVC_ONCE_SMALL_WAVE_BYTES >= KVC_ONCE_IMAGE_BYTES && KVC_ONCE_SMALL_WAVE_BYTES % 16 == 0, "an area holds any one image");
 static_assert(KVC_STAGE_VSYM_BYTES >= KVC_STAGE_K_BYTES, "symbols in: the staging area serves K and V tiles");
-static_assert(kvc_once_area_bytes(0) - kvc_once_stage_bytes(0) >= KVC_IMAGE_WORDS * 4 &&
-              kvc_once_area_bytes(1) - kvc_once_stage_bytes(1) >= KVC_IMAGE_WORDS * 4 &&
-              kvc_once_area_bytes(2) - kvc_once_stage_bytes(2) >= KVC_IMAGE_WORDS * 4, "the largest payload must leave the staging area free");
-__device__ __forceinline__ uint32_t kvc_once_image_words(uint32_t bn) { return (bn + 3u) / 4u + 1u; }
+static_assert(kvc_once_area_bytes(0) - kvc_once_stage_bytes(0) >= KVC_ONCE_IMAGE_BYTES &&
+              kvc_once_area_bytes(1) - kvc_once_stage_bytes(1) >= KVC_ONCE_IMAGE_BYTES &&
+              kvc_once_area_bytes(2) - kvc_once_stage_bytes(2) >= KVC_ONCE_IMAGE_BYTES, "the largest payload must leave the staging area free");
+// (whole 16-byte pieces, which the symbols kernel clears one per lane at a time)
+__device__ __forceinline__ uint32_t kvc_once_image_words(uint32_t bn) { return ((bn + 3u) / 4u + 4u) & ~3u; }
 
 // A tile whose payload is packed but not yet placed; the words its look-back reads were asked for when its size was
 // published.
@@ -1183,7 +1292,7 @@ __global__ void __launch_bounds__(KVC_WG, 3) kvc_encode_once_kernel(KvcStoreArgs
         const bool bad = bits >= KVC_NO_CODE_LEN;          // a symbol without a code: the lane emits nothing
         if (bad) bits = 0;
         const uint32_t bytes = (bits + 7u) >> 3;
-        const uint32_t end = kvc_wave_inclusive_scan(bytes, lane);
+        const uint32_t end = kvc_wave_inclusive_scan(bytes);
         a.e.thread_infos[tile * KVC_WAVE + lane] = (uint16_t)((end << 3) + (bytes << 3) - bits);
         const uint32_t start = end - bytes;
         const uint32_t tile_bytes = (uint32_t)__builtin_amdgcn_readlane((int)end, KVC_WAVE - 1);
@@ -1291,6 +1400,261 @@ __global__ void __launch_bounds__(KVC_WG, 3) kvc_encode_once_kernel(KvcStoreArgs
     }
 }
 
+// ---- one pass from symbols: vectors of 64, 96 or 128 of them, one codebook of short codes, 16-byte aligned symbols and rows --
+//
+// What kvc_encode_once_kernel<0> does, in fewer instructions and with less waiting inside a tile.  That kernel does not know
+// the vector's length when it is compiled: a branch per register of symbols made the wave wait for the LDS 32 times per tile
+// (13.4 vector instructions per symbol, vector ALUs 44 % busy, 58 % of the wave cycles spent waiting).  Here the length is
+// known, symbols come sixteen per load (K: 727 -> 540 MB fetched for 402 MB of symbols with head size 96), alphabets of at
+// most 16 symbols are looked up two at a time with one instruction per address, what is the same for a wave is kept in scalar
+// registers, and codes of more than 8 bits are left to the other kernel, whose loops for them took most of the registers: 7.5
+// (K) and 6 (V) vector instructions per symbol.  From symbols, us: K 8 x 32 heads x 128 x 4096 tokens 111 -> 75, V 104 ->
+// 71; 4 x 32 x 96 x 32 768 tokens 338 -> 257 and 242 -> 182.  What is left is the wait for the tiles before a wave's own (14
+// and 13 of the 75 and 71 us, 65 of 257: measured with made-up offsets) and the tickets (4).  Sixteen waves per compute unit
+// are best: 20 of them (five per SIMD, for which the registers would do) take 293 instead of 257 us, and a second tile on
+// its way while the first is packed gains nothing for the registers it takes.
+// A few registers of symbols at a time, without a branch inside, so that their look-ups are in flight together.  The symbols of
+// a register are looked up and their codes joined, at most 32 bits; gl receives the joined lengths, four to a register.
+// PAIRS: the table has an entry per two symbols below 16, first symbol in the index's upper half.  Returns the vector's bits.
+static_assert(255 * (128 + 8) + 8 <= (KVC_WAVES_PER_WG * KVC_ONCE_SMALL_WAVE_BYTES) + 2048, "look-ups of pairs of any bytes stay inside the LDS");
+typedef __attribute__((address_space(3))) uint64_t kvc_lds_u64;
+template <bool PAIRS, int ND, int STEP>
+__device__ __forceinline__ uint32_t kvc_join_vector(const uint2 *s_table, uint32_t (&v)[32], uint32_t (&gl)[8])
+{
+    uint32_t bits = 0, over = 0;
+    uint32_t table_at = (uint32_t)(uintptr_t)(const kvc_lds_u64 *)s_table;
+#pragma unroll
+    for (int c = 0; c < ND / STEP; c++) {
+        // (opaque, and the barrier below: or the addresses of all look-ups are worked out, and kept, before the first one)
+        asm volatile("" : "+v"(table_at));
+#pragma unroll
+        for (int j = STEP * c; j < STEP * (c + 1); j++) {
+            const uint32_t w = v[j];
+            uint32_t x, len;
+            if constexpr (PAIRS) {
+                over |= w;
+                // The byte address of a pair's entry in one instruction: 8 * (16 * first + second), behind where the table starts.
+                // (Symbols from 16 on reach up to 34 KB further, which is still the workgroup's own memory.)
+                const uint64_t e0 = *(const kvc_lds_u64 *)(uintptr_t)__builtin_amdgcn_udot4(w, 0x00000880u, table_at, false);
+                const uint64_t e1 = *(const kvc_lds_u64 *)(uintptr_t)__builtin_amdgcn_udot4(w, 0x08800000u, table_at, false);
+                const uint32_t second = (uint32_t)(e1 >> 32);
+                len = (uint32_t)(e0 >> 32) + second;
+                x = ((uint32_t)e0 << (second & 31u)) | (uint32_t)e1;
+            } else {
+                const uint2 e0 = s_table[w & 0xffu], e1 = s_table[(w >> 8) & 0xffu];
+                const uint2 e2 = s_table[(w >> 16) & 0xffu], e3 = s_table[w >> 24];
+                len = e0.y + e1.y + e2.y + e3.y;
+                // (the marked length of a symbol without a code shifts by nothing)
+                x = ((((e0.x << (e1.y & 31u)) | e1.x) << (e2.y & 31u) | e2.x) << (e3.y & 31u)) | e3.x;
+            }
+            v[j] = x;
+            bits += len;
+            gl[j >> 2] |= len << (8 * (j & 3));            // (a marked length spoils the others': the lane then emits nothing)
+        }
+        __builtin_amdgcn_sched_barrier(0);                 // (more look-ups in flight cost registers that the wave does not have)
+    }
+    return PAIRS && (over & 0xf0f0f0f0u) ? 0x4000u : bits; // (a larger symbol is one without a code: KVC_NO_CODE_LEN)
+}
+
+// A lane's bits on their way to the image: `cur` is the word being filled, `left` the bits it still takes, negated.
+struct KvcPacker {
+    uint32_t cur;
+    int left;
+    uint32_t *at;
+    __device__ __forceinline__ KvcPacker(uint32_t start, uint32_t *image) : cur(0), left((int)((start * 8u) & 31u) - 32), at(image + (start >> 2)) {}
+    __device__ __forceinline__ void push(uint32_t bits, uint32_t len)        // len 0 .. 32 (0: bits are 0)
+    {
+        const uint32_t x = bits << ((0u - len) & 31u);     // from the word's upper end down
+        cur |= x >> (left & 31);
+        const int now = left + (int)len;
+        if (now >= 0) {
+            atomicOr(at++, kvc_bswap(cur));
+            cur = __builtin_amdgcn_alignbit(x, 0u, (uint32_t)left);
+            left = now - 32;
+        } else {
+            left = now;
+        }
+    }
+    __device__ __forceinline__ void finish()
+    {
+        if (left != -32) atomicOr(at, kvc_bswap(cur));
+    }
+};
+
+// The joined codes to the image, from payload byte `start` on.  TWO: the codes of two registers are joined where those of every
+// lane fit a word together.
+template <int ND, bool TWO>
+__device__ __forceinline__ void kvc_pack_joined(uint32_t start, const uint32_t (&v)[32], const uint32_t (&gl)[8], uint32_t *image)
+{
+    KvcPacker p(start, image);
+#pragma unroll
+    for (int j = 0; j < ND; j += 2) {
+        const uint32_t l0 = (gl[j >> 2] >> (8 * (j & 3))) & 0xffu, l1 = (gl[j >> 2] >> (8 * (j & 3) + 8)) & 0xffu;
+        if (TWO && !__any(l0 + l1 > 32u)) {
+            p.push((v[j] << (l1 & 31u)) | v[j + 1], l0 + l1);
+        } else {
+            p.push(v[j], l0);
+            p.push(v[j + 1], l1);
+        }
+    }
+    p.finish();
+}
+
+// The workgroup's copy of the encode table: an entry without a code, or with one of more than 8 bits (which the launcher has
+// been told do not occur), gets the length KVC_NO_CODE_LEN.  pairs (at most sixteen entries): the 256 pairs of symbols.
+__device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint2 *s_table, bool pairs)
+{
+    const uint2 *t = reinterpret_cast<const uint2 *>(a.table);
+    auto entry = [&](int i) {
+        const uint2 e = i < a.table_entries ? t[i] : make_uint2(0u, 0u);
+        return e.y == 0u || e.y > 8u ? make_uint2(0u, KVC_NO_CODE_LEN) : make_uint2(e.x & ((1u << e.y) - 1u), e.y);
+    };
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) {
+        uint2 e = entry(pairs ? i >> 4 : i);
+        if (pairs) {
+            const uint2 f = entry(i & 15);
+            e = make_uint2((e.x << (f.y & 31u)) | f.x, e.y + f.y);
+        }
+        s_table[i] = e;
+    }
+}
+
+// FRONT 0: K, 1: V.  ND: registers that a vector fills.
+template <int FRONT, int ND>
+__global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int run)
+{
+    constexpr int STAGE = FRONT == 0 ? KVC_STAGE_VSYM_BYTES : KVC_STAGE_VF16_BYTES;
+    extern __shared__ __align__(16) uint8_t s_dyn[];
+    __shared__ uint32_t s_err, s_max_tile, s_longest, s_polls, s_ticket;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+    uint2 *s_table = reinterpret_cast<uint2 *>(s_dyn);
+    uint32_t *area = reinterpret_cast<uint32_t *>(s_dyn + 256 * sizeof(uint2) + wave * a.wave_bytes);
+    uint8_t *s_stage = reinterpret_cast<uint8_t *>(area) + a.wave_bytes - STAGE;
+    uint32_t ticket = 0;
+    if (tid == 0) ticket = atomicAdd(&a.status[KVC_ONCE_TICKET_WORD], 1u);
+    const bool pairs = a.table_entries <= 16;
+    kvc_load_pair_table(a, s_table, pairs);
+    if (tid == 0) { s_err = 0; s_max_tile = 0; s_longest = 0; s_polls = 0; s_ticket = ticket; }
+    __syncthreads();
+    const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + wave) * run;
+    const int tiles = (int)a.tiles;
+    const uint32_t base = a.status[KVC_ONCE_BASE_WORD];
+    uint32_t err = 0, max_tile = 0, longest = 0, next_off = 0;
+    int polls = 0;
+    bool placed = false;                                   // the tiles of the run up to the first kept one have been; they end at next_off
+    // Tiles whose images wait in the area: `kept` of them, their payload bytes (sixteen bits each, the oldest lowest), the words
+    // they take and what the oldest one's look-back has asked for.
+    int kept = 0;
+    uint64_t kept_bytes = 0;
+    uint32_t kept_words = 0;
+    KvcOncePending first;
+    first.in_group = 0;
+#pragma unroll 1
+    for (int it = 0; it < run; it++) {
+        const int tile = tile0 + it;
+        if (tile >= tiles) break;
+        int lane = tid & 63;                               // (opaque, as in kvc_encode_once_kernel)
+        asm volatile("" : "+v"(lane));
+        const KvcEncodeArgs &a = kvc_kernarg_again<KvcEncodeArgs>();
+        uint32_t v[32];
+        {
+            kvc_u32x4 q[8];
+            if constexpr (FRONT == 0) {
+                kvc_load_k_wide<ND>(a, tile, lane, q);
+                kvc_stage_k_wide<ND>(lane, s_stage, q, v);
+            } else {
+                kvc_load_v_wide(a, tile, lane, q);
+                kvc_stage_v_wide(lane, s_stage, q, v);
+            }
+        }
+        uint32_t bits = 0, gl[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};     // the joined lengths of registers 4 i .. 4 i + 3
+        if (pairs) bits = kvc_join_vector<true, ND, 8>(s_table, v, gl);
+        else bits = kvc_join_vector<false, ND, 4>(s_table, v, gl);
+        const bool bad = bits >= KVC_NO_CODE_LEN;          // a symbol without a code: the lane emits nothing
+        if (bad) bits = 0;
+        const uint32_t bytes = (bits + 7u) >> 3, end = kvc_wave_inclusive_scan(bytes), start = end - bytes;
+        a.thread_infos[(int64_t)tile * KVC_WAVE + lane] = (uint16_t)((end << 3) + (bytes << 3) - bits);
+        const uint32_t tile_bytes = (uint32_t)__builtin_amdgcn_readlane((int)end, KVC_WAVE - 1);
+        if (__any(bad)) err |= KVC_ENC_ERR_NO_CODE;
+        if (tile_bytes > (uint32_t)KVC_MAX_TILE_BYTES) err |= KVC_ENC_ERR_TILE_TOO_BIG;
+        const uint32_t lg = kvc_wave_max_dpp(bytes);
+        const uint32_t bn = tile_bytes > 0xffffu ? 0xffffu : tile_bytes;
+        const bool packs = bn <= (uint32_t)KVC_MAX_TILE_BYTES;
+        longest = lg > longest ? lg : longest;
+        max_tile = bn > max_tile ? bn : max_tile;
+        if (lane == 0) kvc_status_store(reinterpret_cast<uint64_t *>(a.block_infos) + tile, kvc_bi_word(0u, bn, KVC_BI_SIZE));
+        // the tile that the run's place is looked for with; and the wave that speaks for a group must not sit on its size (as in
+        // kvc_encode_once_kernel)
+        const bool opens = kept == 0 && !placed, closes = kvc_once_closes(a, tile);
+        if (opens) {
+            first.looks = kvc_look_back_ask(a, tile, lane);
+            first.in_group_known = closes;
+        }
+        if (closes) {
+            const uint64_t word = opens ? first.looks.tile_word : kvc_look_back_ask(a, tile, lane).tile_word;
+            const uint32_t in_group = kvc_look_back_in_group(a, tile, bn, lane, word, &polls);
+            if (opens) first.in_group = in_group;
+        }
+        // The image goes behind the kept ones.  If it does not fit there, those are written out first, and this tile starts again
+        // (its size is published: nobody waits for it meanwhile).
+        const uint32_t my_words = packs ? kvc_once_image_words(bn) : 0u;
+        const bool fits = kept == 0 || (kept_words + my_words) * 4u <= (uint32_t)a.wave_bytes;
+        if (fits && packs) {
+            uint32_t *image = area + kept_words;
+            for (uint32_t i = lane; i < my_words / 4u; i += KVC_WAVE) reinterpret_cast<uint4 *>(image)[i] = make_uint4(0u, 0u, 0u, 0u);
+            kvc_wave_lds_sync();
+            if (!bad) {
+                // (streams of at most 2 3/4 bits per symbol: eight symbols next to always fit a word)
+                if (lg * 32u <= 11u * 4u * (uint32_t)ND) kvc_pack_joined<ND, true>(start, v, gl, image);
+                else kvc_pack_joined<ND, false>(start, v, gl, image);
+            }
+            kvc_wave_lds_sync();
+        }
+        if (fits) {
+            kept_bytes |= (uint64_t)bn << (16 * kept);
+            kept_words += my_words;
+            kept++;
+        }
+        // Images wait for the run's other tiles, unless they reach to where those are to be staged.
+        const bool more = it + 1 < run && tile + 1 < tiles;
+        if (!fits || !more || kept_words * 4u > (uint32_t)(a.wave_bytes - STAGE)) {
+            const int oldest = tile + (fits ? 1 : 0) - kept;
+            uint32_t at = 0;
+#pragma unroll 1
+            for (int k = 0; k < kept; k++) {               // one look-back (none behind tiles that have been placed), the others follow
+                KvcOncePending which = first;
+                which.tile = oldest + k;
+                which.bn = (uint32_t)(kept_bytes >> (16 * k)) & 0xffffu;
+                which.packs = which.bn <= (uint32_t)KVC_MAX_TILE_BYTES;
+                uint32_t off = 0;
+                err |= kvc_once_place(a, which, area + at, base, lane, &polls, &off, placed, next_off);
+                at += which.packs ? kvc_once_image_words(which.bn) : 0u;
+                next_off = off + which.bn;
+                placed = true;
+            }
+            kept = 0;
+            kept_bytes = 0;
+            kept_words = 0;
+            kvc_wave_lds_sync();                           // the images are read: the area is free
+            if (!fits) it--;
+        }
+    }
+    if ((tid & 63) == 0 && tile0 < tiles) {
+        if (err) atomicOr(&s_err, err);
+        atomicMax(&s_max_tile, max_tile);
+        atomicMax(&s_longest, longest);
+        atomicMax(&s_polls, (uint32_t)polls);
+    }
+    __syncthreads();
+    if (tid == 0) {                                        // to one of the slot's lines, picked by the ticket
+        uint32_t *part = a.status + KVC_ONCE_PART_WORD + (s_ticket % KVC_ONCE_PART_LINES) * KVC_ONCE_PART_STRIDE;
+        if (s_err) atomicOr(&part[0], s_err);
+        atomicMax(&part[1], s_max_tile);
+        atomicMax(&part[2], s_longest);
+        atomicMax(&part[3], s_polls);
+    }
+}
+
 // After the one-pass kernel, one workgroup: joins what the workgroups reported on their 32 lines into the call's status
 // words.  If a wave gave up on its look-back (KVC_ENC_ERR_ORDER: the payload and the block_infos are then incomplete)
 // this workgroup encodes the whole call again in two passes of its own -- count every tile, add up the offsets, emit
@@ -1339,7 +1703,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
     }
     __syncthreads();
     if (!s_again) {                                       // the rule
-        if (tid == 0) kvc_encode_publish(a.e);
+        kvc_encode_publish(a.e, tid);
         return;
     }
     // ---- the whole call again, two passes inside this workgroup ----
@@ -1373,7 +1737,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
         for (int64_t t0 = 0; t0 < tiles; t0 += KVC_WAVE) {
             const int64_t tile = t0 + lane;
             const uint32_t bn = tile < tiles ? bi[2 * tile + 1] & 0xffffu : 0u;
-            const uint32_t incl = kvc_wave_inclusive_scan(bn, lane);
+            const uint32_t incl = kvc_wave_inclusive_scan(bn);
             if (tile < tiles) bi[2 * tile] = at + incl - bn;
             at += (uint32_t)__builtin_amdgcn_readlane((int)incl, KVC_WAVE - 1);
             const uint32_t m = kvc_wave_max_dpp(bn);
@@ -1424,8 +1788,10 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
     if (tid == 0) {
         a.e.status[1] = (a.e.status[1] & KVC_ENC_ERR_CODEBOOK) | s_err;
         a.e.status[3] = s_longest;
-        kvc_encode_publish(a.e);
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __syncthreads();
+    kvc_encode_publish(a.e, tid);
 }
 
 // What the fused path adds to an encode call: the fp16 source and how to quantize it.
@@ -1462,6 +1828,7 @@ struct KvcEncodeCall {
     bool first_launch_only;
     int first_launch;                                      // what is done already: KVC_ENC_FRESH, KVC_ENC_CLEARED or KVC_ENC_MARKED
     uint32_t *h_outcome, outcome_number;
+    int longest_code;                                      // of the (one) codebook, 0: not known
 };
 
 static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
@@ -1573,11 +1940,10 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         // image beside its staging area.  The room in `encoded` bounds the mean tile (a first store reserves what its code
         // needs): where that leaves a fifth of margin, waves get less LDS and four of them fit; the odd run whose first image
         // is larger is placed before its second tile is counted, as a wave's only tile would be.  402 M symbols: 316 -> 288 us,
-        // 134 M: 110 -> 101 us.
+        // 134 M: 110 -> 101 us (of kvc_encode_once_kernel).
         const bool small = front == 0 && a.rows_per_codebook == 0 &&
                            a.encoded_cap / a.tiles <= (KVC_ONCE_SMALL_WAVE_BYTES - kvc_once_stage_bytes(0)) * 4 / 5;
         sa.e.wave_bytes = small ? KVC_ONCE_SMALL_WAVE_BYTES : KVC_ONCE_WAVE_BYTES;
-        const size_t lds = (size_t)(a.rows_per_codebook ? KVC_WAVES_PER_WG : 1) * 256 * sizeof(uint2) + (size_t)KVC_WAVES_PER_WG * sa.e.wave_bytes;
         // two tiles per wave (the look-back of the first hides behind the count of the second) where all tiles share
         // the codebook and there are enough of them to keep the chip full.  Longer runs would need the payloads of
         // more than one waiting tile in LDS.
@@ -1585,8 +1951,25 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         int run = want == 1 ? (a.tiles >= 8192 ? 2 : 1) : want - 1;       // 2, 3: always one, two tiles per wave
         run = run < 1 ? 1 : run > 2 ? 2 : run;
         if (a.rows_per_codebook != 0) run = 1;
-        const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * KVC_WAVES_PER_WG - 1) / ((int64_t)run * KVC_WAVES_PER_WG));
-        if (front == 0) {
+        // Vectors of 128, 96 and 64 symbols with codes known to be short have a kernel of their own where the alignment is for
+        // sixteen symbols per load.  It takes
+        // eight waves per workgroup where they get little LDS (two such workgroups per compute unit): half as many tickets, of
+        // which the chip hands out one in 11 ns.
+        const bool wide = front == 0 && a.rows_per_codebook == 0 && c.longest_code >= 1 && c.longest_code <= 8 && ((uintptr_t)c.d_sym & 15) == 0 && c.stride % 16 == 0 &&
+                          (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 64);
+        const int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
+        const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
+        // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (a run stays inside a group, or
+        // the wave that speaks for a group would wait before all its tiles are counted).
+        if (wide && small && run == 2 && want == 1 && !is_k && a.tiles >= 16384 && 3 * (a.encoded_cap / a.tiles * 9 / 8) <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) run = 4;
+        const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
+        const auto symbols_kernel = !is_k ? kvc_encode_symbols_kernel<1, 32> :
+                                    a.vec_len == 128 ? kvc_encode_symbols_kernel<0, 32> :
+                                    a.vec_len == 96 ? kvc_encode_symbols_kernel<0, 24> : kvc_encode_symbols_kernel<0, 16>;
+        if (wide) {
+            hipLaunchKernelGGL(symbols_kernel, dim3(wgs1), dim3(waves * KVC_WAVE), lds, stream, sa.e, run);
+            hipLaunchKernelGGL(kvc_encode_finish_kernel<0>, dim3(1), dim3(KVC_WG), 0, stream, sa);
+        } else if (front == 0) {
             hipLaunchKernelGGL(kvc_encode_once_kernel<0>, dim3(wgs1), dim3(KVC_WG), lds, stream, sa, run);
             hipLaunchKernelGGL(kvc_encode_finish_kernel<0>, dim3(1), dim3(KVC_WG), 0, stream, sa);
         } else if (front == 1) {
@@ -1607,7 +1990,7 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     if (!src) hipLaunchKernelGGL(kvc_encode_emit_kernel, dim3(wgs), dim3(KVC_WG), 0, stream, a);
     else if (is_k) hipLaunchKernelGGL(kvc_store_emit_kernel<true>, dim3(wgs), dim3(KVC_WG), 0, stream, sa);
     else hipLaunchKernelGGL(kvc_store_emit_kernel<false>, dim3(wgs), dim3(KVC_WG), 0, stream, sa);
-    if (a.result || a.stream_bytes) hipLaunchKernelGGL(kvc_encode_publish_kernel, dim3(1), dim3(1), 0, stream, a);
+    if (a.result || a.stream_bytes) hipLaunchKernelGGL(kvc_encode_publish_kernel, dim3(1), dim3(KVC_WAVE), 0, stream, a);
     KVC_HIP(hipGetLastError());
     return 0;
 }
@@ -1777,7 +2160,8 @@ extern "C" int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, in
     return 0;
 }
 
-extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, uint32_t *h_outcome, uint32_t outcome_number, void *stream)
+extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,
+                                uint32_t outcome_number, void *stream)
 {
     KvcEncodeCall c = {};
     if (int rc = kvc_encode_job_check(job, c)) return rc;
@@ -1789,6 +2173,7 @@ extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int 
     c.first_launch = prepared;
     c.h_outcome = h_outcome;
     c.outcome_number = outcome_number;
+    c.longest_code = longest_code;
     KvcStoreSource src = {job->d_x_f16, job->batch, job->heads, job->quant_mask, job->eb, job->d_min_i8, job->d_scale_f16};
     if (!job->d_sym) {
         KVC_REQUIRE(kvc_store_fused_supported(job->is_k, job->quant_mask, job->batch, job->heads, job->head_dim),
@@ -1809,7 +2194,7 @@ extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int 
     return kvc_encode_launch(c, &slot, (hipStream_t)stream);
 }
 
-extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream) { return kvc_encode_queue(job, nullptr, KVC_ENC_FRESH, nullptr, 0u, stream); }
+extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream) { return kvc_encode_queue(job, nullptr, KVC_ENC_FRESH, 0, nullptr, 0u, stream); }
 
 extern "C" int kvc_encode_result(const uint32_t *d_result, int64_t encoded_cap, int64_t *h_total_bytes, int64_t *h_max_tile_bytes,
                                  int64_t *h_max_stream_bytes, int64_t *h_tiles, void *stream)

@@ -54,7 +54,7 @@ kvc_h2_count_kernel(const uint8_t *__restrict__ sym, int64_t n, const uint32_t *
     uint32_t len[KVC_H2_SYMS_PER_THREAD], s[KVC_H2_SYMS_PER_THREAD];
     const int64_t first = ((int64_t)blockIdx.x * KVC_WG + threadIdx.x) * KVC_H2_SYMS_PER_THREAD;
     const uint32_t bits = kvc_h2_thread_bits(sym, n, first, s_len, len, s);
-    const uint32_t wave_bits = kvc_wave_inclusive_scan(bits, threadIdx.x & 63);
+    const uint32_t wave_bits = kvc_wave_inclusive_scan(bits);
     if ((threadIdx.x & 63) == 63) atomicAdd(&s_total, wave_bits);
     __syncthreads();
     if (threadIdx.x == 0) chunk_bits[blockIdx.x] = s_total;
@@ -103,7 +103,7 @@ kvc_h2_emit_kernel(const uint8_t *__restrict__ sym, int64_t n, const uint32_t *_
     uint32_t len[KVC_H2_SYMS_PER_THREAD], s[KVC_H2_SYMS_PER_THREAD];
     const int64_t first = ((int64_t)blockIdx.x * KVC_WG + threadIdx.x) * KVC_H2_SYMS_PER_THREAD;
     const uint32_t bits = kvc_h2_thread_bits(sym, n, first, s_len, len, s);
-    const uint32_t incl = kvc_wave_inclusive_scan(bits, lane);
+    const uint32_t incl = kvc_wave_inclusive_scan(bits);
     if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
     uint32_t before = incl - bits;

@@ -601,10 +601,10 @@ class KVCompCtx:
     COPY_PENDING = 8 << 20
 
     def _encode_direct(self, T: int, *, tables, table_bytes, symbols=None, cache=None, mask=0, most_bytes=None, keep=None,
-                       lost_if_dropped=False, certain=False, codebook=False, prepared=None):
+                       lost_if_dropped=False, certain=False, codebook=False, prepared=None, longest_code=0):
         """Queue one encode whose outputs go straight to their final places in this context's buffers; nothing waits.
         Quantizes `cache` on the fly (fused store) or takes `symbols` whose parameters are in place already.  most_bytes:
-        what the payload is known not to exceed; prepared: what _prepare_encode returned."""
+        what the payload is known not to exceed; prepared, longest_code: what _prepare_encode returned, the codebook's longest code."""
         nb = T // self.block_size
         B, H, D = self.batch_size, self.head_num, self.head_dim
         sizes = kvcomp_cuda.buffer_sizes(T, B * H * D, self.is_k, H, D) if prepared is None else prepared.sizes
@@ -632,7 +632,7 @@ class KVCompCtx:
         outcome = self._ask_outcome()
         told = None if outcome is None else outcome.ask(_lib.stream_of(state))
         if prepared is not None:
-            kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told)
+            kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told, longest_code)
         else:
             kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
                                      table_bytes=table_bytes, block_infos=bi, thread_infos=ti, encoded=self._encoded.data,
@@ -686,7 +686,7 @@ class KVCompCtx:
         queued = self.async_store and (cannot_fail or small)
         self._encode_direct(T, symbols=sym, tables=enc, table_bytes=enc.numel(), most_bytes=book.payload_bits // 8 + vectors + 1,
                             keep=blocked.flatten(0, 1).clone() if queued and not cannot_fail else None, certain=cannot_fail, codebook=True,
-                            prepared=prepared[0] if prepared else None)
+                            prepared=prepared[0] if prepared else None, longest_code=book.max_code_bits)
         if queued:
             self._issue_probe()
         else:

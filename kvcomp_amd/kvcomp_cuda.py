@@ -306,7 +306,7 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
         job.d_result = result.data_ptr()
     address, number = (0, 0) if outcome is None else outcome
     with _lib.device_guard(encoded):
-        check(_lib.lib().kvc_encode_queue(C.byref(job), 0, 0, address, number, _lib.stream_of(encoded)))
+        check(_lib.lib().kvc_encode_queue(C.byref(job), 0, 0, 0, address, number, _lib.stream_of(encoded)))
 
 
 class PreparedEncode(NamedTuple):
@@ -339,8 +339,9 @@ def encode_prepare(is_k: bool, *, batch: int, head_num: int, head_dim: int, toke
     return PreparedEncode(job, scratch, done.value, sizes)
 
 
-def encode_prepared(prepared: PreparedEncode, encode_table: torch.Tensor, encoded: torch.Tensor, outcome=None):
-    """What encode_prepare left to be done, now that the table and the payload buffer are there (once per preparation)."""
+def encode_prepared(prepared: PreparedEncode, encode_table: torch.Tensor, encoded: torch.Tensor, outcome=None, longest_code: int = 0):
+    """What encode_prepare left to be done, now that the table and the payload buffer are there (once per preparation).
+    longest_code: bits of the table's longest code, 0 if not known."""
     job, at = prepared.job, prepared.scratch.data_ptr()
     for t, n in ((encode_table, "encode_table"), (encoded, "encoded")):
         _dev_u8(t, n)
@@ -348,7 +349,7 @@ def encode_prepared(prepared: PreparedEncode, encode_table: torch.Tensor, encode
     job.d_encoded, job.encoded_cap = encoded.data_ptr(), encoded.numel()
     address, number = (0, 0) if outcome is None else outcome
     with _lib.device_guard(encoded):
-        check(_lib.lib().kvc_encode_queue(C.byref(job), at, prepared.done, address, number, _lib.stream_of(encoded)))
+        check(_lib.lib().kvc_encode_queue(C.byref(job), at, prepared.done, longest_code, address, number, _lib.stream_of(encoded)))
 
 
 def encode_result(result: torch.Tensor, encoded_cap: int):
