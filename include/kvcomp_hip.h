@@ -476,7 +476,11 @@ int kvc_quant_error(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int6
  * kvc_quant_in_place: quant_error (utils/compute.py:108-133) on `tokens` tokens (whole blocks) where they lie: element
  *   (b, h, t, d) at d_x_f16[b * stride_b + h * stride_h + t * head_dim + d]; KVC_MASK_CHANNEL, _VECTOR, _SIM_TOKEN or
  *   _SIM_BLOCK groups, results bit for bit kvc_quant_error's.  Returns 1, having done nothing, for a layout it does not
- *   take (head_dim not a multiple of 8 or above 128, rows off 16-byte boundaries, groups beyond a workgroup's registers). */
+ *   take (head_dim not a multiple of 8 or above 128, rows off 16-byte boundaries, groups beyond a workgroup's registers).
+ * kvc_append_quantized: kvc_append_dense, then kvc_quant_in_place of the first k_tokens new keys and v_tokens new values
+ *   (whole blocks), without the values in between; the same bits.  KVC_MASK_CHANNEL groups over blocks of 64 tokens for the
+ *   keys, KVC_MASK_SIM_TOKEN or _VECTOR for the values; returns 1, having done nothing, for others and for a head_dim that is
+ *   not a multiple of 16, or rows off 16-byte boundaries. */
 typedef struct kvc_append_job {
     const void *d_k, *d_v, *d_cos, *d_sin;
     void *d_k_cache, *d_v_cache;
@@ -485,6 +489,8 @@ typedef struct kvc_append_job {
     int64_t cos_stride_b, cos_stride_t, sin_stride_b, sin_stride_t;
 } kvc_append_job;
 int kvc_append_dense(const kvc_append_job *job, void *stream);
+int kvc_append_quantized(const kvc_append_job *job, int64_t k_tokens, int64_t k_block_size, int k_mask, float k_eb,
+                         int64_t v_tokens, int64_t v_block_size, int v_mask, float v_eb, void *stream);
 int kvc_quant_in_place(void *d_x_f16, int64_t batch, int64_t heads, int64_t tokens, int64_t head_dim, int64_t stride_b,
                        int64_t stride_h, int64_t block_size, int quant_mask, float eb, void *stream);
 

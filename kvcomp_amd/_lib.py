@@ -88,6 +88,7 @@ _SIGNATURES = {
     "kvc_quant_counted": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp, _vp, C.POINTER(_vp), _vp],
     "kvc_counted_codebook": [_vp, _int, C.POINTER(Codebook), _vp],
     "kvc_append_dense": [_vp, _vp],
+    "kvc_append_quantized": [_vp, _i64, _i64, _int, C.c_float, _i64, _i64, _int, C.c_float, _vp],
     "kvc_quant_in_place": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp],
     "kvc_put_codebook": [_vp, _vp, _vp, _vp],
     "kvc_put_bytes": [_vp, _vp, _i64, _vp],

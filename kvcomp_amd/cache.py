@@ -26,7 +26,7 @@ from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
-from .compute import append_dense, apply_rotary_pos_emb_single, blocks_to_compress, quant_in_place, safe_cat, takes_append
+from .compute import append_dense, append_quantized, apply_rotary_pos_emb_single, blocks_to_compress, quant_in_place, safe_cat, takes_append
 from .ctx import KVCompCacheConfigStatic, KVCompCtx
 
 
@@ -182,6 +182,26 @@ class KVCompCachePytorchQuant:
         k.append(key_states)
         v.append(value_states)
 
+    def _append_prompt(self, key_states, value_states, layer_idx, cache_kwargs, cfg) -> bool:
+        """A prompt whose first blocks leave the tails at once: appended and quantized together.  False, having done nothing,
+        where the layer holds tokens already or the tensors are not for it."""
+        k, v, n = self._k[layer_idx], self._v[layer_idx], key_states.shape[2]
+        if k.length or v.length or cfg.enable_pre_rope:
+            return False
+        plans = [(max(blocks_to_compress(n, block, recent), 0) * block, block, eb, mode) for block, recent, eb, mode in (
+            (cfg.k_block_size, cfg.k_recent_size, cfg.k_quant_scale_rel, cfg.k_quant_mode),
+            (cfg.v_block_size, cfg.v_recent_size, cfg.v_quant_scale_rel, cfg.v_quant_mode))]
+        cos, sin = cache_kwargs['cos'], cache_kwargs['sin']
+        if plans[0][0] == 0 or not takes_append(key_states, value_states, cos, sin):
+            return False
+        k.make_room(key_states)
+        v.make_room(value_states)
+        if not append_quantized(key_states, value_states, cos, sin, k.data, v.data, 0, *plans):
+            return False
+        k.length = v.length = n
+        k.quantized, v.quantized = plans[0][0], plans[1][0]
+        return True
+
     def _publish(self, layer_idx):
         k, v = self._k[layer_idx], self._v[layer_idx]
         k.updates += 1
@@ -199,8 +219,10 @@ class KVCompCachePytorchQuant:
             assert not cfg.enable_quant, "Disable quant to enable cache collect."
         if cfg.enable_quant is False:
             return self.update_disable(key_states, value_states, layer_idx, cache_kwargs)
-        self._append(key_states, value_states, layer_idx, cache_kwargs)
         k, v = self._k[layer_idx], self._v[layer_idx]
+        if not k.length and self._append_prompt(key_states, value_states, layer_idx, cache_kwargs, cfg):
+            return self._publish(layer_idx)
+        self._append(key_states, value_states, layer_idx, cache_kwargs)
         k.quantize_blocks(cfg.k_block_size, cfg.k_recent_size, cfg.k_quant_scale_rel, cfg.k_quant_mode)
         v.quantize_blocks(cfg.v_block_size, cfg.v_recent_size, cfg.v_quant_scale_rel, cfg.v_quant_mode)
         return self._publish(layer_idx)

@@ -190,24 +190,46 @@ def takes_append(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], 
     return _append_job(k, v, cos, sin) is not None
 
 
-def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], k_cache: torch.Tensor,
-                 v_cache: torch.Tensor, at: int) -> bool:
-    """kvc_append_dense: k (rotated by cos / sin [1 or B, T, D], unless they are None) and v, [B, H, T, D] fp16, to
-    positions at .. of the [B, H, capacity, D] caches.  False, having done nothing, for tensors it does not take or that
-    PyTorch would record.  (No view handed out before holds the positions written: their version need not move.)"""
+def _packed_append(k, v, cos, sin, k_cache, v_cache, at):
+    """kvc_append_job of these tensors, or None for ones that the kernels do not take or that PyTorch would record."""
     job = _append_job(k, v, cos, sin)
     if job is None or _lib.recorded(k, v, cos, sin, k_cache, v_cache):
-        return False
+        return None
     k_p, v_p, cos_p, sin_p, B, H, T, D, *strides = job
     f16, gpu, held = torch.float16, k.get_device(), k_cache.shape
     if not (k_cache.dtype is f16 and v_cache.dtype is f16 and k_cache.get_device() == gpu and v_cache.get_device() == gpu and
             len(held) == 4 and held[0] == B and held[1] == H and held[3] == D and v_cache.shape == held and
             k_cache.is_contiguous() and v_cache.is_contiguous()):
+        return None
+    return _APPEND.pack(k_p, v_p, cos_p, sin_p, k_cache.data_ptr(), v_cache.data_ptr(), B, H, T, D, held[2], at, *strides)
+
+
+def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], k_cache: torch.Tensor,
+                 v_cache: torch.Tensor, at: int) -> bool:
+    """kvc_append_dense: k (rotated by cos / sin [1 or B, T, D], unless they are None) and v, [B, H, T, D] fp16, to
+    positions at .. of the [B, H, capacity, D] caches.  False, having done nothing, for tensors it does not take or that
+    PyTorch would record.  (No view handed out before holds the positions written: their version need not move.)"""
+    packed = _packed_append(k, v, cos, sin, k_cache, v_cache, at)
+    if packed is None:
         return False
-    packed = _APPEND.pack(k_p, v_p, cos_p, sin_p, k_cache.data_ptr(), v_cache.data_ptr(), B, H, T, D, held[2], at, *strides)
     with _lib.device_guard(k):
         check(_lib.lib().kvc_append_dense(packed, _lib.stream_of(k)))
     return True
+
+
+def append_quantized(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], k_cache: torch.Tensor,
+                     v_cache: torch.Tensor, at: int, k_plan, v_plan) -> bool:
+    """kvc_append_quantized: append_dense with the first tokens replaced by their simulated-quantization values on the way.
+    The plans are (tokens, block size, error bound, mode).  False, having done nothing, for what it does not take."""
+    packed = _packed_append(k, v, cos, sin, k_cache, v_cache, at)
+    if packed is None:
+        return False
+    (kn, kb, ke, km), (vn, vb, ve, vm) = k_plan, v_plan
+    with _lib.device_guard(k):
+        rc = _lib.lib().kvc_append_quantized(packed, kn, kb, _SIM_PLAN[km][1], float(ke), vn, vb, _SIM_PLAN[vm][1], float(ve), _lib.stream_of(k))
+    if rc < 0:
+        check(rc)
+    return rc == 0
 
 
 def quant_error(error_cache, buffer, new_tensor, block_size: int, recent_size: int, quant_scale_rel: float,

@@ -3,6 +3,7 @@
 //   kvc_append_dense   <- apply_rotary_pos_emb_single (utils/compute.py:25-33) and the two safe_cat(..., dim=2) of an
 //                         update: keys rotated and values copied straight to their place in the [B, H, capacity, D] caches
 //   kvc_quant_in_place <- quant_error (utils/compute.py:108-133) on a stretch of such a cache
+//   kvc_append_quantized  both, for the first tokens of a cache
 //
 // Both are bound by HBM for a prompt and by launches for a token: one launch per update of a layer (the rotation and the
 // two appends took eight), and one or two for blocks that leave the tail, where they lie, without the contiguous copies
@@ -34,31 +35,16 @@ __device__ __forceinline__ void kvc_store_halves(_Float16 *p, const KvcHalves<VE
     else *p = r.v[0];
 }
 
-// A thread takes VEC adjacent channels of a token and the VEC that lie half a head further on, which the rotation pairs
-// them with.  Grid (items, 2): y = 0 the keys, 1 the values.  The rotation is the reference's: t * cos and
-// rotate_half(t) * sin, each rounded to fp16, then their sum.
+// VEC adjacent channels of a new key from channel c on, and the VEC that lie half a head further on, which the rotation pairs
+// them with.  The rotation is the reference's: t * cos and rotate_half(t) * sin, each rounded to fp16, then their sum.
 template <int VEC>
-__global__ void __launch_bounds__(KVC_WG) kvc_append_dense_kernel(kvc_append_job a)
+__device__ __forceinline__ void kvc_rotated_key(const kvc_append_job &a, int64_t b, int64_t h, int64_t t, int c, int half, KvcHalves<VEC> &lo,
+                                                KvcHalves<VEC> &hi)
 {
 #pragma clang fp contract(off)
-    const int half = (int)a.head_dim / 2, per = half / VEC;
-    const int64_t item = (int64_t)blockIdx.x * KVC_WG + threadIdx.x;
-    if (item >= a.batch * a.heads * a.tokens * per) return;
-    int64_t r = item / per;
-    const int c = (int)(item - r * per) * VEC;
-    const int64_t bh = r / a.tokens, t = r - bh * a.tokens, b = bh / a.heads, h = bh - b * a.heads;
-    const int64_t to = (bh * a.capacity + a.at + t) * a.head_dim + c;
-    if (blockIdx.y == 1) {
-        const _Float16 *p = reinterpret_cast<const _Float16 *>(a.d_v) + b * a.v_stride_b + h * a.v_stride_h + t * a.v_stride_t + c;
-        _Float16 *o = reinterpret_cast<_Float16 *>(a.d_v_cache) + to;
-        const KvcHalves<VEC> lo = kvc_load_halves<VEC>(p), hi = kvc_load_halves<VEC>(p + half);
-        kvc_store_halves<VEC>(o, lo);
-        kvc_store_halves<VEC>(o + half, hi);
-        return;
-    }
     const _Float16 *p = reinterpret_cast<const _Float16 *>(a.d_k) + b * a.k_stride_b + h * a.k_stride_h + t * a.k_stride_t + c;
-    _Float16 *o = reinterpret_cast<_Float16 *>(a.d_k_cache) + to;
-    KvcHalves<VEC> lo = kvc_load_halves<VEC>(p), hi = kvc_load_halves<VEC>(p + half);
+    lo = kvc_load_halves<VEC>(p);
+    hi = kvc_load_halves<VEC>(p + half);
     if (a.d_cos) {                                         // uniform
         const _Float16 *cp = reinterpret_cast<const _Float16 *>(a.d_cos) + b * a.cos_stride_b + t * a.cos_stride_t + c;
         const _Float16 *sp = reinterpret_cast<const _Float16 *>(a.d_sin) + b * a.sin_stride_b + t * a.sin_stride_t + c;
@@ -72,17 +58,43 @@ __global__ void __launch_bounds__(KVC_WG) kvc_append_dense_kernel(kvc_append_job
             hi.v[k] = yc + xs;
         }
     }
+}
+
+// A thread takes VEC adjacent channels of a token and their partners.  Grid (items, 2): y = 0 the keys from token k_from on,
+// 1 the values from v_from on.
+template <int VEC>
+__global__ void __launch_bounds__(KVC_WG) kvc_append_dense_kernel(kvc_append_job a, int64_t k_from, int64_t v_from)
+{
+    const int half = (int)a.head_dim / 2, per = half / VEC;
+    const int64_t item = (int64_t)blockIdx.x * KVC_WG + threadIdx.x, from = blockIdx.y ? v_from : k_from, tokens = a.tokens - from;
+    if (item >= a.batch * a.heads * tokens * per) return;
+    int64_t r = item / per;
+    const int c = (int)(item - r * per) * VEC;
+    const int64_t bh = r / tokens, t = r - bh * tokens + from, b = bh / a.heads, h = bh - b * a.heads;
+    const int64_t to = (bh * a.capacity + a.at + t) * a.head_dim + c;
+    if (blockIdx.y == 1) {
+        const _Float16 *p = reinterpret_cast<const _Float16 *>(a.d_v) + b * a.v_stride_b + h * a.v_stride_h + t * a.v_stride_t + c;
+        _Float16 *o = reinterpret_cast<_Float16 *>(a.d_v_cache) + to;
+        const KvcHalves<VEC> lo = kvc_load_halves<VEC>(p), hi = kvc_load_halves<VEC>(p + half);
+        kvc_store_halves<VEC>(o, lo);
+        kvc_store_halves<VEC>(o + half, hi);
+        return;
+    }
+    _Float16 *o = reinterpret_cast<_Float16 *>(a.d_k_cache) + to;
+    KvcHalves<VEC> lo, hi;
+    kvc_rotated_key<VEC>(a, b, h, t, c, half, lo, hi);
     kvc_store_halves<VEC>(o, lo);
     kvc_store_halves<VEC>(o + half, hi);
 }
 
-extern "C" int kvc_append_dense(const kvc_append_job *job, void *stream_)
+static int kvc_append_check(const kvc_append_job *job, int *vec)
 {
     KVC_REQUIRE(job != nullptr, "NULL argument");
     const kvc_append_job &a = *job;
     KVC_REQUIRE(a.batch > 0 && a.heads > 0 && a.head_dim > 0 && a.head_dim % 2 == 0 && a.tokens >= 0, "bad shape");
     KVC_REQUIRE(a.at >= 0 && a.at + a.tokens <= a.capacity, "the cache holds %lld tokens, %lld + %lld are to lie in it", (long long)a.capacity,
                 (long long)a.at, (long long)a.tokens);
+    *vec = 1;
     if (a.tokens == 0) return 0;
     KVC_REQUIRE(a.d_k && a.d_v && a.d_k_cache && a.d_v_cache && (!a.d_cos == !a.d_sin), "NULL argument");
     // the widest loads that every address allows
@@ -92,15 +104,28 @@ extern "C" int kvc_append_dense(const kvc_append_job *job, void *stream_)
                       a.sin_stride_b, a.sin_stride_t, half})
         bits |= (uint64_t)s * 2;
     KVC_REQUIRE((bits & 1) == 0, "fp16 buffers are misaligned");
-    const int vec = (bits & 15) == 0 ? 8 : (bits & 7) == 0 ? 4 : 1;
-    const int64_t wgs = (a.batch * a.heads * a.tokens * (half / vec) + KVC_WG - 1) / KVC_WG;
+    *vec = (bits & 15) == 0 ? 8 : (bits & 7) == 0 ? 4 : 1;
+    const int64_t wgs = (a.batch * a.heads * a.tokens * (half / *vec) + KVC_WG - 1) / KVC_WG;
     KVC_REQUIRE(wgs < (1ll << 31), "too many tokens for one call");
-    const dim3 grid((unsigned)wgs, 2);
-    hipStream_t stream = (hipStream_t)stream_;
-    if (vec == 8) hipLaunchKernelGGL(kvc_append_dense_kernel<8>, grid, dim3(KVC_WG), 0, stream, a);
-    else if (vec == 4) hipLaunchKernelGGL(kvc_append_dense_kernel<4>, grid, dim3(KVC_WG), 0, stream, a);
-    else hipLaunchKernelGGL(kvc_append_dense_kernel<1>, grid, dim3(KVC_WG), 0, stream, a);
+    return 0;
+}
+
+static int kvc_append_launch(const kvc_append_job &a, int vec, int64_t k_from, int64_t v_from, hipStream_t stream)
+{
+    const int64_t most = a.tokens - (k_from < v_from ? k_from : v_from);
+    if (most <= 0) return 0;
+    const dim3 grid((unsigned)((a.batch * a.heads * most * (a.head_dim / 2 / vec) + KVC_WG - 1) / KVC_WG), 2);
+    if (vec == 8) hipLaunchKernelGGL(kvc_append_dense_kernel<8>, grid, dim3(KVC_WG), 0, stream, a, k_from, v_from);
+    else if (vec == 4) hipLaunchKernelGGL(kvc_append_dense_kernel<4>, grid, dim3(KVC_WG), 0, stream, a, k_from, v_from);
+    else hipLaunchKernelGGL(kvc_append_dense_kernel<1>, grid, dim3(KVC_WG), 0, stream, a, k_from, v_from);
     return kvc_check_hip(hipGetLastError(), "kvc_append_dense_kernel launch");
+}
+
+extern "C" int kvc_append_dense(const kvc_append_job *job, void *stream)
+{
+    int vec;
+    if (int rc = kvc_append_check(job, &vec)) return rc;
+    return kvc_append_launch(*job, vec, 0, 0, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -109,6 +134,8 @@ extern "C" int kvc_append_dense(const kvc_append_job *job, void *stream_)
 struct KvcInPlaceArgs {
     _Float16 *x;                  // first token of the stretch, batch entry 0, head 0
     int64_t stride_b, stride_h;   // elements; a token's row follows the one before it
+    const _Float16 *from;         // where the tokens are read (x itself, unless they are appended by the same launch)
+    int64_t from_b, from_h, from_t;
     int NB, BS, B, H, D;
     float eb;
     uint32_t *minmax;             // block groups: {ord(min), ord(max)} per (batch entry, block)
@@ -187,6 +214,82 @@ __global__ void __launch_bounds__(KVC_WG) kvc_in_place_channel_kernel(KvcInPlace
     }
 }
 
+// New keys with per-channel groups over blocks of 64 tokens, rotated, quantized and put in place by one launch (appended
+// first and then quantized in place, a prompt's keys went over the bus twice more).  A workgroup takes a (batch entry, head,
+// block): sixteen bytes of a token and their partners per load; the rotated block lies in LDS for the channels' minima and
+// maxima, and stays in registers to be quantized.  Bound by HBM: K of 4 x 32 heads x 128 x 2048 tokens 35 us (134 MB), V, whose
+// tokens are read where they come from, 26; appended first and then quantized in place the two took 113.  A cache update with
+// that prompt and two more tokens: 110 -> 72 us; with 32 more the host's calls take longer than the prompt (576 -> 570).
+template <int ITEMS>
+__global__ void __launch_bounds__(KVC_WG) kvc_append_channel_kernel(kvc_append_job a, int NB, float eb)
+{
+    constexpr int BS = KVC_WAVE, PAIRS = KVC_K_VEC_LEN / 2;
+    __shared__ __align__(16) uint32_t s_tile[BS * PAIRS];              // [token][channel pair]
+    __shared__ __align__(16) uint2 s_minmax[KVC_WG];                   // {minima, maxima} of a pair's part of the block, then of the block
+    __shared__ __align__(16) uint4 s_packed[PAIRS];
+    __shared__ __align__(16) uint4 s_value[PAIRS];                     // {min2, scale2, whether the packed arithmetic applies}
+    const int tid = threadIdx.x, D = (int)a.head_dim, half = D / 2, per = half / 8, pairs = D / 2;
+    const int64_t bh = blockIdx.x / (unsigned)NB, nb = blockIdx.x - bh * NB, b = bh / a.heads, h = bh - b * a.heads;
+    KvcHalves<8> lo[ITEMS], hi[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const int item = tid + KVC_WG * j, t = item / per, c = (item - t * per) * 8;
+        if (t < BS) kvc_rotated_key<8>(a, b, h, nb * BS + t, c, half, lo[j], hi[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const int item = tid + KVC_WG * j, t = item / per, c = (item - t * per) * 8;
+        if (t < BS) {
+            *reinterpret_cast<uint4 *>(s_tile + t * pairs + c / 2) = __builtin_bit_cast(uint4, lo[j]);
+            *reinterpret_cast<uint4 *>(s_tile + t * pairs + (c + half) / 2) = __builtin_bit_cast(uint4, hi[j]);
+        }
+    }
+    __syncthreads();
+    const int parts = KVC_WG / pairs, part = tid / pairs, pair = tid - part * pairs;
+    if (part < parts) {
+        kvc_half2 mn = kvc_as_half2(s_tile[part * pairs + pair]), mx = mn;
+        for (int t = part + parts; t < BS; t += parts) {
+            const kvc_half2 x = kvc_as_half2(s_tile[t * pairs + pair]);
+            mn = __builtin_elementwise_min(mn, x);
+            mx = __builtin_elementwise_max(mx, x);
+        }
+        s_minmax[tid] = make_uint2(__builtin_bit_cast(uint32_t, mn), __builtin_bit_cast(uint32_t, mx));
+    }
+    __syncthreads();
+    if (tid < pairs) {
+        kvc_half2 mn = kvc_as_half2(s_minmax[tid].x), mx = kvc_as_half2(s_minmax[tid].y);
+        for (int q = 1; q < parts; q++) {
+            mn = __builtin_elementwise_min(mn, kvc_as_half2(s_minmax[tid + q * pairs].x));
+            mx = __builtin_elementwise_max(mx, kvc_as_half2(s_minmax[tid + q * pairs].y));
+        }
+        const uint32_t mnw = __builtin_bit_cast(uint32_t, mn), mxw = __builtin_bit_cast(uint32_t, mx);
+        const KvcGroupParams g0 = kvc_group_params(kvc_half_lo(mnw), kvc_half_lo(mxw), eb), g1 = kvc_group_params(kvc_half_hi(mnw), kvc_half_hi(mxw), eb);
+        const bool packed = kvc_packed_quantizer_applies(g0, kvc_half_lo(mxw)) && kvc_packed_quantizer_applies(g1, kvc_half_hi(mxw));
+        const KvcPackedParams pp = kvc_packed_params(g0, g1);
+        s_packed[tid] = make_uint4(pp.P2, pp.S2, pp.r2, pp.c2);
+        s_value[tid] = make_uint4(kvc_half_pair_bits(g0.min_h, g1.min_h), kvc_half_pair_bits(g0.scale_h, g1.scale_h), packed ? 1u : 0u, 0u);
+        s_minmax[tid] = make_uint2(mnw, mxw);
+    }
+    __syncthreads();
+    auto value = [&](uint32_t w, int p) {
+        const uint4 c = s_packed[p], v = s_value[p];
+        if (v.z) return kvc_quant_error_pair(kvc_quant_pair_biased(w, KvcPackedParams{c.x, c.y, c.z, c.w}), v.x, v.y);
+        const uint2 mm = s_minmax[p];
+        const KvcGroupParams g0 = kvc_group_params(kvc_half_lo(mm.x), kvc_half_lo(mm.y), eb), g1 = kvc_group_params(kvc_half_hi(mm.x), kvc_half_hi(mm.y), eb);
+        return kvc_half_pair_bits(kvc_quant_error_one(kvc_half_lo(w), g0), kvc_quant_error_one(kvc_half_hi(w), g1));
+    };
+#pragma unroll
+    for (int j = 0; j < ITEMS; j++) {
+        const int item = tid + KVC_WG * j, t = item / per, c = (item - t * per) * 8;
+        if (t >= BS) continue;
+        _Float16 *o = reinterpret_cast<_Float16 *>(a.d_k_cache) + (bh * a.capacity + a.at + nb * BS + t) * D + c;
+        const uint4 x = __builtin_bit_cast(uint4, lo[j]), y = __builtin_bit_cast(uint4, hi[j]);
+        const int p = c / 2, q = (c + half) / 2;
+        *reinterpret_cast<uint4 *>(o) = make_uint4(value(x.x, p), value(x.y, p + 1), value(x.z, p + 2), value(x.w, p + 3));
+        *reinterpret_cast<uint4 *>(o + half) = make_uint4(value(y.x, q), value(y.y, q + 1), value(y.z, q + 2), value(y.w, q + 3));
+    }
+}
+
 // Per-vector groups: a group is one token's row of one head; 16 lanes take it, eight elements each.
 __global__ void __launch_bounds__(KVC_WG) kvc_in_place_vector_kernel(KvcInPlaceArgs a)
 {
@@ -199,7 +302,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_in_place_vector_kernel(KvcInPlaceA
     uint4 v = make_uint4(0u, 0u, 0u, 0u);
     float lo = INFINITY, hi = -INFINITY;
     if (live) {
-        v = *p;
+        v = *reinterpret_cast<const uint4 *>(a.from + b * a.from_b + h * a.from_h + t * a.from_t + c);
         kvc_half2 mn = kvc_as_half2(v.x), mx = mn;
         for (uint32_t w : {v.y, v.z, v.w}) {
             mn = __builtin_elementwise_min(mn, kvc_as_half2(w));
@@ -232,15 +335,20 @@ __global__ void __launch_bounds__(KVC_WG) kvc_in_place_token_kernel(KvcInPlaceAr
     const int64_t b = g / tokens, t = g - b * tokens;
     _Float16 *x = a.x + b * a.stride_b + t * a.D;
     const int at = WPR == 1 ? lane : (int)threadIdx.x, per = a.D >> 3, pieces = a.H * per;
+    const _Float16 *from = a.from + b * a.from_b + t * a.from_t;
     auto where = [&](int j) {
         const int i = at + 64 * WPR * j, h = i / per;
         return reinterpret_cast<uint4 *>(x + h * a.stride_h + 8 * (i - h * per));
+    };
+    auto read = [&](int j) {
+        const int i = at + 64 * WPR * j, h = i / per;
+        return *reinterpret_cast<const uint4 *>(from + h * a.from_h + 8 * (i - h * per));
     };
     uint4 raw[NIT];
     kvc_half2 mn = {(_Float16)INFINITY, (_Float16)INFINITY}, mx = -mn;
 #pragma unroll
     for (int j = 0; j < NIT; j++)
-        if (at + 64 * WPR * j < pieces) raw[j] = *where(j);
+        if (at + 64 * WPR * j < pieces) raw[j] = read(j);
 #pragma unroll
     for (int j = 0; j < NIT; j++) {
         if (at + 64 * WPR * j < pieces) {
@@ -316,6 +424,25 @@ __global__ void __launch_bounds__(KVC_WG) kvc_in_place_block_kernel(KvcInPlaceAr
     }
 }
 
+static dim3 kvc_wgs(int64_t threads) { return dim3((unsigned)((threads + KVC_WG - 1) / KVC_WG)); }
+
+// groups of one token of one batch entry, or of one token of one head
+static void kvc_launch_token_groups(const KvcInPlaceArgs &a, int quant_mask, hipStream_t stream)
+{
+    const int64_t tokens = (int64_t)a.NB * a.BS, row = (int64_t)a.H * a.D;
+    if (quant_mask == KVC_MASK_VECTOR) {
+        hipLaunchKernelGGL(kvc_in_place_vector_kernel, kvc_wgs(a.B * a.H * tokens * 16), dim3(KVC_WG), 0, stream, a);
+        return;
+    }
+    constexpr int W = KVC_WAVES_PER_WG;
+    const dim3 one = kvc_wgs(a.B * tokens * KVC_WAVE), all((unsigned)(a.B * tokens));
+    if (row <= 512 * 4) hipLaunchKernelGGL((kvc_in_place_token_kernel<4, 1>), one, dim3(KVC_WG), 0, stream, a);
+    else if (row <= 512 * 8) hipLaunchKernelGGL((kvc_in_place_token_kernel<8, 1>), one, dim3(KVC_WG), 0, stream, a);
+    else if (row <= 512 * 16) hipLaunchKernelGGL((kvc_in_place_token_kernel<16, 1>), one, dim3(KVC_WG), 0, stream, a);
+    else if (row <= 512 * W * 16) hipLaunchKernelGGL((kvc_in_place_token_kernel<16, W>), all, dim3(KVC_WG), 0, stream, a);
+    else hipLaunchKernelGGL((kvc_in_place_token_kernel<32, W>), all, dim3(KVC_WG), 0, stream, a);
+}
+
 // 1: not a layout these kernels take
 extern "C" int kvc_quant_in_place(void *d_x_f16, int64_t B, int64_t H, int64_t tokens, int64_t D, int64_t stride_b, int64_t stride_h,
                                   int64_t block_size, int quant_mask, float eb, void *stream_)
@@ -337,34 +464,73 @@ extern "C" int kvc_quant_in_place(void *d_x_f16, int64_t B, int64_t H, int64_t t
     a.D = (int)D;
     a.eb = eb;
     a.minmax = nullptr;
-    auto wgs = [](int64_t threads) { return dim3((unsigned)((threads + KVC_WG - 1) / KVC_WG)); };
+    a.from = a.x;
+    a.from_b = stride_b;
+    a.from_h = stride_h;
+    a.from_t = D;
     if (quant_mask == KVC_MASK_CHANNEL) {
-        const dim3 grid = wgs(B * H * a.NB * (D / 2));
+        const dim3 grid = kvc_wgs(B * H * a.NB * (D / 2));
         if (block_size == KVC_WAVE) hipLaunchKernelGGL(kvc_in_place_channel_kernel<true>, grid, dim3(KVC_WG), 0, stream, a);
         else hipLaunchKernelGGL(kvc_in_place_channel_kernel<false>, grid, dim3(KVC_WG), 0, stream, a);
-    } else if (quant_mask == KVC_MASK_VECTOR) {
-        hipLaunchKernelGGL(kvc_in_place_vector_kernel, wgs(B * H * tokens * 16), dim3(KVC_WG), 0, stream, a);
-    } else if (quant_mask == KVC_MASK_SIM_TOKEN) {
-        if (H * D > KVC_IN_PLACE_TOKEN_MAX) return 1;
-        constexpr int W = KVC_WAVES_PER_WG;
-        const dim3 one = wgs(B * tokens * KVC_WAVE), all((unsigned)(B * tokens));
-        if (H * D <= 512 * 4) hipLaunchKernelGGL((kvc_in_place_token_kernel<4, 1>), one, dim3(KVC_WG), 0, stream, a);
-        else if (H * D <= 512 * 8) hipLaunchKernelGGL((kvc_in_place_token_kernel<8, 1>), one, dim3(KVC_WG), 0, stream, a);
-        else if (H * D <= 512 * 16) hipLaunchKernelGGL((kvc_in_place_token_kernel<16, 1>), one, dim3(KVC_WG), 0, stream, a);
-        else if (H * D <= 512 * W * 16) hipLaunchKernelGGL((kvc_in_place_token_kernel<16, W>), all, dim3(KVC_WG), 0, stream, a);
-        else hipLaunchKernelGGL((kvc_in_place_token_kernel<32, W>), all, dim3(KVC_WG), 0, stream, a);
+    } else if (quant_mask == KVC_MASK_VECTOR || quant_mask == KVC_MASK_SIM_TOKEN) {
+        if (quant_mask == KVC_MASK_SIM_TOKEN && H * D > KVC_IN_PLACE_TOKEN_MAX) return 1;
+        kvc_launch_token_groups(a, quant_mask, stream);
     } else if (quant_mask == KVC_MASK_SIM_BLOCK) {
         const int groups = (int)B * a.NB;
         if ((size_t)groups * 8 > KVC_WS_SLOT_BYTES) return 1;
         void *slot;
         if (int rc = kvc_workspace_slot(&slot, stream_)) return rc;
         a.minmax = reinterpret_cast<uint32_t *>(slot);
-        const dim3 grid = wgs(B * H * a.NB * KVC_WAVE);
-        hipLaunchKernelGGL(kvc_in_place_block_init_kernel, wgs(groups), dim3(KVC_WG), 0, stream, a.minmax, groups);
+        const dim3 grid = kvc_wgs(B * H * a.NB * KVC_WAVE);
+        hipLaunchKernelGGL(kvc_in_place_block_init_kernel, kvc_wgs(groups), dim3(KVC_WG), 0, stream, a.minmax, groups);
         hipLaunchKernelGGL(kvc_in_place_block_kernel<false>, grid, dim3(KVC_WG), 0, stream, a);
         hipLaunchKernelGGL(kvc_in_place_block_kernel<true>, grid, dim3(KVC_WG), 0, stream, a);
     } else {
         return kvc_fail(-1, "unsupported quantization group mask 0x%x", quant_mask);
     }
     return kvc_check_hip(hipGetLastError(), "in-place quantizer launch");
+}
+
+// ---------------------------------------------------------------------------------------------------
+// both at once, for a prompt
+// ---------------------------------------------------------------------------------------------------
+// 1: not tensors or groups this takes
+extern "C" int kvc_append_quantized(const kvc_append_job *job, int64_t k_tokens, int64_t k_block_size, int k_mask, float k_eb, int64_t v_tokens,
+                                    int64_t v_block_size, int v_mask, float v_eb, void *stream_)
+{
+    hipStream_t stream = (hipStream_t)stream_;
+    int vec;
+    if (int rc = kvc_append_check(job, &vec)) return rc;
+    const kvc_append_job &a = *job;
+    KVC_REQUIRE(k_block_size > 0 && v_block_size > 0 && k_tokens >= 0 && v_tokens >= 0 && k_tokens <= a.tokens && v_tokens <= a.tokens &&
+                    k_tokens % k_block_size == 0 && v_tokens % v_block_size == 0, "bad stretch");
+    KVC_REQUIRE(k_eb > 0.f && v_eb > 0.f, "error bound must be positive");
+    const int64_t D = a.head_dim, blocks = k_tokens / KVC_WAVE;
+    if (vec != 8 || D % 16 != 0 || D > KVC_K_VEC_LEN || k_mask != KVC_MASK_CHANNEL || k_block_size != KVC_WAVE) return 1;
+    if (!(v_mask == KVC_MASK_VECTOR || (v_mask == KVC_MASK_SIM_TOKEN && a.heads * D <= KVC_IN_PLACE_TOKEN_MAX))) return 1;
+    if (a.batch * a.heads * a.tokens >= (1ll << 31)) return 1;
+    if (blocks > 0) {
+        const dim3 grid((unsigned)(a.batch * a.heads * blocks));
+        if (D / 16 * KVC_WAVE <= KVC_WG) hipLaunchKernelGGL(kvc_append_channel_kernel<1>, grid, dim3(KVC_WG), 0, stream, a, (int)blocks, k_eb);
+        else hipLaunchKernelGGL(kvc_append_channel_kernel<2>, grid, dim3(KVC_WG), 0, stream, a, (int)blocks, k_eb);
+    }
+    if (v_tokens > 0) {
+        KvcInPlaceArgs v = {};
+        v.x = reinterpret_cast<_Float16 *>(a.d_v_cache) + a.at * D;
+        v.stride_b = a.heads * a.capacity * D;
+        v.stride_h = a.capacity * D;
+        v.from = reinterpret_cast<const _Float16 *>(a.d_v);
+        v.from_b = a.v_stride_b;
+        v.from_h = a.v_stride_h;
+        v.from_t = a.v_stride_t;
+        v.NB = (int)(v_tokens / v_block_size);
+        v.BS = (int)v_block_size;
+        v.B = (int)a.batch;
+        v.H = (int)a.heads;
+        v.D = (int)D;
+        v.eb = v_eb;
+        kvc_launch_token_groups(v, v_mask, stream);
+    }
+    if (int rc = kvc_append_launch(a, vec, k_tokens, v_tokens, stream)) return rc;
+    return kvc_check_hip(hipGetLastError(), "append and quantize launch");
 }
