@@ -1409,10 +1409,11 @@ __global__ void __launch_bounds__(KVC_WG, 3) kvc_encode_once_kernel(KvcStoreArgs
 // most 16 symbols are looked up two at a time with one instruction per address, what is the same for a wave is kept in scalar
 // registers, and codes of more than 8 bits are left to the other kernel, whose loops for them took most of the registers: 7.5
 // (K) and 6 (V) vector instructions per symbol.  From symbols, us: K 8 x 32 heads x 128 x 4096 tokens 111 -> 75, V 104 ->
-// 71; 4 x 32 x 96 x 32 768 tokens 338 -> 257 and 242 -> 182.  What is left is the wait for the tiles before a wave's own (14
-// and 13 of the 75 and 71 us, 65 of 257: measured with made-up offsets) and the tickets (4).  Sixteen waves per compute unit
-// are best: 20 of them (five per SIMD, for which the registers would do) take 293 instead of 257 us, and a second tile on
-// its way while the first is packed gains nothing for the registers it takes.
+// 71; 4 x 32 x 96 x 32 768 tokens 338 -> 257 and 242 -> 182 (60, 238 and 164 with neighbouring tiles read together, below).
+// What is left is the wait for the tiles before a wave's own (14 and 13 of the 75 and 71 us, 65 of 257: measured with made-up
+// offsets) and the tickets (4).  Sixteen waves per compute unit are best: 20 of them (five per SIMD, for which the registers
+// would do) take 293 instead of 257 us, and a second tile on its way while the first is packed gains nothing for the
+// registers it takes.
 // A few registers of symbols at a time, without a branch inside, so that their look-ups are in flight together.  The symbols of
 // a register are looked up and their codes joined, at most 32 bits; gl receives the joined lengths, four to a register.
 // PAIRS: the table has an entry per two symbols below 16, first symbol in the index's upper half.  Returns the vector's bits.
@@ -1536,7 +1537,14 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     kvc_load_pair_table(a, s_table, pairs);
     if (tid == 0) { s_err = 0; s_max_tile = 0; s_longest = 0; s_polls = 0; s_ticket = ticket; }
     __syncthreads();
-    const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + wave) * run;
+    // Neighbouring tiles share the cache lines that their symbols come in (V and head_dim 64: 64 bytes of each token's row, 96: 96),
+    // and the lines of all waves are more than an L2 holds.  So STEP waves, whose tiles of one moment are whole lines, take the
+    // tiles of all their runs in turn, and their loads meet.  (A group is a multiple of what they take.)  HBM traffic and time: V,
+    // 8 x 32 heads x 128 x 4096 tokens 295 -> 173 MB, 71 -> 60 us; 4 x 32 x 96 x 32 768: K 757 -> 603 MB, 260 -> 238 us, V 798 ->
+    // 483 MB, 182 -> 164 us; K, 2 x 32 x 64 x 8192: 41 -> 39 us.
+    constexpr int STEP = FRONT == 1 ? 2 : ND == 24 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
+    static_assert(KVC_ONCE_GROUP_TILES % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
+    const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
     const int tiles = (int)a.tiles;
     const uint32_t base = a.status[KVC_ONCE_BASE_WORD];
     uint32_t err = 0, max_tile = 0, longest = 0, next_off = 0;
@@ -1551,7 +1559,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     first.in_group = 0;
 #pragma unroll 1
     for (int it = 0; it < run; it++) {
-        const int tile = tile0 + it;
+        const int tile = tile0 + STEP * it;
         if (tile >= tiles) break;
         int lane = tid & 63;                               // (opaque, as in kvc_encode_once_kernel)
         asm volatile("" : "+v"(lane));
@@ -1616,17 +1624,30 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
             kept++;
         }
         // Images wait for the run's other tiles, unless they reach to where those are to be staged.
-        const bool more = it + 1 < run && tile + 1 < tiles;
+        const bool more = it + 1 < run && tile + STEP < tiles;
         if (!fits || !more || kept_words * 4u > (uint32_t)(a.wave_bytes - STAGE)) {
-            const int oldest = tile + (fits ? 1 : 0) - kept;
+            const int oldest = tile + STEP * ((fits ? 1 : 0) - kept);
             uint32_t at = 0;
+            // the sizes of the other waves' tiles that lie in between: those in front of the k-th kept tile from lane k OTHERS on
+            const uint64_t *between_at = reinterpret_cast<const uint64_t *>(a.block_infos) + oldest + STEP * (lane / OTHERS) - 1 - lane % OTHERS;
+            const bool between = STEP > 1 && lane < OTHERS * kept && (lane >= OTHERS || placed);
+            uint64_t between_word = between ? kvc_status_load(between_at) : 0ull;
 #pragma unroll 1
             for (int k = 0; k < kept; k++) {               // one look-back (none behind tiles that have been placed), the others follow
                 KvcOncePending which = first;
-                which.tile = oldest + k;
+                which.tile = oldest + STEP * k;
                 which.bn = (uint32_t)(kept_bytes >> (16 * k)) & 0xffffu;
                 which.packs = which.bn <= (uint32_t)KVC_MAX_TILE_BYTES;
                 uint32_t off = 0;
+                if (STEP > 1 && placed) {
+                    while (__any((uint32_t)(between_word >> 48) == KVC_BI_NOT_READY) && ++polls <= a.max_polls) {
+                        __builtin_amdgcn_s_sleep(2);
+                        if (between) between_word = kvc_status_load(between_at);
+                    }
+#pragma unroll
+                    for (int i = 0; i < OTHERS; i++)
+                        next_off += (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(between_word >> 32), k * OTHERS + i) & 0xffffu;
+                }
                 err |= kvc_once_place(a, which, area + at, base, lane, &polls, &off, placed, next_off);
                 at += which.packs ? kvc_once_image_words(which.bn) : 0u;
                 next_off = off + which.bn;
@@ -1959,8 +1980,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
                           (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 64);
         const int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
-        // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (a run stays inside a group, or
-        // the wave that speaks for a group would wait before all its tiles are counted).
+        // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
+        // together take stays inside a group, or the wave that speaks for a group would wait before all its tiles are counted).
         if (wide && small && run == 2 && want == 1 && !is_k && a.tiles >= 16384 && 3 * (a.encoded_cap / a.tiles * 9 / 8) <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) run = 4;
         const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
         const auto symbols_kernel = !is_k ? kvc_encode_symbols_kernel<1, 32> :

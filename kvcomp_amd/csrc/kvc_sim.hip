@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_in_place_channel_kernel(KvcInPlace
 // first and then quantized in place, a prompt's keys went over the bus twice more).  A workgroup takes a (batch entry, head,
 // block): sixteen bytes of a token and their partners per load; the rotated block lies in LDS for the channels' minima and
 // maxima, and stays in registers to be quantized.  Bound by HBM: K of 4 x 32 heads x 128 x 2048 tokens 35 us (134 MB), V, whose
-// tokens are read where they come from, 26; appended first and then quantized in place the two took 113.  A cache update with
+// tokens are read where they come from, 26; appended first (43) and then quantized in place (28 and 29) the two took 99.  A cache update with
 // that prompt and two more tokens: 110 -> 72 us; with 32 more the host's calls take longer than the prompt (576 -> 570).
 template <int ITEMS>
 __global__ void __launch_bounds__(KVC_WG) kvc_append_channel_kernel(kvc_append_job a, int NB, float eb)
