@@ -321,6 +321,43 @@ __device__ __forceinline__ void kvc_stage_k_wide(int lane, uint8_t *s_stage, con
     }
 }
 
+// Vectors of 72 symbols, whose rows start at multiples of eight bytes: nine lanes of eight symbols cover a token's run, seven
+// tokens a load instruction, in two parts through the area (rows 18 words apart: no conflicts).
+constexpr int KVC_K72_PIECES = 9, KVC_K72_PER = KVC_WAVE / KVC_K72_PIECES, KVC_K72_LOADS = (KVC_WAVE + KVC_K72_PER - 1) / KVC_K72_PER;
+typedef uint32_t kvc_u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void kvc_front_k72(const KvcEncodeArgs &a, int64_t tile, int lane, uint8_t *s_stage, uint32_t (&v)[32])
+{
+    constexpr int PIECES = KVC_K72_PIECES, PER = KVC_K72_PER, HALF = KVC_K72_LOADS / 2;
+    static_assert(KVC_K72_LOADS % 2 == 0 && HALF * PER * PIECES * 8 <= KVC_STAGE_VSYM_BYTES, "half the loads fit the area");
+    const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
+    const int r = lane / PIECES, piece = lane - r * PIECES;
+    const uint8_t *p = a.sym + (row * KVC_WAVE + r) * a.stride + col * (8 * PIECES) + 8 * piece;
+    kvc_u32x2 q[2 * HALF];
+#pragma unroll
+    for (int i = 0; i < 2 * HALF; i++) {
+        const bool mine = r < PER && r + PER * i < KVC_WAVE;       // (else what another lane loads)
+        q[i] = *reinterpret_cast<const kvc_u32x2 *>(p + (mine ? (int64_t)(PER * i) * a.stride : -(int64_t)r * a.stride));
+    }
+    kvc_u32x2 *area = reinterpret_cast<kvc_u32x2 *>(s_stage);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int i = 0; i < HALF; i++)
+            if (r < PER) area[(r + PER * i) * PIECES + piece] = q[HALF * h + i];
+        kvc_wave_lds_sync();
+        const int mine = lane - HALF * PER * h;
+        if (mine >= 0 && mine < HALF * PER) {
+#pragma unroll
+            for (int j = 0; j < PIECES; j++) {
+                const kvc_u32x2 w = area[mine * PIECES + j];
+                v[2 * j] = w.x;
+                v[2 * j + 1] = w.y;
+            }
+        }
+        kvc_wave_lds_sync();
+    }
+}
+
 // V: four lanes cover a token's 64 symbols, a lane has eight consecutive tokens of sixteen channels; four tokens of four
 // channels are transposed in registers.  The area holds a quarter of the tile at a time (tokens 0 .. 3 of every eight of the
 // first 64, then of the others, then 4 .. 7), as [channel][8 words]: the less it takes, the more images can wait beside it.
@@ -1400,7 +1437,7 @@ __global__ void __launch_bounds__(KVC_WG, 3) kvc_encode_once_kernel(KvcStoreArgs
     }
 }
 
-// ---- one pass from symbols: vectors of 64, 96 or 128 of them, one codebook of short codes, 16-byte aligned symbols and rows --
+// ---- one pass from symbols: vectors of 64, 72, 96 or 128 of them, one codebook of short codes, 16-byte aligned symbols and rows --
 //
 // What kvc_encode_once_kernel<0> does, in fewer instructions and with less waiting inside a tile.  That kernel does not know
 // the vector's length when it is compiled: a branch per register of symbols made the wave wait for the LDS 32 times per tile
@@ -1422,6 +1459,7 @@ typedef __attribute__((address_space(3))) uint64_t kvc_lds_u64;
 template <bool PAIRS, int ND, int STEP>
 __device__ __forceinline__ uint32_t kvc_join_vector(const uint2 *s_table, uint32_t (&v)[32], uint32_t (&gl)[8])
 {
+    static_assert(ND % STEP == 0 && ND % 2 == 0, "whole steps");
     uint32_t bits = 0, over = 0;
     uint32_t table_at = (uint32_t)(uintptr_t)(const kvc_lds_u64 *)s_table;
 #pragma unroll
@@ -1537,12 +1575,12 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     kvc_load_pair_table(a, s_table, pairs);
     if (tid == 0) { s_err = 0; s_max_tile = 0; s_longest = 0; s_polls = 0; s_ticket = ticket; }
     __syncthreads();
-    // Neighbouring tiles share the cache lines that their symbols come in (V and head_dim 64: 64 bytes of each token's row, 96: 96),
+    // Neighbouring tiles share the cache lines that their symbols come in (V and head_dim 64: 64 bytes of each token's row, 96: 96, 72: 72),
     // and the lines of all waves are more than an L2 holds.  So STEP waves, whose tiles of one moment are whole lines, take the
     // tiles of all their runs in turn, and their loads meet.  (A group is a multiple of what they take.)  HBM traffic and time: V,
     // 8 x 32 heads x 128 x 4096 tokens 295 -> 173 MB, 71 -> 60 us; 4 x 32 x 96 x 32 768: K 757 -> 603 MB, 260 -> 238 us, V 798 ->
     // 483 MB, 182 -> 164 us; K, 2 x 32 x 64 x 8192: 41 -> 39 us.
-    constexpr int STEP = FRONT == 1 ? 2 : ND == 24 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
+    constexpr int STEP = FRONT == 1 ? 2 : ND == 24 || ND == 18 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
     static_assert(KVC_ONCE_GROUP_TILES % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
     const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
     const int tiles = (int)a.tiles;
@@ -1565,7 +1603,9 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         asm volatile("" : "+v"(lane));
         const KvcEncodeArgs &a = kvc_kernarg_again<KvcEncodeArgs>();
         uint32_t v[32];
-        {
+        if constexpr (ND == 18) {
+            kvc_front_k72(a, tile, lane, s_stage, v);
+        } else {
             kvc_u32x4 q[8];
             if constexpr (FRONT == 0) {
                 kvc_load_k_wide<ND>(a, tile, lane, q);
@@ -1576,8 +1616,8 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
             }
         }
         uint32_t bits = 0, gl[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};     // the joined lengths of registers 4 i .. 4 i + 3
-        if (pairs) bits = kvc_join_vector<true, ND, 8>(s_table, v, gl);
-        else bits = kvc_join_vector<false, ND, 4>(s_table, v, gl);
+        if (pairs) bits = kvc_join_vector<true, ND, ND % 8 == 0 ? 8 : 6>(s_table, v, gl);
+        else bits = kvc_join_vector<false, ND, ND % 4 == 0 ? 4 : 6>(s_table, v, gl);
         const bool bad = bits >= KVC_NO_CODE_LEN;          // a symbol without a code: the lane emits nothing
         if (bad) bits = 0;
         const uint32_t bytes = (bits + 7u) >> 3, end = kvc_wave_inclusive_scan(bytes), start = end - bytes;
@@ -1972,12 +2012,13 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         int run = want == 1 ? (a.tiles >= 8192 ? 2 : 1) : want - 1;       // 2, 3: always one, two tiles per wave
         run = run < 1 ? 1 : run > 2 ? 2 : run;
         if (a.rows_per_codebook != 0) run = 1;
-        // Vectors of 128, 96 and 64 symbols with codes known to be short have a kernel of their own where the alignment is for
+        // Vectors of 128, 96, 72 and 64 symbols with codes known to be short have a kernel of their own where the alignment is for
         // sixteen symbols per load.  It takes
         // eight waves per workgroup where they get little LDS (two such workgroups per compute unit): half as many tickets, of
         // which the chip hands out one in 11 ns.
-        const bool wide = front == 0 && a.rows_per_codebook == 0 && c.longest_code >= 1 && c.longest_code <= 8 && ((uintptr_t)c.d_sym & 15) == 0 && c.stride % 16 == 0 &&
-                          (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 64);
+        const int unit = a.vec_len == 72 ? 8 : 16;         // symbols per load (head_dim 72: rows start at multiples of eight)
+        const bool wide = front == 0 && a.rows_per_codebook == 0 && c.longest_code >= 1 && c.longest_code <= 8 && (uintptr_t)c.d_sym % unit == 0 && c.stride % unit == 0 &&
+                          (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 72 || a.vec_len == 64);
         const int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
         // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
@@ -1986,7 +2027,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
         const auto symbols_kernel = !is_k ? kvc_encode_symbols_kernel<1, 32> :
                                     a.vec_len == 128 ? kvc_encode_symbols_kernel<0, 32> :
-                                    a.vec_len == 96 ? kvc_encode_symbols_kernel<0, 24> : kvc_encode_symbols_kernel<0, 16>;
+                                    a.vec_len == 96 ? kvc_encode_symbols_kernel<0, 24> :
+                                    a.vec_len == 72 ? kvc_encode_symbols_kernel<0, 18> : kvc_encode_symbols_kernel<0, 16>;
         if (wide) {
             hipLaunchKernelGGL(symbols_kernel, dim3(wgs1), dim3(waves * KVC_WAVE), lds, stream, sa.e, run);
             hipLaunchKernelGGL(kvc_encode_finish_kernel<0>, dim3(1), dim3(KVC_WG), 0, stream, sa);

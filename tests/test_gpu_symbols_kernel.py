@@ -59,7 +59,8 @@ CASES = [(True, 64, 1, 1, 128, 13, 7), (True, 128, 1, 5, 96, 16, 8), (True, 192,
          (False, 384, 1, 3, 128, 23, 8), (True, 64 * 33, 8, 32, 64, 13, 7), (True, 64 * 43, 6, 32, 96, 11, 6), (True, 64 * 33, 8, 32, 128, 16, 8),
          (False, 128 * 17, 4, 32, 256 // 2, 8, 7), (False, 128 * 65, 8, 32, 64, 7, 6), (False, 128 * 33, 8, 32, 128, 8, 5), (False, 128 * 33, 8, 32, 128, 20, 8),
          (False, 128 * 129, 1, 65, 64, 7, 5), (False, 128 * 253, 1, 65, 64, 7, 5),
-         (True, 64 * 127, 1, 65, 64, 7, 5), (True, 64 * 127, 1, 65, 96, 9, 6), (True, 64 * 129, 1, 66, 96, 9, 6)]   # last tiles without all their neighbours
+         (True, 64 * 127, 1, 65, 64, 7, 5), (True, 64 * 127, 1, 65, 96, 9, 6), (True, 64 * 129, 1, 66, 96, 9, 6),
+         (True, 64, 1, 1, 72, 13, 7), (True, 192, 1, 3, 72, 17, 8), (True, 64 * 43, 6, 32, 72, 11, 6), (True, 64 * 129, 1, 66, 72, 23, 8)]   # last tiles without all their neighbours
 
 
 @pytest.mark.parametrize("rare_tiles", [0.0, 0.15])
