@@ -2019,11 +2019,16 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         const int unit = a.vec_len == 72 ? 8 : 16;         // symbols per load (head_dim 72: rows start at multiples of eight)
         const bool wide = front == 0 && a.rows_per_codebook == 0 && c.longest_code >= 1 && c.longest_code <= 8 && (uintptr_t)c.d_sym % unit == 0 && c.stride % unit == 0 &&
                           (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 72 || a.vec_len == 64);
+        // Its 4096 waves at a time: runs of two from where single tiles would be a second, part-filled round of them.  K and
+        // V of 2 x 32 heads x 128 x 6144 tokens (6144 tiles): 58 -> 42 and 56 -> 39 us; K of 4 x 24 x 72 x 4096: 53 -> 37.
+        // (V's runs of four begin where those of two would be a second round: 2 x 32 x 128 x 12 288 tokens 64 -> 57 us.)
+        constexpr int KVC_WIDE_WAVES = 4096;
+        if (wide && small && want == 1 && a.tiles > KVC_WIDE_WAVES) run = 2;
         const int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
         // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
         // together take stays inside a group, or the wave that speaks for a group would wait before all its tiles are counted).
-        if (wide && small && run == 2 && want == 1 && !is_k && a.tiles >= 16384 && 3 * (a.encoded_cap / a.tiles * 9 / 8) <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) run = 4;
+        if (wide && small && run == 2 && want == 1 && !is_k && a.tiles > 2 * KVC_WIDE_WAVES && 3 * (a.encoded_cap / a.tiles * 9 / 8) <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) run = 4;
         const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
         const auto symbols_kernel = !is_k ? kvc_encode_symbols_kernel<1, 32> :
                                     a.vec_len == 128 ? kvc_encode_symbols_kernel<0, 32> :
