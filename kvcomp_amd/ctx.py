@@ -13,6 +13,7 @@ get_only_compressed, get_decode_quant_ints, mat_vec_mul, build_codebook, get_cr)
 """
 import ast
 import collections
+import contextlib
 import ctypes as C
 import itertools
 import math
@@ -184,9 +185,16 @@ class _Outcome:
         self._seen[9] = 0
 
     def ask(self, stream: int) -> Tuple[int, int]:
-        """What the next encode on `stream` is to be told."""
+        """What the next encode on `stream` is to be told; if the library refuses it, refused() has to follow."""
         self.number, self.stream = (next(_Outcome._numbers) & 0x7fffffff) or 1, stream
         return self.words.data_ptr(), self.number
+
+    def refused(self, number: int, stream: int):
+        """The encode that was told the latest number has failed, and nothing of it is queued any more: whoever waits for an
+        earlier one goes on waiting for its `number` on `stream`.  (A call can fail behind its launches, for an error that
+        something else had left; its number is there then, and its words are the newer ones.)"""
+        if not self.query():
+            self.number, self.stream = number, stream
 
     def query(self) -> bool:
         return int(self._seen[9]) == self.number
@@ -630,14 +638,22 @@ class KVCompCtx:
                 self._sync_sizes()
             self._encoded.reserve(worst, (), torch.uint8, self.device, self._enc_pending)
         outcome = self._ask_outcome()
+        before = None if outcome is None else (outcome.number, outcome.stream)
         told = None if outcome is None else outcome.ask(_lib.stream_of(state))
-        if prepared is not None:
-            kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told, longest_code)
-        else:
-            kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
-                                     table_bytes=table_bytes, block_infos=bi, thread_infos=ti, encoded=self._encoded.data,
-                                     symbols=symbols, cache=cache, quant_mask=mask, eb=self.quant_scale_rel, min_ints=mn, scales=sc,
-                                     stream_bytes=state[8:9], result=state[:8], outcome=told)
+        try:
+            if prepared is not None:
+                kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told, longest_code)
+            else:
+                kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
+                                         table_bytes=table_bytes, block_infos=bi, thread_infos=ti, encoded=self._encoded.data,
+                                         symbols=symbols, cache=cache, quant_mask=mask, eb=self.quant_scale_rel, min_ints=mn, scales=sc,
+                                         stream_bytes=state[8:9], result=state[:8], outcome=told)
+        except BaseException:
+            if outcome is not None:
+                with contextlib.suppress(RuntimeError):        # (the words must not go while a part of the call may write them)
+                    torch.cuda.current_stream(self.device).synchronize()
+                outcome.refused(*before)
+            raise
         self._block_infos.used += sizes[0]
         self._thread_infos.used += sizes[1]
         self._min_ints.used += nb

@@ -1,0 +1,126 @@
+"""What a context learns of its queued stores where something else goes wrong or differs: a later call that the library refuses,
+streams other than the one its buffers came from, buffers that grow meanwhile."""
+import struct
+import types
+
+import pytest
+import torch
+
+from kvcomp_amd import _lib, kvcomp_cuda
+from kvcomp_amd._lib import KvcompError
+from kvcomp_amd.ctx import KVCompCacheConfig, KVCompCacheConfigStatic, KVCompCtx, QuantMode, _Outcome
+
+DEV = "cuda:0"
+
+
+def _config():
+    KVCompCacheConfigStatic.config = KVCompCacheConfig("t", QuantMode.ChannelQuant, QuantMode.TokenQuant, 64, 128, 64, 128, 0.1, 0.2)
+
+
+def _ordinary_words():
+    """An _Outcome in ordinary memory: the test writes what a kernel would."""
+    outcome = object.__new__(_Outcome)
+    outcome.words = torch.zeros(16, dtype=torch.int32)
+    outcome._seen, outcome.number, outcome.stream = outcome.words.numpy(), 0, 0
+    return outcome
+
+
+@pytest.fixture
+def queued(monkeypatch):
+    """A context with one queued store of 384 tokens through a library that queues nothing, and the list of what its encodes
+    were told; an encode fails while `refuse` is not empty."""
+    _config()
+    ctx, told, refuse = KVCompCtx(True, 1, 2, 64, 0.1), [], []
+    ctx.async_store, ctx._outcome = True, _ordinary_words()
+    book = _lib.Codebook(tree_format=5, max_code_bits=7, payload_bits=8 * 100000)
+
+    def encode(is_k, *, tokens, block_infos, outcome, **kw):
+        if refuse:
+            raise KvcompError("the library refuses the call")
+        for i in range(tokens // 64 * 2):
+            block_infos[8 * i:8 * i + 8] = torch.frombuffer(bytearray(struct.pack("<IHH", 700 * i, 700, 0)), dtype=torch.uint8)
+        told.append(outcome)
+    monkeypatch.setattr(kvcomp_cuda, "quant_codebook", lambda x, *a: (x.to(torch.uint8), book))
+    monkeypatch.setattr(kvcomp_cuda, "put_codebook", lambda *a: tuple(torch.zeros(24, dtype=torch.uint8) for _ in range(3)))
+    monkeypatch.setattr(kvcomp_cuda, "encode_async", encode)
+    monkeypatch.setattr(KVCompCtx, "_ask_outcome", lambda self: self._outcome)
+    monkeypatch.setattr(_lib, "stream_of", lambda t: 11)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: types.SimpleNamespace(synchronize=lambda: None))
+    x = torch.arange(512 * 128, dtype=torch.float32).remainder(50).reshape(512, 1, 2, 64).to(torch.float16)
+    ctx._encoded.reserve(1 << 20, (), torch.uint8, torch.device("cpu"))
+    ctx.store(x[:384], want_symbols=False)
+    assert len(ctx._unverified) == 1 and ctx._probe is not None
+    return ctx, told, refuse, x
+
+
+def _arrives(outcome, number, used, largest):
+    outcome.words[2], outcome.words[3], outcome.words[8], outcome.words[9] = largest, 40, used, number
+
+
+@pytest.mark.parametrize("arrives", ["before", "behind"])
+def test_a_refused_encode_does_not_hide_the_outcome_of_an_earlier_one(queued, arrives):
+    ctx, told, refuse, x = queued
+    if arrives == "before":
+        _arrives(ctx._outcome, told[0][1], 12 * 700, 700)
+        ctx._probe, probe = None, ctx._probe                      # (store() would take note of it at once)
+    refuse.append(True)
+    with pytest.raises(KvcompError, match="refuses"):
+        ctx.store(x[384:], want_symbols=False)
+    if arrives == "before":
+        ctx._probe = probe
+    else:
+        assert not ctx._outcome.query() and ctx._outcome.stream == 11
+        _arrives(ctx._outcome, told[0][1], 12 * 700, 700)
+    assert ctx._outcome.query()
+    ctx.poll_stores()
+    assert not ctx._unverified and ctx._enc_pending == 0 and ctx._encoded.used == 12 * 700 and ctx.max_tile_bytes == 700
+    seen = ctx._outcome._seen
+    ctx._outcome = ctx._probe = None
+    assert not any(words is seen for words, _ in _Outcome._late)  # nothing is still to come
+    refuse.clear()
+    ctx._outcome = _ordinary_words()
+    ctx.store(x[384:], want_symbols=False)                        # the refused store, again
+    assert ctx.ctx_len == 512 and len(ctx._unverified) == 1 and told[1][1] == ctx._outcome.number != told[0][1]
+
+
+def test_a_refused_encode_whose_last_kernel_ran_all_the_same():
+    outcome = _ordinary_words()
+    first = outcome.ask(11)[1]
+    second = outcome.ask(11)[1]
+    outcome.words[9] = second
+    outcome.refused(first, 11)
+    assert outcome.query() and outcome.number == second
+
+
+def _store_all(is_k, parts, refuse_behind=()):
+    B, H, D = parts[0].shape[1:]
+    ctx = KVCompCtx(is_k, B, H, D, 0.1)
+    ctx.codebook_smoothing = ctx.async_store = True
+    for i, x in enumerate(parts):
+        ctx.store(x, want_symbols=False)
+        if i in refuse_behind:
+            ctx.quant_scale_rel = 0.0
+            probe, ctx._probe = ctx._probe, None                  # as if nothing of the queued stores had arrived when store() looked
+            with pytest.raises(KvcompError, match="error bound"):
+                ctx.store(x, want_symbols=False)
+            ctx.quant_scale_rel, ctx._probe = 0.1, probe
+    return ctx
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("is_k", [True, False])
+def test_stores_around_a_refused_one(is_k):
+    from tests import _synth as S
+    _config()
+    x = (S.synth_k if is_k else S.synth_v)(1280, 2, 4, 128).to(DEV)
+    parts = [x[:512], x[512:640], x[640:1024], x[1024:]]
+    want, got = _store_all(is_k, parts), _store_all(is_k, parts, (0, 1, 2))
+    got.poll_stores()                                             # nobody waits: what has arrived is found
+    torch.cuda.synchronize()
+    for _ in parts:
+        got.poll_stores()
+    assert not got._unverified and got._enc_pending == 0
+    assert got.ctx_len == want.ctx_len == 1280 and got.compressed_ctx_len == want.compressed_ctx_len
+    for name in ("encoded_data", "block_infos", "thread_infos", "quant_min_ints", "quant_scales", "buffer"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
