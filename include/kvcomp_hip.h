@@ -241,8 +241,11 @@ int kvc_encode_async(const kvc_encode_job *job, void *stream);
  * kvc_encode_queue: kvc_encode_async, continuing what was prepared on the same stream for the same tokens and outputs
  *   (prepared = 0: nothing was; d_scratch is not used then).  longest_code: bits of the longest code in the (one) encode
  *   table, 0 if not known; symbols with longer codes are errors.  h_outcome, if not NULL: 16 words of pinned host memory that
- *   receive d_result's eight words, *d_stream_bytes and, last, outcome_number (word 9), as the call ends on the device.
- * kvc_wait_outcome: waits until outcome_number has arrived in such words. */
+ *   receive d_result's eight words, *d_stream_bytes and, last, outcome_number (word 9), as the call ends on the device; words
+ *   10 - 12 are set to the stream (low half, high half) and the device before an accepted call returns.
+ * kvc_wait_outcome: waits until outcome_number has arrived in such words.  If it has not come after two seconds and
+ *   everything queued on their stream has run, it returns too, with word 9 saying that the number has not come; the stream
+ *   must exist as long.  No other stream is waited for, and the current device does not matter. */
 int64_t kvc_encode_scratch_bytes(void);
 int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream);
 int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,

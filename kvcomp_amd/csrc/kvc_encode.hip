@@ -2258,8 +2258,16 @@ extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int 
         }
         c.src = &src;
     }
+    int dev = 0;
+    if (h_outcome) KVC_HIP(hipGetDevice(&dev));
     void *slot;
-    return kvc_encode_launch(c, &slot, (hipStream_t)stream);
+    if (int rc = kvc_encode_launch(c, &slot, (hipStream_t)stream)) return rc;
+    if (h_outcome) {                                       // for kvc_wait_outcome: where the number is to come from
+        h_outcome[10] = (uint32_t)(uintptr_t)stream;
+        h_outcome[11] = (uint32_t)((uintptr_t)stream >> 32);
+        h_outcome[12] = (uint32_t)dev;
+    }
+    return 0;
 }
 
 extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream) { return kvc_encode_queue(job, nullptr, KVC_ENC_FRESH, 0, nullptr, 0u, stream); }

@@ -110,20 +110,46 @@ static int wait_for_counts(const CountBlock &b, hipStream_t stream)
     return 0;
 }
 
+// Whether everything on the stream that words 10 - 12 of an outcome name has run.  Nothing is asked of a stream that is being
+// recorded (what was queued before that is still on its way), and a runtime that will not answer during a recording has not said yes.
+static int outcome_stream_is_idle(const uint32_t *h_outcome, bool *idle)
+{
+    hipStream_t stream = (hipStream_t)(uintptr_t)(h_outcome[10] | (uint64_t)h_outcome[11] << 32);
+    *idle = false;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (stream) KVC_HIP(hipStreamIsCapturing(stream, &capturing));
+    if (capturing != hipStreamCaptureStatusNone) return 0;
+    int here = 0;
+    KVC_HIP(hipGetDevice(&here));
+    KVC_HIP(hipSetDevice((int)h_outcome[12]));             // (the default stream is the current device's)
+    const hipError_t e = hipStreamQuery(stream);
+    if (e != hipSuccess) (void)hipGetLastError();          // "not ready" is no error of anyone's
+    KVC_HIP(hipSetDevice(here));
+    *idle = e == hipSuccess;
+    return e == hipErrorNotReady || e == hipErrorStreamCaptureImplicit || e == hipErrorStreamCaptureUnsupported ? 0 : kvc_check_hip(e, "hipStreamQuery");
+}
+
+// Looks at the words alone for two seconds (an encode takes 0.01 to 2 ms); from then on also at their stream, ten times a
+// second, so that a number which never comes does not hold the caller.  Other streams are never waited for.
 extern "C" int kvc_wait_outcome(const uint32_t *h_outcome, uint32_t outcome_number)
 {
     KVC_REQUIRE(h_outcome != nullptr, "NULL argument");
     const auto began = std::chrono::steady_clock::now();
+    auto ask = began + std::chrono::seconds(2);
     for (;;) {
         for (int i = 0; i < 256; i++) {
             if (__atomic_load_n(&h_outcome[9], __ATOMIC_ACQUIRE) == outcome_number) return 0;
             __builtin_ia32_pause();
         }
-        const auto waited = std::chrono::steady_clock::now() - began;
-        if (waited > std::chrono::seconds(2)) break;
-        if (waited > std::chrono::milliseconds(5)) std::this_thread::sleep_for(std::chrono::microseconds(20));
+        const auto now = std::chrono::steady_clock::now();
+        if (now > ask) {
+            bool idle;
+            if (int rc = outcome_stream_is_idle(h_outcome, &idle)) return rc;
+            if (idle) return 0;
+            ask = now + std::chrono::milliseconds(100);
+        }
+        if (now - began > std::chrono::milliseconds(5)) std::this_thread::sleep_for(std::chrono::microseconds(20));
     }
-    return kvc_check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");     // (the stream it was queued on may be gone)
 }
 
 extern "C" int kvc_quant_counted(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,

@@ -200,6 +200,7 @@ class _Outcome:
         return int(self._seen[9]) == self.number
 
     def synchronize(self):
+        """Until the number is there; if its stream runs dry without it, query() says so."""
         _lib.check(_lib.lib().kvc_wait_outcome(self.words.data_ptr(), self.number))
 
     def __del__(self):

@@ -1,6 +1,7 @@
 """What a context learns of its queued stores where something else goes wrong or differs: a later call that the library refuses,
 streams other than the one its buffers came from, buffers that grow meanwhile."""
 import struct
+import time
 import types
 
 import pytest
@@ -124,3 +125,75 @@ def test_stores_around_a_refused_one(is_k):
     assert got.ctx_len == want.ctx_len == 1280 and got.compressed_ctx_len == want.compressed_ctx_len
     for name in ("encoded_data", "block_infos", "thread_infos", "quant_min_ints", "quant_scales", "buffer"):
         assert torch.equal(getattr(got, name), getattr(want, name)), name
+
+
+def _busy(stream, seconds):
+    """Keep a stream busy for about that long, with a kernel that counts clock ticks."""
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(1000)
+        start.record()
+        torch.cuda._sleep(100000)
+        end.record()
+        end.synchronize()
+        torch.cuda._sleep(int(100000 * seconds * 1e3 / start.elapsed_time(end)))
+        end.record()
+    return end
+
+
+@pytest.mark.gpu
+def test_a_number_that_never_comes_is_waited_for_on_its_own_stream_alone():
+    from tests import _synth as S
+    _config()
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    x = S.synth_k(512, 1, 2, 64).to(DEV)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        ctx = _store_all(True, [x])
+    outcome = ctx._outcome
+    outcome.synchronize()
+    words = [w & 0xffffffff for w in outcome.words.tolist()]
+    assert outcome.query() and words[10] | words[11] << 32 == side.cuda_stream == outcome.stream and words[12] == torch.cuda.current_device()
+    there = outcome.number
+    end = _busy(other, 6.0)
+    began = time.monotonic()
+    outcome.number = there + 1                                    # as if a call had been told so
+    outcome.synchronize()
+    waited = time.monotonic() - began
+    assert not outcome.query() and not end.query() and 1.9 < waited < 4.0
+    outcome.number = there
+    end.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("is_k", [True, False])
+def test_stores_on_a_stream_are_learnt_of_on_another(is_k):
+    """Queued behind a long kernel on a stream of their own; asked for on the default stream, which is ordered behind nothing."""
+    from tests import _synth as S
+    _config()
+    x = (S.synth_k if is_k else S.synth_v)(1280, 2, 4, 128).to(DEV)
+    parts = [x[:512], x[512:640], x[640:1024], x[1024:]]
+    want = _store_all(is_k, parts)
+    expect = {name: getattr(want, name).clone() for name in ("encoded_data", "block_infos", "thread_infos", "quant_min_ints", "quant_scales", "buffer")}
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        got = _store_all(is_k, parts[:2])
+        _busy(first, 0.2)
+        got.store(parts[2], want_symbols=False)
+        outcome = got._outcome
+        assert not outcome.query() and got._probe[0] is outcome and got._probe[2] == first.cuda_stream
+    second.wait_stream(first)
+    with torch.cuda.stream(second):                               # the words are another stream's: this store has none to write to
+        got.store(parts[3], want_symbols=False)
+        assert got._outcome is outcome and got._probe[1] == len(got._unverified) - 1
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(kvcomp_cuda, "encode_result", None)             # what the words say is enough for the first three
+        outcome.synchronize()
+        got.poll_stores()
+    assert len(got._unverified) == 1
+    second.synchronize()
+    assert got.ctx_len == 1280
+    for name, value in expect.items():
+        assert torch.equal(getattr(got, name), value), name
+    assert not got._unverified
