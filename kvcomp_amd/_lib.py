@@ -164,6 +164,13 @@ def stream_of(t) -> int:
     return torch._C._cuda_getCurrentRawStream(index)
 
 
+def let_go(t):
+    """To be called before the last reference to `t` goes while kernels queued on the current stream may still use its memory:
+    that may have come from another stream, to which the allocator would hand it back at once."""
+    if t is not None and t.is_cuda:
+        t.record_stream(torch.cuda.current_stream(t.device))
+
+
 class KvcompError(RuntimeError):
     pass
 

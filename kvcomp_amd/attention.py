@@ -111,6 +111,7 @@ class CompressedAttention:
         if key != self._workspace_key:
             need = int(L.kvc_attention_workspace_bytes(key[0] * 1024, key[0] * 1024, B, Hq, D))
             if self._workspace is None or self._workspace.numel() < need or self._workspace.device != q.device:
+                _lib.let_go(self._workspace)
                 self._workspace = torch.empty(need + need // 4, dtype=torch.uint8, device=q.device)
             self._workspace_key = key
         if out is None:

@@ -26,6 +26,7 @@ from typing import Any, Dict, List, Optional, Tuple
 
 import torch
 
+from . import _lib
 from .compute import append_dense, append_quantized, apply_rotary_pos_emb_single, blocks_to_compress, quant_in_place, safe_cat, takes_append
 from .ctx import KVCompCacheConfigStatic, KVCompCtx
 
@@ -59,6 +60,7 @@ class _DenseHistory:
             grown = torch.empty(t.shape[0], t.shape[1], cap, t.shape[3], dtype=t.dtype, device=t.device)
             if self.data is not None:
                 grown[:, :, :self.length].copy_(self.data[:, :, :self.length])
+                _lib.let_go(self.data)
             self.data = grown
 
     def append(self, t: torch.Tensor):

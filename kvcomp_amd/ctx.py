@@ -115,6 +115,7 @@ class _Growable:
         self.row = 1              # elements per row of `data`
 
     def _hold(self, data: torch.Tensor):
+        _lib.let_go(self.data)                                 # (copied from on this stream, and written to by queued encodes)
         self.data, self.row = data, math.prod(data.shape[1:])
 
     @property
@@ -375,6 +376,8 @@ class KVCompCtx:
             if self._tail_len:
                 rows.append(self._tail[:self._tail_len])
             self._tail = torch.cat(rows, dim=0)
+            for t in rows:
+                _lib.let_go(t)
             self._tail_len = self._tail.shape[0]
         if any(u.codebook for u in dropped):
             self.encode_codebook = self.decode_codebook = self._lut = self._lut_source = None
@@ -455,6 +458,7 @@ class KVCompCtx:
             grown = torch.empty((cap,) + tuple(cache.shape[1:]), dtype=cache.dtype, device=cache.device)
             if self._tail_len:
                 grown[:self._tail_len] = self._tail[:self._tail_len]
+            _lib.let_go(self._tail)
             self._tail = grown
         row = self._row_bytes
         to, src = self._tail.data_ptr() + self._tail_len * row, cache.data_ptr()

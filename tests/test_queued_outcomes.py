@@ -9,7 +9,7 @@ import torch
 
 from kvcomp_amd import _lib, kvcomp_cuda
 from kvcomp_amd._lib import KvcompError
-from kvcomp_amd.ctx import KVCompCacheConfig, KVCompCacheConfigStatic, KVCompCtx, QuantMode, _Outcome
+from kvcomp_amd.ctx import KVCompCacheConfig, KVCompCacheConfigStatic, KVCompCtx, QuantMode, _Growable, _Outcome
 
 DEV = "cuda:0"
 
@@ -197,3 +197,80 @@ def test_stores_on_a_stream_are_learnt_of_on_another(is_k):
     for name, value in expect.items():
         assert torch.equal(getattr(got, name), value), name
     assert not got._unverified
+
+
+class _FromAnotherStream:
+    """Stands for a tensor in device memory that came from another stream; notes the streams it is kept for."""
+    is_cuda = True
+
+    def __init__(self, data):
+        self._data, self.kept_for = data, []
+
+    def __getattr__(self, name):
+        return getattr(self._data, name)
+
+    def __getitem__(self, at):
+        return self._data[at]
+
+    def record_stream(self, stream):
+        self.kept_for.append(stream)
+
+
+@pytest.mark.parametrize("grow", [lambda g: g.reserve(400, (), torch.uint8, None, 32), lambda g: g.append(torch.zeros(400, dtype=torch.uint8)), lambda g: g.trim()])
+def test_a_buffer_that_is_replaced_is_kept_for_the_stream_that_uses_it(monkeypatch, grow):
+    """Queued encodes may still write to it, and the copy into the new one reads it."""
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: "the current stream")
+    g = _Growable()
+    g.append(torch.arange(200, dtype=torch.uint8))
+    g.used = 8
+    old = g.data = _FromAnotherStream(g.data)
+    grow(g)
+    assert g.data is not old and old.kept_for == ["the current stream"] and torch.equal(g.data[:8], torch.arange(8, dtype=torch.uint8))
+
+
+def test_other_memory_that_is_replaced_is_kept_for_the_stream_that_uses_it(monkeypatch):
+    from kvcomp_amd.cache import _DenseHistory
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: "the current stream")
+    h = _DenseHistory()
+    h.append(torch.ones(1, 2, 200, 8, dtype=torch.float16))
+    old = h.data = _FromAnotherStream(h.data)
+    h.append(torch.ones(1, 2, 1000, 8, dtype=torch.float16))
+    assert old.kept_for == ["the current stream"] and bool((h.view() == 1).all())
+    _config()
+    ctx = KVCompCtx(True, 1, 2, 64, 0.1)
+    ctx.store(torch.ones(20, 1, 2, 64, dtype=torch.float16))
+    old = ctx._tail = _FromAnotherStream(ctx._tail)
+    ctx._tail_append(torch.ones(200, 1, 2, 64, dtype=torch.float16))
+    assert old.kept_for == ["the current stream"] and bool((ctx.buffer == 1).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("is_k", [True, False])
+def test_a_context_of_one_stream_grows_on_another_with_stores_outstanding(is_k):
+    """The payload buffer comes from the default stream; queued encodes write to it on a busy side stream while it is
+    replaced.  Nothing that the default stream allocates then may lie where they write."""
+    from tests import _synth as S
+    _config()
+    x = (S.synth_k if is_k else S.synth_v)(1280, 2, 4, 128).to(DEV)
+    parts = [x[:512], x[512:640], x[640:768], x[768:896], x[896:1152], x[1152:]]
+    want = _store_all(is_k, parts)
+    expect = {name: getattr(want, name).clone() for name in ("encoded_data", "block_infos", "thread_infos", "quant_min_ints", "quant_scales", "buffer")}
+    got = _store_all(is_k, parts[:1])                             # on the default stream
+    got.encoded_data
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.default_stream())
+    growing, addresses, sizes = got._encoded, [got._encoded.address], [got._encoded.data.numel()]
+    with torch.cuda.stream(side):
+        end = _busy(side, 1.0)
+        for part in parts[1:]:
+            got.store(part, want_symbols=False)
+            if growing.address != addresses[-1]:
+                addresses.append(growing.address)
+                sizes.append(growing.data.numel())
+        assert len(addresses) > 2 and not end.query() and len(got._unverified) > 2 and got.waits == 2     # (the codebook, encoded_data)
+    other = [torch.full((n,), 0xA5, dtype=torch.uint8, device=DEV) for n in sizes]
+    assert not {t.data_ptr() for t in other} & set(addresses)
+    side.synchronize()
+    assert all(bool((t == 0xA5).all()) for t in other)
+    for name, value in expect.items():
+        assert torch.equal(getattr(got, name), value), name
