@@ -142,7 +142,7 @@ def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: floa
                    smoothed_symbols: int, meanwhile=None):
     """kvc_quant_codebook on a device fp16 [NB, BS, B, H, D] tensor: (symbols uint8 of the same shape, _lib.Codebook).
     min_ints (int8) and scales (fp16) receive the group parameters.  Waits for the symbol counts only; `meanwhile`, if given, is
-    called with the symbol tensor once the quantizer is queued."""
+    called with the symbol tensor between the call's halves (kvc_quant_counted, kvc_counted_codebook), the quantizer being queued."""
     _require(blocked.is_cuda and blocked.dtype == torch.float16 and blocked.dim() == 5 and blocked.is_contiguous(),
              "a contiguous device float16 tensor of shape [NB, BS, B, H, D] is expected")
     L = _lib.lib()
@@ -153,12 +153,14 @@ def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: floa
     book = _lib.Codebook()
     stream = _lib.stream_of(blocked)
     with _lib.device_guard(blocked):
+        args = (blocked.data_ptr(), *blocked.shape, quant_mask, float(quant_scale_rel), sym.data_ptr(), min_ints.data_ptr(), scales.data_ptr())
+        if meanwhile is None:
+            check(L.kvc_quant_codebook(*args, smoothed_symbols, C.byref(book), stream))
+            return sym, book
         counted = C.c_void_p(0)
-        check(L.kvc_quant_counted(blocked.data_ptr(), *blocked.shape, quant_mask, float(quant_scale_rel), sym.data_ptr(), min_ints.data_ptr(),
-                                  scales.data_ptr(), C.byref(counted), stream))
+        check(L.kvc_quant_counted(*args, C.byref(counted), stream))
         try:
-            if meanwhile is not None:
-                meanwhile(sym)
+            meanwhile(sym)
         finally:
             rc = L.kvc_counted_codebook(counted, smoothed_symbols, C.byref(book), stream)
         check(rc)
@@ -259,7 +261,7 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
     one table per `rows_per_codebook` tile rows, and return without waiting.  `result` (device int32[8], zeroed once)
     and `stream_bytes` (device int32[1]: payload bytes already in `encoded`, moved on by the call) stay on the device;
     encode_result() reads them.  The output tensors are written from their first element on.
-    outcome: (address of 16 words of pinned host memory, number), see kvc_encode_queue."""
+    outcome: (address of 16 words of pinned host memory, number); the call is kvc_encode_queue then."""
     job = _lib.EncodeJob()
     job.is_k, job.quant_mask, job.eb = int(is_k), int(quant_mask), float(eb)
     _require((symbols is None) != (cache is None), "give either symbols or cache")
@@ -304,9 +306,9 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
         job.d_stream_bytes = stream_bytes.data_ptr()
     if result is not None:
         job.d_result = result.data_ptr()
-    address, number = (0, 0) if outcome is None else outcome
     with _lib.device_guard(encoded):
-        check(_lib.lib().kvc_encode_queue(C.byref(job), 0, 0, 0, address, number, _lib.stream_of(encoded)))
+        L, stream = _lib.lib(), _lib.stream_of(encoded)
+        check(L.kvc_encode_async(C.byref(job), stream) if outcome is None else L.kvc_encode_queue(C.byref(job), 0, 0, 0, *outcome, stream))
 
 
 class PreparedEncode(NamedTuple):

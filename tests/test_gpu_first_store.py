@@ -71,3 +71,17 @@ def test_put_bytes_beyond_one_launch():
         out = torch.zeros(9010, dtype=torch.uint8, device=DEV)
         _lib.check(_lib.lib().kvc_put_bytes(C.c_void_p(out.data_ptr()), data[:n].tobytes(), n, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
         assert np.array_equal(out.cpu().numpy()[:n], data[:n]) and int(out[n:].max()) == 0
+
+
+@pytest.mark.parametrize("is_k,mask", [(True, "MASK_K_BLOCK"), (False, "MASK_V_TOKEN")])
+def test_one_call_and_its_halves_give_the_same_code(is_k, mask):
+    import kvcomp_amd.kvcomp_cuda as m
+    T, B, H, D = 256, 2, 3, 128
+    blocked = S.blocked((S.synth_k if is_k else S.synth_v)(T, B, H, D), 64 if is_k else 128).to(DEV)
+    results = []
+    for meanwhile in (None, lambda sym: None):
+        groups = m._lib.lib().kvc_quant_groups(*blocked.shape, getattr(m, mask))
+        mins, scales = torch.empty(groups, dtype=torch.int8, device=DEV), torch.empty(groups, dtype=torch.float16, device=DEV)
+        sym, book = m.quant_codebook(blocked, getattr(m, mask), 0.1, mins, scales, 13, meanwhile)
+        results.append((sym, mins, scales, bytes(book)))
+    assert all(torch.equal(a, b) for a, b in zip(results[0][:3], results[1][:3])) and results[0][3] == results[1][3]
