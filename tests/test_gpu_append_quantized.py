@@ -41,3 +41,38 @@ def test_what_it_does_not_take_is_left_alone():
         x = torch.randn(1, heads, 130, D, dtype=torch.float16, device=DEV)
         cache = torch.full_like(x, 3.0)
         assert not append_quantized(x, x, None, None, cache, cache, 0, k_plan, v_plan) and (cache == 3).all()
+
+
+@pytest.mark.parametrize("angles", [False, True])
+@pytest.mark.parametrize("D", [128, 96, 16])
+def test_special_values(D, angles):
+    """Channels whose minima and maxima are joined from parts: constant ones, zeros of both signs, infinities, NaN in one part,
+    in several and everywhere, the largest and the smallest values.  The same bits as the two steps (of a NaN, that it is one)."""
+    from kvcomp_amd.compute import QuantMode, append_dense, append_quantized, quant_in_place
+    B, H, T = 2, 3, 140
+    g = torch.Generator().manual_seed(D)
+    k, v = (torch.randn(B, H, T, D, generator=g).to(torch.float16) for _ in range(2))
+    inf, nan = float("inf"), float("nan")
+    for x in (k, v):
+        x[..., 0] = 0.375
+        x[..., 1] = 0.0
+        x[..., 2] = torch.where(torch.arange(T) % 3 == 0, -0.0, 0.0).to(torch.float16)
+        x[0, :, 17, 3], x[0, :, 90, 4] = inf, -inf
+        x[1, 0, 5, 5], x[1, 0, 40, 5], x[1, 0, 41, 5] = inf, -inf, nan
+        x[:, 1, 0, 6], x[:, 1, 63, 7], x[:, 1, 64:128, 8] = nan, nan, nan
+        x[:, 2, 2:64:4, 9] = nan
+        x[..., 10] = torch.where(torch.arange(T) % 2 == 0, 65504.0, -65504.0).to(torch.float16)
+        x[..., 11] = 6e-8 * (torch.arange(T) % 5).to(torch.float16)
+        x[0, 0, 70], x[1, 2, 71], x[1, 2, 72] = nan, inf, 1.5       # whole vectors
+    k, v = k.to(DEV), v.to(DEV)
+    cos, sin = (t.to(DEV) for t in _rope(T, D)) if angles else (None, None)
+    caches = [torch.full((B, H, T + 3, D), 7.0, dtype=torch.float16, device=DEV) for _ in range(4)]
+    for v_mode in (QuantMode.TokenQuant, QuantMode.VectorQuant):
+        assert append_quantized(k, v, cos, sin, caches[0], caches[1], 0, (128, 64, 0.1, QuantMode.ChannelQuant), (128, 64, 0.2, v_mode))
+        assert append_dense(k, v, cos, sin, caches[2], caches[3], 0)
+        quant_in_place(caches[2][:, :, :128], 64, 0.1, QuantMode.ChannelQuant)
+        quant_in_place(caches[3][:, :, :128], 64, 0.2, v_mode)
+        for one, two in ((caches[0], caches[2]), (caches[1], caches[3])):
+            assert bool(((one.view(torch.int16) == two.view(torch.int16)) | (one.isnan() & two.isnan())).all())
+        if not angles:                                            # (a rotation carries a NaN to the channel's partner)
+            assert bool(torch.isfinite(caches[0][0, 1, :128, D - 1]).all())
