@@ -1445,10 +1445,11 @@ __global__ void __launch_bounds__(KVC_WG, 3) kvc_encode_once_kernel(KvcStoreArgs
 // known, symbols come sixteen per load (K: 727 -> 540 MB fetched for 402 MB of symbols with head size 96), alphabets of at
 // most 16 symbols are looked up two at a time with one instruction per address, what is the same for a wave is kept in scalar
 // registers, and codes of more than 8 bits are left to the other kernel, whose loops for them took most of the registers: 7.5
-// (K) and 6 (V) vector instructions per symbol.  From symbols, us: K 8 x 32 heads x 128 x 4096 tokens 111 -> 75, V 104 ->
-// 71; 4 x 32 x 96 x 32 768 tokens 338 -> 257 and 242 -> 182 (60, 238 and 164 with neighbouring tiles read together, below).
-// What is left is the wait for the tiles before a wave's own (14 and 13 of the 75 and 71 us, 65 of 257: measured with made-up
-// offsets) and the tickets (4).  Sixteen waves per compute unit are best: 20 of them (five per SIMD, for which the registers
+// (K) and 6 (V) vector instructions per symbol.  Kernel times in first stores, K and V on average: 8 x 32 heads x 128 x 4096
+// tokens 104 -> 74 us, 4 x 32 x 96 x 32 768 tokens 294 -> 220 (K 259 and V 182; 238 and 163 with neighbouring tiles read
+// together, below; the first pair 69 and 58).  What is left is the wait for the tiles before a wave's own and the tickets:
+// in a loop over one call, launches included, that took 75 (K), 71 (V) and 257 us (K of the second), made-up offsets saved 14,
+// 13 and 65, and tickets 4.  Sixteen waves per compute unit are best: 20 of them (five per SIMD, for which the registers
 // would do) take 293 instead of 257 us, and a second tile on its way while the first is packed gains nothing for the
 // registers it takes.
 // A few registers of symbols at a time, without a branch inside, so that their look-ups are in flight together.  The symbols of
@@ -1578,8 +1579,8 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     // Neighbouring tiles share the cache lines that their symbols come in (V and head_dim 64: 64 bytes of each token's row, 96: 96, 72: 72),
     // and the lines of all waves are more than an L2 holds.  So STEP waves, whose tiles of one moment are whole lines, take the
     // tiles of all their runs in turn, and their loads meet.  (A group is a multiple of what they take.)  HBM traffic and time: V,
-    // 8 x 32 heads x 128 x 4096 tokens 295 -> 173 MB, 71 -> 60 us; 4 x 32 x 96 x 32 768: K 757 -> 603 MB, 260 -> 238 us, V 798 ->
-    // 483 MB, 182 -> 164 us; K, 2 x 32 x 64 x 8192: 41 -> 39 us.
+    // 8 x 32 heads x 128 x 4096 tokens in runs of two 295 -> 173 MB, 78 -> 68 us (58 in runs of four); 4 x 32 x 96 x 32 768: K 757 ->
+    // 603 MB, 259 -> 238 us, V 798 -> 483 MB, 182 -> 163 us; K, 2 x 32 x 64 x 8192: 32 -> 31 us.
     constexpr int STEP = FRONT == 1 ? 2 : ND == 24 || ND == 18 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
     static_assert(KVC_ONCE_GROUP_TILES % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
     const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
@@ -1998,10 +1999,12 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         sa.e = a;
         const int front = !src ? 0 : is_k ? 1 : 2;
         // From symbols the kernel has registers for five waves per SIMD, and LDS for three where a wave must hold any tile's
-        // image beside its staging area.  The room in `encoded` bounds the mean tile (a first store reserves what its code
+        // image beside its staging area.  The room in `encoded` bounds the mean tile (a first store gives what its code
         // needs): where that leaves a fifth of margin, waves get less LDS and four of them fit; the odd run whose first image
         // is larger is placed before its second tile is counted, as a wave's only tile would be.  402 M symbols: 316 -> 288 us,
-        // 134 M: 110 -> 101 us (of kvc_encode_once_kernel).
+        // 134 M: 110 -> 101 us (of kvc_encode_once_kernel).  The room is not the buffer: with the quarter that a context's buffer
+        // has beyond it, V of 4 x 32 heads x 128 x 4096 tokens, error bound 0.05, took 94 us for 70, and V's runs of four
+        // below were not taken at an error bound of 0.2: 8 x 32 x 128 x 4096 68 us for 58.
         const bool small = front == 0 && a.rows_per_codebook == 0 &&
                            a.encoded_cap / a.tiles <= (KVC_ONCE_SMALL_WAVE_BYTES - kvc_once_stage_bytes(0)) * 4 / 5;
         sa.e.wave_bytes = small ? KVC_ONCE_SMALL_WAVE_BYTES : KVC_ONCE_WAVE_BYTES;
@@ -2020,8 +2023,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         const bool wide = front == 0 && a.rows_per_codebook == 0 && c.longest_code >= 1 && c.longest_code <= 8 && (uintptr_t)c.d_sym % unit == 0 && c.stride % unit == 0 &&
                           (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 72 || a.vec_len == 64);
         // Its 4096 waves at a time: runs of two from where single tiles would be a second, part-filled round of them.  K and
-        // V of 2 x 32 heads x 128 x 6144 tokens (6144 tiles): 58 -> 42 and 56 -> 39 us; K of 4 x 24 x 72 x 4096: 53 -> 37.
-        // (V's runs of four begin where those of two would be a second round: 2 x 32 x 128 x 12 288 tokens 64 -> 57 us.)
+        // V of 2 x 32 heads x 128 x 6144 tokens (6144 tiles) in first stores: 50 -> 35 and 47 -> 32 us; K of 4 x 24 x 72 x 4096: 47 -> 31.
+        // (V's runs of four begin where those of two would be a second round: 2 x 32 x 128 x 12 288 tokens 58 -> 51 us, 9216 49 -> 48.)
         constexpr int KVC_WIDE_WAVES = 4096;
         if (wide && small && want == 1 && a.tiles > KVC_WIDE_WAVES) run = 2;
         const int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;

@@ -642,17 +642,19 @@ class KVCompCtx:
             if self._enc_pending > self.COPY_PENDING or (self._enc_pending and torch.cuda.is_current_stream_capturing()):
                 self._sync_sizes()
             self._encoded.reserve(worst, (), torch.uint8, self.device, self._enc_pending)
+        # (a payload whose size is bounded is told so: what the buffer keeps for growing would make tiles look larger than they are)
+        room = None if most_bytes is None else self._encoded.used + self._enc_pending + worst
         outcome = self._ask_outcome()
         before = None if outcome is None else (outcome.number, outcome.stream)
         told = None if outcome is None else outcome.ask(_lib.stream_of(state))
         try:
             if prepared is not None:
-                kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told, longest_code)
+                kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told, longest_code, room)
             else:
                 kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
                                          table_bytes=table_bytes, block_infos=bi, thread_infos=ti, encoded=self._encoded.data,
                                          symbols=symbols, cache=cache, quant_mask=mask, eb=self.quant_scale_rel, min_ints=mn, scales=sc,
-                                         stream_bytes=state[8:9], result=state[:8], outcome=told)
+                                         stream_bytes=state[8:9], result=state[:8], outcome=told, room=room)
         except BaseException:
             if outcome is not None:
                 with contextlib.suppress(RuntimeError):        # (the words must not go while a part of the call may write them)

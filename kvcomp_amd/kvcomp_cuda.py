@@ -256,12 +256,14 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
                  symbols: torch.Tensor = None, cache: torch.Tensor = None, quant_mask: int = 0, eb: float = 0.0,
                  min_ints: torch.Tensor = None, scales: torch.Tensor = None, table_stride: int = 0, rows_per_codebook: int = 0,
                  codebook_meta: torch.Tensor = None, base_global_offset: int = 0, stream_bytes: torch.Tensor = None,
-                 result: torch.Tensor = None, outcome=None):
+                 result: torch.Tensor = None, outcome=None, room: int = None):
     """kvc_encode_async: queue one encode (from `symbols`, or quantizing `cache` on the fly into min_ints / scales) with
     one table per `rows_per_codebook` tile rows, and return without waiting.  `result` (device int32[8], zeroed once)
     and `stream_bytes` (device int32[1]: payload bytes already in `encoded`, moved on by the call) stay on the device;
     encode_result() reads them.  The output tensors are written from their first element on.
-    outcome: (address of 16 words of pinned host memory, number); the call is kvc_encode_queue then."""
+    outcome: (address of 16 words of pinned host memory, number); the call is kvc_encode_queue then.
+    room: bytes of `encoded` that the payload may take, all of them by default; for symbols it says how large tiles can be on
+    average, so it should be no more than the codes need."""
     job = _lib.EncodeJob()
     job.is_k, job.quant_mask, job.eb = int(is_k), int(quant_mask), float(eb)
     _require((symbols is None) != (cache is None), "give either symbols or cache")
@@ -296,7 +298,8 @@ def encode_async(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens
     if codebook_meta is not None:
         job.d_codebook_meta = codebook_meta.data_ptr()
     job.d_block_infos, job.d_thread_infos = block_infos.data_ptr(), thread_infos.data_ptr()
-    job.d_encoded, job.encoded_cap = encoded.data_ptr(), encoded.numel()
+    _require(room is None or 0 < room <= encoded.numel(), "room: bytes of encoded")
+    job.d_encoded, job.encoded_cap = encoded.data_ptr(), encoded.numel() if room is None else room
     job.base_global_offset = int(base_global_offset) & 0xFFFFFFFF
     for t, n in ((stream_bytes, "stream_bytes"), (result, "result")):
         if t is not None:
@@ -341,14 +344,16 @@ def encode_prepare(is_k: bool, *, batch: int, head_num: int, head_dim: int, toke
     return PreparedEncode(job, scratch, done.value, sizes)
 
 
-def encode_prepared(prepared: PreparedEncode, encode_table: torch.Tensor, encoded: torch.Tensor, outcome=None, longest_code: int = 0):
+def encode_prepared(prepared: PreparedEncode, encode_table: torch.Tensor, encoded: torch.Tensor, outcome=None, longest_code: int = 0,
+                    room: int = None):
     """What encode_prepare left to be done, now that the table and the payload buffer are there (once per preparation).
-    longest_code: bits of the table's longest code, 0 if not known."""
+    longest_code: bits of the table's longest code, 0 if not known; room: as for encode_async."""
     job, at = prepared.job, prepared.scratch.data_ptr()
     for t, n in ((encode_table, "encode_table"), (encoded, "encoded")):
         _dev_u8(t, n)
     job.d_encode_tables, job.encode_table_bytes = encode_table.data_ptr(), encode_table.numel()
-    job.d_encoded, job.encoded_cap = encoded.data_ptr(), encoded.numel()
+    _require(room is None or 0 < room <= encoded.numel(), "room: bytes of encoded")
+    job.d_encoded, job.encoded_cap = encoded.data_ptr(), encoded.numel() if room is None else room
     address, number = (0, 0) if outcome is None else outcome
     with _lib.device_guard(encoded):
         check(_lib.lib().kvc_encode_queue(C.byref(job), at, prepared.done, longest_code, address, number, _lib.stream_of(encoded)))
