@@ -166,7 +166,7 @@ class _Growable:
 
 class _Outcome:
     """Pinned host words that a context's queued encodes leave their result in: written by an encode's last kernel and closed
-    with the number of the call (word 9).  Used like an event; looking costs no call into the runtime, where a copy and an
+    with the number of the call (word 9); words 10 - 12 say which stream and device that is to come from.  Used like an event; looking costs no call into the runtime, where a copy and an
     event behind every encode cost ten microseconds of host time and a launch."""
     _numbers = itertools.count(1)
     _late: collections.deque = collections.deque()       # words whose context is gone while a kernel may still write to them
@@ -183,7 +183,7 @@ class _Outcome:
         self.number = self.stream = 0
         self.words = torch.empty(16, dtype=torch.int32, pin_memory=True)
         self._seen = self.words.numpy()
-        self._seen[9] = 0
+        self._seen[9:13] = 0
 
     def ask(self, stream: int) -> Tuple[int, int]:
         """What the next encode on `stream` is to be told; if the library refuses it, refused() has to follow."""
