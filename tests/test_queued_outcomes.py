@@ -133,10 +133,10 @@ def _busy(stream, seconds):
     with torch.cuda.stream(stream):
         torch.cuda._sleep(1000)
         start.record()
-        torch.cuda._sleep(100000)
+        torch.cuda._sleep(5000000)
         end.record()
         end.synchronize()
-        torch.cuda._sleep(int(100000 * seconds * 1e3 / start.elapsed_time(end)))
+        torch.cuda._sleep(int(5000000 * seconds * 1e3 / start.elapsed_time(end)))
         end.record()
     return end
 
@@ -274,3 +274,28 @@ def test_a_context_of_one_stream_grows_on_another_with_stores_outstanding(is_k):
     assert all(bool((t == 0xA5).all()) for t in other)
     for name, value in expect.items():
         assert torch.equal(getattr(got, name), value), name
+
+
+@pytest.mark.gpu
+def test_words_that_another_stream_will_write_to_are_not_used_again():
+    """A store on a second stream while nobody follows the first one's outcome any more (as behind stores that were taken back)."""
+    from tests import _synth as S
+    _config()
+    x = S.synth_k(1024, 2, 4, 128).to(DEV)
+    want = _store_all(True, [x[:512], x[512:640], x[640:]]).encoded_data.clone()
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        ctx = _store_all(True, [x[:512]])
+        _busy(first, 0.2)
+        ctx.store(x[512:640], want_symbols=False)
+    words, ctx._probe = ctx._outcome, None
+    assert not words.query()
+    second.wait_stream(first)
+    with torch.cuda.stream(second):
+        ctx.store(x[640:], want_symbols=False)
+    assert ctx._outcome is not words and ctx._probe[0] is ctx._outcome and ctx._probe[1] == len(ctx._unverified) == 2
+    words.synchronize()
+    ctx._outcome.synchronize()
+    ctx.poll_stores()
+    assert words.query() and not ctx._unverified and torch.equal(ctx.encoded_data, want)
