@@ -238,6 +238,7 @@ int kvc_encode_async(const kvc_encode_job *job, void *stream);
  *   (d_encode_tables, encode_table_bytes, d_encoded and encoded_cap are not looked at).  d_result's eight words and
  *   *d_stream_bytes are cleared.  d_scratch: kvc_encode_scratch_bytes() of device memory on a 16-byte boundary, in use until
  *   the encode has run.  *prepared receives what to pass on.
+ * kvc_encode_prepare_packed: the same for symbols that kvc_quant_counted_packed writes, two to a byte.
  * kvc_encode_queue: kvc_encode_async, continuing what was prepared on the same stream for the same tokens and outputs
  *   (prepared = 0: nothing was; d_scratch is not used then).  longest_code: bits of the longest code in the (one) encode
  *   table, 0 if not known; symbols with longer codes are errors.  h_outcome, if not NULL: 16 words of pinned host memory that
@@ -248,6 +249,7 @@ int kvc_encode_async(const kvc_encode_job *job, void *stream);
  *   must exist as long.  No other stream is waited for, and the current device does not matter. */
 int64_t kvc_encode_scratch_bytes(void);
 int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream);
+int kvc_encode_prepare_packed(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream);
 int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,
                      uint32_t outcome_number, void *stream);
 int kvc_wait_outcome(const uint32_t *h_outcome, uint32_t outcome_number);
@@ -445,6 +447,12 @@ int kvc_quant(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H,
  *   pair_bits: index bits of a decode table that next to all pairs of these symbols fit, 2 .. 7, or 0.
  * kvc_quant_counted, kvc_counted_codebook: the two halves of kvc_quant_codebook.  The first queues the quantizer and hands out
  *   what the second, called exactly once, waits with; the host is free in between.
+ * kvc_packed_symbols_supported: 1 where symbols can go from the quantizer to the encoder two to a byte: the error bound leaves at most
+ *   sixteen of them and the layout is one of K's (head_dim 64, 72, 96 or 128, per-channel or block groups over 64 tokens) or V's
+ *   per-token one with rows of 512 to 65 536.  kvc_quant_counted_packed then writes tokens * batch * heads * head_dim / 2 bytes (16-byte
+ *   aligned, like the input) for kvc_encode_prepare_packed and the kvc_encode_queue behind it, in an order of their own.  Data whose
+ *   scales are among fp16's smallest numbers can still give a symbol from 16 on: the codebook's encode table then has more than
+ *   sixteen entries, the packed symbols are worth nothing, and kvc_quant has to write them a byte each.
  * kvc_put_codebook: the encode table to d_tables, the decode tree behind it on the next 16-byte boundary, and the decode
  *   tables of kvc_build_lut (one codebook) to d_lut, in stream order without waiting; book may be reused at once.
  * kvc_put_bytes: copies host bytes to device memory in stream order without waiting; h_src may be reused at once. */
@@ -457,6 +465,9 @@ typedef struct kvc_codebook {
 } kvc_codebook;
 int kvc_quant_counted(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                       float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, void **counted, void *stream);
+int kvc_packed_symbols_supported(int is_k, int quant_mask, int64_t batch, int64_t heads, int64_t head_dim, float eb);
+int kvc_quant_counted_packed(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
+                             float eb, uint8_t *d_packed, int8_t *d_min_i8, void *d_scale_f16, void **counted, void *stream);
 int kvc_counted_codebook(void *counted, int smoothed_symbols, kvc_codebook *out, void *stream);
 int kvc_quant_codebook(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                        float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, int smoothed_symbols,

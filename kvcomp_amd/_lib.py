@@ -64,6 +64,7 @@ _SIGNATURES = {
     "kvc_encode_async": [C.POINTER(EncodeJob), _vp],
     "kvc_encode_scratch_bytes": [],
     "kvc_encode_prepare": [C.POINTER(EncodeJob), _vp, _i64, _intp, _vp],
+    "kvc_encode_prepare_packed": [C.POINTER(EncodeJob), _vp, _i64, _intp, _vp],
     "kvc_encode_queue": [C.POINTER(EncodeJob), _vp, _int, _int, _vp, _u32, _vp],
     "kvc_encode_result": [_vp, _i64, _i64p, _i64p, _i64p, _i64p, _vp],
     "kvc_k_entropy_decode": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _int, _vp, _i64, _i64, _i64, _i64, _f32p, _vp],
@@ -90,6 +91,8 @@ _SIGNATURES = {
     "kvc_append_dense": [_vp, _vp],
     "kvc_append_quantized": [_vp, _i64, _i64, _int, C.c_float, _i64, _i64, _int, C.c_float, _vp],
     "kvc_quant_in_place": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp],
+    "kvc_packed_symbols_supported": [_int, _int, _i64, _i64, _i64, C.c_float],
+    "kvc_quant_counted_packed": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp, _vp, C.POINTER(_vp), _vp],
     "kvc_put_codebook": [_vp, _vp, _vp, _vp],
     "kvc_put_bytes": [_vp, _vp, _i64, _vp],
     "kvc_quant_error": [_vp, _i64, _i64, _i64, _i64, _i64, _int, C.c_float, _vp, _vp],

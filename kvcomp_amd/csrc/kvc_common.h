@@ -77,6 +77,8 @@ int kvc_check_hip(hipError_t e, const char *what);
 // reference-signature entry points derive from the decode tree on every call.
 constexpr size_t KVC_WS_SLOT_BYTES = 16384;
 int kvc_workspace_slot(void **slot, void *stream);   // stream: the one the call launches on (a recorded call gets a slot of its own)
+int kvc_quant_packed(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask, float eb,
+                     uint8_t *d_packed, int8_t *d_min_i8, void *d_scale_f16, int64_t *d_counts, void *stream);
 int kvc_quant_params(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                      float eb, int8_t *d_min_i8, void *d_scale_f16, void *stream);
 // What a caller that keeps its decode tables knows beyond the stream itself (all zero: nothing).
@@ -143,6 +145,20 @@ struct KvcTimer {
 // device helpers
 // ---------------------------------------------------------------------------------------------------
 #ifdef __HIPCC__
+// kvc_packed_symbols: symbols below 16 on their way from the quantizer to the encoder, two neighbouring channels to a byte, the
+// even one in the low half.
+//   V   [tokens][channels / 2], as the symbols themselves
+//   K   a tile (64 tokens of one head) in 32 D bytes of its own, one tile behind the other; in it a token's D / 2 bytes in pieces
+//       of 16 (4 where D is no multiple of 32), piece j of token t at (64 j + t) pieces: lane t of the encoder loads them in
+//       whole lines, straight into the registers it packs from.
+__device__ __forceinline__ constexpr uint32_t kvc_packed_k_chunk(uint32_t D) { return D % 32 == 0 ? 16u : 4u; }
+// where in its tile the eight channels that channel c belongs to lie, four bytes
+__device__ __forceinline__ constexpr uint32_t kvc_packed_k_place(uint32_t D, uint32_t c, uint32_t token)
+{
+    const uint32_t o = c >> 3;
+    return D % 32 == 0 ? (o >> 2) * (16 * KVC_WAVE) + token * 16 + (o & 3) * 4 : o * (4 * KVC_WAVE) + token * 4;
+}
+
 __device__ __forceinline__ uint32_t kvc_bswap(uint32_t v) { return __builtin_bswap32(v); }
 
 __device__ __forceinline__ float kvc_readlane(float v, int lane)

@@ -60,6 +60,8 @@ struct KvcEncodeArgs {
     // call is to be treated as if a wave had given up (both from the option "encode_lookback_polls")
     int max_polls, force_order;
     int wave_bytes;                // one-pass kernel from symbols: LDS of a wave
+    int packed;                    // sym holds two symbols a byte (kvc_packed_symbols)
+    int groups;                    // one pass: groups of tiles, see KVC_ONCE_GROUP_TILES
 };
 
 constexpr int KVC_ENC_STATUS_WORDS = 16;            // status words in front of the per-1024-tile payload totals
@@ -136,6 +138,24 @@ __global__ void __launch_bounds__(KVC_WAVE) kvc_encode_publish_kernel(KvcEncodeA
 __device__ __forceinline__ void kvc_load_vector(const KvcEncodeArgs &a, int64_t tile, int lane, uint32_t v[32])
 {
     const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
+    if (a.packed) {
+        const uint8_t *p = a.is_k ? a.sym + tile * (KVC_WAVE / 2 * a.vec_len) : a.sym + (row * KVC_V_TOKENS * a.stride + col * KVC_WAVE + (lane & ~1)) / 2;
+#pragma unroll
+        for (int j = 0; j < 32; j++) {
+            uint32_t w = 0;
+            if (a.is_k) {
+                if (4 * j < a.vec_len) {
+                    const uint32_t n = *reinterpret_cast<const uint16_t *>(p + kvc_packed_k_place((uint32_t)a.vec_len, 4u * j, (uint32_t)lane) + 2 * (j & 1));
+                    w = (n & 0xfu) | (n & 0xf0u) << 4 | (n & 0xf00u) << 8 | (n & 0xf000u) << 12;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++) w |= ((uint32_t)p[(int64_t)(4 * j + k) * (a.stride / 2)] >> (4 * (lane & 1)) & 0xfu) << (8 * k);
+            }
+            v[j] = w;
+        }
+        return;
+    }
     if (a.is_k) {
         const uint8_t *p = a.sym + (row * KVC_WAVE + lane) * a.stride + col * a.vec_len;
         const int nd = a.vec_len >> 2;
@@ -393,6 +413,82 @@ __device__ __forceinline__ void kvc_stage_v_wide(int lane, uint8_t *s_stage, con
             for (int j = 0; j < 8; j++) v[16 * g + 2 * j + h] = *reinterpret_cast<const uint32_t *>(s_stage + lane * RS + 4 * j);
             kvc_wave_lds_sync();
         }
+    }
+}
+
+// ---- the same for symbols two to a byte (kvc_packed_symbols): eight symbols a word ----
+// K: a lane's token, straight into the registers it packs from; every load is whole lines.
+template <int NW>
+__device__ __forceinline__ void kvc_load_k_packed(const KvcEncodeArgs &a, int tile, int lane, uint32_t (&w)[16])
+{
+    const uint8_t *p = a.sym + (int64_t)tile * (KVC_WAVE * 4 * NW);
+    if constexpr (NW % 4 == 0) {
+#pragma unroll
+        for (int j = 0; j < NW / 4; j++) {
+            const kvc_u32x4 q = *reinterpret_cast<const kvc_u32x4 *>(p + (KVC_WAVE * j + lane) * 16);
+            w[4 * j] = q.x;
+            w[4 * j + 1] = q.y;
+            w[4 * j + 2] = q.z;
+            w[4 * j + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < NW; j++) w[j] = *reinterpret_cast<const uint32_t *>(p + (KVC_WAVE * j + lane) * 4);
+    }
+}
+
+// V: a token's 64 symbols are 32 bytes, four lanes of sixteen channels; a lane has eight consecutive tokens, whose symbols of eight
+// channels are transposed in registers (halves of bytes, bytes, halves of words).  Through the area in two halves, as
+// [channel][eight words], the channels from 32 on eight words further: reads and writes touch every bank once.
+constexpr int KVC_STAGE_VPACKED_BYTES = 64 * 36 + 32;
+__device__ __forceinline__ void kvc_transpose_8x8(const uint32_t (&t)[8], uint32_t (&c)[8])
+{
+    uint32_t even[4], odd[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        even[k] = (t[2 * k] & 0x0f0f0f0fu) | ((t[2 * k + 1] << 4) & 0xf0f0f0f0u);
+        odd[k] = ((t[2 * k] >> 4) & 0x0f0f0f0fu) | (t[2 * k + 1] & 0xf0f0f0f0u);
+    }
+    uint32_t e[4], o[4];
+    kvc_transpose_4x4(even[0], even[1], even[2], even[3], e);
+    kvc_transpose_4x4(odd[0], odd[1], odd[2], odd[3], o);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        c[2 * k] = e[k];
+        c[2 * k + 1] = o[k];
+    }
+}
+
+__device__ __forceinline__ void kvc_front_v_packed(const KvcEncodeArgs &a, int tile, int lane, uint8_t *s_stage, uint32_t (&w)[16])
+{
+    constexpr int RS = 36;
+    const int64_t row = (uint32_t)tile / (uint32_t)a.cols, col = tile - row * a.cols;
+    const int group = lane >> 2, piece = lane & 3;
+    const uint8_t *p = a.sym + ((row * KVC_V_TOKENS + 8 * group) * a.stride + col * KVC_WAVE + 16 * piece) / 2;
+    uint32_t x[8], y[8], cx[8], cy[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint2 q = *reinterpret_cast<const uint2 *>(p + i * (a.stride / 2));
+        x[i] = q.x;
+        y[i] = q.y;
+    }
+    kvc_transpose_8x8(x, cx);
+    kvc_transpose_8x8(y, cy);
+    uint8_t *dst = s_stage + 16 * piece * RS + 32 * (piece >> 1) + 4 * (group & 7);
+    const uint8_t *src = s_stage + lane * RS + 32 * (lane >> 5);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (group >> 3 == h) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                *reinterpret_cast<uint32_t *>(dst + k * RS) = cx[k];
+                *reinterpret_cast<uint32_t *>(dst + (8 + k) * RS) = cy[k];
+            }
+        }
+        kvc_wave_lds_sync();
+#pragma unroll
+        for (int j = 0; j < 8; j++) w[8 * h + j] = *reinterpret_cast<const uint32_t *>(src + 4 * j);
+        kvc_wave_lds_sync();
     }
 }
 
@@ -1033,10 +1129,15 @@ constexpr int KVC_ONCE_MAX_GROUPS = (int)((KVC_WS_SLOT_BYTES - KVC_ONCE_GROUP_WO
 // group (measured: 10 us per wave there, 3 us on the die with the last tiles).
 constexpr int KVC_ONCE_GROUP_TILES = 56;
 static_assert(KVC_ONCE_GROUP_TILES <= KVC_WAVE && KVC_ONCE_GROUP_TILES % 2 == 0, "one look of 64 lanes covers a group; a run of two stays inside one");
-__device__ __forceinline__ int64_t kvc_once_group(int64_t tile) { return (int64_t)((uint32_t)tile / (uint32_t)KVC_ONCE_GROUP_TILES); }
+// (V from packed symbols: four waves take the sixteen tiles of their runs in turn, which must lie in one group.  48 tiles are
+// one and a half of its workgroups, so those waves change dies as well.)
+constexpr int KVC_ONCE_GROUP_TILES_VPACKED = 48;
+template <int G = KVC_ONCE_GROUP_TILES>
+__device__ __forceinline__ int64_t kvc_once_group(int64_t tile) { return (int64_t)((uint32_t)tile / (uint32_t)G); }
+template <int G = KVC_ONCE_GROUP_TILES>
 __device__ __forceinline__ bool kvc_once_closes(const KvcEncodeArgs &a, int64_t tile)
 {
-    return (uint32_t)tile % (uint32_t)KVC_ONCE_GROUP_TILES == (uint32_t)KVC_ONCE_GROUP_TILES - 1u || tile == a.tiles - 1;
+    return (uint32_t)tile % (uint32_t)G == (uint32_t)G - 1u || tile == a.tiles - 1;
 }
 
 __device__ __forceinline__ uint64_t kvc_bi_word(uint32_t offset, uint32_t byte_num, uint32_t state)
@@ -1056,7 +1157,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_mark_kernel(KvcEncodeArgs a
 {
     const int64_t tile = (int64_t)blockIdx.x * KVC_WG + threadIdx.x;
     if (tile < a.tiles) reinterpret_cast<uint64_t *>(a.block_infos)[tile] = kvc_bi_word(0u, 0u, KVC_BI_NOT_READY);
-    if (tile < (a.tiles + KVC_ONCE_GROUP_TILES - 1) / KVC_ONCE_GROUP_TILES) kvc_group_words(a)[tile] = kvc_group_word(0u, KVC_BI_NOT_READY);
+    if (tile < a.groups) kvc_group_words(a)[tile] = kvc_group_word(0u, KVC_BI_NOT_READY);
     if (blockIdx.x == 0) {
         kvc_encode_init(a);
         for (int i = threadIdx.x; i < KVC_ONCE_PART_LINES * KVC_ONCE_PART_STRIDE; i += KVC_WG) a.status[KVC_ONCE_PART_WORD + i] = 0u;
@@ -1074,25 +1175,27 @@ struct KvcFirstLooks {
     uint64_t tile_word, group_word;
 };
 
+template <int G = KVC_ONCE_GROUP_TILES>
 __device__ __forceinline__ KvcFirstLooks kvc_look_back_ask(const KvcEncodeArgs &a, int64_t tile, int lane)
 {
     const uint64_t *bi64 = reinterpret_cast<const uint64_t *>(a.block_infos);
-    const int64_t group = kvc_once_group(tile);
-    const int r = (int)(tile - group * KVC_ONCE_GROUP_TILES);
+    const int64_t group = kvc_once_group<G>(tile);
+    const int r = (int)(tile - group * G);
     KvcFirstLooks f;
-    f.tile_word = lane < r ? kvc_status_load(bi64 + group * KVC_ONCE_GROUP_TILES + lane) : 0ull;
+    f.tile_word = lane < r ? kvc_status_load(bi64 + group * G + lane) : 0ull;
     f.group_word = group - 1 - lane >= 0 ? kvc_status_load(kvc_group_words(a) + group - 1 - lane) : kvc_group_word(0u, 0u);
     return f;
 }
 
 // First half of the look-back: the payload bytes of the tiles before `tile` in its own group; the wave of a group's last
 // tile then publishes the group's size.  *polls counts the looks that found a word not ready (wave-uniform).
+template <int G = KVC_ONCE_GROUP_TILES>
 __device__ __forceinline__ uint32_t kvc_look_back_in_group(const KvcEncodeArgs &a, int64_t tile, uint32_t bn, int lane, uint64_t first_look,
                                                            int *polls)
 {
     const uint64_t *bi64 = reinterpret_cast<const uint64_t *>(a.block_infos);
-    const int64_t group = kvc_once_group(tile);
-    const int r = (int)(tile - group * KVC_ONCE_GROUP_TILES);
+    const int64_t group = kvc_once_group<G>(tile);
+    const int r = (int)(tile - group * G);
     uint32_t in_group = 0;
     uint64_t w = first_look;
     while (r > 0) {
@@ -1102,20 +1205,21 @@ __device__ __forceinline__ uint32_t kvc_look_back_in_group(const KvcEncodeArgs &
         }
         if (++*polls > a.max_polls) break;
         __builtin_amdgcn_s_sleep(2);
-        w = lane < r ? kvc_status_load(bi64 + group * KVC_ONCE_GROUP_TILES + lane) : 0ull;
+        w = lane < r ? kvc_status_load(bi64 + group * G + lane) : 0ull;
     }
-    if (kvc_once_closes(a, tile) && lane == 0)             // this wave speaks for its group
+    if (kvc_once_closes<G>(a, tile) && lane == 0)             // this wave speaks for its group
         kvc_status_store(kvc_group_words(a) + group, kvc_group_word(in_group + bn, KVC_BI_SIZE));
     return in_group;
 }
 
 // Second half: the payload bytes of the groups before the tile's own; the wave of a group's last tile then publishes
 // the bytes up to the end of its group.
+template <int G = KVC_ONCE_GROUP_TILES>
 __device__ __forceinline__ uint32_t kvc_look_back_groups(const KvcEncodeArgs &a, int64_t tile, uint32_t in_group_and_own, int lane,
                                                          uint64_t first_look, int *polls)
 {
     uint64_t *groups = kvc_group_words(a);
-    const int64_t group = kvc_once_group(tile);
+    const int64_t group = kvc_once_group<G>(tile);
     uint32_t before = 0;
     int64_t j = group - 1;                                 // nearest group not yet accounted for
     uint64_t w = first_look;                               // taken at j = group - 1
@@ -1134,7 +1238,7 @@ __device__ __forceinline__ uint32_t kvc_look_back_groups(const KvcEncodeArgs &a,
         const int64_t idx = j - lane;
         w = idx >= 0 ? kvc_status_load(groups + idx) : kvc_group_word(0u, 0u);   // in front of the first group: nothing, and known
     }
-    if (kvc_once_closes(a, tile) && lane == 0)
+    if (kvc_once_closes<G>(a, tile) && lane == 0)
         kvc_status_store(groups + group, kvc_group_word(before + in_group_and_own, 0u));
     return before;
 }
@@ -1188,6 +1292,7 @@ struct KvcOncePending {
 // before it, which this wave has just placed at follows_off), publish its block_info and write its payload from the LDS
 // image (which starts on a word; the payload lands p.head bytes into an aligned word).  Returns error bits; *off_out
 // receives the tile's global offset.
+template <int G = KVC_ONCE_GROUP_TILES>
 __device__ __forceinline__ uint32_t kvc_once_place(const KvcEncodeArgs &a, const KvcOncePending &pd, const uint32_t *image, uint32_t base,
                                                    int lane, int *polls, uint32_t *off_out, bool follows = false, uint32_t follows_off = 0)
 {
@@ -1196,12 +1301,12 @@ __device__ __forceinline__ uint32_t kvc_once_place(const KvcEncodeArgs &a, const
     uint32_t off;
     if (follows) {
         off = follows_off;
-        if (kvc_once_closes(a, tile) && lane == 0)         // this wave speaks for its group: the group's end
-            kvc_status_store(kvc_group_words(a) + kvc_once_group(tile), kvc_group_word(off + bn - base, 0u));
+        if (kvc_once_closes<G>(a, tile) && lane == 0)         // this wave speaks for its group: the group's end
+            kvc_status_store(kvc_group_words(a) + kvc_once_group<G>(tile), kvc_group_word(off + bn - base, 0u));
     } else {
         uint32_t in_group = pd.in_group;
-        if (!pd.in_group_known) in_group = kvc_look_back_in_group(a, tile, bn, lane, pd.looks.tile_word, polls);
-        off = base + in_group + kvc_look_back_groups(a, tile, in_group + bn, lane, pd.looks.group_word, polls);
+        if (!pd.in_group_known) in_group = kvc_look_back_in_group<G>(a, tile, bn, lane, pd.looks.tile_word, polls);
+        off = base + in_group + kvc_look_back_groups<G>(a, tile, in_group + bn, lane, pd.looks.group_word, polls);
     }
     *off_out = off;
     uint32_t err = 0;
@@ -1496,6 +1601,48 @@ __device__ __forceinline__ uint32_t kvc_join_vector(const uint2 *s_table, uint32
     return PAIRS && (over & 0xf0f0f0f0u) ? 0x4000u : bits; // (a larger symbol is one without a code: KVC_NO_CODE_LEN)
 }
 
+// The same from symbols two to a byte: a byte is the index of its pair (first symbol in the lower half).
+template <int ND>
+__device__ __forceinline__ uint32_t kvc_join_packed(const uint2 *s_table, const uint32_t (&w)[16], uint32_t (&v)[32], uint32_t (&gl)[8])
+{
+    uint32_t bits = 0;
+    uint32_t table_at = (uint32_t)(uintptr_t)(const kvc_lds_u64 *)s_table;
+    constexpr int STEP = ND % 4 == 0 ? 2 : 1;              // words, of eight symbols each
+#pragma unroll
+    for (int c = 0; c < ND / 2 / STEP; c++) {
+        asm volatile("" : "+v"(table_at));                 // (as above)
+#pragma unroll
+        for (int j = STEP * c; j < STEP * (c + 1); j++) {
+            const uint64_t e0 = *(const kvc_lds_u64 *)(uintptr_t)__builtin_amdgcn_udot4(w[j], 0x00000008u, table_at, false);
+            const uint64_t e1 = *(const kvc_lds_u64 *)(uintptr_t)__builtin_amdgcn_udot4(w[j], 0x00000800u, table_at, false);
+            const uint64_t e2 = *(const kvc_lds_u64 *)(uintptr_t)__builtin_amdgcn_udot4(w[j], 0x00080000u, table_at, false);
+            const uint64_t e3 = *(const kvc_lds_u64 *)(uintptr_t)__builtin_amdgcn_udot4(w[j], 0x08000000u, table_at, false);
+            const uint32_t second = (uint32_t)(e1 >> 32), fourth = (uint32_t)(e3 >> 32);
+            const uint32_t l0 = (uint32_t)(e0 >> 32) + second, l1 = (uint32_t)(e2 >> 32) + fourth;
+            v[2 * j] = ((uint32_t)e0 << (second & 31u)) | (uint32_t)e1;
+            v[2 * j + 1] = ((uint32_t)e2 << (fourth & 31u)) | (uint32_t)e3;
+            asm volatile("" : "+v"(v[2 * j]), "+v"(v[2 * j + 1]));     // (joined here: or it is the pairs that are kept until they are packed)
+            bits += l0 + l1;
+            gl[j >> 1] |= (l0 | l1 << 8) << (16 * (j & 1));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    return bits;
+}
+
+// A vector's bits, for codes of any length (alphabets of sixteen have none of more than fifteen bits).
+template <int ND>
+__device__ __forceinline__ uint32_t kvc_count_packed(const uint2 *s_table, const uint32_t (&w)[16])
+{
+    uint32_t bits = 0;
+#pragma unroll
+    for (int j = 0; j < ND / 2; j++) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) bits += s_table[(w[j] >> (8 * k)) & 0xffu].y;
+    }
+    return bits;
+}
+
 // A lane's bits on their way to the image: `cur` is the word being filled, `left` the bits it still takes, negated.
 struct KvcPacker {
     uint32_t cur;
@@ -1540,30 +1687,62 @@ __device__ __forceinline__ void kvc_pack_joined(uint32_t start, const uint32_t (
     p.finish();
 }
 
-// The workgroup's copy of the encode table: an entry without a code, or with one of more than 8 bits (which the launcher has
-// been told do not occur), gets the length KVC_NO_CODE_LEN.  pairs (at most sixteen entries): the 256 pairs of symbols.
-__device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint2 *s_table, bool pairs)
+// Symbols two to a byte and codes of more than 8 bits: the pairs are looked up again, and pushed one by one where two of them
+// do not fit a word in every lane.
+template <int ND>
+__device__ __forceinline__ void kvc_pack_packed(uint32_t start, const uint2 *s_table, const uint32_t (&w)[16], uint32_t *image)
+{
+    KvcPacker p(start, image);
+#pragma unroll
+    for (int j = 0; j < ND; j++) {
+        const uint32_t h = w[j >> 1] >> (16 * (j & 1));
+        const uint2 e0 = s_table[h & 0xffu], e1 = s_table[(h >> 8) & 0xffu];
+        if (!__any(e0.y + e1.y > 32u)) {
+            p.push((uint32_t)(((uint64_t)e0.x << e1.y) | e1.x), e0.y + e1.y);
+        } else {
+            p.push(e0.x, e0.y);
+            p.push(e1.x, e1.y);
+        }
+    }
+    p.finish();
+}
+
+// The workgroup's copy of the encode table: an entry without a code, or with one of more than `longest` bits (which the launcher
+// has been told do not occur), gets the length KVC_NO_CODE_LEN.  pairs (at most sixteen entries): the 256 pairs of symbols, the
+// first one in the index's upper half, or (LOW) in its lower half.
+template <bool LOW>
+__device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint2 *s_table, bool pairs, uint32_t longest)
 {
     const uint2 *t = reinterpret_cast<const uint2 *>(a.table);
     auto entry = [&](int i) {
         const uint2 e = i < a.table_entries ? t[i] : make_uint2(0u, 0u);
-        return e.y == 0u || e.y > 8u ? make_uint2(0u, KVC_NO_CODE_LEN) : make_uint2(e.x & ((1u << e.y) - 1u), e.y);
+        return e.y == 0u || e.y > longest ? make_uint2(0u, KVC_NO_CODE_LEN) : make_uint2(e.x & ((1u << e.y) - 1u), e.y);
     };
     for (int i = threadIdx.x; i < 256; i += blockDim.x) {
-        uint2 e = entry(pairs ? i >> 4 : i);
+        uint2 e = entry(!pairs ? i : LOW ? i & 15 : i >> 4);
         if (pairs) {
-            const uint2 f = entry(i & 15);
+            const uint2 f = entry(LOW ? i >> 4 : i & 15);
             e = make_uint2((e.x << (f.y & 31u)) | f.x, e.y + f.y);
         }
         s_table[i] = e;
     }
 }
 
-// FRONT 0: K, 1: V.  ND: registers that a vector fills.
-template <int FRONT, int ND>
+// Two symbols a byte: first stores whose symbols nobody else wants and which have at most sixteen of them.  Both sides of the symbols
+// wait for memory, so half the bytes is what it gives: the quantizers write half (K 80 -> 76 and V 82 -> 73 us for 8 x 32 heads x 128 x
+// 4096 tokens, 236 -> 214 and 238 -> 224 for 4 x 32 x 96 x 32 768) and this kernel reads half (70 -> 61, 58 -> 51; 241 -> 206, 162 -> 130).  A
+// K tile needs no staging, since the quantizer, which has it in registers, writes it in the order of the lanes.  A byte is the index of
+// a pair's look-up; V's pairs lie along the other axis, and are turned in registers.  Codes of any length are taken, since what
+// would be left over would have to be written out again (K of 2 x 32 x 96 x 4480 in block groups, codes of 11 bits).
+// FRONT 0: K, 1: V.  ND: registers that a vector fills, a byte per symbol.  FORM: a byte per symbol, or two symbols a byte with codes
+// of at most eight bits, or of any length.
+enum { KVC_FORM_BYTES = 0, KVC_FORM_PACKED = 1, KVC_FORM_PACKED_LONG = 2 };
+template <int FRONT, int ND, int FORM>
 __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int run)
 {
-    constexpr int STAGE = FRONT == 0 ? KVC_STAGE_VSYM_BYTES : KVC_STAGE_VF16_BYTES;
+    constexpr bool PACKED = FORM != KVC_FORM_BYTES, LONG = FORM == KVC_FORM_PACKED_LONG;
+    constexpr int G = PACKED && FRONT == 1 ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES;
+    constexpr int STAGE = PACKED ? (FRONT == 0 ? 0 : KVC_STAGE_VPACKED_BYTES) : FRONT == 0 ? KVC_STAGE_VSYM_BYTES : KVC_STAGE_VF16_BYTES;
     extern __shared__ __align__(16) uint8_t s_dyn[];
     __shared__ uint32_t s_err, s_max_tile, s_longest, s_polls, s_ticket;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
@@ -1572,8 +1751,8 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     uint8_t *s_stage = reinterpret_cast<uint8_t *>(area) + a.wave_bytes - STAGE;
     uint32_t ticket = 0;
     if (tid == 0) ticket = atomicAdd(&a.status[KVC_ONCE_TICKET_WORD], 1u);
-    const bool pairs = a.table_entries <= 16;
-    kvc_load_pair_table(a, s_table, pairs);
+    const bool pairs = PACKED || a.table_entries <= 16;
+    kvc_load_pair_table<PACKED>(a, s_table, pairs, LONG ? 16u : 8u);
     if (tid == 0) { s_err = 0; s_max_tile = 0; s_longest = 0; s_polls = 0; s_ticket = ticket; }
     __syncthreads();
     // Neighbouring tiles share the cache lines that their symbols come in (V and head_dim 64: 64 bytes of each token's row, 96: 96, 72: 72),
@@ -1581,8 +1760,9 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     // tiles of all their runs in turn, and their loads meet.  (A group is a multiple of what they take.)  HBM traffic and time: V,
     // 8 x 32 heads x 128 x 4096 tokens in runs of two 295 -> 173 MB, 78 -> 68 us (58 in runs of four); 4 x 32 x 96 x 32 768: K 757 ->
     // 603 MB, 259 -> 238 us, V 798 -> 483 MB, 182 -> 163 us; K, 2 x 32 x 64 x 8192: 32 -> 31 us.
-    constexpr int STEP = FRONT == 1 ? 2 : ND == 24 || ND == 18 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
-    static_assert(KVC_ONCE_GROUP_TILES % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
+    // Two symbols a byte: four V tiles are a line of each token's row, and a K tile is lines of its own.
+    constexpr int STEP = PACKED ? (FRONT == 1 ? 4 : 1) : FRONT == 1 ? 2 : ND == 24 || ND == 18 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
+    static_assert(G % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
     const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
     const int tiles = (int)a.tiles;
     const uint32_t base = a.status[KVC_ONCE_BASE_WORD];
@@ -1603,8 +1783,11 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         int lane = tid & 63;                               // (opaque, as in kvc_encode_once_kernel)
         asm volatile("" : "+v"(lane));
         const KvcEncodeArgs &a = kvc_kernarg_again<KvcEncodeArgs>();
-        uint32_t v[32];
-        if constexpr (ND == 18) {
+        uint32_t v[32], w[16];
+        if constexpr (PACKED) {
+            if constexpr (FRONT == 0) kvc_load_k_packed<ND / 2>(a, tile, lane, w);
+            else kvc_front_v_packed(a, tile, lane, s_stage, w);
+        } else if constexpr (ND == 18) {
             kvc_front_k72(a, tile, lane, s_stage, v);
         } else {
             kvc_u32x4 q[8];
@@ -1617,7 +1800,9 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
             }
         }
         uint32_t bits = 0, gl[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};     // the joined lengths of registers 4 i .. 4 i + 3
-        if (pairs) bits = kvc_join_vector<true, ND, ND % 8 == 0 ? 8 : 6>(s_table, v, gl);
+        if constexpr (LONG) bits = kvc_count_packed<ND>(s_table, w);
+        else if constexpr (PACKED) bits = kvc_join_packed<ND>(s_table, w, v, gl);
+        else if (pairs) bits = kvc_join_vector<true, ND, ND % 8 == 0 ? 8 : 6>(s_table, v, gl);
         else bits = kvc_join_vector<false, ND, ND % 4 == 0 ? 4 : 6>(s_table, v, gl);
         const bool bad = bits >= KVC_NO_CODE_LEN;          // a symbol without a code: the lane emits nothing
         if (bad) bits = 0;
@@ -1634,14 +1819,14 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         if (lane == 0) kvc_status_store(reinterpret_cast<uint64_t *>(a.block_infos) + tile, kvc_bi_word(0u, bn, KVC_BI_SIZE));
         // the tile that the run's place is looked for with; and the wave that speaks for a group must not sit on its size (as in
         // kvc_encode_once_kernel)
-        const bool opens = kept == 0 && !placed, closes = kvc_once_closes(a, tile);
+        const bool opens = kept == 0 && !placed, closes = kvc_once_closes<G>(a, tile);
         if (opens) {
-            first.looks = kvc_look_back_ask(a, tile, lane);
+            first.looks = kvc_look_back_ask<G>(a, tile, lane);
             first.in_group_known = closes;
         }
         if (closes) {
-            const uint64_t word = opens ? first.looks.tile_word : kvc_look_back_ask(a, tile, lane).tile_word;
-            const uint32_t in_group = kvc_look_back_in_group(a, tile, bn, lane, word, &polls);
+            const uint64_t word = opens ? first.looks.tile_word : kvc_look_back_ask<G>(a, tile, lane).tile_word;
+            const uint32_t in_group = kvc_look_back_in_group<G>(a, tile, bn, lane, word, &polls);
             if (opens) first.in_group = in_group;
         }
         // The image goes behind the kept ones.  If it does not fit there, those are written out first, and this tile starts again
@@ -1654,7 +1839,8 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
             kvc_wave_lds_sync();
             if (!bad) {
                 // (streams of at most 2 3/4 bits per symbol: eight symbols next to always fit a word)
-                if (lg * 32u <= 11u * 4u * (uint32_t)ND) kvc_pack_joined<ND, true>(start, v, gl, image);
+                if constexpr (LONG) kvc_pack_packed<ND>(start, s_table, w, image);
+                else if (lg * 32u <= 11u * 4u * (uint32_t)ND) kvc_pack_joined<ND, true>(start, v, gl, image);
                 else kvc_pack_joined<ND, false>(start, v, gl, image);
             }
             kvc_wave_lds_sync();
@@ -1689,7 +1875,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
                     for (int i = 0; i < OTHERS; i++)
                         next_off += (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(between_word >> 32), k * OTHERS + i) & 0xffffu;
                 }
-                err |= kvc_once_place(a, which, area + at, base, lane, &polls, &off, placed, next_off);
+                err |= kvc_once_place<G>(a, which, area + at, base, lane, &polls, &off, placed, next_off);
                 at += which.packs ? kvc_once_image_words(which.bn) : 0u;
                 next_off = off + which.bn;
                 placed = true;
@@ -1868,7 +2054,7 @@ struct KvcStoreSource {
 
 // How far an encode call has come before kvc_encode_launch: nothing, the status words set, the block_infos marked as well
 // (then it takes one pass, else two).
-enum { KVC_ENC_FRESH = 0, KVC_ENC_CLEARED = 1, KVC_ENC_MARKED = 2 };
+enum { KVC_ENC_FRESH = 0, KVC_ENC_CLEARED = 1, KVC_ENC_MARKED = 2, KVC_ENC_PACKED = 4 };   // (PACKED: beside one of the others, for kvc_encode_queue's caller)
 
 // Everything an encode call is made of; the classic entry points fill in what they have and leave the rest zero.
 struct KvcEncodeCall {
@@ -1891,6 +2077,7 @@ struct KvcEncodeCall {
     int first_launch;                                      // what is done already: KVC_ENC_FRESH, KVC_ENC_CLEARED or KVC_ENC_MARKED
     uint32_t *h_outcome, outcome_number;
     int longest_code;                                      // of the (one) codebook, 0: not known
+    bool packed;                                           // d_sym: two symbols a byte (kvc_packed_symbols)
 };
 
 static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
@@ -1903,6 +2090,20 @@ static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
         return kvc_fail(-3, "payload (%u bytes) does not fit the encoded_data buffer (%lld bytes)", total, (long long)encoded_cap);
     if (bits & KVC_ENC_ERR_ORDER) return kvc_fail(-3, "one-pass encoder: a tile waited too long for the tiles before it");
     return 0;
+}
+
+template <int FORM>
+static auto kvc_symbols_kernel_of(int is_k, int vec_len)
+{
+    return !is_k ? kvc_encode_symbols_kernel<1, 32, FORM> :
+           vec_len == 128 ? kvc_encode_symbols_kernel<0, 32, FORM> :
+           vec_len == 96 ? kvc_encode_symbols_kernel<0, 24, FORM> :
+           vec_len == 72 ? kvc_encode_symbols_kernel<0, 18, FORM> : kvc_encode_symbols_kernel<0, 16, FORM>;
+}
+static auto kvc_symbols_kernel(int is_k, int vec_len, int form)
+{
+    return form == KVC_FORM_BYTES ? kvc_symbols_kernel_of<KVC_FORM_BYTES>(is_k, vec_len) :
+           form == KVC_FORM_PACKED ? kvc_symbols_kernel_of<KVC_FORM_PACKED>(is_k, vec_len) : kvc_symbols_kernel_of<KVC_FORM_PACKED_LONG>(is_k, vec_len);
 }
 
 // Queue the launches of one encode call (init, count, per-1024-tile sums, offsets, emit, publish); waits for nothing.
@@ -1921,6 +2122,10 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
                 ((uintptr_t)c.d_stream_bytes & 3) == 0 && ((uintptr_t)c.d_result & 3) == 0,
                 "encode buffers are misaligned");
     KVC_REQUIRE(c.src != nullptr || c.d_sym != nullptr, "symbol pointer is NULL");
+    KVC_REQUIRE(!c.packed || (c.d_sym && ((uintptr_t)c.d_sym & 15) == 0 && c.rows_per_codebook == 0 && (c.is_k || c.stride % KVC_V_VEC_PER_BLK == 0) &&
+                              c.head_dim <= 128 && c.tokens * c.stride <= INT64_C(1) << 40 &&
+                              (!c.is_k || c.head_dim == 128 || c.head_dim == 96 || c.head_dim == 72 || c.head_dim == 64)),
+                "these symbols cannot be packed two to a byte");
     KVC_REQUIRE(c.stride % 4 == 0, "stride must be a multiple of 4");
     KVC_REQUIRE(c.rows_per_codebook >= 0 && (c.rows_per_codebook == 0 || (c.table_stride >= c.table_bytes && c.table_stride % 8 == 0)),
                 "tables of several codebooks must be a multiple of 8 bytes apart and not overlap");
@@ -1953,6 +2158,9 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     a.outcome = c.h_outcome;
     a.outcome_number = c.outcome_number;
     a.clear = c.clear;
+    a.packed = c.packed;
+    const int group_tiles = c.packed && !c.is_k ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES;
+    a.groups = (int)((a.tiles + group_tiles - 1) / group_tiles);
     a.max_polls = 0;
     a.force_order = 0;
     const int64_t chunks = (a.tiles + 1023) / 1024;
@@ -2005,8 +2213,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         // 134 M: 110 -> 101 us (of kvc_encode_once_kernel).  The room is not the buffer: with the quarter that a context's buffer
         // has beyond it, V of 4 x 32 heads x 128 x 4096 tokens, error bound 0.05, took 94 us for 70, and V's runs of four
         // below were not taken at an error bound of 0.2: 8 x 32 x 128 x 4096 68 us for 58.
-        const bool small = front == 0 && a.rows_per_codebook == 0 &&
-                           a.encoded_cap / a.tiles <= (KVC_ONCE_SMALL_WAVE_BYTES - kvc_once_stage_bytes(0)) * 4 / 5;
+        const bool small = front == 0 && a.rows_per_codebook == 0 && (c.packed ||
+                           a.encoded_cap / a.tiles <= (KVC_ONCE_SMALL_WAVE_BYTES - kvc_once_stage_bytes(0)) * 4 / 5);
         sa.e.wave_bytes = small ? KVC_ONCE_SMALL_WAVE_BYTES : KVC_ONCE_WAVE_BYTES;
         // two tiles per wave (the look-back of the first hides behind the count of the second) where all tiles share
         // the codebook and there are enough of them to keep the chip full.  Longer runs would need the payloads of
@@ -2020,8 +2228,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         // eight waves per workgroup where they get little LDS (two such workgroups per compute unit): half as many tickets, of
         // which the chip hands out one in 11 ns.
         const int unit = a.vec_len == 72 ? 8 : 16;         // symbols per load (head_dim 72: rows start at multiples of eight)
-        const bool wide = front == 0 && a.rows_per_codebook == 0 && c.longest_code >= 1 && c.longest_code <= 8 && (uintptr_t)c.d_sym % unit == 0 && c.stride % unit == 0 &&
-                          (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 72 || a.vec_len == 64);
+        const bool wide = c.packed || (front == 0 && a.rows_per_codebook == 0 && c.longest_code >= 1 && c.longest_code <= 8 && (uintptr_t)c.d_sym % unit == 0 && c.stride % unit == 0 &&
+                          (a.vec_len == 128 || a.vec_len == 96 || a.vec_len == 72 || a.vec_len == 64));
         // Its 4096 waves at a time: runs of two from where single tiles would be a second, part-filled round of them.  K and
         // V of 2 x 32 heads x 128 x 6144 tokens (6144 tiles) in first stores: 50 -> 35 and 47 -> 32 us; K of 4 x 24 x 72 x 4096: 47 -> 31.
         // (V's runs of four begin where those of two would be a second round: 2 x 32 x 128 x 12 288 tokens 58 -> 51 us, 9216 49 -> 48.)
@@ -2031,12 +2239,9 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
         // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
         // together take stays inside a group, or the wave that speaks for a group would wait before all its tiles are counted).
-        if (wide && small && run == 2 && want == 1 && !is_k && a.tiles > 2 * KVC_WIDE_WAVES && 3 * (a.encoded_cap / a.tiles * 9 / 8) <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) run = 4;
+        if (wide && small && run == 2 && want == 1 && !is_k && a.tiles > 2 * KVC_WIDE_WAVES && 3 * (a.encoded_cap / a.tiles * 9 / 8) <= sa.e.wave_bytes - (c.packed ? KVC_STAGE_VPACKED_BYTES : KVC_STAGE_VF16_BYTES)) run = 4;
         const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
-        const auto symbols_kernel = !is_k ? kvc_encode_symbols_kernel<1, 32> :
-                                    a.vec_len == 128 ? kvc_encode_symbols_kernel<0, 32> :
-                                    a.vec_len == 96 ? kvc_encode_symbols_kernel<0, 24> :
-                                    a.vec_len == 72 ? kvc_encode_symbols_kernel<0, 18> : kvc_encode_symbols_kernel<0, 16>;
+        const auto symbols_kernel = kvc_symbols_kernel(is_k, a.vec_len, !c.packed ? KVC_FORM_BYTES : c.longest_code >= 1 && c.longest_code <= 8 ? KVC_FORM_PACKED : KVC_FORM_PACKED_LONG);
         if (wide) {
             hipLaunchKernelGGL(symbols_kernel, dim3(wgs1), dim3(waves * KVC_WAVE), lds, stream, sa.e, run);
             hipLaunchKernelGGL(kvc_encode_finish_kernel<0>, dim3(1), dim3(KVC_WG), 0, stream, sa);
@@ -2205,18 +2410,21 @@ static int kvc_encode_job_check(const kvc_encode_job *job, KvcEncodeCall &c)
     return 0;
 }
 
-extern "C" int64_t kvc_encode_scratch_bytes(void) { return KVC_WS_SLOT_BYTES; }
+// (more than a slot of the ring: a call from packed V symbols has more groups)
+constexpr int64_t KVC_ENC_SCRATCH_BYTES = KVC_WS_SLOT_BYTES + KVC_WS_SLOT_BYTES / 4;
+static_assert((KVC_ENC_SCRATCH_BYTES - KVC_ONCE_GROUP_WORD * 4) / 8 * KVC_ONCE_GROUP_TILES_VPACKED >= (int64_t)KVC_ONCE_MAX_GROUPS * KVC_ONCE_GROUP_TILES, "as many tiles");
+extern "C" int64_t kvc_encode_scratch_bytes(void) { return KVC_ENC_SCRATCH_BYTES; }
 
 // The launches in front of an encode whose table is not known yet (a first store: they run while the host builds the code).
-extern "C" int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream)
+static int kvc_encode_prepare_form(const kvc_encode_job *job, bool packed, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream)
 {
     KVC_REQUIRE(prepared != nullptr, "NULL argument");
     *prepared = KVC_ENC_FRESH;
     KvcEncodeCall c = {};
     if (int rc = kvc_encode_job_check(job, c)) return rc;
     KVC_REQUIRE(job->d_result != nullptr && job->d_stream_bytes != nullptr, "NULL argument");
-    KVC_REQUIRE(d_scratch != nullptr && ((uintptr_t)d_scratch & 15) == 0 && scratch_bytes >= (int64_t)KVC_WS_SLOT_BYTES, "scratch memory: %lld bytes, on a 16-byte boundary",
-                (long long)KVC_WS_SLOT_BYTES);
+    KVC_REQUIRE(d_scratch != nullptr && ((uintptr_t)d_scratch & 15) == 0 && scratch_bytes >= KVC_ENC_SCRATCH_BYTES, "scratch memory: %lld bytes, on a 16-byte boundary",
+                (long long)KVC_ENC_SCRATCH_BYTES);
     KVC_REQUIRE(job->d_sym != nullptr && job->rows_per_codebook == 0 && job->d_codebook_meta == nullptr, "only an encode from symbols with one codebook can be prepared");
     static const uint8_t no_table[8] = {};
     c.d_tables = no_table;                                 // (not read by the launch; the call has its own)
@@ -2224,11 +2432,23 @@ extern "C" int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, in
     c.scratch = d_scratch;
     c.clear = 1;
     c.first_launch_only = true;
+    c.packed = packed;
     void *slot;
     const int rc = kvc_encode_launch(c, &slot, (hipStream_t)stream);
     if (rc < 0) return rc;
-    *prepared = rc;
+    *prepared = rc | (packed ? KVC_ENC_PACKED : 0);
     return 0;
+}
+
+extern "C" int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream)
+{
+    return kvc_encode_prepare_form(job, false, d_scratch, scratch_bytes, prepared, stream);
+}
+
+// d_sym as kvc_quant_counted_packed writes it
+extern "C" int kvc_encode_prepare_packed(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream)
+{
+    return kvc_encode_prepare_form(job, true, d_scratch, scratch_bytes, prepared, stream);
 }
 
 extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,
@@ -2236,7 +2456,9 @@ extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int 
 {
     KvcEncodeCall c = {};
     if (int rc = kvc_encode_job_check(job, c)) return rc;
-    KVC_REQUIRE(prepared == KVC_ENC_FRESH || ((prepared == KVC_ENC_CLEARED || prepared == KVC_ENC_MARKED) && d_scratch && job->d_sym &&
+    c.packed = (prepared & KVC_ENC_PACKED) != 0;
+    if (c.packed) prepared &= ~KVC_ENC_PACKED;
+    KVC_REQUIRE((prepared == KVC_ENC_FRESH && !c.packed) || ((prepared == KVC_ENC_CLEARED || prepared == KVC_ENC_MARKED) && d_scratch && job->d_sym &&
                                               job->rows_per_codebook == 0 && job->d_result && job->d_stream_bytes),
                 "the call does not continue what was prepared");
     KVC_REQUIRE(h_outcome == nullptr || (job->d_result && job->d_stream_bytes && ((uintptr_t)h_outcome & 3) == 0), "an outcome needs d_result and d_stream_bytes");

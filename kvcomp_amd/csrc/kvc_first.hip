@@ -152,8 +152,8 @@ extern "C" int kvc_wait_outcome(const uint32_t *h_outcome, uint32_t outcome_numb
     }
 }
 
-extern "C" int kvc_quant_counted(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
-                                 float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, void **counted, void *stream_)
+static int kvc_quant_counted_form(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask, float eb,
+                                  uint8_t *d_sym, bool packed, int8_t *d_min_i8, void *d_scale_f16, void **counted, void *stream_)
 {
     hipStream_t stream = (hipStream_t)stream_;
     KVC_REQUIRE(counted != nullptr, "NULL argument");
@@ -169,7 +169,8 @@ extern "C" int kvc_quant_counted(const void *d_x_f16, int64_t NB, int64_t BS, in
         return rc;
     }
     block->calls++;
-    int rc = kvc_quant(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, d_min_i8, d_scale_f16, nullptr, (int64_t *)block->d_counts, stream_);
+    int rc = packed ? kvc_quant_packed(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, d_min_i8, d_scale_f16, (int64_t *)block->d_counts, stream_)
+                    : kvc_quant(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, d_min_i8, d_scale_f16, nullptr, (int64_t *)block->d_counts, stream_);
     if (!rc) {
         hipLaunchKernelGGL(kvc_counts_to_host_kernel, dim3(1), dim3(256), 0, stream, block->d_counts, block->h_counts, block->calls);
         rc = kvc_check_hip(hipGetLastError(), "kvc_counts_to_host_kernel launch");
@@ -182,6 +183,18 @@ extern "C" int kvc_quant_counted(const void *d_x_f16, int64_t NB, int64_t BS, in
     }
     *counted = block;
     return 0;
+}
+
+extern "C" int kvc_quant_counted(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
+                                 float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, void **counted, void *stream)
+{
+    return kvc_quant_counted_form(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, false, d_min_i8, d_scale_f16, counted, stream);
+}
+
+extern "C" int kvc_quant_counted_packed(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
+                                        float eb, uint8_t *d_packed, int8_t *d_min_i8, void *d_scale_f16, void **counted, void *stream)
+{
+    return kvc_quant_counted_form(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_packed, true, d_min_i8, d_scale_f16, counted, stream);
 }
 
 extern "C" int kvc_counted_codebook(void *counted, int smoothed_symbols, kvc_codebook *out, void *stream_)

@@ -14,6 +14,8 @@
 #include "kvc_common.h"
 #include "kvc_quant_math.h"
 
+#include <type_traits>
+
 struct KvcQuantArgs {
     const __half *x;
     int64_t NB, BS, B, H, D;
@@ -76,6 +78,15 @@ __device__ __forceinline__ void kvc_hist_flush(const KvcQuantArgs &a, uint32_t *
     }
 }
 
+// ---------------------------------------------------------------------------------------------------
+// two symbols per byte (PACK kernels; kvc_packed_symbols in kvc_common.h says where they go)
+// ---------------------------------------------------------------------------------------------------
+// bytes 0 .. 7 of eight adjacent symbols below 16 -> four bytes, the even one of each pair in the low half
+__device__ __forceinline__ uint32_t kvc_pack8(const uint2 &w)
+{
+    return kvc_low_bytes4(w.x | (w.x >> 4), w.y | (w.y >> 4));
+}
+
 // Writes the symbols and/or the simulated-quantization values of two adjacent elements.
 __device__ __forceinline__ void kvc_quant_store2(const KvcQuantArgs &a, int64_t i, float v0, float v1,
                                                  const KvcGroupParams &g0, const KvcGroupParams &g1)
@@ -90,7 +101,7 @@ __device__ __forceinline__ void kvc_quant_store2(const KvcQuantArgs &a, int64_t 
 }
 
 // ... of eight adjacent elements of one group (i a multiple of 8; 8- and 16-byte stores)
-template <int GSTEP>   // element k belongs to group g[k * GSTEP]: 0 = one group for all eight, 1 = a group each
+template <int GSTEP, bool PACK = false>   // element k belongs to group g[k * GSTEP]: 0 = one group for all eight, 1 = a group each; PACK: the caller stores the symbols
 __device__ __forceinline__ uint2 kvc_quant_store8(const KvcQuantArgs &a, int64_t i, const uint4 &raw, const KvcGroupParams *g)
 {
     uint2 sym = make_uint2(0u, 0u);
@@ -109,7 +120,7 @@ __device__ __forceinline__ uint2 kvc_quant_store8(const KvcQuantArgs &a, int64_t
             hi |= (uint32_t)kvc_quant_one(v[4 + k], g[(4 + k) * GSTEP]) << (8 * k);
         }
         sym = make_uint2(lo, hi);
-        *reinterpret_cast<uint2 *>(a.sym + i) = sym;
+        if constexpr (!PACK) *reinterpret_cast<uint2 *>(a.sym + i) = sym;
     }
     if (a.xhat) {
         uint32_t o[4];
@@ -213,7 +224,11 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_channel8_kernel(KvcQuantArgs
 // 64 tokens in registers, so the block is read once (64 loads in flight), finds minima and maxima with packed fp16
 // min / max and quantizes two channels per instruction (kvc_quant_pair_biased: the same symbols as the fp32 chain for
 // every fp16 input, see kvc_quant_math.h).
-template <bool HIST>
+//
+// PACK (first stores, which encode the symbols and drop them): two symbols per byte, a tile's in the order in which the encoder's
+// lanes load them (kvc_packed_symbols).  Four neighbouring lanes exchange their bytes of four tokens, so that a lane stores
+// eight channels of one token: sixteen stores instead of 64.
+template <bool HIST, bool PACK>
 __global__ void __launch_bounds__(KVC_WG) kvc_quant_channel_once_kernel(KvcQuantArgs a)
 {
     __shared__ uint32_t s_bins[HIST ? KVC_HIST_BINS * 32 : 1];
@@ -226,7 +241,11 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_channel_once_kernel(KvcQuant
         const __half *p = a.x + base;
         uint32_t raw[KVC_WAVE];
 #pragma unroll
-        for (int t = 0; t < KVC_WAVE; t++) raw[t] = *reinterpret_cast<const uint32_t *>(p + t * stride);
+        for (int t = 0; t < KVC_WAVE; t += 8, p += 8 * stride) {
+            asm volatile("" : "+v"(p));                    // (or 64 multiples of the stride are kept in scalar registers, and spilled)
+#pragma unroll
+            for (int k = 0; k < 8; k++) raw[t + k] = *reinterpret_cast<const uint32_t *>(p + k * stride);
+        }
         kvc_half2 mn = __builtin_bit_cast(kvc_half2, raw[0]), mx = mn;
 #pragma unroll
         for (int t = 1; t < KVC_WAVE; t++) {
@@ -240,7 +259,42 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_channel_once_kernel(KvcQuant
         const int64_t g = nb * stride + c;
         kvc_quant_publish(a, g, g0);
         kvc_quant_publish(a, g + 1, g1);
-        if (kvc_packed_quantizer_applies(g0, kvc_half_lo(mxw)) && kvc_packed_quantizer_applies(g1, kvc_half_hi(mxw))) {
+        const bool applies = kvc_packed_quantizer_applies(g0, kvc_half_lo(mxw)) && kvc_packed_quantizer_applies(g1, kvc_half_hi(mxw));
+        if constexpr (PACK) {
+            // (lanes exchange bytes: all of a wave take one way.  The fp32 chain gives the same symbols, to whichever lane)
+            const bool packed = __all(applies);
+            const KvcPackedParams pp = kvc_packed_params(g0, g1);
+            const uint32_t D = (uint32_t)a.D, col = (uint32_t)c / D, lane = threadIdx.x & 3;
+            uint8_t *dst = a.sym + (nb * (stride / D) + col) * (KVC_WAVE / 2 * D) + kvc_packed_k_place(D, (uint32_t)c - col * D, lane);
+            const uint32_t sel1 = lane & 1 ? 0x03070105u : 0x06020400u, sel2 = lane & 2 ? 0x03020706u : 0x05040100u;
+            auto store = [&](auto chunk) {                             // (the offsets are constants then)
+#pragma unroll
+                for (int t = 0; t < KVC_WAVE; t += 4) {
+                    uint2 w;
+                    if (packed) {
+                        w.x = kvc_low_bytes4(kvc_quant_pair_biased(raw[t], pp), kvc_quant_pair_biased(raw[t + 1], pp));
+                        w.y = kvc_low_bytes4(kvc_quant_pair_biased(raw[t + 2], pp), kvc_quant_pair_biased(raw[t + 3], pp));
+                    } else {
+                        uint32_t s[4];
+#pragma unroll
+                        for (int k = 0; k < 4; k++)
+                            s[k] = (uint32_t)kvc_quant_one(kvc_half_lo(raw[t + k]), g0) | (uint32_t)kvc_quant_one(kvc_half_hi(raw[t + k]), g1) << 8;
+                        w = make_uint2(s[0] | s[1] << 16, s[2] | s[3] << 16);
+                    }
+                    if constexpr (HIST) {
+                        kvc_hist_add4(a, s_bins, w.x);
+                        kvc_hist_add4(a, s_bins, w.y);
+                    }
+                    const uint32_t mine = kvc_pack8(w);                // this lane's two channels of four tokens, a byte each
+                    const uint32_t next = (uint32_t)__builtin_amdgcn_mov_dpp((int)mine, 0xB1, 0xf, 0xf, true);     // lane ^ 1
+                    const uint32_t four = __builtin_amdgcn_perm(next, mine, sel1);                                 // four channels of two tokens
+                    const uint32_t over = (uint32_t)__builtin_amdgcn_mov_dpp((int)four, 0x4E, 0xf, 0xf, true);     // lane ^ 2
+                    *reinterpret_cast<uint32_t *>(dst + t * chunk.value) = __builtin_amdgcn_perm(over, four, sel2);       // eight of one
+                }
+            };
+            if (kvc_packed_k_chunk(D) == 16) store(std::integral_constant<int, 16>());
+            else store(std::integral_constant<int, 4>());
+        } else if (applies) {
             const KvcPackedParams pp = kvc_packed_params(g0, g1);
             const uint32_t min2 = kvc_half_pair_bits(g0.min_h, g1.min_h), scale2 = kvc_half_pair_bits(g0.scale_h, g1.scale_h);
 #pragma unroll
@@ -312,7 +366,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_kernel(KvcQuantArgs a, i
 // Bound by HBM (2 bytes in, 1 out per element).  One wave per row up to 16 384 elements; longer rows do not fit a wave's
 // registers and are spread over the workgroup's four waves, whose minima and maxima meet in LDS: rows of 32 768 (4096 of
 // them, with counts) 82 us against 138 us (without) for kvc_quant_row_kernel, which reads every row twice.
-template <int NIT, int WPR, bool HIST>
+template <int NIT, int WPR, bool HIST, bool PACK>
 __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_once_kernel(KvcQuantArgs a, int64_t R, int64_t groups)
 {
     static_assert(WPR == 1 || WPR == KVC_WAVES_PER_WG, "a wave or a workgroup per row");
@@ -377,7 +431,8 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_once_kernel(KvcQuantArgs
             for (int j = 0; j < NIT; j++) {
                 const int64_t i = 8 * at + STEP * j;
                 if (i < R) {
-                    const uint2 w = kvc_quant_store8<0>(a, g * R + i, raw[j], &gp);
+                    const uint2 w = kvc_quant_store8<0, PACK>(a, g * R + i, raw[j], &gp);
+                    if constexpr (PACK) *reinterpret_cast<uint32_t *>(a.sym + ((g * R + i) >> 1)) = kvc_pack8(w);
                     if constexpr (HIST) {
                         kvc_hist_add4(a, s_bins, w.x);
                         kvc_hist_add4(a, s_bins, w.y);
@@ -395,12 +450,13 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_once_kernel(KvcQuantArgs
                 const uint32_t u0 = kvc_quant_pair_biased(raw[j].x, pp), u1 = kvc_quant_pair_biased(raw[j].y, pp);
                 const uint32_t u2 = kvc_quant_pair_biased(raw[j].z, pp), u3 = kvc_quant_pair_biased(raw[j].w, pp);
                 const uint2 w = make_uint2(kvc_low_bytes4(u0, u1), kvc_low_bytes4(u2, u3));
-                if (a.sym) *reinterpret_cast<uint2 *>(a.sym + g * R + i) = w;
+                if constexpr (PACK) *reinterpret_cast<uint32_t *>(a.sym + ((g * R + i) >> 1)) = kvc_pack8(w);
+                else if (a.sym) *reinterpret_cast<uint2 *>(a.sym + g * R + i) = w;
                 if constexpr (HIST) {
                     kvc_hist_add4(a, s_bins, w.x);
                     kvc_hist_add4(a, s_bins, w.y);
                 }
-                if (a.xhat)
+                if (!PACK && a.xhat)
                     *reinterpret_cast<uint4 *>(a.xhat + g * R + i) = make_uint4(kvc_quant_error_pair(u0, min2, scale2), kvc_quant_error_pair(u1, min2, scale2),
                                                                                kvc_quant_error_pair(u2, min2, scale2), kvc_quant_error_pair(u3, min2, scale2));
             }
@@ -409,7 +465,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_once_kernel(KvcQuantArgs
     if constexpr (HIST) kvc_hist_flush(a, s_bins);
 }
 
-template <bool HIST>
+template <bool HIST, bool PACK>
 static void kvc_launch_row_once(const KvcQuantArgs &a, int64_t R, int64_t groups, hipStream_t stream)
 {
     auto grid = [&](int waves_per_row) {
@@ -417,12 +473,12 @@ static void kvc_launch_row_once(const KvcQuantArgs &a, int64_t R, int64_t groups
         return dim3((unsigned)(HIST && wgs > KVC_HIST_WGS ? KVC_HIST_WGS : wgs));
     };
     constexpr int W = KVC_WAVES_PER_WG;
-    if (R <= 512 * 8) hipLaunchKernelGGL((kvc_quant_row_once_kernel<8, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * 24) hipLaunchKernelGGL((kvc_quant_row_once_kernel<24, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * 32) hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, 1, HIST>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * W * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, W, HIST>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
-    else hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, W, HIST>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
+    if (R <= 512 * 8) hipLaunchKernelGGL((kvc_quant_row_once_kernel<8, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * 24) hipLaunchKernelGGL((kvc_quant_row_once_kernel<24, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * 32) hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
+    else if (R <= 512 * W * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, W, HIST, PACK>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
+    else hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, W, HIST, PACK>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
 }
 constexpr int64_t KVC_ROW_ONCE_MAX = 512 * KVC_WAVES_PER_WG * 32;
 
@@ -520,7 +576,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_block_minmax8_kernel(KvcQuan
     }
 }
 
-template <bool HIST>
+template <bool HIST, bool PACK>
 __global__ void __launch_bounds__(KVC_WG) kvc_quant_block_apply8_kernel(KvcQuantArgs a, int64_t R, int64_t rows)
 {
     __shared__ uint32_t s_bins[HIST ? KVC_HIST_BINS * 32 : 1];
@@ -544,12 +600,17 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_block_apply8_kernel(KvcQuant
                 const uint32_t u0 = kvc_quant_pair_biased(v.x, pp), u1 = kvc_quant_pair_biased(v.y, pp);
                 const uint32_t u2 = kvc_quant_pair_biased(v.z, pp), u3 = kvc_quant_pair_biased(v.w, pp);
                 w = make_uint2(kvc_low_bytes4(u0, u1), kvc_low_bytes4(u2, u3));
-                if (a.sym) *reinterpret_cast<uint2 *>(a.sym + base + i) = w;
-                if (a.xhat)
+                if (!PACK && a.sym) *reinterpret_cast<uint2 *>(a.sym + base + i) = w;
+                if (!PACK && a.xhat)
                     *reinterpret_cast<uint4 *>(a.xhat + base + i) = make_uint4(kvc_quant_error_pair(u0, min2, scale2), kvc_quant_error_pair(u1, min2, scale2),
                                                                               kvc_quant_error_pair(u2, min2, scale2), kvc_quant_error_pair(u3, min2, scale2));
             } else {
-                w = kvc_quant_store8<0>(a, base + i, v, &gp);
+                w = kvc_quant_store8<0, PACK>(a, base + i, v, &gp);
+            }
+            if constexpr (PACK) {                          // (K: a row is a token)
+                const uint32_t D = (uint32_t)a.D, col = (uint32_t)i / D, t = (uint32_t)(row % KVC_WAVE);
+                uint8_t *tile = a.sym + (row / KVC_WAVE * (R / D) + col) * (KVC_WAVE / 2 * D);
+                *reinterpret_cast<uint32_t *>(tile + kvc_packed_k_place(D, (uint32_t)i - col * D, t)) = kvc_pack8(w);
             }
             if constexpr (HIST) {
                 kvc_hist_add4(a, s_bins, w.x);
@@ -566,10 +627,11 @@ extern "C" int64_t kvc_quant_groups(int64_t NB, int64_t BS, int64_t B, int64_t H
 }
 
 extern "C" int kvc_histogram(const uint8_t *d_sym, int64_t n, int64_t *d_counts, void *stream);
+extern "C" int kvc_packed_symbols_supported(int is_k, int quant_mask, int64_t batch, int64_t heads, int64_t head_dim, float eb);
 
 static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                             float eb, uint8_t *d_sym, int8_t *d_min_i8, void *d_scale_f16, void *d_min_f16,
-                            void *d_xhat_f16, int64_t *d_counts, void *stream_)
+                            void *d_xhat_f16, int64_t *d_counts, void *stream_, bool pack = false)
 {
     hipStream_t stream = (hipStream_t)stream_;
     KVC_REQUIRE(NB >= 0 && BS > 0 && B > 0 && H > 0 && D > 0, "bad shape");
@@ -577,6 +639,9 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
     KVC_REQUIRE(((uintptr_t)d_x_f16 & 3) == 0 && ((uintptr_t)d_sym & 1) == 0 && ((uintptr_t)d_xhat_f16 & 3) == 0,
                 "quantizer buffers are misaligned");
     KVC_REQUIRE(eb > 0.f, "error bound must be positive");
+    KVC_REQUIRE(!pack || (d_counts && d_sym && !d_xhat_f16 && (quant_mask == KVC_MASK_V_TOKEN || BS == KVC_WAVE) && (((uintptr_t)d_x_f16 | (uintptr_t)d_sym) & 15) == 0 &&
+                          kvc_packed_symbols_supported(quant_mask != KVC_MASK_V_TOKEN, quant_mask, B, H, D, eb)),
+                "these symbols cannot be packed");
     if (NB == 0) return 0;
     KvcQuantArgs a;
     a.x = reinterpret_cast<const __half *>(d_x_f16);
@@ -599,9 +664,11 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
         const int64_t threads = NB * (once || !wide ? stride / 2 : stride / 8);
         const dim3 grid((unsigned)((threads + KVC_WG - 1) / KVC_WG));
         if (once && want_counts) {
-            hipLaunchKernelGGL(kvc_quant_channel_once_kernel<true>, dim3(grid.x > KVC_HIST_WGS ? KVC_HIST_WGS : grid.x), dim3(KVC_WG), 0, stream, a);
+            const dim3 few(grid.x > KVC_HIST_WGS ? KVC_HIST_WGS : grid.x);
+            if (pack) hipLaunchKernelGGL((kvc_quant_channel_once_kernel<true, true>), few, dim3(KVC_WG), 0, stream, a);
+            else hipLaunchKernelGGL((kvc_quant_channel_once_kernel<true, false>), few, dim3(KVC_WG), 0, stream, a);
             counted = true;
-        } else if (once) hipLaunchKernelGGL(kvc_quant_channel_once_kernel<false>, grid, dim3(KVC_WG), 0, stream, a);
+        } else if (once) hipLaunchKernelGGL((kvc_quant_channel_once_kernel<false, false>), grid, dim3(KVC_WG), 0, stream, a);
         else if (wide) hipLaunchKernelGGL(kvc_quant_channel8_kernel, grid, dim3(KVC_WG), 0, stream, a);
         else hipLaunchKernelGGL(kvc_quant_channel_kernel, grid, dim3(KVC_WG), 0, stream, a);
     } else if (quant_mask == KVC_MASK_V_TOKEN || quant_mask == KVC_MASK_SIM_TOKEN || quant_mask == KVC_MASK_VECTOR) {
@@ -611,8 +678,9 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
         const dim3 grid((unsigned)((groups + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG));
         // the row fits the registers of a wave or a workgroup
         const bool once = wide && (a.sym != nullptr || a.xhat != nullptr) && R >= 512 && R <= KVC_ROW_ONCE_MAX;
-        if (once && want_counts) kvc_launch_row_once<true>(a, R, groups, stream);
-        else if (once) kvc_launch_row_once<false>(a, R, groups, stream);
+        if (once && pack) kvc_launch_row_once<true, true>(a, R, groups, stream);
+        else if (once && want_counts) kvc_launch_row_once<true, false>(a, R, groups, stream);
+        else if (once) kvc_launch_row_once<false, false>(a, R, groups, stream);
         else hipLaunchKernelGGL(kvc_quant_row_kernel, grid, dim3(KVC_WG), 0, stream, a, R, groups, wide);
         counted = once && want_counts;
     } else if (quant_mask == KVC_MASK_K_BLOCK || quant_mask == KVC_MASK_SIM_BLOCK) {
@@ -629,11 +697,12 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
         if (wide) hipLaunchKernelGGL(kvc_quant_block_minmax8_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
         else hipLaunchKernelGGL(kvc_quant_block_minmax_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
         if (wide && want_counts) {
-            hipLaunchKernelGGL(kvc_quant_block_apply8_kernel<true>, dim3(row_wgs > KVC_HIST_WGS ? KVC_HIST_WGS : row_wgs), dim3(KVC_WG), 0, stream,
-                               a, R, rows);
+            const dim3 few(row_wgs > KVC_HIST_WGS ? KVC_HIST_WGS : row_wgs);
+            if (pack) hipLaunchKernelGGL((kvc_quant_block_apply8_kernel<true, true>), few, dim3(KVC_WG), 0, stream, a, R, rows);
+            else hipLaunchKernelGGL((kvc_quant_block_apply8_kernel<true, false>), few, dim3(KVC_WG), 0, stream, a, R, rows);
             counted = true;
         } else if (wide && (a.sym || a.xhat)) {
-            hipLaunchKernelGGL(kvc_quant_block_apply8_kernel<false>, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
+            hipLaunchKernelGGL((kvc_quant_block_apply8_kernel<false, false>), dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
         } else {
             hipLaunchKernelGGL(kvc_quant_block_apply_kernel, dim3(row_wgs), dim3(KVC_WG), 0, stream, a, R, rows);
         }
@@ -641,6 +710,7 @@ static int kvc_quant_launch(const void *d_x_f16, int64_t NB, int64_t BS, int64_t
         return kvc_fail(-1, "unsupported quantization group mask 0x%x", quant_mask);
     }
     KVC_HIP(hipGetLastError());
+    KVC_REQUIRE(!pack || counted, "these symbols cannot be packed");
     if (want_counts && !counted) return kvc_histogram(d_sym, NB * BS * stride, d_counts, stream_);
     return 0;
 }
@@ -652,6 +722,27 @@ extern "C" int kvc_quant(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B,
     KVC_REQUIRE(d_sym != nullptr && d_min_i8 != nullptr && d_scale_f16 != nullptr, "output pointer is NULL");
     return kvc_quant_launch(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, d_min_i8, d_scale_f16, d_min_f16, nullptr,
                             d_counts, stream);
+}
+
+// The layouts whose symbols go two to a byte on their way to the encoder: the error bound gives at most 16 of them (a group's range is 1 / eb
+// steps, whose two ends may round outwards; scales among fp16's smallest numbers can give more, which the counts then say),
+// vectors have a length that the encoder's kernel for them is compiled for, and a quantizer that counts writes them.
+extern "C" int kvc_packed_symbols_supported(int is_k, int quant_mask, int64_t batch, int64_t heads, int64_t head_dim, float eb)
+{
+    if (batch <= 0 || heads <= 0 || head_dim <= 0 || !(eb >= 1.0f / 13.0f)) return 0;
+    const int64_t stride = batch * heads * head_dim;
+    if (is_k)
+        return (head_dim == 128 || head_dim == 96 || head_dim == 72 || head_dim == 64) && stride <= INT32_MAX / KVC_WAVE &&
+               (quant_mask == KVC_MASK_CHANNEL || quant_mask == KVC_MASK_K_BLOCK);
+    return quant_mask == KVC_MASK_V_TOKEN && stride % KVC_V_VEC_PER_BLK == 0 && stride >= 512 && stride <= KVC_ROW_ONCE_MAX;
+}
+
+// kvc_quant with counts, the symbols two to a byte (kvc_packed_symbols in kvc_common.h); only counts below 16 say that they fit
+int kvc_quant_packed(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask, float eb,
+                     uint8_t *d_packed, int8_t *d_min_i8, void *d_scale_f16, int64_t *d_counts, void *stream)
+{
+    KVC_REQUIRE(d_packed != nullptr && d_min_i8 != nullptr && d_scale_f16 != nullptr, "output pointer is NULL");
+    return kvc_quant_launch(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_packed, d_min_i8, d_scale_f16, nullptr, nullptr, d_counts, stream, true);
 }
 
 // group parameters (min_i8, scale) without symbols: the first pass of the fused quantize + encode path

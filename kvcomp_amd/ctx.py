@@ -507,7 +507,7 @@ class KVCompCtx:
     def store(self, cache: torch.Tensor, want_symbols: bool = True):
         """kvcomp_encode.py:69-136: append [T_new, B, H, D]; compress the whole blocks that leave the tail.
         Returns the uint8 symbols that were compressed (None if nothing left the tail, or if want_symbols is
-        False and the fused quantize + encode path ran)."""
+        False and they were never written out a byte each)."""
         self._check(cache)
         if self.device is None:
             self.device = cache.device
@@ -570,7 +570,7 @@ class KVCompCtx:
             return None
         blocked = to_compress.reshape(-1, self.block_size, self.batch_size, self.head_num, self.head_dim)
         if self.encode_codebook is None and self.device_codebook:
-            return self._first_chunk(blocked)
+            return self._first_chunk(blocked, want_symbols)
         quant_ints, min_ints, quant_scale = quant(blocked, self.quant_dims, self.quant_scale_rel)
         sizes = kvcomp_cuda.calculate_buffer_size(quant_ints, self.is_k, self.head_num, self.head_dim)
         KVCompCtx.buffer_ctx_len[self.device] = to_compress.shape[0]
@@ -671,7 +671,7 @@ class KVCompCtx:
         if outcome is not None:
             self._probe = (outcome, len(self._unverified), outcome.stream)
 
-    def _prepare_encode(self, T: int, symbols: torch.Tensor):
+    def _prepare_encode(self, T: int, symbols: torch.Tensor, packed: bool):
         """For a first store, while the quantizer runs: the buffers of the encode and the launch that needs no codebook."""
         B, H, D = self.batch_size, self.head_num, self.head_dim
         sizes = kvcomp_cuda.buffer_sizes(T, B * H * D, self.is_k, H, D)
@@ -679,30 +679,38 @@ class KVCompCtx:
         ti = self._thread_infos.reserve(sizes[1], (), torch.uint8, self.device)
         state = torch.empty(16, dtype=torch.int32, device=self.device)
         prepared = kvcomp_cuda.encode_prepare(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, symbols=symbols,
-                                              block_infos=bi, thread_infos=ti, state=state)
+                                              block_infos=bi, thread_infos=ti, state=state, packed=packed)
         self._state = state                                    # (cleared, on this stream)
         self._ask_outcome()
         return prepared
 
-    def _first_chunk(self, blocked: torch.Tensor) -> torch.Tensor:
+    def _first_chunk(self, blocked: torch.Tensor, want_symbols: bool = True) -> Optional[torch.Tensor]:
         """The first stored chunk: quantized, its codebook built from the symbols just written (kvcomp_encode.py:86-103; the
         one thing that is waited for) and encoded with it.  The counts and the code lengths bound the payload to within a
         byte per lane stream, so the buffer is as large as the stream needs, and with them at hand neither a symbol without
         a code nor too small a buffer is possible; with codes of at most seven bits nor is a tile beyond 8191 bytes, so
-        the encode need not be waited for either."""
+        the encode need not be waited for either.  Symbols that nobody asked for go from the quantizer to the encoder two to a
+        byte where there are at most sixteen of them, and are not returned."""
         nb, T, device = blocked.shape[0], blocked.shape[0] * self.block_size, self.device
         gshape = mask_keepdim_shape(blocked.shape, self._mask)
         min_ints = self._min_ints.reserve(nb, gshape[1:], torch.int8, device)
         quant_scale = self._scales.reserve(nb, gshape[1:], torch.float16, device)
         prepared = []
 
+        fresh = self._state is None and self._encoded.used == 0
+        packed = not want_symbols and fresh and kvcomp_cuda.packed_symbols_supported(self.is_k, self._mask, blocked, self.quant_scale_rel)
+
         def meanwhile(symbols):
-            if self._state is None and self._encoded.used == 0:
-                prepared.extend((self._prepare_encode(T, symbols), kvcomp_cuda.codebook_room(device)))
-        sym, book = kvcomp_cuda.quant_codebook(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale,
+            if fresh:
+                prepared.extend((self._prepare_encode(T, symbols, packed), kvcomp_cuda.codebook_room(device)))
+        quantize = kvcomp_cuda.quant_codebook_packed if packed else kvcomp_cuda.quant_codebook
+        sym, book = quantize(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale,
                                                self._smoothed_symbols() if self.codebook_smoothing else 0, meanwhile)
         self.waits += 1
         enc, dec, lut = kvcomp_cuda.put_codebook(book, device, *prepared[1:])
+        if packed and book.encode_bytes > 16 * 8:              # scales among fp16's smallest numbers: half a byte does not hold these symbols
+            sym = quant(blocked, self.quant_dims, self.quant_scale_rel)[0]
+            prepared, packed = [], False
         vectors = T * self.batch_size * self.head_num * self.head_dim // (self.head_dim if self.is_k else kvcomp_cuda.V_VEC_LEN)
         cannot_fail = book.max_code_bits <= 7
         small = T <= self.ASYNC_KEEP_BLOCKS * self.block_size
@@ -717,7 +725,7 @@ class KVCompCtx:
         self.tree_format, self.max_code_bits, self.pair_bits = book.tree_format, book.max_code_bits, book.pair_bits
         self.encode_codebook, self.decode_codebook = enc, dec
         self._lut, self._lut_source = lut, dec
-        return sym
+        return None if packed else sym
 
     def _smoothed_symbols(self) -> int:
         return min(256, int(math.ceil(1.0 / self.quant_scale_rel)) + 3)      # symbols 0 .. ceil(1 / eb) + 2

@@ -143,13 +143,31 @@ def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: floa
     """kvc_quant_codebook on a device fp16 [NB, BS, B, H, D] tensor: (symbols uint8 of the same shape, _lib.Codebook).
     min_ints (int8) and scales (fp16) receive the group parameters.  Waits for the symbol counts only; `meanwhile`, if given, is
     called with the symbol tensor between the call's halves (kvc_quant_counted, kvc_counted_codebook), the quantizer being queued."""
+    return _quant_codebook(blocked, quant_mask, quant_scale_rel, min_ints, scales, smoothed_symbols, meanwhile, False)
+
+
+def quant_codebook_packed(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: float, min_ints: torch.Tensor, scales: torch.Tensor,
+                          smoothed_symbols: int, meanwhile):
+    """quant_codebook with the symbols two to a byte, for encode_prepare(packed=True) (kvc_quant_counted_packed; where
+    packed_symbols_supported).  They are worth nothing if the codebook turns out to have more than sixteen entries."""
+    return _quant_codebook(blocked, quant_mask, quant_scale_rel, min_ints, scales, smoothed_symbols, meanwhile, True)
+
+
+def packed_symbols_supported(is_k: bool, quant_mask: int, blocked: torch.Tensor, quant_scale_rel: float) -> bool:
+    """Whether the symbols of a contiguous [NB, BS, B, H, D] tensor can go to the encoder two to a byte."""
+    if not blocked.is_cuda or blocked.data_ptr() % 16 or (is_k and blocked.shape[1] != K_VEC_PER_BLK):
+        return False
+    return bool(_lib.lib().kvc_packed_symbols_supported(int(is_k), quant_mask, *blocked.shape[2:], float(quant_scale_rel)))
+
+
+def _quant_codebook(blocked, quant_mask, quant_scale_rel, min_ints, scales, smoothed_symbols, meanwhile, packed):
     _require(blocked.is_cuda and blocked.dtype == torch.float16 and blocked.dim() == 5 and blocked.is_contiguous(),
              "a contiguous device float16 tensor of shape [NB, BS, B, H, D] is expected")
     L = _lib.lib()
     groups = L.kvc_quant_groups(*blocked.shape, quant_mask)
     _require(min_ints.is_cuda and min_ints.dtype == torch.int8 and min_ints.numel() >= groups, "min_ints: int8 device tensor of the group count")
     _require(scales.is_cuda and scales.dtype == torch.float16 and scales.numel() >= groups, "scales: fp16 device tensor of the group count")
-    sym = torch.empty(blocked.shape, dtype=torch.uint8, device=blocked.device)
+    sym = torch.empty(blocked.numel() // 2 if packed else blocked.shape, dtype=torch.uint8, device=blocked.device)
     book = _lib.Codebook()
     stream = _lib.stream_of(blocked)
     with _lib.device_guard(blocked):
@@ -158,7 +176,7 @@ def quant_codebook(blocked: torch.Tensor, quant_mask: int, quant_scale_rel: floa
             check(L.kvc_quant_codebook(*args, smoothed_symbols, C.byref(book), stream))
             return sym, book
         counted = C.c_void_p(0)
-        check(L.kvc_quant_counted(*args, C.byref(counted), stream))
+        check((L.kvc_quant_counted_packed if packed else L.kvc_quant_counted)(*args, C.byref(counted), stream))
         try:
             meanwhile(sym)
         finally:
@@ -322,14 +340,14 @@ class PreparedEncode(NamedTuple):
 
 
 def encode_prepare(is_k: bool, *, batch: int, head_num: int, head_dim: int, tokens: int, symbols: torch.Tensor,
-                   block_infos: torch.Tensor, thread_infos: torch.Tensor, state: torch.Tensor):
+                   block_infos: torch.Tensor, thread_infos: torch.Tensor, state: torch.Tensor, packed: bool = False):
     """kvc_encode_prepare: what an encode from `symbols` can have done before its table is known.  `state` (device int32[16]):
     its first eight words are the encode's `result`, word 8 its `stream_bytes`; they are cleared.  encode_prepared does the
-    rest, on the same stream."""
+    rest, on the same stream.  packed: the symbols are quant_codebook_packed's."""
     L = _lib.lib()
     _dev_u8(symbols, "symbols")
     sizes = buffer_sizes(tokens, batch * head_num * head_dim, is_k, head_num, head_dim)
-    _require(symbols.is_contiguous() and symbols.numel() == tokens * batch * head_num * head_dim, "symbols: wrong size")
+    _require(symbols.is_contiguous() and symbols.numel() == tokens * batch * head_num * head_dim // (2 if packed else 1), "symbols: wrong size")
     for t, n, need in ((block_infos, "block_infos", sizes[0]), (thread_infos, "thread_infos", sizes[1])):
         _dev_u8(t, n)
         _require(t.numel() >= need, n + " buffer too small")
@@ -340,7 +358,7 @@ def encode_prepare(is_k: bool, *, batch: int, head_num: int, head_dim: int, toke
     scratch = torch.empty(L.kvc_encode_scratch_bytes(), dtype=torch.uint8, device=symbols.device)
     done = C.c_int(0)
     with _lib.device_guard(symbols):
-        check(L.kvc_encode_prepare(C.byref(job), scratch.data_ptr(), scratch.numel(), C.byref(done), _lib.stream_of(symbols)))
+        check((L.kvc_encode_prepare_packed if packed else L.kvc_encode_prepare)(C.byref(job), scratch.data_ptr(), scratch.numel(), C.byref(done), _lib.stream_of(symbols)))
     return PreparedEncode(job, scratch, done.value, sizes)
 
 
