@@ -44,7 +44,7 @@ constexpr int KVC_HIST_WGS = 1536;          // at most this many workgroups: eac
 
 __device__ __forceinline__ void kvc_hist_clear(uint32_t *s_bins)
 {
-    for (int i = threadIdx.x; i < KVC_HIST_BINS * 32; i += KVC_WG) s_bins[i] = 0;
+    for (int i = threadIdx.x; i < KVC_HIST_BINS * 32; i += (int)blockDim.x) s_bins[i] = 0;
     __syncthreads();
 }
 // four symbols, one per byte
@@ -363,17 +363,18 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_kernel(KvcQuantArgs a, i
 // Row groups of at least 512 elements and at most 512 NIT WPR (a multiple of 8, 16-byte aligned buffers), symbols and / or
 // simulated-quantization values out: WPR waves keep the row in registers (NIT 16-byte loads per lane in flight), so it is
 // read once, and quantize two elements per instruction (kvc_quant_pair_biased, as the per-channel kernel above).
-// Bound by HBM (2 bytes in, 1 out per element).  One wave per row up to 16 384 elements; longer rows do not fit a wave's
-// registers and are spread over the workgroup's four waves, whose minima and maxima meet in LDS: rows of 32 768 (4096 of
-// them, with counts) 82 us against 138 us (without) for kvc_quant_row_kernel, which reads every row twice.
+// Bound by HBM: 2 bytes per element in, 1 or half a one out.  One wave per row up to 8192 elements; longer rows are spread over 4
+// or 8 waves, a workgroup each, whose minima and maxima meet in LDS: 8 loads per lane leave six waves per SIMD, where a wave
+// with a row of 12 288 or 16 384 to itself had two.  134 M elements, counted and packed: rows of 12 288 80 -> 67 us, 16 384 87 -> 68,
+// 32 768 (16 loads by four waves before) 73 -> 66, 65 536 (32 by four before, a byte per symbol: 94) 79; a large copy of as many bytes takes 66.  Shorter rows do not pay the workgroup's
+// barriers (8192: 67 by one wave, 69 by four; 4096: 68 and 81).
 template <int NIT, int WPR, bool HIST, bool PACK>
-__global__ void __launch_bounds__(KVC_WG) kvc_quant_row_once_kernel(KvcQuantArgs a, int64_t R, int64_t groups)
+__global__ void __launch_bounds__(WPR == 1 ? KVC_WG : WPR * KVC_WAVE) kvc_quant_row_once_kernel(KvcQuantArgs a, int64_t R, int64_t groups)
 {
-    static_assert(WPR == 1 || WPR == KVC_WAVES_PER_WG, "a wave or a workgroup per row");
     __shared__ uint32_t s_bins[HIST ? KVC_HIST_BINS * 32 : 1];
-    __shared__ float s_lo[KVC_WAVES_PER_WG], s_hi[KVC_WAVES_PER_WG];
+    __shared__ float s_lo[WPR], s_hi[WPR];
     if constexpr (HIST) kvc_hist_clear(s_bins);
-    constexpr int ROWS = KVC_WAVES_PER_WG / WPR;           // rows of a workgroup
+    constexpr int ROWS = WPR == 1 ? KVC_WAVES_PER_WG : 1;  // rows of a workgroup
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int at = WPR == 1 ? lane : (int)threadIdx.x;     // this thread's place among those of the row
     constexpr int STEP = 512 * WPR;
@@ -465,22 +466,26 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_row_once_kernel(KvcQuantArgs
     if constexpr (HIST) kvc_hist_flush(a, s_bins);
 }
 
+template <int NIT, int WPR, bool HIST, bool PACK>
+static void kvc_launch_row_once_of(const KvcQuantArgs &a, int64_t R, int64_t groups, hipStream_t stream)
+{
+    const int64_t rows = WPR == 1 ? KVC_WAVES_PER_WG : 1, wgs = (groups + rows - 1) / rows;
+    const int64_t most = WPR <= KVC_WAVES_PER_WG ? KVC_HIST_WGS : KVC_HIST_WGS * KVC_WAVES_PER_WG / WPR;
+    hipLaunchKernelGGL((kvc_quant_row_once_kernel<NIT, WPR, HIST, PACK>), dim3((unsigned)(HIST && wgs > most ? most : wgs)),
+                       dim3(WPR == 1 ? KVC_WG : WPR * KVC_WAVE), 0, stream, a, R, groups);
+}
 template <bool HIST, bool PACK>
 static void kvc_launch_row_once(const KvcQuantArgs &a, int64_t R, int64_t groups, hipStream_t stream)
 {
-    auto grid = [&](int waves_per_row) {
-        const int64_t rows = KVC_WAVES_PER_WG / waves_per_row, wgs = (groups + rows - 1) / rows;
-        return dim3((unsigned)(HIST && wgs > KVC_HIST_WGS ? KVC_HIST_WGS : wgs));
-    };
-    constexpr int W = KVC_WAVES_PER_WG;
-    if (R <= 512 * 8) hipLaunchKernelGGL((kvc_quant_row_once_kernel<8, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * 24) hipLaunchKernelGGL((kvc_quant_row_once_kernel<24, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * 32) hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, 1, HIST, PACK>), grid(1), dim3(KVC_WG), 0, stream, a, R, groups);
-    else if (R <= 512 * W * 16) hipLaunchKernelGGL((kvc_quant_row_once_kernel<16, W, HIST, PACK>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
-    else hipLaunchKernelGGL((kvc_quant_row_once_kernel<32, W, HIST, PACK>), grid(W), dim3(KVC_WG), 0, stream, a, R, groups);
+    if (R <= 512 * 8) kvc_launch_row_once_of<8, 1, HIST, PACK>(a, R, groups, stream);
+    else if (R <= 512 * 16) kvc_launch_row_once_of<16, 1, HIST, PACK>(a, R, groups, stream);
+    else if (R <= 512 * 8 * 4) kvc_launch_row_once_of<8, 4, HIST, PACK>(a, R, groups, stream);
+    else if (R <= 512 * 8 * 8) kvc_launch_row_once_of<8, 8, HIST, PACK>(a, R, groups, stream);
+    else if (PACK) kvc_launch_row_once_of<16, 8, HIST, PACK>(a, R, groups, stream);      // (16 loads: 110 registers packed, 134 and three waves per SIMD else)
+    else kvc_launch_row_once_of<32, 4, HIST, PACK>(a, R, groups, stream);
 }
-constexpr int64_t KVC_ROW_ONCE_MAX = 512 * KVC_WAVES_PER_WG * 32;
+constexpr int64_t KVC_ROW_ONCE_MAX = 512 * 16 * 8;
+static_assert(KVC_ROW_ONCE_MAX == 512 * 32 * 4, "both hold the longest rows");
 
 // ---- block groups (masks 0xF, 0xD): rows of R contiguous elements map many-to-one onto groups;
 // wave-reduce each row, then merge rows with atomics on an order-preserving integer image. -----------
