@@ -62,6 +62,7 @@ struct KvcEncodeArgs {
     int wave_bytes;                // one-pass kernel from symbols: LDS of a wave
     int packed;                    // sym holds two symbols a byte (kvc_packed_symbols)
     int groups;                    // one pass: groups of tiles, see KVC_ONCE_GROUP_TILES
+    int stream_out;                // the payload is long and not written to stay in the caches
 };
 
 constexpr int KVC_ENC_STATUS_WORDS = 16;            // status words in front of the per-1024-tile payload totals
@@ -782,7 +783,10 @@ __device__ __forceinline__ void kvc_write_image_shifted(const KvcEncodeArgs &a, 
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) {
             const uint32_t f = f0 + k * KVC_WAVE;
-            if (f >= first && f < end) dst[f] = word[k];
+            if (f >= first && f < end) {
+                if (a.stream_out) __builtin_nontemporal_store(word[k], dst + f);
+                else dst[f] = word[k];
+            }
         }
     }
     // the bytes at the ragged ends: of word 0 by lanes 0 .. 3, of the last word by lanes 4 .. 7
@@ -2159,6 +2163,9 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     a.outcome_number = c.outcome_number;
     a.clear = c.clear;
     a.packed = c.packed;
+    // From symbols, long: what is not read yet of the symbols is better kept than the payload (K of 8 x 32 heads x 128 x 4096 tokens 61
+    // -> 59 us, of 4 x 32 x 96 x 32 768 203 -> 187).  A short payload may well be read next, by the attention behind the store.
+    a.stream_out = !c.src && a.tiles > 4096;
     const int group_tiles = c.packed && !c.is_k ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES;
     a.groups = (int)((a.tiles + group_tiles - 1) / group_tiles);
     a.max_polls = 0;
