@@ -3,12 +3,14 @@
 There is no CPU fallback: if the library is missing or a call fails, an exception is raised.
 """
 import ctypes as C
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libkvcomp_hip.so")
+HOST_PATH = os.path.join(_HERE, "ext", "kvcomp_host.so")
 _LIB = None
 
 _i64, _int, _vp, _f32p, _u32 = C.c_int64, C.c_int, C.c_void_p, C.POINTER(C.c_float), C.c_uint32
@@ -194,6 +196,22 @@ def lib():
             fn.restype = _RESTYPES.get(name, _int)
         _LIB = L
     return _LIB
+
+
+_HOST = None
+
+
+def host():
+    """The native module of kvcomp_host_module.cpp (loaded once)."""
+    global _HOST
+    if _HOST is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise KvcompError("%s is missing: build it with `python -m kvcomp_amd.build`" % HOST_PATH)
+        spec = importlib.util.spec_from_file_location("kvcomp_host", HOST_PATH)
+        _HOST = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_HOST)
+    return _HOST
 
 
 def set_option(name: str, value: int) -> int:

@@ -101,27 +101,34 @@ class CompressedAttention:
         B, Hq, D = q.shape
         k, v = self.k, self.v
         assert q.dtype is torch.float16 and v.ctx_len == k.ctx_len
-        if not q.device == k.device == v.device:
-            raise KvcompError("queries on %s, keys on %s, values on %s" % (q.device, k.device, v.device))
+        device = q.device
+        if not device == k.device == v.device:
+            raise KvcompError("queries on %s, keys on %s, values on %s" % (device, k.device, v.device))
         if scale is None:
             scale = 1.0 / math.sqrt(D)
         L = _lib.lib()
         # (what the workspace has to hold grows with the tokens: asked for in steps of 1024)
-        key = ((k.ctx_len + 1023) // 1024, B, Hq, D, q.get_device())
+        index = q.get_device()
+        key = ((k.ctx_len + 1023) // 1024, B, Hq, D, index)
         if key != self._workspace_key:
             need = int(L.kvc_attention_workspace_bytes(key[0] * 1024, key[0] * 1024, B, Hq, D))
-            if self._workspace is None or self._workspace.numel() < need or self._workspace.device != q.device:
+            if self._workspace is None or self._workspace.numel() < need or self._workspace.device != device:
                 _lib.let_go(self._workspace)
-                self._workspace = torch.empty(need + need // 4, dtype=torch.uint8, device=q.device)
+                self._workspace = torch.empty(need + need // 4, dtype=torch.uint8, device=device)
             self._workspace_key = key
         if out is None:
-            out = torch.empty(B, Hq, D, dtype=torch.float32, device=q.device)
+            out = torch.empty(B, Hq, D, dtype=torch.float32, device=device)
         kd, vd = k.descriptor(), v.descriptor()
         q = q.contiguous()
         ms = (C.c_float * 2)() if kernel_ms is not None else None
-        with _lib.device_guard(q):
-            rc = L.kvc_attention_decode(kd, vd, q.data_ptr(), scale, self._workspace.data_ptr(), self._workspace.numel(), out.data_ptr(),
-                                        B, k.head_num, Hq, D, None, ms, _lib.stream_of(q))
+        workspace = self._workspace
+        if index >= 0 and torch._C._cuda_getDevice() == index:
+            rc = L.kvc_attention_decode(kd, vd, q.data_ptr(), scale, workspace.data_ptr(), workspace.numel(), out.data_ptr(),
+                                        B, k.head_num, Hq, D, None, ms, torch._C._cuda_getCurrentRawStream(index))
+        else:
+            with _lib.device_guard(q):
+                rc = L.kvc_attention_decode(kd, vd, q.data_ptr(), scale, workspace.data_ptr(), workspace.numel(), out.data_ptr(),
+                                            B, k.head_num, Hq, D, None, ms, _lib.stream_of(q))
         if rc:
             check(rc)
         if kernel_ms is not None:

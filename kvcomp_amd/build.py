@@ -22,6 +22,8 @@ LIBPATH = os.path.join(LIBDIR, "libkvcomp_hip.so")
 EXTDIR = os.path.join(HERE, "ext")
 MODULE_SRC = os.path.join(CSRC, "kvcomp_cuda_module.cpp")
 MODULE_PATH = os.path.join(EXTDIR, "kvcomp_cuda.so")         # `import kvcomp_cuda` with EXTDIR on sys.path
+HOST_MODULE_SRC = os.path.join(CSRC, "kvcomp_host_module.cpp")
+HOST_MODULE_PATH = os.path.join(EXTDIR, "kvcomp_host.so")
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -91,7 +93,13 @@ def build(verbose=True, jobs=None):
 
 
 def build_module(verbose=True):
-    """The reference's `kvcomp_cuda` extension module (kvcomp_cuda_extension/export_kvcomp.cpp:8-26) over the C ABI."""
+    """The reference's `kvcomp_cuda` extension module (kvcomp_cuda_extension/export_kvcomp.cpp:8-26) over the C ABI, and the
+    package's own `kvcomp_host`, both at a time."""
+    with ThreadPoolExecutor(max_workers=2) as pool:
+        return list(pool.map(lambda m: _compile_module(*m, verbose), ((MODULE_SRC, MODULE_PATH), (HOST_MODULE_SRC, HOST_MODULE_PATH))))[0]
+
+
+def _compile_module(source, path, verbose):
     import sysconfig
     import torch
     from torch.utils.cpp_extension import include_paths
@@ -104,12 +112,12 @@ def build_module(verbose=True):
            "-I" + os.path.join(os.path.dirname(HERE), "include"), "-I" + os.path.join(rocm, "include"),
            "-I" + sysconfig.get_paths()["include"]]
     cmd += ["-I" + p for p in include_paths()]
-    cmd += ["-o", MODULE_PATH, MODULE_SRC, "-L" + LIBDIR, "-lkvcomp_hip", "-Wl,-rpath,$ORIGIN/../lib",
+    cmd += ["-o", path, source, "-L" + LIBDIR, "-lkvcomp_hip", "-Wl,-rpath,$ORIGIN/../lib",
             "-L" + torch_lib, "-Wl,-rpath," + torch_lib, "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-ltorch_python"]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
-    return MODULE_PATH
+    return path
 
 
 if __name__ == "__main__":

@@ -209,7 +209,13 @@ def append_dense(k: torch.Tensor, v: torch.Tensor, cos: Optional[torch.Tensor], 
     """kvc_append_dense: k (rotated by cos / sin [1 or B, T, D], unless they are None) and v, [B, H, T, D] fp16, to
     positions at .. of the [B, H, capacity, D] caches.  False, having done nothing, for tensors it does not take or that
     PyTorch would record.  (No view handed out before holds the positions written: their version need not move.)"""
-    packed = _packed_append(k, v, cos, sin, k_cache, v_cache, at)
+    if k.is_cuda and not _lib.hooked():
+        done = _lib.host().append_dense(k, v, cos, sin, k_cache, v_cache, at)
+        if done:
+            if done < 0:
+                check(done)
+            return True
+    packed = _packed_append(k, v, cos, sin, k_cache, v_cache, at)      # (what answers for itself, and what was not taken)
     if packed is None:
         return False
     with _lib.device_guard(k):

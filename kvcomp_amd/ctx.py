@@ -461,6 +461,15 @@ class KVCompCtx:
             _lib.let_go(self._tail)
             self._tail = grown
         row = self._row_bytes
+        if n and cache.is_cuda and not _lib.hooked():
+            done = _lib.host().append_rows(self._tail, self._tail_len, cache, row)
+            if done:
+                if done < 0:
+                    _lib.check(done)
+                if self._tail_len == 0:                              # where views of an earlier tail may lie
+                    torch.autograd.graph.increment_version((self._tail,))
+                self._tail_len += n
+                return
         to, src = self._tail.data_ptr() + self._tail_len * row, cache.data_ptr()
         if (n and (to | src | row) & 15 == 0 and cache.is_cuda and cache.is_contiguous() and
                 not (cache.requires_grad or self._tail.requires_grad or _lib.hooked())):
@@ -827,15 +836,15 @@ class KVCompCtx:
         if tokens == 0:
             _DESC.pack_into(desc, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, self._mask, 0, 0, 0, 0, tail_address, tail)
             return desc
-        lut = self.decode_lut()
-        mins, scales, encoded = self._min_ints, self._scales, self._encoded
+        lut = self._lut if self._lut_source is self.decode_codebook else self.decode_lut()
+        infos, threads, mins, scales, encoded = self._block_infos, self._thread_infos, self._min_ints, self._scales, self._encoded
         # the kernels take the quantization parameters by pointer: they must cover every group of the stream
         groups = tokens // self.block_size * self._groups_per_block
         assert mins.used * mins.row == groups and scales.used * scales.row == groups, \
             "the context holds %d minima and %d scales for %d quantization groups" % (mins.used * mins.row, scales.used * scales.row, groups)
-        _DESC.pack_into(desc, 0, lut.data_ptr(), 0, self._block_infos.address, self._block_infos.used,
-                        self._thread_infos.address, self._thread_infos.used, encoded.address,
-                        min(encoded.used + self._enc_pending, encoded.data.shape[0]), mins.address, scales.address, self._mask,
+        _DESC.pack_into(desc, 0, lut.data_ptr(), 0, infos.data.data_ptr(), infos.used, threads.data.data_ptr(), threads.used,
+                        encoded.data.data_ptr(), min(encoded.used + self._enc_pending, encoded.data.numel()),
+                        mins.data.data_ptr(), scales.data.data_ptr(), self._mask,
                         self.max_tile_bytes, self.max_stream_bytes, self.code_hint, tokens, tail_address, tail)
         return desc
 
