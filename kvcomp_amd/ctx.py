@@ -218,6 +218,7 @@ class _QueuedStore(NamedTuple):
     lost: bool                       # its tokens are gone if it has to be taken back: counted in ctx_len, rows not kept
     certain: bool                    # nothing about it can fail, whatever a later store does
     codebook: bool                   # it brought the codebook, which goes with it
+    done: Optional["torch.cuda.Event"] = None        # behind it on its stream, if it had no outcome's words to write to
 
 
 # the seventeen 8-byte fields of kvc_compressed_desc, in order
@@ -326,6 +327,7 @@ class KVCompCtx:
                 self.poll_stores()
                 return
         self.waits += 1
+        self._behind_the_last_store()
         try:
             _, max_tile, max_stream, _ = kvcomp_cuda.encode_result(self._state[:8], self._encoded.data.numel())
         except KvcompError:
@@ -385,6 +387,12 @@ class KVCompCtx:
         self._unverified = []
         self._probe = None
 
+    def _behind_the_last_store(self):
+        """Order the current stream behind the last queued store, where that may have been queued on another one: one that found
+        the outcome's words taken by a store on a stream of its own."""
+        if self._unverified and self._unverified[-1].done is not None:
+            torch.cuda.current_stream(self.device).wait_event(self._unverified[-1].done)
+
     def _issue_probe(self):
         """Ask for a copy of the device words without waiting for it (nothing is asked for while the stream is being
         recorded into a graph, or while an earlier copy is on its way on another stream; one on this stream is replaced
@@ -397,6 +405,7 @@ class KVCompCtx:
             return
         if self._host_words is None:
             self._host_words = torch.empty(16, dtype=torch.int32, pin_memory=True)
+        self._behind_the_last_store()
         self._host_words.copy_(self._state, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record(torch.cuda.current_stream(self.device))
@@ -676,7 +685,11 @@ class KVCompCtx:
         self._scales.used += nb
         self._enc_pending += worst
         self.compressed_ctx_len += T
-        self._unverified.append(_QueuedStore(T, keep, self._bookkeeping(), worst, lost_if_dropped, certain, codebook))
+        done = None
+        if outcome is None and self.device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
+            done = torch.cuda.Event()
+            done.record(torch.cuda.current_stream(self.device))
+        self._unverified.append(_QueuedStore(T, keep, self._bookkeeping(), worst, lost_if_dropped, certain, codebook, done))
         if outcome is not None:
             self._probe = (outcome, len(self._unverified), outcome.stream)
 

@@ -141,6 +141,18 @@ def _busy(stream, seconds):
     return end
 
 
+def _ticks(stream, seconds):
+    """What _sleep takes for about that long."""
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(1000)
+        start.record()
+        torch.cuda._sleep(5000000)
+        end.record()
+        end.synchronize()
+    return int(5000000 * seconds * 1e3 / start.elapsed_time(end))
+
+
 @pytest.mark.gpu
 def test_a_number_that_never_comes_is_waited_for_on_its_own_stream_alone():
     from tests import _synth as S
@@ -163,6 +175,41 @@ def test_a_number_that_never_comes_is_waited_for_on_its_own_stream_alone():
     assert not outcome.query() and not end.query() and 1.9 < waited < 4.0
     outcome.number = there
     end.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ask", ["poll", "sizes"])
+@pytest.mark.parametrize("is_k", [True, False])
+def test_a_store_without_words_of_its_own_is_waited_for_on_its_stream(is_k, ask):
+    """The words are the first stream's, the last store is the second's, and still behind a long kernel there when the default
+    stream, which is ordered behind nothing, asks for what has become of it."""
+    from tests import _synth as S
+    _config()
+    x = (S.synth_k if is_k else S.synth_v)(1280, 2, 4, 128).to(DEV)
+    parts = [x[:512], x[512:640], x[640:1024], x[1024:]]
+    want = _store_all(is_k, parts)
+    expect = {name: getattr(want, name).clone() for name in ("encoded_data", "block_infos", "thread_infos", "quant_min_ints", "quant_scales", "buffer")}
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    ticks, end = _ticks(first, 0.2), torch.cuda.Event()
+    with torch.cuda.stream(first):
+        got = _store_all(is_k, parts[:2])
+        torch.cuda._sleep(ticks)
+        got.store(parts[2], want_symbols=False)
+        outcome = got._outcome
+    second.wait_stream(first)
+    with torch.cuda.stream(second):
+        torch.cuda._sleep(ticks)
+        end.record()
+        got.store(parts[3], want_symbols=False)
+        assert not outcome.query() and len(got._unverified) > got._probe[1]
+    outcome.synchronize()
+    if ask == "poll":
+        got.poll_stores()
+        assert len(got._unverified) == 1 and not end.query()
+    assert got.encoded_data.numel() == expect["encoded_data"].numel() and end.query() and not got._unverified
+    for name, value in expect.items():
+        assert torch.equal(getattr(got, name), value), name
 
 
 @pytest.mark.gpu
