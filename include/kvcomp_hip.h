@@ -244,6 +244,8 @@ int kvc_encode_async(const kvc_encode_job *job, void *stream);
  *   table, 0 if not known; symbols with longer codes are errors.  h_outcome, if not NULL: 16 words of pinned host memory that
  *   receive d_result's eight words, *d_stream_bytes and, last, outcome_number (word 9), as the call ends on the device; words
  *   10 - 12 are set to the stream (low half, high half) and the device before an accepted call returns.
+ * kvc_encode_queue_book: kvc_put_codebook and kvc_encode_queue with the table that it puts in place (the job's own is not looked at),
+ *   for calls that were prepared; d_tables and d_lut are written by the time the call has run.
  * kvc_wait_outcome: waits until outcome_number has arrived in such words.  If it has not come after two seconds and
  *   everything queued on their stream has run, it returns too, with word 9 saying that the number has not come; the stream
  *   must exist as long.  No other stream is waited for, and the current device does not matter. */
@@ -252,6 +254,9 @@ int kvc_encode_prepare(const kvc_encode_job *job, void *d_scratch, int64_t scrat
 int kvc_encode_prepare_packed(const kvc_encode_job *job, void *d_scratch, int64_t scratch_bytes, int *prepared, void *stream);
 int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,
                      uint32_t outcome_number, void *stream);
+struct kvc_codebook;
+int kvc_encode_queue_book(const kvc_encode_job *job, void *d_scratch, int prepared, const struct kvc_codebook *book, void *d_tables, void *d_lut,
+                          uint32_t *h_outcome, uint32_t outcome_number, void *stream);
 int kvc_wait_outcome(const uint32_t *h_outcome, uint32_t outcome_number);
 int kvc_encode_result(const uint32_t *d_result, int64_t encoded_cap, int64_t *h_total_bytes, int64_t *h_max_tile_bytes,
                       int64_t *h_max_stream_bytes, int64_t *h_tiles, void *stream);

@@ -68,6 +68,7 @@ _SIGNATURES = {
     "kvc_encode_prepare": [C.POINTER(EncodeJob), _vp, _i64, _intp, _vp],
     "kvc_encode_prepare_packed": [C.POINTER(EncodeJob), _vp, _i64, _intp, _vp],
     "kvc_encode_queue": [C.POINTER(EncodeJob), _vp, _int, _int, _vp, _u32, _vp],
+    "kvc_encode_queue_book": [C.POINTER(EncodeJob), _vp, _int, _vp, _vp, _vp, _vp, _u32, _vp],
     "kvc_encode_result": [_vp, _i64, _i64p, _i64p, _i64p, _i64p, _vp],
     "kvc_k_entropy_decode": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _int, _vp, _i64, _i64, _i64, _i64, _f32p, _vp],
     "kvc_v_entropy_decode": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _int, _vp, _i64, _i64, _i64, _i64, _f32p, _vp],

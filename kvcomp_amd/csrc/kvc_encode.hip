@@ -23,8 +23,10 @@
 // hand each lane its vector from there, so the uint8 symbol tensor never exists in HBM (the reference
 // materialises it and several fp16 temporaries, models/cache/kvcomp_encode.py:86-98).
 #include "kvc_common.h"
+#include "kvc_lut_body.h"
 #include "kvc_quant_math.h"
 
+#include <cstring>
 #include <type_traits>
 
 struct KvcEncodeArgs {
@@ -63,6 +65,9 @@ struct KvcEncodeArgs {
     int packed;                    // sym holds two symbols a byte (kvc_packed_symbols)
     int groups;                    // one pass: groups of tiles, see KVC_ONCE_GROUP_TILES
     int stream_out;                // the payload is long and not written to stay in the caches
+    // a first store's table (at most sixteen entries), which comes in the argument block: table is written behind the encode only
+    int codes_here;
+    uint2 codes[16];
 };
 
 constexpr int KVC_ENC_STATUS_WORDS = 16;            // status words in front of the per-1024-tile payload totals
@@ -76,6 +81,15 @@ constexpr uint32_t KVC_ENC_ERR_CODEBOOK = 8u;       // a codebook was not built 
 __device__ __forceinline__ const uint8_t *kvc_table_of_row(const KvcEncodeArgs &a, int64_t row)
 {
     return a.rows_per_codebook ? a.table + (row / a.rows_per_codebook) * a.table_stride : a.table;
+}
+
+// Entry i of a table, in whatever memory it is.  (From the argument block through its own address: a copy of it, indexed by a
+// run-time number, would live in scratch memory.  It opens the argument block of every kernel that gets here.)
+// HERE: the call may be one of those (from symbols).
+template <bool HERE>
+__device__ __forceinline__ uint2 kvc_code_entry(const KvcEncodeArgs &a, const uint8_t *table, int i)
+{
+    return HERE && a.codes_here ? kvc_kernarg_again<KvcEncodeArgs>().codes[i & 15] : reinterpret_cast<const uint2 *>(table)[i];
 }
 
 // First launch of an encode call: clears the status words (a kernel, not a memset, so that the call can be recorded
@@ -549,14 +563,15 @@ __device__ __forceinline__ uint32_t kvc_count_tile(const KvcEncodeArgs &a, int64
 
 // Code lengths of the table that `tile` is encoded with, one copy per wave (the tiles of a workgroup may lie in
 // rows with different codebooks).
+template <bool HERE>
 __device__ __forceinline__ void kvc_load_len_table(const KvcEncodeArgs &a, int64_t tile, uint8_t *s_len, int lane)
 {
-    const uint32_t *t = reinterpret_cast<const uint32_t *>(kvc_table_of_row(a, tile / a.cols));
+    const uint8_t *t = kvc_table_of_row(a, tile / a.cols);
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int i = lane + KVC_WAVE * k;
         uint32_t len = 0;
-        if (i < a.table_entries) len = t[2 * i + 1];
+        if (i < a.table_entries) len = kvc_code_entry<HERE>(a, t, i).y;
         s_len[i] = (uint8_t)(len > 32 ? 0 : len);
     }
 }
@@ -568,7 +583,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_count_kernel(KvcEncodeArgs 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid == 0) { s_err = 0; s_longest = 0; }
     const int64_t tile = (int64_t)blockIdx.x * KVC_WAVES_PER_WG + wave;
-    if (tile < a.tiles) kvc_load_len_table(a, tile, s_len[wave], lane);
+    if (tile < a.tiles) kvc_load_len_table<true>(a, tile, s_len[wave], lane);
     __syncthreads();
     if (tile < a.tiles) {
         uint32_t v[32];
@@ -679,13 +694,14 @@ __device__ __forceinline__ KvcEmitPlace kvc_emit_place(const KvcEncodeArgs &a, i
 // A wave's copy of the encode table of its tile: entries without a usable code become {0, 0} (the count pass has
 // flagged them), and *s_short tells whether every code has at most 8 bits (four then fit one 32-bit group).
 // The caller initialises *s_short (the wave's own word) to 1 and synchronises before and after.
+template <bool HERE>
 __device__ __forceinline__ void kvc_load_code_table(const KvcEncodeArgs &a, int64_t tile, uint2 *s_table, uint32_t *s_short, int lane)
 {
-    const uint2 *t = reinterpret_cast<const uint2 *>(kvc_table_of_row(a, tile / a.cols));
+    const uint8_t *t = kvc_table_of_row(a, tile / a.cols);
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int i = lane + KVC_WAVE * k;
-        uint2 e = i < a.table_entries ? t[i] : make_uint2(0u, 0u);
+        uint2 e = i < a.table_entries ? kvc_code_entry<HERE>(a, t, i) : make_uint2(0u, 0u);
         if (e.y > 32u) e = make_uint2(0u, 0u);
         if (e.y < 32u) e.x &= (1u << e.y) - 1u;           // nothing above the code's own bits
         s_table[i] = e;
@@ -809,7 +825,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_emit_kernel(KvcEncodeArgs a
     const int64_t tile = (int64_t)blockIdx.x * KVC_WAVES_PER_WG + wave;
     if (lane == 0) s_short[wave] = 1u;
     __syncthreads();
-    if (tile < a.tiles) kvc_load_code_table(a, tile, s_table[wave], &s_short[wave], lane);
+    if (tile < a.tiles) kvc_load_code_table<true>(a, tile, s_table[wave], &s_short[wave], lane);
     uint32_t *image = s_image[wave];
     __syncthreads();
     const KvcEmitPlace p = kvc_emit_place(a, tile, tile < a.tiles);
@@ -1030,7 +1046,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_store_count_kernel(KvcStoreArgs a)
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid == 0) { s_err = 0; s_longest = 0; }
     const int64_t tile = (int64_t)blockIdx.x * KVC_WAVES_PER_WG + wave;
-    if (tile < a.e.tiles) kvc_load_len_table(a.e, tile, s_len[wave], lane);
+    if (tile < a.e.tiles) kvc_load_len_table<false>(a.e, tile, s_len[wave], lane);
     __syncthreads();
     if (tile < a.e.tiles) {
         uint32_t v[32];
@@ -1062,7 +1078,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_store_emit_kernel(KvcStoreArgs a)
     const int64_t tile = (int64_t)blockIdx.x * KVC_WAVES_PER_WG + wave;
     if (lane == 0) s_short[wave] = 1u;
     __syncthreads();
-    if (tile < a.e.tiles) kvc_load_code_table(a.e, tile, s_table[wave], &s_short[wave], lane);
+    if (tile < a.e.tiles) kvc_load_code_table<false>(a.e, tile, s_table[wave], &s_short[wave], lane);
     __syncthreads();
     const KvcEmitPlace p = kvc_emit_place(a.e, tile, tile < a.e.tiles);
     if (!p.ok) return;                                 // wave-uniform; nothing below involves another wave
@@ -1717,9 +1733,8 @@ __device__ __forceinline__ void kvc_pack_packed(uint32_t start, const uint2 *s_t
 template <bool LOW>
 __device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint2 *s_table, bool pairs, uint32_t longest)
 {
-    const uint2 *t = reinterpret_cast<const uint2 *>(a.table);
     auto entry = [&](int i) {
-        const uint2 e = i < a.table_entries ? t[i] : make_uint2(0u, 0u);
+        const uint2 e = i < a.table_entries ? kvc_code_entry<true>(a, a.table, i) : make_uint2(0u, 0u);
         return e.y == 0u || e.y > longest ? make_uint2(0u, KVC_NO_CODE_LEN) : make_uint2(e.x & ((1u << e.y) - 1u), e.y);
     };
     for (int i = threadIdx.x; i < 256; i += blockDim.x) {
@@ -1914,7 +1929,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
 // outputs are the ones the call was to produce.  Slow (four waves for all tiles), and next to never needed: the
 // look-back's progress does not depend on the order in which the hardware starts workgroups.
 template <int FRONT>
-__global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs a)
+__device__ __forceinline__ void kvc_encode_finish(const KvcStoreArgs &a)
 {
     __shared__ uint2 s_table[KVC_WAVES_PER_WG][256];
     __shared__ uint8_t s_len[KVC_WAVES_PER_WG][256];
@@ -1961,7 +1976,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
     // ---- the whole call again, two passes inside this workgroup ----
     const int64_t tiles = a.e.tiles;
     for (int64_t tile = wave; tile < tiles; tile += KVC_WAVES_PER_WG) {      // count: thread_infos, byte_nums, group parameters
-        kvc_load_len_table(a.e, tile, s_len[wave], lane);
+        kvc_load_len_table<FRONT == 0>(a.e, tile, s_len[wave], lane);
         kvc_wave_lds_sync();
         uint32_t v[32];
         if constexpr (FRONT == 1) {
@@ -2012,7 +2027,7 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
     for (int64_t tile = wave; tile < tiles; tile += KVC_WAVES_PER_WG) {      // emit
         if (lane == 0) s_short[wave] = 1u;
         kvc_wave_lds_sync();
-        kvc_load_code_table(a.e, tile, s_table[wave], &s_short[wave], lane);
+        kvc_load_code_table<FRONT == 0>(a.e, tile, s_table[wave], &s_short[wave], lane);
         kvc_wave_lds_sync();
         const KvcEmitPlace p = kvc_emit_place(a.e, tile, true);
         if (!p.ok) continue;                                                 // flagged by the count pass or the offsets
@@ -2044,6 +2059,30 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
     kvc_encode_publish(a.e, tid);
+}
+
+template <int FRONT>
+__global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs a) { kvc_encode_finish<FRONT>(a); }
+
+// ... and, by a second workgroup beside it, a first store's codebook to where it is kept and its decode tables
+// (kvc_put_codebook).  The encoder has its codes in the argument block, so between the counts' arrival and the encoder nothing is
+// left but the launch, where this took a launch of its own in front of it: K and V of 8 heads x 777 tokens 246 -> 234 us, 8 x 32 x 128 x
+// 4096 370 -> 363.
+struct KvcPutSmallArgs {
+    uint32_t words[80];            // table, padded to 16 bytes, and tree
+    uint8_t *dst;
+    uint32_t *lut;
+    int bytes, tree_at, node_bytes;
+};
+__global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_put_kernel(KvcStoreArgs a, KvcPutSmallArgs p)
+{
+    if (blockIdx.x == 0) {
+        kvc_encode_finish<0>(a);
+        return;
+    }
+    const uint8_t *src = reinterpret_cast<const uint8_t *>(p.words);
+    for (int i = threadIdx.x; i < p.bytes; i += KVC_WG) p.dst[i] = src[i];
+    kvc_build_lut_body(src + p.tree_at, p.bytes - p.tree_at, p.node_bytes, p.lut);
 }
 
 // What the fused path adds to an encode call: the fp16 source and how to quantize it.
@@ -2082,6 +2121,8 @@ struct KvcEncodeCall {
     uint32_t *h_outcome, outcome_number;
     int longest_code;                                      // of the (one) codebook, 0: not known
     bool packed;                                           // d_sym: two symbols a byte (kvc_packed_symbols)
+    const kvc_codebook *book;                              // packed, one pass: the table, which d_tables receives behind the encode
+    void *d_lut;
 };
 
 static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
@@ -2168,6 +2209,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     a.stream_out = !c.src && a.tiles > 4096;
     const int group_tiles = c.packed && !c.is_k ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES;
     a.groups = (int)((a.tiles + group_tiles - 1) / group_tiles);
+    a.codes_here = c.book != nullptr;
+    if (c.book) std::memcpy(a.codes, c.book->encode_table, (size_t)c.table_bytes);
     a.max_polls = 0;
     a.force_order = 0;
     const int64_t chunks = (a.tiles + 1023) / 1024;
@@ -2251,7 +2294,19 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         const auto symbols_kernel = kvc_symbols_kernel(is_k, a.vec_len, !c.packed ? KVC_FORM_BYTES : c.longest_code >= 1 && c.longest_code <= 8 ? KVC_FORM_PACKED : KVC_FORM_PACKED_LONG);
         if (wide) {
             hipLaunchKernelGGL(symbols_kernel, dim3(wgs1), dim3(waves * KVC_WAVE), lds, stream, sa.e, run);
-            hipLaunchKernelGGL(kvc_encode_finish_kernel<0>, dim3(1), dim3(KVC_WG), 0, stream, sa);
+            if (c.book) {
+                KvcPutSmallArgs put = {};
+                put.tree_at = (int)((c.book->encode_bytes + 15) / 16 * 16);
+                put.bytes = put.tree_at + (int)c.book->decode_bytes;
+                std::memcpy(put.words, c.book->encode_table, (size_t)c.book->encode_bytes);
+                std::memcpy(reinterpret_cast<uint8_t *>(put.words) + put.tree_at, c.book->decode_tree, (size_t)c.book->decode_bytes);
+                put.dst = const_cast<uint8_t *>(c.d_tables);
+                put.lut = reinterpret_cast<uint32_t *>(c.d_lut);
+                put.node_bytes = c.book->tree_format;
+                hipLaunchKernelGGL(kvc_encode_finish_put_kernel, dim3(2), dim3(KVC_WG), 0, stream, sa, put);
+            } else {
+                hipLaunchKernelGGL(kvc_encode_finish_kernel<0>, dim3(1), dim3(KVC_WG), 0, stream, sa);
+            }
         } else if (front == 0) {
             hipLaunchKernelGGL(kvc_encode_once_kernel<0>, dim3(wgs1), dim3(KVC_WG), lds, stream, sa, run);
             hipLaunchKernelGGL(kvc_encode_finish_kernel<0>, dim3(1), dim3(KVC_WG), 0, stream, sa);
@@ -2458,8 +2513,8 @@ extern "C" int kvc_encode_prepare_packed(const kvc_encode_job *job, void *d_scra
     return kvc_encode_prepare_form(job, true, d_scratch, scratch_bytes, prepared, stream);
 }
 
-extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,
-                                uint32_t outcome_number, void *stream)
+static int kvc_encode_queue_form(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, const kvc_codebook *book,
+                                 void *d_lut, uint32_t *h_outcome, uint32_t outcome_number, void *stream)
 {
     KvcEncodeCall c = {};
     if (int rc = kvc_encode_job_check(job, c)) return rc;
@@ -2474,6 +2529,8 @@ extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int 
     c.h_outcome = h_outcome;
     c.outcome_number = outcome_number;
     c.longest_code = longest_code;
+    c.book = book;
+    c.d_lut = d_lut;
     KvcStoreSource src = {job->d_x_f16, job->batch, job->heads, job->quant_mask, job->eb, job->d_min_i8, job->d_scale_f16};
     if (!job->d_sym) {
         KVC_REQUIRE(kvc_store_fused_supported(job->is_k, job->quant_mask, job->batch, job->heads, job->head_dim),
@@ -2500,6 +2557,31 @@ extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int 
         h_outcome[12] = (uint32_t)dev;
     }
     return 0;
+}
+
+extern "C" int kvc_encode_queue(const kvc_encode_job *job, void *d_scratch, int prepared, int longest_code, uint32_t *h_outcome,
+                                uint32_t outcome_number, void *stream)
+{
+    return kvc_encode_queue_form(job, d_scratch, prepared, longest_code, nullptr, nullptr, h_outcome, outcome_number, stream);
+}
+
+// kvc_put_codebook, and kvc_encode_queue with its table: in one go where the call is from packed symbols and takes one pass.
+extern "C" int kvc_encode_queue_book(const kvc_encode_job *job, void *d_scratch, int prepared, const kvc_codebook *book, void *d_tables, void *d_lut,
+                                     uint32_t *h_outcome, uint32_t outcome_number, void *stream)
+{
+    KVC_REQUIRE(job != nullptr && book != nullptr && d_tables != nullptr && d_lut != nullptr, "NULL argument");
+    kvc_encode_job with = *job;
+    with.d_encode_tables = (const uint8_t *)d_tables;
+    with.encode_table_bytes = book->encode_bytes;
+    const int64_t tree_at = (book->encode_bytes + 15) / 16 * 16;
+    const bool together = prepared == (KVC_ENC_MARKED | KVC_ENC_PACKED) && book->encode_bytes > 0 && book->encode_bytes <= 16 * 8 &&
+                          (book->tree_format == KVC_TREE_I8 || book->tree_format == KVC_TREE_I16) && book->decode_bytes >= 2 * book->tree_format &&
+                          book->decode_bytes % book->tree_format == 0 && tree_at + book->decode_bytes <= (int64_t)sizeof(KvcPutSmallArgs::words) &&
+                          ((uintptr_t)d_lut & 15) == 0;
+    if (!together) {
+        if (int rc = kvc_put_codebook(book, d_tables, d_lut, stream)) return rc;
+    }
+    return kvc_encode_queue_form(&with, d_scratch, prepared, book->max_code_bits, together ? book : nullptr, d_lut, h_outcome, outcome_number, stream);
 }
 
 extern "C" int kvc_encode_async(const kvc_encode_job *job, void *stream) { return kvc_encode_queue(job, nullptr, KVC_ENC_FRESH, 0, nullptr, 0u, stream); }

@@ -631,11 +631,12 @@ class KVCompCtx:
     # of this much takes about as long as a wait)
     COPY_PENDING = 8 << 20
 
-    def _encode_direct(self, T: int, *, tables, table_bytes, symbols=None, cache=None, mask=0, most_bytes=None, keep=None,
-                       lost_if_dropped=False, certain=False, codebook=False, prepared=None, longest_code=0):
+    def _encode_direct(self, T: int, *, tables=None, table_bytes=0, symbols=None, cache=None, mask=0, most_bytes=None, keep=None,
+                       lost_if_dropped=False, certain=False, codebook=False, prepared=None, longest_code=0, book=None):
         """Queue one encode whose outputs go straight to their final places in this context's buffers; nothing waits.
         Quantizes `cache` on the fly (fused store) or takes `symbols` whose parameters are in place already.  most_bytes:
-        what the payload is known not to exceed; prepared, longest_code: what _prepare_encode returned, the codebook's longest code."""
+        what the payload is known not to exceed; prepared, longest_code: what _prepare_encode returned, the codebook's longest code; book: instead of
+        tables, a codebook that is still to be put in place, and where."""
         nb = T // self.block_size
         B, H, D = self.batch_size, self.head_num, self.head_dim
         sizes = kvcomp_cuda.buffer_sizes(T, B * H * D, self.is_k, H, D) if prepared is None else prepared.sizes
@@ -666,7 +667,9 @@ class KVCompCtx:
         before = None if outcome is None else (outcome.number, outcome.stream)
         told = None if outcome is None else outcome.ask(_lib.stream_of(state))
         try:
-            if prepared is not None:
+            if book is not None:
+                kvcomp_cuda.encode_prepared_book(prepared, *book, self._encoded.data, told, room)
+            elif prepared is not None:
                 kvcomp_cuda.encode_prepared(prepared, tables, self._encoded.data, told, longest_code, room)
             else:
                 kvcomp_cuda.encode_async(self.is_k, batch=B, head_num=H, head_dim=D, tokens=T, encode_tables=tables,
@@ -729,17 +732,18 @@ class KVCompCtx:
         sym, book = quantize(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale,
                                                self._smoothed_symbols() if self.codebook_smoothing else 0, meanwhile)
         self.waits += 1
-        enc, dec, lut = kvcomp_cuda.put_codebook(book, device, *prepared[1:])
         if packed and book.encode_bytes > 16 * 8:              # scales among fp16's smallest numbers: half a byte does not hold these symbols
             sym = quant(blocked, self.quant_dims, self.quant_scale_rel)[0]
             prepared, packed = [], False
+        enc, dec, lut = kvcomp_cuda.codebook_parts(book, prepared[1]) if packed else kvcomp_cuda.put_codebook(book, device, *prepared[1:])
         vectors = T * self.batch_size * self.head_num * self.head_dim // (self.head_dim if self.is_k else kvcomp_cuda.V_VEC_LEN)
         cannot_fail = book.max_code_bits <= 7
         small = T <= self.ASYNC_KEEP_BLOCKS * self.block_size
         queued = self.async_store and (cannot_fail or small)
         self._encode_direct(T, symbols=sym, tables=enc, table_bytes=enc.numel(), most_bytes=book.payload_bits // 8 + vectors + 1,
                             keep=blocked.flatten(0, 1).clone() if queued and not cannot_fail else None, certain=cannot_fail, codebook=True,
-                            prepared=prepared[0] if prepared else None, longest_code=book.max_code_bits)
+                            prepared=prepared[0] if prepared else None, longest_code=book.max_code_bits,
+                            book=(book, prepared[1]) if packed else None)
         if queued:
             self._issue_probe()
         else:

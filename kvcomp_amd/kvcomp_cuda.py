@@ -196,11 +196,17 @@ def put_codebook(book: "_lib.Codebook", device, room: torch.Tensor = None):
     L = _lib.lib()
     if room is None:
         room = codebook_room(device)
-    enc_bytes, lut_bytes, address = book.encode_bytes, L.kvc_lut_bytes(), room.data_ptr()
-    at = lut_bytes + (enc_bytes + 15) // 16 * 16         # each part on a 16-byte boundary
-    _require(room.numel() >= at + book.decode_bytes, "not enough room for the codebook")
+    parts, address = codebook_parts(book, room), room.data_ptr()
     with _lib.device_guard(room):
-        check(L.kvc_put_codebook(C.addressof(book), address + lut_bytes, address, _lib.stream_of(room)))
+        check(L.kvc_put_codebook(C.addressof(book), address + L.kvc_lut_bytes(), address, _lib.stream_of(room)))
+    return parts
+
+
+def codebook_parts(book: "_lib.Codebook", room: torch.Tensor):
+    """Where put_codebook puts a codebook's (encode table, decode tree, decode tables) in `room`, each on a 16-byte boundary."""
+    enc_bytes, lut_bytes = book.encode_bytes, _lib.lib().kvc_lut_bytes()
+    at = lut_bytes + (enc_bytes + 15) // 16 * 16
+    _require(room.numel() >= at + book.decode_bytes, "not enough room for the codebook")
     return room[lut_bytes:lut_bytes + enc_bytes], room[at:at + book.decode_bytes], room[:lut_bytes]
 
 
@@ -375,6 +381,20 @@ def encode_prepared(prepared: PreparedEncode, encode_table: torch.Tensor, encode
     address, number = (0, 0) if outcome is None else outcome
     with _lib.device_guard(encoded):
         check(_lib.lib().kvc_encode_queue(C.byref(job), at, prepared.done, longest_code, address, number, _lib.stream_of(encoded)))
+
+
+def encode_prepared_book(prepared: PreparedEncode, book: "_lib.Codebook", place: torch.Tensor, encoded: torch.Tensor, outcome, room: int):
+    """put_codebook into `place`, and encode_prepared with its table."""
+    job, at, L = prepared.job, prepared.scratch.data_ptr(), _lib.lib()
+    _dev_u8(encoded, "encoded")
+    _require(0 < room <= encoded.numel(), "room: bytes of encoded")
+    _require(place.numel() >= L.kvc_lut_bytes() + (book.encode_bytes + 15) // 16 * 16 + book.decode_bytes, "not enough room for the codebook")
+    job.d_encoded, job.encoded_cap = encoded.data_ptr(), room
+    address, number = (0, 0) if outcome is None else outcome
+    tables = place.data_ptr()
+    with _lib.device_guard(encoded):
+        check(L.kvc_encode_queue_book(C.byref(job), at, prepared.done, C.addressof(book), tables + L.kvc_lut_bytes(), tables, address, number,
+                                      _lib.stream_of(encoded)))
 
 
 def encode_result(result: torch.Tensor, encoded_cap: int):
