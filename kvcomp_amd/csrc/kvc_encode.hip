@@ -1312,7 +1312,11 @@ struct KvcOncePending {
 // before it, which this wave has just placed at follows_off), publish its block_info and write its payload from the LDS
 // image (which starts on a word; the payload lands p.head bytes into an aligned word).  Returns error bits; *off_out
 // receives the tile's global offset.
-template <int G = KVC_ONCE_GROUP_TILES>
+// ASK: the look-back's words are asked for here, not taken as they were when the size was published.  In the kernel from symbols, whose
+// tiles take half as long, those of the tiles before were not there yet, and then the tiles' and the groups' were asked for again one
+// after the other: K of 4 x 32 heads x 96 x 32 768 tokens 196 -> 178 us, of 8 x 32 x 128 x 4096 61 -> 59, V 125 -> 124 and 50.
+// (Asked for just before the last tile is packed: K the same, V 126 and 51.)
+template <int G = KVC_ONCE_GROUP_TILES, bool ASK = false>
 __device__ __forceinline__ uint32_t kvc_once_place(const KvcEncodeArgs &a, const KvcOncePending &pd, const uint32_t *image, uint32_t base,
                                                    int lane, int *polls, uint32_t *off_out, bool follows = false, uint32_t follows_off = 0)
 {
@@ -1325,8 +1329,11 @@ __device__ __forceinline__ uint32_t kvc_once_place(const KvcEncodeArgs &a, const
             kvc_status_store(kvc_group_words(a) + kvc_once_group<G>(tile), kvc_group_word(off + bn - base, 0u));
     } else {
         uint32_t in_group = pd.in_group;
-        if (!pd.in_group_known) in_group = kvc_look_back_in_group<G>(a, tile, bn, lane, pd.looks.tile_word, polls);
-        off = base + in_group + kvc_look_back_groups<G>(a, tile, in_group + bn, lane, pd.looks.group_word, polls);
+        KvcFirstLooks looks;
+        if constexpr (ASK) looks = kvc_look_back_ask<G>(a, tile, lane);
+        else looks = pd.looks;
+        if (!pd.in_group_known) in_group = kvc_look_back_in_group<G>(a, tile, bn, lane, looks.tile_word, polls);
+        off = base + in_group + kvc_look_back_groups<G>(a, tile, in_group + bn, lane, looks.group_word, polls);
     }
     *off_out = off;
     uint32_t err = 0;
@@ -1789,7 +1796,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     int polls = 0;
     bool placed = false;                                   // the tiles of the run up to the first kept one have been; they end at next_off
     // Tiles whose images wait in the area: `kept` of them, their payload bytes (sixteen bits each, the oldest lowest), the words
-    // they take and what the oldest one's look-back has asked for.
+    // they take and what is known of the bytes in front of the oldest one.
     int kept = 0;
     uint64_t kept_bytes = 0;
     uint32_t kept_words = 0;
@@ -1839,12 +1846,9 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         // the tile that the run's place is looked for with; and the wave that speaks for a group must not sit on its size (as in
         // kvc_encode_once_kernel)
         const bool opens = kept == 0 && !placed, closes = kvc_once_closes<G>(a, tile);
-        if (opens) {
-            first.looks = kvc_look_back_ask<G>(a, tile, lane);
-            first.in_group_known = closes;
-        }
+        if (opens) first.in_group_known = closes;
         if (closes) {
-            const uint64_t word = opens ? first.looks.tile_word : kvc_look_back_ask<G>(a, tile, lane).tile_word;
+            const uint64_t word = kvc_look_back_ask<G>(a, tile, lane).tile_word;
             const uint32_t in_group = kvc_look_back_in_group<G>(a, tile, bn, lane, word, &polls);
             if (opens) first.in_group = in_group;
         }
@@ -1894,7 +1898,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
                     for (int i = 0; i < OTHERS; i++)
                         next_off += (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(between_word >> 32), k * OTHERS + i) & 0xffffu;
                 }
-                err |= kvc_once_place<G>(a, which, area + at, base, lane, &polls, &off, placed, next_off);
+                err |= kvc_once_place<G, true>(a, which, area + at, base, lane, &polls, &off, placed, next_off);
                 at += which.packs ? kvc_once_image_words(which.bn) : 0u;
                 next_off = off + which.bn;
                 placed = true;
