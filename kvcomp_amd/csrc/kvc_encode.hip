@@ -1149,9 +1149,9 @@ constexpr int KVC_ONCE_MAX_GROUPS = (int)((KVC_WS_SLOT_BYTES - KVC_ONCE_GROUP_WO
 // group (measured: 10 us per wave there, 3 us on the die with the last tiles).
 constexpr int KVC_ONCE_GROUP_TILES = 56;
 static_assert(KVC_ONCE_GROUP_TILES <= KVC_WAVE && KVC_ONCE_GROUP_TILES % 2 == 0, "one look of 64 lanes covers a group; a run of two stays inside one");
-// (V from packed symbols: four waves take the sixteen tiles of their runs in turn, which must lie in one group.  48 tiles are
-// one and a half of its workgroups, so those waves change dies as well.)
-constexpr int KVC_ONCE_GROUP_TILES_VPACKED = 48;
+// (From packed symbols a wave's run, V: those of four waves, which take their tiles in turn, must lie in one group: runs of up to
+// four tiles.  Workgroups there take 16, 24 or 32 tiles: the waves that wait change dies as well.)
+constexpr int KVC_ONCE_GROUP_TILES_VPACKED = 48, KVC_ONCE_GROUP_TILES_KPACKED = 60;
 template <int G = KVC_ONCE_GROUP_TILES>
 __device__ __forceinline__ int64_t kvc_once_group(int64_t tile) { return (int64_t)((uint32_t)tile / (uint32_t)G); }
 template <int G = KVC_ONCE_GROUP_TILES>
@@ -1767,7 +1767,7 @@ template <int FRONT, int ND, int FORM>
 __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int run)
 {
     constexpr bool PACKED = FORM != KVC_FORM_BYTES, LONG = FORM == KVC_FORM_PACKED_LONG;
-    constexpr int G = PACKED && FRONT == 1 ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES;
+    constexpr int G = !PACKED ? KVC_ONCE_GROUP_TILES : FRONT == 1 ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES_KPACKED;
     constexpr int STAGE = PACKED ? (FRONT == 0 ? 0 : KVC_STAGE_VPACKED_BYTES) : FRONT == 0 ? KVC_STAGE_VSYM_BYTES : KVC_STAGE_VF16_BYTES;
     extern __shared__ __align__(16) uint8_t s_dyn[];
     __shared__ uint32_t s_err, s_max_tile, s_longest, s_polls, s_ticket;
@@ -1788,7 +1788,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     // 603 MB, 259 -> 238 us, V 798 -> 483 MB, 182 -> 163 us; K, 2 x 32 x 64 x 8192: 32 -> 31 us.
     // Two symbols a byte: four V tiles are a line of each token's row, and a K tile is lines of its own.
     constexpr int STEP = PACKED ? (FRONT == 1 ? 4 : 1) : FRONT == 1 ? 2 : ND == 24 || ND == 18 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
-    static_assert(G % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
+    static_assert(PACKED ? G % (STEP * 3) == 0 && G % (STEP * 4) == 0 : G % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
     const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
     const int tiles = (int)a.tiles;
     const uint32_t base = a.status[KVC_ONCE_BASE_WORD];
@@ -2211,7 +2211,7 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     // From symbols, long: what is not read yet of the symbols is better kept than the payload (K of 8 x 32 heads x 128 x 4096 tokens 61
     // -> 59 us, of 4 x 32 x 96 x 32 768 203 -> 187).  A short payload may well be read next, by the attention behind the store.
     a.stream_out = !c.src && a.tiles > 4096;
-    const int group_tiles = c.packed && !c.is_k ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES;
+    const int group_tiles = !c.packed ? KVC_ONCE_GROUP_TILES : c.is_k ? KVC_ONCE_GROUP_TILES_KPACKED : KVC_ONCE_GROUP_TILES_VPACKED;
     a.groups = (int)((a.tiles + group_tiles - 1) / group_tiles);
     a.codes_here = c.book != nullptr;
     if (c.book) std::memcpy(a.codes, c.book->encode_table, (size_t)c.table_bytes);
@@ -2293,7 +2293,19 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
         // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
         // together take stays inside a group, or the wave that speaks for a group would wait before all its tiles are counted).
-        if (wide && small && run == 2 && want == 1 && !is_k && a.tiles > 2 * KVC_WIDE_WAVES && 3 * (a.encoded_cap / a.tiles * 9 / 8) <= sa.e.wave_bytes - (c.packed ? KVC_STAGE_VPACKED_BYTES : KVC_STAGE_VF16_BYTES)) run = 4;
+        const int64_t image = a.encoded_cap / a.tiles * 9 / 8;
+        if (c.packed) {
+            // Two symbols a byte: the run that takes least, of those whose images fit beside each other (V: beside the last tile's
+            // staging area).  A round of the waves takes as long as a run's tiles and the look-back, 1.2 tiles' worth.  K by two, three
+            // and four tiles, us: 4 x 32 heads x 64 x 32 768 tokens (65 536 tiles) 154, 143, 124; 4 x 24 x 72 x 16 384 (24 576) 67, 59, 63;
+            // 8 x 32 x 64 x 4160 (16 640) 52, 46, 49; 4 x 32 x 96 x 32 768 184 and 170; 8 x 32 x 128 x 4096 (16 384) 56 and 60.
+            // V, 8 x 32 x 96 x 4160 (12 480): 46 by four, 41 by three.
+            auto cost = [&](int r) { return (a.tiles + (int64_t)KVC_WIDE_WAVES * r - 1) / ((int64_t)KVC_WIDE_WAVES * r) * (5 * r + 6); };
+            for (int r = 3; r <= 4 && small && run >= 2 && want == 1; r++)
+                if ((is_k ? r * image <= sa.e.wave_bytes : (r - 1) * image <= sa.e.wave_bytes - KVC_STAGE_VPACKED_BYTES) && cost(r) <= cost(run)) run = r;
+        } else if (wide && small && run == 2 && want == 1 && !is_k && a.tiles > 2 * KVC_WIDE_WAVES && 3 * image <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) {
+            run = 4;
+        }
         const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
         const auto symbols_kernel = kvc_symbols_kernel(is_k, a.vec_len, !c.packed ? KVC_FORM_BYTES : c.longest_code >= 1 && c.longest_code <= 8 ? KVC_FORM_PACKED : KVC_FORM_PACKED_LONG);
         if (wide) {

@@ -1,5 +1,5 @@
 """First stores whose symbols go from the quantizer to the encoder two to a byte write what stores with a byte per symbol write: every
-vector length, code lengths on both sides of eight bits, runs of one, two and four tiles, groups that leave the quantizer's packed
+vector length, code lengths on both sides of eight bits, runs of one to four tiles, groups that leave the quantizer's packed
 arithmetic, and data whose symbols half a byte does not hold.  The oracle's streams are what the byte path is held to elsewhere."""
 import pytest
 import torch
@@ -63,7 +63,10 @@ CASES = [(True, "ChannelQuant", 128, 1, 1, 128, 0.1, False), (True, "ChannelQuan
          (True, "BlockQuant", 64 * 12, 2, 3, 72, 0.2, True), (True, "BlockQuant", 64 * 100, 2, 24, 64, 0.08, True),
          (False, "TokenQuant", 256, 1, 8, 64, 0.2, False), (False, "TokenQuant", 256, 1, 4, 128, 0.1, True), (False, "TokenQuant", 128 * 34, 8, 32, 128, 0.2, False),
          (False, "TokenQuant", 128 * 34, 4, 32, 96, 0.3, True), (False, "TokenQuant", 128 * 20, 8, 24, 72, 0.1, True), (False, "TokenQuant", 128 * 66, 1, 65, 64, 0.2, False),
-         (False, "TokenQuant", 128 * 130, 1, 65, 64, 0.2, False), (False, "TokenQuant", 128 * 131, 2, 40, 64, 0.1, True), (False, "TokenQuant", 128 * 4, 16, 32, 128, 0.08, False)]
+         (False, "TokenQuant", 128 * 130, 1, 65, 64, 0.2, False), (False, "TokenQuant", 128 * 131, 2, 40, 64, 0.1, True), (False, "TokenQuant", 128 * 4, 16, 32, 128, 0.08, False),
+         # more tiles than waves: runs of three and of four, with a last one that is not whole
+         (True, "ChannelQuant", 64 * 131, 2, 40, 64, 0.2, False), (True, "BlockQuant", 64 * 101, 2, 65, 64, 0.3, True), (True, "ChannelQuant", 64 * 131, 2, 64, 72, 0.2, True),
+         (True, "ChannelQuant", 64 * 132, 2, 64, 96, 0.3, False), (False, "TokenQuant", 128 * 99, 2, 67, 64, 0.2, True), (False, "TokenQuant", 128 * 88, 2, 65, 96, 0.3, False)]
 
 
 @pytest.mark.parametrize("smoothed", [True, False])
