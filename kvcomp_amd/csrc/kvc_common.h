@@ -77,8 +77,13 @@ int kvc_check_hip(hipError_t e, const char *what);
 // reference-signature entry points derive from the decode tree on every call.
 constexpr size_t KVC_WS_SLOT_BYTES = 16384;
 int kvc_workspace_slot(void **slot, void *stream);   // stream: the one the call launches on (a recorded call gets a slot of its own)
-int kvc_quant_packed(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask, float eb,
-                     uint8_t *d_packed, int8_t *d_min_i8, void *d_scale_f16, int64_t *d_counts, void *stream);
+struct KvcCountsToHost {
+    unsigned long long *host;      // pinned host memory: [256] counters, [256] the call's number, written last
+    unsigned long long call;
+    bool handed_over;              // by the quantizer; else the counters are on the device, for the caller to fetch and to clear
+};
+int kvc_quant_to_host(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask, float eb, uint8_t *d_sym,
+                      bool packed, int8_t *d_min_i8, void *d_scale_f16, int64_t *d_counts, KvcCountsToHost *to_host, void *stream);
 int kvc_quant_params(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B, int64_t H, int64_t D, int quant_mask,
                      float eb, int8_t *d_min_i8, void *d_scale_f16, void *stream);
 // What a caller that keeps its decode tables knows beyond the stream itself (all zero: nothing).

@@ -6,8 +6,8 @@
 //   kvc_put_bytes          host bytes to device memory without a copy engine or a pinned buffer
 //
 // What a first store waits for is the histogram of its symbols: 256 numbers.  The quantizers count while they write
-// (kvc_quant.hip), a one-workgroup kernel stores the counters to pinned host memory behind them, and the calling thread
-// looks at that memory until they are there.  The host then builds the code in two or three microseconds; the tie-exact
+// (kvc_quant.hip) and the last workgroup stores the counters to pinned host memory (quantizers that do not count: a kernel of one
+// workgroup behind the histogram), and the calling thread looks at that memory until they are there.  The host then builds the code in two or three microseconds; the tie-exact
 // construction is one serial chain, which a lane of the GPU needed 65 us for (13 symbols).
 // The device has nothing to do from the counts' arrival to the encoder's launch, so the host does only what needs the code
 // in between: everything else (buffers, the encoder's status words and marks) is queued while the quantizer runs.  First
@@ -25,7 +25,7 @@ namespace {
 // Counters on the device (zero between calls: the kernel that hands them over clears them) and where the host reads
 // them.  A call holds one block and returns it before it returns; at most KVC_COUNT_BLOCKS unused ones are kept per device.
 struct CountBlock {
-    unsigned long long *d_counts = nullptr;    // [256]
+    unsigned long long *d_counts = nullptr;    // [256] counters, [256] workgroups that have added theirs
     unsigned long long *h_counts = nullptr;    // [256] counters, [256] number of the call that stored them
     unsigned long long calls = 0;
     int dev = -1;
@@ -55,9 +55,9 @@ int take_block(CountBlock &b)
         }
     }
     b.dev = dev;
-    int rc = kvc_check_hip(hipMalloc((void **)&b.d_counts, 256 * 8), "hipMalloc");
+    int rc = kvc_check_hip(hipMalloc((void **)&b.d_counts, 257 * 8), "hipMalloc");
     if (!rc) rc = kvc_check_hip(hipHostMalloc((void **)&b.h_counts, 257 * 8, hipHostMallocDefault), "hipHostMalloc");
-    if (!rc) rc = kvc_check_hip(hipMemset(b.d_counts, 0, 256 * 8), "hipMemset");
+    if (!rc) rc = kvc_check_hip(hipMemset(b.d_counts, 0, 257 * 8), "hipMemset");
     if (!rc) rc = kvc_check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize");       // once per block: the call may be on any stream
     if (rc) {
         free_block(b);
@@ -169,9 +169,9 @@ static int kvc_quant_counted_form(const void *d_x_f16, int64_t NB, int64_t BS, i
         return rc;
     }
     block->calls++;
-    int rc = packed ? kvc_quant_packed(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, d_min_i8, d_scale_f16, (int64_t *)block->d_counts, stream_)
-                    : kvc_quant(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, d_min_i8, d_scale_f16, nullptr, (int64_t *)block->d_counts, stream_);
-    if (!rc) {
+    KvcCountsToHost to_host = {block->h_counts, block->calls, false};
+    int rc = kvc_quant_to_host(d_x_f16, NB, BS, B, H, D, quant_mask, eb, d_sym, packed, d_min_i8, d_scale_f16, (int64_t *)block->d_counts, &to_host, stream_);
+    if (!rc && !to_host.handed_over) {
         hipLaunchKernelGGL(kvc_counts_to_host_kernel, dim3(1), dim3(256), 0, stream, block->d_counts, block->h_counts, block->calls);
         rc = kvc_check_hip(hipGetLastError(), "kvc_counts_to_host_kernel launch");
     }
