@@ -36,8 +36,8 @@ struct KvcQuantArgs {
 // symbol counts on the way out (HIST kernels)
 // ---------------------------------------------------------------------------------------------------
 // A first store needs the histogram of the symbols it has just written.  Counting them while they are in registers
-// costs the quantizers, which wait for HBM, little (402 M symbols: per-token rows of 12 288 222 us without, 239 us with;
-// per-channel groups 214 and 235 us), where kvc_histogram_kernel reads every symbol back (111 us).  One counter per (bin, lane & 31), as there:
+// costs the quantizers, which wait for HBM, little (402 M symbols, a byte each, rows of 12 288 by one wave each: per-token rows 222 us
+// without, 239 us with; per-channel groups 214 and 235 us; today 192 and 199 with counts and two symbols to a byte), where kvc_histogram_kernel reads every symbol back (111 us).  One counter per (bin, lane & 31), as there:
 // counter (bin, c) lies in LDS bank c, so the lanes of a half wave never collide.  64 bins (8 KB, so that the counters do
 // not cost occupancy) hold every symbol that an error bound of 1/62 or more gives; the rare others go to the global
 // counters one by one.
