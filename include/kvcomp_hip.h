@@ -236,8 +236,8 @@ int kvc_encode_async(const kvc_encode_job *job, void *stream);
 /* The same for callers that would rather not wait for what the host has to do in between.
  * kvc_encode_prepare: the first launch of an encode from symbols whose table and payload buffer are not known yet
  *   (d_encode_tables, encode_table_bytes, d_encoded and encoded_cap are not looked at).  d_result's eight words and
- *   *d_stream_bytes are cleared.  d_scratch: kvc_encode_scratch_bytes() of device memory on a 16-byte boundary, in use until
- *   the encode has run.  *prepared receives what to pass on.
+ *   *d_stream_bytes are cleared.  d_scratch: kvc_encode_scratch_bytes() of device memory (16 KiB do if
+ *   the symbols are a byte each) on a 16-byte boundary, in use until the encode has run.  *prepared receives what to pass on.
  * kvc_encode_prepare_packed: the same for symbols that kvc_quant_counted_packed writes, two to a byte.
  * kvc_encode_queue: kvc_encode_async, continuing what was prepared on the same stream for the same tokens and outputs
  *   (prepared = 0: nothing was; d_scratch is not used then).  longest_code: bits of the longest code in the (one) encode

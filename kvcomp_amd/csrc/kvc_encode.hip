@@ -2503,8 +2503,9 @@ static int kvc_encode_prepare_form(const kvc_encode_job *job, bool packed, void 
     KvcEncodeCall c = {};
     if (int rc = kvc_encode_job_check(job, c)) return rc;
     KVC_REQUIRE(job->d_result != nullptr && job->d_stream_bytes != nullptr, "NULL argument");
-    KVC_REQUIRE(d_scratch != nullptr && ((uintptr_t)d_scratch & 15) == 0 && scratch_bytes >= KVC_ENC_SCRATCH_BYTES, "scratch memory: %lld bytes, on a 16-byte boundary",
-                (long long)KVC_ENC_SCRATCH_BYTES);
+    const int64_t scratch_needed = packed ? KVC_ENC_SCRATCH_BYTES : (int64_t)KVC_WS_SLOT_BYTES;
+    KVC_REQUIRE(d_scratch != nullptr && ((uintptr_t)d_scratch & 15) == 0 && scratch_bytes >= scratch_needed, "scratch memory: %lld bytes, on a 16-byte boundary",
+                (long long)scratch_needed);
     KVC_REQUIRE(job->d_sym != nullptr && job->rows_per_codebook == 0 && job->d_codebook_meta == nullptr, "only an encode from symbols with one codebook can be prepared");
     static const uint8_t no_table[8] = {};
     c.d_tables = no_table;                                 // (not read by the launch; the call has its own)

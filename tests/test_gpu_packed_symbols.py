@@ -111,3 +111,19 @@ def test_unaligned_input_keeps_a_byte_per_symbol(packed):
     shifted = torch.empty(x.numel() + 4, dtype=torch.float16, device=DEV)[4:].view(x.shape).copy_(x)
     _both(True, "ChannelQuant", shifted, 0.1)
     assert not packed
+
+
+@pytest.mark.parametrize("name,room,taken", [("kvc_encode_prepare", 16384, True), ("kvc_encode_prepare", 16383, False),
+                                             ("kvc_encode_prepare_packed", 16384, False), ("kvc_encode_prepare_packed", 20480, True)])
+def test_scratch_that_a_preparation_asks_for(name, room, taken):
+    import ctypes as C
+    T, B, H, D = 128, 1, 2, 128
+    sizes = m.buffer_sizes(T, B * H * D, True, H, D)
+    sym, scratch = torch.zeros(T * B * H * D, dtype=torch.uint8, device=DEV), torch.empty(20480, dtype=torch.uint8, device=DEV)
+    infos, state = [torch.empty(n, dtype=torch.uint8, device=DEV) for n in sizes[:2]], torch.zeros(16, dtype=torch.int32, device=DEV)
+    job = _lib.EncodeJob(is_k=1, d_sym=sym.data_ptr(), tokens=T, batch=B, heads=H, head_dim=D, d_block_infos=infos[0].data_ptr(),
+                         d_thread_infos=infos[1].data_ptr(), d_result=state.data_ptr(), d_stream_bytes=state.data_ptr() + 32)
+    done = C.c_int(0)
+    rc = getattr(_lib.lib(), name)(C.byref(job), scratch.data_ptr(), room, C.byref(done), torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert (rc == 0) == taken
