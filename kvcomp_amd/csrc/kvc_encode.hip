@@ -780,38 +780,38 @@ __device__ __forceinline__ void kvc_write_image(const KvcEncodeArgs &a, const Kv
     }
 }
 
-// The same for an image that was packed from its first word on, while the payload starts p.head bytes into an
-// aligned word of the destination: every output word is put together from two image words, four words of a lane at a time.
+// The same for an image that was packed from its first word on, whatever byte of the destination the payload starts at: whole
+// 16-byte pieces of the destination, each put together from five image words, and the bytes at the two ends.
+// (A word per lane and store took a wave of the kernel from symbols 23 % (K) and 16 % (V) of its time, whose stores queue up with the
+// sixteen waves' of its compute unit; a quarter as many stores take 13 and 10.  First stores, K and V, us: 4 x 32 heads x 96 x 32 768
+// tokens 167 -> 159 and 125.5 -> 117.5, 8 x 32 x 128 x 4096 54.6 -> 51.9 and 49.6 -> 47.1.)
 __device__ __forceinline__ void kvc_write_image_shifted(const KvcEncodeArgs &a, const KvcEmitPlace &p, int lane, const uint32_t *image)
 {
-    uint32_t *dst = reinterpret_cast<uint32_t *>(a.encoded + p.off - p.head);
-    const uint32_t lo = p.head, hi = p.head + p.bn;            // valid byte range of the output words
-    const uint32_t shift = 8u * (4u - p.head);                 // 32, 24, 16, 8
-    const uint32_t first = lo ? 1u : 0u, end = hi >> 2;        // whole words
-    for (uint32_t f0 = lane; f0 < end; f0 += 4 * KVC_WAVE) {
-        uint32_t word[4];
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++) {
-            const uint32_t f = f0 + k * KVC_WAVE < end ? f0 + k * KVC_WAVE : f0;
-            const uint32_t cur = image[f], prev = image[f ? f - 1 : 0];
-            word[k] = lo ? (uint32_t)((((uint64_t)cur << 32) | prev) >> shift) : cur;
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < 4; k++) {
-            const uint32_t f = f0 + k * KVC_WAVE;
-            if (f >= first && f < end) {
-                if (a.stream_out) __builtin_nontemporal_store(word[k], dst + f);
-                else dst[f] = word[k];
-            }
-        }
+    const uint32_t head = (uint32_t)(reinterpret_cast<uintptr_t>(a.encoded) + p.off) & 15u;
+    uint8_t *dst = a.encoded + p.off - head;                   // 16-byte aligned
+    const uint32_t hi = head + p.bn;                           // valid bytes: head .. hi - 1
+    const uint32_t first = head ? 1u : 0u, end = hi >> 4;      // whole pieces
+    const uint32_t turn = (4u - head) & 3u;                    // bytes of an image word that belong to the destination word before
+    const uint32_t *from = image - ((head + 3u) >> 2);
+    for (uint32_t c = first + lane; c < end; c += KVC_WAVE) {
+        const uint32_t *w = from + 4u * c;
+        const uint32_t w0 = w[0], w1 = w[1], w2 = w[2], w3 = w[3], w4 = w[4];
+        kvc_u32x4 v;
+        v.x = __builtin_amdgcn_alignbyte(w1, w0, turn);
+        v.y = __builtin_amdgcn_alignbyte(w2, w1, turn);
+        v.z = __builtin_amdgcn_alignbyte(w3, w2, turn);
+        v.w = __builtin_amdgcn_alignbyte(w4, w3, turn);
+        kvc_u32x4 *to = reinterpret_cast<kvc_u32x4 *>(dst) + c;
+        if (a.stream_out) __builtin_nontemporal_store(v, to);
+        else *to = v;
     }
-    // the bytes at the ragged ends: of word 0 by lanes 0 .. 3, of the last word by lanes 4 .. 7
-    if (lane < 8) {
-        const uint32_t f = lane < 4 ? 0u : end, b = 4u * f + (lane & 3);
-        const bool ragged = lane < 4 ? lo != 0u : (end != 0u || lo == 0u) && (hi & 3u) != 0u;
-        if (ragged && b >= lo && b < hi) {
-            const uint32_t at = b - lo;                        // byte of the payload: image word at / 4
-            reinterpret_cast<uint8_t *>(dst)[b] = (uint8_t)(image[at >> 2] >> (8u * (at & 3u)));
+    // the first piece's bytes by lanes 0 .. 15, the last one's by lanes 16 .. 31
+    if (lane < 32) {
+        const uint32_t b = (lane < 16 ? 0u : 16u * end) + (lane & 15);
+        const bool ragged = lane < 16 ? head != 0u : (hi & 15u) != 0u && end >= first;
+        if (ragged && b >= head && b < hi) {
+            const uint32_t at = b - head;                      // byte of the payload: image word at / 4
+            dst[b] = (uint8_t)(image[at >> 2] >> (8u * (at & 3u)));
         }
     }
 }
