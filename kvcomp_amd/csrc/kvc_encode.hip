@@ -1760,8 +1760,10 @@ __device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint
 // K tile needs no staging, since the quantizer, which has it in registers, writes it in the order of the lanes.  A byte is the index of
 // a pair's look-up; V's pairs lie along the other axis, and are turned in registers.  Codes of any length are taken, since what
 // would be left over would have to be written out again (K of 2 x 32 x 96 x 4480 in block groups, codes of 11 bits).
-// With the runs and the late look-back of today this kernel takes 57 and 49 us there, and 167 and 121; made-up offsets, so without any
-// look-back, had given 50 and 42, and 146 and 99 for 60 and 50, and 198 and 126: waves wait for the slowest tile before theirs.
+// With today's runs, late look-back and wide stores this kernel takes 54 and 47 us there, and 159 and 115.  Where a wave's time goes (clock
+// stamps, K | V of 4 x 32 x 96 x 32 768): start 9 | 8 %, loads 12 | 15, look-ups 14 | 18, packing 20 | 22, looking back 28 | 23, writing
+// 13 | 10.  Made-up offsets, so no look-back, had given 146 and 99 us for 198 and 126: waves wait for the slowest tile before theirs.
+// Three workgroups per compute unit with smaller areas and runs of two: K 162 -> 177 us.
 // FRONT 0: K, 1: V.  ND: registers that a vector fills, a byte per symbol.  FORM: a byte per symbol, or two symbols a byte with codes
 // of at most eight bits, or of any length.
 enum { KVC_FORM_BYTES = 0, KVC_FORM_PACKED = 1, KVC_FORM_PACKED_LONG = 2 };
