@@ -245,7 +245,7 @@ int kvc_encode_async(const kvc_encode_job *job, void *stream);
  *   receive d_result's eight words, *d_stream_bytes and, last, outcome_number (word 9), as the call ends on the device; words
  *   10 - 12 are set to the stream (low half, high half) and the device before an accepted call returns.
  * kvc_encode_queue_book: kvc_put_codebook and kvc_encode_queue with the table that it puts in place (the job's own is not looked at),
- *   for calls that were prepared; d_tables and d_lut are written by the time the call has run.
+ *   for calls that were prepared; d_tables and d_lut are written before the outcome's number, as all outputs.
  * kvc_wait_outcome: waits until outcome_number has arrived in such words.  If it has not come after two seconds and
  *   everything queued on their stream has run, it returns too, with word 9 saying that the number has not come; the stream
  *   must exist as long.  No other stream is waited for, and the current device does not matter. */

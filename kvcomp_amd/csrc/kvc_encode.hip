@@ -1138,6 +1138,7 @@ constexpr uint32_t KVC_NO_CODE_LEN = 0x4000u;       // length of a symbol withou
 // maxima go to one of 32 lines picked by the workgroup number (kvc_encode_finish_kernel joins them afterwards).
 // The ticket counter shares the line of the call's status words, which nobody touches before the last tile is placed.
 constexpr int KVC_ONCE_POLLS_WORD = 6;               // status word: most looks of one wave that found a word not ready
+constexpr int KVC_ONCE_DONE_WORD = 7;                // status word: workgroups of kvc_encode_finish_put_kernel that are done
 constexpr int KVC_ONCE_TICKET_WORD = 16;             // workgroups started so far
 constexpr int KVC_ONCE_BASE_WORD = 32;               // copy of status[KVC_ENC_ST_BASE]
 constexpr int KVC_ONCE_PART_WORD = 64, KVC_ONCE_PART_LINES = 32, KVC_ONCE_PART_STRIDE = 32;   // {error bits, largest tile, longest stream, polls}
@@ -1936,6 +1937,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
 // every tile: nothing in it waits for another workgroup, so it always ends, and since the inputs are untouched the
 // outputs are the ones the call was to produce.  Slow (four waves for all tiles), and next to never needed: the
 // look-back's progress does not depend on the order in which the hardware starts workgroups.
+// What is left to the caller is kvc_encode_publish, by the threads of wave 0, which wrote what it reads or are ordered behind it.
 template <int FRONT>
 __device__ __forceinline__ void kvc_encode_finish(const KvcStoreArgs &a)
 {
@@ -1977,10 +1979,7 @@ __device__ __forceinline__ void kvc_encode_finish(const KvcStoreArgs &a)
         }
     }
     __syncthreads();
-    if (!s_again) {                                       // the rule
-        kvc_encode_publish(a.e, tid);
-        return;
-    }
+    if (!s_again) return;                                 // the rule
     // ---- the whole call again, two passes inside this workgroup ----
     const int64_t tiles = a.e.tiles;
     for (int64_t tile = wave; tile < tiles; tile += KVC_WAVES_PER_WG) {      // count: thread_infos, byte_nums, group parameters
@@ -2066,14 +2065,19 @@ __device__ __forceinline__ void kvc_encode_finish(const KvcStoreArgs &a)
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
-    kvc_encode_publish(a.e, tid);
 }
 
 template <int FRONT>
-__global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs a) { kvc_encode_finish<FRONT>(a); }
+__global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs a)
+{
+    kvc_encode_finish<FRONT>(a);
+    kvc_encode_publish(a.e, threadIdx.x);
+}
 
 // ... and, by a second workgroup beside it, a first store's codebook to where it is kept and its decode tables
-// (kvc_put_codebook).  The encoder has its codes in the argument block, so between the counts' arrival and the encoder nothing is
+// (kvc_put_codebook).  Whoever sees the call's number relies on both, on whatever stream: each workgroup makes what it wrote
+// visible (every wave its own stores, to the whole system) and counts itself done, and the one that is second publishes.  Neither
+// waits for the other.  The encoder has its codes in the argument block, so between the counts' arrival and the encoder nothing is
 // left but the launch, where this took a launch of its own in front of it: K and V of 8 heads x 777 tokens 246 -> 234 us, 8 x 32 x 128 x
 // 4096 370 -> 363.
 struct KvcPutSmallArgs {
@@ -2084,13 +2088,21 @@ struct KvcPutSmallArgs {
 };
 __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_put_kernel(KvcStoreArgs a, KvcPutSmallArgs p)
 {
+    __shared__ uint32_t s_done;
     if (blockIdx.x == 0) {
         kvc_encode_finish<0>(a);
-        return;
+    } else {
+        const uint8_t *src = reinterpret_cast<const uint8_t *>(p.words);
+        for (int i = threadIdx.x; i < p.bytes; i += KVC_WG) p.dst[i] = src[i];
+        kvc_build_lut_body(src + p.tree_at, p.bytes - p.tree_at, p.node_bytes, p.lut);
     }
-    const uint8_t *src = reinterpret_cast<const uint8_t *>(p.words);
-    for (int i = threadIdx.x; i < p.bytes; i += KVC_WG) p.dst[i] = src[i];
-    kvc_build_lut_body(src + p.tree_at, p.bytes - p.tree_at, p.node_bytes, p.lut);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) s_done = atomicAdd(&a.e.status[KVC_ONCE_DONE_WORD], 1u);
+    __syncthreads();
+    if (s_done == 0u) return;
+    __threadfence();                                       // (what the other workgroup has written is read from memory)
+    kvc_encode_publish(a.e, threadIdx.x);
 }
 
 // What the fused path adds to an encode call: the fp16 source and how to quantize it.

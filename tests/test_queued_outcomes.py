@@ -246,6 +246,36 @@ def test_stores_on_a_stream_are_learnt_of_on_another(is_k):
     assert not got._unverified
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("is_k", [True, False])
+def test_a_first_store_that_is_learnt_of_has_its_codebook_in_place(monkeypatch, is_k):
+    """What a first store's outcome says on one stream goes for the codebook and the decode tables on any other."""
+    from tests import _synth as S
+    _config()
+    x = (S.synth_k if is_k else S.synth_v)(640, 2, 4, 128).to(DEV)
+    room = kvcomp_cuda.codebook_room
+    monkeypatch.setattr(kvcomp_cuda, "codebook_room", lambda device: room(device).fill_(0xee))     # (not what an earlier one has left there)
+    want = _store_all(is_k, [x])
+    names = ("encode_codebook", "decode_codebook", "_lut", "encoded_data", "block_infos", "thread_infos")
+    expect = {name: getattr(want, name).clone() for name in names}
+    restored = want.get_only_compressed()[0]
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    for i in range(10):
+        with torch.cuda.stream(first):
+            got = _store_all(is_k, [x])
+        with torch.cuda.stream(second):                               # ordered behind nothing
+            if got._unverified:
+                got._outcome.synchronize()
+            copies = [getattr(got, name).clone() for name in names]
+            again = got.get_only_compressed()[0]
+        second.synchronize()
+        for name, value in zip(names, copies):
+            assert torch.equal(value, expect[name]), (name, i)
+        assert torch.equal(again, restored), i
+        torch.cuda.synchronize()
+
+
 class _FromAnotherStream:
     """Stands for a tensor in device memory that came from another stream; notes the streams it is kept for."""
     is_cuda = True
