@@ -1,4 +1,7 @@
 """One-token appends through the native module do what the Python code beside them does, over the forms that either may meet."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -96,3 +99,46 @@ def test_rows_behind_a_tail(monkeypatch, D, form):
             held.append((ctx.buffer, ctx.ctx_len, ctx._tail._version))
     assert torch.equal(held[0][0], held[1][0]) and held[0][1:2] == held[1][1:2] and held[0][0].shape[0] == 7
     assert held[0][2] == held[1][2]
+
+
+def _sleep_for(seconds):
+    """Keep the current stream busy for about that long, with a kernel that counts clock ticks."""
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    torch.cuda._sleep(1000000)
+    start.record()
+    torch.cuda._sleep(10000000)
+    end.record()
+    end.synchronize()
+    torch.cuda._sleep(int(10000000 * seconds * 1e3 / start.elapsed_time(end)))
+
+
+@pytest.mark.parametrize("which", ["append_rows", "append_dense"])
+def test_other_threads_run_on_while_an_append_waits_for_its_queue(which):
+    """Appends behind a kernel of half a second fill their queue (2700 of them do); the launch that waits for room then does so
+    without the interpreter's lock."""
+    tail, rows = torch.zeros(64, 1, 1, 64, dtype=torch.float16, device=DEV), _randn(1, 1, 1, 64)
+    call = {"append_rows": lambda: _lib.host().append_rows(tail, 0, rows, 128),
+            "append_dense": lambda: _lib.host().append_dense(rows, rows, None, None, tail.view(1, 1, 64, 64), tail.view(1, 1, 64, 64), 0)}[which]
+    assert call() == 1
+    gaps, stop = [], threading.Event()
+
+    def other():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.0005)
+            gaps.append(time.perf_counter() - last)
+            last += gaps[-1]
+
+    thread = threading.Thread(target=other)
+    _sleep_for(0.5)
+    begun, longest = time.perf_counter(), 0.0
+    thread.start()
+    while time.perf_counter() - begun < 0.4:
+        before = time.perf_counter()
+        call()
+        longest = max(longest, time.perf_counter() - before)
+    stop.set()
+    thread.join()
+    torch.cuda.synchronize()
+    assert longest > 0.1, "no append has waited"
+    assert max(gaps) < longest / 2
