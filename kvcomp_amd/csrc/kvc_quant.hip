@@ -294,7 +294,8 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_channel_once_kernel(KvcQuant
         kvc_quant_publish(a, g + 1, g1);
         const bool applies = kvc_packed_quantizer_applies(g0, kvc_half_lo(mxw)) && kvc_packed_quantizer_applies(g1, kvc_half_hi(mxw));
         if constexpr (PACK) {
-            // (lanes exchange bytes: all of a wave take one way.  The fp32 chain gives the same symbols, to whichever lane)
+            // (lanes exchange bytes: all of a wave take one way, and where that is the fp32 chain, a lane whose groups the packed
+            // arithmetic applies to takes its symbols all the same: for a NaN they differ, and must not between the passes)
             const bool packed = __all(applies);
             const KvcPackedParams pp = kvc_packed_params(g0, g1);
             const uint32_t D = (uint32_t)a.D, col = (uint32_t)c / D, lane = threadIdx.x & 3;
@@ -303,16 +304,14 @@ __global__ void __launch_bounds__(KVC_WG) kvc_quant_channel_once_kernel(KvcQuant
             auto store = [&](auto chunk) {                             // (the offsets are constants then)
 #pragma unroll
                 for (int t = 0; t < KVC_WAVE; t += 4) {
-                    uint2 w;
-                    if (packed) {
-                        w.x = kvc_low_bytes4(kvc_quant_pair_biased(raw[t], pp), kvc_quant_pair_biased(raw[t + 1], pp));
-                        w.y = kvc_low_bytes4(kvc_quant_pair_biased(raw[t + 2], pp), kvc_quant_pair_biased(raw[t + 3], pp));
-                    } else {
+                    uint2 w = make_uint2(kvc_low_bytes4(kvc_quant_pair_biased(raw[t], pp), kvc_quant_pair_biased(raw[t + 1], pp)),
+                                         kvc_low_bytes4(kvc_quant_pair_biased(raw[t + 2], pp), kvc_quant_pair_biased(raw[t + 3], pp)));
+                    if (!packed) {
                         uint32_t s[4];
 #pragma unroll
                         for (int k = 0; k < 4; k++)
                             s[k] = (uint32_t)kvc_quant_one(kvc_half_lo(raw[t + k]), g0) | (uint32_t)kvc_quant_one(kvc_half_hi(raw[t + k]), g1) << 8;
-                        w = make_uint2(s[0] | s[1] << 16, s[2] | s[3] << 16);
+                        if (!applies) w = make_uint2(s[0] | s[1] << 16, s[2] | s[3] << 16);
                     }
                     if constexpr (HIST) {
                         kvc_hist_add4(a, s_bins, w.x);

@@ -127,3 +127,19 @@ def test_scratch_that_a_preparation_asks_for(name, room, taken):
     rc = getattr(_lib.lib(), name)(C.byref(job), scratch.data_ptr(), room, C.byref(done), torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert (rc == 0) == taken
+
+
+@pytest.mark.parametrize("mode", ["ChannelQuant", "BlockQuant", "TokenQuant"])
+@pytest.mark.parametrize("bits", [0x7e00, 0x7e05, 0xfe0b, 0x7fff])
+@pytest.mark.parametrize("tiny", [False, True])
+def test_not_a_number_gives_the_same_symbol_in_every_pass(packed, mode, bits, tiny):
+    """What a NaN's symbol is depends on which arithmetic its group takes: that of the group, whatever the groups beside it take."""
+    is_k = mode != "TokenQuant"
+    x = _data(256, 1, 4, 128, False, 12)
+    x[70:90, :, 1, 6] = torch.tensor(bits, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.float16)
+    if is_k:
+        x[:128, :, 1, 8:10] = 3.0                                     # no range, a scale of zero
+    if tiny:                                                          # more symbols than half a byte holds
+        x[128:192, :, 2, 4] = torch.arange(64, device=DEV).remainder(19).float().mul(2.0 ** -24).to(torch.float16)[:, None]
+    _both(is_k, mode, x, 0.08)
+    assert len(packed) == 1
