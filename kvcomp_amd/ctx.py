@@ -723,14 +723,17 @@ class KVCompCtx:
         prepared = []
 
         fresh = self._state is None and self._encoded.used == 0
-        packed = not want_symbols and fresh and kvcomp_cuda.packed_symbols_supported(self.is_k, self._mask, blocked, self.quant_scale_rel)
+        smoothed = self._smoothed_symbols() if self.codebook_smoothing else 0
+        # (just below 1/13, where the library's fp32 bound is 1/13, smoothing gives codes to seventeen symbols: packed ones would
+        # always be written again a byte each)
+        packed = (not want_symbols and fresh and smoothed <= 16 and
+                  kvcomp_cuda.packed_symbols_supported(self.is_k, self._mask, blocked, self.quant_scale_rel))
 
         def meanwhile(symbols):
             if fresh:
                 prepared.extend((self._prepare_encode(T, symbols, packed), kvcomp_cuda.codebook_room(device)))
         quantize = kvcomp_cuda.quant_codebook_packed if packed else kvcomp_cuda.quant_codebook
-        sym, book = quantize(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale,
-                                               self._smoothed_symbols() if self.codebook_smoothing else 0, meanwhile)
+        sym, book = quantize(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale, smoothed, meanwhile)
         self.waits += 1
         if packed and book.encode_bytes > 16 * 8:              # scales among fp16's smallest numbers: half a byte does not hold these symbols
             sym = quant(blocked, self.quant_dims, self.quant_scale_rel)[0]

@@ -143,3 +143,11 @@ def test_not_a_number_gives_the_same_symbol_in_every_pass(packed, mode, bits, ti
         x[128:192, :, 2, 4] = torch.arange(64, device=DEV).remainder(19).float().mul(2.0 ** -24).to(torch.float16)[:, None]
     _both(is_k, mode, x, 0.08)
     assert len(packed) == 1
+
+
+@pytest.mark.parametrize("is_k,mode", [(True, "ChannelQuant"), (False, "TokenQuant")])
+@pytest.mark.parametrize("eb,smoothed,taken", [(1 / 13, True, 1), (0.0769230769, False, 1), (0.0769230769, True, 0)])
+def test_codes_for_seventeen_symbols_keep_a_byte_per_symbol(packed, is_k, mode, eb, smoothed, taken):
+    """An error bound that is 1/13 as an fp32 number and a little less in double precision: smoothing starts from ceil(1 / eb)."""
+    ctx = _both(is_k, mode, _data(256, 1, 4, 128, False, 4), eb, smoothed)
+    assert len(packed) == taken and (ctx.encode_codebook.numel() > 16 * 8) == (not taken)
