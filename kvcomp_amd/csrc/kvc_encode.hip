@@ -64,7 +64,6 @@ struct KvcEncodeArgs {
     int wave_bytes;                // one-pass kernel from symbols: LDS of a wave
     int packed;                    // sym holds two symbols a byte (kvc_packed_symbols)
     int groups;                    // one pass: groups of tiles, see KVC_ONCE_GROUP_TILES
-    int stream_out;                // the payload is long and not written to stay in the caches
     // a first store's table (at most sixteen entries), which comes in the argument block: table is written behind the encode only
     int codes_here;
     uint2 codes[16];
@@ -784,7 +783,8 @@ __device__ __forceinline__ void kvc_write_image(const KvcEncodeArgs &a, const Kv
 // 16-byte pieces of the destination, each put together from five image words, and the bytes at the two ends.
 // (A word per lane and store took a wave of the kernel from symbols 23 % (K) and 16 % (V) of its time, whose stores queue up with the
 // sixteen waves' of its compute unit; a quarter as many stores take 13 and 10.  First stores, K and V, us: 4 x 32 heads x 96 x 32 768
-// tokens 167 -> 159 and 125.5 -> 117.5, 8 x 32 x 128 x 4096 54.6 -> 51.9 and 49.6 -> 47.1.)
+// tokens 167 -> 159 and 125.5 -> 117.5, 8 x 32 x 128 x 4096 54.6 -> 51.9 and 49.6 -> 47.1.  Past the caches they gain nothing more: first
+// stores of 512 to 65 536 tiles, symbols of half a byte and of a byte, with attention behind them and without, within 0.5 % either way.)
 __device__ __forceinline__ void kvc_write_image_shifted(const KvcEncodeArgs &a, const KvcEmitPlace &p, int lane, const uint32_t *image)
 {
     const uint32_t head = (uint32_t)(reinterpret_cast<uintptr_t>(a.encoded) + p.off) & 15u;
@@ -801,9 +801,7 @@ __device__ __forceinline__ void kvc_write_image_shifted(const KvcEncodeArgs &a, 
         v.y = __builtin_amdgcn_alignbyte(w2, w1, turn);
         v.z = __builtin_amdgcn_alignbyte(w3, w2, turn);
         v.w = __builtin_amdgcn_alignbyte(w4, w3, turn);
-        kvc_u32x4 *to = reinterpret_cast<kvc_u32x4 *>(dst) + c;
-        if (a.stream_out) __builtin_nontemporal_store(v, to);
-        else *to = v;
+        reinterpret_cast<kvc_u32x4 *>(dst)[c] = v;
     }
     // the first piece's bytes by lanes 0 .. 15, the last one's by lanes 16 .. 31
     if (lane < 32) {
@@ -2224,9 +2222,6 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
     a.outcome_number = c.outcome_number;
     a.clear = c.clear;
     a.packed = c.packed;
-    // From symbols, long: what is not read yet of the symbols is better kept than the payload (K of 8 x 32 heads x 128 x 4096 tokens 61
-    // -> 59 us, of 4 x 32 x 96 x 32 768 203 -> 187).  A short payload may well be read next, by the attention behind the store.
-    a.stream_out = !c.src && a.tiles > 4096;
     const int group_tiles = !c.packed ? KVC_ONCE_GROUP_TILES : c.is_k ? KVC_ONCE_GROUP_TILES_KPACKED : KVC_ONCE_GROUP_TILES_VPACKED;
     a.groups = (int)((a.tiles + group_tiles - 1) / group_tiles);
     a.codes_here = c.book != nullptr;
