@@ -21,6 +21,20 @@ class _Own(torch.Tensor):
     pass
 
 
+def _note_answers(monkeypatch):
+    """What the native functions answer from now on."""
+    module, answers = _lib.host(), []
+
+    def noting(function):
+        def call(*args):
+            answers.append(function(*args))
+            return answers[-1]
+        return call
+    noted = type("Noted", (), {name: staticmethod(noting(getattr(module, name))) for name in ("append_dense", "append_rows")})
+    monkeypatch.setattr(_lib, "host", lambda: noted)
+    return answers
+
+
 def _randn(*shape, dtype=torch.float16):
     g = torch.Generator(device=DEV).manual_seed(sum(shape))
     return torch.randn(*shape, generator=g, device=DEV).to(dtype)
@@ -47,6 +61,7 @@ FORMS = {
     "no tokens": lambda k, v, c, s: (k[:, :, :0], v[:, :, :0], c[:, :0], s[:, :0]),
     "rows of 15": lambda k, v, c, s: (k[..., :15], v[..., :15], c[..., :15], s[..., :15]),
 }
+TAKEN = {"plain", "angles of every sequence", "no angles", "tokens first", "slices", "a parameter", "no tokens"}      # by the native function
 
 
 @pytest.mark.parametrize("form", FORMS)
@@ -55,48 +70,56 @@ def test_append_dense(monkeypatch, form, grad):
     args = FORMS[form](_randn(B, H, T, D), _randn(B, H, T, D) + 1, _randn(1, T, D), _randn(1, T, D))
     wide = args[0].shape[3]
     caches = [torch.zeros(B, H, 12, wide, dtype=torch.float16, device=DEV) for _ in range(4)]
+    answers = _note_answers(monkeypatch)
     with torch.set_grad_enabled(grad):
         native = append_dense(*args, *caches[:2], 4)
         monkeypatch.setattr(_lib, "host", lambda: _NotTaken)
         assert append_dense(*args, *caches[2:], 4) is native
-    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3]) and (not native or T == 0 or bool(args[0].numel()) == bool(caches[0].any()))
+    taken = form in TAKEN or (not grad and form.startswith("a gradient"))
+    assert answers == ([] if form == "host memory" else [int(taken)]) and native >= taken
+    assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3]) and (not native or bool(args[0].numel()) == bool(caches[0].any()))
 
 
 def test_append_dense_to_other_caches(monkeypatch):
     args = (_randn(B, H, T, D), _randn(B, H, T, D), None, None)
     room = torch.zeros(B, H, 12, D, dtype=torch.float16, device=DEV)
+    noted = _note_answers(monkeypatch)
     for caches in ((room, room[:, :, :10]), (room[:1], room[:1]), (room.permute(0, 2, 1, 3), room), (room.float(), room), (room, room.cpu())):
         answers = [append_dense(*args, *caches, 4)]
         with monkeypatch.context() as m:
             m.setattr(_lib, "host", lambda: _NotTaken)
             answers.append(append_dense(*args, *caches, 4))
-        assert answers == [False, False]
+        assert answers == [False, False] and noted.pop() == 0 and not noted
     with pytest.raises(_lib.KvcompError):
         append_dense(*args, room, room.clone(), 8)                 # five tokens behind eight of twelve
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
         assert append_dense(*args, room, room.clone(), 4)
     side.synchronize()
+    assert len(noted) == 2 and noted[0] < 0 and noted[1] == 1
     assert torch.equal(room[:, :, 4:4 + T], args[0])
 
 
 @pytest.mark.parametrize("D,form", [(D, f) for D in (64, 8) for f in ("plain", "permuted", "offset", "gradient", "own")])
 def test_rows_behind_a_tail(monkeypatch, D, form):
     KVCompCacheConfigStatic.config = KVCompCacheConfig("t", QuantMode("ChannelQuant"), QuantMode("TokenQuant"), 64, 128, 64, 128, 0.1, 0.2)
-    heads = 1
+    heads = 2
     rows = {"plain": lambda x: x, "permuted": lambda x: x.permute(2, 1, 0, 3).contiguous().permute(2, 1, 0, 3),
             "offset": lambda x: torch.empty(x.numel() + 3, dtype=x.dtype, device=DEV)[3:].view(x.shape).copy_(x),
             "gradient": lambda x: x.clone().requires_grad_(), "own": lambda x: x.as_subclass(_Own)}[form]
-    held = []
+    held, counts = [], (1, 3, 1, 2)
     for native in (True, False):
         with monkeypatch.context() as m:
+            answers = _note_answers(m)
             if not native:
                 m.setattr(_lib, "host", lambda: _NotTaken)
             ctx = KVCompCtx(True, 1, heads, D, 0.1)
             with torch.no_grad():
-                for n in (1, 3, 1, 2):
+                for n in counts:
                     ctx.store(rows(_randn(n, 1, heads, D)))
             held.append((ctx.buffer, ctx.ctx_len, ctx._tail._version))
+            taken = {"plain": [1] * 4, "permuted": [int(n == 1) for n in counts]}.get(form, [0] * 4)     # (one token is in order either way)
+            assert answers == (taken if native else [])
     assert torch.equal(held[0][0], held[1][0]) and held[0][1:2] == held[1][1:2] and held[0][0].shape[0] == 7
     assert held[0][2] == held[1][2]
 
