@@ -118,11 +118,6 @@ class _Growable:
         _lib.let_go(self.data)                                 # (copied from on this stream, and written to by queued encodes)
         self.data, self.row = data, math.prod(data.shape[1:])
 
-    @property
-    def address(self) -> int:
-        """Of `data`; asked for every time, since a copy of this object holds memory of its own."""
-        return self.data.data_ptr()
-
     def append(self, t: torch.Tensor):
         n = t.shape[0]
         # room for a quarter more than is needed: re-allocation stays rare while decoding appends small pieces, and a

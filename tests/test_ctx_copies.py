@@ -14,18 +14,31 @@ def _config():
     KVCompCacheConfigStatic.config = KVCompCacheConfig("t", QuantMode.ChannelQuant, QuantMode.TokenQuant, 64, 128, 64, 128, 0.1, 0.2)
 
 
-@pytest.mark.parametrize("how", [copy.deepcopy, lambda x: pickle.loads(pickle.dumps(x))])
-def test_a_copy_refers_to_its_own_memory(how):
+# a context's arrays and the descriptor's fields for them, which are what the kernels get
+ARRAYS = {"_encoded": "d_encoded", "_block_infos": "d_block_infos", "_thread_infos": "d_thread_infos", "_min_ints": "d_quant_min_ints",
+          "_scales": "d_quant_scales_f16"}
+
+
+def _filled():
+    """A context with a block of 64 tokens, 128 groups."""
     _config()
     ctx = KVCompCtx(True, 1, 2, 64, 0.1)
-    for g in (ctx._encoded, ctx._block_infos, ctx._thread_infos, ctx._min_ints, ctx._scales):
-        g.append(torch.arange(40, dtype=torch.uint8))
+    for name in ARRAYS:
+        getattr(ctx, name).append(torch.arange(128, dtype=torch.uint8))
     ctx.decode_codebook = ctx._lut_source = torch.zeros(6, dtype=torch.uint8)
     ctx._lut = torch.zeros(4)
+    ctx.compressed_ctx_len = ctx.ctx_len = 64
+    return ctx
+
+
+@pytest.mark.parametrize("how", [copy.deepcopy, lambda x: pickle.loads(pickle.dumps(x))])
+def test_a_copy_refers_to_its_own_memory(how):
+    ctx = _filled()
     got = how(ctx)
-    for name in ("_encoded", "_block_infos", "_thread_infos", "_min_ints", "_scales"):
+    for name, field in ARRAYS.items():
         mine, theirs = getattr(got, name), getattr(ctx, name)
-        assert torch.equal(mine.view, theirs.view) and mine.address == mine.data.data_ptr() != theirs.address
+        assert torch.equal(mine.view, theirs.view) and getattr(got.descriptor(), field) == mine.data.data_ptr() != getattr(ctx.descriptor(), field)
+    assert got.descriptor().d_luts == got._lut.data_ptr() != ctx.descriptor().d_luts
     assert got._descriptor is not ctx._descriptor
     assert got._lut_source is got.decode_codebook            # the copy's tables still belong to its codebook
 
@@ -68,11 +81,11 @@ def test_every_call_has_a_descriptor_of_its_own():
 
 
 def test_moved_data_is_seen():
-    _config()
-    g = KVCompCtx(False, 1, 2, 64, 0.2)._encoded
-    g.append(torch.zeros(8, dtype=torch.uint8))
-    g.data = g.data.clone()
-    assert g.address == g.data.data_ptr()
+    ctx = _filled()
+    for name, field in ARRAYS.items():
+        before, array = getattr(ctx.descriptor(), field), getattr(ctx, name)
+        array.data = array.data.clone()
+        assert getattr(ctx.descriptor(), field) == array.data.data_ptr() != before
 
 
 def test_dense_caches_can_be_copied():

@@ -336,13 +336,13 @@ def test_a_context_of_one_stream_grows_on_another_with_stores_outstanding(is_k):
     got.encoded_data
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.default_stream())
-    growing, addresses, sizes = got._encoded, [got._encoded.address], [got._encoded.data.numel()]
+    growing, addresses, sizes = got._encoded, [got._encoded.data.data_ptr()], [got._encoded.data.numel()]
     with torch.cuda.stream(side):
         end = _busy(side, 1.0)
         for part in parts[1:]:
             got.store(part, want_symbols=False)
-            if growing.address != addresses[-1]:
-                addresses.append(growing.address)
+            if growing.data.data_ptr() != addresses[-1]:
+                addresses.append(growing.data.data_ptr())
                 sizes.append(growing.data.numel())
         assert len(addresses) > 2 and not end.query() and len(got._unverified) > 2 and got.waits == 2     # (the codebook, encoded_data)
     other = [torch.full((n,), 0xA5, dtype=torch.uint8, device=DEV) for n in sizes]
