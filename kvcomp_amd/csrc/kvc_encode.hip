@@ -118,11 +118,11 @@ __device__ __forceinline__ void kvc_encode_init(const KvcEncodeArgs &a)
 }
 __global__ void __launch_bounds__(KVC_WAVE) kvc_encode_init_kernel(KvcEncodeArgs a) { kvc_encode_init(a); }
 
-// Hands the call's outcome to the caller's words (see kvc_encode_job), behind everything else: by the first ten threads of a
+// Hands the call's outcome to the caller's words (see kvc_encode_job), behind everything else: by the first nine threads of a
 // workgroup, a word each -- one after the other, the round trips to the host's memory took 4 us.
-__device__ __forceinline__ void kvc_encode_publish(const KvcEncodeArgs &a, int tid)
+__device__ __forceinline__ void kvc_encode_results(const KvcEncodeArgs &a, int tid)
 {
-    if (tid >= 10) return;                                     // (word 9 of the outcome is the call's number)
+    if (tid >= 9) return;
     const uint32_t total = a.status[0], err = a.status[1], first = a.status[KVC_ENC_ST_BASE];
     uint32_t word = 0;
     if (a.result && tid < 8) {
@@ -134,10 +134,16 @@ __device__ __forceinline__ void kvc_encode_publish(const KvcEncodeArgs &a, int t
         word = err ? *a.stream_bytes : first - a.base_global_offset + total;
         *a.stream_bytes = word;
     }
+    // the host looks at these words without asking the runtime; a copy and an event behind the call cost 8 us of host time and a launch
+    if (a.outcome) __hip_atomic_store(&a.outcome[tid], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// ... and, in word 9, that they are there: system-scope stores, then the call's number with release order (as
+// kvc_counts_to_host_kernel).
+__device__ __forceinline__ void kvc_encode_publish(const KvcEncodeArgs &a, int tid)
+{
+    if (tid >= 10) return;
+    kvc_encode_results(a, tid);
     if (a.outcome) {
-        // the host looks at these words without asking the runtime: system-scope stores, then the call's number with release
-        // order (as kvc_counts_to_host_kernel); a copy and an event behind the call cost 8 us of host time and a launch
-        if (tid < 9) __hip_atomic_store(&a.outcome[tid], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         __threadfence_system();
         __builtin_amdgcn_wave_barrier();
         if (tid == 9) __hip_atomic_store(&a.outcome[9], a.outcome_number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1935,7 +1941,8 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
 // every tile: nothing in it waits for another workgroup, so it always ends, and since the inputs are untouched the
 // outputs are the ones the call was to produce.  Slow (four waves for all tiles), and next to never needed: the
 // look-back's progress does not depend on the order in which the hardware starts workgroups.
-// What is left to the caller is kvc_encode_publish, by the threads of wave 0, which wrote what it reads or are ordered behind it.
+// What is left to the caller is kvc_encode_publish or kvc_encode_results, by the threads of wave 0, which wrote what these read or are
+// ordered behind it.
 template <int FRONT>
 __device__ __forceinline__ void kvc_encode_finish(const KvcStoreArgs &a)
 {
@@ -2073,11 +2080,12 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_kernel(KvcStoreArgs 
 }
 
 // ... and, by a second workgroup beside it, a first store's codebook to where it is kept and its decode tables
-// (kvc_put_codebook).  Whoever sees the call's number relies on both, on whatever stream: each workgroup makes what it wrote
-// visible (every wave its own stores, to the whole system) and counts itself done, and the one that is second publishes.  Neither
-// waits for the other.  The encoder has its codes in the argument block, so between the counts' arrival and the encoder nothing is
-// left but the launch, where this took a launch of its own in front of it: K and V of 8 heads x 777 tokens 246 -> 234 us, 8 x 32 x 128 x
-// 4096 370 -> 363.
+// (kvc_put_codebook).  Whoever sees the call's number relies on both, on whatever stream, so the workgroup that is done second
+// stores it; neither waits for the other.  A workgroup is done when all its waves' stores have reached the L2 that they share and
+// its first wave has had that written back for the whole system.  (Fences by every wave, and the results written by whichever
+// workgroup is second: 9.2 to 10.5 us for these 6.9 to 8.2; in no order at all 5.6 to 7.0.)
+// The encoder has its codes in the argument block, so between the counts' arrival and the encoder nothing is left but the launch, where
+// this took a launch of its own in front of it: K and V of 8 heads x 777 tokens 246 -> 234 us, 8 x 32 x 128 x 4096 370 -> 363.
 struct KvcPutSmallArgs {
     uint32_t words[80];            // table, padded to 16 bytes, and tree
     uint8_t *dst;
@@ -2086,7 +2094,6 @@ struct KvcPutSmallArgs {
 };
 __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_put_kernel(KvcStoreArgs a, KvcPutSmallArgs p)
 {
-    __shared__ uint32_t s_done;
     if (blockIdx.x == 0) {
         kvc_encode_finish<0>(a);
     } else {
@@ -2094,13 +2101,13 @@ __global__ void __launch_bounds__(KVC_WG) kvc_encode_finish_put_kernel(KvcStoreA
         for (int i = threadIdx.x; i < p.bytes; i += KVC_WG) p.dst[i] = src[i];
         kvc_build_lut_body(src + p.tree_at, p.bytes - p.tree_at, p.node_bytes, p.lut);
     }
-    __threadfence_system();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // (this wave's stores)
     __syncthreads();
-    if (threadIdx.x == 0) s_done = atomicAdd(&a.e.status[KVC_ONCE_DONE_WORD], 1u);
-    __syncthreads();
-    if (s_done == 0u) return;
-    __threadfence();                                       // (what the other workgroup has written is read from memory)
-    kvc_encode_publish(a.e, threadIdx.x);
+    if (threadIdx.x >= KVC_WAVE) return;
+    if (blockIdx.x == 0) kvc_encode_results(a.e, threadIdx.x);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    if (threadIdx.x == 0 && atomicAdd(&a.e.status[KVC_ONCE_DONE_WORD], 1u) == 1u && a.e.outcome)
+        __hip_atomic_store(&a.e.outcome[9], a.e.outcome_number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // What the fused path adds to an encode call: the fp16 source and how to quantize it.
