@@ -2315,9 +2315,9 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         if (c.packed) {
             // Two symbols a byte: the run that takes least, of those whose images fit beside each other (V: beside the last tile's
             // staging area).  A round of the waves takes as long as a run's tiles and the look-back, 1.2 tiles' worth.  K by two, three
-            // and four tiles, us: 4 x 32 heads x 64 x 32 768 tokens (65 536 tiles) 154, 143, 124; 4 x 24 x 72 x 16 384 (24 576) 67, 59, 63;
-            // 8 x 32 x 64 x 4160 (16 640) 52, 46, 49; 4 x 32 x 96 x 32 768 184 and 170; 8 x 32 x 128 x 4096 (16 384) 56 and 60.
-            // V, 8 x 32 x 96 x 4160 (12 480): 46 by four, 41 by three.
+            // and four tiles, us: 4 x 32 heads x 64 x 32 768 tokens (65 536 tiles) 148, 133, 113; 4 x 24 x 72 x 16 384 (24 576) 65, 56, 59;
+            // 8 x 32 x 64 x 4160 (16 640) 50, 44, 48; 4 x 32 x 96 x 32 768 172 and 160 (four do not fit).  V: 8 x 32 x 96 x 4160
+            // (12 480) 47, 39, 43; 4 x 32 x 96 x 32 768 (49 152) 141, 126, 119; 8 x 32 x 128 x 4096 (16 384) 53, 60, 47.
             auto cost = [&](int r) { return (a.tiles + (int64_t)KVC_WIDE_WAVES * r - 1) / ((int64_t)KVC_WIDE_WAVES * r) * (5 * r + 6); };
             for (int r = 3; r <= 4 && small && run >= 2 && want == 1; r++)
                 if ((is_k ? r * image <= sa.e.wave_bytes : (r - 1) * image <= sa.e.wave_bytes - KVC_STAGE_VPACKED_BYTES) && cost(r) <= cost(run)) run = r;

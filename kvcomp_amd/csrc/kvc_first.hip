@@ -12,7 +12,7 @@
 // The device has nothing to do from the counts' arrival to the encoder's launch, so the host does only what needs the code
 // in between: everything else (buffers, the encoder's status words and marks) is queued while the quantizer runs.  First
 // stores of K and V with 32 heads x 128 channels, 8 x 4096 tokens: 579 -> 491 us; 8 heads x 777 tokens: 320 -> 241 us.
-// (Today 350 and 229 us, 4 x 32 x 96 x 32 768 tokens 812: the encoder reads the codes from its argument block, so that the codebook need not
+// (Today 346 and 205 us, 4 x 32 x 96 x 32 768 tokens 810: the encoder reads the codes from its argument block, so that the codebook need not
 // be on the device before it, and the symbols go two to a byte; between the counts' arrival and the encoder the device idles 26 - 38 us.)
 #include "kvc_common.h"
 

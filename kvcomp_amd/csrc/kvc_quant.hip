@@ -766,7 +766,10 @@ extern "C" int kvc_quant(const void *d_x_f16, int64_t NB, int64_t BS, int64_t B,
 
 // The layouts whose symbols go two to a byte on their way to the encoder: the error bound gives at most 16 of them (a group's range is 1 / eb
 // steps, whose two ends may round outwards; scales among fp16's smallest numbers can give more, which the counts then say),
-// vectors have a length that the encoder's kernel for them is compiled for, and a quantizer that counts writes them.
+// vectors have a length that the encoder's kernel for them is compiled for, and a quantizer that counts writes them.  K's lengths
+// are those that kvc_encode_symbols_kernel is compiled for with a byte per symbol too; others (80, 112: a store of 4 x 32 heads x 4096
+// tokens takes 143 and 158 us, 128 a byte each 147) would take the same kernels, two more each, and have not been measured so.  V's
+// groups of one vector are shorter than the quantizer that counts rows takes.
 extern "C" int kvc_packed_symbols_supported(int is_k, int quant_mask, int64_t batch, int64_t heads, int64_t head_dim, float eb)
 {
     if (batch <= 0 || heads <= 0 || head_dim <= 0 || !(eb >= 1.0f / 13.0f)) return 0;

@@ -6,7 +6,7 @@
 // takes: the callers' own code decides then.  Below 0: what the library returned.  What only Python knows (tangents being carried
 // along, a trace being taken) the callers ask first.  The library is called without the interpreter's lock: a launch waits while its
 // stream's queue is full (some 2700 appends behind a kernel that runs on), and Python's other threads run on meanwhile.
-// A one-token append of the simulated cache takes the host 9.2 us with it (13.2 without), one of a context 5.4 (6.6), launches included.
+// A one-token append of the simulated cache takes the host 8.6 us with it (13.2 without), one of a context 5.0 (6.6), launches included.
 //
 //   append_dense(k, v, cos, sin, k_cache, v_cache, at)   kvc_append_dense
 //   append_rows(tail, at, rows, row_bytes)               kvc_copy_rows of all of `rows` to `at` rows into `tail`
