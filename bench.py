@@ -742,8 +742,9 @@ def main():
     # template arguments: query heads per KV head, then 0 = K tile, 3 / 4 = V tile with the softmax on the fly
     # (4: head_dim is not a multiple of 64, tiles may straddle two heads), then rounded mode
     v_kind = 3 if D % 64 == 0 else 4
-    # (codes of more than 7 bits: the last template argument)
-    name = lambda kind, ctx: "kvc_fused_mfma_kernel<%d, %d, true, %s>" % (rep, kind, "true" if ctx.max_code_bits > 7 else "false")
+    # (the last template argument: 2 codes of more than 7 bits, 1 codes of 6 or 7 bits of symbols up to 16, one per look-up)
+    book = lambda kind, ctx: 2 if ctx.max_code_bits > 7 else 1 if ctx.max_code_bits >= 6 and ctx.code_hint & 0x200 and not (kind and ctx.pair_bits) else 0
+    name = lambda kind, ctx: "kvc_fused_mfma_kernel<%d, %d, true, %d>" % (rep, kind, book(kind, ctx))
     dom, dom_ms, dom_bytes = ((name(0, kctx), k_ms, kb) if k_ms >= v_ms else (name(v_kind, vctx), v_ms, vb))
     achieved = dom_bytes / dom_ms / 1e6
     value = (kb + vb) / (ms_per_step * 1e-3) / 1e9

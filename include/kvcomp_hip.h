@@ -335,7 +335,8 @@ int kvc_v_decode_and_mat_vec_mul(const uint8_t *d_decode_tree, int64_t decode_tr
  *                        0 = unknown.  They only size the LDS staging; tiles that exceed them are decoded
  *                        from global memory.
  *     max_code_bits:     longest code of the codebook(s), 0 = unknown; + 256 where every symbol lies below 64 (codes
- *                        longer than 7 bits then take the matrix-core kernels too); + 4096 * kvc_codebook::pair_bits
+ *                        longer than 7 bits then take the matrix-core kernels too); + 512 where none lies above 16 (codes
+ *                        of 6 or 7 bits then take a faster loop); + 4096 * kvc_codebook::pair_bits
  *                        where it is known (V is then decoded two symbols at a time).  It only sizes the table kept in LDS
  *                        (fewer bytes, more waves per CU); a codebook with longer codes than stated still
  *                        decodes correctly, on the slow path. */

@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP
     if (active) {
         const KvcFusedArgs &a = is_k ? j.k : j.v;
         uint32_t first, longest;
-        st = kvc_stage_payload(a, lane, raw, pack, first, longest);
+        st = kvc_stage_payload<true>(a, lane, raw, pack, first, longest);
         if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;               // one or two bits before the lane's first code
         if (is_k) {
             const KvcTablePlan plan = {0, 1, 0};
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP
                 if (n_main) kvc_mfma_pair_dot<3, false, NM, true, true, true>(sbase, u, fe_k, mask, n_main, bptr, msptr, acc, true);
                 kvc_mfma_pair_dot<2, false, NM, true, true, true>(sbase, u, fe_k, mask, D - n_main, bptr, msptr, acc, true);
             } else {
-                kvc_mfma_dot<4, false, NM, true, true, false, true>(sbase, u, fe_k, mask, D, bptr, msptr, acc, true);
+                kvc_mfma_dot<4, false, NM, true, true, KVC_ENTRY_WORD, true>(sbase, u, fe_k, mask, D, bptr, msptr, acc, true);
             }
 #pragma unroll
             for (int q = 0; q < NM; q++) {

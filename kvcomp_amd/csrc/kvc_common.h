@@ -59,6 +59,8 @@ constexpr int KVC_LUT_ESC_BITS = 7, KVC_LUT_ESC_MAX = 64;
 constexpr int KVC_LUT_NARROW_OFFSET = KVC_LUT_ESC_OFFSET + 2 * KVC_LUT_ESC_MAX;
 constexpr int KVC_NARROW_LINE_WORDS = 16, KVC_NARROW_COUNTERS = 64;
 constexpr int KVC_LUT_NARROW_WORD = 6;
+// header word 6: some symbol is above 16 (see KVC_BYTE_CENTRE)
+constexpr uint32_t KVC_LUT_WIDE_SYMBOLS = 0x10000u;
 constexpr uint32_t KVC_LUT_NARROW_OFF = 0x80000000u;
 constexpr int KVC_LUT_WORDS = KVC_LUT_NARROW_OFFSET + KVC_NARROW_LINE_WORDS * KVC_NARROW_COUNTERS;
 constexpr int KVC_LUT_BYTES = KVC_LUT_WORDS * 4;          // 14880
@@ -97,6 +99,7 @@ struct KvcDecodeHints {
 // kvc_codebook::pair_bits
 static inline int kvc_hint_bits(int64_t hint) { return (int)(hint & 0xff); }
 static inline int kvc_hint_pair_bits(int64_t hint) { return (int)(hint >> 12 & 7); }
+static inline bool kvc_hint_byte_symbols(int64_t hint) { return (hint & 0x200) != 0; }      // none above 16
 static inline bool kvc_hint_small_alphabet(int64_t hint) { return (hint & 0x100) != 0; }
 int kvc_expand(int is_k, int deq, const uint8_t *d_decode_tree, int64_t decode_tree_bytes, int tree_format,
                const uint8_t *d_block_infos, int64_t block_infos_bytes, const uint8_t *d_thread_infos,

@@ -970,7 +970,8 @@ static void kvc_launch_fused(int kind, const KvcFusedArgs &a, dim3 grid, size_t 
 // from global memory, so the sizes only affect speed.  Everything stays within 64 KiB per workgroup.
 static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_bytes, int64_t tiles,
                            int64_t max_tile_bytes, int64_t max_stream_bytes, int max_code_bits, int64_t extra_words = 0,
-                           bool allow_pairs = true, int64_t mfma_ops_words = 0, int long_table_words = 0, int narrow_pair_bits = 0)
+                           bool allow_pairs = true, int64_t mfma_ops_words = 0, int long_table_words = 0, int narrow_pair_bits = 0,
+                           bool two_byte_table = false)
 {
     const int64_t slack = KVC_LDS_SLACK_WORDS + (long_table_words ? KVC_LDS_LONG_SLACK_WORDS : 0);
     const int force_rows = kvc_option(KVC_OPT_FUSED_ROWS);   // 0 / 1 overrides the choice below
@@ -998,6 +999,7 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
         a.table_words = (1 << (narrow_pair_bits > max_code_bits ? narrow_pair_bits : max_code_bits)) + (1 << max_code_bits);
         if (a.table_words < 8) a.table_words = 8;
     }
+    if (two_byte_table && a.pair_bits == 0 && a.narrow_pair_bits == 0) a.table_words = a.table_words > 8 ? a.table_words / 2 : 4;
     // per wave, besides the payload
     const int64_t ops_words = mfma_ops_words ? mfma_ops_words : (int64_t)slots * 128 * rep + extra_words;
     const int64_t budget = (65536 / 4 - a.table_words - slack) / KVC_WAVES_PER_WG - ops_words;   // words per wave
@@ -1197,9 +1199,12 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     const bool mfma = want_mfma != 0 && max_code_bits >= 1 && (!long_codes || (rounded && kvc_hint_small_alphabet(code_hint) && kind != 1 && kind != 2)) &&
                       kvc_option(KVC_OPT_FUSED_ROWS) != 1 && ((uintptr_t)d_out & 15) == 0 &&
                       (is_k ? out_stride % 4 == 0 : head_dim % 4 == 0);
+    // codes of 6 or 7 bits, symbols of at most 16, one per look-up: kernels of their own too
+    const bool mid_codes = mfma && rounded && !long_codes && max_code_bits >= 6 && kvc_hint_byte_symbols(code_hint) && kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0;
     const size_t lds = mfma ? kvc_plan_lds(a, slots, (int)rep, encoded_bytes, rows * a.s.cols, max_tile_bytes, max_stream_bytes,
                                            max_code_bits, 0, !long_codes, kvc_mfma_ops_words(slots, (int)rep, rounded),
-                                         long_codes ? KVC_LONG_TABLE_WORDS : 0, is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint))
+                                         long_codes ? KVC_LONG_TABLE_WORDS : 0, is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint),
+                                         mid_codes)
                             : kvc_plan_lds(a, slots, rounded ? (int)rep + 1 : (int)rep, encoded_bytes, rows * a.s.cols,
                                            max_tile_bytes, max_stream_bytes, max_code_bits, 0, !rounded);
     a.rounded = rounded;
@@ -1232,6 +1237,7 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     if (mfma) {
         if (trace_plan) fprintf(stderr, "[kvcomp]   matrix-core kernel\n");
         if (long_codes) kvc_launch_fused_long((int)rep, kind, a, grid, lds, stream);
+        else if (mid_codes && a.pair_bits == 0 && a.narrow_pair_bits == 0) kvc_launch_fused_mid((int)rep, kind, a, grid, lds, stream);
         else kvc_launch_fused_mfma((int)rep, kind, rounded != 0, a, grid, lds, stream);
         KVC_HIP(hipGetLastError());
         return timer.finish();

@@ -83,6 +83,11 @@ constexpr int kvc_fused_mfma_occupancy(int rep, int kind)
 }
 // the same for codebooks with codes of more than 7 bits (kvc_fused_mfma_long.hip)
 constexpr int kvc_fused_long_occupancy(int rep, int kind) { return rep == 1 ? (kind == 0 ? 7 : 6) : rep == 2 ? 5 : rep == 4 ? 4 : 1; }
+// the same for codes of 6 or 7 bits (kvc_fused_mfma_mid.hip)
+constexpr int kvc_fused_mid_occupancy(int rep, int kind)
+{
+    return rep == 1 ? (kind == 2 || kind == 4 ? 7 : 8) : rep == 4 && kind == 0 ? 6 : kvc_fused_occupancy(rep, kind);
+}
 constexpr int KVC_PRE_CHUNKS = 4;     // 16-byte chunks per lane fetched one tile ahead (4 KiB of payload)
 constexpr int KVC_PACK_LEAD = 4;      // zero words in front of the packed payload: bit positions never drop below 2
 
@@ -143,8 +148,14 @@ typedef __attribute__((address_space(3))) uint32_t kvc_lds_word;
 template <bool SKEW>
 __device__ __forceinline__ uint32_t kvc_refill_address(uint32_t stage_base, uint32_t u)
 {
-    const uint32_t a = u >> 5;
-    if (SKEW) return (a << 2) + (__umul24(u >> 10, 8u) + stage_base);     // + 2 words per 32
+    uint32_t a = u >> 5;
+    // (left to itself the compiler makes "u >> 3 & ~3" of the word's address: an instruction more, with the skew two)
+    asm("" : "+v"(a));
+    if (SKEW) {
+        uint32_t run = u >> 10;
+        asm("" : "+v"(run));
+        return (a << 2) + ((run << 3) + stage_base);                      // + 2 words per 32
+    }
     return (a << 2) + stage_base;
 }
 constexpr int KVC_LDS_SLACK_WORDS = 48;
@@ -481,7 +492,9 @@ struct KvcStaged {
 // Move a fetched tile's payload into the wave's packed LDS area (least-significant-bit-first words, skewed if asked
 // for) and work out where this lane's stream lies.  `first`: byte offset of the lane's stream in the packed area;
 // `longest`: with per-lane rows, the longest lane stream of the tile in words.  The caller finishes st.u0.
-template <class Raw>
+// ALIGNED: the packed area starts at a multiple of 16 bytes; unskewed, a chunk is then one 16-byte write (two of 8 bytes, which
+// leave every second pair of banks out, take twice as long).
+template <bool ALIGNED = false, class Raw>
 __device__ __forceinline__ KvcStaged kvc_stage_payload(const KvcFusedArgs &a, int lane, const Raw &raw, uint32_t *pack,
                                                        uint32_t &first_out, uint32_t &longest_out)
 {
@@ -529,6 +542,10 @@ __device__ __forceinline__ KvcStaged kvc_stage_payload(const KvcFusedArgs &a, in
             v.y = kvc_stream_word(v.y);
             v.z = kvc_stream_word(v.z);
             v.w = kvc_stream_word(v.w);
+            if (ALIGNED && !skew) {
+                *reinterpret_cast<uint4 *>(dstw) = v;
+                return;
+            }
             uint2 *dst = reinterpret_cast<uint2 *>(dstw);                            // 8-byte aligned either way
             dst[0] = make_uint2(v.x, v.y);
             dst[1] = make_uint2(v.z, v.w);
@@ -563,6 +580,8 @@ constexpr int kvc_mfma_ops_words(int slots, int rep, bool rounded)
 }
 // codes of more than 7 bits: 128 two-byte entries, then the list of those codes
 constexpr int KVC_LONG_TABLE_WORDS = (1 << KVC_LUT_ESC_BITS) / 2 + 2 * KVC_LUT_ESC_MAX;
+// rounded arithmetic only
+void kvc_launch_fused_mid(int rep, int kind, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);
 // kinds 0, 3 and 4, rounded arithmetic only
 void kvc_launch_fused_long(int rep, int kind, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);
 void kvc_launch_fused_mfma(int rep, int kind, bool rounded, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);

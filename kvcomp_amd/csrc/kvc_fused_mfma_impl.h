@@ -79,6 +79,9 @@ __device__ __forceinline__ kvc_w2 kvc_read_columns(uint32_t addr, bool holder)
 // btab  [slot][group g][set][column j][element k]  fp16: weight part of element 4 g + k for column 4 set + j;
 //       column 2 r is the high part of query head r's weight, column 2 r + 1 its low part times 4096
 // mstab [slot][group g] = {min 4g, min 4g+1 | min 4g+2, min 4g+3 | scale 4g, 4g+1 | scale 4g+2, 4g+3}  (rounded mode)
+// second bytes of two table entries, each in the upper byte of a half: {a & 0xff00, b & 0xff00}
+__device__ __forceinline__ uint32_t kvc_pack_byte1(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x050c010cu); }
+
 template <int REP>
 struct KvcMfmaTables {
     static constexpr int NM = kvc_mfma_sets(REP);
@@ -102,16 +105,17 @@ __device__ __forceinline__ void kvc_split_weight(float v, float &hi, float &lo)
 // Rounded mode: the minima of a lane's two elements as two fp16, and their two scales, in the order the decode loops read
 // them.  Where both elements' parameters came in one word each (wave-uniform `pmode`), the scales are that word and the
 // two int8 minima are converted together: the byte m ^ 0x80 = m + 128 under the byte 0x64 is the fp16 number 1152 + m.
+// `centre`: added to the minima (what the table's symbols are short of).
 template <class Raw>
-__device__ __forceinline__ void kvc_mfma_min_scale_words(const Raw &raw, int s, int pmode, uint32_t &mins, uint32_t &scales)
+__device__ __forceinline__ void kvc_mfma_min_scale_words(const Raw &raw, int s, int pmode, uint32_t &mins, uint32_t &scales, int centre = 0)
 {
     if (pmode == KVC_PAIR_ADJACENT) {
         const uint32_t biased = __builtin_amdgcn_perm(0x64u, raw.mnw[s][0] ^ 0x8080u, 0x04010400u);
-        const kvc_h2 off = {(_Float16)-1152.f, (_Float16)-1152.f};
-        mins = __builtin_bit_cast(uint32_t, __builtin_bit_cast(kvc_h2, biased) + off);                              // exact
+        const uint32_t off = centre ? 0xe478e478u : 0xe480e480u;                                                   // -1144 or -1152, twice
+        mins = __builtin_bit_cast(uint32_t, __builtin_bit_cast(kvc_h2, biased) + __builtin_bit_cast(kvc_h2, off));     // exact
         scales = raw.scw[s][0];
     } else {
-        mins = kvc_half_pair((float)raw.min_int(s, 0, pmode), (float)raw.min_int(s, 1, pmode));                    // exact
+        mins = kvc_half_pair((float)(raw.min_int(s, 0, pmode) + centre), (float)(raw.min_int(s, 1, pmode) + centre));  // exact
         scales = raw.scale_bits(s, 0, pmode) | (raw.scale_bits(s, 1, pmode) << 16);
     }
 }
@@ -190,7 +194,7 @@ template <int REP, int KIND, bool ROUNDED>
 __device__ __forceinline__ void kvc_mfma_stage_ops(const KvcFusedArgs &a, const KvcTilePos &pos, const KvcTablePlan &pl, int lane,
                                                    const KvcRaw<REP, KvcGeom<KIND>::SLOTS, KvcGeom<KIND>::XW> &raw,
                                                    uint32_t *btab, uint32_t *mstab, float (&bias)[REP], float &unscale,
-                                                   int &sel_out, KvcTableState &st)
+                                                   int &sel_out, KvcTableState &st, int centre = 0)
 {
     constexpr int SLOTS = KvcGeom<KIND>::SLOTS;
     constexpr int NM = kvc_mfma_sets(REP);
@@ -237,7 +241,7 @@ __device__ __forceinline__ void kvc_mfma_stage_ops(const KvcFusedArgs &a, const 
 #pragma unroll
                     for (int r = 0; r < REP; r++) bg[(((2 * r) >> 2) * 4 + ((2 * r) & 3)) * 2] = raw.x[s][r][0];
                     uint32_t *mg = mstab + ts * T::MSTAB_SLOT_WORDS + g * 4 + odd;
-                    kvc_mfma_min_scale_words(raw, s, pmode_of(s), mg[0], mg[2]);
+                    kvc_mfma_min_scale_words(raw, s, pmode_of(s), mg[0], mg[2], centre);
                 }
                 st.set_lo(ts, 0);
             }
@@ -322,7 +326,7 @@ __device__ __forceinline__ void kvc_mfma_stage_ops(const KvcFusedArgs &a, const 
             }
             if (ROUNDED) {
                 uint32_t *mg = mstab + ts * T::MSTAB_SLOT_WORDS + g * 4 + odd;
-                kvc_mfma_min_scale_words(raw, s, pmode_of(s), mg[0], mg[2]);
+                kvc_mfma_min_scale_words(raw, s, pmode_of(s), mg[0], mg[2], centre);
             }
         }
     }
@@ -339,12 +343,23 @@ __device__ __forceinline__ void kvc_mfma_stage_ops(const KvcFusedArgs &a, const 
 // word, which the LDS serves in one cycle (with four-byte entries a 64-entry table has two words per bank and 42 % of
 // its LDS cycles are bank conflicts).  Costs an instruction per two symbols (join and mask instead of a byte permute);
 // the lengths of a half window (at most 4 x 7 bits) are summed in five bits, above which symbol bits pile up.
-template <int G, bool SKEW, int NM, bool ROUNDED, bool BCAST, bool HALF = false, bool EVERY = false>
+// BYTE: two-byte entries {the symbol less 8 in fp16's upper byte | code length in the lower byte}, for symbols of at most 16 in
+// rounded mode (the minima are 8 larger): what is left of an fp16 number without its lower byte holds the integers from -8 to 8
+// exactly, so one byte permute joins two symbols and drops their lengths, and the lengths of a refill add up in their byte
+// without a mask.  8 symbols with codes of 6 or 7 bits: 52 -> 42 vector instructions.  With seven-bit codes it is then the LDS that
+// the loop waits for (a look-up among 64 words takes it 4.2 cycles, among 32 words 2.3), and the table's size that decides how
+// many workgroups a CU holds (20 736 bytes: seven, 20 480: eight).  8 x 32 heads x 128 x 4177 tokens K 43.0 -> 39.6, V 41.8 -> 38.0 us;
+// 4 x 32 x 96 x 32 768 (six bits) K 102.5 -> 91; 16 x 8 x 4 x 128 x 8192 K 43.2 -> 43.0, V 47.6 -> 47.0.
+enum { KVC_ENTRY_WORD = 0, KVC_ENTRY_HALF = 1, KVC_ENTRY_BYTE = 2 };
+constexpr int KVC_BYTE_CENTRE = 8;
+template <int G, bool SKEW, int NM, bool ROUNDED, bool BCAST, int FORM = KVC_ENTRY_WORD, bool EVERY = false>
 __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32_t fe, uint32_t mask4, int n,
                                              uint32_t &bptr, uint32_t &msptr, kvc_f4 (&acc)[NM], bool holder)
 {
     static_assert((2 * G) % 4 == 0, "whole groups of four per refill");
+    constexpr bool HALF = FORM == KVC_ENTRY_HALF, BYTE = FORM == KVC_ENTRY_BYTE;
     static_assert(!HALF || G <= 4, "the lengths of a half window must fit five bits");
+    static_assert(!BYTE || ROUNDED, "the symbols are short of eight, which the minima make up for");
     asm volatile("" : "+v"(msptr));      // kept in a vector register: one add per round instead of a move per read
     for (int i = 0; i < n; i += 2 * G) {
         const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
@@ -358,7 +373,7 @@ __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32
                 R = __builtin_amdgcn_alignbit(hi, lo, es);       // (shifts by the low five bits of es)
                 if (HALF) used1 = es & 31u, es = 0;
             }
-            if constexpr (HALF) e[g] = *(const kvc_lds_u16 *)(uintptr_t)((R & mask4) | fe);
+            if constexpr (HALF || BYTE) e[g] = *(const kvc_lds_u16 *)(uintptr_t)((R & mask4) | fe);
             else e[g] = *(const kvc_lds_u32 *)(uintptr_t)((R & mask4) | fe);
             if (g != G - 1 && g != 2 * G - 1) R = __builtin_amdgcn_alignbit(R, R, e[g]);
             es += e[g];
@@ -368,6 +383,9 @@ __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32
                 if constexpr (HALF) {
                     a01 = ((e[g - 2] << 16) | e[g - 3]) & 0xffe0ffe0u;
                     a23 = ((e[g] << 16) | e[g - 1]) & 0xffe0ffe0u;
+                } else if constexpr (BYTE) {
+                    a01 = kvc_pack_byte1(e[g - 3], e[g - 2]);
+                    a23 = kvc_pack_byte1(e[g - 1], e[g]);
                 } else {
                     a01 = kvc_pack_hi16(e[g - 3], e[g - 2]);
                     a23 = kvc_pack_hi16(e[g - 1], e[g]);
@@ -510,7 +528,7 @@ __device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, u
 template <int REP, bool GSRC, bool ROUNDED>
 __device__ __noinline__ KvcVec<REP> kvc_mfma_slow_tile(const uint32_t *words, uint32_t nwords, uint32_t pos,
                                                        const uint32_t *__restrict__ lut_g, int n, const uint32_t *btab,
-                                                       const uint32_t *mstab, uint32_t skew)
+                                                       const uint32_t *mstab, uint32_t skew, int centre = 0)
 {
     constexpr int NM = kvc_mfma_sets(REP);
     const uint32_t lshift = 32u - lut_g[0], nlong = lut_g[2];
@@ -543,7 +561,7 @@ __device__ __noinline__ KvcVec<REP> kvc_mfma_slow_tile(const uint32_t *words, ui
             }
         }
         const int g = i >> 2, k = i & 3;
-        float x = (float)sym;
+        float x = (float)((int)sym - centre);
         if (ROUNDED) {
             const uint32_t ms = (uint32_t)mh[g * 8 + k] | ((uint32_t)mh[g * 8 + 4 + k] << 16);
             x = kvc_rounded_value(__float2half_rn(x), ms);
@@ -566,12 +584,22 @@ __device__ __forceinline__ float kvc_quad_next(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xF5 /* quad_perm:[1,1,3,3] */, 0xf, 0xf, false));
 }
 
-// LONG: for codebooks with codes of more than 7 bits (kvc_mfma_dot_long), kernels of their own
-// (kvc_fused_mfma_long.hip): beside the other loops it would cost them registers.
-template <int REP, int KIND, bool ROUNDED, bool LONG = false>
-__global__ void __launch_bounds__(KVC_WG, LONG ? kvc_fused_long_occupancy(REP, KIND) : kvc_fused_mfma_occupancy(REP, KIND))
+// BOOK: what the codebooks' longest codes ask for.  Codes of 6 or 7 bits of symbols up to 16 (kvc_mfma_dot's BYTE) and codes
+// of more than 7 bits (kvc_mfma_dot_long) have kernels of their own (kvc_fused_mfma_mid.hip, kvc_fused_mfma_long.hip): beside
+// the other loops theirs would cost registers and spilled scalars (one query head, the former: K 14 -> 25 spilled scalars, the
+// plain V kernel seven waves per SIMD instead of eight).
+enum { KVC_BOOK_SHORT = 0, KVC_BOOK_MID = 1, KVC_BOOK_LONG = 2 };
+constexpr int kvc_fused_book_occupancy(int rep, int kind, int book)
+{
+    return book == KVC_BOOK_LONG ? kvc_fused_long_occupancy(rep, kind) : book == KVC_BOOK_MID ? kvc_fused_mid_occupancy(rep, kind)
+                                                                       : kvc_fused_mfma_occupancy(rep, kind);
+}
+template <int REP, int KIND, bool ROUNDED, int BOOK = KVC_BOOK_SHORT>
+__global__ void __launch_bounds__(KVC_WG, kvc_fused_book_occupancy(REP, KIND, BOOK))
 kvc_fused_mfma_kernel(KvcFusedArgs a_in)
 {
+    constexpr bool LONG = BOOK == KVC_BOOK_LONG, MID = BOOK == KVC_BOOK_MID;
+    static_assert(ROUNDED || BOOK == KVC_BOOK_SHORT, "kernels of the default arithmetic");
     const KvcFusedArgs &a = a_in;
     constexpr bool IS_K = KIND == 0;
     constexpr int SLOTS = KvcGeom<KIND>::SLOTS;
@@ -626,7 +654,8 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     const uint32_t nesc = LONG ? lut_g[7] : 0u;
     const bool fast_book = LONG ? lmax > (uint32_t)KVC_LUT_ESC_BITS && nesc <= (uint32_t)KVC_LUT_ESC_MAX &&
                                       (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u && a.table_words >= KVC_LONG_TABLE_WORDS
-                                : nlong == 0 && lmax >= 1u && lmax <= 7u && (1u << lbits) <= (uint32_t)a.table_words;
+                                : nlong == 0 && lmax >= 1u && lmax <= 7u && (1u << lbits) <= (uint32_t)a.table_words << (MID ? 1 : 0) &&
+                                      !(MID && (lut_g[6] & KVC_LUT_WIDE_SYMBOLS) != 0u);
     // one-symbol entries: the symbol as fp16 in the upper half, the code length (never beyond the index width, which
     // bounds how far a corrupt stream can run) in the lowest byte
     auto fentry = [&](uint32_t i) {
@@ -643,21 +672,22 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     // Batch 4 x 32 heads x 96 x 32 768 tokens, heavy-tailed data, 7 index bits for codes of up to 6: V 88 -> 74 us.  With 8
     // bits (three pairs per half window, 256 words) it measured no better than one symbol per look-up (38.6 / 39.8 us at
     // batch 8 x 32 x 128 x 4096), and K, which has no such codebooks, 8 % slower for the scalars spilled.
-    constexpr bool NARROW_OK = !IS_K && !LONG;
+    constexpr bool NARROW_OK = !IS_K && BOOK == KVC_BOOK_SHORT;
     const uint32_t one_at = (uint32_t)a.narrow_pair_bits > lbits ? (uint32_t)a.narrow_pair_bits : lbits;
     const bool narrow = NARROW_OK && fast_book && a.narrow_pair_bits != 0 && (uint32_t)a.narrow_pair_bits < 2u * lmax &&
                         (1u << one_at) + (1u << lbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
     const uint32_t pbits = narrow ? (uint32_t)a.narrow_pair_bits : 2u * lmax;
     // two symbols per look-up: twice the longest code fits the index, and no symbol's fp16 pattern needs the five
     // bits the lengths of a two-symbol entry go to (header word 6: OR of all the patterns)
-    const bool pairs = narrow || (!LONG && fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
+    const bool pairs = narrow || (BOOK == KVC_BOOK_SHORT && fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
                                  (1u << pbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u);
     // codes of 6 or 7 bits: two-byte entries (see kvc_mfma_dot), where no symbol's fp16 pattern needs its five lowest bits.
     // Not for V tiles that may straddle two heads: with that loop beside the others the kernel needs one register more
     // than six waves per SIMD leave it, and the compiler then spills in the per-tile path of every variant.
-    constexpr bool HALF_OK = SLOTS == 1 && !LONG;
+    constexpr bool HALF_OK = SLOTS == 1 && BOOK == KVC_BOOK_SHORT;
     const bool half_table = HALF_OK && fast_book && !pairs && lbits >= 6u && a.half_table != 0 && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
-    const uint32_t lead_bits = LONG || half_table ? 1u : 2u;                   // bits of the window below the table index
+    constexpr int centre = MID ? KVC_BYTE_CENTRE : 0;
+    const uint32_t lead_bits = LONG || MID || half_table ? 1u : 2u;                   // bits of the window below the table index
     if constexpr (LONG) {
         if (fast_book) {
             uint16_t *t16 = reinterpret_cast<uint16_t *>(smem);
@@ -691,6 +721,13 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
             smem[idx] = (e1 & 0xffff0000u) | (e0 >> 16) | ((e0 & 0xffu) + (e1 & 0xffu));
         }
         __syncthreads();
+    } else if (MID) {
+        uint16_t *t16 = reinterpret_cast<uint16_t *>(smem);
+        if (fast_book) for (uint32_t i = tid; i < (1u << lbits); i += KVC_WG) {
+            const uint32_t e = lut_g[KVC_LUT_FENTRY_OFFSET + i];
+            const uint32_t len = (e & 0xffu) > lbits ? lbits : (e & 0xffu);
+            t16[i] = (uint16_t)(__half_as_ushort(__float2half_rn(__uint_as_float(e & 0xffffff00u) - (float)KVC_BYTE_CENTRE)) | len);
+        }
     } else if (half_table) {
         uint16_t *t16 = reinterpret_cast<uint16_t *>(smem);
         for (uint32_t i = tid; i < (1u << lbits); i += KVC_WG) {
@@ -740,9 +777,9 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     float bias[REP], unscale;
     int sel = 0;
     uint32_t first, longest;
-    KvcStaged st = kvc_stage_payload(a, lane, raw, pack, first, longest);
+    KvcStaged st = kvc_stage_payload<true>(a, lane, raw, pack, first, longest);
     if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;       // one or two bits before the lane's first code
-    kvc_mfma_stage_ops<REP, KIND, ROUNDED>(a, pos, plan, lane, raw, btab, mstab, bias, unscale, sel, tabs);
+    kvc_mfma_stage_ops<REP, KIND, ROUNDED>(a, pos, plan, lane, raw, btab, mstab, bias, unscale, sel, tabs, centre);
     kvc_wave_sync();
     for (int it = 0; it < ntiles; it++) {
         // the arguments are read again per tile rather than kept in scalar registers through the decode loops (the
@@ -800,12 +837,13 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
                     else kvc_mfma_pair_dot<3, SK, NM, ROUNDED, BCAST, EV>(sbase, u, fe, maskp, n_main, bptr, msptr, acc, holder);
                     if (n - n_main) kvc_mfma_pair_dot<2, SK, NM, ROUNDED, BCAST, EV>(sbase, u, fe, maskp, n - n_main, bptr, msptr, acc, holder);
                 } else {
-                    if (!whole && per == 16) kvc_mfma_dot<8, SK, NM, ROUNDED, BCAST, false, EV>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
-                    else if (!whole && per == 12) kvc_mfma_dot<6, SK, NM, ROUNDED, BCAST, false, EV>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
-                    const int rest = whole || per == 8 ? n : n - n_main;
+                    if (!MID && !whole && per == 16) kvc_mfma_dot<8, SK, NM, ROUNDED, BCAST, KVC_ENTRY_WORD, EV>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
+                    else if (!MID && !whole && per == 12) kvc_mfma_dot<6, SK, NM, ROUNDED, BCAST, KVC_ENTRY_WORD, EV>(sbase, u, fe, mask4, n_main, bptr, msptr, acc, holder);
+                    const int rest = MID || whole || per == 8 ? n : n - n_main;
                     const uint32_t tab = whole ? fe + (4u << one_at) : fe;
-                    if (HALF_OK && rest && half_table) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, HALF_OK, EV>(sbase, u, fe, mask4, rest, bptr, msptr, acc, holder);
-                    else if (rest) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, false, EV>(sbase, u, tab, mask4, rest, bptr, msptr, acc, holder);
+                    if (MID) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, MID ? KVC_ENTRY_BYTE : KVC_ENTRY_WORD, EV>(sbase, u, fe, mask4, rest, bptr, msptr, acc, holder);
+                    else if (HALF_OK && rest && half_table) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, HALF_OK ? KVC_ENTRY_HALF : KVC_ENTRY_WORD, EV>(sbase, u, fe, mask4, rest, bptr, msptr, acc, holder);
+                    else if (rest) kvc_mfma_dot<4, SK, NM, ROUNDED, BCAST, KVC_ENTRY_WORD, EV>(sbase, u, tab, mask4, rest, bptr, msptr, acc, holder);
                 }
             };
             for (int m = mode;; m = 1) {
@@ -858,9 +896,9 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
             KvcVec<REP> res;
             if (st.fits)
                 res = kvc_mfma_slow_tile<REP, false, ROUNDED>(pack, (uint32_t)a.pack_logical, st.u0 + lead_bits, lut_g, n, my_btab,
-                                                              my_mstab, (uint32_t)a.skew);
+                                                              my_mstab, (uint32_t)a.skew, centre);
             else
-                res = kvc_mfma_slow_tile<REP, true, ROUNDED>(st.gwords, st.gnwords, st.gpos, lut_g, n, my_btab, my_mstab, 0u);
+                res = kvc_mfma_slow_tile<REP, true, ROUNDED>(st.gwords, st.gnwords, st.gpos, lut_g, n, my_btab, my_mstab, 0u, centre);
             // here a lane holds the results of its own row; in a V tile every lane's head slot is its block's
             int lane_o = lane;
             if constexpr (REP == 1) asm volatile("" : "+v"(lane_o));
@@ -876,10 +914,10 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
             kvc_wave_sync();     // every lane is done reading this tile's LDS data
             int lane_s = lane;
             asm volatile("" : "+v"(lane_s));
-            st = kvc_stage_payload(a, lane_s, raw, pack, first, longest);
+            st = kvc_stage_payload<true>(a, lane_s, raw, pack, first, longest);
             if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;
             late_params(a, pos_next, plan_next, lane_s);
-            kvc_mfma_stage_ops<REP, KIND, ROUNDED>(a, pos_next, plan_next, lane_s, raw, btab, mstab, bias, unscale, sel, tabs);
+            kvc_mfma_stage_ops<REP, KIND, ROUNDED>(a, pos_next, plan_next, lane_s, raw, btab, mstab, bias, unscale, sel, tabs, centre);
             kvc_wave_sync();
         }
         pos = pos_next;

@@ -5,9 +5,9 @@
 template <int REP>
 static void kvc_launch_long_kind(int kind, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream)
 {
-    if (kind == 0) hipLaunchKernelGGL((kvc_fused_mfma_kernel<REP, 0, true, true>), grid, dim3(KVC_WG), lds, stream, a);
-    else if (kind == 3) hipLaunchKernelGGL((kvc_fused_mfma_kernel<REP, 3, true, true>), grid, dim3(KVC_WG), lds, stream, a);
-    else hipLaunchKernelGGL((kvc_fused_mfma_kernel<REP, 4, true, true>), grid, dim3(KVC_WG), lds, stream, a);
+    if (kind == 0) hipLaunchKernelGGL((kvc_fused_mfma_kernel<REP, 0, true, KVC_BOOK_LONG>), grid, dim3(KVC_WG), lds, stream, a);
+    else if (kind == 3) hipLaunchKernelGGL((kvc_fused_mfma_kernel<REP, 3, true, KVC_BOOK_LONG>), grid, dim3(KVC_WG), lds, stream, a);
+    else hipLaunchKernelGGL((kvc_fused_mfma_kernel<REP, 4, true, KVC_BOOK_LONG>), grid, dim3(KVC_WG), lds, stream, a);
 }
 
 void kvc_launch_fused_long(int rep, int kind, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream)

@@ -78,7 +78,8 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
                 my_code[k] = code;
                 atomicMax(&s_lmax, len);
                 atomicAdd(&s_avg, (float)len * exp2f(-(float)len));
-                atomicOr(&s_symbits, (uint32_t)__half_as_ushort(__float2half_rn((float)(s_child[0][n] & 0xff))));
+                const int sym = s_child[0][n] & 0xff;
+                atomicOr(&s_symbits, (uint32_t)__half_as_ushort(__float2half_rn((float)sym)) | (sym > 16 ? KVC_LUT_WIDE_SYMBOLS : 0u));
             }
         }
     }
@@ -144,7 +145,7 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
         // enough for the window to overflow rarely (lut[5] = 1: the kernel checks and falls back)
         lut[4] = (lmax <= 3 || roomy8) ? 8u : lmax <= 7 ? 30u / lmax : roomy ? 4u : 2u;
         lut[5] = (roomy8 || (lmax > 7 && roomy)) ? 1u : 0u;
-        lut[6] = s_symbits;       // low bits clear in every symbol's fp16 pattern: room for lengths in a packed entry
+        lut[6] = s_symbits;       // low bits clear in every symbol's fp16 pattern: room for lengths in a packed entry; KVC_LUT_WIDE_SYMBOLS
         lut[7] = s_nesc;
     }
 }
