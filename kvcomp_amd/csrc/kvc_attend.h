@@ -9,10 +9,20 @@
 //   4 query heads   1536            36.8 : 34.8 / 30.4 : 28.6    2048 41.3 : 40.5 / 32.4 : 31.9    3072 58.5 : 58.0 / 41.2 : 45.4
 //   8 query heads   2048            70.5 : 48.6 / 47.0 : 37.7    3072 81.8 : 72.0 / 54.8 : 53.8
 constexpr int64_t kvc_attend_max_wgs(int64_t rep) { return rep <= 2 ? 1536 : rep == 4 ? 2048 : 3072; }
+// ... and from which a wave takes a group by itself (head_dim 128, codes of 6 or 7 bits of symbols up to 16).  Two kernels, the joint
+// kernel and this one in us, per decode attention call:
+//   1 query head    1536 groups 28 : 29 : 30    2048 31.5 : 31.9 : 31.2    4096 49.7 : 55.6 : 43.1    8192  79 : 94 : 71
+//   4 query heads   1536        34 : 33 : 34    2048 38.2 : 38.1 : 35.1    4096 61.1 : 65.8 : 48.9    8192  96 : 118 : 81
+//   8 query heads   1536        46 : 42 : 42    2048 61.1 : 48.4 : 43.8    4096 98.2 : 85.1 : 71.9    8192 161 : 155 : 112
+constexpr int64_t KVC_ATTEND_WAVES_MIN_WGS = 1536;
 constexpr int KVC_ATTEND_K_PAIR_BITS = 6;         // longest code for which K's table of two symbols per look-up is built
 
 // Partials [groups, B * Hq, D] and their (maximum, sum of weights) of all whole groups of 128 tokens that V holds compressed,
 // and the scores of the tokens that only K does.  *taken: false where the call is not one for it (nothing launched).
+struct KvcFusedArgs;
+// (k, v: filled by kvc_attend_groups) the same for larger caches, kvc_attend_waves.hip
+int kvc_attend_waves(const KvcFusedArgs &k, const KvcFusedArgs &v, const kvc_compressed_desc *kd, const kvc_compressed_desc *vd, int64_t rep, int64_t bh,
+                     hipStream_t stream, bool *taken);
 int kvc_attend_groups(const kvc_compressed_desc *k, const kvc_compressed_desc *v, const void *d_q_f16, float softmax_scale,
                       float *scores, int64_t scores_stride, float *part, float *ml, int64_t batch, int64_t kv_heads, int64_t q_heads,
                       int64_t head_dim, hipStream_t stream, bool *taken);

@@ -404,7 +404,11 @@ int kvc_attend_groups(const kvc_compressed_desc *k, const kvc_compressed_desc *v
     const int64_t groups = v->tokens / KVC_V_TOKENS, wgs = groups * bh;
     const int64_t k_tiles = k->tokens / KVC_WAVE * bh, k_rest = k_tiles - wgs * KVC_ATTEND_K_TILES;
     if (k_tiles > (int64_t)1 << 30) return 0;
-    if (want < 0 && wgs > kvc_attend_max_wgs(rep)) return 0;
+    // beyond, a wave per group (kvc_attend_waves.hip) where both codebooks are its
+    const bool by_waves = want != 1 && (want > 1 || wgs > KVC_ATTEND_WAVES_MIN_WGS) && head_dim == 2 * KVC_WAVE && kb >= 6 && vb >= 6 &&
+                          kvc_hint_byte_symbols(k->max_code_bits) && kvc_hint_byte_symbols(v->max_code_bits) && kvc_hint_pair_bits(v->max_code_bits) == 0 &&
+                          kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0;
+    if (!by_waves && (want > 1 || (want < 0 && wgs > kvc_attend_max_wgs(rep)))) return 0;
     KvcAttendArgs j = {};
     if (int rc = kvc_attend_fill(j.k, k, 1, batch, kv_heads, q_heads, head_dim)) return rc;
     if (int rc = kvc_attend_fill(j.v, v, 0, batch, kv_heads, q_heads, head_dim)) return rc;
@@ -414,6 +418,7 @@ int kvc_attend_groups(const kvc_compressed_desc *k, const kvc_compressed_desc *v
     j.v.out = part;
     j.v.ml = ml;
     j.v.sm_scale = softmax_scale;
+    if (by_waves) return kvc_attend_waves(j.k, j.v, k, v, rep, bh, stream, taken);
     j.k_bits = kb;
     j.v_bits = vb;
     j.group_wgs = (int)wgs;

@@ -1018,13 +1018,7 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
     // payload).  The skewed layout cures that at the cost of 1/16 more LDS and two instructions per refill;
     // per-lane rows (an odd number of words apart) cure it too, but double the LDS a tile needs and cost a
     // copy, so they are only used when asked for.
-    const double mean_stream_words = (double)encoded_bytes / (double)(tiles > 0 ? tiles : 1) / KVC_WAVE / 4.0;
-    bool resonant = false;
-    for (int k = 1; k <= 4; k++) {
-        const double x = k * mean_stream_words / 32.0;
-        const double dist = (x - (double)(int64_t)(x + 0.5)) * 32.0;
-        if (x >= 0.5 && dist > -1.0 && dist < 1.0) resonant = true;
-    }
+    const bool resonant = kvc_streams_resonate(encoded_bytes, tiles);
     const bool use_rows = force_rows == 1 && pack_rows + KVC_WAVE * row <= budget;
     const int force_skew = kvc_option(KVC_OPT_FUSED_SKEW);
     const bool use_skew = !use_rows && (force_skew >= 0 ? force_skew != 0 : resonant);

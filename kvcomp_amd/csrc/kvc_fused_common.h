@@ -141,6 +141,19 @@ __device__ __forceinline__ uint32_t kvc_stream_word(uint32_t raw) { return __bre
 //   word w of the payload lives at w + skew * (w >> 5), skew = 2 (or 0: plain layout)
 __device__ __forceinline__ uint32_t kvc_skewed(uint32_t w, uint32_t skew) { return __umul24(w >> 5, skew) + w; }
 
+// Whether the lanes line up: a small multiple of the mean stream length is close to a multiple of the 32 banks.
+static inline bool kvc_streams_resonate(int64_t encoded_bytes, int64_t tiles)
+{
+    const double mean_stream_words = (double)encoded_bytes / (double)(tiles > 0 ? tiles : 1) / KVC_WAVE / 4.0;
+    bool resonant = false;
+    for (int k = 1; k <= 4; k++) {
+        const double x = k * mean_stream_words / 32.0;
+        const double dist = (x - (double)(int64_t)(x + 0.5)) * 32.0;
+        if (x >= 0.5 && dist > -1.0 && dist < 1.0) resonant = true;
+    }
+    return resonant;
+}
+
 // Byte address in LDS of payload word u >> 5 for a refill.  No clamp: a lane's position cannot pass its start
 // by more than 128 symbols x 10 bits, and the workgroup's LDS ends with that much slack (KVC_LDS_SLACK_WORDS),
 // so even a corrupt stream only ever reads this workgroup's own LDS.
@@ -384,7 +397,8 @@ __device__ __forceinline__ void kvc_fetch_separate_params(const KvcFusedArgs &a,
 // `skip_x`: bit s set = the weights of head slot s are not needed (the wave still has that head's operand table).
 // LATE_SECOND: the separate-groups parameters of a tile's second head are left to the caller, who fetches them when the
 // tile is staged (kvc_fetch_separate_params): four registers less to hold through the previous tile's decode loops.
-template <int REP, int KIND, int EXPAND = 0, bool LATE_SECOND = false>
+// PAYLOAD = false: the operands only (the payload comes by kvc_fetch_streams).
+template <int REP, int KIND, int EXPAND = 0, bool LATE_SECOND = false, bool PAYLOAD = true>
 __device__ __forceinline__ void kvc_fetch_tile(const KvcFusedArgs &a, const KvcTilePos &pos, uint32_t bi_off, uint32_t bi_bn,
                                                int lane, KvcRaw<REP, KvcGeom<KIND>::SLOTS, KvcGeom<KIND>::XW> &raw, int skip_x = 0)
 {
@@ -399,7 +413,7 @@ __device__ __forceinline__ void kvc_fetch_tile(const KvcFusedArgs &a, const KvcT
     else if ((int64_t)off + bn > a.s.enc_bytes) bn = (uint32_t)(a.s.enc_bytes - off);
     raw.off = off;
     raw.bn = bn;
-    raw.ti_cur = kvc_load_at<uint16_t>(a.s.thread_infos + tile * KVC_WAVE, 2u * (uint32_t)lane);
+    if constexpr (PAYLOAD) raw.ti_cur = kvc_load_at<uint16_t>(a.s.thread_infos + tile * KVC_WAVE, 2u * (uint32_t)lane);
     // payload: whole aligned 16-byte chunks that each hold at least one payload byte (such reads never leave
     // the pages the payload lives in)
     const uint8_t *src = a.s.enc + off;
@@ -407,7 +421,7 @@ __device__ __forceinline__ void kvc_fetch_tile(const KvcFusedArgs &a, const KvcT
     const uint32_t nchunks = bn ? (head + bn + 15u) >> 4 : 0u;
     const uint8_t *g = src - head;
 #pragma unroll
-    for (int j = 0; j < KVC_PRE_CHUNKS; j++) {
+    for (int j = 0; j < (PAYLOAD ? KVC_PRE_CHUNKS : 0); j++) {
         const uint32_t c = (uint32_t)lane + 64u * j;
         if (c < nchunks) raw.pay[j] = kvc_load_at<uint4>(g, 16u * c);
     }
@@ -563,6 +577,113 @@ __device__ __forceinline__ KvcStaged kvc_stage_payload(const KvcFusedArgs &a, in
     first_out = first;
     longest_out = longest;
     return st;
+}
+
+// -- payloads in columns ------------------------------------------------------------------------------
+// A lane loads its own stream, sixteen bytes at a time, and puts word k of it in row k of an LDS area of 64 words a row.  A
+// lane's words then lie in its own bank, wherever the other lanes are: the three words of a refill take the LDS 7.3 cycles, where
+// lanes that read at their streams' places in the packed payload meet in the banks (19.5 cycles; streams of 52 bytes, positions
+// within 6 words).  The loads' addresses are as far apart as the streams are long, which costs nothing: 65 536 tiles of 3360
+// bytes in 33 us, as with whole lines in order.
+struct KvcLane {
+    const uint8_t *base;      // wave-uniform, a multiple of four
+    uint32_t at;              // the stream's first word, in bytes from there
+    uint32_t skip, bytes;     // bytes of that word before the stream, bytes from the word to the stream's end
+};
+// raw.off, raw.bn and raw.ti_cur are there
+template <class Raw>
+__device__ __forceinline__ KvcLane kvc_lane_stream(const KvcFusedArgs &a, int lane, const Raw &raw)
+{
+    // the previous lane's thread_info: one lane shift over the whole wave (lane 0 starts the tile)
+    const uint32_t ti_prev = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)raw.ti_cur, 0x138 /* wave_shr:1 */, 0xf, 0xf, true);
+    uint32_t start = ti_prev >> 3, end = raw.ti_cur >> 3;
+    if (start > raw.bn) start = raw.bn;
+    if (end > raw.bn) end = raw.bn;
+    if (end < start) end = start;
+    const uint8_t *p = a.s.enc + raw.off;
+    const uint32_t ahead = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 3u), from = ahead + start;
+    return {p - ahead, from & ~3u, from & 3u, (from & 3u) + (end - start)};
+}
+// Word k of the lane's stream, whatever lies behind the payload's buffer: words that hold a byte of the stream, and zeros
+__device__ __forceinline__ uint32_t kvc_lane_word(const KvcLane &l, uint32_t k)
+{
+    return l.bytes > l.skip && 4u * k < l.bytes ? kvc_load_at<uint32_t>(l.base, l.at + 4u * k) : 0u;
+}
+// Wave-uniform: the sixteen-byte loads of the tile's lanes stay inside the payload's buffer (all but a stream's last tiles)
+template <class Raw>
+__device__ __forceinline__ bool kvc_streams_inside(const KvcFusedArgs &a, const Raw &raw)
+{
+    return (int64_t)raw.off + raw.bn + 16 * KVC_PRE_CHUNKS <= a.s.enc_bytes;
+}
+// Loads of a tile's payload; rows: words of a stream that the LDS area holds.  Sets fits (wave-uniform: every stream is that short) and
+// u0: `lead_bits` before the lane's first code, and a word on, so that it is never negative (kvc_column_address takes it off again).
+template <class Raw>
+__device__ __forceinline__ KvcStaged kvc_fetch_streams(const KvcFusedArgs &a, int lane, int rows, uint32_t lead_bits, Raw &raw)
+{
+    typedef uint32_t w4 __attribute__((ext_vector_type(4), aligned(4)));
+    const KvcLane l = kvc_lane_stream(a, lane, raw);
+    KvcStaged st;
+    st.gwords = nullptr;
+    st.gnwords = st.gpos = 0;
+    st.fits = !__any((int)(l.bytes > 4u * (uint32_t)rows));
+    st.u0 = l.skip * 8u + 32u - lead_bits;
+    if (!kvc_streams_inside(a, raw)) return st;
+#pragma unroll
+    for (int j = 0; j < KVC_PRE_CHUNKS; j++) {
+        if (4 * j >= rows) break;
+        const w4 v = kvc_load_at<w4>(l.base, l.at + 16u * j);
+        raw.pay[j] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+    return st;
+}
+// ... into the columns.  column: LDS byte address of the lane's word in row 0.
+template <class Raw>
+__device__ __forceinline__ void kvc_stage_streams(const KvcFusedArgs &a, int lane, int rows, const Raw &raw, const KvcStaged &st, uint32_t column)
+{
+    if (!st.fits) return;
+    kvc_lds_u32 *dst = (kvc_lds_u32 *)(uintptr_t)column;
+    const bool inside = kvc_streams_inside(a, raw);
+    if (inside) {
+#pragma unroll
+        for (int j = 0; j < KVC_PRE_CHUNKS; j++) {
+            if (4 * j < rows) dst[64 * (4 * j)] = kvc_stream_word(raw.pay[j].x);
+            if (4 * j + 1 < rows) dst[64 * (4 * j + 1)] = kvc_stream_word(raw.pay[j].y);
+            if (4 * j + 2 < rows) dst[64 * (4 * j + 2)] = kvc_stream_word(raw.pay[j].z);
+            if (4 * j + 3 < rows) dst[64 * (4 * j + 3)] = kvc_stream_word(raw.pay[j].w);
+        }
+        if (rows <= 4 * KVC_PRE_CHUNKS) return;
+    }
+    const KvcLane l = kvc_lane_stream(a, lane, raw);
+#pragma unroll 1
+    for (int k = inside ? 4 * KVC_PRE_CHUNKS : 0; k < rows; k++) dst[64 * k] = kvc_stream_word(kvc_lane_word(l, k));     // streams beyond 61 bytes
+}
+// What the one-symbol decoder needs to know of a lane's stream
+template <class Raw>
+__device__ __forceinline__ void kvc_stream_in_memory(const KvcFusedArgs &a, int lane, const Raw &raw, KvcStaged &st)
+{
+    const KvcLane l = kvc_lane_stream(a, lane, raw);
+    st.gwords = reinterpret_cast<const uint32_t *>(l.base + l.at);
+    st.gnwords = l.bytes > l.skip ? (l.bytes + 3u) >> 2 : 0u;
+    st.gpos = l.skip * 8u;
+}
+// Byte address in LDS of row (u >> 5) - 1 of a lane's column; `column`: that of row 0.  A lane's position cannot pass its start by
+// more than 128 codes of 7 bits, so even a corrupt stream stays within KVC_COLUMN_REACH rows; the row before the first is read too
+// (bits before the first code, which nothing looks at).
+constexpr int KVC_COLUMN_REACH = 34;
+__device__ __forceinline__ uint32_t kvc_column_address(uint32_t column, uint32_t u)
+{
+    uint32_t row = u >> 5;
+    asm("" : "+v"(row));                                                                  // (see kvc_refill_address)
+    return (row << 8) + (column - 256u);
+}
+// Rows for the streams of a payload: the longest one where the encoder said it (it may start anywhere in its first word), else
+// somewhat more than the mean
+static inline int kvc_stream_rows(int64_t max_stream_bytes, int64_t encoded_bytes, int64_t tiles)
+{
+    const int64_t mean = encoded_bytes / (tiles > 0 ? tiles : 1) / KVC_WAVE;
+    int64_t bytes = max_stream_bytes > 0 ? max_stream_bytes : mean + mean / 2 + 8;
+    if (bytes > 112) bytes = 112;                                                         // 128 codes of 7 bits
+    return (int)((bytes + 3 + 3) / 4);
 }
 
 // ---------------------------------------------------------------------------------------------------

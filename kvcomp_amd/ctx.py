@@ -817,8 +817,8 @@ class KVCompCtx:
     def code_hint(self) -> int:
         """kvc_compressed_desc::max_code_bits of this context's codebook."""
         table = self.encode_codebook
-        return self.max_code_bits | self.pair_bits << 12 | (0x100 if table is not None and table.shape[0] <= 64 * 8 else 0) \
-            | (0x200 if table is not None and table.shape[0] <= 17 * 8 else 0)
+        rows = 0 if table is None else table.shape[0]        # eight bytes per symbol
+        return self.max_code_bits | self.pair_bits << 12 | (0 if rows == 0 or rows > 64 * 8 else 0x100 if rows > 17 * 8 else 0x300)
 
     def _build_lut(self):
         """The decode tables of the codebook that has just been put in place, on the stream that put it there: whoever is
