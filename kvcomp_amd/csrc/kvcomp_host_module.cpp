@@ -10,6 +10,7 @@
 //
 //   append_dense(k, v, cos, sin, k_cache, v_cache, at)   kvc_append_dense
 //   append_rows(tail, at, rows, row_bytes)               kvc_copy_rows of all of `rows` to `at` rows into `tail`
+//   first_encode(counted, ...)                           a first store from the wait for its symbol counts to the encode's launch
 //
 // Host C++ only, over the C ABI of include/kvcomp_hip.h.
 #include <torch/csrc/autograd/python_variable.h>
@@ -19,6 +20,8 @@
 #include <c10/core/GradMode.h>
 #include <c10/hip/HIPStream.h>
 #include <pybind11/pybind11.h>
+
+#include <algorithm>
 
 #include "kvcomp_hip.h"
 
@@ -121,7 +124,53 @@ PyObject *append_rows(PyObject *, PyObject *const *args, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// While the host is between a first store's counts and its encode the GPU has nothing to do, and this was some 20 us of Python (views
+// of the codebook's parts, the payload buffer, the job, three calls).  Here it is the codebook (3 us), an allocation and the launches.
+// (counted, smoothed_symbols, book, job, scratch, prepared, place, table_at, vectors, outcome, number, stream); book, job, scratch and
+// outcome are addresses, place is the tensor for the decode tables with the codebook's parts from table_at on.  Returns (what
+// kvc_counted_codebook returned, what kvc_encode_queue_book did, the payload's most bytes, its buffer or None): None where the codebook is
+// not one for it (more than sixteen symbols, codes of more than seven bits), and nothing is queued then.
+PyObject *first_encode(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(n == 12, "first_encode takes twelve arguments");
+    int64_t v[12] = {};
+    for (int i = 0; i < 12; i++) {
+        if (i == 6) continue;
+        v[i] = (int64_t)PyLong_AsUnsignedLongLongMask(args[i]);
+        if (PyErr_Occurred()) return nullptr;
+    }
+    const at::Tensor *place = plain(args[6]);
+    TORCH_CHECK(place && place->scalar_type() == at::kByte && place->is_contiguous(), "place: a device uint8 tensor");
+    const c10::DeviceGuard guard(place->device());
+    kvc_codebook *book = (kvc_codebook *)(uintptr_t)v[2];
+    kvc_encode_job *job = (kvc_encode_job *)(uintptr_t)v[3];
+    void *stream = (void *)(uintptr_t)v[11];
+    int counted_rc, queue_rc = 0;
+    int64_t most = 0;
+    at::Tensor payload;
+    {
+        const pybind11::gil_scoped_release released;
+        counted_rc = kvc_counted_codebook((void *)(uintptr_t)v[0], (int)v[1], book, stream);
+        if (!counted_rc && book->encode_bytes > 0 && book->encode_bytes <= 16 * 8 && book->max_code_bits <= 7 &&
+            place->numel() >= v[7] + (book->encode_bytes + 15) / 16 * 16 + book->decode_bytes) {
+            // (the same room for growing as any buffer of a context's)
+            most = book->payload_bits / 8 + v[8] + 1;
+            payload = at::empty({most + std::max<int64_t>(most / 4, 16)}, place->options());
+            job->d_encoded = (uint8_t *)payload.data_ptr();
+            job->encoded_cap = most;
+            uint8_t *lut = (uint8_t *)place->data_ptr();
+            queue_rc = kvc_encode_queue_book(job, (void *)(uintptr_t)v[4], (int)v[5], book, lut + v[7], lut, (uint32_t *)(uintptr_t)v[9], (uint32_t)v[10], stream);
+        }
+    }
+    PyObject *buffer = payload.defined() ? THPVariable_Wrap(payload) : (Py_INCREF(Py_None), Py_None);
+    if (!buffer) return nullptr;
+    return Py_BuildValue("iiLN", counted_rc, queue_rc, (long long)most, buffer);
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"first_encode", (PyCFunction)(void (*)())first_encode, METH_FASTCALL, "a first store's codebook and the encode with it"},
     {"append_dense", (PyCFunction)(void (*)())append_dense, METH_FASTCALL, "kvc_append_dense where it takes the tensors; whether it did"},
     {"append_rows", (PyCFunction)(void (*)())append_rows, METH_FASTCALL, "kvc_copy_rows where it takes the tensors; whether it did"},
     {nullptr, nullptr, 0, nullptr},

@@ -216,6 +216,28 @@ class _QueuedStore(NamedTuple):
     done: Optional["torch.cuda.Event"] = None        # behind it on its stream, if it had no outcome's words to write to
 
 
+class _NativeFirst:
+    """What _first_chunk hands the quantizer's second half: the codebook and the encode with it in one native call
+    (first_encode of kvcomp_host_module.cpp)."""
+    __slots__ = ("prepared", "place", "vectors", "outcome", "before", "told", "failed", "most", "payload")
+
+    def __init__(self, prepared, place, vectors, outcome, stream):
+        self.prepared, self.place, self.vectors, self.outcome = prepared, place, vectors, outcome
+        self.failed, self.most, self.payload = 0, 0, None
+        self.before = outcome.number, outcome.stream
+        self.told = outcome.ask(stream)
+
+    def __call__(self, counted, smoothed, book, stream):
+        p = self.prepared
+        rc, self.failed, self.most, self.payload = _lib.host().first_encode(
+            counted, smoothed, C.addressof(book), C.addressof(p.job), p.scratch.data_ptr(), p.done, self.place, _lib.lib().kvc_lut_bytes(),
+            self.vectors, *self.told, stream)
+        return rc
+
+    def refused(self):
+        self.outcome.refused(*self.before)
+
+
 # the seventeen 8-byte fields of kvc_compressed_desc, in order
 _DESC = struct.Struct("=17q")
 
@@ -677,6 +699,11 @@ class KVCompCtx:
                     torch.cuda.current_stream(self.device).synchronize()
                 outcome.refused(*before)
             raise
+        self._has_queued(T, sizes, worst, outcome, keep, lost_if_dropped, certain, codebook)
+
+    def _has_queued(self, T: int, sizes, worst: int, outcome, keep=None, lost_if_dropped=False, certain=False, codebook=False):
+        """The bookkeeping behind an encode of T tokens that has been queued."""
+        nb = T // self.block_size
         self._block_infos.used += sizes[0]
         self._thread_infos.used += sizes[1]
         self._min_ints.used += nb
@@ -724,17 +751,45 @@ class KVCompCtx:
         packed = (not want_symbols and fresh and smoothed <= 16 and
                   kvcomp_cuda.packed_symbols_supported(self.is_k, self._mask, blocked, self.quant_scale_rel))
 
+        native, vectors = None, T * self.batch_size * self.head_num * self.head_dim // (self.head_dim if self.is_k else kvcomp_cuda.V_VEC_LEN)
+
         def meanwhile(symbols):
-            if fresh:
-                prepared.extend((self._prepare_encode(T, symbols, packed), kvcomp_cuda.codebook_room(device)))
+            nonlocal native
+            if not fresh:
+                return None
+            prepared.extend((self._prepare_encode(T, symbols, packed), kvcomp_cuda.codebook_room(device)))
+            if packed and self.async_store and not self._unverified and not _lib.hooked():
+                self._sync_sizes()                             # (as _encode_direct)
+                self._verified = self._bookkeeping() + (self._encoded.used,)
+                outcome = self._ask_outcome()
+                if outcome is not None:
+                    native = _NativeFirst(*prepared, vectors, outcome, _lib.stream_of(self._state))
+            return native
         quantize = kvcomp_cuda.quant_codebook_packed if packed else kvcomp_cuda.quant_codebook
-        sym, book = quantize(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale, smoothed, meanwhile)
+        try:
+            sym, book = quantize(blocked, self._mask, self.quant_scale_rel, min_ints, quant_scale, smoothed, meanwhile)
+            if native is not None:
+                _lib.check(native.failed)
+        except BaseException:
+            if native is not None:
+                with contextlib.suppress(RuntimeError):        # (as in _encode_direct)
+                    torch.cuda.current_stream(device).synchronize()
+                native.refused()
+            raise
         self.waits += 1
+        if native is not None and native.payload is not None:
+            enc, dec, lut = kvcomp_cuda.codebook_parts(book, prepared[1])
+            self._encoded._hold(native.payload)
+            self._has_queued(T, prepared[0].sizes, native.most, native.outcome, certain=True, codebook=True)
+            self._issue_probe()
+            self._take_book(book, enc, dec, lut)
+            return None
+        if native is not None:
+            native.refused()                                   # (nothing of it has been queued)
         if packed and book.encode_bytes > 16 * 8:              # scales among fp16's smallest numbers: half a byte does not hold these symbols
             sym = quant(blocked, self.quant_dims, self.quant_scale_rel)[0]
             prepared, packed = [], False
         enc, dec, lut = kvcomp_cuda.codebook_parts(book, prepared[1]) if packed else kvcomp_cuda.put_codebook(book, device, *prepared[1:])
-        vectors = T * self.batch_size * self.head_num * self.head_dim // (self.head_dim if self.is_k else kvcomp_cuda.V_VEC_LEN)
         cannot_fail = book.max_code_bits <= 7
         small = T <= self.ASYNC_KEEP_BLOCKS * self.block_size
         queued = self.async_store and (cannot_fail or small)
@@ -746,10 +801,13 @@ class KVCompCtx:
             self._issue_probe()
         else:
             self._sync_sizes()                                 # (a failure leaves the context as it was before the encode)
+        self._take_book(book, enc, dec, lut)
+        return None if packed else sym
+
+    def _take_book(self, book, enc, dec, lut):
         self.tree_format, self.max_code_bits, self.pair_bits = book.tree_format, book.max_code_bits, book.pair_bits
         self.encode_codebook, self.decode_codebook = enc, dec
         self._lut, self._lut_source = lut, dec
-        return None if packed else sym
 
     def _smoothed_symbols(self) -> int:
         return min(256, int(math.ceil(1.0 / self.quant_scale_rel)) + 3)      # symbols 0 .. ceil(1 / eb) + 2

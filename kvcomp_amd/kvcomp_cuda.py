@@ -177,10 +177,13 @@ def _quant_codebook(blocked, quant_mask, quant_scale_rel, min_ints, scales, smoo
             return sym, book
         counted = C.c_void_p(0)
         check((L.kvc_quant_counted_packed if packed else L.kvc_quant_counted)(*args, C.byref(counted), stream))
+        finish = None
         try:
-            meanwhile(sym)
+            finish = meanwhile(sym)
         finally:
-            rc = L.kvc_counted_codebook(counted, smoothed_symbols, C.byref(book), stream)
+            # `finish` (or None): does this itself, and with the codebook what it likes; returns what kvc_counted_codebook returned
+            rc = (finish(counted.value, smoothed_symbols, book, stream) if finish is not None
+                  else L.kvc_counted_codebook(counted, smoothed_symbols, C.byref(book), stream))
         check(rc)
     return sym, book
 
