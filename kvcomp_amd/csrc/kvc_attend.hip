@@ -252,10 +252,10 @@ __global__ void __launch_bounds__(KVC_WG) __attribute__((amdgpu_waves_per_eu(REP
                 // 30 bits of a half window hold three pairs of codes of up to 5 bits, two of 6
                 int n_main = kb <= 5u ? D / 12 * 12 : 0;
                 while ((D - n_main) % 8 != 0) n_main -= 12;
-                if (n_main) kvc_mfma_pair_dot<3, false, NM, true, true, true>(sbase, u, fe_k, mask, n_main, bptr, msptr, acc, true);
-                kvc_mfma_pair_dot<2, false, NM, true, true, true>(sbase, u, fe_k, mask, D - n_main, bptr, msptr, acc, true);
+                if (n_main) kvc_mfma_pair_dot<3, KVC_PACKED_PLAIN, NM, true, true, true>(sbase, u, fe_k, mask, n_main, bptr, msptr, acc, true);
+                kvc_mfma_pair_dot<2, KVC_PACKED_PLAIN, NM, true, true, true>(sbase, u, fe_k, mask, D - n_main, bptr, msptr, acc, true);
             } else {
-                kvc_mfma_dot<4, false, NM, true, true, KVC_ENTRY_WORD, true>(sbase, u, fe_k, mask, D, bptr, msptr, acc, true);
+                kvc_mfma_dot<4, KVC_PACKED_PLAIN, NM, true, true, KVC_ENTRY_WORD, true>(sbase, u, fe_k, mask, D, bptr, msptr, acc, true);
             }
 #pragma unroll
             for (int q = 0; q < NM; q++) {

@@ -971,7 +971,7 @@ static void kvc_launch_fused(int kind, const KvcFusedArgs &a, dim3 grid, size_t 
 static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_bytes, int64_t tiles,
                            int64_t max_tile_bytes, int64_t max_stream_bytes, int max_code_bits, int64_t extra_words = 0,
                            bool allow_pairs = true, int64_t mfma_ops_words = 0, int long_table_words = 0, int narrow_pair_bits = 0,
-                           bool two_byte_table = false)
+                           bool two_byte_table = false, bool columns = false)
 {
     const int64_t slack = KVC_LDS_SLACK_WORDS + (long_table_words ? KVC_LDS_LONG_SLACK_WORDS : 0);
     const int force_rows = kvc_option(KVC_OPT_FUSED_ROWS);   // 0 / 1 overrides the choice below
@@ -1013,6 +1013,18 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
     // lead word + the stream's words (it may start anywhere in its first word) + look-ahead, forced odd
     const int64_t row = ((stream_bytes + 3 + 3) / 4 + 3) | 1;
     const int64_t pack_rows = (pack + row + 3) / 4 * 4;      // spare words for the fixed-length copy into rows
+    a.column_rows = 0;
+    if (columns) {
+        int rows = kvc_stream_rows(max_stream_bytes, encoded_bytes, tiles);
+        while (rows > 1 && KVC_WAVE * rows > budget) rows--;
+        a.column_rows = rows;
+        a.row_words = a.skew = 0;
+        a.pack_logical = a.pack_words = 0;
+        int64_t words = a.table_words + KVC_WAVES_PER_WG * (ops_words + KVC_WAVE * rows);
+        // what a corrupt payload of the last wave may lead to
+        const int64_t reach = a.table_words + KVC_WAVE * ((KVC_WAVES_PER_WG - 1) * rows + KVC_COLUMN_REACH);
+        return 4 * (size_t)(words > reach ? words : reach);
+    }
     // Decoding from the plain packed payload lines the lanes up on a few banks when a small multiple of the mean
     // stream length is close to a multiple of the 32 banks (lane l reads about l mean-stream-lengths into the
     // payload).  The skewed layout cures that at the cost of 1/16 more LDS and two instructions per refill;
@@ -1198,7 +1210,7 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     const size_t lds = mfma ? kvc_plan_lds(a, slots, (int)rep, encoded_bytes, rows * a.s.cols, max_tile_bytes, max_stream_bytes,
                                            max_code_bits, 0, !long_codes, kvc_mfma_ops_words(slots, (int)rep, rounded),
                                          long_codes ? KVC_LONG_TABLE_WORDS : 0, is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint),
-                                         mid_codes)
+                                         mid_codes, !long_codes)
                             : kvc_plan_lds(a, slots, rounded ? (int)rep + 1 : (int)rep, encoded_bytes, rows * a.s.cols,
                                            max_tile_bytes, max_stream_bytes, max_code_bits, 0, !rounded);
     a.rounded = rounded;
@@ -1226,8 +1238,8 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
                 a.sched_wg[2], a.sched_wg[3], a.sched_tile[0], a.sched_tile[1], a.sched_tile[2], a.sched_tile[3], a.sched_tile[4]);
     if (trace_plan)
         fprintf(stderr, "[kvcomp] fused kind %d rep %d: grid %u x %u, lds %zu B (table %d w, payload %d w of %d logical, "
-                "skew %d, rows %d), pair bits %d, tiles per wave %d, rounded %d\n", kind, (int)rep, grid.x, grid.y, lds,
-                a.table_words, a.pack_words, a.pack_logical, a.skew, a.row_words, a.pair_bits, a.s.tiles_per_wave, a.rounded);
+                "skew %d, rows %d, columns of %d), pair bits %d, tiles per wave %d, rounded %d\n", kind, (int)rep, grid.x, grid.y, lds,
+                a.table_words, a.pack_words, a.pack_logical, a.skew, a.row_words, a.column_rows, a.pair_bits, a.s.tiles_per_wave, a.rounded);
     if (mfma) {
         if (trace_plan) fprintf(stderr, "[kvcomp]   matrix-core kernel\n");
         if (long_codes) kvc_launch_fused_long((int)rep, kind, a, grid, lds, stream);

@@ -31,6 +31,7 @@ struct KvcFusedArgs {
     int pack_logical;    // payload words (lead words included) that fit there; fewer than pack_words when skewed
     int skew;            // 0, or 2: every 32 payload words are followed by a copy of the next two (see kvc_skewed)
     int row_words;       // LDS words per lane stream (odd); 0 = decode from the packed payload
+    int column_rows;     // payloads in columns: words of a stream that the LDS holds
     int pair_bits;       // index width of the two-symbol table the host made room for; 0 = none
     int narrow_pair_bits; // matrix-core V kernels: index bits of a two-symbol table that next to all pairs that occur fit; 0 = none
     int double_window;   // refill 64 stream bits at a time where the vector length allows
@@ -497,7 +498,8 @@ __device__ __forceinline__ float kvc_half_bits_to_float(uint32_t bits16)
 
 // What the decode step needs to know about a staged tile.
 struct KvcStaged {
-    bool fits;            // staged in LDS (wave-uniform); otherwise decode from global memory
+    int fits;             // staged in LDS (wave-uniform); otherwise decode from global memory  (no bool: copies of the struct's padding
+                          // would go through scratch memory)
     uint32_t u0;          // fast-path start position (`lb` bits before the first code) in the lane's LDS words
     const uint32_t *gwords;   // the lane's stream in global memory, from the aligned word holding its first byte
     uint32_t gnwords, gpos;
@@ -585,12 +587,18 @@ __device__ __forceinline__ KvcStaged kvc_stage_payload(const KvcFusedArgs &a, in
 // lanes that read at their streams' places in the packed payload meet in the banks (19.5 cycles; streams of 52 bytes, positions
 // within 6 words).  The loads' addresses are as far apart as the streams are long, which costs nothing: 65 536 tiles of 3360
 // bytes in 33 us, as with whole lines in order.
+// With them the attention kernels of 4 x 32 heads x 96 x 32 768 tokens (K six bits and skewed before, V two symbols per look-up) take 152 us
+// for 161; there is no skewed variant of a loop any more, and the kernels need two to six registers less.
 struct KvcLane {
     const uint8_t *base;      // wave-uniform, a multiple of four
     uint32_t at;              // the stream's first word, in bytes from there
     uint32_t skip, bytes;     // bytes of that word before the stream, bytes from the word to the stream's end
 };
 // raw.off, raw.bn and raw.ti_cur are there
+struct KvcTileBytes {
+    uint32_t off, bn;         // block_info, clamped to the payload buffer (wave-uniform)
+    uint32_t ti_cur;          // thread_info of this lane
+};
 template <class Raw>
 __device__ __forceinline__ KvcLane kvc_lane_stream(const KvcFusedArgs &a, int lane, const Raw &raw)
 {
@@ -676,6 +684,18 @@ __device__ __forceinline__ uint32_t kvc_column_address(uint32_t column, uint32_t
     asm("" : "+v"(row));                                                                  // (see kvc_refill_address)
     return (row << 8) + (column - 256u);
 }
+enum { KVC_PACKED_PLAIN = 0, KVC_PACKED_SKEWED = 1, KVC_COLUMNS = 2 };
+// The three words of a refill.  base: kvc_refill_address's, or the lane's column.
+template <int LAYOUT>
+__device__ __forceinline__ void kvc_refill(uint32_t base, uint32_t u, uint32_t &w0, uint32_t &w1, uint32_t &w2)
+{
+    constexpr int STEP = LAYOUT == KVC_COLUMNS ? KVC_WAVE : 1;
+    const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)(LAYOUT == KVC_COLUMNS ? kvc_column_address(base, u) : kvc_refill_address<LAYOUT == KVC_PACKED_SKEWED>(base, u));
+    w0 = wp[0];
+    w1 = wp[STEP];
+    w2 = wp[2 * STEP];
+}
+
 // Rows for the streams of a payload: the longest one where the encoder said it (it may start anywhere in its first word), else
 // somewhat more than the mean
 static inline int kvc_stream_rows(int64_t max_stream_bytes, int64_t encoded_bytes, int64_t tiles)

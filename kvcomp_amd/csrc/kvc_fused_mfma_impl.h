@@ -352,7 +352,7 @@ __device__ __forceinline__ void kvc_mfma_stage_ops(const KvcFusedArgs &a, const 
 // 4 x 32 x 96 x 32 768 (six bits) K 102.5 -> 91; 16 x 8 x 4 x 128 x 8192 K 43.2 -> 43.0, V 47.6 -> 47.0.
 enum { KVC_ENTRY_WORD = 0, KVC_ENTRY_HALF = 1, KVC_ENTRY_BYTE = 2 };
 constexpr int KVC_BYTE_CENTRE = 8;
-template <int G, bool SKEW, int NM, bool ROUNDED, bool BCAST, int FORM = KVC_ENTRY_WORD, bool EVERY = false>
+template <int G, int LAYOUT, int NM, bool ROUNDED, bool BCAST, int FORM = KVC_ENTRY_WORD, bool EVERY = false>
 __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32_t fe, uint32_t mask4, int n,
                                              uint32_t &bptr, uint32_t &msptr, kvc_f4 (&acc)[NM], bool holder)
 {
@@ -362,8 +362,8 @@ __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32
     static_assert(!BYTE || ROUNDED, "the symbols are short of eight, which the minima make up for");
     asm volatile("" : "+v"(msptr));      // kept in a vector register: one add per round instead of a move per read
     for (int i = 0; i < n; i += 2 * G) {
-        const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
-        const uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2];
+        uint32_t w0, w1, w2;
+        kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
         const uint32_t lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
         uint32_t R = lo, es = 0, used1 = 0;
         uint32_t e[2 * G];
@@ -407,14 +407,14 @@ __device__ __forceinline__ void kvc_mfma_dot(uint32_t sbase, uint32_t &u, uint32
 }
 
 // Two symbols per look-up: PG pairs from each half window, 4 PG symbols per refill; n a multiple of 4 PG.
-template <int PG, bool SKEW, int NM, bool ROUNDED, bool BCAST, bool EVERY = false>
+template <int PG, int LAYOUT, int NM, bool ROUNDED, bool BCAST, bool EVERY = false>
 __device__ __forceinline__ void kvc_mfma_pair_dot(uint32_t sbase, uint32_t &u, uint32_t fe, uint32_t maskp, int n,
                                                   uint32_t &bptr, uint32_t &msptr, kvc_f4 (&acc)[NM], bool holder)
 {
     asm volatile("" : "+v"(msptr));      // kept in a vector register: one add per round instead of a move per read
     for (int i = 0; i < n; i += 4 * PG) {
-        const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
-        const uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2];
+        uint32_t w0, w1, w2;
+        kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
         const uint32_t lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
         uint32_t R = lo, es = 0, used1 = 0;
         uint32_t e[2 * PG];
@@ -454,15 +454,15 @@ __device__ __forceinline__ void kvc_mfma_pair_dot(uint32_t sbase, uint32_t &u, u
 // the list in LDS (esc_addr: {code, length | symbol << 8} each), and starts a new window behind it.  The fp32-FMA kernels,
 // which served these codebooks, look symbols up one per refill in global memory once a code has more than 10 bits:
 // K products of 1 x 32 heads x 128 x 8192 tokens, one scale per block, 68 us.
-template <bool SKEW, int NM, bool ROUNDED, bool BCAST>
+template <int LAYOUT, int NM, bool ROUNDED, bool BCAST>
 __device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, uint32_t fe, uint32_t mask, uint32_t esc_addr, uint32_t nesc,
                                                   int n, uint32_t &bptr, uint32_t &msptr, kvc_f4 (&acc)[NM], bool holder)
 {
     asm volatile("" : "+v"(msptr));
 #pragma unroll 1
     for (int i = 0; i < n; i += 8) {
-        const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
-        uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2];
+        uint32_t w0, w1, w2;
+        kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
         uint32_t lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
         uint32_t R = lo, es = 0;
         uint32_t e[4];
@@ -477,8 +477,7 @@ __device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, u
             uint32_t f = *(const kvc_lds_u16 *)(uintptr_t)((R & mask) | fe);
             if (__builtin_expect(__any(f == 0u), 0)) {           // wave-uniform
                 u += es & 31u;
-                wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
-                w0 = wp[0], w1 = wp[1], w2 = wp[2];
+                kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
                 // the 32 bits from the code on (the window starts a bit before it)
                 const uint32_t win = __builtin_amdgcn_alignbit(__builtin_amdgcn_alignbit(w2, w1, u), __builtin_amdgcn_alignbit(w1, w0, u), 1u);
                 uint32_t len = f & 31u;
@@ -495,8 +494,7 @@ __device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, u
                 }
                 u += len;
                 es = 0;
-                wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<SKEW>(sbase, u);
-                w0 = wp[0], w1 = wp[1], w2 = wp[2];
+                kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
                 lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
                 R = lo;
             } else {
@@ -605,17 +603,20 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     constexpr int SLOTS = KvcGeom<KIND>::SLOTS;
     constexpr int NM = kvc_mfma_sets(REP);
     using T = KvcMfmaTables<REP>;
+    // Codes of at most 7 bits: payloads in columns (kvc_fetch_streams); the kernels for longer ones decode packed payloads.
+    constexpr bool COLUMNS = !LONG;
     // dynamic LDS: the decode table (at offset 0, so that its address folds into the look-ups), then per wave:
-    // operand tables, packed payload
+    // operand tables, packed payload; in columns, all waves' payloads, then all waves' operand tables
     extern __shared__ __align__(16) uint32_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int D = a.head_dim;
     constexpr int OPS_WORDS = kvc_mfma_ops_words(SLOTS, REP, ROUNDED);
-    const int per_wave = OPS_WORDS + a.pack_words;
-    uint32_t *btab = smem + a.table_words + wave * per_wave;
+    const int payload_words = COLUMNS ? KVC_WAVE * a.column_rows : a.pack_words;
+    uint32_t *pack = smem + a.table_words + (COLUMNS ? wave * payload_words : wave * (OPS_WORDS + payload_words) + OPS_WORDS);
+    uint32_t *btab = COLUMNS ? smem + a.table_words + KVC_WAVES_PER_WG * payload_words + wave * OPS_WORDS : pack - OPS_WORDS;
     uint32_t *mstab = btab + SLOTS * T::BTAB_SLOT_WORDS;
-    uint32_t *pack = btab + OPS_WORDS;
+    auto column_of = [&](int lane) { return kvc_lds_addr(smem) + 4u * (uint32_t)(a.table_words + wave * payload_words + lane); };
     // Which tiles this wave takes.  Plain launch: grid (column groups, tile rows), every wave `tiles_per_wave`
     // consecutive columns of its row.  Scheduled launch (sched_nseg > 0; one codebook for the whole stream): a 1-D grid
     // over the row-major tile sequence in a few segments, the waves of segment k taking sched_run[k] consecutive tiles
@@ -647,6 +648,15 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
         const uint32_t *bi = reinterpret_cast<const uint32_t *>(a.s.block_infos + 8 * ((int64_t)t_first + lane));
         bi_off = bi[0];
         bi_bn = bi[1];
+    }
+    // in columns: the lanes' thread_infos of the first tile and of the one behind it, which its loads' addresses need
+    auto thread_info = [&](const KvcFusedArgs &a, int tile, int lane) {
+        return (uint32_t)kvc_load_at<uint16_t>(a.s.thread_infos + (int64_t)tile * KVC_WAVE, 2u * (uint32_t)lane);
+    };
+    uint32_t ti_first = 0, ti_next = 0;
+    if constexpr (COLUMNS) {
+        if (ntiles > 0) ti_first = thread_info(a, t_first, lane);
+        if (ntiles > 1) ti_next = thread_info(a, t_first + 1, lane);
     }
     const int64_t cb = a.s.rows_per_codebook ? (a.sched_nseg ? 0 : (int)blockIdx.y) / a.s.rows_per_codebook : 0;
     const uint32_t *__restrict__ lut_g = a.s.luts + cb * KVC_LUT_WORDS;
@@ -739,7 +749,7 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     }
     // columns that no query head owns (REP 1: columns 2 and 3) are multiplied too: give them zeros once
     for (int i = lane; i < SLOTS * T::BTAB_SLOT_WORDS; i += KVC_WAVE) btab[i] = 0;
-    if (lane < KVC_PACK_LEAD) pack[lane] = 0;
+    if (!COLUMNS && lane < KVC_PACK_LEAD) pack[lane] = 0;
     __syncthreads();
     const uint32_t mask4 = ((1u << (LONG ? (uint32_t)KVC_LUT_ESC_BITS : lbits)) - 1u) << lead_bits, maskp = ((1u << pbits) - 1u) << 2;
     const int n = IS_K ? D : KVC_V_TOKENS;                             // symbols per lane stream
@@ -759,7 +769,12 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     tabs.head0 = tabs.head1 = tabs.row = -1;
     tabs.lo0 = tabs.lo1 = 0;                                             // (the low-part columns start as zeros)
     KvcTablePlan plan = kvc_plan_tables<KIND, ROUNDED>(a, pos, tabs);
-    kvc_fetch_tile<REP, KIND, 0, SLOTS == 2>(a, pos, __builtin_amdgcn_readlane(bi_off, 0), __builtin_amdgcn_readlane(bi_bn, 0), lane, raw);
+    kvc_fetch_tile<REP, KIND, 0, SLOTS == 2, !COLUMNS>(a, pos, __builtin_amdgcn_readlane(bi_off, 0), __builtin_amdgcn_readlane(bi_bn, 0), lane, raw);
+    KvcStaged st;
+    if constexpr (COLUMNS) {
+        raw.ti_cur = ti_first;
+        st = kvc_fetch_streams(a, lane, a.column_rows, lead_bits, raw);
+    }
     // the second head's parameters where every token has groups of its own per batch entry or head: fetched only now
     auto late_params = [&](const KvcFusedArgs &a, const KvcTilePos &p, const KvcTablePlan &pl, int lane) {
         if constexpr (SLOTS == 2) {
@@ -776,9 +791,13 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     late_params(a, pos, plan, lane);
     float bias[REP], unscale;
     int sel = 0;
-    uint32_t first, longest;
-    KvcStaged st = kvc_stage_payload<true>(a, lane, raw, pack, first, longest);
-    if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;       // one or two bits before the lane's first code
+    if constexpr (COLUMNS) {
+        kvc_stage_streams(a, lane, a.column_rows, raw, st, column_of(lane));
+    } else {
+        uint32_t first, longest;
+        st = kvc_stage_payload<true>(a, lane, raw, pack, first, longest);
+        if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;   // one or two bits before the lane's first code
+    }
     kvc_mfma_stage_ops<REP, KIND, ROUNDED>(a, pos, plan, lane, raw, btab, mstab, bias, unscale, sel, tabs, centre);
     kvc_wave_sync();
     for (int it = 0; it < ntiles; it++) {
@@ -794,9 +813,17 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
         // are not kept in registers through the decode loops
         int lane_f = lane;
         asm volatile("" : "+v"(lane_f));
-        if (more)   // loads for the next tile fly while this one is decoded
-            kvc_fetch_tile<REP, KIND, 0, SLOTS == 2>(a, pos_next, __builtin_amdgcn_readlane(bi_off, it + 1),
-                                                     __builtin_amdgcn_readlane(bi_bn, it + 1), lane_f, raw, ~plan_next.build);
+        const KvcTileBytes here = {raw.off, raw.bn, raw.ti_cur};
+        KvcStaged st_next = st;
+        if (more) {   // loads for the next tile fly while this one is decoded
+            kvc_fetch_tile<REP, KIND, 0, SLOTS == 2, !COLUMNS>(a, pos_next, __builtin_amdgcn_readlane(bi_off, it + 1),
+                                                               __builtin_amdgcn_readlane(bi_bn, it + 1), lane_f, raw, ~plan_next.build);
+            if constexpr (COLUMNS) {
+                raw.ti_cur = ti_next;
+                st_next = kvc_fetch_streams(a, lane_f, a.column_rows, lead_bits, raw);
+                if (it + 2 < ntiles) ti_next = thread_info(a, t_first + it + 2, lane_f);
+            }
+        }
         const int my_slot = sel ? 1 - plan.slot0 : plan.slot0;
         const uint32_t *my_btab = btab + my_slot * T::BTAB_SLOT_WORDS, *my_mstab = mstab + my_slot * T::MSTAB_SLOT_WORDS;
         // (wave-uniform: some low-part column of the tables this tile reads holds something)
@@ -815,7 +842,7 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
         }
         if (fast_book && st.fits) {
             kvc_f4 acc[NM];
-            const uint32_t sbase = kvc_lds_addr(pack);
+            const uint32_t sbase = COLUMNS ? column_of(lane) : kvc_lds_addr(pack);
             // one head per tile: all sixteen blocks share their operand columns, which lanes 0 - 15 then hold for all
             constexpr bool BCAST = SLOTS == 1;
             const bool holder = lane < 16;
@@ -825,7 +852,7 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
             // as long as it is broad (8 x 32 x 128 x 4177: 84.4 -> 84.7, 4 x 32 x 96 x 32 768: 164.5 -> 161.8 altogether).
             constexpr bool EV = BCAST && (REP == 2 || REP == 8);
             auto run = [&](auto skew_, bool whole) {
-                constexpr bool SK = decltype(skew_)::value;
+                constexpr int SK = decltype(skew_)::value;
 #pragma unroll
                 for (int s = 0; s < NM; s++) acc[s] = kvc_f4{0.f, 0.f, 0.f, 0.f};
                 uint32_t u = st.u0;
@@ -847,8 +874,9 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
                 }
             };
             for (int m = mode;; m = 1) {
-                if (a.skew) run(std::true_type{}, (m & 1) != 0);
-                else run(std::false_type{}, (m & 1) != 0);
+                if constexpr (COLUMNS) run(std::integral_constant<int, KVC_COLUMNS>{}, (m & 1) != 0);
+                else if (a.skew) run(std::integral_constant<int, KVC_PACKED_SKEWED>{}, (m & 1) != 0);
+                else run(std::integral_constant<int, KVC_PACKED_PLAIN>{}, (m & 1) != 0);
                 if (!NARROW_OK || (m & 2)) break;
                 const bool nan = __any(__builtin_isnan(acc[0][0]) || __builtin_isnan(acc[0][1]) || __builtin_isnan(acc[0][2]) || __builtin_isnan(acc[0][3]));
                 if (m & 1) {                                   // (NaN of q or of the weights: no miss, and the same again)
@@ -894,7 +922,8 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
             }
         } else {
             KvcVec<REP> res;
-            if (st.fits)
+            if constexpr (COLUMNS) kvc_stream_in_memory(a, lane, here, st);
+            if (!COLUMNS && st.fits)
                 res = kvc_mfma_slow_tile<REP, false, ROUNDED>(pack, (uint32_t)a.pack_logical, st.u0 + lead_bits, lut_g, n, my_btab,
                                                               my_mstab, (uint32_t)a.skew, centre);
             else
@@ -914,8 +943,14 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
             kvc_wave_sync();     // every lane is done reading this tile's LDS data
             int lane_s = lane;
             asm volatile("" : "+v"(lane_s));
-            st = kvc_stage_payload<true>(a, lane_s, raw, pack, first, longest);
-            if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;
+            if constexpr (COLUMNS) {
+                st = st_next;
+                kvc_stage_streams(a, lane_s, a.column_rows, raw, st, column_of(lane_s));
+            } else {
+                uint32_t first, longest;
+                st = kvc_stage_payload<true>(a, lane_s, raw, pack, first, longest);
+                if (st.fits) st.u0 = 32u * KVC_PACK_LEAD + first * 8u - lead_bits;
+            }
             late_params(a, pos_next, plan_next, lane_s);
             kvc_mfma_stage_ops<REP, KIND, ROUNDED>(a, pos_next, plan_next, lane_s, raw, btab, mstab, bias, unscale, sel, tabs, centre);
             kvc_wave_sync();
