@@ -1765,21 +1765,29 @@ __device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint
 // K tile needs no staging, since the quantizer, which has it in registers, writes it in the order of the lanes.  A byte is the index of
 // a pair's look-up; V's pairs lie along the other axis, and are turned in registers.  Codes of any length are taken, since what
 // would be left over would have to be written out again (K of 2 x 32 x 96 x 4480 in block groups, codes of 11 bits).
-// With today's runs, late look-back and wide stores this kernel takes 54 and 47 us there, and 159 and 115.  Where a wave's time goes (clock
-// stamps, K | V of 4 x 32 x 96 x 32 768): start 9 | 8 %, loads 12 | 15, look-ups 14 | 18, packing 20 | 22, looking back 28 | 23, writing
-// 13 | 10.  Made-up offsets, so no look-back, had given 146 and 99 us for 198 and 126: waves wait for the slowest tile before theirs.
-// Three workgroups per compute unit with smaller areas and runs of two: K 162 -> 177 us.
+// With runs, late look-back and wide stores this kernel took 54 and 47 us there, and 159 and 115, with 28 | 23 % of a wave's time (clock
+// stamps, K | V of 4 x 32 x 96 x 32 768) spent looking back -- waves wait for the slowest tile before theirs -- and 9 | 8 % on the
+// start; loads 12 | 15, look-ups 14 | 18, packing 20 | 22, writing 13 | 10.  Made-up offsets, so no look-back, had shown what that costs:
+// 146 and 99 us for 198 and 126.  So where there are more runs than waves, the workgroups that the chip holds stay (`persistent`),
+// load the table once and draw run after run, and a run's images are placed when the next run's first tile has been counted
+// and its size published: what the look-back waits for has had a tile's loads and look-ups longer to arrive, and nobody waits for
+// the placing.  54 -> 50 us and 47 -> 47; 159 -> 146 and 115 -> 107.  A wave publishes and places in the order of the tiles, and
+// waits in a placing only for sizes before its own, so the earliest run not yet placed always can be.
+// Taken back: the next tile's symbols read ahead (146 -> 141 us, but 4 x 32 x 128 x 9000 tokens 56 -> 58); three workgroups per
+// compute unit with smaller areas and runs of two (K 162 -> 177 us).
 // FRONT 0: K, 1: V.  ND: registers that a vector fills, a byte per symbol.  FORM: a byte per symbol, or two symbols a byte with codes
 // of at most eight bits, or of any length.
 enum { KVC_FORM_BYTES = 0, KVC_FORM_PACKED = 1, KVC_FORM_PACKED_LONG = 2 };
+constexpr int KVC_SYM_TICKETS = 8;                         // tickets of a workgroup that are kept: more than its fastest wave is ahead of its slowest
 template <int FRONT, int ND, int FORM>
-__global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int run)
+__global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int run, int persistent)
 {
     constexpr bool PACKED = FORM != KVC_FORM_BYTES, LONG = FORM == KVC_FORM_PACKED_LONG;
     constexpr int G = !PACKED ? KVC_ONCE_GROUP_TILES : FRONT == 1 ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES_KPACKED;
     constexpr int STAGE = PACKED ? (FRONT == 0 ? 0 : KVC_STAGE_VPACKED_BYTES) : FRONT == 0 ? KVC_STAGE_VSYM_BYTES : KVC_STAGE_VF16_BYTES;
     extern __shared__ __align__(16) uint8_t s_dyn[];
-    __shared__ uint32_t s_err, s_max_tile, s_longest, s_polls, s_ticket;
+    __shared__ uint32_t s_err, s_max_tile, s_longest, s_polls, s_drawn;
+    __shared__ uint64_t s_tickets[KVC_SYM_TICKETS];        // the workgroup's n-th ticket in the lower half of word n % KVC_SYM_TICKETS, n + 1 in the upper
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
     uint2 *s_table = reinterpret_cast<uint2 *>(s_dyn);
     uint32_t *area = reinterpret_cast<uint32_t *>(s_dyn + 256 * sizeof(uint2) + wave * a.wave_bytes);
@@ -1788,7 +1796,8 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     if (tid == 0) ticket = atomicAdd(&a.status[KVC_ONCE_TICKET_WORD], 1u);
     const bool pairs = PACKED || a.table_entries <= 16;
     kvc_load_pair_table<PACKED>(a, s_table, pairs, LONG ? 16u : 8u);
-    if (tid == 0) { s_err = 0; s_max_tile = 0; s_longest = 0; s_polls = 0; s_ticket = ticket; }
+    if (tid < KVC_SYM_TICKETS) s_tickets[tid] = tid == 0 ? (uint64_t)1 << 32 | ticket : 0ull;
+    if (tid == 0) { s_err = 0; s_max_tile = 0; s_longest = 0; s_polls = 0; s_drawn = 1; }
     __syncthreads();
     // Neighbouring tiles share the cache lines that their symbols come in (V and head_dim 64: 64 bytes of each token's row, 96: 96, 72: 72),
     // and the lines of all waves are more than an L2 holds.  So STEP waves, whose tiles of one moment are whole lines, take the
@@ -1798,7 +1807,6 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     // Two symbols a byte: four V tiles are a line of each token's row, and a K tile is lines of its own.
     constexpr int STEP = PACKED ? (FRONT == 1 ? 4 : 1) : FRONT == 1 ? 2 : ND == 24 || ND == 18 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
     static_assert(PACKED ? G % (STEP * 3) == 0 && G % (STEP * 4) == 0 : G % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
-    const int tile0 = (__builtin_amdgcn_readfirstlane((int)s_ticket) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
     const int tiles = (int)a.tiles;
     const uint32_t base = a.status[KVC_ONCE_BASE_WORD];
     uint32_t err = 0, max_tile = 0, longest = 0, next_off = 0;
@@ -1811,6 +1819,70 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     uint32_t kept_words = 0;
     KvcOncePending first;
     first.in_group = 0;
+    int newest = 0;                                        // the youngest kept tile
+    // Writes the kept images out: one look-back (none behind tiles of the run that have been placed), the others follow
+    auto place_kept = [&](const KvcEncodeArgs &a, int lane) {
+        const int oldest = newest - STEP * (kept - 1);
+        uint32_t at = 0;
+        // the sizes of the other waves' tiles that lie in between: those in front of the k-th kept tile from lane k OTHERS on
+        const uint64_t *between_at = reinterpret_cast<const uint64_t *>(a.block_infos) + oldest + STEP * (lane / OTHERS) - 1 - lane % OTHERS;
+        const bool between = STEP > 1 && lane < OTHERS * kept && (lane >= OTHERS || placed);
+        uint64_t between_word = between ? kvc_status_load(between_at) : 0ull;
+#pragma unroll 1
+        for (int k = 0; k < kept; k++) {
+            KvcOncePending which = first;
+            which.tile = oldest + STEP * k;
+            which.bn = (uint32_t)(kept_bytes >> (16 * k)) & 0xffffu;
+            which.packs = which.bn <= (uint32_t)KVC_MAX_TILE_BYTES;
+            uint32_t off = 0;
+            if (STEP > 1 && placed) {
+                while (__any((uint32_t)(between_word >> 48) == KVC_BI_NOT_READY) && ++polls <= a.max_polls) {
+                    __builtin_amdgcn_s_sleep(2);
+                    if (between) between_word = kvc_status_load(between_at);
+                }
+#pragma unroll
+                for (int i = 0; i < OTHERS; i++)
+                    next_off += (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(between_word >> 32), k * OTHERS + i) & 0xffffu;
+            }
+            err |= kvc_once_place<G, true>(a, which, area + at, base, lane, &polls, &off, placed, next_off);
+            at += which.packs ? kvc_once_image_words(which.bn) : 0u;
+            next_off = off + which.bn;
+            placed = true;
+        }
+        kept = 0;
+        kept_bytes = 0;
+        kept_words = 0;
+        kvc_wave_lds_sync();                               // the images are read: the area is free
+    };
+    int tile0 = 0;
+#pragma unroll 1
+    for (uint32_t n = 0;; n++) {
+    // The wave's n-th run.  Whichever of the workgroup's waves comes first draws the ticket, the others find it.  (A wave's images are
+    // placed when the sizes of all runs before theirs are known, so no wave is eight runs ahead of another -- unless it has given
+    // up waiting, and then the call is encoded again anyway.)
+    {
+        uint64_t *slot = &s_tickets[n % KVC_SYM_TICKETS];
+        uint64_t word = __hip_atomic_load(slot, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        while ((uint32_t)(word >> 32) < n + 1u) {
+            uint32_t mine = 0;
+            if ((tid & 63) == 0) {
+                uint32_t expected = n;
+                if (__hip_atomic_compare_exchange_strong(&s_drawn, &expected, n + 1u, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) {
+                    const uint32_t drawn = atomicAdd(&a.status[KVC_ONCE_TICKET_WORD], 1u);
+                    __hip_atomic_store(slot, (uint64_t)(n + 1u) << 32 | drawn, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    mine = 1;
+                }
+            }
+            if (!__any((int)mine)) __builtin_amdgcn_s_sleep(1);
+            word = __hip_atomic_load(slot, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        if ((uint32_t)(word >> 32) != n + 1u) {
+            err |= KVC_ENC_ERR_ORDER;
+            break;
+        }
+        tile0 = (__builtin_amdgcn_readfirstlane((int)(uint32_t)word) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
+    }
+    if (tile0 >= tiles) break;
 #pragma unroll 1
     for (int it = 0; it < run; it++) {
         const int tile = tile0 + STEP * it;
@@ -1852,6 +1924,11 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         longest = lg > longest ? lg : longest;
         max_tile = bn > max_tile ? bn : max_tile;
         if (lane == 0) kvc_status_store(reinterpret_cast<uint64_t *>(a.block_infos) + tile, kvc_bi_word(0u, bn, KVC_BI_SIZE));
+        // Now that this size is known too, the run before is placed: what it waits for has had a tile's work longer to arrive.
+        if (it == 0) {
+            if (kept) place_kept(a, lane);
+            placed = false;
+        }
         // the tile that the run's place is looked for with; and the wave that speaks for a group must not sit on its size (as in
         // kvc_encode_once_kernel)
         const bool opens = kept == 0 && !placed, closes = kvc_once_closes<G>(a, tile);
@@ -1881,53 +1958,26 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
             kept_bytes |= (uint64_t)bn << (16 * kept);
             kept_words += my_words;
             kept++;
+            newest = tile;
         }
-        // Images wait for the run's other tiles, unless they reach to where those are to be staged.
-        const bool more = it + 1 < run && tile + STEP < tiles;
-        if (!fits || !more || kept_words * 4u > (uint32_t)(a.wave_bytes - STAGE)) {
-            const int oldest = tile + STEP * ((fits ? 1 : 0) - kept);
-            uint32_t at = 0;
-            // the sizes of the other waves' tiles that lie in between: those in front of the k-th kept tile from lane k OTHERS on
-            const uint64_t *between_at = reinterpret_cast<const uint64_t *>(a.block_infos) + oldest + STEP * (lane / OTHERS) - 1 - lane % OTHERS;
-            const bool between = STEP > 1 && lane < OTHERS * kept && (lane >= OTHERS || placed);
-            uint64_t between_word = between ? kvc_status_load(between_at) : 0ull;
-#pragma unroll 1
-            for (int k = 0; k < kept; k++) {               // one look-back (none behind tiles that have been placed), the others follow
-                KvcOncePending which = first;
-                which.tile = oldest + STEP * k;
-                which.bn = (uint32_t)(kept_bytes >> (16 * k)) & 0xffffu;
-                which.packs = which.bn <= (uint32_t)KVC_MAX_TILE_BYTES;
-                uint32_t off = 0;
-                if (STEP > 1 && placed) {
-                    while (__any((uint32_t)(between_word >> 48) == KVC_BI_NOT_READY) && ++polls <= a.max_polls) {
-                        __builtin_amdgcn_s_sleep(2);
-                        if (between) between_word = kvc_status_load(between_at);
-                    }
-#pragma unroll
-                    for (int i = 0; i < OTHERS; i++)
-                        next_off += (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(between_word >> 32), k * OTHERS + i) & 0xffffu;
-                }
-                err |= kvc_once_place<G, true>(a, which, area + at, base, lane, &polls, &off, placed, next_off);
-                at += which.packs ? kvc_once_image_words(which.bn) : 0u;
-                next_off = off + which.bn;
-                placed = true;
-            }
-            kept = 0;
-            kept_bytes = 0;
-            kept_words = 0;
-            kvc_wave_lds_sync();                           // the images are read: the area is free
+        // Images wait for the run's other tiles and the next run's first, unless they reach to where those are to be staged.
+        if (!fits || kept_words * 4u > (uint32_t)(a.wave_bytes - STAGE)) {
+            place_kept(a, lane);
             if (!fits) it--;
         }
     }
-    if ((tid & 63) == 0 && tile0 < tiles) {
+    if (!persistent) break;
+    }
+    if (kept) place_kept(a, tid & 63);
+    if ((tid & 63) == 0) {
         if (err) atomicOr(&s_err, err);
         atomicMax(&s_max_tile, max_tile);
         atomicMax(&s_longest, longest);
         atomicMax(&s_polls, (uint32_t)polls);
     }
     __syncthreads();
-    if (tid == 0) {                                        // to one of the slot's lines, picked by the ticket
-        uint32_t *part = a.status + KVC_ONCE_PART_WORD + (s_ticket % KVC_ONCE_PART_LINES) * KVC_ONCE_PART_STRIDE;
+    if (tid == 0) {                                        // to one of the slot's lines, picked by the first ticket
+        uint32_t *part = a.status + KVC_ONCE_PART_WORD + (ticket % KVC_ONCE_PART_LINES) * KVC_ONCE_PART_STRIDE;
         if (s_err) atomicOr(&part[0], s_err);
         atomicMax(&part[1], s_max_tile);
         atomicMax(&part[2], s_longest);
@@ -2327,7 +2377,12 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
         const auto symbols_kernel = kvc_symbols_kernel(is_k, a.vec_len, !c.packed ? KVC_FORM_BYTES : c.longest_code >= 1 && c.longest_code <= 8 ? KVC_FORM_PACKED : KVC_FORM_PACKED_LONG);
         if (wide) {
-            hipLaunchKernelGGL(symbols_kernel, dim3(wgs1), dim3(waves * KVC_WAVE), lds, stream, sa.e, run);
+            // Where the runs are more than one round of the waves, the first round's workgroups draw the others' too (kernel against
+            // kernel in first stores of K and V, us: 4 x 32 x 96 x 32 768 159 + 115 -> 146 + 107; whole first stores: 2 x 32 x 128 x 8192
+            // 280 -> 247, 4 x 24 x 72 x 9000 265 -> 237, 4 x 32 x 128 x 9000 390 -> 346).
+            const unsigned resident = KVC_WIDE_WAVES / (unsigned)waves;
+            const int persistent = waves == 2 * KVC_WAVES_PER_WG && wgs1 > resident;
+            hipLaunchKernelGGL(symbols_kernel, dim3(persistent ? resident : wgs1), dim3(waves * KVC_WAVE), lds, stream, sa.e, run, persistent);
             if (c.book) {
                 KvcPutSmallArgs put = {};
                 put.tree_at = (int)((c.book->encode_bytes + 15) / 16 * 16);
