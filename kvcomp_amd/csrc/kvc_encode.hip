@@ -1773,14 +1773,19 @@ __device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint
 // and its size published: what the look-back waits for has had a tile's loads and look-ups longer to arrive, and nobody waits for
 // the placing.  54 -> 50 us and 47 -> 47; 159 -> 146 and 115 -> 107.  A wave publishes and places in the order of the tiles, and
 // waits in a placing only for sizes before its own, so the earliest run not yet placed always can be.
-// Taken back: the next tile's symbols read ahead (146 -> 141 us, but 4 x 32 x 128 x 9000 tokens 56 -> 58); three workgroups per
-// compute unit with smaller areas and runs of two (K 162 -> 177 us).
+// Those workgroups are of sixteen waves, one per compute unit: half as many tickets, which arrive one in 11 ns, than of eight.
+// K 50 -> 46 us and 142 -> 131, V the same.  Tickets and table are 1 % now, loads 10 | 13, look-ups 17 | 20, packing 25 | 26, placing 43 | 36, two
+// thirds of that looking back.
+// Taken back: the next tile's symbols read ahead (146 -> 141 us, but 4 x 32 x 128 x 9000 tokens 56 -> 58); pairs in entries of four
+// bytes (half the LDS time, no gain); a workgroup's runs handed out in the order in which its waves ask (131 -> 135 us, with four
+// to a ticket 149); three workgroups per compute unit with smaller areas and runs of two (K 162 -> 177 us).
 // FRONT 0: K, 1: V.  ND: registers that a vector fills, a byte per symbol.  FORM: a byte per symbol, or two symbols a byte with codes
 // of at most eight bits, or of any length.
 enum { KVC_FORM_BYTES = 0, KVC_FORM_PACKED = 1, KVC_FORM_PACKED_LONG = 2 };
 constexpr int KVC_SYM_TICKETS = 8;                         // tickets of a workgroup that are kept: more than its fastest wave is ahead of its slowest
+// long_run: tiles of a wave's run, short_run: of those of tickets from short_from on (0: no workgroup draws a second one).
 template <int FRONT, int ND, int FORM>
-__global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int run, int persistent)
+__global__ void __launch_bounds__(4 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int long_run, int short_run, int short_from)
 {
     constexpr bool PACKED = FORM != KVC_FORM_BYTES, LONG = FORM == KVC_FORM_PACKED_LONG;
     constexpr int G = !PACKED ? KVC_ONCE_GROUP_TILES : FRONT == 1 ? KVC_ONCE_GROUP_TILES_VPACKED : KVC_ONCE_GROUP_TILES_KPACKED;
@@ -1854,7 +1859,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         kept_words = 0;
         kvc_wave_lds_sync();                               // the images are read: the area is free
     };
-    int tile0 = 0;
+    int tile0 = 0, run = 0;
 #pragma unroll 1
     for (uint32_t n = 0;; n++) {
     // The wave's n-th run.  Whichever of the workgroup's waves comes first draws the ticket, the others find it.  (A wave's images are
@@ -1880,7 +1885,9 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
             err |= KVC_ENC_ERR_ORDER;
             break;
         }
-        tile0 = (__builtin_amdgcn_readfirstlane((int)(uint32_t)word) * waves + (wave & ~(STEP - 1))) * run + (wave & (STEP - 1));
+        const int drawn = __builtin_amdgcn_readfirstlane((int)(uint32_t)word);
+        run = drawn < short_from ? long_run : short_run;
+        tile0 = (short_from * (long_run - run) + drawn * run) * waves + (wave & ~(STEP - 1)) * run + (wave & (STEP - 1));
     }
     if (tile0 >= tiles) break;
 #pragma unroll 1
@@ -1966,7 +1973,7 @@ __global__ void __launch_bounds__(2 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
             if (!fits) it--;
         }
     }
-    if (!persistent) break;
+    if (!short_run) break;                                 // (one run per wave)
     }
     if (kept) place_kept(a, tid & 63);
     if ((tid & 63) == 0) {
@@ -2212,6 +2219,21 @@ static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
     return 0;
 }
 
+// What the encoder from symbols takes for runs of `run` tiles, in fifths of a tile's time: its waves in whole rounds, and what is
+// left beyond those in shorter runs (`tail`) where that is less.  The waves that take their tiles in turn stay inside a group with
+// those too where the first of them starts at a multiple of their tiles.
+constexpr int KVC_WIDE_WAVES = 4096;
+static int64_t kvc_runs_cost(int64_t tiles, int run, int *tail)
+{
+    auto rounds = [](int64_t t, int r) { return (t + (int64_t)KVC_WIDE_WAVES * r - 1) / ((int64_t)KVC_WIDE_WAVES * r) * (5 * r + 6); };
+    const int64_t whole = tiles / ((int64_t)KVC_WIDE_WAVES * run) * run * KVC_WIDE_WAVES, rest = tiles - whole;
+    int best = run;
+    for (int r = run - 1; r >= 1; r--)
+        if (whole % (4 * r) == 0 && rounds(rest, r) < rounds(rest, best)) best = r;
+    if (tail) *tail = best;
+    return rounds(whole, run) + rounds(rest, best);
+}
+
 template <int FORM>
 static auto kvc_symbols_kernel_of(int is_k, int vec_len)
 {
@@ -2355,9 +2377,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         // Its 4096 waves at a time: runs of two from where single tiles would be a second, part-filled round of them.  K and
         // V of 2 x 32 heads x 128 x 6144 tokens (6144 tiles) in first stores: 50 -> 35 and 47 -> 32 us; K of 4 x 24 x 72 x 4096: 47 -> 31.
         // (V's runs of four begin where those of two would be a second round: 2 x 32 x 128 x 12 288 tokens 58 -> 51 us, 9216 49 -> 48.)
-        constexpr int KVC_WIDE_WAVES = 4096;
         if (wide && small && want == 1 && a.tiles > KVC_WIDE_WAVES) run = 2;
-        const int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
+        int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
         // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
         // together take stays inside a group, or the wave that speaks for a group would wait before all its tiles are counted).
@@ -2368,21 +2389,31 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
             // and four tiles, us: 4 x 32 heads x 64 x 32 768 tokens (65 536 tiles) 148, 133, 113; 4 x 24 x 72 x 16 384 (24 576) 65, 56, 59;
             // 8 x 32 x 64 x 4160 (16 640) 50, 44, 48; 4 x 32 x 96 x 32 768 172 and 160 (four do not fit).  V: 8 x 32 x 96 x 4160
             // (12 480) 47, 39, 43; 4 x 32 x 96 x 32 768 (49 152) 141, 126, 119; 8 x 32 x 128 x 4096 (16 384) 53, 60, 47.
-            auto cost = [&](int r) { return (a.tiles + (int64_t)KVC_WIDE_WAVES * r - 1) / ((int64_t)KVC_WIDE_WAVES * r) * (5 * r + 6); };
             for (int r = 3; r <= 4 && small && run >= 2 && want == 1; r++)
-                if ((is_k ? r * image <= sa.e.wave_bytes : (r - 1) * image <= sa.e.wave_bytes - KVC_STAGE_VPACKED_BYTES) && cost(r) <= cost(run)) run = r;
+                if ((is_k ? r * image <= sa.e.wave_bytes : (r - 1) * image <= sa.e.wave_bytes - KVC_STAGE_VPACKED_BYTES) && kvc_runs_cost(a.tiles, r, nullptr) <= kvc_runs_cost(a.tiles, run, nullptr)) run = r;
         } else if (wide && small && run == 2 && want == 1 && !is_k && a.tiles > 2 * KVC_WIDE_WAVES && 3 * image <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) {
             run = 4;
         }
-        const unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
+        unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
         const auto symbols_kernel = kvc_symbols_kernel(is_k, a.vec_len, !c.packed ? KVC_FORM_BYTES : c.longest_code >= 1 && c.longest_code <= 8 ? KVC_FORM_PACKED : KVC_FORM_PACKED_LONG);
         if (wide) {
             // Where the runs are more than one round of the waves, the first round's workgroups draw the others' too (kernel against
             // kernel in first stores of K and V, us: 4 x 32 x 96 x 32 768 159 + 115 -> 146 + 107; whole first stores: 2 x 32 x 128 x 8192
             // 280 -> 247, 4 x 24 x 72 x 9000 265 -> 237, 4 x 32 x 128 x 9000 390 -> 346).
-            const unsigned resident = KVC_WIDE_WAVES / (unsigned)waves;
-            const int persistent = waves == 2 * KVC_WAVES_PER_WG && wgs1 > resident;
-            hipLaunchKernelGGL(symbols_kernel, dim3(persistent ? resident : wgs1), dim3(waves * KVC_WAVE), lds, stream, sa.e, run, persistent);
+            // Where the runs are more than one round of the waves, the first round's workgroups draw the others' too (kernel against
+            // kernel in first stores of K and V, us: 4 x 32 x 96 x 32 768 159 + 115 -> 146 + 107; whole first stores: 2 x 32 x 128 x 8192
+            // 280 -> 247, 4 x 24 x 72 x 9000 265 -> 237, 4 x 32 x 128 x 9000 390 -> 346).  What whole rounds leave over goes in shorter runs
+            // where those end sooner: 4 x 32 x 128 x 9000 (17 920 tiles) 55.9 + 55.2 -> 54.2 + 53.8.
+            int short_run = 0, short_from = 0x7fffffff;
+            size_t wide_lds = lds;
+            if (waves == 2 * KVC_WAVES_PER_WG && wgs1 > KVC_WIDE_WAVES / waves) {
+                waves = 4 * KVC_WAVES_PER_WG;
+                wide_lds = 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
+                wgs1 = KVC_WIDE_WAVES / waves;
+                kvc_runs_cost(a.tiles, run, &short_run);
+                short_from = (int)(a.tiles / ((int64_t)KVC_WIDE_WAVES * run)) * (KVC_WIDE_WAVES / waves);
+            }
+            hipLaunchKernelGGL(symbols_kernel, dim3(wgs1), dim3(waves * KVC_WAVE), wide_lds, stream, sa.e, run, short_run, short_from);
             if (c.book) {
                 KvcPutSmallArgs put = {};
                 put.tree_at = (int)((c.book->encode_bytes + 15) / 16 * 16);
