@@ -6,6 +6,8 @@
 //   2. record each node's parent and incoming bit, then every leaf walks up to the root: that gives its
 //      code length, hence lmax, and the left-aligned code of every "long" code (length > lbits);
 //   3. every table index walks down from the root along its own bits until it meets a leaf.
+// All of it is waiting: for LDS, a read per step of a walk.  With a node in one word (leaf flag, then child: two reads after one
+// another before) and one walk for both tables, 7.6 -> 7.1 us of the launch behind a large first store and 7.1 -> 6.3 behind a small one.
 // A malformed tree (child index out of range, cycles) cannot hang or fault: walks are bounded by 32
 // steps and indices are range-checked; the affected entries stay 0 (= "no code").
 #pragma once
@@ -13,10 +15,11 @@
 
 __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ tree, int tree_bytes, int node_bytes, uint32_t *__restrict__ lut)
 {
-    __shared__ int16_t s_child[2][KVC_TREE_MAX_NODES];
-    __shared__ int16_t s_parent[KVC_TREE_MAX_NODES];
-    __shared__ uint8_t s_leaf[KVC_TREE_MAX_NODES];
-    __shared__ uint8_t s_bit[KVC_TREE_MAX_NODES];
+    // A step of a walk waits for one LDS read, so a node is one word: LEAF | symbol, or the two children, NONE where out of range; and so is
+    // its way up: its parent, NONE at the root, and the bit that leads to it.
+    constexpr uint32_t LEAF = 0x80000000u, NONE = 0x3ffu;
+    static_assert(KVC_TREE_MAX_NODES <= (int)NONE, "node numbers of ten bits");
+    __shared__ uint32_t s_node[KVC_TREE_MAX_NODES], s_up[KVC_TREE_MAX_NODES];
     __shared__ uint32_t s_lmax, s_nlong, s_nesc;
     __shared__ float s_avg;   // sum over leaves of len * 2^-len: the mean code length if the code is well matched
     __shared__ uint32_t s_symbits;   // OR over the symbols' fp16 patterns
@@ -40,18 +43,17 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
             }
             if (leaf) { a &= 0xff; b = a; }   // symbol value 0..255 (the int8 form stores it sign-wrapped)
         }
-        s_leaf[n] = (uint8_t)leaf;
-        s_child[0][n] = (int16_t)a;
-        s_child[1][n] = (int16_t)b;
-        s_parent[n] = -1;
-        s_bit[n] = (uint8_t)(n & 1);          // nodes 0 / 1 hang off the implicit root by bit 0 / 1
+        auto child = [&](int c) { return c >= 0 && c < n_nodes ? (uint32_t)c : NONE; };
+        s_node[n] = leaf ? LEAF | (uint32_t)a : child(a) | child(b) << 10;
+        s_up[n] = NONE | (uint32_t)(n & 1) << 10;         // nodes 0 / 1 hang off the implicit root by bit 0 / 1
     }
     __syncthreads();
     for (int n = tid; n < n_nodes; n += KVC_WG) {
-        if (s_leaf[n]) continue;
+        const uint32_t node = s_node[n];
+        if (node & LEAF) continue;
         for (int bit = 0; bit < 2; bit++) {
-            int c = s_child[bit][n];
-            if (c >= 2 && c < n_nodes) { s_parent[c] = (int16_t)n; s_bit[c] = (uint8_t)bit; }
+            const uint32_t c = (node >> (10 * bit)) & 0x3ffu;
+            if (c >= 2u && c != NONE) s_up[c] = (uint32_t)n | (uint32_t)bit << 10;
         }
     }
     __syncthreads();
@@ -62,15 +64,15 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
         int n = tid + k * KVC_WG;
         my_len[k] = 0;
         my_code[k] = 0;
-        if (n < n_nodes && s_leaf[n]) {
+        if (n < n_nodes && (s_node[n] & LEAF)) {
             uint32_t len = 0, code = 0;
             int cur = n;
             while (len < 33) {
-                code |= (uint32_t)s_bit[cur] << (len & 31);
+                const uint32_t up = s_up[cur];
+                code |= (up >> 10) << (len & 31);
                 len++;
-                int par = s_parent[cur];
-                if (par < 0) break;
-                cur = par;
+                if ((up & 0x3ffu) == NONE) break;
+                cur = (int)(up & 0x3ffu);
             }
             // a valid chain ends at node 0 or 1; anything else (orphan, over-long) is ignored
             if (len <= 32 && cur < 2) {
@@ -78,7 +80,7 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
                 my_code[k] = code;
                 atomicMax(&s_lmax, len);
                 atomicAdd(&s_avg, (float)len * exp2f(-(float)len));
-                const int sym = s_child[0][n] & 0xff;
+                const int sym = (int)(s_node[n] & 0xffu);
                 atomicOr(&s_symbits, (uint32_t)__half_as_ushort(__float2half_rn((float)sym)) | (sym > 16 ? KVC_LUT_WIDE_SYMBOLS : 0u));
             }
         }
@@ -92,7 +94,7 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
             const uint32_t slot = atomicAdd(&s_nesc, 1u);
             if (slot < (uint32_t)KVC_LUT_ESC_MAX) {
                 lut[KVC_LUT_ESC_OFFSET + 2 * slot] = __brev(my_code[k] << (32 - my_len[k]));
-                lut[KVC_LUT_ESC_OFFSET + 2 * slot + 1] = my_len[k] | ((uint32_t)(s_child[0][tid + k * KVC_WG] & 0xff) << 8);
+                lut[KVC_LUT_ESC_OFFSET + 2 * slot + 1] = my_len[k] | ((s_node[tid + k * KVC_WG] & 0xffu) << 8);
             }
         }
         if (my_len[k] > lbits) {
@@ -100,35 +102,29 @@ __device__ __forceinline__ void kvc_build_lut_body(const uint8_t *__restrict__ t
             if (slot < (uint32_t)KVC_LUT_MAX_LONG) {
                 int n = tid + k * KVC_WG;
                 lut[KVC_LUT_HEADER_WORDS + 2 * slot] = my_code[k] << (32 - my_len[k]);
-                lut[KVC_LUT_HEADER_WORDS + 2 * slot + 1] = my_len[k] | ((uint32_t)(s_child[0][n] & 0xff) << 8);
+                lut[KVC_LUT_HEADER_WORDS + 2 * slot + 1] = my_len[k] | ((s_node[n] & 0xffu) << 8);
             }
         }
     }
-    // table entries: walk down along the index bits
+    // table entries: walk down along the index bits.  The fused kernels' entry is that of the reversed index: their index bits are the
+    // stream bits in arrival order from bit 0 up (they keep their window least-significant-bit first).
     uint32_t *entries = lut + KVC_LUT_HEADER_WORDS + KVC_LUT_LONG_WORDS;
     for (uint32_t idx = tid; idx < (1u << lbits); idx += KVC_WG) {
-        uint32_t e = 0;
-        int cur = (int)((idx >> (lbits - 1)) & 1u);
+        uint32_t e = 0, fused = 1u;            // no code / code longer than the index: none, and "symbol 0, length 1"
+        uint32_t cur = (idx >> (lbits - 1)) & 1u;
         for (uint32_t depth = 1; depth <= lbits; depth++) {
-            if (cur < 0 || cur >= n_nodes) break;
-            if (s_leaf[cur]) { e = depth | ((uint32_t)(s_child[0][cur] & 0xff) << 8); break; }
+            if (cur >= (uint32_t)n_nodes) break;
+            const uint32_t node = s_node[cur];
+            if (node & LEAF) {
+                e = depth | (node & 0xffu) << 8;
+                fused = __float_as_uint((float)(node & 0xffu)) | depth;
+                break;
+            }
             if (depth == lbits) break;
-            cur = s_child[(idx >> (lbits - 1 - depth)) & 1u][cur];
+            cur = (node >> (10u * ((idx >> (lbits - 1 - depth)) & 1u))) & 0x3ffu;
         }
         entries[idx] = e;
-    }
-    // fused-kernel entries: the index bits are the stream bits in arrival order from bit 0 up (the fused
-    // kernels keep their window least-significant-bit first), so walk with bit j of the index at depth j
-    for (uint32_t idx = tid; idx < (1u << lbits); idx += KVC_WG) {
-        uint32_t e = 1u;                       // no code / code longer than the index: "symbol 0, length 1"
-        int cur = (int)(idx & 1u);
-        for (uint32_t depth = 1; depth <= lbits; depth++) {
-            if (cur < 0 || cur >= n_nodes) break;
-            if (s_leaf[cur]) { e = __float_as_uint((float)(s_child[0][cur] & 0xff)) | depth; break; }
-            if (depth == lbits) break;
-            cur = s_child[(idx >> depth) & 1u][cur];
-        }
-        lut[KVC_LUT_FENTRY_OFFSET + idx] = e;
+        lut[KVC_LUT_FENTRY_OFFSET + (__brev(idx) >> (32u - lbits))] = fused;
     }
     for (int i = KVC_LUT_NARROW_OFFSET + tid; i < KVC_LUT_WORDS; i += KVC_WG) lut[i] = 0u;
     __syncthreads();
