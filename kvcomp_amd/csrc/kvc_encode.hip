@@ -2220,16 +2220,16 @@ static int kvc_encode_errors(uint32_t bits, uint32_t total, int64_t encoded_cap)
 }
 
 // What the encoder from symbols takes for runs of `run` tiles, in fifths of a tile's time: its waves in whole rounds, and what is
-// left beyond those in shorter runs (`tail`) where that is less.  The waves that take their tiles in turn stay inside a group with
-// those too where the first of them starts at a multiple of their tiles.
+// left beyond those in shorter runs (`tail`) where that is less.  The waves that take their tiles in turn (four at most) stay inside a
+// group of `group` tiles with those too where they divide it and the first of them starts at a multiple of their tiles.
 constexpr int KVC_WIDE_WAVES = 4096;
-static int64_t kvc_runs_cost(int64_t tiles, int run, int *tail)
+static int64_t kvc_runs_cost(int64_t tiles, int run, int step, int group, int *tail)
 {
     auto rounds = [](int64_t t, int r) { return (t + (int64_t)KVC_WIDE_WAVES * r - 1) / ((int64_t)KVC_WIDE_WAVES * r) * (5 * r + 6); };
     const int64_t whole = tiles / ((int64_t)KVC_WIDE_WAVES * run) * run * KVC_WIDE_WAVES, rest = tiles - whole;
     int best = run;
     for (int r = run - 1; r >= 1; r--)
-        if (whole % (4 * r) == 0 && rounds(rest, r) < rounds(rest, best)) best = r;
+        if (whole % (step * r) == 0 && group % (step * r) == 0 && rounds(rest, r) < rounds(rest, best)) best = r;
     if (tail) *tail = best;
     return rounds(whole, run) + rounds(rest, best);
 }
@@ -2380,6 +2380,8 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         if (wide && small && want == 1 && a.tiles > KVC_WIDE_WAVES) run = 2;
         int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
+        // waves that take their tiles in turn, as the kernel's STEP
+        const int step = c.packed ? (is_k ? 1 : 4) : !is_k ? 2 : a.vec_len == 96 || a.vec_len == 72 ? 4 : a.vec_len == 64 ? 2 : 1;
         // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
         // together take stays inside a group, or the wave that speaks for a group would wait before all its tiles are counted).
         const int64_t image = a.encoded_cap / a.tiles * 9 / 8;
@@ -2390,16 +2392,13 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
             // 8 x 32 x 64 x 4160 (16 640) 50, 44, 48; 4 x 32 x 96 x 32 768 172 and 160 (four do not fit).  V: 8 x 32 x 96 x 4160
             // (12 480) 47, 39, 43; 4 x 32 x 96 x 32 768 (49 152) 141, 126, 119; 8 x 32 x 128 x 4096 (16 384) 53, 60, 47.
             for (int r = 3; r <= 4 && small && run >= 2 && want == 1; r++)
-                if ((is_k ? r * image <= sa.e.wave_bytes : (r - 1) * image <= sa.e.wave_bytes - KVC_STAGE_VPACKED_BYTES) && kvc_runs_cost(a.tiles, r, nullptr) <= kvc_runs_cost(a.tiles, run, nullptr)) run = r;
+                if ((is_k ? r * image <= sa.e.wave_bytes : (r - 1) * image <= sa.e.wave_bytes - KVC_STAGE_VPACKED_BYTES) && kvc_runs_cost(a.tiles, r, step, group_tiles, nullptr) <= kvc_runs_cost(a.tiles, run, step, group_tiles, nullptr)) run = r;
         } else if (wide && small && run == 2 && want == 1 && !is_k && a.tiles > 2 * KVC_WIDE_WAVES && 3 * image <= sa.e.wave_bytes - KVC_STAGE_VF16_BYTES) {
             run = 4;
         }
         unsigned wgs1 = (unsigned)((a.tiles + (int64_t)run * waves - 1) / ((int64_t)run * waves));
         const auto symbols_kernel = kvc_symbols_kernel(is_k, a.vec_len, !c.packed ? KVC_FORM_BYTES : c.longest_code >= 1 && c.longest_code <= 8 ? KVC_FORM_PACKED : KVC_FORM_PACKED_LONG);
         if (wide) {
-            // Where the runs are more than one round of the waves, the first round's workgroups draw the others' too (kernel against
-            // kernel in first stores of K and V, us: 4 x 32 x 96 x 32 768 159 + 115 -> 146 + 107; whole first stores: 2 x 32 x 128 x 8192
-            // 280 -> 247, 4 x 24 x 72 x 9000 265 -> 237, 4 x 32 x 128 x 9000 390 -> 346).
             // Where the runs are more than one round of the waves, the first round's workgroups draw the others' too (kernel against
             // kernel in first stores of K and V, us: 4 x 32 x 96 x 32 768 159 + 115 -> 146 + 107; whole first stores: 2 x 32 x 128 x 8192
             // 280 -> 247, 4 x 24 x 72 x 9000 265 -> 237, 4 x 32 x 128 x 9000 390 -> 346).  What whole rounds leave over goes in shorter runs
@@ -2410,7 +2409,7 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
                 waves = 4 * KVC_WAVES_PER_WG;
                 wide_lds = 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
                 wgs1 = KVC_WIDE_WAVES / waves;
-                kvc_runs_cost(a.tiles, run, &short_run);
+                kvc_runs_cost(a.tiles, run, step, group_tiles, &short_run);
                 short_from = (int)(a.tiles / ((int64_t)KVC_WIDE_WAVES * run)) * (KVC_WIDE_WAVES / waves);
             }
             hipLaunchKernelGGL(symbols_kernel, dim3(wgs1), dim3(waves * KVC_WAVE), wide_lds, stream, sa.e, run, short_run, short_from);

@@ -52,7 +52,9 @@ def _room(is_k, sym):
 
 # tiles a little beyond one round of 4096 waves' runs, beyond two and beyond three
 CASES = [(True, 64 * 129, 1, 64, 64), (True, 64 * 257, 1, 65, 64), (True, 64 * 131, 1, 67, 96), (True, 64 * 131, 1, 67, 72), (True, 64 * 385, 1, 65, 128),
-         (False, 128 * 129, 1, 130, 64), (False, 128 * 253, 1, 199, 64), (False, 128 * 131, 1, 67, 128)]
+         (False, 128 * 129, 1, 130, 64), (False, 128 * 253, 1, 199, 64), (False, 128 * 131, 1, 67, 128),
+         # three whole rounds, and a rest that runs of three would fill, which do not divide a group
+         (False, 128 * 300, 1, 197, 64)]
 
 
 @pytest.mark.parametrize("rare_tiles", [0.0, 0.2])
