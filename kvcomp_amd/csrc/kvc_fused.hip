@@ -1000,6 +1000,8 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
         if (a.table_words < 8) a.table_words = 8;
     }
     if (two_byte_table && a.pair_bits == 0 && a.narrow_pair_bits == 0) a.table_words = a.table_words > 8 ? a.table_words / 2 : 4;
+    // The refill at a stream's start reads the row before its column's first too (kvc_column_address): the first wave's lies in the table
+    if (columns && a.table_words < KVC_WAVE) a.table_words = KVC_WAVE;
     // per wave, besides the payload
     const int64_t ops_words = mfma_ops_words ? mfma_ops_words : (int64_t)slots * 128 * rep + extra_words;
     const int64_t budget = (65536 / 4 - a.table_words - slack) / KVC_WAVES_PER_WG - ops_words;   // words per wave
