@@ -1207,12 +1207,13 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     const bool mfma = want_mfma != 0 && max_code_bits >= 1 && (!long_codes || (rounded && kvc_hint_small_alphabet(code_hint) && kind != 1 && kind != 2)) &&
                       kvc_option(KVC_OPT_FUSED_ROWS) != 1 && ((uintptr_t)d_out & 15) == 0 &&
                       (is_k ? out_stride % 4 == 0 : head_dim % 4 == 0);
+    const bool columns = mfma && kvc_mfma_columns((int)rep, is_k != 0, long_codes);
     // codes of 6 or 7 bits, symbols of at most 16, one per look-up: kernels of their own too
-    const bool mid_codes = mfma && rounded && !long_codes && max_code_bits >= 6 && kvc_hint_byte_symbols(code_hint) && kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0;
+    const bool mid_codes = mfma && rounded && !long_codes && max_code_bits >= 6 && columns && kvc_hint_byte_symbols(code_hint) && kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0;
     const size_t lds = mfma ? kvc_plan_lds(a, slots, (int)rep, encoded_bytes, rows * a.s.cols, max_tile_bytes, max_stream_bytes,
                                            max_code_bits, 0, !long_codes, kvc_mfma_ops_words(slots, (int)rep, rounded),
                                          long_codes ? KVC_LONG_TABLE_WORDS : 0, is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint),
-                                         mid_codes, !long_codes)
+                                         mid_codes, columns)
                             : kvc_plan_lds(a, slots, rounded ? (int)rep + 1 : (int)rep, encoded_bytes, rows * a.s.cols,
                                            max_tile_bytes, max_stream_bytes, max_code_bits, 0, !rounded);
     a.rounded = rounded;

@@ -684,6 +684,10 @@ __device__ __forceinline__ uint32_t kvc_column_address(uint32_t column, uint32_t
     asm("" : "+v"(row));                                                                  // (see kvc_refill_address)
     return (row << 8) + (column - 256u);
 }
+// Which matrix-core kernels have them: those for codes of at most 7 bits, but for V with eight query heads.  A wave there holds three to a
+// SIMD and waits for its one tile, and columns and one-byte entries made that longer (2 x 8 x 8 heads x 128 x 1905 tokens, K's codes
+// longer: 40.4 us packed, 41.3 in columns, 41.9 with both; 8 x 8 x 8 x 128 x 4096 59.2 : 60.3).
+constexpr bool kvc_mfma_columns(int rep, bool is_k, bool long_codes) { return !long_codes && (is_k || rep != 8); }
 enum { KVC_PACKED_PLAIN = 0, KVC_PACKED_SKEWED = 1, KVC_COLUMNS = 2 };
 // The three words of a refill.  base: kvc_refill_address's, or the lane's column.
 template <int LAYOUT>

@@ -603,8 +603,8 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     constexpr int SLOTS = KvcGeom<KIND>::SLOTS;
     constexpr int NM = kvc_mfma_sets(REP);
     using T = KvcMfmaTables<REP>;
-    // Codes of at most 7 bits: payloads in columns (kvc_fetch_streams); the kernels for longer ones decode packed payloads.
-    constexpr bool COLUMNS = !LONG;
+    // payloads in columns (kvc_fetch_streams), or packed
+    constexpr bool COLUMNS = kvc_mfma_columns(REP, IS_K, LONG);
     // dynamic LDS: the decode table (at offset 0, so that its address folds into the look-ups), then per wave:
     // operand tables, packed payload; in columns, all waves' payloads, then all waves' operand tables
     extern __shared__ __align__(16) uint32_t smem[];
