@@ -52,7 +52,7 @@ __device__ __forceinline__ void kvc_decode_bytes(uint32_t sbase, uint32_t u, uin
     constexpr int N = PAIRS ? 4 : 8;                             // look-ups per refill: 8 symbols, half from each half window
 #pragma unroll 1
     for (int i = 0; i < KVC_V_TOKENS / 8; i++) {
-        const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<false>(sbase, u);
+        const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)kvc_refill_address<false, true>(sbase, u);
         const uint32_t w0 = wp[0], w1 = wp[1], w2 = wp[2];
         const uint32_t lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
         uint32_t R = lo, es = 0;

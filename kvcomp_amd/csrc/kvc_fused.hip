@@ -1207,9 +1207,11 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     const bool mfma = want_mfma != 0 && max_code_bits >= 1 && (!long_codes || (rounded && kvc_hint_small_alphabet(code_hint) && kind != 1 && kind != 2)) &&
                       kvc_option(KVC_OPT_FUSED_ROWS) != 1 && ((uintptr_t)d_out & 15) == 0 &&
                       (is_k ? out_stride % 4 == 0 : head_dim % 4 == 0);
-    const bool columns = mfma && kvc_mfma_columns((int)rep, is_k != 0, long_codes);
-    // codes of 6 or 7 bits, symbols of at most 16, one per look-up: kernels of their own too
-    const bool mid_codes = mfma && rounded && !long_codes && max_code_bits >= 6 && columns && kvc_hint_byte_symbols(code_hint) && kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0;
+    // codes of 6 or 7 bits, symbols of at most 16, one per look-up: kernels of their own too (eight query heads: see kvc_mfma_columns)
+    const bool mid_codes = mfma && rounded && !long_codes && max_code_bits >= 6 && kvc_hint_byte_symbols(code_hint) && kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0 &&
+                           2 * max_code_bits > kvc_option(KVC_OPT_FUSED_PAIR_BITS) && (is_k || kvc_hint_pair_bits(code_hint) == 0) &&
+                           (rep != 8 || (is_k && rows * a.s.cols >= KVC_COLUMNS_REP8_TILES));
+    const bool columns = mfma && kvc_mfma_columns((int)rep, long_codes, mid_codes);
     const size_t lds = mfma ? kvc_plan_lds(a, slots, (int)rep, encoded_bytes, rows * a.s.cols, max_tile_bytes, max_stream_bytes,
                                            max_code_bits, 0, !long_codes, kvc_mfma_ops_words(slots, (int)rep, rounded),
                                          long_codes ? KVC_LONG_TABLE_WORDS : 0, is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint),
@@ -1246,7 +1248,7 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
     if (mfma) {
         if (trace_plan) fprintf(stderr, "[kvcomp]   matrix-core kernel\n");
         if (long_codes) kvc_launch_fused_long((int)rep, kind, a, grid, lds, stream);
-        else if (mid_codes && a.pair_bits == 0 && a.narrow_pair_bits == 0) kvc_launch_fused_mid((int)rep, kind, a, grid, lds, stream);
+        else if (mid_codes) kvc_launch_fused_mid((int)rep, kind, a, grid, lds, stream);
         else kvc_launch_fused_mfma((int)rep, kind, rounded != 0, a, grid, lds, stream);
         KVC_HIP(hipGetLastError());
         return timer.finish();

@@ -159,17 +159,14 @@ static inline bool kvc_streams_resonate(int64_t encoded_bytes, int64_t tiles)
 // by more than 128 symbols x 10 bits, and the workgroup's LDS ends with that much slack (KVC_LDS_SLACK_WORDS),
 // so even a corrupt stream only ever reads this workgroup's own LDS.
 typedef __attribute__((address_space(3))) uint32_t kvc_lds_word;
-template <bool SKEW>
+// WORD: left to itself the compiler makes "u >> 3 & ~3" of the word's address, an instruction more than shift and shifted add.  1 x 8 x 4 heads x
+// 128 x 1000 tokens 16.64 -> 16.47 us; but with codes of more than 7 bits 2 x 8 x 8 x 128 x 1905 takes 41.0 us for 40.6.
+template <bool SKEW, bool WORD = false>
 __device__ __forceinline__ uint32_t kvc_refill_address(uint32_t stage_base, uint32_t u)
 {
     uint32_t a = u >> 5;
-    // (left to itself the compiler makes "u >> 3 & ~3" of the word's address: an instruction more, with the skew two)
-    asm("" : "+v"(a));
-    if (SKEW) {
-        uint32_t run = u >> 10;
-        asm("" : "+v"(run));
-        return (a << 2) + ((run << 3) + stage_base);                      // + 2 words per 32
-    }
+    if (WORD) asm("" : "+v"(a));
+    if (SKEW) return (a << 2) + (__umul24(u >> 10, 8u) + stage_base);     // + 2 words per 32
     return (a << 2) + stage_base;
 }
 constexpr int KVC_LDS_SLACK_WORDS = 48;
@@ -684,17 +681,19 @@ __device__ __forceinline__ uint32_t kvc_column_address(uint32_t column, uint32_t
     asm("" : "+v"(row));                                                                  // (see kvc_refill_address)
     return (row << 8) + (column - 256u);
 }
-// Which matrix-core kernels have them: those for codes of at most 7 bits, but for V with eight query heads.  A wave there holds three to a
-// SIMD and waits for its one tile, and columns and one-byte entries made that longer (2 x 8 x 8 heads x 128 x 1905 tokens, K's codes
-// longer: 40.4 us packed, 41.3 in columns, 41.9 with both; 8 x 8 x 8 x 128 x 4096 59.2 : 60.3).
-constexpr bool kvc_mfma_columns(int rep, bool is_k, bool long_codes) { return !long_codes && (is_k || rep != 8); }
+// Which matrix-core kernels have them: those for codes of at most 7 bits; with eight query heads only K's for one-byte entries.  A wave with
+// that many heads holds three or four to a SIMD, and in caches of few tiles it waits for its one tile, which columns and one-byte
+// entries made longer (2 x 8 x 8 heads x 128 x 1905 tokens, K's codes longer: V packed 40.4 us, in columns 41.3, with both 41.9; 8 x 8 x 8 x 128 x
+// 4096 59.2 : 60.3; 2 x 8 x 8 x 96 x 4000, K in both 33.9, in neither 33.5).  K of many tiles gains: 8 x 8 x 8 x 96 x 8192 80.6 -> 74.3.
+constexpr int64_t KVC_COLUMNS_REP8_TILES = 4096;
+constexpr bool kvc_mfma_columns(int rep, bool long_codes, bool mid_codes) { return mid_codes || (!long_codes && rep != 8); }
 enum { KVC_PACKED_PLAIN = 0, KVC_PACKED_SKEWED = 1, KVC_COLUMNS = 2 };
 // The three words of a refill.  base: kvc_refill_address's, or the lane's column.
-template <int LAYOUT>
+template <int LAYOUT, bool WORD = true>
 __device__ __forceinline__ void kvc_refill(uint32_t base, uint32_t u, uint32_t &w0, uint32_t &w1, uint32_t &w2)
 {
     constexpr int STEP = LAYOUT == KVC_COLUMNS ? KVC_WAVE : 1;
-    const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)(LAYOUT == KVC_COLUMNS ? kvc_column_address(base, u) : kvc_refill_address<LAYOUT == KVC_PACKED_SKEWED>(base, u));
+    const kvc_lds_word *wp = (const kvc_lds_word *)(uintptr_t)(LAYOUT == KVC_COLUMNS ? kvc_column_address(base, u) : kvc_refill_address<LAYOUT == KVC_PACKED_SKEWED, WORD>(base, u));
     w0 = wp[0];
     w1 = wp[STEP];
     w2 = wp[2 * STEP];

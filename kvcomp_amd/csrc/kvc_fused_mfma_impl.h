@@ -462,7 +462,7 @@ __device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, u
 #pragma unroll 1
     for (int i = 0; i < n; i += 8) {
         uint32_t w0, w1, w2;
-        kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
+        kvc_refill<LAYOUT, false>(sbase, u, w0, w1, w2);
         uint32_t lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
         uint32_t R = lo, es = 0;
         uint32_t e[4];
@@ -477,7 +477,7 @@ __device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, u
             uint32_t f = *(const kvc_lds_u16 *)(uintptr_t)((R & mask) | fe);
             if (__builtin_expect(__any(f == 0u), 0)) {           // wave-uniform
                 u += es & 31u;
-                kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
+                kvc_refill<LAYOUT, false>(sbase, u, w0, w1, w2);
                 // the 32 bits from the code on (the window starts a bit before it)
                 const uint32_t win = __builtin_amdgcn_alignbit(__builtin_amdgcn_alignbit(w2, w1, u), __builtin_amdgcn_alignbit(w1, w0, u), 1u);
                 uint32_t len = f & 31u;
@@ -494,7 +494,7 @@ __device__ __forceinline__ void kvc_mfma_dot_long(uint32_t sbase, uint32_t &u, u
                 }
                 u += len;
                 es = 0;
-                kvc_refill<LAYOUT>(sbase, u, w0, w1, w2);
+                kvc_refill<LAYOUT, false>(sbase, u, w0, w1, w2);
                 lo = __builtin_amdgcn_alignbit(w1, w0, u), hi = __builtin_amdgcn_alignbit(w2, w1, u);
                 R = lo;
             } else {
@@ -604,7 +604,7 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     constexpr int NM = kvc_mfma_sets(REP);
     using T = KvcMfmaTables<REP>;
     // payloads in columns (kvc_fetch_streams), or packed
-    constexpr bool COLUMNS = kvc_mfma_columns(REP, IS_K, LONG);
+    constexpr bool COLUMNS = kvc_mfma_columns(REP, LONG, MID);
     // dynamic LDS: the decode table (at offset 0, so that its address folds into the look-ups), then per wave:
     // operand tables, packed payload; in columns, all waves' payloads, then all waves' operand tables
     extern __shared__ __align__(16) uint32_t smem[];

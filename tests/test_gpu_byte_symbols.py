@@ -73,3 +73,17 @@ def test_symbols_beyond_what_the_hint_states_take_the_slow_path():
         type(kc).code_hint = hint
     # the slow path's products are added up one by one in fp32: 128 roundings of 2^-24, then fp16's 2^-11
     assert (got.float() - want.float()).abs().max() <= 1e-3 * want.float().abs().max()
+
+
+@pytest.mark.parametrize("T", [32704, 32768])           # K tiles either side of the line from which eight query heads have kernels of their own
+def test_eight_query_heads(T):
+    from kvcomp_amd import _lib
+    kc, _ = _contexts(T, 1, 8, 64, 11)
+    assert kc.code_hint & 0x200 and kc.max_code_bits in (6, 7) and (kc.compressed_ctx_len // 64 * 8 >= 4096) == (T == 32768)
+    q = S.synth_q(1, 64, 64).to(DEV)
+    got = kc.mat_vec_mul(q)[0]
+    was = _lib.set_option("fused_half_table", 0)
+    try:
+        assert torch.equal(kc.mat_vec_mul(q)[0], got)
+    finally:
+        _lib.set_option("fused_half_table", was)
