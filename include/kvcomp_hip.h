@@ -65,7 +65,8 @@ int kvc_abi_version(void);
  *   "fused_skew":           -1 (default) decided per call: the tile payload is staged with two spare words after
  *                           every 32 when the mean stream length would otherwise line the lanes up on a few LDS
  *                           banks; 0 never; 1 always (where payloads are packed: the fp32-FMA kernels, the plain decoders and codes of
- *                           more than 7 bits; the others keep every lane's words in a bank of their own).
+ *                           more than 7 bits, and most kernels for eight query heads per KV head; the others keep every lane's
+ *                           words in a bank of their own).
  *   "fused_tiles_per_wave":  0 (default) chosen per call; n > 0: consecutive tiles one wave works through.
  *   "fused_pair_bits":       widest index of the two-symbols-per-look-up table (default 8; 0 = one symbol per look-up).
  *   "fused_double_window":   1 (default): 64 stream bits per refill in the one-symbol loops; 0: 32.
