@@ -381,6 +381,9 @@ class KVCompCtx:
             books = self._unverified[good - 1].books
             infos = self._block_infos.data[:books[0]].cpu().view(torch.int32)            # {offset, byte_num} per tile
             self.max_tile_bytes = max(self.max_tile_bytes, int((infos[1::2] & 0xffff).max()))
+            # thread_infos: the byte of its tile where each lane's stream ends, above three bits
+            ends = (self._thread_infos.data[:books[1]].cpu().view(torch.int16).int() & 0xffff).view(-1, 64) >> 3
+            self.max_stream_bytes = max(self.max_stream_bytes, int(ends.diff(prepend=ends.new_zeros(len(ends), 1)).max()))
             self._verified = books + ((int(infos[-2]) & 0xffffffff) + (int(infos[-1]) & 0xffff),)
         (self._block_infos.used, self._thread_infos.used, self._min_ints.used, self._scales.used, self.compressed_ctx_len,
          self._encoded.used) = self._verified

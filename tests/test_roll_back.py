@@ -82,3 +82,42 @@ def test_a_second_store_that_fails_right_behind_the_prompt():
     assert ctx.ctx_len == 64 * 13 and ctx.compressed_ctx_len == 64 * 12 and torch.equal(ctx.buffer, wide)
     assert torch.equal(ctx.get()[0], torch.cat([flat, wide]))
     assert ctx.encoded_data.numel() == good.numel() and torch.equal(ctx.encoded_data, good)
+
+
+def test_what_is_kept_says_how_long_its_streams_are(monkeypatch):
+    """A prompt that nobody has looked at stays when the store behind it fails; the hint that the decoders' LDS is planned by covers its
+    longest stream."""
+    from kvcomp_amd import _lib
+    _config()
+    ctx = KVCompCtx(True, 1, 2, 64, 0.1)
+    ctx.async_store = True
+    book = _lib.Codebook(tree_format=5, max_code_bits=7, payload_bits=8 * 100000)
+    lengths = torch.randint(9, 40, (12, 64), generator=torch.Generator().manual_seed(3))
+    lengths[7, 0], lengths[9, 63] = 55, 51
+    calls = []
+
+    def encode(is_k, *, tokens, block_infos, thread_infos, encoded, **kw):
+        if not calls:                                             # the second call fails and leaves nothing
+            ends = lengths.cumsum(1)
+            at = torch.cat([torch.zeros(1, dtype=torch.int64), ends[:, -1].cumsum(0)])
+            for i in range(12):
+                block_infos[8 * i:8 * i + 8] = torch.frombuffer(bytearray(struct.pack("<IHH", int(at[i]), int(ends[i, -1]), 0)), dtype=torch.uint8)
+            thread_infos[:12 * 128] = ((ends << 3) + 5).to(torch.int16).view(torch.uint8).flatten()
+        calls.append(tokens)
+    monkeypatch.setattr(kvcomp_cuda, "quant_codebook", lambda x, *a: (x.to(torch.uint8), book))
+    monkeypatch.setattr(kvcomp_cuda, "put_codebook", lambda *a: tuple(torch.zeros(24, dtype=torch.uint8) for _ in range(3)))
+    monkeypatch.setattr(kvcomp_cuda, "encode_async", encode)
+    monkeypatch.setattr(KVCompCtx, "_issue_probe", lambda self: None)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    ctx._encoded.reserve(1 << 20, (), torch.uint8, torch.device("cpu"))
+    x = torch.zeros(512, 1, 2, 64, dtype=torch.float16)
+    ctx.store(x[:384], want_symbols=False)
+    ctx.store(x[384:], want_symbols=False)
+    assert calls == [384, 128]
+
+    def failed(*a):
+        raise KvcompError("a symbol has no code")
+    monkeypatch.setattr(kvcomp_cuda, "encode_result", failed)
+    with pytest.raises(KvcompError, match="no code"):
+        ctx.encoded_data
+    assert ctx.compressed_ctx_len == 384 and ctx.max_tile_bytes == int(lengths.sum(1).max()) and ctx.max_stream_bytes == 55
