@@ -11,6 +11,7 @@ reference's get_cr(), models/cache/kvcomp_encode.py:317-326, for K and V togethe
 One JSON line goes to stdout; progress goes to stderr.
 """
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -653,7 +654,6 @@ def main():
                 "k_ms": k_ms, "v_ms": v_ms, "out": out}
 
     if args.copy_calibration:
-        import ctypes
         src = torch.empty(256 << 20, dtype=torch.uint8, device=dev).fill_(1)
         dst = torch.empty_like(src)
         _lib.check(_lib.lib().kvc_calibration_copy(ctypes.c_void_p(dst.data_ptr()), ctypes.c_void_p(src.data_ptr()),
@@ -742,10 +742,11 @@ def main():
     # template arguments: query heads per KV head, then 0 = K tile, 3 / 4 = V tile with the softmax on the fly
     # (4: head_dim is not a multiple of 64, tiles may straddle two heads), then rounded mode
     v_kind = 3 if D % 64 == 0 else 4
-    # (the last template argument: 2 codes of more than 7 bits, 1 codes of 6 or 7 bits of symbols up to 16, one per look-up)
-    book = lambda kind, ctx: 2 if ctx.max_code_bits > 7 else 1 if ctx.max_code_bits >= 6 and ctx.code_hint & 0x200 and not (kind and ctx.pair_bits) else 0
-    name = lambda kind, ctx: "kvc_fused_mfma_kernel<%d, %d, true, %d>" % (rep, kind, book(kind, ctx))
-    dom, dom_ms, dom_bytes = ((name(0, kctx), k_ms, kb) if k_ms >= v_ms else (name(v_kind, vctx), v_ms, vb))
+    # (the last template argument: which codes and layout of payloads, KVC_BOOK_* of kvc_fused_common.h)
+    books = _lib.lib().kvc_attention_kernels(
+        ctypes.byref(kctx.descriptor()), ctypes.byref(vctx.descriptor()), *(ctypes.c_int64(n) for n in (B, H, Hq, D)))
+    name = lambda kind: "kvc_fused_mfma_kernel<%d, %d, true, %d>" % (rep, kind, books >> (4 if kind else 0) & 15)
+    dom, dom_ms, dom_bytes = ((name(0), k_ms, kb) if k_ms >= v_ms else (name(v_kind), v_ms, vb))
     achieved = dom_bytes / dom_ms / 1e6
     value = (kb + vb) / (ms_per_step * 1e-3) / 1e9
     result = {

@@ -62,11 +62,13 @@ int kvc_abi_version(void);
  * variable KVCOMP_<NAME IN CAPITALS>, read once on first use.
  *   "fused_rows":           1: the fused decoders re-lay a tile's lane streams as LDS rows an odd number of words
  *                           apart whenever they fit; otherwise (default -1) never.
- *   "fused_skew":           -1 (default) decided per call: the tile payload is staged with two spare words after
- *                           every 32 when the mean stream length would otherwise line the lanes up on a few LDS
- *                           banks; 0 never; 1 always (where payloads are packed: the fp32-FMA kernels, the plain decoders and codes of
- *                           more than 7 bits, and most kernels for eight query heads per KV head; the others keep every lane's
- *                           words in a bank of their own).
+ *   "fused_skew":           how a tile's payload lies in LDS.  -1 (default) decided per call: in columns, every lane's words in a
+ *                           bank of their own, in the matrix-core kernels for codes of at most 7 bits where the cache has
+ *                           some thousand tiles and no stream is so long that the columns would leave the LDS to few
+ *                           workgroups; else packed, with two spare words after every 32 when the mean stream length
+ *                           would otherwise line the lanes up on a few LDS banks.  0: packed without spare words; 1: packed
+ *                           with them; 2: in columns wherever there are such kernels.  (Decode attention in one launch and
+ *                           the expanding decoders have layouts of their own or pack.)
  *   "fused_tiles_per_wave":  0 (default) chosen per call; n > 0: consecutive tiles one wave works through.
  *   "fused_pair_bits":       widest index of the two-symbols-per-look-up table (default 8; 0 = one symbol per look-up).
  *   "fused_double_window":   1 (default): 64 stream bits per refill in the one-symbol loops; 0: 32.

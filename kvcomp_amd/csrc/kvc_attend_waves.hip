@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(KVC_WG, REP == 8 ? 3 : 4) kvc_attend_waves_ker
         }
     }
     KvcRaw<REP, 1, 1> raw[T];
-    KvcStaged st[T], st_v[T];
+    KvcStreams st[T], st_v[T];
     KvcTilePos pos = {0, bh, b, h, 0};
     if (active) {
 #pragma unroll

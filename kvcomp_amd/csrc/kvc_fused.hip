@@ -1035,7 +1035,7 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
     const bool resonant = kvc_streams_resonate(encoded_bytes, tiles);
     const bool use_rows = force_rows == 1 && pack_rows + KVC_WAVE * row <= budget;
     const int force_skew = kvc_option(KVC_OPT_FUSED_SKEW);
-    const bool use_skew = !use_rows && (force_skew >= 0 ? force_skew != 0 : resonant);
+    const bool use_skew = !use_rows && (force_skew == 0 || force_skew == 1 ? force_skew != 0 : resonant);
     a.row_words = 0;
     a.skew = 0;
     if (use_rows) {
@@ -1049,6 +1049,43 @@ static size_t kvc_plan_lds(KvcFusedArgs &a, int slots, int rep, int64_t encoded_
     a.pack_words = (int)physical(pack);
     return 4 * ((size_t)a.table_words + (size_t)slack +
                 (size_t)KVC_WAVES_PER_WG * (size_t)(ops_words + a.pack_words + KVC_WAVE * a.row_words));
+}
+
+// Which kernels a call takes, and their LDS (left in `a` as well).
+struct KvcFusedPlan {
+    int book;            // KVC_BOOK_*; KVC_NO_BOOK: the fp32-FMA kernels
+    size_t lds;
+};
+constexpr int KVC_NO_BOOK = 4;
+static KvcFusedPlan kvc_plan_fused(KvcFusedArgs &a, bool is_k, int kind, int rep, bool rounded, int64_t tiles, int64_t encoded_bytes, int64_t max_tile_bytes,
+                                   int64_t max_stream_bytes, int64_t code_hint, bool stored_by_fours)
+{
+    // The matrix-core kernels take the common case: a codebook whose longest code is known, results that can be stored four at a time.
+    const int slots = is_k || kind == 1 || kind == 3 ? 1 : 2;
+    const int max_code_bits = kvc_hint_bits(code_hint);
+    // longer codes: kernels of their own, where a list of at most 64 codes and the entries' format are sure to do
+    const bool long_codes = max_code_bits > KVC_LUT_ESC_BITS;
+    const bool mfma = kvc_option(KVC_OPT_FUSED_MFMA) != 0 && max_code_bits >= 1 &&
+                      (!long_codes || (rounded && kvc_hint_small_alphabet(code_hint) && kind != 1 && kind != 2)) &&
+                      kvc_option(KVC_OPT_FUSED_ROWS) != 1 && stored_by_fours;
+    if (!mfma)
+        return {KVC_NO_BOOK, kvc_plan_lds(a, slots, rounded ? rep + 1 : rep, encoded_bytes, tiles, max_tile_bytes, max_stream_bytes, max_code_bits, 0, !rounded)};
+    // codes of 6 or 7 bits, symbols of at most 16, one per look-up: kernels of their own too, in columns
+    const bool byte_entries = rounded && !long_codes && max_code_bits >= 6 && kvc_hint_byte_symbols(code_hint) && kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0 &&
+                              2 * max_code_bits > kvc_option(KVC_OPT_FUSED_PAIR_BITS) && (is_k || kvc_hint_pair_bits(code_hint) == 0);
+    auto plan = [&](bool columns) {
+        return kvc_plan_lds(a, slots, rep, encoded_bytes, tiles, max_tile_bytes, max_stream_bytes, max_code_bits, 0, !long_codes,
+                            kvc_mfma_ops_words(slots, rep, rounded), long_codes ? KVC_LONG_TABLE_WORDS : 0,
+                            is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint), columns && byte_entries, columns);
+    };
+    const int want = kvc_option(KVC_OPT_FUSED_SKEW);
+    // (a layout that was asked for; else packed without the longest stream's length, which would decide which tiles the LDS holds)
+    if (!long_codes && (rep != 8 || (is_k && byte_entries)) &&
+        (want == 2 || (want < 0 && max_stream_bytes > 0 && tiles >= kvc_columns_from(is_k, rep, byte_entries, rounded)))) {
+        const size_t lds = plan(true);
+        if (want == 2 || kvc_lds_workgroups(lds) >= kvc_columns_workgroups(rep, slots)) return {byte_entries ? KVC_BOOK_MID : KVC_BOOK_SHORT, lds};
+    }
+    return {long_codes ? KVC_BOOK_LONG : KVC_BOOK_PACKED, plan(false)};
 }
 
 // Consecutive tiles of a row that one wave works through (fetching one ahead): as many as still leave
@@ -1197,27 +1234,10 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
         if (int rc = kvc_launch_v_small_heads((int)rep, a, rows, stream)) return rc;
         return timer.finish();
     }
-    // The matrix-core kernels take the common case: a codebook whose longest code is known, the plain or
-    // skewed packed payload, results that can be stored four at a time.
-    const int64_t out_stride = (extra && extra->out_stride) ? extra->out_stride : tokens;
-    const int want_mfma = kvc_option(KVC_OPT_FUSED_MFMA);
-    const int max_code_bits = kvc_hint_bits(code_hint);
-    // longer codes: kernels of their own, where a list of at most 64 codes and the entries' format are sure to do
-    const bool long_codes = max_code_bits > KVC_LUT_ESC_BITS;
-    const bool mfma = want_mfma != 0 && max_code_bits >= 1 && (!long_codes || (rounded && kvc_hint_small_alphabet(code_hint) && kind != 1 && kind != 2)) &&
-                      kvc_option(KVC_OPT_FUSED_ROWS) != 1 && ((uintptr_t)d_out & 15) == 0 &&
-                      (is_k ? out_stride % 4 == 0 : head_dim % 4 == 0);
-    // codes of 6 or 7 bits, symbols of at most 16, one per look-up: kernels of their own too (eight query heads: see kvc_mfma_columns)
-    const bool mid_codes = mfma && rounded && !long_codes && max_code_bits >= 6 && kvc_hint_byte_symbols(code_hint) && kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0 &&
-                           2 * max_code_bits > kvc_option(KVC_OPT_FUSED_PAIR_BITS) && (is_k || kvc_hint_pair_bits(code_hint) == 0) &&
-                           (rep != 8 || (is_k && rows * a.s.cols >= KVC_COLUMNS_REP8_TILES));
-    const bool columns = mfma && kvc_mfma_columns((int)rep, long_codes, mid_codes);
-    const size_t lds = mfma ? kvc_plan_lds(a, slots, (int)rep, encoded_bytes, rows * a.s.cols, max_tile_bytes, max_stream_bytes,
-                                           max_code_bits, 0, !long_codes, kvc_mfma_ops_words(slots, (int)rep, rounded),
-                                         long_codes ? KVC_LONG_TABLE_WORDS : 0, is_k || long_codes ? 0 : kvc_hint_pair_bits(code_hint),
-                                         mid_codes, columns)
-                            : kvc_plan_lds(a, slots, rounded ? (int)rep + 1 : (int)rep, encoded_bytes, rows * a.s.cols,
-                                           max_tile_bytes, max_stream_bytes, max_code_bits, 0, !rounded);
+    const KvcFusedPlan plan = kvc_plan_fused(a, is_k, kind, (int)rep, rounded, rows * a.s.cols, encoded_bytes, max_tile_bytes, max_stream_bytes, code_hint,
+                                             ((uintptr_t)d_out & 15) == 0 && (is_k ? a.out_stride % 4 == 0 : head_dim % 4 == 0));
+    const bool mfma = plan.book != KVC_NO_BOOK;
+    const size_t lds = plan.lds;
     a.rounded = rounded;
     // V tiles after which the heads repeat (the kernels that keep a head's operand tables from tile to tile)
     int unit = 0;
@@ -1247,8 +1267,9 @@ static int kvc_fused(int is_k, const uint8_t *d_decode_tree, int64_t decode_tree
                 a.table_words, a.pack_words, a.pack_logical, a.skew, a.row_words, a.column_rows, a.pair_bits, a.s.tiles_per_wave, a.rounded);
     if (mfma) {
         if (trace_plan) fprintf(stderr, "[kvcomp]   matrix-core kernel\n");
-        if (long_codes) kvc_launch_fused_long((int)rep, kind, a, grid, lds, stream);
-        else if (mid_codes) kvc_launch_fused_mid((int)rep, kind, a, grid, lds, stream);
+        if (plan.book == KVC_BOOK_LONG) kvc_launch_fused_long((int)rep, kind, a, grid, lds, stream);
+        else if (plan.book == KVC_BOOK_MID) kvc_launch_fused_mid((int)rep, kind, a, grid, lds, stream);
+        else if (plan.book == KVC_BOOK_PACKED) kvc_launch_fused_packed((int)rep, kind, rounded != 0, a, grid, lds, stream);
         else kvc_launch_fused_mfma((int)rep, kind, rounded != 0, a, grid, lds, stream);
         KVC_HIP(hipGetLastError());
         return timer.finish();
@@ -1888,6 +1909,21 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
 #undef KVC_COMBINE
     KVC_HIP(hipGetLastError());
     return timer.finish();
+}
+
+// Which kernels a kvc_attention_decode of these caches takes, without running it (nothing is read through the descriptors' pointers): K's
+// KVC_BOOK_* (KVC_NO_BOOK) where two kernels decode K and V, V's << 4.
+extern "C" int kvc_attention_kernels(const kvc_compressed_desc *k, const kvc_compressed_desc *v, int64_t batch, int64_t kv_heads, int64_t q_heads,
+                                     int64_t head_dim)
+{
+    const int rep = (int)(q_heads / kv_heads);
+    const bool rounded = kvc_option(KVC_OPT_FUSED_ROUNDED) != 0;
+    KvcFusedArgs a = {};
+    auto book = [&](const kvc_compressed_desc *c, bool is_k, int64_t tiles) {
+        const int kind = is_k ? 0 : head_dim % KVC_WAVE == 0 ? 3 : 4;
+        return kvc_plan_fused(a, is_k, kind, rep, rounded, tiles, c->encoded_bytes, c->max_tile_bytes, c->max_stream_bytes, c->max_code_bits, true).book;
+    };
+    return book(k, true, k->tokens / KVC_WAVE * batch * kv_heads) | book(v, false, kvc_v_tiles(v, batch, kv_heads, head_dim)) << 4;
 }
 
 extern "C" int kvc_attention_decode(const kvc_compressed_desc *k, const kvc_compressed_desc *v, const void *d_q_f16,

@@ -493,14 +493,21 @@ __device__ __forceinline__ float kvc_half_bits_to_float(uint32_t bits16)
     return __half2float(__ushort_as_half((unsigned short)bits16));
 }
 
+// Workgroups that a compute unit's LDS holds (160 KiB, handed out in pieces of 1280 bytes)
+static inline int kvc_lds_workgroups(size_t lds) { return (int)(163840 / ((lds + 1279) / 1280 * 1280)); }
+
 // What the decode step needs to know about a staged tile.
-struct KvcStaged {
-    int fits;             // staged in LDS (wave-uniform); otherwise decode from global memory  (no bool: copies of the struct's padding
-                          // would go through scratch memory)
+template <class Flag>
+struct KvcStagedAs {
+    Flag fits;            // staged in LDS (wave-uniform); otherwise decode from global memory
     uint32_t u0;          // fast-path start position (`lb` bits before the first code) in the lane's LDS words
     const uint32_t *gwords;   // the lane's stream in global memory, from the aligned word holding its first byte
     uint32_t gnwords, gpos;
 };
+// A bool is a bit per lane in scalar registers, an int a vector register; but copies of the struct with a bool, whose padding is copied
+// too, would go through scratch memory: streams in columns are copied.
+using KvcStaged = KvcStagedAs<bool>;
+using KvcStreams = KvcStagedAs<int>;
 
 // Move a fetched tile's payload into the wave's packed LDS area (least-significant-bit-first words, skewed if asked
 // for) and work out where this lane's stream lies.  `first`: byte offset of the lane's stream in the packed area;
@@ -623,11 +630,11 @@ __device__ __forceinline__ bool kvc_streams_inside(const KvcFusedArgs &a, const 
 // Loads of a tile's payload; rows: words of a stream that the LDS area holds.  Sets fits (wave-uniform: every stream is that short) and
 // u0: `lead_bits` before the lane's first code, and a word on, so that it is never negative (kvc_column_address takes it off again).
 template <class Raw>
-__device__ __forceinline__ KvcStaged kvc_fetch_streams(const KvcFusedArgs &a, int lane, int rows, uint32_t lead_bits, Raw &raw)
+__device__ __forceinline__ KvcStreams kvc_fetch_streams(const KvcFusedArgs &a, int lane, int rows, uint32_t lead_bits, Raw &raw)
 {
     typedef uint32_t w4 __attribute__((ext_vector_type(4), aligned(4)));
     const KvcLane l = kvc_lane_stream(a, lane, raw);
-    KvcStaged st;
+    KvcStreams st;
     st.gwords = nullptr;
     st.gnwords = st.gpos = 0;
     st.fits = !__any((int)(l.bytes > 4u * (uint32_t)rows));
@@ -643,7 +650,7 @@ __device__ __forceinline__ KvcStaged kvc_fetch_streams(const KvcFusedArgs &a, in
 }
 // ... into the columns.  column: LDS byte address of the lane's word in row 0.
 template <class Raw>
-__device__ __forceinline__ void kvc_stage_streams(const KvcFusedArgs &a, int lane, int rows, const Raw &raw, const KvcStaged &st, uint32_t column)
+__device__ __forceinline__ void kvc_stage_streams(const KvcFusedArgs &a, int lane, int rows, const Raw &raw, const KvcStreams &st, uint32_t column)
 {
     if (!st.fits) return;
     kvc_lds_u32 *dst = (kvc_lds_u32 *)(uintptr_t)column;
@@ -664,7 +671,7 @@ __device__ __forceinline__ void kvc_stage_streams(const KvcFusedArgs &a, int lan
 }
 // What the one-symbol decoder needs to know of a lane's stream
 template <class Raw>
-__device__ __forceinline__ void kvc_stream_in_memory(const KvcFusedArgs &a, int lane, const Raw &raw, KvcStaged &st)
+__device__ __forceinline__ void kvc_stream_in_memory(const KvcFusedArgs &a, int lane, const Raw &raw, KvcStreams &st)
 {
     const KvcLane l = kvc_lane_stream(a, lane, raw);
     st.gwords = reinterpret_cast<const uint32_t *>(l.base + l.at);
@@ -681,12 +688,29 @@ __device__ __forceinline__ uint32_t kvc_column_address(uint32_t column, uint32_t
     asm("" : "+v"(row));                                                                  // (see kvc_refill_address)
     return (row << 8) + (column - 256u);
 }
-// Which matrix-core kernels have them: those for codes of at most 7 bits; with eight query heads only K's for one-byte entries.  A wave with
-// that many heads holds three or four to a SIMD, and in caches of few tiles it waits for its one tile, which columns and one-byte
-// entries made longer (2 x 8 x 8 heads x 128 x 1905 tokens, K's codes longer: V packed 40.4 us, in columns 41.3, with both 41.9; 8 x 8 x 8 x 128 x
-// 4096 59.2 : 60.3; 2 x 8 x 8 x 96 x 4000, K in both 33.9, in neither 33.5).  K of many tiles gains: 8 x 8 x 8 x 96 x 8192 80.6 -> 74.3.
-constexpr int64_t KVC_COLUMNS_REP8_TILES = 4096;
-constexpr bool kvc_mfma_columns(int rep, bool long_codes, bool mid_codes) { return mid_codes || (!long_codes && rep != 8); }
+enum { KVC_BOOK_SHORT = 0, KVC_BOOK_MID = 1, KVC_BOOK_LONG = 2, KVC_BOOK_PACKED = 3 };       // of kvc_fused_mfma_kernel
+// Which launches of the matrix-core kernels for codes of at most 7 bits take their payloads in columns (eight query heads: K's with one-byte
+// entries only; the rest has no such kernels, V's took 41.3 us for 40.4 at 2 x 8 x 8 heads x 128 x 1905 tokens).  From `tiles` of a kind on: a wave of fewer waits for its one tile, which the lanes' own loads
+// make longer.  Packed against columns in us, 4 x 8 KV heads, head_dim 128, rounded arithmetic, one-byte entries in columns:
+//   K  1 query head   2048 tiles 11.8 : 11.9    3072 13.1 : 12.5    4096 14.9 : 13.5    8192 26.3 : 23.1   32768 70 : 61
+//      2              2048       11.0 : 11.6    3072 12.6 : 12.4    4096 14.4 : 13.8    8192 26.0 : 23.2   32768 73 : 64
+//      4              2048       12.7 : 13.0    3072 14.3 : 14.2    4096 16.3 : 15.4    8192 28.7 : 26.2   32768 80 : 72
+//      8              2048       15.4 : 15.9    3072 18.6 : 18.4    4096 27.3 : 21.1    6144 33.6 : 31.4   32768 141 : 118
+//   V  1, 2, 4        from 512 tiles on 11.1 : 11.2, 10.5 : 10.7 (256), 12.4 : 12.0 (128); 4096 16.0 : 14.2, 15.6 : 14.6, 17.7 : 16.2
+// other codebooks (K and V one query head; with two and four the same to 0.5 us):
+//   K 2048 10.5 : 10.9   4096 13.2 : 13.3   8192 19.8 : 19.2      V 2048 9.4 : 10.1   3072 12.1 : 10.9   8192 20.7 : 19.8
+// and products that are not rounded: K 2048 10.4 : 11.6   8192 21.5 : 23.3   16384 35.2 : 34.5    V 2048 11.0 : 11.6   4096 14.4 : 14.6   8192 23.8 : 22.4
+constexpr int64_t kvc_columns_from(bool is_k, int rep, bool byte_entries, bool rounded)
+{
+    return !rounded ? (is_k ? 16384 : 4096) : !byte_entries ? (is_k ? 4096 : 3072) : !is_k ? 0 : rep == 8 ? 4096 : 3072;
+}
+// ... and where the LDS still holds this many workgroups of a compute unit: columns are as long as the longest stream of the whole cache,
+// packed payloads take their tile's bytes.  K of 4 x 32 heads x 96 x 32 768 tokens, packed 99 us: columns of 13, 17, 19, 21 and 29 words 84, 91,
+// 96, 107 and 127 (eight, six, six, five and four workgroups); V (71): 6, 11 and 15 words 70, 73 and 80 (seven, six, five).  K and V of
+// 8 x 8 heads x 128 x 8320, two query heads, 53: 17, 25 and 27 words 49, 51 and 60 (six, five, four); four query heads, 60: 17, 21 and 23 words 57,
+// 58 and 74 (five, five, four), of head_dim 96 and 8192 tokens V (29.8): 12 and 19 words 27.9 and 28.5 (five, four; its registers allow four);
+// eight, K and V 99: 21 and 23 words 95.8 and 99.1 (four, three).
+constexpr int kvc_columns_workgroups(int rep, int slots) { return rep == 1 ? 6 : rep == 2 || (rep == 4 && slots == 1) ? 5 : 4; }
 enum { KVC_PACKED_PLAIN = 0, KVC_PACKED_SKEWED = 1, KVC_COLUMNS = 2 };
 // The three words of a refill.  base: kvc_refill_address's, or the lane's column.
 template <int LAYOUT, bool WORD = true>
@@ -728,4 +752,6 @@ constexpr int KVC_LONG_TABLE_WORDS = (1 << KVC_LUT_ESC_BITS) / 2 + 2 * KVC_LUT_E
 void kvc_launch_fused_mid(int rep, int kind, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);
 // kinds 0, 3 and 4, rounded arithmetic only
 void kvc_launch_fused_long(int rep, int kind, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);
+// payloads in columns: one, two or four query heads per KV head
+void kvc_launch_fused_packed(int rep, int kind, bool rounded, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);
 void kvc_launch_fused_mfma(int rep, int kind, bool rounded, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream);

@@ -1,5 +1,6 @@
-// kvc_fused_mfma.hip -- launchers of the matrix-core fused decode + matvec kernels (kvc_fused_mfma_impl.h) and all of
-// their instances but the ones that have a translation unit of their own (kvc_fused_mfma_v96.hip).
+// kvc_fused_mfma.hip -- launchers of the matrix-core fused decode + matvec kernels for codes of at most 7 bits whose payloads lie in
+// columns (kvc_fused_mfma_impl.h) and all of their instances but the ones that have a translation unit of their own
+// (kvc_fused_mfma_v96.hip).
 #include "kvc_fused_mfma_impl.h"
 
 // compiled in kvc_fused_mfma_v96.hip
@@ -16,6 +17,7 @@ static void kvc_launch_mfma_kind(int kind, const KvcFusedArgs &a, dim3 grid, siz
     else hipLaunchKernelGGL((kvc_fused_mfma_kernel<REP, 4, ROUNDED>), grid, dim3(KVC_WG), lds, stream, a);
 }
 
+// one, two or four query heads per KV head
 void kvc_launch_fused_mfma(int rep, int kind, bool rounded, const KvcFusedArgs &a, dim3 grid, size_t lds, hipStream_t stream)
 {
 #define KVC_MFMA_REP(R)                                                         \
@@ -24,8 +26,7 @@ void kvc_launch_fused_mfma(int rep, int kind, bool rounded, const KvcFusedArgs &
     switch (rep) {
         case 1: KVC_MFMA_REP(1); break;
         case 2: KVC_MFMA_REP(2); break;
-        case 4: KVC_MFMA_REP(4); break;
-        default: KVC_MFMA_REP(8); break;
+        default: KVC_MFMA_REP(4); break;
     }
 #undef KVC_MFMA_REP
 }

@@ -582,29 +582,28 @@ __device__ __forceinline__ float kvc_quad_next(float v)
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xF5 /* quad_perm:[1,1,3,3] */, 0xf, 0xf, false));
 }
 
-// BOOK: what the codebooks' longest codes ask for.  Codes of 6 or 7 bits of symbols up to 16 (kvc_mfma_dot's BYTE) and codes
+// BOOK: what the codebooks' longest codes ask for, and with codes of at most 7 bits whether payloads lie in columns (kvc_fetch_streams)
+// or packed.  Codes of 6 or 7 bits of symbols up to 16 (kvc_mfma_dot's BYTE) and codes
 // of more than 7 bits (kvc_mfma_dot_long) have kernels of their own (kvc_fused_mfma_mid.hip, kvc_fused_mfma_long.hip): beside
 // the other loops theirs would cost registers and spilled scalars (one query head, the former: K 14 -> 25 spilled scalars, the
 // plain V kernel seven waves per SIMD instead of eight).
-enum { KVC_BOOK_SHORT = 0, KVC_BOOK_MID = 1, KVC_BOOK_LONG = 2 };
 constexpr int kvc_fused_book_occupancy(int rep, int kind, int book)
 {
     return book == KVC_BOOK_LONG ? kvc_fused_long_occupancy(rep, kind) : book == KVC_BOOK_MID ? kvc_fused_mid_occupancy(rep, kind)
-                                                                       : kvc_fused_mfma_occupancy(rep, kind);
+           : book == KVC_BOOK_PACKED && rep == 2 && kind == 3 ? 6 : kvc_fused_mfma_occupancy(rep, kind);
 }
 template <int REP, int KIND, bool ROUNDED, int BOOK = KVC_BOOK_SHORT>
 __global__ void __launch_bounds__(KVC_WG, kvc_fused_book_occupancy(REP, KIND, BOOK))
 kvc_fused_mfma_kernel(KvcFusedArgs a_in)
 {
-    constexpr bool LONG = BOOK == KVC_BOOK_LONG, MID = BOOK == KVC_BOOK_MID;
-    static_assert(ROUNDED || BOOK == KVC_BOOK_SHORT, "kernels of the default arithmetic");
+    constexpr bool LONG = BOOK == KVC_BOOK_LONG, MID = BOOK == KVC_BOOK_MID, ANY_SHORT = BOOK == KVC_BOOK_SHORT || BOOK == KVC_BOOK_PACKED;
+    static_assert(ROUNDED || ANY_SHORT, "kernels of the default arithmetic");
     const KvcFusedArgs &a = a_in;
     constexpr bool IS_K = KIND == 0;
     constexpr int SLOTS = KvcGeom<KIND>::SLOTS;
     constexpr int NM = kvc_mfma_sets(REP);
     using T = KvcMfmaTables<REP>;
-    // payloads in columns (kvc_fetch_streams), or packed
-    constexpr bool COLUMNS = kvc_mfma_columns(REP, LONG, MID);
+    constexpr bool COLUMNS = BOOK == KVC_BOOK_SHORT || MID;
     // dynamic LDS: the decode table (at offset 0, so that its address folds into the look-ups), then per wave:
     // operand tables, packed payload; in columns, all waves' payloads, then all waves' operand tables
     extern __shared__ __align__(16) uint32_t smem[];
@@ -682,19 +681,19 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     // Batch 4 x 32 heads x 96 x 32 768 tokens, heavy-tailed data, 7 index bits for codes of up to 6: V 88 -> 74 us.  With 8
     // bits (three pairs per half window, 256 words) it measured no better than one symbol per look-up (38.6 / 39.8 us at
     // batch 8 x 32 x 128 x 4096), and K, which has no such codebooks, 8 % slower for the scalars spilled.
-    constexpr bool NARROW_OK = !IS_K && BOOK == KVC_BOOK_SHORT;
+    constexpr bool NARROW_OK = !IS_K && ANY_SHORT;
     const uint32_t one_at = (uint32_t)a.narrow_pair_bits > lbits ? (uint32_t)a.narrow_pair_bits : lbits;
     const bool narrow = NARROW_OK && fast_book && a.narrow_pair_bits != 0 && (uint32_t)a.narrow_pair_bits < 2u * lmax &&
                         (1u << one_at) + (1u << lbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
     const uint32_t pbits = narrow ? (uint32_t)a.narrow_pair_bits : 2u * lmax;
     // two symbols per look-up: twice the longest code fits the index, and no symbol's fp16 pattern needs the five
     // bits the lengths of a two-symbol entry go to (header word 6: OR of all the patterns)
-    const bool pairs = narrow || (BOOK == KVC_BOOK_SHORT && fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
+    const bool pairs = narrow || (ANY_SHORT && fast_book && a.pair_bits != 0 && pbits <= (uint32_t)a.pair_bits && pbits <= 10u &&
                                  (1u << pbits) <= (uint32_t)a.table_words && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u);
     // codes of 6 or 7 bits: two-byte entries (see kvc_mfma_dot), where no symbol's fp16 pattern needs its five lowest bits.
     // Not for V tiles that may straddle two heads: with that loop beside the others the kernel needs one register more
     // than six waves per SIMD leave it, and the compiler then spills in the per-tile path of every variant.
-    constexpr bool HALF_OK = SLOTS == 1 && BOOK == KVC_BOOK_SHORT;
+    constexpr bool HALF_OK = SLOTS == 1 && ANY_SHORT;
     const bool half_table = HALF_OK && fast_book && !pairs && lbits >= 6u && a.half_table != 0 && (lut_g[6] & KVC_PAIR_LEN_MASK) == 0u;
     constexpr int centre = MID ? KVC_BYTE_CENTRE : 0;
     const uint32_t lead_bits = LONG || MID || half_table ? 1u : 2u;                   // bits of the window below the table index
@@ -770,7 +769,7 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
     tabs.lo0 = tabs.lo1 = 0;                                             // (the low-part columns start as zeros)
     KvcTablePlan plan = kvc_plan_tables<KIND, ROUNDED>(a, pos, tabs);
     kvc_fetch_tile<REP, KIND, 0, SLOTS == 2, !COLUMNS>(a, pos, __builtin_amdgcn_readlane(bi_off, 0), __builtin_amdgcn_readlane(bi_bn, 0), lane, raw);
-    KvcStaged st;
+    std::conditional_t<COLUMNS, KvcStreams, KvcStaged> st;
     if constexpr (COLUMNS) {
         raw.ti_cur = ti_first;
         st = kvc_fetch_streams(a, lane, a.column_rows, lead_bits, raw);
@@ -813,8 +812,9 @@ kvc_fused_mfma_kernel(KvcFusedArgs a_in)
         // are not kept in registers through the decode loops
         int lane_f = lane;
         asm volatile("" : "+v"(lane_f));
-        const KvcTileBytes here = {raw.off, raw.bn, raw.ti_cur};
-        KvcStaged st_next = st;
+        [[maybe_unused]] const KvcTileBytes here = {raw.off, raw.bn, raw.ti_cur};
+        [[maybe_unused]] KvcStreams st_next;
+        if constexpr (COLUMNS) st_next = st;
         if (more) {   // loads for the next tile fly while this one is decoded
             kvc_fetch_tile<REP, KIND, 0, SLOTS == 2, !COLUMNS>(a, pos_next, __builtin_amdgcn_readlane(bi_off, it + 1),
                                                                __builtin_amdgcn_readlane(bi_bn, it + 1), lane_f, raw, ~plan_next.build);

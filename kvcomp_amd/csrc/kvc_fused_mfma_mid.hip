@@ -21,7 +21,7 @@ void kvc_launch_fused_mid(int rep, int kind, const KvcFusedArgs &a, dim3 grid, s
         case 1: kvc_launch_mid_kind<1>(kind, a, grid, lds, stream); break;
         case 2: kvc_launch_mid_kind<2>(kind, a, grid, lds, stream); break;
         case 4: kvc_launch_mid_kind<4>(kind, a, grid, lds, stream); break;
-        default:               // V: kvc_mfma_columns
+        default:               // (K only)
             hipLaunchKernelGGL((kvc_fused_mfma_kernel<8, 0, true, KVC_BOOK_MID>), grid, dim3(KVC_WG), lds, stream, a);
             break;
     }

@@ -7,3 +7,5 @@
 template __global__ void kvc_fused_mfma_kernel<1, 4, true>(KvcFusedArgs);
 template __global__ void kvc_fused_mfma_kernel<1, 4, false>(KvcFusedArgs);
 template __global__ void kvc_fused_mfma_kernel<1, 4, true, KVC_BOOK_MID>(KvcFusedArgs);
+template __global__ void kvc_fused_mfma_kernel<1, 4, true, KVC_BOOK_PACKED>(KvcFusedArgs);
+template __global__ void kvc_fused_mfma_kernel<1, 4, false, KVC_BOOK_PACKED>(KvcFusedArgs);

@@ -48,7 +48,7 @@ const OptionDef g_option_defs[KVC_OPT_COUNT] = {
     {"fused_tiles_per_wave", "KVCOMP_FUSED_TILES_PER_WAVE", 0},  // 0 choose per call
     {"fused_pair_bits", "KVCOMP_FUSED_PAIR_BITS", 8},            // widest two-symbol table index; 0 = one symbol per look-up
     {"fused_double_window", "KVCOMP_FUSED_DOUBLE_WINDOW", 1},    // 64 stream bits per refill in the one-symbol loops
-    {"fused_skew", "KVCOMP_FUSED_SKEW", -1},                     // skewed payload layout: -1 choose per call, 0 never, 1 always
+    {"fused_skew", "KVCOMP_FUSED_SKEW", -1},                     // payload layout: -1 choose per call, 0 packed, 1 packed and skewed, 2 in columns
     {"decode_pipelined", "KVCOMP_DECODE_PIPELINED", 1},          // plain decode / decode + dequantize on the fused kernels' machinery
     {"fused_rounded", "KVCOMP_FUSED_ROUNDED", 1},                // 1: round each dequantized value to fp16 before the matvec, as the reference's dequantizer does
     {"attention_tail_in_merge", "KVCOMP_ATTENTION_TAIL_IN_MERGE", 1},   // kvc_attention_decode: V's fp16 tail inside the merge kernel

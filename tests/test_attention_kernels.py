@@ -1,0 +1,80 @@
+"""Which kernels decode attention takes a cache with: kvc_attention_kernels answers from the descriptors alone."""
+import ctypes as C
+
+import pytest
+
+from kvcomp_amd import _lib
+
+COLUMNS, BYTES, LONG, PACKED, FMA = 0, 1, 2, 3, 4      # KVC_BOOK_*: columns with word entries, with byte entries, long codes, packed; none
+BYTE_SYMBOLS = 0x300
+
+
+def _desc(is_k, tokens, B, H, D, bits, mean, longest, pair_bits=0, symbols=BYTE_SYMBOLS):
+    """mean: bytes of a stream; longest: of the longest one, 0 = not known"""
+    tiles = tokens // 64 * B * H if is_k else tokens // 128 * B * H * D // 64
+    return _lib.CompressedDesc(tokens=tokens, encoded_bytes=tiles * 64 * mean, max_tile_bytes=int(64 * mean * 1.05), max_stream_bytes=longest,
+                               max_code_bits=bits | symbols | pair_bits << 12, quant_mask=1 if is_k else 0xE)
+
+
+def _kernels(B, H, rep, D, tokens, k=(7, 52, 59), v=(7, 32, 39), **kw):
+    f = C.CDLL(_lib.LIB_PATH).kvc_attention_kernels
+    f.argtypes = [C.POINTER(_lib.CompressedDesc)] * 2 + [C.c_int64] * 4
+    _lib.lib()
+    got = f(C.byref(_desc(True, tokens, B, H, D, *k, **kw)), C.byref(_desc(False, tokens, B, H, D, *v, **kw)), B, H, H * rep, D)
+    return got & 15, got >> 4 & 15
+
+
+@pytest.mark.parametrize("rep,first", [(1, 3072), (2, 3072), (4, 3072), (8, 4096)])
+def test_columns_begin_where_they_pay(rep, first):
+    """A wave of a small cache waits for its one tile, which the lanes' own loads make longer."""
+    v = PACKED if rep == 8 else BYTES
+    assert _kernels(1, 8, rep, 128, (first // 8 - 2) * 64) == (PACKED, v)
+    assert _kernels(1, 8, rep, 128, first // 8 * 64) == (BYTES, v)
+
+
+@pytest.mark.parametrize("rep", [1, 2, 4])
+def test_shorter_codes_and_products_that_are_not_rounded(rep):
+    short = dict(k=(5, 38, 44), v=(5, 30, 36))
+    assert _kernels(1, 8, rep, 128, 64 * 510, **short) == (PACKED, COLUMNS)
+    assert _kernels(1, 8, rep, 128, 64 * 512, **short) == (COLUMNS, COLUMNS)
+    assert _kernels(1, 8, rep, 128, 64 * 382, **short) == (PACKED, PACKED)
+    was = _lib.set_option("fused_rounded", 0)
+    try:
+        assert _kernels(1, 8, rep, 128, 64 * 2046) == (PACKED, COLUMNS) and _kernels(1, 8, rep, 128, 64 * 2048) == (COLUMNS, COLUMNS)
+        assert _kernels(1, 8, rep, 128, 64 * 510) == (PACKED, PACKED)
+    finally:
+        _lib.set_option("fused_rounded", was)
+
+
+@pytest.mark.parametrize("rep,D", [(1, 128), (1, 96), (2, 128), (4, 128), (4, 96), (8, 128)])
+def test_one_long_stream_does_not_size_every_waves_lds(rep, D):
+    """A single token whose symbols are all rare: 112 bytes where the others have some 50."""
+    v = PACKED if rep == 8 else BYTES
+    even = dict(k=(7, 52 * D // 128, 59 * D // 128), v=(7, 32, 40))
+    assert _kernels(4, 8, rep, D, 32768, **even) == (BYTES, v)
+    odd = (7, 52 * D // 128, 112)
+    assert _kernels(4, 8, rep, D, 32768, k=odd, v=even["v"])[0] == PACKED
+    assert _kernels(4, 8, rep, D, 32768, k=even["k"], v=(7, 32, 112)) == (BYTES, PACKED)
+
+
+def test_a_stream_hint_that_is_not_there():
+    """The tile's bytes decide then, as they are known or near their mean; a single stream would not be."""
+    assert _kernels(4, 8, 1, 128, 32768, k=(7, 52, 0), v=(7, 32, 0)) == (PACKED, PACKED)
+
+
+def test_a_layout_that_is_asked_for():
+    for value, want in ((0, PACKED), (1, PACKED), (2, BYTES)):
+        was = _lib.set_option("fused_skew", value)
+        try:
+            assert _kernels(1, 8, 2, 128, 512) == (want, want) and _kernels(4, 8, 2, 128, 32768) == (want, want)
+            assert _kernels(1, 8, 2, 128, 512, k=(9, 52, 59), v=(9, 32, 39)) == (LONG, LONG)
+        finally:
+            _lib.set_option("fused_skew", was)
+
+
+def test_other_codebooks():
+    assert _kernels(4, 8, 2, 128, 32768, k=(9, 52, 59), v=(12, 60, 70)) == (LONG, LONG)
+    assert _kernels(4, 8, 2, 128, 32768, k=(9, 52, 59), v=(12, 60, 70), symbols=0) == (FMA, FMA)      # an alphabet of any size
+    assert _kernels(4, 8, 2, 128, 32768, symbols=0x100) == (COLUMNS, COLUMNS)
+    assert _kernels(4, 8, 8, 128, 32768, symbols=0x100) == (PACKED, PACKED)
+    assert _kernels(4, 8, 1, 96, 32768, k=(6, 42, 47), v=(6, 20, 24), pair_bits=7) == (BYTES, COLUMNS)
