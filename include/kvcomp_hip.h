@@ -81,7 +81,9 @@ int kvc_abi_version(void);
  *                           (v_mfma_f32_4x4x4_16b_f16) wherever those kernels apply (codes of at most 7 bits, results
  *                           that can be stored four at a time); 0: never (fp32 multiply-adds on the vector units).
  *   "fused_half_table":      1 (default): for codes of 6 or 7 bits the matrix-core kernels use two-byte decode table entries
- *                           (64 entries = one LDS word per bank); 0: four-byte entries.
+ *                           (64 entries = one LDS word per bank), and those for symbols up to 16, one byte of an entry, are
+ *                           taken, the one with a group per wave ("attention_joint") among them; 0: four-byte entries, and
+ *                           none of those kernels.
  *   "fused_builtin_dpp":     0 (default): the fp32-FMA kernels pick their operand out of a quad of lanes with a permute
  *                           written as inline assembly on the multiply-add itself; 1: through the compiler's lane-
  *                           permute intrinsic (same result bit for bit; a cross-check against toolchain changes).
@@ -110,9 +112,12 @@ int kvc_abi_version(void);
  *                           share their heads' operand tables).
  *   "attention_tail_in_merge": 1 (default): kvc_attention_decode handles V's fp16 tail (up to 1024 tokens, K compressed
  *                           at least as far as V) inside its merge kernel; 0: with two kernels of its own.
- *   "attention_joint":       -1 (default): kvc_attention_decode takes K and V of small caches in one launch, a 128-token group
- *                           of a head per workgroup, where head_dim is a multiple of 64 and codes have at most 7 bits;
- *                           0: never; 1: whatever the cache's size.
+ *   "attention_joint":       -1 (default): kvc_attention_decode takes K and V in one launch where that is faster: small caches, head_dim
+ *                           a multiple of 64 and codes of at most 7 bits, with a 128-token group of a head per workgroup;
+ *                           more than 1536 groups, head_dim 128 and codes of 6 or 7 bits of symbols up to 16, none two to a
+ *                           look-up, with a group per wave, unless the longest streams would leave the LDS to few
+ *                           workgroups.  0: never; 1: a group per workgroup, whatever the cache's size; 2: a group per
+ *                           wave wherever such a kernel takes the cache and its LDS fits, else K and V by a kernel each.
  *   "decode_pipelined":      1 (default): plain decode and decode + dequantize run on the fused kernels' tile
  *                           pipeline; 0: on the simpler stand-alone kernels. */
 int kvc_set_option(const char *name, int value);

@@ -384,31 +384,66 @@ static int kvc_attend_fill(KvcFusedArgs &a, const kvc_compressed_desc *c, int is
     a.q_heads = (int)q_heads;
     a.head_dim = (int)head_dim;
     a.rounded = 1;
-    a.pack_words = a.pack_logical = kvc_attend_pack_words(c, rows * a.s.cols);
     return 0;
+}
+
+// The joint kernel's LDS
+struct KvcJointPlan {
+    int k_pack_words, v_pack_words, ktab_words;
+    size_t lds;          // more than 64 KiB: does not fit
+};
+static KvcJointPlan kvc_plan_joint(const kvc_compressed_desc *k, const kvc_compressed_desc *v, int64_t rep, int64_t bh, int64_t head_dim)
+{
+    KvcJointPlan p = {};
+    const int kb = kvc_hint_bits(k->max_code_bits);
+    const int64_t groups = v->tokens / KVC_V_TOKENS, k_tiles = k->tokens / KVC_WAVE * bh;
+    p.k_pack_words = kvc_attend_pack_words(k, k_tiles);
+    p.v_pack_words = kvc_attend_pack_words(v, groups * bh * (head_dim / KVC_WAVE));
+    const int sets = kvc_mfma_sets((int)rep), btab = KVC_MFMA_GROUPS * sets * 8, mstab = KVC_MFMA_GROUPS * 4;
+    const int k_area = btab + mstab + p.k_pack_words, v_area = mstab + p.v_pack_words;
+    int waves = KVC_ATTEND_K_TILES * k_area + (int)(head_dim / KVC_WAVE) * v_area;
+    if (k_tiles > groups * bh * KVC_ATTEND_K_TILES && waves < KVC_WAVES_PER_WG * k_area) waves = KVC_WAVES_PER_WG * k_area;
+    const int fixed = KVC_ATTEND_VTAB_WORDS + KVC_ATTEND_TMP_WORDS + btab + (int)rep * KVC_V_TOKENS + waves + KVC_LDS_SLACK_WORDS;
+    p.ktab_words = KVC_ATTEND_VTAB_WORDS;
+    if (kb <= KVC_ATTEND_K_PAIR_BITS && (1 << (2 * kb)) > p.ktab_words) p.ktab_words = 1 << (2 * kb);
+    if (4 * (p.ktab_words + fixed) > 65536) p.ktab_words = KVC_ATTEND_VTAB_WORDS;
+    p.lds = 4 * (size_t)(p.ktab_words + fixed);
+    return p;
+}
+
+KvcAttendRoute kvc_attend_route(const kvc_compressed_desc *k, const kvc_compressed_desc *v, int64_t batch, int64_t kv_heads, int64_t q_heads,
+                                int64_t head_dim)
+{
+    const int want = kvc_option(KVC_OPT_ATTENTION_JOINT);
+    const int64_t rep = q_heads / kv_heads, bh = batch * kv_heads;
+    const int kb = kvc_hint_bits(k->max_code_bits), vb = kvc_hint_bits(v->max_code_bits);
+    if (want == 0 || v->tokens == 0 || k->tokens < v->tokens || head_dim % KVC_WAVE != 0 || kb < 1 || kb > 7 || vb < 1 || vb > 7) return KVC_ATTEND_SEPARATE;
+    if (k->rows_per_codebook != 0 || v->rows_per_codebook != 0 || !(rep == 1 || rep == 2 || rep == 4 || rep == 8)) return KVC_ATTEND_SEPARATE;
+    if (!(k->quant_mask == KVC_MASK_K_BLOCK || k->quant_mask == KVC_MASK_CHANNEL)) return KVC_ATTEND_SEPARATE;
+    if (!(v->quant_mask == KVC_MASK_V_TOKEN || v->quant_mask == KVC_MASK_SIM_TOKEN || v->quant_mask == KVC_MASK_VECTOR)) return KVC_ATTEND_SEPARATE;
+    if (kvc_option(KVC_OPT_FUSED_ROUNDED) == 0 || kvc_option(KVC_OPT_FUSED_MFMA) == 0 || kvc_option(KVC_OPT_FUSED_ROWS) == 1) return KVC_ATTEND_SEPARATE;
+    const int64_t wgs = v->tokens / KVC_V_TOKENS * bh;
+    if (k->tokens / KVC_WAVE * bh > (int64_t)1 << 30) return KVC_ATTEND_SEPARATE;
+    // a wave per group (kvc_attend_waves.hip) where both codebooks are its
+    if (want != 1 && (want > 1 || wgs > KVC_ATTEND_WAVES_MIN_WGS) && head_dim == 2 * KVC_WAVE && kb >= 6 && vb >= 6 &&
+        kvc_hint_byte_symbols(k->max_code_bits) && kvc_hint_byte_symbols(v->max_code_bits) && kvc_hint_pair_bits(v->max_code_bits) == 0 &&
+        kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0) {
+        const int per_cu = kvc_plan_attend_waves(k, v, rep, bh).per_cu;
+        if (want > 1 ? per_cu > 0 : kvc_attend_waves_pays(rep, wgs, per_cu)) return KVC_ATTEND_WAVES;
+    }
+    if (want > 1 || (want < 0 && wgs > kvc_attend_max_wgs(rep))) return KVC_ATTEND_SEPARATE;
+    return kvc_plan_joint(k, v, rep, bh, head_dim).lds <= 65536 ? KVC_ATTEND_JOINT : KVC_ATTEND_SEPARATE;
 }
 
 int kvc_attend_groups(const kvc_compressed_desc *k, const kvc_compressed_desc *v, const void *d_q_f16, float softmax_scale,
                       float *scores, int64_t scores_stride, float *part, float *ml, int64_t batch, int64_t kv_heads, int64_t q_heads,
                       int64_t head_dim, hipStream_t stream, bool *taken)
 {
+    const KvcAttendRoute route = kvc_attend_route(k, v, batch, kv_heads, q_heads, head_dim);
     *taken = false;
-    const int want = kvc_option(KVC_OPT_ATTENTION_JOINT);
-    const int64_t rep = q_heads / kv_heads, bh = batch * kv_heads;
-    const int kb = kvc_hint_bits(k->max_code_bits), vb = kvc_hint_bits(v->max_code_bits);
-    if (want == 0 || v->tokens == 0 || k->tokens < v->tokens || head_dim % KVC_WAVE != 0 || kb < 1 || kb > 7 || vb < 1 || vb > 7) return 0;
-    if (k->rows_per_codebook != 0 || v->rows_per_codebook != 0 || !(rep == 1 || rep == 2 || rep == 4 || rep == 8)) return 0;
-    if (!(k->quant_mask == KVC_MASK_K_BLOCK || k->quant_mask == KVC_MASK_CHANNEL)) return 0;
-    if (!(v->quant_mask == KVC_MASK_V_TOKEN || v->quant_mask == KVC_MASK_SIM_TOKEN || v->quant_mask == KVC_MASK_VECTOR)) return 0;
-    if (kvc_option(KVC_OPT_FUSED_ROUNDED) == 0 || kvc_option(KVC_OPT_FUSED_MFMA) == 0 || kvc_option(KVC_OPT_FUSED_ROWS) == 1) return 0;
-    const int64_t groups = v->tokens / KVC_V_TOKENS, wgs = groups * bh;
+    if (route == KVC_ATTEND_SEPARATE) return 0;
+    const int64_t rep = q_heads / kv_heads, bh = batch * kv_heads, wgs = v->tokens / KVC_V_TOKENS * bh;
     const int64_t k_tiles = k->tokens / KVC_WAVE * bh, k_rest = k_tiles - wgs * KVC_ATTEND_K_TILES;
-    if (k_tiles > (int64_t)1 << 30) return 0;
-    // beyond, a wave per group (kvc_attend_waves.hip) where both codebooks are its
-    const bool by_waves = want != 1 && (want > 1 || wgs > KVC_ATTEND_WAVES_MIN_WGS) && head_dim == 2 * KVC_WAVE && kb >= 6 && vb >= 6 &&
-                          kvc_hint_byte_symbols(k->max_code_bits) && kvc_hint_byte_symbols(v->max_code_bits) && kvc_hint_pair_bits(v->max_code_bits) == 0 &&
-                          kvc_option(KVC_OPT_FUSED_HALF_TABLE) != 0;
-    if (!by_waves && (want > 1 || (want < 0 && wgs > kvc_attend_max_wgs(rep)))) return 0;
     KvcAttendArgs j = {};
     if (int rc = kvc_attend_fill(j.k, k, 1, batch, kv_heads, q_heads, head_dim)) return rc;
     if (int rc = kvc_attend_fill(j.v, v, 0, batch, kv_heads, q_heads, head_dim)) return rc;
@@ -418,31 +453,26 @@ int kvc_attend_groups(const kvc_compressed_desc *k, const kvc_compressed_desc *v
     j.v.out = part;
     j.v.ml = ml;
     j.v.sm_scale = softmax_scale;
-    if (by_waves) return kvc_attend_waves(j.k, j.v, k, v, rep, bh, stream, taken);
-    j.k_bits = kb;
-    j.v_bits = vb;
+    *taken = true;
+    if (route == KVC_ATTEND_WAVES) return kvc_attend_waves(j.k, j.v, k, v, kvc_plan_attend_waves(k, v, rep, bh), rep, stream);
+    const KvcJointPlan plan = kvc_plan_joint(k, v, rep, bh, head_dim);
+    j.k.pack_words = j.k.pack_logical = plan.k_pack_words;
+    j.v.pack_words = j.v.pack_logical = plan.v_pack_words;
+    j.k_bits = kvc_hint_bits(k->max_code_bits);
+    j.v_bits = kvc_hint_bits(v->max_code_bits);
     j.group_wgs = (int)wgs;
     j.k_tiles = (int)k_tiles;
-    const int sets = kvc_mfma_sets((int)rep), btab = KVC_MFMA_GROUPS * sets * 8, mstab = KVC_MFMA_GROUPS * 4;
-    const int k_area = btab + mstab + j.k.pack_words, v_area = mstab + j.v.pack_words;
-    int waves = KVC_ATTEND_K_TILES * k_area + (int)(head_dim / KVC_WAVE) * v_area;
-    if (k_rest > 0 && waves < KVC_WAVES_PER_WG * k_area) waves = KVC_WAVES_PER_WG * k_area;
-    const int fixed = KVC_ATTEND_VTAB_WORDS + KVC_ATTEND_TMP_WORDS + btab + (int)rep * KVC_V_TOKENS + waves + KVC_LDS_SLACK_WORDS;
-    j.ktab_words = KVC_ATTEND_VTAB_WORDS;
-    if (kb <= KVC_ATTEND_K_PAIR_BITS && (1 << (2 * kb)) > j.ktab_words) j.ktab_words = 1 << (2 * kb);
-    if (4 * (j.ktab_words + fixed) > 65536) j.ktab_words = KVC_ATTEND_VTAB_WORDS;
-    const size_t lds = 4 * (size_t)(j.ktab_words + fixed);
-    if (lds > 65536) return 0;
+    j.ktab_words = plan.ktab_words;
+    const size_t lds = plan.lds;
     const unsigned grid = (unsigned)(wgs + (k_rest + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG);
     static const bool trace_plan = getenv("KVCOMP_TRACE_PLAN") != nullptr;
     if (trace_plan)
         fprintf(stderr, "[kvcomp] joint attention rep %d: %u workgroups (%d of whole groups), lds %zu B (K table %d w, codes %d / %d bits, payload %d / %d w)\n",
-                (int)rep, grid, (int)wgs, lds, j.ktab_words, kb, vb, j.k.pack_words, j.v.pack_words);
+                (int)rep, grid, (int)wgs, lds, j.ktab_words, j.k_bits, j.v_bits, j.k.pack_words, j.v.pack_words);
     if (rep == 1) hipLaunchKernelGGL(kvc_attend_group_kernel<1>, dim3(grid), dim3(KVC_WG), lds, stream, j);
     else if (rep == 2) hipLaunchKernelGGL(kvc_attend_group_kernel<2>, dim3(grid), dim3(KVC_WG), lds, stream, j);
     else if (rep == 4) hipLaunchKernelGGL(kvc_attend_group_kernel<4>, dim3(grid), dim3(KVC_WG), lds, stream, j);
     else hipLaunchKernelGGL(kvc_attend_group_kernel<8>, dim3(grid), dim3(KVC_WG), lds, stream, j);
     KVC_HIP(hipGetLastError());
-    *taken = true;
     return 0;
 }

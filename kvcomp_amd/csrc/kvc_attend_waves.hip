@@ -347,39 +347,56 @@ __global__ void __launch_bounds__(KVC_WG, REP == 8 ? 3 : 4) kvc_attend_waves_ker
     }
 }
 
-int kvc_attend_waves(const KvcFusedArgs &k, const KvcFusedArgs &v, const kvc_compressed_desc *kd, const kvc_compressed_desc *vd, int64_t rep, int64_t bh,
-                     hipStream_t stream, bool *taken)
+KvcWavesPlan kvc_plan_attend_waves(const kvc_compressed_desc *k, const kvc_compressed_desc *v, int64_t rep, int64_t bh)
+{
+    KvcWavesPlan p = {};
+    const int64_t groups = v->tokens / KVC_V_TOKENS, k_rows = k->tokens / KVC_WAVE;
+    p.k_only = (k_rows - KVC_WAVES_TILES * groups) * bh;
+    const int cols = KVC_MFMA_GROUPS * kvc_mfma_sets((int)rep) * 8, ms = KVC_MFMA_GROUPS * 4;
+    p.k_rows_lds = kvc_stream_rows(k->max_stream_bytes, k->encoded_bytes, k_rows * bh);
+    p.v_rows_lds = kvc_stream_rows(v->max_stream_bytes, v->encoded_bytes, groups * bh * KVC_WAVES_TILES);
+    const int k_area = KVC_WAVES_TILES * 64 * p.k_rows_lds, v_area = cols + KVC_WAVES_TILES * 64 * p.v_rows_lds;
+    p.area_words = k_area > v_area ? k_area : v_area;
+    if (p.area_words < (int)rep * KVC_V_TOKENS) p.area_words = (int)rep * KVC_V_TOKENS;
+    if (p.k_only > 0 && p.area_words < 64 * p.k_rows_lds + cols) p.area_words = 64 * p.k_rows_lds + cols;
+    // the last wave's second payload, and what a corrupt one may lead to
+    int least = 2 * KVC_WAVES_TAB_WORDS + (KVC_WAVES_PER_WG - 1) * p.area_words + 64 * KVC_COLUMN_REACH;
+    least += cols + 64 * p.v_rows_lds > 64 * p.k_rows_lds ? cols + 64 * p.v_rows_lds : 64 * p.k_rows_lds;
+    auto bytes = [&](int heads) {
+        const int words = 2 * KVC_WAVES_TAB_WORDS + KVC_WAVES_PER_WG * (p.area_words + KVC_WAVES_TILES * ms) + heads * cols;
+        return 4 * (size_t)(words < least ? least : words);
+    };
+    auto workgroups = [&](size_t lds) {
+        const int n = lds > 65536 ? 0 : kvc_lds_workgroups(lds), most = rep == 8 ? 3 : 4;       // by their registers
+        return n < most ? n : most;
+    };
+    // A workgroup across two heads leaves no wave without a group, and takes room for the columns of two: where the groups are no
+    // multiple of four, unless it costs a compute unit a workgroup.  3 x 24 heads x 14 464 tokens (113 groups) 79.1 -> 71 us
+    const bool two_heads = groups % KVC_WAVES_PER_WG != 0 && groups >= KVC_WAVES_PER_WG - 1 && workgroups(bytes(2)) == workgroups(bytes(1));
+    p.heads_per_wg = two_heads ? 2 : 1;
+    p.group_wgs = two_heads ? (groups * bh + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG : (groups + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG * bh;
+    p.lds = bytes(p.heads_per_wg);
+    p.per_cu = workgroups(p.lds);
+    return p;
+}
+
+int kvc_attend_waves(const KvcFusedArgs &k, const KvcFusedArgs &v, const kvc_compressed_desc *kd, const kvc_compressed_desc *vd, const KvcWavesPlan &p,
+                     int64_t rep, hipStream_t stream)
 {
     KvcAttendWavesArgs j = {};
-    const int64_t groups = vd->tokens / KVC_V_TOKENS, k_rows = kd->tokens / KVC_WAVE;
     j.k = k;
     j.v = v;
     j.k_bits = kvc_hint_bits(kd->max_code_bits);
     j.v_bits = kvc_hint_bits(vd->max_code_bits);
-    j.groups = (int)groups;
-    j.k_rows = (int)k_rows;
-    const int64_t rest = k_rows - KVC_WAVES_TILES * groups;
-    const int cols = KVC_MFMA_GROUPS * kvc_mfma_sets((int)rep) * 8, ms = KVC_MFMA_GROUPS * 4;
-    j.k_rows_lds = kvc_stream_rows(kd->max_stream_bytes, kd->encoded_bytes, k_rows * bh);
-    j.v_rows_lds = kvc_stream_rows(vd->max_stream_bytes, vd->encoded_bytes, groups * bh * KVC_WAVES_TILES);
-    const int k_area = KVC_WAVES_TILES * 64 * j.k_rows_lds, v_area = cols + KVC_WAVES_TILES * 64 * j.v_rows_lds;
-    j.area_words = k_area > v_area ? k_area : v_area;
-    if (j.area_words < (int)rep * KVC_V_TOKENS) j.area_words = (int)rep * KVC_V_TOKENS;
-    if (rest > 0 && j.area_words < 64 * j.k_rows_lds + cols) j.area_words = 64 * j.k_rows_lds + cols;
-    int words = 2 * KVC_WAVES_TAB_WORDS + KVC_WAVES_PER_WG * (j.area_words + KVC_WAVES_TILES * ms) + cols;
-    // A workgroup across two heads leaves no wave without a group, and takes room for the columns of two: where the groups are no
-    // multiple of four, unless it costs a compute unit its fourth workgroup.  3 x 24 heads x 14 464 tokens (113 groups) 79.1 -> 71 us
-    const bool two_heads = groups % KVC_WAVES_PER_WG != 0 && groups >= KVC_WAVES_PER_WG - 1 && (words > 40960 / 4 || words + cols <= 40960 / 4);
-    if (two_heads) words += cols;
-    j.heads_per_wg = two_heads ? 2 : 1;
-    j.group_wgs = (int)(two_heads ? (groups * bh + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG : (groups + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG * bh);
-    // the last wave's second payload, and what a corrupt one may lead to
-    const int last = 2 * KVC_WAVES_TAB_WORDS + (KVC_WAVES_PER_WG - 1) * j.area_words + 64 * KVC_COLUMN_REACH;
-    for (int second : {64 * j.k_rows_lds, cols + 64 * j.v_rows_lds})
-        if (words < last + second) words = last + second;
-    const size_t lds = 4 * (size_t)words;
-    if (lds > 65536) return 0;
-    const unsigned grid = (unsigned)(j.group_wgs + (rest * bh + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG);
+    j.groups = (int)(vd->tokens / KVC_V_TOKENS);
+    j.k_rows = (int)(kd->tokens / KVC_WAVE);
+    j.k_rows_lds = p.k_rows_lds;
+    j.v_rows_lds = p.v_rows_lds;
+    j.area_words = p.area_words;
+    j.heads_per_wg = p.heads_per_wg;
+    j.group_wgs = (int)p.group_wgs;
+    const size_t lds = p.lds;
+    const unsigned grid = (unsigned)(p.group_wgs + (p.k_only + KVC_WAVES_PER_WG - 1) / KVC_WAVES_PER_WG);
     static const bool trace_plan = getenv("KVCOMP_TRACE_PLAN") != nullptr;
     if (trace_plan)
         fprintf(stderr, "[kvcomp] attention by waves rep %d: %u workgroups (%d of whole groups), lds %zu B (codes %d / %d bits, rows %d / %d)\n",
@@ -389,6 +406,5 @@ int kvc_attend_waves(const KvcFusedArgs &k, const KvcFusedArgs &v, const kvc_com
     else if (rep == 4) hipLaunchKernelGGL(kvc_attend_waves_kernel<4>, dim3(grid), dim3(KVC_WG), lds, stream, j);
     else hipLaunchKernelGGL(kvc_attend_waves_kernel<8>, dim3(grid), dim3(KVC_WG), lds, stream, j);
     KVC_HIP(hipGetLastError());
-    *taken = true;
     return 0;
 }

@@ -1803,6 +1803,11 @@ extern "C" int64_t kvc_attention_workspace_bytes(int64_t total_tokens, int64_t v
     return kvc_attention_plan(total_tokens, v_compressed_tokens, batch, q_heads, head_dim).bytes;
 }
 
+static bool kvc_tail_in_merge(const kvc_compressed_desc *k, const kvc_compressed_desc *v)
+{
+    return v->tail_tokens > 0 && v->tail_tokens <= KVC_FINISH_MAX_TAIL && k->tokens >= v->tokens && kvc_option(KVC_OPT_ATTENTION_TAIL_IN_MERGE) != 0;
+}
+
 static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_desc *v, const void *d_q_f16,
                              float softmax_scale, void *d_workspace, int64_t workspace_bytes, float *d_out_f32,
                              int64_t batch, int64_t kv_heads, int64_t q_heads, int64_t head_dim,
@@ -1831,8 +1836,7 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
     // V's fp16 tail is handled by the merge kernel itself when it is short enough and K's compressed part reaches at
     // least as far as V's (the V kernel then needs no score of K's tail); otherwise by two kernels of its own
     KvcTailArgs tail = {};
-    const bool tail_in_merge = v->tail_tokens > 0 && v->tail_tokens <= KVC_FINISH_MAX_TAIL && k->tokens >= v->tokens &&
-                               kvc_option(KVC_OPT_ATTENTION_TAIL_IN_MERGE) != 0;
+    const bool tail_in_merge = kvc_tail_in_merge(k, v);
     if (tail_in_merge) {
         tail.k_tail = reinterpret_cast<const __half *>(k->d_tail_f16);
         tail.v_tail = reinterpret_cast<const __half *>(v->d_tail_f16);
@@ -1848,7 +1852,7 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
         tail.kv_heads = (int)kv_heads;
         tail.rep = rep;
     }
-    // small caches: K and V in one launch (unless the caller asked for the two kernels' times)
+    // K and V in one launch (unless the caller asked for the two kernels' times)
     bool joint = false;
     if (!fused_kernel_ms && (tail_in_merge || v->tail_tokens == 0)) {
         if (int rc = kvc_attend_groups(k, v, d_q_f16, softmax_scale, scores, p.scores_stride, part, ml, batch, kv_heads, q_heads, head_dim,
@@ -1912,7 +1916,7 @@ static int kvc_attention_run(const kvc_compressed_desc *k, const kvc_compressed_
 }
 
 // Which kernels a kvc_attention_decode of these caches takes, without running it (nothing is read through the descriptors' pointers): K's
-// KVC_BOOK_* (KVC_NO_BOOK) where two kernels decode K and V, V's << 4.
+// KVC_BOOK_* (KVC_NO_BOOK) where two kernels decode K and V, V's << 4, and KvcAttendRoute << 8, which says whether they do.
 extern "C" int kvc_attention_kernels(const kvc_compressed_desc *k, const kvc_compressed_desc *v, int64_t batch, int64_t kv_heads, int64_t q_heads,
                                      int64_t head_dim)
 {
@@ -1923,7 +1927,8 @@ extern "C" int kvc_attention_kernels(const kvc_compressed_desc *k, const kvc_com
         const int kind = is_k ? 0 : head_dim % KVC_WAVE == 0 ? 3 : 4;
         return kvc_plan_fused(a, is_k, kind, rep, rounded, tiles, c->encoded_bytes, c->max_tile_bytes, c->max_stream_bytes, c->max_code_bits, true).book;
     };
-    return book(k, true, k->tokens / KVC_WAVE * batch * kv_heads) | book(v, false, kvc_v_tiles(v, batch, kv_heads, head_dim)) << 4;
+    const int route = kvc_tail_in_merge(k, v) || v->tail_tokens == 0 ? kvc_attend_route(k, v, batch, kv_heads, q_heads, head_dim) : KVC_ATTEND_SEPARATE;
+    return book(k, true, k->tokens / KVC_WAVE * batch * kv_heads) | book(v, false, kvc_v_tiles(v, batch, kv_heads, head_dim)) << 4 | route << 8;
 }
 
 extern "C" int kvc_attention_decode(const kvc_compressed_desc *k, const kvc_compressed_desc *v, const void *d_q_f16,

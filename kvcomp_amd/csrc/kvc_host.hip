@@ -56,11 +56,11 @@ const OptionDef g_option_defs[KVC_OPT_COUNT] = {
     {"fused_builtin_dpp", "KVCOMP_FUSED_BUILTIN_DPP", 0},        // fp32-FMA kernels: the quad permute through the compiler's intrinsic, not inline assembly
     {"fused_schedule", "KVCOMP_FUSED_SCHEDULE", -1},             // matrix-core kernels: runs of tiles per wave that shorten towards the end of the launch; -1 choose per call, 0 never, r * 10000 + p * 100 + q: runs of r for the first p % of the tiles, r / 2 for the next q %
     {"encode_one_pass", "KVCOMP_ENCODE_ONE_PASS", 1},            // tile encoder: 1: one pass (a wave counts, places by a look-back over the tiles before it, and emits its tiles); 0: two passes; 2 / 3: one pass with one / two tiles per wave
-    {"fused_half_table", "KVCOMP_FUSED_HALF_TABLE", 1},          // matrix-core kernels: two-byte decode table entries for codes of 6 or 7 bits (one LDS word per bank)
+    {"fused_half_table", "KVCOMP_FUSED_HALF_TABLE", 1},          // matrix-core kernels: two-byte decode table entries for codes of 6 or 7 bits (one LDS word per bank), and the kernels with a symbol in one byte of them
     {"encode_lookback_polls", "KVCOMP_ENCODE_LOOKBACK_POLLS", 1 << 18},   // one-pass encoder: looks that may find a word not ready before a wave gives up (some tenths of a second); -1: treat every call as given up
     {"fused_schedule_v", "KVCOMP_FUSED_SCHEDULE_V", -1},         // the same for V launches: -1 follow fused_schedule (default schedule: runs that cover whole heads)
     {"fused_tiles_per_wave_v", "KVCOMP_FUSED_TILES_PER_WAVE_V", -1},   // plain grid, V launches: -1 follow fused_tiles_per_wave (default: the tiles of one head or head pair)
-    {"attention_joint", "KVCOMP_ATTENTION_JOINT", -1},             // kvc_attention_decode: K and V of a 128-token group in one workgroup; -1 choose per call, 0 never, 1 wherever it applies
+    {"attention_joint", "KVCOMP_ATTENTION_JOINT", -1},             // kvc_attention_decode: K and V of a 128-token group in one launch; -1 choose per call, 0 never, 1 by a workgroup, 2 by a wave, wherever those apply
 };
 std::atomic<int> g_options[KVC_OPT_COUNT];
 std::once_flag g_options_once;
