@@ -99,10 +99,11 @@ int kvc_abi_version(void);
  *                           block_infos is not 8-byte aligned or the call has more than 84 224 tiles, and by the other
  *                           encoders that start from uint8 symbols; 2 / 3: one pass for every encoder, with
  *                           always one / two tiles per wave.  Same bytes either way.
- *   "encode_lookback_polls": how often a wave of the one-pass encoder asks again for a size that an earlier tile has not
- *                           published yet before it gives the call up (default 262144; a wave normally asks 50 - 60
- *                           times at most, reported in d_result[6]).  Workgroups take their tiles by a ticket drawn when
- *                           they start, so what a wave waits for has always started before it; a call that is given up
+ *   "encode_lookback_polls": how often a wave of the one-pass encoder asks again, for one run of its tiles, for sizes that earlier tiles
+ *                           have not published yet before it gives the call up (default 262144; 20 - 170 times at most in calls
+ *                           of up to 84 224 tiles, reported in d_result[6]).  Runs of tiles are handed out in their order, by
+ *                           tickets; a wave publishes and places its own in that order and waits, in a placing, only for sizes
+ *                           before its own, so the earliest run not yet placed always can be.  A call that is given up
  *                           all the same is encoded again by one workgroup in two passes inside the same launch
  *                           sequence (same bytes, no error, 50 - 100 x slower).  0: every wait gives up at once, -1:
  *                           every call is treated as given up -- both only drive that path from a test.

@@ -1768,7 +1768,7 @@ __device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint
 // With runs, late look-back and wide stores this kernel took 54 and 47 us there, and 159 and 115, with 28 | 23 % of a wave's time (clock
 // stamps, K | V of 4 x 32 x 96 x 32 768) spent looking back -- waves wait for the slowest tile before theirs -- and 9 | 8 % on the
 // start; loads 12 | 15, look-ups 14 | 18, packing 20 | 22, writing 13 | 10.  Made-up offsets, so no look-back, had shown what that costs:
-// 146 and 99 us for 198 and 126.  So where there are more runs than waves, the workgroups that the chip holds stay (`persistent`),
+// 146 and 99 us for 198 and 126.  So where there are more runs than waves, the workgroups that the chip holds stay,
 // load the table once and draw run after run, and a run's images are placed when the next run's first tile has been counted
 // and its size published: what the look-back waits for has had a tile's loads and look-ups longer to arrive, and nobody waits for
 // the placing.  54 -> 50 us and 47 -> 47; 159 -> 146 and 115 -> 107.  A wave publishes and places in the order of the tiles, and
@@ -1815,7 +1815,7 @@ __global__ void __launch_bounds__(4 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     const int tiles = (int)a.tiles;
     const uint32_t base = a.status[KVC_ONCE_BASE_WORD];
     uint32_t err = 0, max_tile = 0, longest = 0, next_off = 0;
-    int polls = 0;
+    int polls = 0, most_polls = 0;                         // of this run and the placing of the one before, of any
     bool placed = false;                                   // the tiles of the run up to the first kept one have been; they end at next_off
     // Tiles whose images wait in the area: `kept` of them, their payload bytes (sixteen bits each, the oldest lowest), the words
     // they take and what is known of the bytes in front of the oldest one.
@@ -1935,6 +1935,10 @@ __global__ void __launch_bounds__(4 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         if (it == 0) {
             if (kept) place_kept(a, lane);
             placed = false;
+            if (polls <= a.max_polls) {                    // (a wave that has given up waits for nothing any more)
+                most_polls = polls > most_polls ? polls : most_polls;
+                polls = 0;
+            }
         }
         // the tile that the run's place is looked for with; and the wave that speaks for a group must not sit on its size (as in
         // kvc_encode_once_kernel)
@@ -1980,7 +1984,7 @@ __global__ void __launch_bounds__(4 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
         if (err) atomicOr(&s_err, err);
         atomicMax(&s_max_tile, max_tile);
         atomicMax(&s_longest, longest);
-        atomicMax(&s_polls, (uint32_t)polls);
+        atomicMax(&s_polls, (uint32_t)(polls > most_polls ? polls : most_polls));
     }
     __syncthreads();
     if (tid == 0) {                                        // to one of the slot's lines, picked by the first ticket

@@ -97,3 +97,11 @@ def test_waves_that_give_up_waiting(is_k, T, B, H, D, polls):
                                                        (False, "TokenQuant", 128 * 131, 2, 67, 96, 0.1, True)])
 def test_first_stores_of_several_rounds(is_k, mode, T, B, H, D, eb, wide, polls):
     _both(is_k, mode, _data(T, B, H, D, wide, 3), eb, polls=polls)
+
+
+def test_the_budget_of_waiting_is_a_runs():
+    """What is reported is the most that a wave has asked in vain for a run of its tiles, not for the five or six that it takes in this call:
+    50 to 170 here, added up over the runs 180 to 330.  The least of a few calls, which other work on the machine does not raise."""
+    sym = _symbols(128 * 650, 1, 129, 64, False, 0.0)
+    cap = _room(False, sym)
+    assert min(int(_encode(False, sym, cap, 7)[3][6]) for _ in range(8)) < 140
