@@ -1130,6 +1130,9 @@ __global__ void __launch_bounds__(KVC_WG) kvc_store_emit_kernel(KvcStoreArgs a)
 // published, and a group's size only needs the sizes of its own tiles.  So whatever a wave waits for is published
 // by waves that are running and wait for nothing before they publish.  (Placing a run's first tile before its
 // second was counted breaks rule 2 and turns the launch into one chain from wave to wave: 18 ms instead of 0.2.)
+// Workgroups that stay (kvc_encode_symbols_kernel) draw a ticket per run, and a wave places a run when the next one's first tile is
+// published; it then waits only for tiles before the run that it places.  The wave of the earliest tile not yet published waits, if at
+// all, in placing a run that lies before that tile, for tiles that are all published.
 // A wave that has found a word not ready more than max_polls times gives up all the same, flags the call
 // (KVC_ENC_ERR_ORDER) and publishes what it has, so that every wave ends; kvc_encode_finish_kernel then encodes the
 // whole call again the slow, safe way (two passes inside one workgroup), so a give-up costs time, not the result.
@@ -1783,6 +1786,11 @@ __device__ __forceinline__ void kvc_load_pair_table(const KvcEncodeArgs &a, uint
 // of at most eight bits, or of any length.
 enum { KVC_FORM_BYTES = 0, KVC_FORM_PACKED = 1, KVC_FORM_PACKED_LONG = 2 };
 constexpr int KVC_SYM_TICKETS = 8;                         // tickets of a workgroup that are kept: more than its fastest wave is ahead of its slowest
+// Waves that take the tiles of their runs in turn (see there); vec_len: symbols of a vector, 4 ND where they fill ND registers
+constexpr int kvc_symbols_step(bool is_k, int vec_len, bool packed)
+{
+    return packed ? (is_k ? 1 : 4) : !is_k ? 2 : vec_len == 96 || vec_len == 72 ? 4 : vec_len == 64 ? 2 : 1;
+}
 // long_run: tiles of a wave's run, short_run: of those of tickets from short_from on (0: no workgroup draws a second one).
 template <int FRONT, int ND, int FORM>
 __global__ void __launch_bounds__(4 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEncodeArgs a, int long_run, int short_run, int short_from)
@@ -1810,7 +1818,7 @@ __global__ void __launch_bounds__(4 * KVC_WG, 4) kvc_encode_symbols_kernel(KvcEn
     // 8 x 32 heads x 128 x 4096 tokens in runs of two 295 -> 173 MB, 78 -> 68 us (58 in runs of four); 4 x 32 x 96 x 32 768: K 757 ->
     // 603 MB, 259 -> 238 us, V 798 -> 483 MB, 182 -> 163 us; K, 2 x 32 x 64 x 8192: 32 -> 31 us.
     // Two symbols a byte: four V tiles are a line of each token's row, and a K tile is lines of its own.
-    constexpr int STEP = PACKED ? (FRONT == 1 ? 4 : 1) : FRONT == 1 ? 2 : ND == 24 || ND == 18 ? 4 : ND == 16 ? 2 : 1, OTHERS = STEP > 1 ? STEP - 1 : 1;
+    constexpr int STEP = kvc_symbols_step(FRONT == 0, 4 * ND, PACKED), OTHERS = STEP > 1 ? STEP - 1 : 1;
     static_assert(PACKED ? G % (STEP * 3) == 0 && G % (STEP * 4) == 0 : G % (STEP * (FRONT == 1 ? 4 : 2)) == 0, "their tiles lie in one group");
     const int tiles = (int)a.tiles;
     const uint32_t base = a.status[KVC_ONCE_BASE_WORD];
@@ -2384,8 +2392,7 @@ static int kvc_encode_launch(const KvcEncodeCall &c, void **slot_out, hipStream_
         if (wide && small && want == 1 && a.tiles > KVC_WIDE_WAVES) run = 2;
         int waves = wide && small && run >= 2 ? 2 * KVC_WAVES_PER_WG : KVC_WAVES_PER_WG;
         const size_t lds = (size_t)(a.rows_per_codebook ? waves : 1) * 256 * sizeof(uint2) + (size_t)waves * sa.e.wave_bytes;
-        // waves that take their tiles in turn, as the kernel's STEP
-        const int step = c.packed ? (is_k ? 1 : 4) : !is_k ? 2 : a.vec_len == 96 || a.vec_len == 72 ? 4 : a.vec_len == 64 ? 2 : 1;
+        const int step = kvc_symbols_step(is_k, a.vec_len, c.packed);
         // Four V tiles to a look-back where the images of three wait beside the fourth's staging area (what the waves that read
         // together take stays inside a group, or the wave that speaks for a group would wait before all its tiles are counted).
         const int64_t image = a.encoded_cap / a.tiles * 9 / 8;
