@@ -159,8 +159,9 @@ static inline bool kvc_streams_resonate(int64_t encoded_bytes, int64_t tiles)
 // by more than 128 symbols x 10 bits, and the workgroup's LDS ends with that much slack (KVC_LDS_SLACK_WORDS),
 // so even a corrupt stream only ever reads this workgroup's own LDS.
 typedef __attribute__((address_space(3))) uint32_t kvc_lds_word;
-// WORD: left to itself the compiler makes "u >> 3 & ~3" of the word's address, an instruction more than shift and shifted add.  1 x 8 x 4 heads x
-// 128 x 1000 tokens 16.64 -> 16.47 us; but with codes of more than 7 bits 2 x 8 x 8 x 128 x 1905 takes 41.0 us for 40.6.
+// WORD: left to itself the compiler makes "u >> 3 & ~3" of the word's address, an instruction more than shift and shifted add.  A percent at
+// most either way, as measured in turn: attention of 1 x 8 x 4 heads x 128 x 1000 tokens 16.49 -> 16.44 us, but with codes of more than 7
+// bits, whose loop asks in several places, 2 x 8 x 8 x 128 x 1905 tokens 40.6 -> 41.0.
 template <bool SKEW, bool WORD = false>
 __device__ __forceinline__ uint32_t kvc_refill_address(uint32_t stage_base, uint32_t u)
 {

@@ -23,24 +23,25 @@ def _attend(kc, vc, q, joint):
 # T: one group and nothing else, a token more; K a block ahead of V; every number of groups in the last workgroup; both tails
 @pytest.mark.parametrize("T", [128, 129, 192, 257, 448, 520, 700, 1000])
 @pytest.mark.parametrize("B,H,rep", [(1, 1, 1), (3, 2, 2), (1, 8, 4), (1, 2, 8)])
-@pytest.mark.parametrize("skew", [0, 1])
+@pytest.mark.parametrize("skew", [0, 1, 2])
 def test_equals_the_two_kernels(T, B, H, rep, skew):
     from kvcomp_amd import _lib
     kc, vc = _contexts(T, B, H, 128)
     assert kc.code_hint & 0x200 and vc.code_hint & 0x200 and kc.max_code_bits in (6, 7) and vc.max_code_bits in (6, 7)
     q = S.synth_q(B, H * rep, 128).to(DEV)
-    was = _lib.set_option("fused_skew", skew)
+    got = _attend(kc, vc, q, 2)
+    was = _lib.set_option("fused_skew", skew)                   # how the two kernels' payloads lie
     try:
-        got = _attend(kc, vc, q, 2)
+        want = _attend(kc, vc, q, 0)
     finally:
         _lib.set_option("fused_skew", was)
-    assert torch.isfinite(got).all() and torch.equal(_attend(kc, vc, q, 0), got)
+    assert torch.isfinite(got).all() and torch.equal(want, got)
 
 
 @pytest.mark.parametrize("k_mode,v_mode,B", [("BlockQuant", "VectorQuant", 2), ("ChannelQuant", "VectorQuant", 1), ("ChannelQuant", "TokenQuant", 2)])
 @pytest.mark.parametrize("eb_k,eb_v", [(0.1, 0.2), (0.2, 0.3), (0.08, 0.12), (0.05, 0.05)])
 def test_code_lengths_and_layouts(k_mode, v_mode, B, eb_k, eb_v):
-    """(where the codes are not this kernel's, the call goes to the others)"""
+    """(where the codes are not this kernel's, the call goes to the others; its own in test_gpu_waves_default.py)"""
     kc, vc = _contexts(330, B, 3, 128, k_mode, v_mode, eb_k, eb_v)
     q = S.synth_q(B, 6, 128).to(DEV)
     assert torch.equal(_attend(kc, vc, q, 0), _attend(kc, vc, q, 2))

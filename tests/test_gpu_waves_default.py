@@ -9,6 +9,7 @@ from kvcomp_amd import _lib
 from kvcomp_amd.attention import CompressedAttention
 from kvcomp_amd.ctx import KVCompCacheConfig, KVCompCacheConfigStatic, KVCompCtx, QuantMode
 from tests import _synth as S
+from tests.test_gpu_joint_attention import _contexts as _some_contexts
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -66,6 +67,21 @@ def test_a_token_of_rare_symbols(rep):
     assert _route(kc, vc, 8, 32, rep) == (JOINT if rep == 8 else TWO_KERNELS) and _equal(kc, vc, q, -1) and _equal(kc, vc, q, 1)
     small = _contexts(900, 1, 2, odd=(70, 391))
     assert _equal(*small, S.synth_q(1, 2 * rep, 128).to(DEV), 2)
+
+
+@pytest.mark.parametrize("k_mode,v_mode,B", [("BlockQuant", "VectorQuant", 2), ("BlockQuant", "TokenQuant", 1), ("ChannelQuant", "VectorQuant", 1),
+                                             ("ChannelQuant", "TokenQuant", 2)])
+@pytest.mark.parametrize("eb_k,eb_v", [(0.2, 0.2), (0.2, 0.25), (0.25, 0.2), (0.3, 0.3)])
+def test_layouts_of_both_code_lengths(k_mode, v_mode, B, eb_k, eb_v):
+    kc, vc = _some_contexts(330, B, 3, 128, k_mode, v_mode, eb_k, eb_v)
+    assert kc.max_code_bits in (6, 7) and vc.max_code_bits in (6, 7)
+    q = S.synth_q(B, 6, 128).to(DEV)
+    was = _lib.set_option("attention_joint", 2)
+    try:
+        assert _route(kc, vc, B, 3, 2) == WAVES
+    finally:
+        _lib.set_option("attention_joint", was)
+    assert _equal(kc, vc, q, 2)
 
 
 @pytest.mark.parametrize("longest", [0, 40, 56])
