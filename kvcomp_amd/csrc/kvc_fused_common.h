@@ -593,7 +593,8 @@ __device__ __forceinline__ KvcStaged kvc_stage_payload(const KvcFusedArgs &a, in
 // within 6 words).  The loads' addresses are as far apart as the streams are long, which costs nothing: 65 536 tiles of 3360
 // bytes in 33 us, as with whole lines in order.
 // With them the attention kernels of 4 x 32 heads x 96 x 32 768 tokens (K six bits and skewed before, V two symbols per look-up) take 152 us
-// for 161; there is no skewed variant of a loop any more, and the kernels need two to six registers less.
+// for 161; such a kernel has no skewed variant of its loops and needs two to six registers less than the packed one.  Which calls
+// take columns: kvc_columns_from, kvc_columns_workgroups.
 struct KvcLane {
     const uint8_t *base;      // wave-uniform, a multiple of four
     uint32_t at;              // the stream's first word, in bytes from there

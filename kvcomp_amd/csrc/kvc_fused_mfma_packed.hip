@@ -1,4 +1,4 @@
-// kvc_fused_mfma_packed.hip -- the matrix-core kernels for codes of at most 7 bits whose payloads are packed (kvc_mfma_columns says
+// kvc_fused_mfma_packed.hip -- the matrix-core kernels for codes of at most 7 bits whose payloads are packed (kvc_plan_fused says
 // which calls those are).
 #include "kvc_fused_mfma_impl.h"
 

@@ -46,7 +46,7 @@ def test_matrix_core_kernels_keep_the_occupancy_they_are_launched_for(resources)
     (with one query head per KV head: 8 for the K kernel, 7 for the V kernels that decode attention uses -- softmax on
     the fly, kinds 3 and 4 --, at least 6 for the others)."""
     per = {}
-    for src in ("kvc_fused_mfma.hip", "kvc_fused_mfma_v96.hip"):
+    for src in ("kvc_fused_mfma.hip", "kvc_fused_mfma_v96.hip", "kvc_fused_mfma_packed.hip"):
         per.update(resources[src])
     assert any("ILi1ELi4ELb1E" in name for name in resources["kvc_fused_mfma_v96.hip"])
     for name, r in per.items():
