@@ -1081,9 +1081,9 @@ static KvcFusedPlan kvc_plan_fused(KvcFusedArgs &a, bool is_k, int kind, int rep
     const int want = kvc_option(KVC_OPT_FUSED_SKEW);
     // (a layout that was asked for; else packed without the longest stream's length, which would decide which tiles the LDS holds)
     if (!long_codes && (rep != 8 || (is_k && byte_entries)) &&
-        (want == 2 || (want < 0 && max_stream_bytes > 0 && tiles >= kvc_columns_from(is_k, rep, byte_entries, rounded)))) {
+        (want == 2 || (want < 0 && max_stream_bytes > 0 && tiles >= kvc_columns_from(is_k, rep, a.head_dim, byte_entries, rounded)))) {
         const size_t lds = plan(true);
-        if (want == 2 || kvc_lds_workgroups(lds) >= kvc_columns_workgroups(rep, slots)) return {byte_entries ? KVC_BOOK_MID : KVC_BOOK_SHORT, lds};
+        if (want == 2 || kvc_lds_workgroups(lds) >= kvc_columns_workgroups(is_k, rep, slots, byte_entries)) return {byte_entries ? KVC_BOOK_MID : KVC_BOOK_SHORT, lds};
     }
     return {long_codes ? KVC_BOOK_LONG : KVC_BOOK_PACKED, plan(false)};
 }
@@ -1923,6 +1923,7 @@ extern "C" int kvc_attention_kernels(const kvc_compressed_desc *k, const kvc_com
     const int rep = (int)(q_heads / kv_heads);
     const bool rounded = kvc_option(KVC_OPT_FUSED_ROUNDED) != 0;
     KvcFusedArgs a = {};
+    a.head_dim = (int)head_dim;
     auto book = [&](const kvc_compressed_desc *c, bool is_k, int64_t tiles) {
         const int kind = is_k ? 0 : head_dim % KVC_WAVE == 0 ? 3 : 4;
         return kvc_plan_fused(a, is_k, kind, rep, rounded, tiles, c->encoded_bytes, c->max_tile_bytes, c->max_stream_bytes, c->max_code_bits, true).book;

@@ -692,27 +692,36 @@ __device__ __forceinline__ uint32_t kvc_column_address(uint32_t column, uint32_t
 }
 enum { KVC_BOOK_SHORT = 0, KVC_BOOK_MID = 1, KVC_BOOK_LONG = 2, KVC_BOOK_PACKED = 3 };       // of kvc_fused_mfma_kernel
 // Which launches of the matrix-core kernels for codes of at most 7 bits take their payloads in columns (eight query heads: K's with one-byte
-// entries only; the rest has no such kernels, V's took 41.3 us for 40.4 at 2 x 8 x 8 heads x 128 x 1905 tokens).  From `tiles` of a kind on: a wave of fewer waits for its one tile, which the lanes' own loads
-// make longer.  Packed against columns in us, 4 x 8 KV heads, head_dim 128, rounded arithmetic, one-byte entries in columns:
-//   K  1 query head   2048 tiles 11.8 : 11.9    3072 13.1 : 12.5    4096 14.9 : 13.5    8192 26.3 : 23.1   32768 70 : 61
-//      2              2048       11.0 : 11.6    3072 12.6 : 12.4    4096 14.4 : 13.8    8192 26.0 : 23.2   32768 73 : 64
-//      4              2048       12.7 : 13.0    3072 14.3 : 14.2    4096 16.3 : 15.4    8192 28.7 : 26.2   32768 80 : 72
-//      8              2048       15.4 : 15.9    3072 18.6 : 18.4    4096 27.3 : 21.1    6144 33.6 : 31.4   32768 141 : 118
-//   V  1, 2, 4        from 512 tiles on 11.1 : 11.2, 10.5 : 10.7 (256), 12.4 : 12.0 (128); 4096 16.0 : 14.2, 15.6 : 14.6, 17.7 : 16.2
-// other codebooks (K and V one query head; with two and four the same to 0.5 us):
+// entries only; the rest has no such kernels, V's took 41.3 us for 40.4 at 2 x 8 x 8 heads x 128 x 1905 tokens).  From `tiles` of a kind on: a
+// wave of fewer waits for its one tile, which the lanes' own loads make longer, by how much depends on a stream's sixteen-byte loads.
+// K with one-byte entries, whole attention calls over 4 x 8 KV heads with K packed, and what its columns add, us:
+//   head_dim 128  1 query head  1024 tiles 23.1 +0.2   2048 24.2 +0.0   2560 26.1 -0.4      96  512 21.5 -0.3       72  256 20.2 -0.4
+//                 2             1024       22.3 +0.8   2048 23.9 +0.5   2560 26.1 +0.0      96 1024 21.5 +0.4   2560 23.9 -0.2      72 2048 21.8 +0.1
+//                 4             1024       26.6 +0.2   2048 28.0 +0.2   2560 30.5 -0.3      96 1024 25.7 +0.3   2560 28.5 -0.6      72 1024 24.3 -0.1
+//                 8             1024       31.0 +0.5   2048 36.2 +0.2   2560 42.3 +0.0    3584 61.9 -6.1                        72 2048 34.3 +0.0
+//   and the kernel alone at 32 768 tiles of 128, 1, 2, 4 and 8 query heads: 70, 73, 80 and 141 -> 61, 64, 72 and 118
+// V with one-byte entries, the kernel with 1, 2 and 4 query heads: 512, 256 and 128 tiles 11.1 : 11.2, 10.5 : 10.7 and 12.4 : 12.0, 4096 tiles 16.0 :
+// 14.2, 15.6 : 14.6 and 17.7 : 16.2.  Other codebooks (one query head; with two and four the same to 0.5 us):
 //   K 2048 10.5 : 10.9   4096 13.2 : 13.3   8192 19.8 : 19.2      V 2048 9.4 : 10.1   3072 12.1 : 10.9   8192 20.7 : 19.8
 // and products that are not rounded: K 2048 10.4 : 11.6   8192 21.5 : 23.3   16384 35.2 : 34.5    V 2048 11.0 : 11.6   4096 14.4 : 14.6   8192 23.8 : 22.4
-constexpr int64_t kvc_columns_from(bool is_k, int rep, bool byte_entries, bool rounded)
+constexpr int64_t kvc_columns_from(bool is_k, int rep, int head_dim, bool byte_entries, bool rounded)
 {
-    return !rounded ? (is_k ? 16384 : 4096) : !byte_entries ? (is_k ? 4096 : 3072) : !is_k ? 0 : rep == 8 ? 4096 : 3072;
+    if (!rounded) return is_k ? 16384 : 4096;
+    if (!byte_entries) return is_k ? 4096 : 3072;
+    return !is_k || (rep == 1 && head_dim <= 96) || (rep == 4 && head_dim <= 72) ? 0 : 2560;
 }
 // ... and where the LDS still holds this many workgroups of a compute unit: columns are as long as the longest stream of the whole cache,
 // packed payloads take their tile's bytes.  K of 4 x 32 heads x 96 x 32 768 tokens, packed 99 us: columns of 13, 17, 19, 21 and 29 words 84, 91,
 // 96, 107 and 127 (eight, six, six, five and four workgroups); V (71): 6, 11 and 15 words 70, 73 and 80 (seven, six, five).  K and V of
 // 8 x 8 heads x 128 x 8320, two query heads, 53: 17, 25 and 27 words 49, 51 and 60 (six, five, four); four query heads, 60: 17, 21 and 23 words 57,
 // 58 and 74 (five, five, four), of head_dim 96 and 8192 tokens V (29.8): 12 and 19 words 27.9 and 28.5 (five, four; its registers allow four);
-// eight, K and V 99: 21 and 23 words 95.8 and 99.1 (four, three).
-constexpr int kvc_columns_workgroups(int rep, int slots) { return rep == 1 ? 6 : rep == 2 || (rep == 4 && slots == 1) ? 5 : 4; }
+// eight, K and V 99: 21 and 23 words 95.8 and 99.1 (four, three).  K with wider entries of 7-bit codes, whose loop is longer: 8192 and 16 384 tiles of
+// head_dim 128 (20 words, five) 25.9 and 41.2 -> 26.8 and 45.7 with two query heads, 28.3 and 50.1 -> 29.3 and 51.2 with four; of 72 (13
+// words, eight and six) 16.6 and 27.0 -> 16.5 and 26.8, 19.6 and 30.8 -> 18.7 and 30.0.
+constexpr int kvc_columns_workgroups(bool is_k, int rep, int slots, bool byte_entries)
+{
+    return rep == 1 || (is_k && !byte_entries) ? 6 : rep == 2 || (rep == 4 && slots == 1) ? 5 : 4;
+}
 enum { KVC_PACKED_PLAIN = 0, KVC_PACKED_SKEWED = 1, KVC_COLUMNS = 2 };
 // The three words of a refill.  base: kvc_refill_address's, or the lane's column.
 template <int LAYOUT, bool WORD = true>

@@ -33,12 +33,18 @@ def _route(*args, **kw):
     return _asked(*args, **kw) >> 8
 
 
-@pytest.mark.parametrize("rep,first", [(1, 3072), (2, 3072), (4, 3072), (8, 4096)])
-def test_columns_begin_where_they_pay(rep, first):
+@pytest.mark.parametrize("rep,D,first", [(1, 128, 2560), (2, 128, 2560), (2, 72, 2560), (4, 128, 2560), (4, 96, 2560), (8, 128, 2560), (8, 72, 2560)])
+def test_columns_begin_where_they_pay(rep, D, first):
     """A wave of a small cache waits for its one tile, which the lanes' own loads make longer."""
     v = PACKED if rep == 8 else BYTES
-    assert _kernels(1, 8, rep, 128, (first // 8 - 2) * 64) == (PACKED, v)
-    assert _kernels(1, 8, rep, 128, first // 8 * 64) == (BYTES, v)
+    assert _kernels(1, 8, rep, D, (first // 8 - 2) * 64) == (PACKED, v)
+    assert _kernels(1, 8, rep, D, first // 8 * 64) == (BYTES, v)
+
+
+@pytest.mark.parametrize("rep,D", [(1, 96), (1, 72), (1, 64), (4, 72), (4, 64)])
+def test_short_streams_lie_in_columns_from_the_first_tile(rep, D):
+    for tokens in (128, 1024, 16384):
+        assert _kernels(1, 8, rep, D, tokens, k=(7, 52 * D // 128, 59 * D // 128)) == (BYTES, BYTES)
 
 
 @pytest.mark.parametrize("rep", [1, 2, 4])
@@ -64,6 +70,14 @@ def test_one_long_stream_does_not_size_every_waves_lds(rep, D):
     odd = (7, 52 * D // 128, 112)
     assert _kernels(4, 8, rep, D, 32768, k=odd, v=even["v"])[0] == PACKED
     assert _kernels(4, 8, rep, D, 32768, k=even["k"], v=(7, 32, 112)) == (BYTES, PACKED)
+
+
+@pytest.mark.parametrize("rep", [1, 2, 4])
+def test_wider_entries_of_long_codes_keep_more_workgroups(rep):
+    """Codes of 7 bits of symbols beyond 16, K of an error bound of 0.05: streams of 76 bytes leave five workgroups, of 44 six and more."""
+    assert _kernels(4, 8, rep, 128, 16384, k=(7, 70, 76), symbols=0x100)[0] == PACKED
+    assert _kernels(4, 8, rep, 72, 16384, k=(7, 39, 44), symbols=0x100)[0] == COLUMNS
+    assert _kernels(4, 8, rep, 128, 16384, k=(7, 52, 67))[0] == BYTES
 
 
 def test_a_stream_hint_that_is_not_there():

@@ -75,7 +75,7 @@ def test_symbols_beyond_what_the_hint_states_take_the_slow_path():
     assert (got.float() - want.float()).abs().max() <= 1e-3 * want.float().abs().max()
 
 
-@pytest.mark.parametrize("T", [32704, 32768])           # K tiles either side of the line from which eight query heads have kernels of their own
+@pytest.mark.parametrize("T", [32704, 32768])           # (the line from which columns are taken: test_gpu_payload_layouts.py)
 def test_eight_query_heads(T):
     from kvcomp_amd import _lib
     kc, _ = _contexts(T, 1, 8, 64, 11)

@@ -43,7 +43,7 @@ def test_every_layout_gives_the_same_bits(B, H, rep, D, T, eb_k, eb_v, smooth, r
     assert (few.float() - want).abs().max() <= 1e-3 * want.abs().max()
 
 
-@pytest.mark.parametrize("rep,tiles", [(1, 3072), (8, 4096)])
+@pytest.mark.parametrize("rep,tiles", [(2, 2560), (8, 2560)])
 def test_either_side_of_the_line_for_columns(rep, tiles):
     for T in (tiles // 8 * 64 - 64, tiles // 8 * 64):
         kc, _ = _contexts(T, 1, 8, 64)
